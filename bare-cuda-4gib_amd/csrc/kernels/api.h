@@ -52,6 +52,11 @@ int bc4g_rmsnorm_sum(float* x, const float* parts, int n_parts, const float* bia
 int bc4g_gemm_generic(const void* a, int a_dtype, const void* w, int w_dtype, void* out,
                       int out_dtype, int accumulate, const float* bias, int m, int n, int k, void* stream);
 
+// The same for float operands on the matrix cores: x [m, k], w [n, k], k a multiple of 4, x and w on 16-byte boundaries.
+// epilogue 0: stored; 1: added to out, with bias [n] (null: none); 2, 3: w holds n / 2 gate rows, then as many up rows, and
+// out [m, n / 2] is silu (3: the gelu written with tanh) of the gate times up.
+int bc4g_gemm_f32(const float* x, const float* w, const float* bias, float* out, int epilogue, int m, int n, int k, void* stream);
+
 // out[t, i] = silu(gate_i) * up_i                                        (swiglu.cu:17-25)
 // interleaved 0: gu[t] = all gates, then all ups.  1: blocks of 16 = eight gates, then the eight
 // ups of the same outputs.  act 1: the gelu written with tanh instead of the silu.

@@ -1,0 +1,475 @@
+// out[m, n] (+)= sum_k x[m, k] * w[n, k] in float32 on the matrix cores (v_mfma_f32_*_f32: float operands, float sums, no operand
+// rounded anywhere): the products of the 32-bit path.  Operands lie by rows; k a multiple of 4, rows on 16-byte boundaries
+// (gemm_generic takes what these refuse).  Both kernels add up k in the same order, eight shares from zero and the shares in
+// order: a row's bits do not depend on how many rows came with it.
+//
+// gemm_f32_stream_kernel, few rows (a decode step), bound by reading w once.  A workgroup owns 16 rows of w (or eight gate
+// rows and the eight up rows of the same outputs) and all of k, a share of it each of its 8 waves.  A wave's part of w and of x goes
+// from memory into a ring of its own in LDS without passing registers -- whole cache lines of 128 bytes a row (lanes that read 16
+// rows' 16 bytes straight into operand order keep the texture path busy four times as long), several steps of 32 k ahead and
+// with no barrier; it reads its fragments there and feeds 16x16x4 MFMAs with w as the A operand.  The shares meet in LDS.
+// Eight rows, weights not in a cache, plain float FMA (gemm_generic) -> this: 32,000 x 2,048 142 -> 49 us (5.4 TB/s), 11,264 x
+// 2,048 61 -> 21, 2,048 x 5,632 86 -> 19; 32 decode steps of 8 requests after their prompts at TinyLlama's sizes 211 -> 87 ms.
+//
+// gemm_f32_tiled_kernel, many rows, bound by the matrix cores (157 TFLOP/s of float32 at the full clock).  A step's 32 k of the
+// tile's rows of x and of w go straight into a ring of stages in LDS; the waves feed 32x32x2 MFMAs from there and keep
+// two sets of sums, the share's and the total.  2,048 x 11,264 x 2,048: 124 TFLOP/s, 2,048 x 2,048 x 5,632: 125 (plain FMA: 45 to 50); a
+// 1,000-token prompt at TinyLlama's sizes 74 -> 48 ms (30 of which is attention).
+#include <math.h>
+
+#include "api.h"
+#include "mfma.h"
+
+namespace bc4g {
+namespace {
+
+constexpr int kWaves = 8;                     // of the few rows' kernel: one a share of k
+constexpr int kThreads = kWaves * kWave;
+constexpr int kStepK = 32;                    // floats of a row a step brings: one cache line
+constexpr int kStepBytes = kStepK * 4;
+constexpr int kRedPad = 17;
+constexpr int kXcds = 8;
+
+enum Epilogue : int { kStore = 0, kAccum = 1, kSwiglu = 2, kGeglu = 3 };
+constexpr bool gated(int epi) { return epi == kSwiglu || epi == kGeglu; }
+
+// The activations as the elementwise kernel has them.
+template <int EPI>
+__device__ inline float gate_act(float g) {
+  if constexpr (EPI == kGeglu) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
+  return g / (1.0f + expf(-g));
+}
+
+struct Args {
+  const float* x;           // [m, k]
+  const float* w;           // [n, k]; gated: n / 2 gate rows, then the up rows
+  const float* bias;        // kAccum: [n] (null: none)
+  float* out;               // [m, n], gated: [m, n / 2]
+  int m, n, k;
+};
+
+// k is added up in eight shares of whole steps, each from zero, and the shares' sums in order: by both kernels, so that a row's
+// bits do not depend on how many rows came with it.
+constexpr int kShares = 8;
+__host__ __device__ inline int steps_a_share(int k) { return ((k + kStepK - 1) / kStepK + kShares - 1) / kShares; }
+
+__device__ inline floatx4 mfma_16x16x4(float a, float b, floatx4 acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
+
+// Where 16-byte segment s of row r of a step lies in the row's 128 bytes of LDS: s ^ key(r), so that the 16 rows' reads of one
+// segment (two rows share the 64 banks' span) meet different banks.
+__device__ inline int slot_key(int row) { return (row >> 1) & 7; }
+
+// N wave-wide loads to N KB of consecutive LDS as one statement, load i from its own scalar base and lane offsets: the LDS
+// address travels in m0, set once, and the loads' offset field (which moves the memory address too: taken off the base here)
+// steps through the stretch.
+template <int N>
+__device__ inline void load_pieces_to_lds(const float* const (&bases)[N], const unsigned (&offsets)[N], unsigned lds_first) {
+  static_assert(N == 3 || N == 4 || N == 6, "two pieces of weights and one, two or four of x");
+  constexpr int kMid = N / 2;
+  const void* b[N];
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(bases[r]) - (r - kMid) * 1024;
+    const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(bits));
+    const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(bits >> 32));
+    b[r] = reinterpret_cast<const void*>((static_cast<uintptr_t>(hi) << 32) | lo);
+  }
+  const unsigned mid = __builtin_amdgcn_readfirstlane(lds_first + kMid * 1024);
+#define BC4G_PIECE(i, v, s) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #i "\n\t"
+  if constexpr (N == 3) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-1024, 1, 4) BC4G_PIECE(0, 2, 5) BC4G_PIECE(1024, 3, 6)
+                 ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "v"(offsets[2]), "s"(b[0]), "s"(b[1]), "s"(b[2]) : "memory", "m0");
+  } else if constexpr (N == 4) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-2048, 1, 5) BC4G_PIECE(-1024, 2, 6) BC4G_PIECE(0, 3, 7) BC4G_PIECE(1024, 4, 8)
+                 ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "v"(offsets[2]), "v"(offsets[3]), "s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3])
+                 : "memory", "m0");
+  } else {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-3072, 1, 7) BC4G_PIECE(-2048, 2, 8) BC4G_PIECE(-1024, 3, 9) BC4G_PIECE(0, 4, 10)
+                 BC4G_PIECE(1024, 5, 11) BC4G_PIECE(2048, 6, 12)
+                 ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "v"(offsets[2]), "v"(offsets[3]), "v"(offsets[4]), "v"(offsets[5]), "s"(b[0]),
+                 "s"(b[1]), "s"(b[2]), "s"(b[3]), "s"(b[4]), "s"(b[5]) : "memory", "m0");
+  }
+#undef BC4G_PIECE
+}
+
+// Which tile a workgroup takes: consecutive ones stay on one XCD (workgroups are dealt to the eight in turn) and walk the output
+// in bands of eight rows of tiles, so that those on an XCD at one time share their rows of x and of w in its L2.
+__device__ inline void tile_of(int block, int m_blocks, int n_blocks, int& bm, int& bn) {
+  const int total = m_blocks * n_blocks;
+  const int logical = total % kXcds == 0 ? (block % kXcds) * (total / kXcds) + block / kXcds : block;
+  const int per_band = 8 * n_blocks, first = (logical / per_band) * 8, rows = min(8, m_blocks - first);
+  bm = first + logical % per_band % rows;
+  bn = logical % per_band / rows;
+}
+
+// Waits until only the loads of `later` steps of PER loads each are outstanding (they finish in order).
+template <int PER, int MAX>
+__device__ inline void wait_for_step(int later) {
+  if constexpr (MAX == 0) {
+    wait_loads<0>();
+  } else {
+    if (later >= MAX) wait_loads<PER * MAX>();
+    else wait_for_step<PER, MAX - 1>(later);
+  }
+}
+
+// XR: rows of x a workgroup takes (blockIdx.y: which).
+template <int XR, int STAGES, int EPI>
+__global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a) {
+  constexpr int MT = (XR + 15) / 16, PER = 2 + XR / 8, kRing = PER * 1024;
+  extern __shared__ __align__(1024) unsigned char stream_lds[];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int col = lane % 16, grp = lane / 16;
+  const int k = a.k, row0 = blockIdx.y * XR, m = min(XR, a.m - row0);
+  constexpr int kCols = gated(EPI) ? 8 : 16;                 // outputs of a workgroup
+  const int n_out = gated(EPI) ? a.n / 2 : a.n, n0 = blockIdx.x * kCols;
+
+  // this wave's steps of k
+  const int per_wave = steps_a_share(k), first = wave * per_wave;
+  const int n_steps = max(0, min((k + kStepK - 1) / kStepK, first + per_wave) - first);
+  unsigned char* ring = stream_lds + wave * (STAGES * kRing);
+  const unsigned ring_at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)ring));
+
+  // What is added to is asked for now: item j of a thread is output (threadIdx.x + j * kThreads) of the workgroup's.
+  constexpr int kItems = (XR * kCols + kThreads - 1) / kThreads;
+  float prev[kItems], bias[kItems];
+  if constexpr (EPI == kAccum) {
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const int idx = threadIdx.x + j * kThreads, row = idx / kCols, gn = n0 + idx % kCols;
+      const bool live = row < m && gn < n_out;
+      prev[j] = live ? a.out[static_cast<long>(row0 + row) * n_out + gn] : 0.f;
+      bias[j] = live && a.bias != nullptr ? a.bias[gn] : 0.f;
+    }
+  }
+
+  // Lane l of a load brings segment (l % 8) ^ key of the eight rows' row l / 8.  Rows beyond the matrix are read from its
+  // last row (their results are not stored).
+  const float* bases[PER];
+  unsigned offsets[PER], back[PER];                          // (back: from a segment to its row's first one)
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int r = (i < 2 ? i : i - 2) * 8 + lane / 8, seg = (lane % 8) ^ slot_key(r);
+    back[i] = seg * 16;
+    if (i < 2) {                                             // (a load's eight rows of w lie together, from a scalar base)
+      const int from = gated(EPI) ? n0 : min(n0 + i * 8, n_out - 1);
+      const int at = min(gated(EPI) ? n0 + lane / 8 : n0 + r, n_out - 1);
+      bases[i] = a.w + static_cast<long>(from + (gated(EPI) ? i * (a.n / 2) : 0)) * k + first * kStepK;
+      offsets[i] = static_cast<unsigned>(at - from) * k * 4 + seg * 16;
+    } else {
+      bases[i] = a.x + static_cast<long>(row0) * k + first * kStepK;
+      offsets[i] = static_cast<unsigned>(min(r, m - 1)) * k * 4 + seg * 16;
+    }
+  }
+  auto ask = [&](int s) {                                    // step s of this wave's
+    const int k0 = (first + s) * kStepK;
+    const float* b[PER];
+    unsigned o[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      b[i] = bases[i] + s * kStepK;
+      // (a segment beyond the row's end: its row's first, it is not used)
+      o[i] = k0 + kStepK <= k || k0 * 4 + static_cast<int>(back[i]) < k * 4 ? offsets[i] : offsets[i] - back[i];
+    }
+    load_pieces_to_lds<PER>(b, o, ring_at + (s % STAGES) * kRing);
+  };
+
+  floatx4 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s)
+    if (s < n_steps) ask(s);
+
+  for (int s = 0; s < n_steps; ++s) {
+    wait_for_step<PER, STAGES - 1>(min(n_steps - 1, s + STAGES - 1) - s);
+    const unsigned char* at = ring + (s % STAGES) * kRing;
+    const int k0 = (first + s) * kStepK;
+    floatx4 wf[2], xf[MT][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int seg = 4 * h + grp;
+      wf[h] = *reinterpret_cast<const floatx4*>(at + col * kStepBytes + ((seg ^ slot_key(col)) * 16));
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int r = (t * 16 + col) % XR;
+        xf[t][h] = *reinterpret_cast<const floatx4*>(at + 2048 + r * kStepBytes + ((seg ^ slot_key(r)) * 16));
+      }
+      if (k0 + kStepK > k && k0 + seg * 4 >= k) {
+        wf[h] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < MT; ++t) xf[t][h] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    if (s + STAGES < n_steps) {
+      __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));        // the reads are done: their place is filled anew
+      ask(s + STAGES);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[t] = mfma_16x16x4(wf[h][e], xf[t][h][e], acc[t]);
+  }
+
+  __syncthreads();                                           // the rings' place takes the waves' sums
+  typedef float Red[MT][16][kRedPad];
+  Red* red = reinterpret_cast<Red*>(stream_lds);
+  static_assert(sizeof(Red) <= STAGES * kRing, "the sums fit the rings");
+  // acc[t][r] is this wave's share of weight row 4 grp + r and row t * 16 + col
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][t][4 * grp + r][col] = acc[t][r];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    const int idx = threadIdx.x + j * kThreads, nl = idx % kCols, row = idx / kCols, gn = n0 + nl;
+    if (row >= m || gn >= n_out) continue;
+    float sum = 0.f, up = 0.f;
+#pragma unroll
+    for (int v = 0; v < kShares; ++v) sum += red[v][row / 16][nl][row % 16];
+    if constexpr (gated(EPI)) {
+#pragma unroll
+      for (int v = 0; v < kShares; ++v) up += red[v][row / 16][nl + 8][row % 16];
+    }
+    float* to = a.out + static_cast<long>(row0 + row) * n_out + gn;
+    if constexpr (EPI == kAccum) *to = prev[j] + bias[j] + sum;
+    else if constexpr (gated(EPI)) *to = gate_act<EPI>(sum) * up;
+    else *to = sum;
+  }
+}
+
+template <int XR, int STAGES, int EPI>
+int launch_stream_form(const Args& a, hipStream_t s) {
+  auto kernel = gemm_f32_stream_kernel<XR, STAGES, EPI>;
+  constexpr int kLds = kWaves * STAGES * (2 + XR / 8) * 1024;
+  static_assert(kLds <= 160 * 1024, "a workgroup's LDS");
+  static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
+  if (!raised) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+      return fail("gemm_f32: cannot raise the dynamic LDS limit");
+    raised = true;
+  }
+  const int cols = gated(EPI) ? 8 : 16, n_out = gated(EPI) ? a.n / 2 : a.n;
+  kernel<<<dim3((n_out + cols - 1) / cols, (a.m + XR - 1) / XR), kThreads, kLds, s>>>(a);
+  return 0;
+}
+
+template <int EPI>
+int launch_stream(const Args& a, hipStream_t s) {
+  const int cols = gated(EPI) ? 8 : 16, n_out = gated(EPI) ? a.n / 2 : a.n;
+  // One workgroup a CU where there are no more: a ring as deep as LDS allows.  Else two that overlap.
+  const bool few = (n_out + cols - 1) / cols <= compute_units();
+  if (a.m <= 8) return few ? launch_stream_form<8, 6, EPI>(a, s) : launch_stream_form<8, 3, EPI>(a, s);
+  if (a.m <= 16) return few ? launch_stream_form<16, 4, EPI>(a, s) : launch_stream_form<16, 2, EPI>(a, s);
+  return few && a.m <= 32 ? launch_stream_form<32, 3, EPI>(a, s) : launch_stream_form<32, 2, EPI>(a, s);
+}
+
+// ---- many rows ----------------------------------------------------------------------------------
+
+// WM x WN waves of TM x TN blocks of 32 x 32.  Gated: of a wave's blocks of columns the even ones are gate rows of w, the odd
+// ones the up rows of the same outputs, which so meet in the same registers of the same lane.
+template <int WM, int WN, int TM, int TN, int STAGES, int MINWG, int EPI>
+__global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_f32_tiled_kernel(const Args a, int m_blocks, int n_blocks) {
+  constexpr int RA = 32 * TM * WM, RW = 32 * TN * WN, NW = WM * WN, kStage = (RA + RW) * kStepBytes;
+  constexpr int GA = RA / 8, GW = RW / 8, PER = (GA + GW) / NW;              // wave-wide loads a step: eight rows each
+  static_assert((GA + GW) % NW == 0 && (!gated(EPI) || TN % 2 == 0), "whole loads a wave; gates beside ups");
+  constexpr int kOut = gated(EPI) ? RW / 2 : RW;                             // columns of the output tile
+  extern __shared__ __align__(1024) unsigned char tile_lds[];
+  const unsigned lds_at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)tile_lds));
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wm = wave / WN, wn = wave % WN, col = lane % 32, half = lane / 32;
+  const int n_out = gated(EPI) ? a.n / 2 : a.n;
+  int bm, bn;
+  tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
+  const int m0 = bm * RA, n0 = bn * kOut;
+
+  const unsigned char* src[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int g = wave * PER + i, r = (g < GA ? g : g - GA) * 8 + lane / 8, seg = (lane % 8) ^ slot_key(r);
+    long row;
+    if (g < GA) {
+      row = min(m0 + r, a.m - 1);
+    } else if constexpr (gated(EPI)) {
+      const int block = r / 32;                                              // (wave column block / TN, its block block % TN)
+      row = min(n0 + (block / 2) * 32 + r % 32, n_out - 1) + (block % 2 ? n_out : 0);
+    } else {
+      row = min(n0 + r, n_out - 1);
+    }
+    src[i] = reinterpret_cast<const unsigned char*>((g < GA ? a.x : a.w) + row * a.k) + seg * 16;
+  }
+  auto ask = [&](int t) {
+    const unsigned base = lds_at + (t % STAGES) * kStage + wave * PER * 1024;
+    const size_t at = static_cast<size_t>(t) * kStepBytes;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) load_to_lds_16(src[i] + at, __builtin_amdgcn_readfirstlane(base + i * 1024));
+  };
+
+  floatx16 acc[TM][TN], sum[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f, sum[i][j][r] = 0.f;
+  const int n_steps = a.k / kStepK, share = steps_a_share(a.k);
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < n_steps) ask(s);
+
+  int left = share;                                          // steps until the share of k that is being added up ends
+  for (int t = 0; t < n_steps; ++t) {
+    wait_for_step<PER, STAGES - 2>(min(n_steps - 1, t + STAGES - 2) - t);
+    lds_barrier();          // everybody's part of step t is there, and nobody reads step t - 1 any more
+    if (t + STAGES - 1 < n_steps) ask(t + STAGES - 1);
+    const unsigned char* at = tile_lds + (t % STAGES) * kStage;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // segments 4 h + half and 4 h + 2 + half: with the first's element e and then the second's, an output adds up k in the
+      // order of the few rows' kernel, four segments' element 0, then 1 ...
+      floatx4 xf[TM][2], wf[TN][2];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int r = (wm * TM + i) * 32 + col;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) xf[i][p] = *reinterpret_cast<const floatx4*>(at + r * kStepBytes + (((4 * h + 2 * p + half) ^ slot_key(r)) * 16));
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int r = (wn * TN + j) * 32 + col;
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          wf[j][p] = *reinterpret_cast<const floatx4*>(at + RA * kStepBytes + r * kStepBytes + (((4 * h + 2 * p + half) ^ slot_key(r)) * 16));
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xf[i][p][e], wf[j][p][e], acc[i][j], 0, 0, 0);
+    }
+    if (--left == 0) {
+      left = share;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          sum[i][j] += acc[i][j];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        }
+    }
+  }
+  // [i][j][r] is row i 32 + 8 (r / 4) + 4 half + r % 4 and column j 32 + col of the wave's part: a store writes two rows'
+  // 128 bytes
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; j += gated(EPI) ? 2 : 1) {
+      const int gn = n0 + (gated(EPI) ? (wn * TN + j) / 2 : wn * TN + j) * 32 + col;
+      if (gn >= n_out) continue;
+      const float bias = EPI == kAccum && a.bias != nullptr ? a.bias[gn] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int gm = m0 + (wm * TM + i) * 32 + 8 * (r / 4) + 4 * half + r % 4;
+        if (gm >= a.m) continue;
+        float* to = a.out + static_cast<long>(gm) * n_out + gn;
+        const float s = sum[i][j][r] + acc[i][j][r];
+        if constexpr (EPI == kAccum) *to = *to + bias + s;
+        else if constexpr (gated(EPI)) *to = gate_act<EPI>(s) * (sum[i][j + 1][r] + acc[i][j + 1][r]);
+        else *to = s;
+      }
+    }
+}
+
+template <int WM, int WN, int TM, int TN, int STAGES, int MINWG, int EPI>
+int launch_tiled_form(const Args& a, hipStream_t s) {
+  auto kernel = gemm_f32_tiled_kernel<WM, WN, TM, TN, STAGES, MINWG, EPI>;
+  constexpr int RA = 32 * TM * WM, RW = 32 * TN * WN, kLds = STAGES * (RA + RW) * kStepBytes;
+  static_assert(kLds * MINWG <= 160 * 1024, "the workgroups' LDS");
+  static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
+  if (!raised) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+      return fail("gemm_f32: cannot raise the dynamic LDS limit");
+    raised = true;
+  }
+  const int n_out = gated(EPI) ? a.n / 2 : a.n, out = gated(EPI) ? RW / 2 : RW;
+  const int m_blocks = (a.m + RA - 1) / RA, n_blocks = (n_out + out - 1) / out;
+  kernel<<<m_blocks * n_blocks, 64 * WM * WN, kLds, s>>>(a, m_blocks, n_blocks);
+  return 0;
+}
+
+// Which kernel and tile, by what each was measured to take (microseconds, the weights not in a cache; both add up k in the same
+// order, so the choice moves no bit).  The few rows' kernel sustains 52 TFLOP/s once its rows are 32 a workgroup (64 rows x
+// 2,048 x 5,632: 27 us; 64 x 11,264 x 2,048: 58).  The tiled one sustains 115 on all CUs (0.49 a CU's tile at a time) but no tile
+// is faster than its chain of steps, 0.8 us each (65 to 256 rows x 2,048 x 5,632: 140 us whatever the rows, 128 rows x 2,560 x
+// 2,048: 55): for 64 to about 250 rows of a narrow output the first is up to twice as fast, for wide ones and more rows the second.
+constexpr int kTileForms = 3;
+constexpr int kTileForm[kTileForms][2] = {{128, 128}, {64, 128}, {64, 64}};   // rows of x, rows of w
+
+double stream_time(int m, int n, int k) { return 4.0 + 2.0e-6 * ((m + 31) / 32 * 32) * n * k / 52.0; }
+
+int tile_form(int m, int n, int k, double& time) {
+  int best = 0;
+  for (int f = 0; f < kTileForms; ++f) {
+    const long tiles = static_cast<long>((m + kTileForm[f][0] - 1) / kTileForm[f][0]) * ((n + kTileForm[f][1] - 1) / kTileForm[f][1]);
+    const long turns = (tiles + compute_units() - 1) / compute_units();
+    const double work = turns * 2.0e-6 * kTileForm[f][0] * kTileForm[f][1] * k * (1.0 + 0.05 * f) / 0.49;
+    const double chain = 5.0 + 0.8 * (k / kStepK), t = work > chain ? work : chain;
+    if (f == 0 || t < time) best = f, time = t;
+  }
+  return best;
+}
+
+template <int EPI>
+int launch_tiled(const Args& a, int form, hipStream_t s) {
+  switch (form) {
+    case 0: return launch_tiled_form<2, 2, 2, 2, 2, 2, EPI>(a, s);
+    case 1: return launch_tiled_form<2, 2, 1, 2, 3, 2, EPI>(a, s);
+    default:
+      if constexpr (gated(EPI)) return launch_tiled_form<2, 1, 1, 2, 3, 3, EPI>(a, s);
+      else return launch_tiled_form<2, 2, 1, 1, 3, 3, EPI>(a, s);
+  }
+}
+
+template <int EPI>
+int launch(const Args& a, hipStream_t s) {
+  if (a.m <= 64 || a.k % kStepK != 0) return launch_stream<EPI>(a, s);
+  double tiled;
+  const int form = tile_form(a.m, a.n, a.k, tiled);
+  return stream_time(a.m, a.n, a.k) < tiled ? launch_stream<EPI>(a, s) : launch_tiled<EPI>(a, form, s);
+}
+
+}  // namespace
+}  // namespace bc4g
+
+using namespace bc4g;
+
+extern "C" int bc4g_gemm_f32(const float* x, const float* w, const float* bias, float* out, int epilogue, int m, int n, int k, void* stream) {
+  BC4G_REQUIRE(m >= 0 && n > 0 && k > 0 && k % 4 == 0 && k <= (1 << 24), "gemm_f32: bad sizes M=%d N=%d K=%d (K a multiple of 4)", m, n, k);
+  BC4G_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0, "gemm_f32: operands must lie on 16-byte boundaries");
+  BC4G_REQUIRE((m + 31L) / 32 <= 65535 && ((m + 63L) / 64) * ((n + 31L) / 32) <= 2147483647L, "gemm_f32: M=%d N=%d are beyond the grid limit", m, n);
+  BC4G_REQUIRE(!bias || epilogue == kAccum, "gemm_f32: only an adding product takes a bias");
+  BC4G_REQUIRE(!gated(epilogue) || n % 2 == 0, "gemm_f32: a gated product has as many gate rows as up rows (N=%d)", n);
+  if (m == 0) return 0;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const Args a{x, w, bias, out, m, n, k};
+  int e = 0;
+  switch (epilogue) {
+    case kStore: e = launch<kStore>(a, s); break;
+    case kAccum: e = launch<kAccum>(a, s); break;
+    case kSwiglu: e = launch<kSwiglu>(a, s); break;
+    case kGeglu: e = launch<kGeglu>(a, s); break;
+    default: return fail("gemm_f32: unknown epilogue %d", epilogue);
+  }
+  if (e) return e;
+  return check_launch("gemm_f32");
+}

@@ -1,13 +1,12 @@
 // out[m, n] (+)= sum_k a[m, k] * w[n, k] for any sizes and any mix of float and
-// bfloat16 operands, in plain float FMA (no matrix cores): the matrix product
-// of the 32-bit path, and the fallback where the MFMA kernels refuse a size.
+// bfloat16 operands, in plain float FMA (no matrix cores): what the matrix-core
+// kernels refuse (mixed operands, k no multiple of 4 or 8, odd addresses).
 //
 // Each output element is the sum over k in ascending order in one thread, so
 // a row's result does not depend on how many rows the call has -- nor on which of the
 // two tile sizes below serves the call: 64 x 64 outputs a block (four by four a thread),
 // or, for up to 16 rows (a decode step), 16 x 16 (one a thread, k staged 64 at a time),
-// which brings sixteen times the blocks to stream the weights of a product with few rows
-// (a decode step of the 32-bit path at TinyLlama's sizes: 43 ms with the large tile alone).
+// which brings sixteen times the blocks to stream the weights of a product with few rows.
 #include "api.h"
 #include "common.h"
 

@@ -240,6 +240,38 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = None
     return out
 
 
+F32_STORE, F32_ACCUM = 0, 1
+F32_GATED = {"silu": 2, "gelu_tanh": 3}       # epilogues of the float32 matrix-core product
+
+
+def gemm_f32(x: torch.Tensor, w, accumulate_into: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
+             act: Optional[str] = None) -> Optional[torch.Tensor]:
+    """x [M, K] times w [N, K] transposed, float32 operands and sums on the matrix cores, where the kernels take them (k a
+    multiple of 4, operands on 16-byte boundaries), else None (the caller then uses the plain float kernel).
+    ``accumulate_into`` and ``bias`` as in gemm_generic.  ``act`` ("silu" or "gelu_tanh"): w is gate rows followed by as many
+    up rows, and the result is act(gate) * up, [M, N / 2]."""
+    if (x.dtype != torch.float32 or w.dtype != torch.float32 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]
+            or x.shape[1] % 4 or not 0 < x.shape[0] <= 32 * 65535 or (act is not None and w.shape[0] % 2)):
+        return None
+    w = _rows(w)
+    if x.data_ptr() % 16 or w.data_ptr() % 16:
+        return None
+    _dev("gemm", x, w, accumulate_into, bias)
+    _check_bias("gemm", bias, w.shape[0], accumulate_into)
+    m, k = x.shape
+    n = w.shape[0]
+    if accumulate_into is not None:
+        out, epi = accumulate_into, F32_ACCUM
+        if out.dtype != torch.float32 or tuple(out.shape) != (m, n):
+            raise KernelError(f"gemm: accumulate_into must be float32 [{m}, {n}], got {out.dtype} {tuple(out.shape)}")
+    else:
+        epi = F32_GATED[act] if act is not None else F32_STORE
+        out = torch.empty((m, n // 2 if act is not None else n), dtype=torch.float32, device=x.device)
+    library.call("bc4g_gemm_f32", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), epi, m, n, k, _stream(),
+                 cost=_gemm_cost(m, n, k, 4, 4, 8 if accumulate_into is not None else 4.0 * out.shape[1] / n))
+    return out
+
+
 def _check_bias(what: str, bias: Optional[torch.Tensor], n: int, accumulate_into: Optional[torch.Tensor]) -> None:
     if bias is not None and (accumulate_into is None or bias.dtype != torch.float32 or tuple(bias.shape) != (n,)):
         raise KernelError(f"{what}: a bias is float32 [{n}] and joins a product that is added to something, got {bias.dtype} {tuple(bias.shape)}")
@@ -771,6 +803,8 @@ def gemm_swiglu(a: torch.Tensor, w_gate_up, interleaved: bool = False, act: str 
         else:
             library.call("bc4g_gemm_mfma", _ptr(a), *_tiled_weight(rows, packed, a), _ptr(out), None, gated_epilogue(act), m, n, k, _stream(),
                          cost=_tiled_cost(m, n, k, 1))
+        return out
+    if not interleaved and (out := gemm_f32(a, w_gate_up, act=act)) is not None:
         return out
     gu = gemm_fast(a, w_gate_up, a.dtype)
     if gu is None:

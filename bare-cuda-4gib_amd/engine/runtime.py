@@ -29,8 +29,8 @@ class Runtime:
     """device: where tensors live.  act_dtype: the storage type of activations
     between kernels and of the cache -- bfloat16 (what serving uses; float
     accumulation everywhere, float residual stream and logits) or float32 (a
-    true 32-bit path: every weight widened to float, plain float arithmetic, no
-    matrix-core mode of reduced precision)."""
+    true 32-bit path: every weight widened to float, float32 operands and sums
+    throughout, no matrix-core mode of reduced precision)."""
     device: torch.device
     act_dtype: torch.dtype
 

@@ -3,7 +3,8 @@ a linear layer in; reference: engine/include/llm/kernels.h:48-57), and the
 choice of kernel for it (reference: matmul dispatch, engine/src/model.cpp:153-192):
 up to 64 rows the weight-streaming kernel (with RMSNorm fused in up to 16 rows),
 beyond that the tiled matrix-core kernel, and the plain float kernel for
-everything those refuse (float32 operands, k no multiple of 8)."""
+what those refuse (k no multiple of 8).  Float32 operands go to the
+float32 matrix-core kernel where it takes them, else to the plain one."""
 from __future__ import annotations
 
 from typing import Optional, Union
@@ -67,6 +68,8 @@ def linear(x: Union[torch.Tensor, Normed], w, out_dtype: Optional[torch.dtype] =
             ctx.handoff.leave(norm, ops.gemm_accumulate_emit(x, w, accumulate_into, scale[0], scale[1], bias=bias))
             return accumulate_into
     fast = ops.gemm_fast(x, w, out_dtype, accumulate_into, bias=bias)
+    if fast is None and out_dtype in (None, torch.float32):
+        fast = ops.gemm_f32(x, w, accumulate_into, bias=bias)
     if fast is not None:
         return fast
     return ops.gemm_generic(x, w, out_dtype, accumulate_into, bias=bias)
