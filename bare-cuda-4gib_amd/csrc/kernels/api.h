@@ -104,6 +104,12 @@ int bc4g_attention_generic(const void* qkv, int q_stride, void* out, int dtype, 
                            const int32_t* row_seq, const int32_t* positions, int n_tokens,
                            int n_heads, int n_kv_heads, int head_dim, int page_tokens,
                            int num_pages, int window, float scale, void* stream);
+// The same over a float32 cache on the matrix cores: request s's rows are seq_start[s] .. seq_start[s + 1] - 1 at positions
+// seq_ctx[s] ...; most_rows: the most any request brings; few != 0: some request brings no more than 16 rows times query heads a
+// key/value head.  head_dim a multiple of 16 up to 128, page_tokens one of 4, every tensor on a 16-byte boundary.
+int bc4g_attention_f32(const float* q, int q_stride, float* out, const float* k_cache, const float* v_cache, const int32_t* block_table,
+                       int table_stride, const int32_t* seq_start, const int32_t* seq_ctx, int n_seqs, int most_rows, int few,
+                       int n_heads, int n_kv_heads, int head_dim, int page_tokens, int window, float scale, void* stream);
 
 // out[r] = lowest index of the row's maximum                      (logits_argmax.cu:22-65)
 // part_v, part_i: scratch [n_rows, 64] each (the best of every slice of a row).

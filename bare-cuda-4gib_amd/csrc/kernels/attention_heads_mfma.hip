@@ -63,24 +63,6 @@ __device__ inline void split_three(const float (&x)[8], uint4 (&part)[3]) {
   }
 }
 
-// maximum / sum of a value over the four lanes l, l ^ 16, l ^ 32, l ^ 48, in every lane
-__device__ inline float four_lanes_max(float x) {
-  const unsigned u = __float_as_uint(x);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const unsigned v = __float_as_uint(y);
-  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ inline float four_lanes_sum(float x) {
-  const unsigned u = __float_as_uint(x);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const unsigned v = __float_as_uint(y);
-  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // DS: 32-wide steps of the keys' dimensions (dim <= 32 DS), EB: blocks of 16 values (vdim <= 16 EB), KT: keys of a tile.
 template <int DS, int EB, int KT>
 __global__ __launch_bounds__(kThreads, (DS <= 4 && EB <= 4) || (DS <= 2 && EB <= 8) ? 3 : 2) void attention_heads_mfma_kernel(const HeadsArgs a) {

@@ -53,8 +53,6 @@ struct Args {
 constexpr int kShares = 8;
 __host__ __device__ inline int steps_a_share(int k) { return ((k + kStepK - 1) / kStepK + kShares - 1) / kShares; }
 
-__device__ inline floatx4 mfma_16x16x4(float a, float b, floatx4 acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
-
 // Where 16-byte segment s of row r of a step lies in the row's 128 bytes of LDS: s ^ key(r), so that the 16 rows' reads of one
 // segment (two rows share the 64 banks' span) meet different banks.
 __device__ inline int slot_key(int row) { return (row >> 1) & 7; }

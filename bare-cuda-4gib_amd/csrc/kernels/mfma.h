@@ -26,6 +26,28 @@ __device__ inline floatx16 mfma_32x32x16(uint4 a, uint4 b, floatx16 acc) {
                                                  acc, 0, 0, 0);
 }
 
+// D[16x16] += A[16x4] * B[4x16], float operands, products and sums.  Lane l holds, of A, row l%16 and k-slot l/16; of B, column
+// l%16 and that slot; D as in mfma_16x16x32.
+__device__ inline floatx4 mfma_16x16x4(float a, float b, floatx4 acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
+
+// maximum / sum of a value over the four lanes l, l ^ 16, l ^ 32, l ^ 48, in every lane
+__device__ inline float four_lanes_max(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const unsigned v = __float_as_uint(y);
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ inline float four_lanes_sum(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const unsigned v = __float_as_uint(y);
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 // x / (1 + e^-x) for the bfloat16 products' SwiGLU epilogues, by the hardware's 2^x and reciprocal (each good to a unit
 // in the last place of a float; the result is rounded to bfloat16).  expf and a true division are an eighth of the
 // tiled kernel's epilogue, and that a sixth of a wide gate-up product's time.

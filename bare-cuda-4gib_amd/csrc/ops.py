@@ -422,6 +422,36 @@ def attention_generic(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
     return out
 
 
+ATTENTION_F32_FEW_ROWS = 16         # rows times query heads a key/value head that one wave of the float32 kernel holds
+
+
+def attention_f32_takes(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, head_dim: int) -> bool:
+    """Whether the float32 matrix-core kernel takes a plain attention call: a float32 cache in pages of a multiple of 4
+    tokens, a head size of a multiple of 16 up to 128, everything on 16-byte boundaries."""
+    return (q.dtype == torch.float32 and k_cache.dtype == torch.float32 and head_dim % 16 == 0 and 0 < head_dim <= 128
+            and k_cache.shape[2] % 4 == 0 and q.shape[1] % 4 == 0
+            and not any(t.data_ptr() % 16 for t in (q, k_cache, v_cache)))
+
+
+def attention_f32(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor, ctx,
+                  n_heads: int, n_kv_heads: int, head_dim: int, window: int, scale: float, work=None) -> torch.Tensor:
+    """attention_generic for the rows of a step's context where attention_f32_takes it."""
+    _dev("attention", qkv, k_cache, v_cache, block_table, ctx.seq_start_dev, ctx.seq_ctx_dev)
+    _check_queries("attention", qkv, n_heads, n_kv_heads, head_dim)
+    _check_cache("attention", k_cache, v_cache, n_kv_heads, head_dim, qkv.dtype)
+    if block_table.dim() != 2 or block_table.dtype != torch.int32:
+        raise KernelError("attention: block_table must be int32 [requests, pages]")
+    _i32("attention", "seq_start", ctx.seq_start_dev, ctx.n_seqs + 1)
+    _i32("attention", "seq_ctx", ctx.seq_ctx_dev, ctx.n_seqs)
+    group = n_heads // n_kv_heads
+    few = any((b - a) * group <= ATTENTION_F32_FEW_ROWS for a, b in zip(ctx.seq_start, ctx.seq_start[1:]))
+    out = torch.empty((qkv.shape[0], n_heads * head_dim), dtype=qkv.dtype, device=qkv.device)
+    library.call("bc4g_attention_f32", _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(k_cache), _ptr(v_cache), _ptr(block_table),
+                 block_table.shape[1], _ptr(ctx.seq_start_dev), _ptr(ctx.seq_ctx_dev), ctx.n_seqs, ctx.max_q_len, 1 if few else 0,
+                 n_heads, n_kv_heads, head_dim, k_cache.shape[2], int(window), float(scale), _stream(), cost=work)
+    return out
+
+
 def argmax(logits: torch.Tensor) -> torch.Tensor:
     """Lowest index of each row's maximum, int32 [rows]."""
     _dev("argmax", logits)
@@ -1239,8 +1269,8 @@ def attention_plan(batch, n_heads: int, n_kv_heads: int, head_dim: int, window: 
 def attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
               ctx, plan, n_heads: int, n_kv_heads: int, head_dim: int, window: int, scale: float) -> torch.Tensor:
     """Attention of a step's rows over the cache: the matrix-core kernel where it takes the
-    sizes (bfloat16, head size a multiple of 16 up to 256, pages of a multiple of 16 tokens),
-    else the plain float kernel.  ``plan``: (device arrays, notes) of attention_plan() for this
+    sizes (bfloat16, head size a multiple of 16 up to 256, pages of a multiple of 16 tokens; or
+    float32, see attention_f32_takes), else the plain float kernel.  ``plan``: (device arrays, notes) of attention_plan() for this
     batch.  The number of parts the keys are cut into follows from ctx.max_kv_len: in a captured
     step that is the bound of the graph's context bucket, so the choice holds for every replay."""
     work = lambda: attention_work(ctx, n_heads, n_kv_heads, head_dim, window, qkv.element_size())
@@ -1271,6 +1301,8 @@ def attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
             attention_mfma(*args, arrays["short_tiles"], notes["n_short"], *sizes, n_splits, 1, 1, out=out,
                            row_seq=ctx.row_seq)
         return out
+    if ctx.n_seqs <= 65535 and attention_f32_takes(qkv, k_cache, v_cache, head_dim):
+        return attention_f32(qkv, k_cache, v_cache, block_table, ctx, n_heads, n_kv_heads, head_dim, window, scale, work=work)
     return attention_generic(qkv, k_cache, v_cache, block_table, ctx.row_seq, ctx.positions,
                              n_heads, n_kv_heads, head_dim, window, scale, work=work)
 
