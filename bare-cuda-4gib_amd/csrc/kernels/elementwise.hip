@@ -1,5 +1,5 @@
-// Embedding gather, RMSNorm, SwiGLU, rotary positions + cache write, argmax
-// and sampling.  One instantiation per storage type; all arithmetic in float.
+// Embedding gather, RMSNorm, SwiGLU, rotary positions + cache write and
+// argmax.  One instantiation per storage type; all arithmetic in float.
 #include <float.h>
 #include <math.h>
 
@@ -456,186 +456,6 @@ __global__ void argmax_pick_kernel(const float* __restrict__ part_v, const int32
   if (threadIdx.x == 0) out[blockIdx.x] = idx < vocab ? idx : 0;
 }
 
-// ---- temperature sampling --------------------------------------------------
-// The law: weights w_i = exp((l_i - max) / T) in float, summed in double; the token is the first i,
-// in vocabulary order, at which u * total - (w_0 + ... + w_i) turns negative.  One workgroup a row.
-// The vocabulary is cut into groups of 512 consecutive tokens, a lane holding eight in a row (more
-// beyond 2,097,152 tokens, so that the groups' sums fit LDS): a lane sums its own tokens in order
-// without a word to its neighbours (sums of doubles across lanes go through the LDS crossbar, which
-// sixteen waves share), a wave then a group; every pass over the row reads whole cache lines.  The
-// groups' sums, a running sum over them (one wave, 64 groups a step) and a last look inside the one
-// group where the target is crossed find the token.
-// (Sums in another order than the host's one-by-one walk: a boundary may move by one token when u
-// falls within rounding of it.)
-constexpr int kSampleThreads = 1024;
-constexpr int kSampleMaxGroups = 4096;
-constexpr int kSamplePerLane = 8;           // consecutive tokens a lane holds of a group
-constexpr int kSampleAhead = 4;             // loads of 16 bytes (pairs of them in the second pass) a thread has in flight
-
-__device__ inline double wave_sum_f64(double v) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
-}
-// inclusive running sum over the wave's lanes, in lane order
-__device__ inline double wave_scan_f64(double v, int lane) {
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const double up = __shfl_up(v, off, kWave);
-    if (lane >= off) v += up;
-  }
-  return v;
-}
-
-__global__ __launch_bounds__(kSampleThreads) void sample_kernel(const float* __restrict__ logits,
-                                                               const float* __restrict__ temperature,
-                                                               const double* __restrict__ u, int32_t* __restrict__ out,
-                                                               int vocab) {
-  __shared__ double group_sum[kSampleMaxGroups];      // then: the running sum up to and with each group
-  constexpr int kWaves = kSampleThreads / kWave;
-  __shared__ float best_v[kWaves];
-  __shared__ int best_i[kWaves];
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const float* row = logits + static_cast<size_t>(blockIdx.x) * vocab;
-
-  // the maximum and where it stands first
-  float v = -FLT_MAX;
-  int idx = vocab;
-  // in fours where every row starts on 16 bytes (the base does and the vocabulary is a multiple of four): no group of
-  // four then straddles a row's end
-  const bool by_four = vocab % 4 == 0 && reinterpret_cast<uintptr_t>(logits) % 16 == 0;
-  if (by_four) {
-    const float4* row4 = reinterpret_cast<const float4*>(row);
-    const int n4 = vocab / 4;
-    for (int at = threadIdx.x; at < n4; at += kSampleAhead * kSampleThreads) {
-      float4 t[kSampleAhead];               // the loads first, so that they are in flight together
-#pragma unroll
-      for (int j = 0; j < kSampleAhead; ++j) {
-        const int i4 = at + j * kSampleThreads;
-        t[j] = i4 < n4 ? row4[i4] : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-#pragma unroll
-      for (int j = 0; j < kSampleAhead; ++j) {
-        const int i4 = at + j * kSampleThreads;
-        if (i4 < n4) {
-          better(v, idx, t[j].x, 4 * i4);
-          better(v, idx, t[j].y, 4 * i4 + 1);
-          better(v, idx, t[j].z, 4 * i4 + 2);
-          better(v, idx, t[j].w, 4 * i4 + 3);
-        }
-      }
-    }
-  } else {
-    for (int at = threadIdx.x; at < vocab; at += kSampleThreads) better(v, idx, row[at], at);
-  }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) better(v, idx, __shfl_xor(v, off, kWave), __shfl_xor(idx, off, kWave));
-  if (lane == 0) {
-    best_v[wave] = v;
-    best_i[wave] = idx;
-  }
-  __syncthreads();
-  float row_max = best_v[0];
-  int best = best_i[0];
-  for (int w = 1; w < kWaves; ++w) better(row_max, best, best_v[w], best_i[w]);
-  const int arg = best < vocab ? best : 0;
-  const float temp = temperature[blockIdx.x];
-  if (!(temp > 0.f)) {
-    if (threadIdx.x == 0) out[blockIdx.x] = arg;
-    return;
-  }
-  const float inv_t = 1.0f / temp;
-  const int per_lane = max(kSamplePerLane, (vocab + kWave * kSampleMaxGroups - 1) / (kWave * kSampleMaxGroups));
-  const int group_size = kWave * per_lane;
-  const int n_groups = (vocab + group_size - 1) / group_size;
-  auto lane_weight_sum = [&](int g) {      // this lane's tokens of group g, in order
-    double s = 0.0;
-    const int first = g * group_size + lane * per_lane;
-    for (int j = 0; j < per_lane; ++j) {
-      const int i = first + j;
-      if (i < vocab) s += static_cast<double>(expf((row[i] - row_max) * inv_t));
-    }
-    return s;
-  };
-  if (by_four && per_lane == kSamplePerLane) {        // a wave's groups at once: their loads are in flight together
-    static_assert(kSamplePerLane == 8, "two loads of four a lane");
-    for (int g0 = wave; g0 < n_groups; g0 += kWaves * kSampleAhead) {
-      float4 t[kSampleAhead][2];
-#pragma unroll
-      for (int j = 0; j < kSampleAhead; ++j) {
-        const int first = (g0 + j * kWaves) * group_size + lane * kSamplePerLane;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          t[j][h] = first + 4 * h < vocab ? *reinterpret_cast<const float4*>(row + first + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-#pragma unroll
-      for (int j = 0; j < kSampleAhead; ++j) {
-        const int g = g0 + j * kWaves;
-        const int first = g * group_size + lane * kSamplePerLane;
-        double s = 0.0;                     // the order of lane_weight_sum: the look inside a group sums the same
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (first + 4 * h < vocab) {
-            s += static_cast<double>(expf((t[j][h].x - row_max) * inv_t));
-            s += static_cast<double>(expf((t[j][h].y - row_max) * inv_t));
-            s += static_cast<double>(expf((t[j][h].z - row_max) * inv_t));
-            s += static_cast<double>(expf((t[j][h].w - row_max) * inv_t));
-          }
-        }
-        s = wave_sum_f64(s);
-        if (lane == 0 && g < n_groups) group_sum[g] = s;
-      }
-    }
-  } else {
-    for (int g = wave; g < n_groups; g += kWaves) {
-      const double s = wave_sum_f64(lane_weight_sum(g));
-      if (lane == 0) group_sum[g] = s;
-    }
-  }
-  __syncthreads();
-  if (wave != 0) return;
-
-  // one wave: running sums over the groups, 64 at a step; then the first group they cross the target in
-  double carry = 0.0;
-  for (int c = 0; c < n_groups; c += kWave) {
-    const int g = c + lane;
-    const double incl = carry + wave_scan_f64(g < n_groups ? group_sum[g] : 0.0, lane);
-    if (g < n_groups) group_sum[g] = incl;
-    carry = __shfl(incl, kWave - 1, kWave);
-  }
-  const double target = u[blockIdx.x] * carry;
-  int found = n_groups;
-  for (int c = 0; c < n_groups && found == n_groups; c += kWave) {
-    const int g = c + lane;
-    const unsigned long long over = __ballot(g < n_groups && target - group_sum[g] < 0.0);
-    if (over != 0ull) found = c + __ffsll(static_cast<long long>(over)) - 1;
-  }
-  int result = arg;        // rounding may leave the target a hair above zero after the last token
-  if (found < n_groups) {
-    const double before = found > 0 ? group_sum[found - 1] : 0.0;
-    const double mine = lane_weight_sum(found);
-    const double upto = before + wave_scan_f64(mine, lane);              // with this lane's tokens
-    const unsigned long long over = __ballot(target - upto < 0.0);
-    if (over != 0ull) {
-      const int at = __ffsll(static_cast<long long>(over)) - 1;          // the lane whose tokens cross it
-      double left = target - (upto - mine);
-      const int first = found * group_size + lane * per_lane;
-      int hit = min(vocab - 1, first + per_lane - 1);
-      for (int j = 0; j < per_lane; ++j) {
-        const int i = first + j;
-        if (i >= vocab) break;
-        left -= static_cast<double>(expf((row[i] - row_max) * inv_t));
-        if (left < 0.0) {
-          hit = i;
-          break;
-        }
-      }
-      result = __shfl(hit, at, kWave);
-    }
-  }
-  if (lane == 0) out[blockIdx.x] = result;
-}
-
 int grid_for(long total) {
   long g = (total + kBlock - 1) / kBlock;
   if (g < 1) g = 1;
@@ -913,12 +733,4 @@ extern "C" int bc4g_argmax_static(const float* logits, int32_t* out, int n_rows,
   if (int e = check_launch("argmax_slices")) return e;
   argmax_pick_kernel<<<n_rows, kWave, 0, s>>>(part_v, part_i, out, vocab);
   return check_launch("argmax_pick");
-}
-
-extern "C" int bc4g_sample(const float* logits, const float* temperature, const double* u, int32_t* out,
-                           int n_rows, int vocab, void* stream) {
-  BC4G_REQUIRE(n_rows >= 0 && vocab > 0, "sample: bad sizes rows=%d V=%d", n_rows, vocab);
-  if (n_rows == 0) return 0;
-  sample_kernel<<<n_rows, kSampleThreads, 0, static_cast<hipStream_t>(stream)>>>(logits, temperature, u, out, vocab);
-  return check_launch("sample");
 }

@@ -1,30 +1,28 @@
-// Top-k / top-p sampling on the device, one workgroup a row.
+// Choosing tokens on the device, one workgroup of 16 waves a row of logits: greedy, by temperature, and by top-k / top-p.
 //
-// The law (the reference's, engine/src/sampler.cpp:63-104): weights w_i = exp((l_i - max) / T) in float; the
+// The law with filters (the reference's, engine/src/sampler.cpp:63-104): weights w_i = exp((l_i - max) / T) in float; the
 // tokens in the order of falling weight, lower id first among equal weights; the k likeliest are kept; of
 // those, the fewest whose running sum reaches top_p times their total; the token drawn is the first of the
 // kept ones at which u times their total minus the running sum turns negative.
 //
-// No sort.  A float weight's bit pattern rises with its value, so each of the three questions -- where does
+// No sort of the row.  A float weight's bit pattern rises with its value, so each of the three questions -- where does
 // the count reach k, where does the running sum reach top_p of the total, where does it pass u of the kept
-// mass -- is a walk down the patterns' digits: a histogram over the top 8 bits (the exponent) of the tokens
-// in question, the bucket in which the answer lies, then the next 8 bits of that bucket's tokens, and so on
-// over four levels to one exact pattern; tokens that share it are told apart by id.  A bucket's mass is kept
-// as the integer sum of its tokens' mantissas (below the exponent level all tokens of a bucket share the
-// exponent, and at that level a bucket is an exponent), added with integer atomics: exact, and the same in
-// every run whatever order the adds arrive in.  The sums over buckets are doubles added from the top down in a
-// fixed order.  (Sums in another order than the host's one-by-one walk over a sorted list: a boundary may move
-// by one token when u falls within rounding of it.)
+// mass -- is a search in a histogram over the patterns' leading bits, 64 buckets an octave: the bucket in which the answer
+// lies, and then the bucket's tokens put in order (each counts the keys before its own) with a running sum over them.
+// Where the first question's bucket and those above it hold up to 512 tokens -- a model's peaked rows, every small top-k --
+// these are put in order at once and answer all three.  A bucket's mass is kept as the integer sum of its tokens' mantissas
+// (they share the exponent), added with integer atomics: exact, and the same in every run whatever order the adds arrive in.
+// Rows whose answers lie in a bucket of more tokens than that, or below 2^-32 of the likeliest, go by walks down the patterns'
+// digits: a histogram over the top 8 bits (the exponent) of the tokens in question, the bucket in which the answer lies, then the
+// next 8 bits of that bucket's tokens, and so on over four levels to one exact pattern; tokens that share it are told apart by id.
+// The sums over buckets are doubles.  (Sums in another order than the host's one-by-one walk over a sorted list: a boundary may
+// move by one token when u falls within rounding of it.)
 //
-// A CU takes 64 lanes' instructions a clock, so what a row costs is the number of passes over its tokens times
-// the instructions a token takes in each.  A first look at the exponents alone tells in which bucket the first
-// question's answer lies; the tokens from that bucket up -- for a model's peaked rows a few dozen -- are copied,
-// in the order of their ids, into a list in LDS (up to 18,432), and every walk runs over the list: three passes
-// over the row (the maximum, the look, the list).  A flatter row's walks go over all its tokens, their patterns
-// kept in LDS where the vocabulary fits (up to 36,864 tokens) and worked out again from the logits where not.
-// (64 rows of 32,000 tokens: 50-64 us; of 128,256: 125-140 us, and 490 where rows are so flat that no list holds
-// their candidates.  Rows run beside each other, a CU each.  On the host the same takes a download and a sort of
-// the vocabulary for every row, milliseconds each, and holds the next step back until it is done.)
+// A CU takes 64 lanes' instructions a clock, so what a row costs is the number of passes over its tokens times the instructions a
+// token takes in each, and the barriers between them: a vocabulary of up to 32,768 is read once and its patterns stay in LDS.
+// 64 rows of 32,000 tokens, a mixture of limits, two in five of them flat: 26 us, 32 with the rows that have none beside them in one launch (before,
+// with walks for every question and every row's candidates listed in the order of their ids: 73, and 16 for the others' launch);
+// of 128,256: 73, flat rows 100 (130 and 450).
 #include <float.h>
 #include <math.h>
 
@@ -39,8 +37,8 @@ namespace {
 constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kBuckets = 256;
-constexpr int kMaxCached = 36864;            // tokens whose patterns fit LDS beside the histogram (144 KB)
-constexpr int kMaxListed = kMaxCached / 2;   // ... or this many (pattern, id) pairs
+constexpr int kMaxHeld = 32768;              // tokens whose patterns go into LDS when they are first read (128 KB)
+constexpr int kRoom = kMaxHeld + 4096;       // 32-bit words of LDS a row has: the patterns, and beside them the buckets' sums or the sorted tokens
 // A bucket's count rides in the top bits of its mantissa sum, one atomic add for both, where the vocabulary
 // leaves room: 2^19 tokens of 24-bit mantissas sum to less than 2^43.
 constexpr int kCountShift = 44;
@@ -59,6 +57,8 @@ struct Shared {
   unsigned int cnt[kBuckets];
   unsigned long long msum[kBuckets];
   float red_v[kWaves];
+  double red_d[kWaves];
+  unsigned int red_u[kWaves];
   __align__(16) int wave_cnt[kWaves];
   // a walk's state: the wave that walks a level's buckets writes it between barriers, all read it after
   unsigned int prefix;         // the digits settled so far
@@ -71,6 +71,12 @@ struct Shared {
   long long res_bits;
   int res_ties;
   int res_count;
+  int listed;                  // tokens gathered
+  int first_ge, first_gt;      // places found in the sorted tokens
+  int bucket;                  // a question's answer among the fine buckets: which, what lies above it, how many tokens it holds
+  unsigned int bucket_above;
+  double bucket_mass;
+  int bucket_count;
   int alone_level;             // (>= 0: the answer is the one token of the bucket settled at this level; its pattern is looked up)
   int hit;
 };
@@ -108,47 +114,45 @@ __device__ int ties_needed(int mode, unsigned int k, double target, unsigned int
   return r < 1 ? 1 : r > c ? c : r;
 }
 
-// The tokens a walk looks at: the whole row -- patterns from LDS or from the logits -- or a list of some of them.
-struct Row {
+// A row's tokens, their patterns from LDS or worked out from the logits.  each(f): f(pattern, id) for every token that is this
+// thread's.
+struct Cached {
+  const unsigned int* bits;
+  int n;
+  __device__ unsigned int at(int i) const { return bits[i]; }
+  template <typename F>
+  __device__ inline void each(F f) const {
+    for (int base = 4 * threadIdx.x; base < n; base += 4 * kThreads) {
+      const uint4 four = *reinterpret_cast<const uint4*>(bits + base);
+      const unsigned int b[4] = {four.x, four.y, four.z, four.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (base + e < n) f(b[e], base + e);
+    }
+  }
+};
+struct Logits {
   const float* logits;
-  const unsigned int* cached;    // the patterns of all tokens in LDS (null: worked out from the logits)
-  const unsigned int* listed;    // (not null: the patterns of the n listed tokens, ids rising, and
-  const int* listed_id;          //  their ids)
   int n;
   float row_max, inv_t;
-  __device__ unsigned int bits_at(int i) const {
-    if (listed) return listed[i];
-    return cached ? cached[i] : __float_as_uint(expf((logits[i] - row_max) * inv_t));
-  }
-  __device__ int id_at(int i) const { return listed ? listed_id[i] : i; }
-};
-
-// f(pattern, index) for every token of the row that is this thread's (every kThreads-th).  From the logits, eight
-// loads are on their way together: a load from memory takes hundreds of clocks, and four waves a SIMD hide few.
-template <typename F>
-__device__ inline void each_token(const Row& row, F f) {
-  constexpr int kAhead = 8;
-  if (row.listed || row.cached) {
-    const unsigned int* from = row.listed ? row.listed : row.cached;
-    for (int base = threadIdx.x; base < row.n; base += kAhead * kThreads) {
-      unsigned int b[kAhead];
+  __device__ unsigned int bits_of(float l) const { return __float_as_uint(expf((l - row_max) * inv_t)); }
+  __device__ unsigned int at(int i) const { return bits_of(logits[i]); }
+  template <typename F>
+  __device__ inline void each(F f) const {
+    // (eight loads are on their way together: a load from memory takes hundreds of clocks, and four waves a SIMD hide few)
+    constexpr int kAhead = 8;
+    for (int base = threadIdx.x; base < n; base += kAhead * kThreads) {
+      float l[kAhead];
 #pragma unroll
-      for (int j = 0; j < kAhead; ++j) b[j] = base + j * kThreads < row.n ? from[base + j * kThreads] : 0u;
+      for (int j = 0; j < kAhead; ++j) l[j] = base + j * kThreads < n ? logits[base + j * kThreads] : 0.f;
 #pragma unroll
       for (int j = 0; j < kAhead; ++j)
-        if (base + j * kThreads < row.n) f(b[j], base + j * kThreads);
+        if (base + j * kThreads < n) f(bits_of(l[j]), base + j * kThreads);
     }
-    return;
   }
-  for (int base = threadIdx.x; base < row.n; base += kAhead * kThreads) {
-    float l[kAhead];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) l[j] = base + j * kThreads < row.n ? row.logits[base + j * kThreads] : 0.f;
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j)
-      if (base + j * kThreads < row.n) f(__float_as_uint(expf((l[j] - row.row_max) * row.inv_t)), base + j * kThreads);
-  }
-}
+};
+
+constexpr int kHeldTurns = kMaxHeld / (4 * kThreads);
 
 __device__ inline unsigned int wave_scan_u32(unsigned int v, int lane) {
 #pragma unroll
@@ -171,20 +175,20 @@ __device__ inline double wave_scan_f64(double v, int lane) {
 // count of k tokens, or a running sum that reaches (kByMassGe) or passes (kByMassGt) a target -- `goal` itself, or
 // that fraction of the universe's mass where `of_total` (the mass is then left in sh.total).  Leaves in sh: found
 // (0: the universe ends first), res_bits / res_ties (the prefix that reaches the goal ends with the res_ties-th of
-// the res_count tokens of this pattern), above_count / above_mass (what lies above that pattern).  With `levels`
-// below 4 the walk stops after so many digits: sh.prefix is then the bucket the answer lies in, res_count how
-// many tokens it holds, above_* what lies above the bucket.  Every thread of the workgroup calls it.
+// the res_count tokens of this pattern), above_count / above_mass (what lies above that pattern).
+// Every thread of the workgroup calls it.
 //
 // A level's buckets are walked by one wave, four buckets a lane from the top down: every lane adds up its own,
 // a running sum over the lanes gives each what lies above it, and the first lane in which the goal is reached
 // settles the bucket.
-__device__ void walk(Shared& sh, const Row& row, const Prefix& universe, int mode, unsigned int k, double goal,
-                     bool of_total, int levels = 4) {
+template <typename R>
+__device__ void walk(Shared& sh, const R& row, int vocab, const Prefix& universe, int mode, unsigned int k, double goal,
+                     bool of_total) {
   constexpr int kShift[4] = {23, 15, 7, 0};
   constexpr unsigned int kMask[4] = {0xffu, 0xffu, 0xffu, 0x7fu};
   constexpr int kPerLane = kBuckets / kWave;
   const int tid = threadIdx.x, lane = tid % kWave;
-  const bool packed = row.n <= kMaxPacked;
+  const bool packed = vocab <= kMaxPacked;
   if (tid == 0) {
     sh.prefix = 0;
     sh.above_count = 0;
@@ -193,7 +197,7 @@ __device__ void walk(Shared& sh, const Row& row, const Prefix& universe, int mod
     sh.found = 0;
     sh.alone_level = -1;
   }
-  for (int level = 0; level < levels; ++level) {
+  for (int level = 0; level < 4; ++level) {
     for (int i = tid; i < kBuckets; i += kThreads) {
       sh.cnt[i] = 0;
       sh.msum[i] = 0;
@@ -214,7 +218,7 @@ __device__ void walk(Shared& sh, const Row& row, const Prefix& universe, int mod
     };
     const bool bounded = universe.bits >= 0;
     const unsigned int floor_bits = static_cast<unsigned int>(universe.bits);
-    each_token(row, [&](unsigned int b, int) {
+    row.each([&](unsigned int b, int) {
       if (bounded && b <= floor_bits) return;
       if (level > 0 && (b >> kShift[level - 1]) != prefix) return;
       const int bucket = static_cast<int>((b >> kShift[level]) & kMask[level]);
@@ -309,14 +313,12 @@ __device__ void walk(Shared& sh, const Row& row, const Prefix& universe, int mod
         sh.above_count = above_count;
         sh.above_mass = above_mass;
         sh.res_count = count;
-        if (level == levels - 1) {
+        if (level == 3) {
           sh.done = 1;
           sh.found = 1;
-          if (level == 3) {
-            sh.res_bits = settled;
-            sh.res_ties = ties_needed(mode, k, target, above_count, above_mass, value_of(settled), count);
-          }
-        } else if (count == 1 && levels == 4) {
+          sh.res_bits = settled;
+          sh.res_ties = ties_needed(mode, k, target, above_count, above_mass, value_of(settled), count);
+        } else if (count == 1) {
           // one token in the bucket: it is the answer, whatever its other digits are
           sh.done = 1;
           sh.found = 1;
@@ -333,11 +335,87 @@ __device__ void walk(Shared& sh, const Row& row, const Prefix& universe, int mod
     const unsigned int digits = sh.prefix;
     const bool bounded = universe.bits >= 0;
     const unsigned int floor_bits = static_cast<unsigned int>(universe.bits);
-    each_token(row, [&](unsigned int b, int) {
+    row.each([&](unsigned int b, int) {
       if ((!bounded || b > floor_bits) && (b >> kShift[alone_level]) == digits) sh.res_bits = b;
     });
     __syncthreads();
   }
+}
+
+// The row's tokens in 2,048 buckets in the law's order: 64 an octave from 1 down to 2^-32, and all below that in the last one.
+// A bucket's tokens share the exponent, so its mass is the sum of their mantissas, exactly -- but for the last one's, which is
+// summed as it comes.  Thread t owns buckets 2 t and 2 t + 1 from then on, with what lies above them.
+constexpr int kFine = 2 * kThreads;
+__device__ inline int fine_bucket(unsigned int b) {
+  const int i = 0x1fc0 - static_cast<int>(b >> 17);
+  return i < 0 ? 0 : i < kFine ? i : kFine - 1;
+}
+struct Fine {
+  unsigned int count[2], above[2];
+  double mass[2], above_mass[2];
+  double total;
+};
+template <typename R>
+__device__ Fine look(Shared& sh, const R& row, unsigned long long* sums) {
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  sums[2 * tid] = sums[2 * tid + 1] = 0;
+  __syncthreads();
+  double low = 0.0;
+  row.each([&](unsigned int b, int) {
+    const int bucket = fine_bucket(b);
+    atomicAdd(&sums[bucket], (1ull << kCountShift) + mantissa(b));
+    if (bucket == kFine - 1) low += static_cast<double>(__uint_as_float(b));
+  });
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) low += __shfl_xor(low, off, kWave);
+  if (lane == 0) sh.red_d[wave] = low;
+  __syncthreads();
+  Fine f;
+  low = 0.0;
+  for (int w = 0; w < kWaves; ++w) low += sh.red_d[w];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const unsigned long long sum = sums[2 * tid + j];
+    f.count[j] = static_cast<unsigned int>(sum >> kCountShift);
+    f.mass[j] = 2 * tid + j == kFine - 1 ? low : f.count[j] ? scaled(sum & ((1ull << kCountShift) - 1ull), (0x1fc0u - (2 * tid + j)) >> 6) : 0.0;
+  }
+  const unsigned int with_count = wave_scan_u32(f.count[0] + f.count[1], lane);
+  const double with_mass = wave_scan_f64(f.mass[0] + f.mass[1], lane);
+  __syncthreads();
+  if (lane == kWave - 1) sh.red_u[wave] = with_count, sh.red_d[wave] = with_mass;
+  const unsigned int lanes_count = __shfl_up(with_count, 1, kWave);
+  const double lanes_mass = __shfl_up(with_mass, 1, kWave);
+  __syncthreads();
+  unsigned int above = 0;
+  double above_mass = 0.0;
+  f.total = 0.0;
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < wave) above += sh.red_u[w], above_mass += sh.red_d[w];
+    f.total += sh.red_d[w];
+  }
+  f.above[0] = above + (lane ? lanes_count : 0u);
+  f.above_mass[0] = above_mass + (lane ? lanes_mass : 0.0);
+  f.above[1] = f.above[0] + f.count[0];
+  f.above_mass[1] = f.above_mass[0] + f.mass[0];
+  return f;
+}
+
+// The bucket in which a goal is reached (as walk's modes have it), into sh.bucket (kFine: in none), and what lies above it.
+__device__ void find_bucket(Shared& sh, const Fine& f, int mode, unsigned int k, double target) {
+  if (threadIdx.x == 0) sh.bucket = kFine;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (f.count[j] && reached(mode, k, target, f.above[j] + f.count[j], f.above_mass[j] + f.mass[j])) {
+      atomicMin(&sh.bucket, 2 * static_cast<int>(threadIdx.x) + j);
+      break;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (sh.bucket == 2 * static_cast<int>(threadIdx.x) + j)
+      sh.bucket_above = f.above[j], sh.bucket_mass = f.above_mass[j], sh.bucket_count = static_cast<int>(f.count[j]);
+  __syncthreads();
 }
 
 // Where this thread's `mine` items go among those of all the workgroup's threads, in the order of the threads, and
@@ -360,168 +438,449 @@ __device__ inline void place_among(Shared& sh, unsigned int mine, int& place, in
   __syncthreads();
 }
 
-// The id of the r-th of the `count` tokens, in the order of the ids, whose weight has this pattern; into sh.hit.
-__device__ void locate(Shared& sh, const Row& row, unsigned int bits, int r, int count) {
-  if (count == 1) {                                     // the one there is: nothing to put in order
-    each_token(row, [&](unsigned int b, int i) {
-      if (b == bits) sh.hit = row.id_at(i);
-    });
-    return;
-  }
+// The id of the r-th of the tokens, in the order of the ids, whose weight has this pattern; into sh.hit.
+template <typename R>
+__device__ void locate(Shared& sh, const R& whole, unsigned int bits, int r) {
   int seen = 0;
-  for (int base = 0; base < row.n; base += kThreads) {
+  for (int base = 0; base < whole.n; base += kThreads) {
     const int i = base + threadIdx.x;
-    const bool match = i < row.n && row.bits_at(i) == bits;
+    const bool match = i < whole.n && whole.at(i) == bits;
     int place, all;
     place_among(sh, match ? 1u : 0u, place, all);
-    if (match && seen + place + 1 == r) sh.hit = row.id_at(i);
+    if (match && seen + place + 1 == r) sh.hit = i;
     seen += all;
     if (seen >= r) break;
   }
 }
 
-// The row's tokens whose pattern is `bound` or above, in the order of their ids, into the list; how many.
-// The row is one whose patterns come from the logits.  Eight tokens in a row to a thread and turn; a turn's
-// logits are asked for a turn ahead, so that the way from memory lies beside the turn before's barriers.
-__device__ int list_from(Shared& sh, const Row& row, unsigned int bound, unsigned int* listed, int* listed_id) {
-  constexpr int kEach = 8;
-  auto ask = [&](int base, float (&l)[kEach]) {
-    const int first = base + kEach * threadIdx.x;
-#pragma unroll
-    for (int j = 0; j < kEach; ++j) l[j] = first + j < row.n ? row.logits[first + j] : 0.f;
-  };
-  int seen = 0;
-  float next[kEach];
-  ask(0, next);
-  for (int base = 0; base < row.n; base += kEach * kThreads) {
-    const int first = base + kEach * threadIdx.x;
-    unsigned int b[kEach];
-    unsigned int mine = 0;
-#pragma unroll
-    for (int j = 0; j < kEach; ++j) {
-      b[j] = __float_as_uint(expf((next[j] - row.row_max) * row.inv_t));
-      mine += first + j < row.n && b[j] >= bound ? 1u : 0u;
-    }
-    if (base + kEach * kThreads < row.n) ask(base + kEach * kThreads, next);
-    int place, all;
-    place_among(sh, mine, place, all);
-    int at = seen + place;
-#pragma unroll
-    for (int j = 0; j < kEach; ++j) {
-      if (first + j < row.n && b[j] >= bound) {
-        listed[at] = b[j];
-        listed_id[at] = first + j;
-        ++at;
-      }
-    }
-    seen += all;
+// The tokens of fine buckets first .. last, up to kFew of them, in the law's order: their keys (a weight's pattern above, the id's
+// complement below) in `room` + kFew, and returns this thread's running sum, up to and with the token of its number, from `above` on.
+constexpr int kFew = 512;
+template <typename R>
+__device__ double sort_few(Shared& sh, const R& row, int first, int last, double above, unsigned long long* room, int& n) {
+  unsigned long long* keys = room;
+  unsigned long long* sorted = room + kFew;
+  int* rank = reinterpret_cast<int*>(room + 2 * kFew);
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  if (tid == 0) sh.listed = 0, sh.first_ge = kFew, sh.first_gt = kFew;
+  if (tid < kFew) rank[tid] = 0;
+  __syncthreads();
+  row.each([&](unsigned int b, int i) {
+    const int bucket = fine_bucket(b);
+    if (bucket < first || bucket > last) return;
+    const int at = atomicAdd(&sh.listed, 1);
+    if (at < kFew) keys[at] = static_cast<unsigned long long>(b) << 32 | static_cast<unsigned int>(~i);
+  });
+  __syncthreads();
+  n = min(sh.listed, kFew);
+  // every key counts those before it; where there are few, several threads share a key's count
+  int width = kWave;
+  while (width < n) width *= 2;
+  const int parts = kThreads / width, mine = tid % width, part = tid / width, each = (n + parts - 1) / parts;
+  if (mine < n) {
+    const unsigned long long key = keys[mine];
+    int before = 0;
+    const int end = min(n, (part + 1) * each);
+#pragma unroll 4
+    for (int j = part * each; j < end; ++j) before += keys[j] > key ? 1 : 0;
+    if (before) atomicAdd(&rank[mine], before);
   }
   __syncthreads();
-  return seen;
+  if (tid < n) sorted[rank[tid]] = keys[tid];
+  __syncthreads();
+  double mass = 0.0;
+  if (tid < kFew) {
+    mass = wave_scan_f64(tid < n ? value_of(static_cast<long long>(sorted[tid] >> 32)) : 0.0, lane);
+    if (lane == kWave - 1) sh.red_d[wave] = mass;
+  }
+  __syncthreads();
+  for (int w = 0; w < wave && w < kFew / kWave; ++w) above += sh.red_d[w];
+  mass += above;
+  if (tid < n) reinterpret_cast<double*>(keys)[tid] = mass;   // (the keys have been put in order)
+  __syncthreads();
+  return mass;
+}
+// The first of the sorted tokens below `end` at which a running sum reaches (ge) or passes the target; end - 1 if none does.
+__device__ int first_at(int& place, double mass, bool ge, double target, int end) {
+  const int tid = threadIdx.x;
+  const unsigned long long over = __ballot(tid < end && (ge ? mass >= target : mass > target));
+  if (over != 0ull && tid % kWave == 0) atomicMin(&place, tid + __ffsll(static_cast<long long>(over)) - 1);
+  __syncthreads();
+  return min(place, end - 1);
 }
 
-__global__ __launch_bounds__(kThreads) void sample_filtered_kernel(
-    const float* __restrict__ logits, const int32_t* __restrict__ rows, const float* __restrict__ temperature,
-    const double* __restrict__ u, const int32_t* __restrict__ top_k, const double* __restrict__ top_p,
-    int32_t* __restrict__ out, int vocab, int cache_patterns) {
-  __shared__ Shared sh;
-  extern __shared__ unsigned int room[];            // the row's patterns, or the list's patterns and ids
-  const int which = blockIdx.x;
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  Row whole;
-  whole.logits = logits + static_cast<size_t>(rows[which]) * vocab;
-  whole.cached = nullptr;
-  whole.listed = nullptr;
-  whole.listed_id = nullptr;
-  whole.n = vocab;
+// The three questions by walks over the row, whatever its weights.
+template <typename R>
+__device__ int draw_by_walks(Shared& sh, const R& row, unsigned int k, double p, double u) {
+  const int vocab = row.n;
+  const Prefix everything = {-1, 0, -1.0};
+  Prefix kept = everything;
+  // the k likeliest; of those, the fewest that reach top_p of their total; the first of those at which the running sum
+  // passes u of their mass; and, where rounding keeps that from being reached, the last of the row's tokens
+  int question = k < static_cast<unsigned int>(vocab) ? 0 : p < 1.0 ? 1 : 2;
+  for (;;) {
+    const bool of_total = question > 0 && question < 3 && kept.mass < 0.0;
+    const double share = question == 1 ? p : u;
+    walk(sh, row, vocab, question == 3 ? everything : kept, question == 0 || question == 3 ? kByCount : question == 1 ? kByMassGe : kByMassGt,
+         question == 3 ? static_cast<unsigned int>(vocab) : k, of_total ? share : share * kept.mass, of_total);
+    const bool found = sh.found;
+    const long long bits = sh.res_bits;
+    const int ties = sh.res_ties;
+    const double mass = sh.above_mass, all = sh.total;
+    __syncthreads();
+    if (question < 2) {
+      if (found) kept = {bits, ties, mass + ties * value_of(bits)};
+      else if (question == 1 && of_total) kept.mass = all;      // (rounding left the sum a hair short: everything is kept)
+      question = question == 0 && p < 1.0 ? 1 : 2;
+      continue;
+    }
+    if (!found && question == 2 && !(kept.bits >= 0 && kept.ties > 0)) {
+      question = 3;
+      continue;
+    }
+    const bool of_kept = !found && question == 2;               // (rounding again: the last of the kept tokens)
+    locate(sh, row, static_cast<unsigned int>(of_kept ? kept.bits : bits), of_kept ? kept.ties : ties);
+    __syncthreads();
+    return sh.hit;
+  }
+}
 
+template <typename R>
+__device__ int draw_from(Shared& sh, const R& row, int top_k, double p, double u, unsigned long long* room) {
+  const int vocab = row.n;
+  const bool count_first = top_k > 0 && top_k < vocab;
+  const unsigned int k = count_first ? static_cast<unsigned int>(top_k) : static_cast<unsigned int>(vocab);
+  if (vocab > kMaxPacked) return draw_by_walks(sh, row, k, p, u);
+  const Fine fine = look(sh, row, room);
+  // The first question's bucket.  (Questions whose answer lies in the last bucket, which holds many exponents, or in one
+  // with more tokens than can be put in order go the general way.)
+  find_bucket(sh, fine, count_first ? kByCount : kByMassGe, k, p * fine.total);
+  int bucket = sh.bucket;
+  if (bucket >= kFine - 1 || sh.bucket_count > kFew) return draw_by_walks(sh, row, k, p, u);
+  const unsigned long long* sorted = room + kFew;
+  const double* upto = reinterpret_cast<const double*>(room);
+  const bool all = sh.bucket_above + static_cast<unsigned int>(sh.bucket_count) <= static_cast<unsigned int>(kFew);
+  double above = all ? 0.0 : sh.bucket_mass;
+  int before = all ? 0 : static_cast<int>(sh.bucket_above);         // tokens above the sorted ones
+  int n;
+  __syncthreads();
+  double mass = sort_few(sh, row, all ? 0 : bucket, bucket, above, room, n);
+  int kept = count_first ? min(static_cast<int>(k) - before, n) : n;      // of the sorted tokens
+  double kept_mass = upto[kept - 1];
+  if (p < 1.0) {
+    const double target = p * (count_first ? kept_mass : fine.total);
+    if (count_first && !all) {
+      // the nucleus may end in an earlier bucket than the k likeliest do
+      find_bucket(sh, fine, kByMassGe, 0, target);
+      const int earlier = sh.bucket, count = sh.bucket_count;
+      above = sh.bucket_mass;
+      __syncthreads();
+      if (earlier < bucket) {
+        if (count > kFew) return draw_by_walks(sh, row, k, p, u);
+        bucket = earlier;
+        mass = sort_few(sh, row, bucket, bucket, above, room, n);
+        kept = n;
+      }
+    }
+    kept = first_at(sh.first_ge, mass, true, target, kept) + 1;
+    kept_mass = upto[kept - 1];
+  }
+  const double target = u * kept_mass;
+  if (!all) {
+    find_bucket(sh, fine, kByMassGt, 0, target);
+    const int earlier = sh.bucket, count = sh.bucket_count;
+    above = sh.bucket_mass;
+    __syncthreads();
+    if (earlier < bucket) {
+      if (count > kFew) return draw_by_walks(sh, row, k, p, u);
+      mass = sort_few(sh, row, earlier, earlier, above, room, n);
+      kept = n;
+    }
+  }
+  return static_cast<int>(~static_cast<unsigned int>(sorted[first_at(sh.first_gt, mass, false, target, kept)]));
+}
+
+// HELD: the vocabulary's patterns fit LDS beside the few candidates' keys.
+template <bool HELD>
+__device__ int draw_filtered(Shared& sh, const float* logits, int vocab, float temperature, double u, int top_k, double p, unsigned int* room) {
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   float v = -FLT_MAX;
-  for (int base = threadIdx.x; base < vocab; base += 8 * kThreads) {
-    float l[8];
+  const bool by_four = vocab % 4 == 0 && reinterpret_cast<uintptr_t>(logits) % 16 == 0;
+  auto four_at = [&](int first) {                   // four logits from `first` on (below the vocabulary), -FLT_MAX beyond its end
+    if (by_four) return *reinterpret_cast<const float4*>(logits + first);
+    return make_float4(logits[first], first + 1 < vocab ? logits[first + 1] : -FLT_MAX, first + 2 < vocab ? logits[first + 2] : -FLT_MAX,
+                       first + 3 < vocab ? logits[first + 3] : -FLT_MAX);
+  };
+  float4 l[kHeldTurns];
+  for (int begin = 0; begin < vocab; begin += kMaxHeld) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) l[j] = base + j * kThreads < vocab ? whole.logits[base + j * kThreads] : -FLT_MAX;
+    for (int j = 0; j < kHeldTurns; ++j) {
+      const int first = begin + (j * kThreads + threadIdx.x) * 4;
+      l[j] = first < vocab ? four_at(first) : make_float4(-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX);
+    }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v = fmaxf(v, l[j]);
+    for (int j = 0; j < kHeldTurns; ++j) v = fmaxf(fmaxf(fmaxf(v, l[j].x), fmaxf(l[j].y, l[j].z)), l[j].w);
   }
   v = wave_max(v);
   if (lane == 0) sh.red_v[wave] = v;
   __syncthreads();
   v = sh.red_v[0];
   for (int w = 1; w < kWaves; ++w) v = fmaxf(v, sh.red_v[w]);
-  whole.row_max = v;
-  whole.inv_t = 1.0f / temperature[which];
+  const Logits row{logits, vocab, v, 1.0f / temperature};
   if (threadIdx.x == 0) sh.hit = 0;
-  __syncthreads();
+  if constexpr (HELD) {                             // (the logits are still in registers)
+#pragma unroll
+    for (int j = 0; j < kHeldTurns; ++j)
+      *reinterpret_cast<uint4*>(room + (j * kThreads + threadIdx.x) * 4) =
+          make_uint4(row.bits_of(l[j].x), row.bits_of(l[j].y), row.bits_of(l[j].z), row.bits_of(l[j].w));
+    return draw_from(sh, Cached{room, vocab}, top_k, p, u, reinterpret_cast<unsigned long long*>(room + kMaxHeld));
+  } else {
+    return draw_from(sh, row, top_k, p, u, reinterpret_cast<unsigned long long*>(room));
+  }
+}
 
-  const unsigned int k = top_k[which] > 0 && top_k[which] < vocab ? static_cast<unsigned int>(top_k[which])
-                                                                 : static_cast<unsigned int>(vocab);
-  const bool count_first = k < static_cast<unsigned int>(vocab);
-  const double p = top_p[which];
-  const Prefix everything = {-1, 0, -1.0};
-  Prefix kept = everything;
-  Row row = whole;
-  {
-    // a look at the exponents alone: the bucket in which the first question's answer lies, and how many tokens
-    // there are from that bucket up -- if the list holds them, they are all that the walks have to look at
-    if (count_first) walk(sh, whole, everything, kByCount, k, 0.0, false, 1);
-    else walk(sh, whole, everything, kByMassGe, 0, p, true, 1);
-    const bool found = sh.found;
-    const unsigned int bucket = sh.prefix, candidates = sh.above_count + static_cast<unsigned int>(sh.res_count);
-    if (!count_first) kept.mass = sh.total;
-    __syncthreads();
-    if (found && candidates <= static_cast<unsigned int>(kMaxListed)) {
-      int* listed_id = reinterpret_cast<int*>(room + kMaxListed);
-      row.n = list_from(sh, whole, bucket << 23, room, listed_id);
-      row.listed = room;
-      row.listed_id = listed_id;
-    } else if (cache_patterns) {
-      for (int i = threadIdx.x; i < vocab; i += kThreads) room[i] = whole.bits_at(i);
-      __syncthreads();
-      whole.cached = room;
-      row = whole;
+// ---- temperature sampling --------------------------------------------------
+// The law: weights w_i = exp((l_i - max) / T) in float, summed in double; the token is the first i,
+// in vocabulary order, at which u * total - (w_0 + ... + w_i) turns negative.  One workgroup a row.
+// The vocabulary is cut into groups of 512 consecutive tokens, a lane holding eight in a row (more
+// beyond 2,097,152 tokens, so that the groups' sums fit LDS): a lane sums its own tokens in order
+// without a word to its neighbours (sums of doubles across lanes go through the LDS crossbar, which
+// sixteen waves share), a wave then a group; every pass over the row reads whole cache lines.  The
+// groups' sums, a running sum over them (one wave, 64 groups a step) and a last look inside the one
+// group where the target is crossed find the token.
+// (Sums in another order than the host's one-by-one walk: a boundary may move by one token when u
+// falls within rounding of it.)
+constexpr int kSampleMaxGroups = 4096;
+constexpr int kSamplePerLane = 8;           // consecutive tokens a lane holds of a group
+constexpr int kSampleAhead = 4;             // loads of 16 bytes (pairs of them in the second pass) a thread has in flight
+
+__device__ inline void better(float& v, int& i, float ov, int oi) {
+  if (ov > v || (ov == v && oi < i)) {
+    v = ov;
+    i = oi;
+  }
+}
+
+__device__ inline double wave_sum_f64(double v) {
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+  return v;
+}
+// Thread 0 writes the token to `to`.  group_sum: kSampleMaxGroups doubles, then the running sums up to and with each group.
+__device__ void draw_unfiltered(Shared& sh, const float* row, int vocab, float temp, double u, double* group_sum, int32_t* to) {
+  float* best_v = sh.red_v;
+  int* best_i = sh.wave_cnt;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+
+  // the maximum and where it stands first
+  float v = -FLT_MAX;
+  int idx = vocab;
+  // in fours where the row starts on 16 bytes and the vocabulary is a multiple of four
+  const bool by_four = vocab % 4 == 0 && reinterpret_cast<uintptr_t>(row) % 16 == 0;
+  if (by_four) {
+    const float4* row4 = reinterpret_cast<const float4*>(row);
+    const int n4 = vocab / 4;
+    for (int at = threadIdx.x; at < n4; at += kSampleAhead * kThreads) {
+      float4 t[kSampleAhead];               // the loads first, so that they are in flight together
+#pragma unroll
+      for (int j = 0; j < kSampleAhead; ++j) {
+        const int i4 = at + j * kThreads;
+        t[j] = i4 < n4 ? row4[i4] : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+#pragma unroll
+      for (int j = 0; j < kSampleAhead; ++j) {
+        const int i4 = at + j * kThreads;
+        if (i4 < n4) {
+          better(v, idx, t[j].x, 4 * i4);
+          better(v, idx, t[j].y, 4 * i4 + 1);
+          better(v, idx, t[j].z, 4 * i4 + 2);
+          better(v, idx, t[j].w, 4 * i4 + 3);
+        }
+      }
+    }
+  } else {
+    for (int at = threadIdx.x; at < vocab; at += kThreads) better(v, idx, row[at], at);
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) better(v, idx, __shfl_xor(v, off, kWave), __shfl_xor(idx, off, kWave));
+  if (lane == 0) {
+    best_v[wave] = v;
+    best_i[wave] = idx;
+  }
+  __syncthreads();
+  float row_max = best_v[0];
+  int best = best_i[0];
+  for (int w = 1; w < kWaves; ++w) better(row_max, best, best_v[w], best_i[w]);
+  const int arg = best < vocab ? best : 0;
+  if (!(temp > 0.f)) {
+    if (threadIdx.x == 0) *to = arg;
+    return;
+  }
+  const float inv_t = 1.0f / temp;
+  const int per_lane = max(kSamplePerLane, (vocab + kWave * kSampleMaxGroups - 1) / (kWave * kSampleMaxGroups));
+  const int group_size = kWave * per_lane;
+  const int n_groups = (vocab + group_size - 1) / group_size;
+  auto lane_weight_sum = [&](int g) {      // this lane's tokens of group g, in order
+    double s = 0.0;
+    const int first = g * group_size + lane * per_lane;
+    for (int j = 0; j < per_lane; ++j) {
+      const int i = first + j;
+      if (i < vocab) s += static_cast<double>(expf((row[i] - row_max) * inv_t));
+    }
+    return s;
+  };
+  if (by_four && per_lane == kSamplePerLane) {        // a wave's groups at once: their loads are in flight together
+    static_assert(kSamplePerLane == 8, "two loads of four a lane");
+    for (int g0 = wave; g0 < n_groups; g0 += kWaves * kSampleAhead) {
+      float4 t[kSampleAhead][2];
+#pragma unroll
+      for (int j = 0; j < kSampleAhead; ++j) {
+        const int first = (g0 + j * kWaves) * group_size + lane * kSamplePerLane;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          t[j][h] = first + 4 * h < vocab ? *reinterpret_cast<const float4*>(row + first + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+#pragma unroll
+      for (int j = 0; j < kSampleAhead; ++j) {
+        const int g = g0 + j * kWaves;
+        const int first = g * group_size + lane * kSamplePerLane;
+        double s = 0.0;                     // the order of lane_weight_sum: the look inside a group sums the same
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if (first + 4 * h < vocab) {
+            s += static_cast<double>(expf((t[j][h].x - row_max) * inv_t));
+            s += static_cast<double>(expf((t[j][h].y - row_max) * inv_t));
+            s += static_cast<double>(expf((t[j][h].z - row_max) * inv_t));
+            s += static_cast<double>(expf((t[j][h].w - row_max) * inv_t));
+          }
+        }
+        s = wave_sum_f64(s);
+        if (lane == 0 && g < n_groups) group_sum[g] = s;
+      }
+    }
+  } else {
+    for (int g = wave; g < n_groups; g += kWaves) {
+      const double s = wave_sum_f64(lane_weight_sum(g));
+      if (lane == 0) group_sum[g] = s;
     }
   }
-  // the k likeliest
-  if (count_first) {
-    walk(sh, row, everything, kByCount, k, 0.0, false);
-    if (sh.found) kept = {sh.res_bits, sh.res_ties, sh.above_mass + sh.res_ties * value_of(sh.res_bits)};
-    __syncthreads();
-  }
-  // of those, the fewest that reach top_p of their total
-  Prefix nucleus = kept;
-  if (p < 1.0) {
-    const bool of_total = kept.mass < 0.0;
-    walk(sh, row, kept, kByMassGe, 0, of_total ? p : p * kept.mass, of_total);
-    if (sh.found) nucleus = {sh.res_bits, sh.res_ties, sh.above_mass + sh.res_ties * value_of(sh.res_bits)};
-    else if (of_total) nucleus.mass = sh.total;       // (rounding left the sum a hair short: everything is kept)
-    __syncthreads();
-  }
-  // the first of those at which the running sum passes u of their mass
-  const bool of_total = nucleus.mass < 0.0;
-  walk(sh, row, nucleus, kByMassGt, 0, of_total ? u[which] : u[which] * nucleus.mass, of_total);
-  long long bits = sh.res_bits;
-  int r = sh.res_ties, count = sh.res_count;
-  const bool found = sh.found;
   __syncthreads();
-  if (!found) {                                        // rounding again: the last of the kept tokens
-    if (nucleus.bits >= 0 && nucleus.ties > 0) {
-      bits = nucleus.bits, r = nucleus.ties, count = 0;            // (how many there are of it is not known here)
-    } else {
-      row = whole;
-      walk(sh, row, everything, kByCount, static_cast<unsigned int>(vocab), 0.0, false);
-      bits = sh.res_bits, r = sh.res_ties, count = sh.res_count;
-      __syncthreads();
+  if (wave != 0) return;
+
+  // one wave: running sums over the groups, 64 at a step; then the first group they cross the target in
+  double carry = 0.0;
+  for (int c = 0; c < n_groups; c += kWave) {
+    const int g = c + lane;
+    const double incl = carry + wave_scan_f64(g < n_groups ? group_sum[g] : 0.0, lane);
+    if (g < n_groups) group_sum[g] = incl;
+    carry = __shfl(incl, kWave - 1, kWave);
+  }
+  const double target = u * carry;
+  int found = n_groups;
+  for (int c = 0; c < n_groups && found == n_groups; c += kWave) {
+    const int g = c + lane;
+    const unsigned long long over = __ballot(g < n_groups && target - group_sum[g] < 0.0);
+    if (over != 0ull) found = c + __ffsll(static_cast<long long>(over)) - 1;
+  }
+  int result = arg;        // rounding may leave the target a hair above zero after the last token
+  if (found < n_groups) {
+    const double before = found > 0 ? group_sum[found - 1] : 0.0;
+    const double mine = lane_weight_sum(found);
+    const double upto = before + wave_scan_f64(mine, lane);              // with this lane's tokens
+    const unsigned long long over = __ballot(target - upto < 0.0);
+    if (over != 0ull) {
+      const int at = __ffsll(static_cast<long long>(over)) - 1;          // the lane whose tokens cross it
+      double left = target - (upto - mine);
+      const int first = found * group_size + lane * per_lane;
+      int hit = min(vocab - 1, first + per_lane - 1);
+      for (int j = 0; j < per_lane; ++j) {
+        const int i = first + j;
+        if (i >= vocab) break;
+        left -= static_cast<double>(expf((row[i] - row_max) * inv_t));
+        if (left < 0.0) {
+          hit = i;
+          break;
+        }
+      }
+      result = __shfl(hit, at, kWave);
     }
   }
-  locate(sh, row, static_cast<unsigned int>(bits), r, count);
-  __syncthreads();
-  if (threadIdx.x == 0) out[rows[which]] = sh.hit;
+  if (lane == 0) *to = result;
+}
+
+
+// What the rows of a launch ask for, in its arguments: nothing to bring to the device before it.
+constexpr int kChooseRows = 64;
+struct ChooseArgs {
+  double u[kChooseRows], top_p[kChooseRows];
+  float temperature[kChooseRows];
+  int top_k[kChooseRows];
+};
+
+template <bool HELD>
+__global__ __launch_bounds__(kThreads) void choose_kernel(const float* __restrict__ logits, int32_t* __restrict__ out, int vocab,
+                                                          const ChooseArgs a) {
+  __shared__ Shared sh;
+  extern __shared__ __align__(16) unsigned int room[];
+  const int row = blockIdx.x;
+  const float* from = logits + static_cast<size_t>(row) * vocab;
+  if (a.temperature[row] > 0.f && ((a.top_k[row] > 0 && a.top_k[row] < vocab) || a.top_p[row] < 1.0)) {
+    const int token = draw_filtered<HELD>(sh, from, vocab, a.temperature[row], a.u[row], a.top_k[row], a.top_p[row], room);
+    if (threadIdx.x == 0) out[row] = token;
+  } else {
+    draw_unfiltered(sh, from, vocab, a.temperature[row], a.u[row], reinterpret_cast<double*>(room), out + row);
+  }
+}
+
+__global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
+                                                          const double* __restrict__ u, int32_t* __restrict__ out, int vocab) {
+  __shared__ Shared sh;
+  __shared__ double group_sum[kSampleMaxGroups];
+  const int row = blockIdx.x;
+  draw_unfiltered(sh, logits + static_cast<size_t>(row) * vocab, vocab, temperature[row], u[row], group_sum, out + row);
+}
+
+template <bool HELD>
+__global__ __launch_bounds__(kThreads) void sample_filtered_kernel(
+    const float* __restrict__ logits, const int32_t* __restrict__ rows, const float* __restrict__ temperature,
+    const double* __restrict__ u, const int32_t* __restrict__ top_k, const double* __restrict__ top_p,
+    int32_t* __restrict__ out, int vocab) {
+  __shared__ Shared sh;
+  extern __shared__ __align__(16) unsigned int room[];
+  const int i = blockIdx.x, row = rows[i];
+  const int token = draw_filtered<HELD>(sh, logits + static_cast<size_t>(row) * vocab, vocab, temperature[i], u[i], top_k[i], top_p[i], room);
+  if (threadIdx.x == 0) out[row] = token;
+}
+
+constexpr int kRoomBytes = kRoom * 4;
+static_assert((kRoom - kMaxHeld) * 4 >= 3 * kFew * 8 && (kRoom - kMaxHeld) * 4 >= kFine * 8 && kRoomBytes >= kSampleMaxGroups * 8,
+              "the sorted tokens, the buckets, and in a mixed launch a plain row's sums over groups");
+
+int raise_room() {
+  static std::once_flag once;
+  static hipError_t raised = hipSuccess;
+  std::call_once(once, [] {
+    const void* kernels[] = {reinterpret_cast<const void*>(sample_filtered_kernel<true>), reinterpret_cast<const void*>(sample_filtered_kernel<false>),
+                             reinterpret_cast<const void*>(choose_kernel<true>), reinterpret_cast<const void*>(choose_kernel<false>)};
+    for (const void* kernel : kernels)
+      if (raised == hipSuccess) raised = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kRoomBytes);
+  });
+  if (raised != hipSuccess) return fail("sampling: cannot raise the dynamic LDS limit to %d bytes", kRoomBytes);
+  return 0;
 }
 
 }  // namespace
 }  // namespace bc4g
 
 using namespace bc4g;
+
+extern "C" int bc4g_sample(const float* logits, const float* temperature, const double* u, int32_t* out,
+                           int n_rows, int vocab, void* stream) {
+  BC4G_REQUIRE(n_rows >= 0 && vocab > 0, "sample: bad sizes rows=%d V=%d", n_rows, vocab);
+  if (n_rows == 0) return 0;
+  sample_kernel<<<n_rows, kThreads, 0, static_cast<hipStream_t>(stream)>>>(logits, temperature, u, out, vocab);
+  return check_launch("sample");
+}
 
 // For each of n rows: draws the token of logits row rows[i] by the law above with temperature[i] (> 0), the
 // uniform number u[i] in [0, 1), top_k[i] (0 or >= vocab: no limit) and top_p[i] (>= 1: no limit), into
@@ -531,17 +890,31 @@ extern "C" int bc4g_sample_filtered(const float* logits, const int32_t* rows, co
                                     void* stream) {
   BC4G_REQUIRE(n >= 0 && vocab > 0, "sample_filtered: bad sizes rows=%d V=%d", n, vocab);
   if (n == 0) return 0;
-  const int cache_patterns = vocab <= kMaxCached ? 1 : 0;
-  const size_t lds = static_cast<size_t>(kMaxCached) * sizeof(unsigned int);      // the list's room, or the patterns'
-  static std::once_flag once;
-  static hipError_t raised = hipSuccess;
-  std::call_once(once, [] {
-    raised = hipFuncSetAttribute(reinterpret_cast<const void*>(sample_filtered_kernel),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, kMaxCached * sizeof(unsigned int));
-  });
-  if (raised != hipSuccess) return fail("sample_filtered: cannot raise the dynamic LDS limit to %d bytes",
-                                        static_cast<int>(kMaxCached * sizeof(unsigned int)));
-  sample_filtered_kernel<<<n, kThreads, lds, static_cast<hipStream_t>(stream)>>>(logits, rows, temperature, u, top_k,
-                                                                               top_p, out, vocab, cache_patterns);
+  if (int e = raise_room()) return e;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (vocab <= kMaxHeld)
+    sample_filtered_kernel<true><<<n, kThreads, kRoomBytes, s>>>(logits, rows, temperature, u, top_k, top_p, out, vocab);
+  else
+    sample_filtered_kernel<false><<<n, kThreads, kRoomBytes, s>>>(logits, rows, temperature, u, top_k, top_p, out, vocab);
   return check_launch("sample_filtered");
+}
+
+// temperature, u, top_k and top_p lie on the host.
+extern "C" int bc4g_choose(const float* logits, const float* temperature, const double* u, const int32_t* top_k, const double* top_p,
+                           int32_t* out, int n_rows, int vocab, void* stream) {
+  BC4G_REQUIRE(n_rows >= 0 && vocab > 0 && logits && temperature && u && top_k && top_p && out, "choose: bad sizes rows=%d V=%d, or a tensor is missing",
+               n_rows, vocab);
+  if (int e = raise_room()) return e;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  for (int first = 0; first < n_rows; first += kChooseRows) {
+    const int rows = n_rows - first < kChooseRows ? n_rows - first : kChooseRows;
+    ChooseArgs a{};
+    for (int i = 0; i < rows; ++i)
+      a.temperature[i] = temperature[first + i], a.u[i] = u[first + i], a.top_k[i] = top_k[first + i], a.top_p[i] = top_p[first + i];
+    const float* from = logits + static_cast<size_t>(first) * vocab;
+    if (vocab <= kMaxHeld) choose_kernel<true><<<rows, kThreads, kRoomBytes, s>>>(from, out + first, vocab, a);
+    else choose_kernel<false><<<rows, kThreads, kRoomBytes, s>>>(from, out + first, vocab, a);
+    if (int e = check_launch("choose")) return e;
+  }
+  return 0;
 }

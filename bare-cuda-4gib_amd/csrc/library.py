@@ -36,6 +36,7 @@ _SIGNATURES = {
     "bc4g_attention_f32": [_P, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _P],
     "bc4g_argmax": [_P, _P, _P, _P, _I, _I, _P],
     "bc4g_sample": [_P, _P, _P, _P, _I, _I, _P],
+    "bc4g_choose": [_P, _P, _P, _P, _P, _P, _I, _I, _P],
     "bc4g_sample_filtered": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _P],
     "bc4g_argmax_static": [_P, _P, _I, _I, _P],
     "bc4g_probe_read": [_P, c_long, _P, _I, _P],

@@ -7,6 +7,7 @@ library, or on a CPU tensor, they raise.
 """
 from __future__ import annotations
 
+import array
 import ctypes
 import dataclasses
 import math
@@ -504,6 +505,24 @@ def sample_filtered(logits: torch.Tensor, out: torch.Tensor, rows: torch.Tensor,
     vocab = logits.shape[1]
     library.call("bc4g_sample_filtered", _ptr(logits), _ptr(rows), _ptr(temperature), _ptr(u), _ptr(top_k), _ptr(top_p),
                  _ptr(out), n, vocab, _stream(), cost=lambda: (40.0 * n * vocab, n * vocab * 4))
+    return out
+
+
+def choose(logits: torch.Tensor, temperature: Sequence[float], u: Sequence[float], top_k: Sequence[int],
+           top_p: Sequence[float]) -> torch.Tensor:
+    """Every row's token, int32 [rows], in one launch: row i is greedy where temperature[i] is not above 0, drawn by the law of
+    sample_filtered where top_k[i] (of 1 .. vocab - 1) or top_p[i] (below 1) limits it, else by that of sample, with the
+    uniform number u[i].  The options are host numbers: they go along as arguments of the launch."""
+    _dev("choose", logits)
+    if logits.dtype != torch.float32 or logits.dim() != 2:
+        raise KernelError("choose: logits must be float32 [rows, vocab]")
+    rows, vocab = logits.shape
+    if not len(temperature) == len(u) == len(top_k) == len(top_p) == rows:
+        raise KernelError(f"choose: options for {len(temperature)}, {len(u)}, {len(top_k)} and {len(top_p)} rows of {rows}")
+    out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
+    options = array.array("f", temperature), array.array("d", u), array.array("i", top_k), array.array("d", top_p)
+    library.call("bc4g_choose", _ptr(logits), *(o.buffer_info()[0] for o in options), _ptr(out), rows, vocab, _stream(),
+                 cost=lambda: (20.0 * rows * vocab, rows * vocab * 4))
     return out
 
 

@@ -35,8 +35,8 @@ class DevicePicker:
     temperature are drawn from the request's own uniform number -- by inverse CDF in the order of the ids where
     nothing filters them, and, with top-k or top-p, by the reference's law for those (the tokens by falling weight,
     the k likeliest, the fewest of them that reach top_p, the first at which u of the kept mass is passed:
-    engine/src/sampler.cpp:63-104) in a kernel of its own over just those rows.  One small download per step,
-    and none before the next step may start (pick_later)."""
+    engine/src/sampler.cpp:63-104).  One launch for a step's rows, whose options go along as its arguments; one small
+    download, and none before the next step may start (pick_later)."""
 
     @staticmethod
     def _filters(p: SamplingParams, vocab: int) -> bool:
@@ -47,32 +47,17 @@ class DevicePicker:
     def _on_device(self, logits: torch.Tensor, params: Sequence[SamplingParams], rngs: Sequence) -> torch.Tensor:
         n, vocab = logits.shape
         assert n == len(params) == len(rngs)
-        temps = [0.0] * n
-        us = [0.0] * n
-        filtered = []
+        temps, us, ks, ps = [0.0] * n, [0.0] * n, [0] * n, [1.0] * n
+        greedy = True
         for i, p in enumerate(params):
             if p.greedy():
                 continue
+            greedy = False
             us[i] = rngs[i].uniform()
+            temps[i] = p.temperature
             if self._filters(p, vocab):
-                filtered.append(i)             # (temperature 0 for the first kernel: it leaves the argmax there)
-            else:
-                temps[i] = float(p.temperature)
-        if any(t > 0.0 for t in temps):
-            t_dev = torch.tensor(temps, dtype=torch.float32).to(logits.device, non_blocking=True)
-            u_dev = torch.tensor(us, dtype=torch.float64).to(logits.device, non_blocking=True)
-            ids = ops.sample(logits, t_dev, u_dev)
-        else:
-            ids = ops.argmax(logits)
-        if filtered:
-            dev = logits.device
-            # one upload for the rows' numbers: (row, top_k) as int32, (temperature) as float32, (u, top_p) as float64
-            ints = torch.tensor([filtered, [params[i].top_k for i in filtered]], dtype=torch.int32).to(dev, non_blocking=True)
-            temp = torch.tensor([params[i].temperature for i in filtered], dtype=torch.float32).to(dev, non_blocking=True)
-            reals = torch.tensor([[us[i] for i in filtered], [params[i].top_p for i in filtered]],
-                                 dtype=torch.float64).to(dev, non_blocking=True)
-            ops.sample_filtered(logits, ids, ints[0], temp, reals[0], ints[1], reals[1])
-        return ids
+                ks[i], ps[i] = p.top_k, p.top_p
+        return ops.argmax(logits) if greedy else ops.choose(logits, temps, us, ks, ps)
 
     def pick(self, logits: torch.Tensor, params: Sequence[SamplingParams], rngs: Sequence) -> List[int]:
         return [int(t) for t in self._on_device(logits, params, rngs).tolist()]
