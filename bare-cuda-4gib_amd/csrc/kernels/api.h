@@ -245,6 +245,8 @@ int bc4g_gemm_skinny_emit(const void* x, const void* w, float* out, const float*
                           float* emit_ssq, int emit_stride, int m, int n, int k, void* stream);
 int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, float eps,
                                const void* w, void* out, int epilogue, int m, int n, int k, void* stream);
+// out (bfloat16) = xielu(x w^T) with its two numbers pq, of the product rounded to bfloat16: at most 64 rows.
+int bc4g_gemm_skinny_xielu(const void* x, const void* w, void* out, const float* pq, int m, int n, int k, void* stream);
 }
 
 extern "C" {
@@ -259,8 +261,15 @@ int bc4g_probe_mfma(const void* operands, int iters, float* sink, int workgroups
 
 extern "C" {
 // x[r, :] += y[r, :] * rsqrt(mean(y[r]^2) + eps) * w: the norm after a sublayer, added to the float residual stream
-// (w float32, as it multiplies; y float32 or bfloat16).
-int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const float* w, int n_rows, int hidden, float eps, void* stream);
+// (w float32, as it multiplies; y float32 or bfloat16).  With next_w and out (null: neither), also the RMSNorm of the new x with that
+// scale: hidden a multiple of 8 up to 8192, everything on 16-byte boundaries.
+int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const float* w, const void* next_w, int next_w_dtype, float next_eps,
+                     void* out, int out_dtype, int n_rows, int hidden, float eps, void* stream);
+// out[r] = h + bias + (the causal convolution of h) with h = the RMSNorm of x[r], for a step in which request r brings row r alone:
+// bc4g_rmsnorm and bc4g_causal_conv (add_input) in one launch, the same bits.  w float32 [taps][hidden], state [slots, taps - 1, hidden]
+// in the output's type; 2 to 4 taps, hidden a multiple of 8 up to 4096, everything on 16-byte boundaries.
+int bc4g_rmsnorm_conv(const float* x, const void* norm_w, int norm_w_dtype, float eps, const float* w, const float* bias, void* out,
+                      void* state, int dtype, const int32_t* slots, int n_rows, int hidden, int taps, void* stream);
 // out = act(in) elementwise with act(z) = softplus(p) z^2 + z / 2 for z > 0 and (1/2 + softplus(q)) (e^z - 1 - z) + z / 2
 // otherwise; pq = (p, q) float32 on the device.
 int bc4g_xielu(const void* in, void* out, int dtype, const float* pq, long total, void* stream);
@@ -288,7 +297,7 @@ int bc4g_causal_conv(const void* in, int dtype, const float* in_bias, const floa
 // sigmoid(Ra u + ra_b) softplus(lam)), S_t = a S_(t-1) + sqrt(1 - a^2) sigmoid(Ri u + ri_b) u along every request's
 // rows, from state [slots, width] (float32) and back into it; out[t] = S_t * gelu_tanh(y[t] + y_bias).  A request's
 // rows are walked in chunks of 64 by threads of their own: chunk_a, chunk_b [S, ceil(most_rows / 64), width] and
-// before [S, width] are scratch (float32); most_rows: the most rows one request brings; y_row: elements from one row of y
+// before [S, width] are scratch (float32; null will do for most_rows up to 64); most_rows: the most rows one request brings; y_row: elements from one row of y
 // to the next.
 int bc4g_rglru_scan(const float* pre, const void* u, const void* y, int dtype, const float* ra_b, const float* ri_b,
                     const float* lam, const float* y_bias, void* out, float* state, float* chunk_a, float* chunk_b,

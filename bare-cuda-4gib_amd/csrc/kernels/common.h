@@ -118,6 +118,12 @@ int fail(const char* fmt, ...);
 int check_launch(const char* what);
 int compute_units();   // of the current device (256 if it cannot be asked)
 
+__device__ inline float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
+// softplus(p) z^2 + z / 2 for z > 0, (1/2 + softplus(q)) (e^z - 1 - z) + z / 2 otherwise: ap = softplus(p), aq = 1/2 + softplus(q).
+__device__ inline float xielu_f(float z, float ap, float aq) {
+  return z > 0.f ? ap * z * z + 0.5f * z : aq * (expm1f(z) - z) + 0.5f * z;
+}
+
 inline int ceil_div(long a, long b) { return static_cast<int>((a + b - 1) / b); }
 
 }  // namespace bc4g

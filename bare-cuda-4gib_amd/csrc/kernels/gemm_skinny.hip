@@ -29,7 +29,9 @@
 //            (below), together with parts of every row's sum of squares: the row's scale is worked out
 //            from the parts while the weights are on their way and multiplies the finished sum -- the
 //            norm costs neither a kernel of its own nor the staging of the float rows.
-// What goes out (EPI): bfloat16 or float stored; float added into the residual stream; SwiGLU,
+// What goes out (EPI): bfloat16 or float stored; bfloat16 after max(., 0)^2 or xIELU (8 rows,
+// 2,048 to 8,192: product with its norm inside 13.0 us and the activation behind it 5.5; normed before and activated here 8.8);
+// float added into the residual stream; SwiGLU,
 // when every 16 rows of w are eight gate rows followed by the eight up rows of the same outputs; or
 // rotary positions and the cache write, when w holds query, key and value heads with every head's
 // rows reordered in blocks of 16 (eight dimensions, then their rotation partners): queries are
@@ -51,7 +53,7 @@ constexpr int kThreads = kWaves * kWave;
 constexpr int kRedPad = 17;
 constexpr int kStagePad = 8;     // bf16 elements appended to each staged row of x
 
-enum Epilogue : int { kStoreBf16 = 0, kStoreF32 = 1, kAccumF32 = 2, kSwigluBf16 = 3, kRopeKvBf16 = 4, kSquaredReluBf16 = 6, kGegluBf16 = 7 };
+enum Epilogue : int { kStoreBf16 = 0, kStoreF32 = 1, kAccumF32 = 2, kSwigluBf16 = 3, kRopeKvBf16 = 4, kSquaredReluBf16 = 6, kGegluBf16 = 7, kXieluBf16 = 8 };
 // products whose weight holds blocks of eight gate rows and the eight up rows of the same outputs
 constexpr bool gated(int epi) { return epi == kSwigluBf16 || epi == kGegluBf16; }
 
@@ -79,7 +81,7 @@ struct SkinnyArgs {
   // prenormed x (plain mode): parts [ssq_blocks][ssq_stride] of the rows' sums of squares (null: x as it is)
   const float* ssq_parts;
   int ssq_blocks, ssq_stride;
-  // kAccumF32: a number a column that joins every row's sums (null: none)
+  // kAccumF32: a number a column that joins every row's sums (null: none); kXieluBf16: the activation's two numbers
   const float* bias;
   // kAccumF32: what the RMSNorm after this product needs (emit_g null: nothing)
   const void* emit_g;       // [n] its scale, bfloat16 or float (emit_g_f32)
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
     const long row0 = static_cast<long>(blockIdx.y) * args.rows_per_block;
     a.m = min(args.rows_per_block, args.m - static_cast<int>(row0));
     a.x = static_cast<const bf16_t*>(args.x) + row0 * args.k;
-    if constexpr (EPI == kStoreBf16 || EPI == kSquaredReluBf16) a.out = static_cast<bf16_t*>(args.out) + row0 * args.n;
+    if constexpr (EPI == kStoreBf16 || EPI == kSquaredReluBf16 || EPI == kXieluBf16) a.out = static_cast<bf16_t*>(args.out) + row0 * args.n;
     else if constexpr (gated(EPI)) a.out = static_cast<bf16_t*>(args.out) + row0 * (args.n / 2);
     else if constexpr (EPI == kRopeKvBf16) {
       a.out = static_cast<bf16_t*>(args.out) + row0 * args.rope.n_heads * args.rope.head_dim;
@@ -182,6 +184,9 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
       if (a.bias != nullptr && live) prev[j] += a.bias[gn];
     }
   }
+
+  float xielu_p = 0.f, xielu_q = 0.f;
+  if constexpr (EPI == kXieluBf16) xielu_p = softplus_f(a.bias[0]), xielu_q = 0.5f + softplus_f(a.bias[1]);
 
   // The rotation a thread will apply in the epilogue (its output's angle: position and pair are
   // known now) and the place in the cache it will write to are worked out while the weights are
@@ -481,6 +486,9 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
     } else if constexpr (EPI == kSquaredReluBf16) {
       const float z = fmaxf(sum, 0.f);
       static_cast<bf16_t*>(a.out)[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(z * z);
+    } else if constexpr (EPI == kXieluBf16) {
+      const float z = to_float(from_float<bf16_t>(sum));       // as a kernel behind the product would find it
+      static_cast<bf16_t*>(a.out)[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(xielu_f(z, xielu_p, xielu_q));
     } else if constexpr (EPI == kStoreF32) {
       static_cast<float*>(a.out)[static_cast<long>(row) * a.n + gn] = sum;
     } else if constexpr (EPI == kAccumF32) {
@@ -669,6 +677,16 @@ extern "C" int bc4g_gemm_skinny(const void* x, const void* w, void* out, const f
   SkinnyArgs a = plain_args(x, w, out, m, n, k);
   a.bias = bias;
   return launch_epilogue<kPlain>(a, epilogue, static_cast<hipStream_t>(stream));
+}
+
+// out (bfloat16) = xielu(x w^T), pq its two numbers.
+extern "C" int bc4g_gemm_skinny_xielu(const void* x, const void* w, void* out, const float* pq, int m, int n, int k, void* stream) {
+  if (int e = check_common("gemm_skinny_xielu", m, 64, n, k, kXieluBf16)) return e;
+  BC4G_REQUIRE(x && w && out && pq, "gemm_skinny_xielu: a tensor is missing");
+  if (m == 0) return 0;
+  SkinnyArgs a = plain_args(x, w, out, m, n, k);
+  a.bias = pq;
+  return launch<kXieluBf16, kPlain>(a, static_cast<hipStream_t>(stream));
 }
 
 // out (the float residual stream, [m, n]) += x w^T + bias (null: none), and what the RMSNorm after it needs: emit_x

@@ -791,6 +791,21 @@ def gemm_fast(a: torch.Tensor, w, out_dtype=None,
     return out
 
 
+def gemm_xielu(a: torch.Tensor, w, pq: torch.Tensor) -> Optional[torch.Tensor]:
+    """xielu(a w^T) in bfloat16 with the activation in the streaming kernel's epilogue (to the product rounded to bfloat16, as
+    the kernel behind a product would find it), where that kernel takes the product; else None."""
+    w, packed = _weight(w)
+    if not _fast_operands(a, w) or packed is None or a.shape[0] > SKINNY_MAX_ROWS or not streams_weights(a.shape[0], *w.shape):
+        return None
+    _dev("gemm_xielu", a, w, pq)
+    _f32("gemm_xielu", "pq", pq, (2,))
+    m, k = a.shape
+    n = w.shape[0]
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
+    library.call("bc4g_gemm_skinny_xielu", _ptr(a), _ptr(packed), _ptr(out), _ptr(pq), m, n, k, _stream(), cost=_skinny_cost(m, n, k, 2, 2))
+    return out
+
+
 def _normed_rows_fit(n_rows: int, k: int, n: int = 0) -> bool:
     """Whether an RMSNorm before a product of these rows is fused into the streaming kernel: few rows (the plan's
     fused_norm_rows: at most 8), which fit LDS rounded up to 4 with k + 8 bfloat16 each (8 rows do up to k = 6,136)."""
@@ -1356,17 +1371,57 @@ def _f32(what: str, name: str, t: Optional[torch.Tensor], shape) -> None:
         raise KernelError(f"{what}: {name} must be float32 {tuple(shape)}, got {t.dtype} {tuple(t.shape)}")
 
 
-def rmsnorm_add(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+def _norms_whole_rows(hidden: int, *tensors: Optional[torch.Tensor]) -> bool:
+    """Whether the kernels that hold a row in registers take this width and these addresses."""
+    return hidden % 8 == 0 and hidden <= 8192 and not any(t.data_ptr() % 16 for t in tensors if t is not None)
+
+
+def rmsnorm_add(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float, next_norm=None) -> Optional[torch.Tensor]:
     """x += y * rsqrt(mean(y^2) + eps) * weight, row by row, in place on the float residual stream x [T, H];
-    y [T, H] float32 or bfloat16, weight float32 [H] (as it multiplies)."""
+    y [T, H] float32 or bfloat16, weight float32 [H] (as it multiplies).  Returns x.  With ``next_norm`` (scale, eps, dtype) the
+    RMSNorm of the new x is made in the same kernel and returned instead, where the kernel takes the width (else None is)."""
     _dev("rmsnorm_add", x, y, weight)
     if x.dtype != torch.float32 or x.dim() != 2 or tuple(y.shape) != tuple(x.shape):
         raise KernelError(f"rmsnorm_add: x must be float32 [T, H] and y of its shape, got {x.dtype} {tuple(x.shape)} and {tuple(y.shape)}")
     n, hidden = x.shape
     _f32("rmsnorm_add", "weight", weight, (hidden,))
-    library.call("bc4g_rmsnorm_add", _ptr(x), _ptr(y), _code(y, "rmsnorm_add"), _ptr(weight), n, hidden, float(eps), _stream(),
-                 cost=lambda: (5.0 * n * hidden, n * hidden * (8 + y.element_size())))
-    return x
+    scale = out = None
+    next_eps, dtypes = 0.0, (0, 0)
+    if next_norm is not None and _norms_whole_rows(hidden, x, y, weight, next_norm[0]):
+        scale, next_eps = next_norm[0], float(next_norm[1])
+        _dev("rmsnorm_add", scale)
+        if tuple(scale.shape) != (hidden,):
+            raise KernelError(f"rmsnorm_add: the next norm's scale must be [{hidden}], got {tuple(scale.shape)}")
+        out = torch.empty((n, hidden), dtype=next_norm[2], device=x.device)
+        dtypes = _code(scale, "rmsnorm_add"), _code(out, "rmsnorm_add")
+    library.call("bc4g_rmsnorm_add", _ptr(x), _ptr(y), _code(y, "rmsnorm_add"), _ptr(weight), _ptr(scale), dtypes[0], next_eps, _ptr(out), dtypes[1],
+                 n, hidden, float(eps), _stream(), cost=lambda: (5.0 * n * hidden, n * hidden * (8 + y.element_size())))
+    return x if next_norm is None else out
+
+
+def rmsnorm_conv(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, out_dtype: torch.dtype, weight: torch.Tensor, state: torch.Tensor,
+                 ctx, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """h + causal_conv(h) with h = rmsnorm(x) in one kernel, for a step in which every request brings one row (the state moves
+    on as causal_conv moves it, bit for bit); None where the kernel does not take the step, the width (a multiple of 8 up to 4,096)
+    or the taps (2 to 4)."""
+    taps, hidden = weight.shape
+    if (ctx.n_tokens != ctx.n_seqs or ctx.n_tokens == 0 or x.dim() != 2 or x.dtype != torch.float32 or not 2 <= taps <= 4 or hidden > 4096 or state.dtype != out_dtype
+            or not _norms_whole_rows(hidden, x, norm_weight, weight, state, bias)):
+        return None
+    _dev("rmsnorm_conv", x, norm_weight, weight, state, bias)
+    if tuple(x.shape) != (ctx.n_tokens, hidden) or tuple(norm_weight.shape) != (hidden,) or tuple(state.shape[1:]) != (taps - 1, hidden):
+        raise KernelError(f"rmsnorm_conv: x {tuple(x.shape)}, norm scale {tuple(norm_weight.shape)} and state {tuple(state.shape)} do not go with {taps} taps of {hidden}")
+    _f32("rmsnorm_conv", "weight", weight, (taps, hidden))
+    _f32("rmsnorm_conv", "bias", bias, (hidden,))
+    if max(ctx.seq_slots, default=0) >= state.shape[0]:
+        raise KernelError(f"rmsnorm_conv: a slot beyond the state's {state.shape[0]}")
+    n = ctx.n_tokens
+    _check_grouping("rmsnorm_conv", ctx, n)
+    out = torch.empty((n, hidden), dtype=out_dtype, device=x.device)
+    library.call("bc4g_rmsnorm_conv", _ptr(x), _ptr(norm_weight), _code(norm_weight, "rmsnorm_conv"), float(eps), _ptr(weight), _ptr(bias), _ptr(out),
+                 _ptr(state), _code(out, "rmsnorm_conv"), _ptr(ctx.seq_slots_dev), n, hidden, taps, _stream(),
+                 cost=lambda: ((3.0 + 2 * taps) * n * hidden, n * hidden * (4 + (2 * taps - 1) * out.element_size())))
+    return out
 
 
 def xielu(z: torch.Tensor, pq: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -1481,10 +1536,11 @@ def rglru(u: torch.Tensor, y: torch.Tensor, w_gates: torch.Tensor, ra_b: torch.T
     heads_gemm(u.view(t, blocks, bs), w_gates, pre, k=bs, n=2 * bs)
     most = max(int(ctx.seq_start[s + 1] - ctx.seq_start[s]) for s in range(ctx.n_seqs))
     chunks = -(-most // RGLRU_CHUNK)
-    scratch = torch.empty((2 * chunks + 1, ctx.n_seqs, w), dtype=torch.float32, device=u.device)
+    scratch = torch.empty((2 * chunks + 1, ctx.n_seqs, w), dtype=torch.float32, device=u.device) if chunks > 1 else None
     out = torch.empty_like(u)
+    notes = (scratch[:chunks], scratch[chunks:2 * chunks], scratch[2 * chunks]) if chunks > 1 else (None, None, None)
     library.call("bc4g_rglru_scan", _ptr(pre), _ptr(u), _ptr(y), _code(y, "rglru"), _ptr(ra_b), _ptr(ri_b), _ptr(lam), _ptr(y_bias),
-                 _ptr(out), _ptr(state), _ptr(scratch[:chunks]), _ptr(scratch[chunks:2 * chunks]), _ptr(scratch[2 * chunks]),
+                 _ptr(out), _ptr(state), *map(_ptr, notes),
                  _ptr(ctx.seq_start_dev), _ptr(ctx.seq_slots_dev), t, ctx.n_seqs, most, w, blocks, y_row, _stream(),
                  cost=lambda: (40.0 * t * w, t * w * (16 + 5 * u.element_size())))
     return out

@@ -157,19 +157,28 @@ class SandwichBlock(Part):
         return Bundle((("mixer", self.mixer.cache_spec()), ("conv", self.mixer_conv.cache_spec())))
 
     def forward(self, x, ctx, cache, writes: bool = True) -> None:
-        h = self.mixer_norm.forward(x, ctx)
-        mixer_cache = cache
+        mixer_cache, h = cache, None
         if self.mixer_conv is not None:
-            h = self.mixer_conv.forward(h, ctx, cache.conv, add_input=True)
             mixer_cache = cache.mixer
+            if hasattr(self.mixer_conv, "behind"):             # (norm and convolution in one kernel where there is one)
+                h = self.mixer_conv.behind(self.mixer_norm, x, ctx, cache.conv)
+        if h is None:
+            h = self.mixer_norm.forward(x, ctx)
+            if self.mixer_conv is not None:
+                h = self.mixer_conv.forward(h, ctx, cache.conv, add_input=True)
         y = self._sum_for(self.mixer, x)
         self.mixer.forward(h, ctx, mixer_cache, y, writes)
-        self.mixer_post_norm.add_to(x, self._sum_of(y))
+        h = None
+        if self.ffn is not None and hasattr(self.mixer_post_norm, "add_and_norm"):     # (one kernel where there is one)
+            h = self.mixer_post_norm.add_and_norm(x, self._sum_of(y), self.ffn_norm)
+        else:
+            self.mixer_post_norm.add_to(x, self._sum_of(y))
         if self.ffn is not None:
             y = self._sum_for(self.ffn, x)
             # (a feed-forward that says so gets the norm not yet computed: its first product absorbs it for few rows)
-            lazy = getattr(self.ffn, "accepts_lazy_norm", False)
-            self.ffn.forward(Normed(x, self.ffn_norm, ctx) if lazy else self.ffn_norm.forward(x, ctx), ctx, y)
+            if h is None:
+                h = Normed(x, self.ffn_norm, ctx) if getattr(self.ffn, "accepts_lazy_norm", False) else self.ffn_norm.forward(x, ctx)
+            self.ffn.forward(h, ctx, y)
             self.ffn_post_norm.add_to(x, self._sum_of(y))
 
     @staticmethod

@@ -10,6 +10,7 @@ from ..csrc import ops
 from ..errors import ConfigError
 from ..weights.loader import WeightSpec
 from .base import Part, register_part
+from .norm import RMSNorm
 
 
 class CausalConv(Part):
@@ -42,6 +43,13 @@ class CausalConv(Part):
     def forward(self, v: torch.Tensor, ctx, view, add_input: bool = False, in_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         return ops.causal_conv(v, self.w, view.tail if self.taps > 1 else None, ctx, in_bias=in_bias, out_bias=self.b,
                                add_input=add_input)
+
+    def behind(self, norm, x: torch.Tensor, ctx, view) -> Optional[torch.Tensor]:
+        """h + the convolution of h with h = norm(x), in one kernel where there is one for the step; else None."""
+        scale = norm.fusable() if isinstance(norm, RMSNorm) else None
+        if scale is None or self.taps == 1:
+            return None
+        return ops.rmsnorm_conv(x, scale[0], scale[1], norm.out_dtype, self.w, view.tail, ctx, bias=self.b)
 
 
 class TokenShift(Part):

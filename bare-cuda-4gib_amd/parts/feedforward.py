@@ -9,7 +9,7 @@ from ..csrc import ops
 from ..errors import ConfigError
 from ..weights.loader import WeightSpec
 from .base import Part, register_part
-from .linear import linear, linear_squared_relu, linear_swiglu
+from .linear import linear, linear_squared_relu, linear_swiglu, linear_xielu
 
 
 class SwiGLU(Part):
@@ -82,8 +82,7 @@ class DenseXIELU(Part):
         self.act_dtype = rt.act_dtype
 
     def forward(self, h, ctx, residual) -> None:
-        z = linear(h, self.w_up, out_dtype=self.act_dtype)
-        linear(ops.xielu(z, self.pq, out=z), self.w_down, accumulate_into=residual, ctx=ctx)
+        linear(linear_xielu(h, self.w_up, self.pq, self.act_dtype), self.w_down, accumulate_into=residual, ctx=ctx)
 
 
 class ClampedGLU(Part):

@@ -93,6 +93,19 @@ def linear_squared_relu(x: Union[torch.Tensor, Normed], w, out_dtype: torch.dtyp
     return ops.squared_relu(z, out=z)
 
 
+def linear_xielu(x: Union[torch.Tensor, Normed], w, pq: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
+    """xielu(x W^T) with its two numbers pq: inside the product's kernel where few rows stream the weights, else by a kernel
+    behind it."""
+    if out_dtype == torch.bfloat16 and not (isinstance(x, Normed) and x.pre is not None):
+        if isinstance(x, Normed):
+            x = x.tensor()
+        fast = ops.gemm_xielu(x, w, pq)
+        if fast is not None:
+            return fast
+    z = linear(x, w, out_dtype=out_dtype)
+    return ops.xielu(z, pq, out=z)
+
+
 def linear_swiglu(x: Union[torch.Tensor, Normed], w_gate_up, interleaved: bool = False, act: str = "silu") -> torch.Tensor:
     """act(x Wg^T) * (x Wu^T) (``act``: "silu", or "gelu_tanh", the gelu written with tanh) for w_gate_up = gate rows followed by up rows, or (interleaved)
     blocks of eight gate rows and the eight up rows of the same outputs."""

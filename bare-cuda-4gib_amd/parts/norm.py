@@ -4,7 +4,7 @@ counted from it: y = x * rsqrt(...) * (offset + w) -- a weight stored around zer
 is cut into that many equal runs of neighbouring channels, every run is brought to unit mean square by itself, and one weight spans the row."""
 from __future__ import annotations
 
-from typing import Dict
+from typing import Dict, Optional
 
 import torch
 
@@ -36,11 +36,22 @@ class RMSNorm(Part):
 
     def add_to(self, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
         """x += norm(y), in place on the float32 residual stream: the norm after a sublayer."""
+        return ops.rmsnorm_add(x, y, self._adds_as(), self.eps)
+
+    def add_and_norm(self, x: torch.Tensor, y: torch.Tensor, following) -> Optional[torch.Tensor]:
+        """add_to, and where one kernel can make it too the norm ``following`` of the new x -- else None."""
+        scale = following.fusable() if isinstance(following, RMSNorm) else None
+        if scale is None:
+            self.add_to(x, y)
+            return None
+        return ops.rmsnorm_add(x, y, self._adds_as(), self.eps, next_norm=(*scale, following.out_dtype))
+
+    def _adds_as(self) -> torch.Tensor:
         if self.groups != 1:
             raise ConfigError("rmsnorm: a norm in groups is not added to the stream by a kernel of its own")
         if self._multiplier is None:
             self._multiplier = self.weight.to(torch.float32).contiguous()
-        return ops.rmsnorm_add(x, y, self._multiplier, self.eps)
+        return self._multiplier
 
     def fusable(self):
         """What a product needs to absorb this norm: (scale vector, eps); None for a norm in groups, which no product absorbs."""
