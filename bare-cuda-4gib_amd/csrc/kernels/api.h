@@ -142,7 +142,9 @@ extern "C" {
 // 3 SwiGLU: every 16 rows of w are eight gate rows and the eight up rows of the same outputs
 // (n = 2 * inter), out bfloat16 [m, inter] = silu(gate) * up; 6 store max(sum, 0)^2 as bfloat16 [m, n]; 7 as 3 with
 // the gelu written with tanh for the silu.  bias [n] (float32; null: none) joins the sums of epilogue 2.
-int bc4g_gemm_skinny(const void* x, const void* w, void* out, const float* bias, int epilogue, int m, int n, int k, void* stream);
+// halves: two workgroups share a block of 16 rows of w (at most 8 rows of x, epilogues 0 to 2; the same bits).
+int bc4g_gemm_skinny(const void* x, const void* w, void* out, const float* bias, int epilogue, int m, int n, int k, int halves,
+                     void* stream);
 }
 
 extern "C" {
@@ -228,7 +230,7 @@ extern "C" {
 // With ssq_parts (g null) x is bfloat16(residual * g) and the rows' scales come from the parts, as
 // in bc4g_gemm_skinny_prenormed.
 int bc4g_gemm_skinny_qkv(const void* x, const void* g, int g_dtype, float eps, const float* ssq_parts, int ssq_blocks,
-                         int ssq_stride, const void* w, void* q_out,
+                         int ssq_stride, int ssq_halves, const void* w, void* q_out,
                          const int32_t* positions, const int32_t* slot_map, void* k_cache, void* v_cache,
                          int m, int k, int n_heads, int n_kv_heads, int head_dim, int rotary_dim, float theta,
                          int page_tokens, int write_kv, void* stream);
@@ -241,9 +243,11 @@ extern "C" {
 // squares.  bc4g_gemm_skinny_prenormed takes such an x (k = this n) and the parts instead of a norm:
 // out = rmsnorm(residual) w^T, the row's rsqrt(sum of the parts / k + eps) applied to the finished
 // sums; epilogues of bc4g_gemm_skinny except the adding one.
+// With halves (at most 8 rows) two workgroups share a block and emit_ssq is [ceil(n / 16)][emit_stride][2], the parts of a block's
+// halves, which the products that take it are told by ssq_halves.
 int bc4g_gemm_skinny_emit(const void* x, const void* w, float* out, const float* bias, const void* g, int g_dtype, void* emit_x,
-                          float* emit_ssq, int emit_stride, int m, int n, int k, void* stream);
-int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, float eps,
+                          float* emit_ssq, int emit_stride, int m, int n, int k, int halves, void* stream);
+int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, int ssq_halves, float eps,
                                const void* w, void* out, int epilogue, int m, int n, int k, void* stream);
 // out (bfloat16) = xielu(x w^T) with its two numbers pq, of the product rounded to bfloat16: at most 64 rows.
 int bc4g_gemm_skinny_xielu(const void* x, const void* w, void* out, const float* pq, int m, int n, int k, void* stream);

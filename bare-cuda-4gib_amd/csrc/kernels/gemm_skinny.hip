@@ -81,12 +81,14 @@ struct SkinnyArgs {
   // prenormed x (plain mode): parts [ssq_blocks][ssq_stride] of the rows' sums of squares (null: x as it is)
   const float* ssq_parts;
   int ssq_blocks, ssq_stride;
+  int ssq_halves;           // the parts are pairs, [ssq_blocks][ssq_stride][2]
+  int halves;               // host: two workgroups a block (see launch)
   // kAccumF32: a number a column that joins every row's sums (null: none); kXieluBf16: the activation's two numbers
   const float* bias;
   // kAccumF32: what the RMSNorm after this product needs (emit_g null: nothing)
   const void* emit_g;       // [n] its scale, bfloat16 or float (emit_g_f32)
   bf16_t* emit_x;           // [m, n] bfloat16(new residual * g)
-  float* emit_ssq;          // [ceil(n / 16)][emit_stride]: block b's part of row r's sum of squares
+  float* emit_ssq;          // [ceil(n / 16)][emit_stride]: block b's part of row r's sum of squares (with halves [..][2]: of its halves)
   int emit_g_f32, emit_stride;
   RopeKvArgs rope;          // kRopeKvBf16 only
 };
@@ -95,10 +97,12 @@ __device__ inline uint32_t pack2(float a, float b) {
   return static_cast<uint32_t>(bf16_bits_from_float(a)) | (static_cast<uint32_t>(bf16_bits_from_float(b)) << 16);
 }
 
-template <int MT, int EPI, int XMODE, int U>
+// MT tiles of 16 rows of x; U k-steps of 32 a batch; ROWS: 16, or 8 where there are no more rows than that (plain x: half the
+// loads and LDS writes for x); HALF: two workgroups share a weight block, each with eight of its outputs (see launch).
+template <int MT, int EPI, int XMODE, int U, int ROWS = 16, bool HALF = false>
 // (The normed form keeps to 80 registers, so that three workgroups share a CU and all the blocks of
 // a 5,632 x 2 wide gate-up matrix are in flight at once.)
-__global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) ? 6 : 4) void gemm_skinny_kernel(const SkinnyArgs args) {
+__global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) ? 6 : U == 8 ? 2 : 4) void gemm_skinny_kernel(const SkinnyArgs args) {
   constexpr bool kNormed = XMODE != kPlain;
   // Where the weight blocks are too few to occupy the CUs, the rows are shared out over blockIdx.y:
   // such a workgroup sees its own rows only, as if they were the whole batch.
@@ -123,12 +127,14 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
   constexpr bool kTurned = !kNormed;                      // x reaches operand order through LDS
   constexpr int kPieces = 4 * U;                       // 16-byte pieces of a row in one batch of k-steps
   static_assert(!kNormed || MT == 1, "the fused norm handles one tile of rows");
+  static_assert(ROWS == 16 || (ROWS == 8 && MT == 1 && !kNormed), "eight rows: one tile of plain rows");
+  static_assert(!HALF || (MT == 1 && XMODE == kPlain && !gated(EPI) && EPI != kRopeKvBf16), "half blocks: few plain rows, unpaired outputs");
   static_assert(!kTurned || 64 % kPieces == 0, "a load instruction covers whole rows of a batch");
   static_assert(!kTurned || kPieces >= 8, "the buffer's swizzle (piece ^ row % 8) must stay inside a row's pieces");
   // The waves' partial sums, and before them (kTurned) every wave's buffer for x: the same memory.
   typedef float Red[MT][16][kRedPad];
   constexpr int kRedBytes = kWaves * static_cast<int>(sizeof(Red));
-  constexpr int kTurnBytes = kTurned ? kWaves * MT * 16 * kPieces * 16 : 0;
+  constexpr int kTurnBytes = kTurned ? kWaves * MT * ROWS * kPieces * 16 : 0;
   __shared__ __align__(16) unsigned char pool[kRedBytes > kTurnBytes ? kRedBytes : kTurnBytes];
   Red* red = reinterpret_cast<Red*>(pool);
   __shared__ float ssq_row[16];
@@ -136,7 +142,8 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // uniform: k ranges and bases stay scalar
   const int col = lane % 16, grp = lane / 16;
-  const int n0 = blockIdx.x * 16;
+  const int wblock_index = HALF ? blockIdx.x / 2 : blockIdx.x, half = HALF ? blockIdx.x % 2 : 0;
+  const int n0 = wblock_index * 16 + 8 * half;
   const int k = a.k, m = a.m;
 
   // every wave's part of k starts on a cache line of x (64 elements), whatever the number of rows:
@@ -152,8 +159,9 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
   // this workgroup's block of 16 rows in the packed weights: k-step ks at wblock + ks * 512 elements
   // (a scalar base and a 32-bit lane offset, so the loads of a batch differ in their scalar part only)
   const int ksteps_total = (k + 31) / 32;
-  const bf16_t* wblock = a.w + static_cast<long>(blockIdx.x) * ksteps_total * (kWave * 8);
-  const int wlane = lane * 8;
+  const bf16_t* wblock = a.w + static_cast<long>(wblock_index) * ksteps_total * (kWave * 8);
+  // (half a block: the lanes of the other eight rows ask for what their neighbours ask for, and their results are not used)
+  const int wlane = (HALF ? (lane & ~8) | (8 * half) : lane) * 8;
 
   // where this lane's B operand comes from
   const bf16_t* xptr[MT];
@@ -172,14 +180,16 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
 
   // The float sums that the product is added to (the residual stream) are asked for now, not
   // after the weights: item j of a thread is output (threadIdx.x + j * kThreads) of the block.
-  constexpr int kAccItems = (MT * 256 + kThreads - 1) / kThreads;
+  constexpr bool kPaired = gated(EPI) || EPI == kRopeKvBf16;   // columns nl and nl + 8 belong together
+  constexpr int kCols = kPaired || HALF ? 8 : 16;
+  constexpr int kAccItems = (MT * 16 * kCols + kThreads - 1) / kThreads;
   float prev[kAccItems];
   if constexpr (EPI == kAccumF32) {
 #pragma unroll
     for (int j = 0; j < kAccItems; ++j) {
       const int idx = threadIdx.x + j * kThreads;
-      const int row = idx / 16, gn = n0 + idx % 16;
-      const bool live = idx < MT * 256 && row < m && gn < a.n;
+      const int row = idx / kCols, gn = n0 + idx % kCols;
+      const bool live = idx < MT * 16 * kCols && row < m && gn < a.n;
       prev[j] = live ? static_cast<const float*>(a.out)[static_cast<long>(row) * a.n + gn] : 0.f;
       if (a.bias != nullptr && live) prev[j] += a.bias[gn];
     }
@@ -245,7 +255,21 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
             for (int i = 0; i < kAhead; ++i) ss += part[i];      // (in ascending order; a part that is not there adds 0)
           }
         };
-        if ((U == 4 || gated(EPI)) && m <= 8) chain(std::integral_constant<int, 16>{});
+        if (a.ssq_halves) {
+          // (left by half blocks: the two halves of a part side by side, their sum the part itself)
+          const float2* p2 = reinterpret_cast<const float2*>(a.ssq_parts) + row;
+          constexpr int kAhead = 8;
+          for (int b0 = j0; b0 < a.ssq_blocks; b0 += kAhead * kPartSums) {
+            float2 part[kAhead];
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) {
+              const int b = b0 + i * kPartSums;
+              part[i] = b < a.ssq_blocks ? p2[static_cast<long>(b) * a.ssq_stride] : make_float2(0.f, 0.f);
+            }
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) ss += part[i].x + part[i].y;
+          }
+        } else if ((U == 4 || gated(EPI)) && m <= 8) chain(std::integral_constant<int, 16>{});
         else chain(std::integral_constant<int, 4>{});
       }
       part_sum[j0][row] = ss;
@@ -258,7 +282,8 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
   constexpr int kRowsPerLoad = kTurned ? 64 / kPieces : 1;
   const int turn_row = lane / kPieces, turn_piece = lane % kPieces;
   const bf16_t* turn_src = static_cast<const bf16_t*>(a.x) + static_cast<long>(turn_row) * k + turn_piece * 8;
-  uint4* turn = reinterpret_cast<uint4*>(pool) + wave * (MT * 16 * kPieces);
+  uint4* turn = reinterpret_cast<uint4*>(pool) + wave * (MT * ROWS * kPieces);
+  constexpr int kXLoads = kTurned ? MT * U * ROWS / 16 : 1;      // a batch's loads of x, kRowsPerLoad rows each
 
   struct Batch {
     uint4 w[U];
@@ -275,10 +300,10 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
   // 128 a wave has (spilled, the q|k|v product of 64 rows and 4,096 columns took 127 instead of 44 us).
   constexpr bool kPingPong = MT == 2;
   const int last_row_offset = (m - 1) * k;              // (m <= 64 rows: an int)
-  int turn_offset[kTurned ? MT * U : 1];
+  int turn_offset[kXLoads];
   if constexpr (kTurned) {
 #pragma unroll
-    for (int i = 0; i < MT * U; ++i) turn_offset[i] = min((turn_row + i * kRowsPerLoad) * k, last_row_offset) + turn_piece * 8;
+    for (int i = 0; i < kXLoads; ++i) turn_offset[i] = min((turn_row + i * kRowsPerLoad) * k, last_row_offset) + turn_piece * 8;
   }
   const bf16_t* xptr_any[MT];                           // (the row itself, or the last row for rows past m)
 #pragma unroll
@@ -294,7 +319,7 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
     }
     if constexpr (kTurned) {
 #pragma unroll
-      for (int i = 0; i < MT * U; ++i) b.x[i / U][i % U] = load16(static_cast<const bf16_t*>(a.x) + turn_offset[i] + k0);
+      for (int i = 0; i < kXLoads; ++i) b.x[i / U][i % U] = load16(static_cast<const bf16_t*>(a.x) + turn_offset[i] + k0);
     }
   };
   auto load = [&](Batch& b, int k0) {
@@ -311,7 +336,7 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
     if constexpr (kTurned) {
       const bool k_ok = k0 + turn_piece * 8 < k_end;
 #pragma unroll
-      for (int i = 0; i < MT * U; ++i) {
+      for (int i = 0; i < kXLoads; ++i) {
         const bool ok = k_ok && turn_row + i * kRowsPerLoad < m;
         b.x[i / U][i % U] = ok ? load16(turn_src + static_cast<long>(i * kRowsPerLoad) * k + k0) : zero16();
       }
@@ -320,7 +345,7 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
   auto compute = [&](const Batch& b, int k0) {
     if constexpr (kTurned) {
 #pragma unroll
-      for (int i = 0; i < MT * U; ++i) {
+      for (int i = 0; i < kXLoads; ++i) {
         const int row = turn_row + i * kRowsPerLoad;
         turn[row * kPieces + (turn_piece ^ (row % 8))] = b.x[i / U][i % U];
       }
@@ -338,7 +363,7 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
           const int kk = k0 + 32 * u + 8 * grp;
           xb = kk < k_end ? *reinterpret_cast<const uint4*>(xptr[t] + kk) : zero16();
         } else if constexpr (kTurned) {
-          xb = turn[(t * 16 + col) * kPieces + ((4 * u + grp) ^ (col % 8))];
+          xb = turn[(t * 16 + (ROWS == 8 ? col % 8 : col)) * kPieces + ((4 * u + grp) ^ (col % 8))];
         } else {
           xb = b.x[t][u];
         }
@@ -447,8 +472,6 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
     for (int r = 0; r < 4; ++r) red[wave][t][4 * grp + r][col] = acc[t][r];
   __syncthreads();
 
-  constexpr bool kPaired = gated(EPI) || EPI == kRopeKvBf16;   // columns nl and nl + 8 belong together
-  constexpr int kCols = kPaired ? 8 : 16;
   constexpr int kItems = (MT * 16 * kCols + kThreads - 1) / kThreads;
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
@@ -496,7 +519,7 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
       if (live) static_cast<float*>(a.out)[static_cast<long>(row) * a.n + gn] = nv;
       if (a.emit_g != nullptr) {
         // for the RMSNorm that follows: bf16(new residual * g), and this block's part of the row's sum
-        // of squares (a row's 16 columns lie in 16 neighbouring lanes)
+        // of squares (a row's 16 columns, or eight of half a block, lie in as many neighbouring lanes)
         float sq = 0.f;
         if (live) {
           const float g = a.emit_g_f32 ? static_cast<const float*>(a.emit_g)[gn]
@@ -505,8 +528,8 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
           sq = nv * nv;
         }
 #pragma unroll
-        for (int off = 1; off < 16; off <<= 1) sq += __shfl_xor(sq, off, kWave);
-        if (nl == 0 && idx < MT * 256 && row < m) a.emit_ssq[static_cast<long>(blockIdx.x) * a.emit_stride + row] = sq;
+        for (int off = 1; off < kCols; off <<= 1) sq += __shfl_xor(sq, off, kWave);
+        if (nl == 0 && idx < MT * 16 * kCols && row < m) a.emit_ssq[(static_cast<long>(wblock_index) * a.emit_stride + row) * (HALF ? 2 : 1) + half] = sq;
       }
     } else if constexpr (gated(EPI)) {
       // block b = n0 / 16 holds gates and ups of outputs 8b .. 8b + 7
@@ -585,12 +608,35 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
       tiles = (b.rows_per_block + 15) / 16;
       grid.y = 2;
     }
+    if (a.m <= kSplitMinRows) {
+      // Few rows.  What bounds a weight of few blocks (2,048 x 5,632: 128 of 180 KB) is how many of its bytes are on their way
+      // at once, so with at most three blocks for every four CUs a wave asks for eight k-steps together (two workgroups of
+      // four would not share a CU anyway), and with at most a block for every other CU and a long k two workgroups
+      // share a block, each with eight of its outputs (b.halves; the lanes of the other eight rows repeat
+      // theirs, the same sums in the same order).  One row, weights from memory: 2,048 x 5,632 8.6 -> 7.3 us, 2,048 x
+      // 2,048 4.6 -> 4.3, 2,560 x 2,048 4.75 -> 4.5; a decode step at TinyLlama's sizes 0.846 -> 0.806 ms for one request, 0.949 ->
+      // 0.894 for 4, 0.99 -> 0.959 for 8 (eight k-steps from 9 rows on: 16 requests 1.054 -> 1.082, so only here).
+      // (Four k-steps for more blocks: 4,096 x 4,096 takes 8.3 us, with eight 8.5.)
+      // (a wide product's many workgroups, more than two a CU: with fewer k-steps in flight each they
+      // need half the registers, and all of them are on the CUs at once -- the gate-up product of 8
+      // rows after a prepared norm: a decode step 1.020 -> 0.990 ms)
+      const int blocks = static_cast<int>(grid.x);
+      if constexpr (EPI == kAccumF32 || EPI == kStoreF32 || EPI == kStoreBf16) {
+        if (b.halves) {
+          grid.x *= 2;
+          gemm_skinny_kernel<1, EPI, XMODE, 8, 8, true><<<grid, block, 0, s>>>(b);
+          return check_launch("gemm_skinny");
+        }
+      }
+      if (blocks > 2 * compute_units()) gemm_skinny_kernel<1, EPI, XMODE, 2, 8><<<grid, block, 0, s>>>(b);
+      else if (4 * blocks <= 3 * compute_units()) gemm_skinny_kernel<1, EPI, XMODE, 8, 8><<<grid, block, 0, s>>>(b);
+      else gemm_skinny_kernel<1, EPI, XMODE, 4, 8><<<grid, block, 0, s>>>(b);
+      return check_launch("gemm_skinny");
+    }
     switch (tiles) {
       // k-steps per batch chosen so that two batches of operands fit 128 registers (two workgroups a CU)
       case 1:
-        // (a wide product's many workgroups, more than two a CU: with fewer k-steps in flight each they
-        // need half the registers, and all of them are on the CUs at once -- the gate-up product of 8
-        // rows after a prepared norm: a decode step 1.020 -> 0.990 ms)
+        // (a wide product's many workgroups: as above)
         if (static_cast<int>(grid.x) > 2 * compute_units()) gemm_skinny_kernel<1, EPI, XMODE, 2><<<grid, block, 0, s>>>(b);
         else gemm_skinny_kernel<1, EPI, XMODE, 4><<<grid, block, 0, s>>>(b);
         break;
@@ -669,13 +715,15 @@ int check_parts(const char* what, const float* ssq_parts, int ssq_blocks, int ss
 }  // namespace bc4g
 
 extern "C" int bc4g_gemm_skinny(const void* x, const void* w, void* out, const float* bias, int epilogue, int m, int n, int k,
-                                void* stream) {
+                                int halves, void* stream) {
   if (int e = check_common("gemm_skinny", m, 64, n, k, epilogue)) return e;
   BC4G_REQUIRE(epilogue != kRopeKvBf16, "gemm_skinny: use bc4g_gemm_skinny_qkv for the rotary epilogue");
   BC4G_REQUIRE(!bias || epilogue == kAccumF32, "gemm_skinny: only the adding epilogue takes a bias");
+  BC4G_REQUIRE(!halves || (m <= kSplitMinRows && epilogue <= kAccumF32), "gemm_skinny: half blocks take at most %d rows and epilogues 0 to 2", kSplitMinRows);
   if (m == 0) return 0;
   SkinnyArgs a = plain_args(x, w, out, m, n, k);
   a.bias = bias;
+  a.halves = halves;
   return launch_epilogue<kPlain>(a, epilogue, static_cast<hipStream_t>(stream));
 }
 
@@ -693,10 +741,11 @@ extern "C" int bc4g_gemm_skinny_xielu(const void* x, const void* w, void* out, c
 // [m, n] = bfloat16(new residual * g) and emit_ssq [ceil(n / 16)][emit_stride], block b's part of
 // every row's sum of squares.
 extern "C" int bc4g_gemm_skinny_emit(const void* x, const void* w, float* out, const float* bias, const void* g, int g_dtype, void* emit_x,
-                                     float* emit_ssq, int emit_stride, int m, int n, int k, void* stream) {
+                                     float* emit_ssq, int emit_stride, int m, int n, int k, int halves, void* stream) {
   if (int e = check_common("gemm_skinny_emit", m, 64, n, k, kAccumF32)) return e;
   BC4G_REQUIRE(g && emit_x && emit_ssq && emit_stride >= m, "gemm_skinny_emit: the norm's scale and both outputs are needed");
   BC4G_REQUIRE(g_dtype == kBF16 || g_dtype == kF32, "gemm_skinny_emit: unknown norm scale dtype %d", g_dtype);
+  BC4G_REQUIRE(!halves || m <= kSplitMinRows, "gemm_skinny_emit: half blocks take at most %d rows", kSplitMinRows);
   if (m == 0) return 0;
   SkinnyArgs a = plain_args(x, w, out, m, n, k);
   a.bias = bias;
@@ -705,13 +754,14 @@ extern "C" int bc4g_gemm_skinny_emit(const void* x, const void* w, float* out, c
   a.emit_x = static_cast<bf16_t*>(emit_x);
   a.emit_ssq = emit_ssq;
   a.emit_stride = emit_stride;
+  a.halves = halves;
   return launch<kAccumF32, kPlain>(a, static_cast<hipStream_t>(stream));
 }
 
 // x is bfloat16(residual * g) and ssq_parts the parts of the rows' sums of squares, as
 // bc4g_gemm_skinny_emit leaves them: out = rmsnorm(residual) w^T with the epilogues of bc4g_gemm_skinny
 // except the adding one.
-extern "C" int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, float eps,
+extern "C" int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, int ssq_halves, float eps,
                                           const void* w, void* out, int epilogue, int m, int n, int k, void* stream) {
   if (int e = check_common("gemm_skinny_prenormed", m, 64, n, k, epilogue)) return e;
   if (int e = check_parts("gemm_skinny_prenormed", ssq_parts, ssq_blocks, ssq_stride, m, eps)) return e;
@@ -722,6 +772,7 @@ extern "C" int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts,
   a.ssq_parts = ssq_parts;
   a.ssq_blocks = ssq_blocks;
   a.ssq_stride = ssq_stride;
+  a.ssq_halves = ssq_halves;
   a.eps = eps;
   return launch_epilogue<kPlain>(a, epilogue, static_cast<hipStream_t>(stream));
 }
@@ -750,7 +801,7 @@ extern "C" int bc4g_gemm_skinny_normed(const float* x, const int32_t* rows, cons
 // with RMSNorm fused (g given, m <= 16).  q_out: bfloat16 [m, n_heads * head_dim], rotated, in the
 // reordered head layout.
 extern "C" int bc4g_gemm_skinny_qkv(const void* x, const void* g, int g_dtype, float eps, const float* ssq_parts,
-                                    int ssq_blocks, int ssq_stride, const void* w, void* q_out,
+                                    int ssq_blocks, int ssq_stride, int ssq_halves, const void* w, void* q_out,
                                     const int32_t* positions, const int32_t* slot_map, void* k_cache, void* v_cache,
                                     int m, int k, int n_heads, int n_kv_heads, int head_dim, int rotary_dim,
                                     float theta, int page_tokens, int write_kv, void* stream) {
@@ -774,6 +825,7 @@ extern "C" int bc4g_gemm_skinny_qkv(const void* x, const void* g, int g_dtype, f
   a.ssq_parts = ssq_parts;
   a.ssq_blocks = ssq_blocks;
   a.ssq_stride = ssq_stride;
+  a.ssq_halves = ssq_halves;
   if (!g) return launch<kRopeKvBf16, kPlain>(a, s);
   if (g_dtype == kBF16) return launch<kRopeKvBf16, kNormedG16>(a, s);
   if (g_dtype == kF32) return launch<kRopeKvBf16, kNormedG32>(a, s);

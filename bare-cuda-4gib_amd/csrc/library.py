@@ -41,15 +41,15 @@ _SIGNATURES = {
     "bc4g_argmax_static": [_P, _P, _I, _I, _P],
     "bc4g_probe_read": [_P, c_long, _P, _I, _P],
     "bc4g_probe_mfma": [_P, _I, _P, _I, _P],
-    "bc4g_gemm_skinny": [_P, _P, _P, _P, _I, _I, _I, _I, _P],
+    "bc4g_gemm_skinny": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "bc4g_gemm_mfma": [_P, _P, _I, _P, _P, _I, _I, _I, _I, _P],
     "bc4g_gemm_mfma_tile": [_P, _P, _I, _I, _I, _I, _P, _P],
     "bc4g_gemm_skinny_normed": [_P, _P, _P, _I, _F, _P, _P, _I, _I, _I, _I, _P],
     "bc4g_attention_mfma": [_P, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _I, _P, _I, _P, _I, _P, _P],
     "bc4g_gemm_mfma_qkv": [_P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
-    "bc4g_gemm_skinny_qkv": [_P, _P, _I, _F, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P],
-    "bc4g_gemm_skinny_emit": [_P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _P],
-    "bc4g_gemm_skinny_prenormed": [_P, _P, _I, _I, _F, _P, _P, _I, _I, _I, _I, _P],
+    "bc4g_gemm_skinny_qkv": [_P, _P, _I, _F, _P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P],
+    "bc4g_gemm_skinny_emit": [_P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _P],
+    "bc4g_gemm_skinny_prenormed": [_P, _P, _I, _I, _I, _F, _P, _P, _I, _I, _I, _I, _P],
     "bc4g_rmsnorm_add": [_P, _P, _I, _P, _P, _I, _F, _P, _I, _I, _I, _F, _P],
     "bc4g_gemm_skinny_xielu": [_P, _P, _P, _P, _I, _I, _I, _P],
     "bc4g_rmsnorm_conv": [_P, _P, _I, _F, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P],

@@ -737,6 +737,16 @@ def streams_weights(m: int, n: int, k: int) -> bool:
     return plan_for(n, k).streams(m)
 
 
+HALF_BLOCKS = 128           # blocks of 16 outputs up to which two workgroups share one: a block for every other CU
+HALF_MIN_K = 1024           # (a block of less is pulled in a fraction of what its product takes anyway)
+
+
+def half_blocks(m: int, n: int, k: int) -> bool:
+    """Whether the weight-streaming kernel gives every block of 16 outputs to two workgroups: up to 8 rows, a weight of few
+    and long blocks (gemm_skinny.hip says why).  The results are the same bits."""
+    return m <= 8 and k >= HALF_MIN_K and -(-n // 16) <= HALF_BLOCKS
+
+
 EPI_STORE_BF16, EPI_STORE_F32, EPI_ACCUM_F32, EPI_SWIGLU = 0, 1, 2, 3
 EPI_SQUARED_RELU = 6      # max(sum, 0)^2 stored as bfloat16
 EPI_GEGLU = 7             # as EPI_SWIGLU, with the gelu written with tanh
@@ -783,7 +793,8 @@ def gemm_fast(a: torch.Tensor, w, out_dtype=None,
         packed = packed if packed is not None else pack_weight(_rows(w))      # (packing per call: tests only)
         for r0 in range(0, m, SKINNY_MAX_ROWS):                        # the weights once for every 64 rows
             rows = min(SKINNY_MAX_ROWS, m - r0)
-            library.call("bc4g_gemm_skinny", _ptr(a[r0:]), _ptr(packed), _ptr(out[r0:]), _ptr(bias), epi, rows, n, k, _stream(),
+            library.call("bc4g_gemm_skinny", _ptr(a[r0:]), _ptr(packed), _ptr(out[r0:]), _ptr(bias), epi, rows, n, k,
+                         1 if epi <= EPI_ACCUM_F32 and half_blocks(m, n, k) else 0, _stream(),
                          cost=_skinny_cost(rows, n, k, 2, out_bytes))
     else:
         library.call("bc4g_gemm_mfma", _ptr(a), *_tiled_weight(w, packed, a), _ptr(out), _ptr(bias), epi, m, n, k, _stream(),
@@ -862,7 +873,7 @@ def gemm_swiglu(a: torch.Tensor, w_gate_up, interleaved: bool = False, act: str 
             packed = packed if packed is not None else pack_weight(_rows(rows))
             for r0 in range(0, m, SKINNY_MAX_ROWS):
                 part = min(SKINNY_MAX_ROWS, m - r0)
-                library.call("bc4g_gemm_skinny", _ptr(a[r0:]), _ptr(packed), _ptr(out[r0:]), None, gated_epilogue(act), part, n, k,
+                library.call("bc4g_gemm_skinny", _ptr(a[r0:]), _ptr(packed), _ptr(out[r0:]), None, gated_epilogue(act), part, n, k, 0,
                              _stream(), cost=_skinny_cost(part, n, k, 2, 1))
         else:
             library.call("bc4g_gemm_mfma", _ptr(a), *_tiled_weight(rows, packed, a), _ptr(out), None, gated_epilogue(act), m, n, k, _stream(),
@@ -889,7 +900,8 @@ class Fresh:
 class Prenormed:
     """What a product that added into the residual stream left for the RMSNorm after it
     (gemm_accumulate_emit): ``xb`` = bfloat16(residual * g) [m, width] and ``parts`` [blocks, m], block
-    b's share (16 columns) of every row's sum of squares.  A product that takes it
+    b's share (16 columns) of every row's sum of squares -- or [blocks, m, 2], the shares of its halves, where two
+    workgroups shared a block (half_blocks).  A product that takes it
     (gemm_prenormed, gemm_qkv_rope) applies the row's rsqrt(sum of parts / width + eps) to its sums."""
 
     def __init__(self, xb: torch.Tensor, parts: torch.Tensor, eps: float):
@@ -965,11 +977,12 @@ def gemm_accumulate_emit(a: torch.Tensor, w, residual: torch.Tensor, g: torch.Te
     if tuple(g.shape) != (n,):
         raise KernelError(f"gemm_accumulate_emit: norm scale must be [{n}], got {tuple(g.shape)}")
     xb = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
-    parts = torch.empty((-(-n // 16), m), dtype=torch.float32, device=a.device)
+    halves = half_blocks(m, n, k)
+    parts = torch.empty((-(-n // 16), m, 2) if halves else (-(-n // 16), m), dtype=torch.float32, device=a.device)
     for r0 in range(0, m, SKINNY_MAX_ROWS):
         rows = min(SKINNY_MAX_ROWS, m - r0)
         library.call("bc4g_gemm_skinny_emit", _ptr(a[r0:]), _ptr(packed), _ptr(residual[r0:]), _ptr(bias), _ptr(g),
-                     _code(g, "gemm_accumulate_emit"), _ptr(xb[r0:]), _ptr(parts[:, r0:]), m, rows, n, k, _stream(),
+                     _code(g, "gemm_accumulate_emit"), _ptr(xb[r0:]), _ptr(parts[:, r0:]), m, rows, n, k, 1 if halves else 0, _stream(),
                      cost=_skinny_cost(rows, n, k, 2, 10))
     return Prenormed(xb, parts, eps)
 
@@ -1008,13 +1021,14 @@ def gemm_prenormed(pre: Prenormed, w, epilogue: int) -> torch.Tensor:
     if not streams_weights(m, n, k):
         if epilogue not in GATED_EPILOGUES:
             raise KernelError("gemm_prenormed: the tiled kernel finishes a prepared norm in its gated epilogues only")
-        library.call("bc4g_gemm_mfma_swiglu_scaled", _ptr(pre.xb), _ptr(pre.parts), pre.parts.shape[0], pre.parts.shape[1], pre.eps,
+        parts = pre.parts if pre.parts.dim() == 2 else pre.parts.sum(-1)      # (few rows, and a plan that has them tiled)
+        library.call("bc4g_gemm_mfma_swiglu_scaled", _ptr(pre.xb), _ptr(parts), pre.parts.shape[0], pre.parts.shape[1], pre.eps,
                      *tiled_w, _ptr(out), 1 if epilogue == EPI_GEGLU else 0, m, n, k, _stream(), cost=_tiled_cost(m, n, k, 1))
         return out
     for r0 in range(0, m, SKINNY_MAX_ROWS):
         rows = min(SKINNY_MAX_ROWS, m - r0)
         library.call("bc4g_gemm_skinny_prenormed", _ptr(pre.xb[r0:]), _ptr(pre.parts[:, r0:]), pre.parts.shape[0], m,
-                     pre.eps, _ptr(packed), _ptr(out[r0:]), epilogue, rows, n, k, _stream(),
+                     pre.parts.dim() - 2, pre.eps, _ptr(packed), _ptr(out[r0:]), epilogue, rows, n, k, _stream(),
                      cost=_skinny_cost(rows, n, k, 2, out.element_size() * out.shape[1] / n))
     return out
 
@@ -1061,7 +1075,7 @@ def gemm_qkv_rope(x: torch.Tensor, g: Optional[torch.Tensor], eps: float, w,
     parts = pre.parts if pre is not None else None
     library.call("bc4g_gemm_skinny_qkv", _ptr(x), _ptr(g), _code(g, "gemm_qkv_rope") if g is not None else 0,
                  float(pre.eps if pre is not None else eps), _ptr(parts), parts.shape[0] if pre is not None else 0,
-                 parts.shape[1] if pre is not None else 0, _ptr(packed), _ptr(q), _ptr(positions), _ptr(slot_map),
+                 parts.shape[1] if pre is not None else 0, parts.dim() - 2 if pre is not None else 0, _ptr(packed), _ptr(q), _ptr(positions), _ptr(slot_map),
                  _ptr(k_cache), _ptr(v_cache), m, k, n_heads, n_kv_heads, head_dim, int(rotary_dim), float(theta),
                  page_tokens, 1 if write_kv else 0, _stream(), cost=_skinny_cost(m, n, k, x.element_size(), 2))
     return q

@@ -178,13 +178,13 @@ bool gemm_skinny() {
     const std::vector<double> want = plain::gemm(widen(x), widen(w), m, n, k);
     Dev<bf16> dx(x), o16(static_cast<size_t>(m) * n), act(static_cast<size_t>(m) * n / 2), gelu(static_cast<size_t>(m) * n / 2);
     Dev<float> db(bias), o32(static_cast<size_t>(m) * n), acc(before);
-    RUN(bc4g_gemm_skinny(dx.p, packed.p, o16.p, nullptr, 0, m, n, k, kStream));
-    RUN(bc4g_gemm_skinny(dx.p, packed.p, o32.p, nullptr, 1, m, n, k, kStream));
-    RUN(bc4g_gemm_skinny(dx.p, packed.p, acc.p, db.p, 2, m, n, k, kStream));
-    RUN(bc4g_gemm_skinny(dx.p, packed.p, act.p, nullptr, 3, m, n, k, kStream));
-    RUN(bc4g_gemm_skinny(dx.p, packed.p, gelu.p, nullptr, 7, m, n, k, kStream));
+    RUN(bc4g_gemm_skinny(dx.p, packed.p, o16.p, nullptr, 0, m, n, k, 0, kStream));
+    RUN(bc4g_gemm_skinny(dx.p, packed.p, o32.p, nullptr, 1, m, n, k, 0, kStream));
+    RUN(bc4g_gemm_skinny(dx.p, packed.p, acc.p, db.p, 2, m, n, k, 0, kStream));
+    RUN(bc4g_gemm_skinny(dx.p, packed.p, act.p, nullptr, 3, m, n, k, 0, kStream));
+    RUN(bc4g_gemm_skinny(dx.p, packed.p, gelu.p, nullptr, 7, m, n, k, 0, kStream));
     ok &= close("bfloat16 out", widen(o16.get()), want, kBf16, 1e-2);
-    RUN(bc4g_gemm_skinny(dx.p, packed.p, o16.p, nullptr, 6, m, n, k, kStream));
+    RUN(bc4g_gemm_skinny(dx.p, packed.p, o16.p, nullptr, 6, m, n, k, 0, kStream));
     std::vector<double> squared = want;
     for (double& v : squared) v = plain::squared_relu(v);
     ok &= close("squared relu", widen(o16.get()), squared, kBf16, 1e-2);
@@ -235,8 +235,8 @@ bool gemm_skinny_norms() {
   const std::vector<float> residual = normals(rng, static_cast<size_t>(m) * hidden, 2.0f);
   Dev<bf16> dx(x), p1(pack_weight(w1, hidden, k1)), p2(pack_weight(w2, n2, hidden)), emit_x(static_cast<size_t>(m) * hidden);
   Dev<float> dres(residual), ssq(static_cast<size_t>((hidden + 15) / 16) * m), y(static_cast<size_t>(m) * n2);
-  RUN(bc4g_gemm_skinny_emit(dx.p, p1.p, dres.p, nullptr, dg.p, 0, emit_x.p, ssq.p, m, m, hidden, k1, kStream));
-  RUN(bc4g_gemm_skinny_prenormed(emit_x.p, ssq.p, (hidden + 15) / 16, m, eps, p2.p, y.p, 1, m, n2, hidden, kStream));
+  RUN(bc4g_gemm_skinny_emit(dx.p, p1.p, dres.p, nullptr, dg.p, 0, emit_x.p, ssq.p, m, m, hidden, k1, 0, kStream));
+  RUN(bc4g_gemm_skinny_prenormed(emit_x.p, ssq.p, (hidden + 15) / 16, m, 0, eps, p2.p, y.p, 1, m, n2, hidden, kStream));
   std::vector<double> after = plain::gemm(widen(x), widen(w1), m, hidden, k1);
   for (size_t i = 0; i < after.size(); ++i) after[i] += residual[i];
   ok &= close("stream after the adding product", widen(dres.get()), after, 1e-4, 1e-4);
@@ -515,7 +515,7 @@ bool qkv_fused() {
       RUN(bc4g_rope_table(dpos.p, table.p, t, d, theta, kStream));
       RUN(bc4g_gemm_mfma_qkv(dx.p, packed.p, 1, dq.p, table.p, dslots.p, kc.p, vc.p, t, n, hidden, nh, nkv, d, page, 1, kStream));
     } else {
-      RUN(bc4g_gemm_skinny_qkv(dx.p, nullptr, 0, 0.0f, nullptr, 0, 0, packed.p, dq.p, dpos.p, dslots.p, kc.p, vc.p, t, hidden,
+      RUN(bc4g_gemm_skinny_qkv(dx.p, nullptr, 0, 0.0f, nullptr, 0, 0, 0, packed.p, dq.p, dpos.p, dslots.p, kc.p, vc.p, t, hidden,
                                nh, nkv, d, d, theta, page, 1, kStream));
     }
     const int tokens_per_tile = 16 / (nh / nkv);
