@@ -9,7 +9,7 @@
 // rows' 16 bytes straight into operand order keep the texture path busy four times as long), several steps of 32 k ahead and
 // with no barrier; it reads its fragments there and feeds 16x16x4 MFMAs with w as the A operand.  The shares meet in LDS.
 // Eight rows, weights not in a cache, plain float FMA (gemm_generic) -> this: 32,000 x 2,048 142 -> 49 us (5.4 TB/s), 11,264 x
-// 2,048 61 -> 21, 2,048 x 5,632 86 -> 19; 32 decode steps of 8 requests after their prompts at TinyLlama's sizes 211 -> 87 ms.
+// 2,048 61 -> 21, 2,048 x 5,632 86 -> 15; 32 decode steps of 8 requests after their prompts at TinyLlama's sizes 211 -> 87 ms.
 //
 // gemm_f32_tiled_kernel, many rows, bound by the matrix cores (157 TFLOP/s of float32 at the full clock).  A step's 32 k of the
 // tile's rows of x and of w go straight into a ring of stages in LDS; the waves feed 32x32x2 MFMAs from there and keep
@@ -62,7 +62,7 @@ __device__ inline int slot_key(int row) { return (row >> 1) & 7; }
 // steps through the stretch.
 template <int N>
 __device__ inline void load_pieces_to_lds(const float* const (&bases)[N], const unsigned (&offsets)[N], unsigned lds_first) {
-  static_assert(N == 3 || N == 4 || N == 6, "two pieces of weights and one, two or four of x");
+  static_assert(N == 2 || N == 3 || N == 4 || N == 6, "one or two pieces of weights and one, two or four of x");
   constexpr int kMid = N / 2;
   const void* b[N];
 #pragma unroll
@@ -74,7 +74,10 @@ __device__ inline void load_pieces_to_lds(const float* const (&bases)[N], const 
   }
   const unsigned mid = __builtin_amdgcn_readfirstlane(lds_first + kMid * 1024);
 #define BC4G_PIECE(i, v, s) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #i "\n\t"
-  if constexpr (N == 3) {
+  if constexpr (N == 2) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-1024, 1, 3) BC4G_PIECE(0, 2, 4)
+                 ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "s"(b[0]), "s"(b[1]) : "memory", "m0");
+  } else if constexpr (N == 3) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-1024, 1, 4) BC4G_PIECE(0, 2, 5) BC4G_PIECE(1024, 3, 6)
                  ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "v"(offsets[2]), "s"(b[0]), "s"(b[1]), "s"(b[2]) : "memory", "m0");
   } else if constexpr (N == 4) {
@@ -111,16 +114,17 @@ __device__ inline void wait_for_step(int later) {
   }
 }
 
-// XR: rows of x a workgroup takes (blockIdx.y: which).
-template <int XR, int STAGES, int EPI>
+// XR: rows of x a workgroup takes (blockIdx.y: which).  HALF: eight rows of w a workgroup instead of 16 (see launch_stream).
+template <int XR, int STAGES, int EPI, bool HALF = false>
 __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a) {
-  constexpr int MT = (XR + 15) / 16, PER = 2 + XR / 8, kRing = PER * 1024;
+  constexpr int MT = (XR + 15) / 16, WP = HALF ? 1 : 2, PER = WP + XR / 8, kRing = PER * 1024;      // (WP: pieces of w a step)
+  static_assert(!HALF || !gated(EPI), "half a block of a gated product would part gates and ups");
   extern __shared__ __align__(1024) unsigned char stream_lds[];
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int col = lane % 16, grp = lane / 16;
   const int k = a.k, row0 = blockIdx.y * XR, m = min(XR, a.m - row0);
-  constexpr int kCols = gated(EPI) ? 8 : 16;                 // outputs of a workgroup
+  constexpr int kCols = gated(EPI) || HALF ? 8 : 16;         // outputs of a workgroup
   const int n_out = gated(EPI) ? a.n / 2 : a.n, n0 = blockIdx.x * kCols;
 
   // this wave's steps of k
@@ -148,9 +152,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
   unsigned offsets[PER], back[PER];                          // (back: from a segment to its row's first one)
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int r = (i < 2 ? i : i - 2) * 8 + lane / 8, seg = (lane % 8) ^ slot_key(r);
+    const int r = (i < WP ? i : i - WP) * 8 + lane / 8, seg = (lane % 8) ^ slot_key(r);
     back[i] = seg * 16;
-    if (i < 2) {                                             // (a load's eight rows of w lie together, from a scalar base)
+    if (i < WP) {                                            // (a load's eight rows of w lie together, from a scalar base)
       const int from = gated(EPI) ? n0 : min(n0 + i * 8, n_out - 1);
       const int at = min(gated(EPI) ? n0 + lane / 8 : n0 + r, n_out - 1);
       bases[i] = a.w + static_cast<long>(from + (gated(EPI) ? i * (a.n / 2) : 0)) * k + first * kStepK;
@@ -188,11 +192,12 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int seg = 4 * h + grp;
-      wf[h] = *reinterpret_cast<const floatx4*>(at + col * kStepBytes + ((seg ^ slot_key(col)) * 16));
+      const int wr = HALF ? col % 8 : col;                     // (the other eight rows repeat them, their sums are not used)
+      wf[h] = *reinterpret_cast<const floatx4*>(at + wr * kStepBytes + ((seg ^ slot_key(wr)) * 16));
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
         const int r = (t * 16 + col) % XR;
-        xf[t][h] = *reinterpret_cast<const floatx4*>(at + 2048 + r * kStepBytes + ((seg ^ slot_key(r)) * 16));
+        xf[t][h] = *reinterpret_cast<const floatx4*>(at + WP * 1024 + r * kStepBytes + ((seg ^ slot_key(r)) * 16));
       }
       if (k0 + kStepK > k && k0 + seg * 4 >= k) {
         wf[h] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -240,10 +245,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
   }
 }
 
-template <int XR, int STAGES, int EPI>
+template <int XR, int STAGES, int EPI, bool HALF = false>
 int launch_stream_form(const Args& a, hipStream_t s) {
-  auto kernel = gemm_f32_stream_kernel<XR, STAGES, EPI>;
-  constexpr int kLds = kWaves * STAGES * (2 + XR / 8) * 1024;
+  auto kernel = gemm_f32_stream_kernel<XR, STAGES, EPI, HALF>;
+  constexpr int kLds = kWaves * STAGES * ((HALF ? 1 : 2) + XR / 8) * 1024;
   static_assert(kLds <= 160 * 1024, "a workgroup's LDS");
   static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
   if (!raised) {
@@ -251,7 +256,7 @@ int launch_stream_form(const Args& a, hipStream_t s) {
       return fail("gemm_f32: cannot raise the dynamic LDS limit");
     raised = true;
   }
-  const int cols = gated(EPI) ? 8 : 16, n_out = gated(EPI) ? a.n / 2 : a.n;
+  const int cols = gated(EPI) || HALF ? 8 : 16, n_out = gated(EPI) ? a.n / 2 : a.n;
   kernel<<<dim3((n_out + cols - 1) / cols, (a.m + XR - 1) / XR), kThreads, kLds, s>>>(a);
   return 0;
 }
@@ -259,6 +264,12 @@ int launch_stream_form(const Args& a, hipStream_t s) {
 template <int EPI>
 int launch_stream(const Args& a, hipStream_t s) {
   const int cols = gated(EPI) ? 8 : 16, n_out = gated(EPI) ? a.n / 2 : a.n;
+  // Outputs that would leave every other CU idle: eight a workgroup, half the weights for each CU to bring and the
+  // same sums.  A decode step's two such products, 2,048 x 2,048 and
+  // 2,048 x 5,632, from memory, 8 rows: 13.05 -> 11.7 us on average; 32 steps of 8 requests after their prompts 67.6 -> 63.5 ms.
+  if constexpr (!gated(EPI)) {
+    if (a.m <= 8 && 2 * ((n_out + 15) / 16) <= compute_units()) return launch_stream_form<8, 8, EPI, true>(a, s);
+  }
   // One workgroup a CU where there are no more: a ring as deep as LDS allows.  Else two that overlap.
   const bool few = (n_out + cols - 1) / cols <= compute_units();
   if (a.m <= 8) return few ? launch_stream_form<8, 6, EPI>(a, s) : launch_stream_form<8, 3, EPI>(a, s);

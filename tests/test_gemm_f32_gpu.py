@@ -32,7 +32,7 @@ def held(got, want, bound, what):
 # rows at the edges of the forms (8, 16, 32 and 64 a workgroup; the tiles' 64 and 128), k at the edges of a step (32) and of the
 # shares it is added up in, n at the edges of a block and of a tile
 @pytest.mark.parametrize("m", [1, 7, 8, 9, 16, 17, 33, 64, 65, 129, 300])
-@pytest.mark.parametrize("n,k", [(1, 4), (16, 32), (130, 176), (301, 260), (64, 2048), (129, 288), (4098, 36), (2100, 64)])
+@pytest.mark.parametrize("n,k", [(1, 4), (16, 32), (130, 176), (301, 260), (64, 2048), (129, 288), (4098, 36), (2100, 64), (24, 5632)])
 def test_products(ops, m, n, k):
     x, w = operands(m, n, k, m + n + k)
     xd, wd = x.to(DEV), w.to(DEV)
