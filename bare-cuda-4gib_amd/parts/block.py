@@ -176,8 +176,10 @@ class SandwichBlock(Part):
         if self.ffn is not None:
             y = self._sum_for(self.ffn, x)
             # (a feed-forward that says so gets the norm not yet computed: its first product absorbs it for few rows)
-            if h is None:
-                h = Normed(x, self.ffn_norm, ctx) if getattr(self.ffn, "accepts_lazy_norm", False) else self.ffn_norm.forward(x, ctx)
+            if getattr(self.ffn, "accepts_lazy_norm", False):
+                h = Normed(x, self.ffn_norm, ctx, done=h)
+            elif h is None:
+                h = self.ffn_norm.forward(x, ctx)
             self.ffn.forward(h, ctx, y)
             self.ffn_post_norm.add_to(x, self._sum_of(y))
 

@@ -46,7 +46,7 @@ class CausalConv(Part):
 
     def behind(self, norm, x: torch.Tensor, ctx, view) -> Optional[torch.Tensor]:
         """h + the convolution of h with h = norm(x), in one kernel where there is one for the step; else None."""
-        scale = norm.fusable() if isinstance(norm, RMSNorm) else None
+        scale = norm.fusable() if type(norm) is RMSNorm else None      # (a norm derived from it may do more)
         if scale is None or self.taps == 1:
             return None
         return ops.rmsnorm_conv(x, scale[0], scale[1], norm.out_dtype, self.w, view.tail, ctx, bias=self.b)

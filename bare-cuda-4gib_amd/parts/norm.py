@@ -40,7 +40,7 @@ class RMSNorm(Part):
 
     def add_and_norm(self, x: torch.Tensor, y: torch.Tensor, following) -> Optional[torch.Tensor]:
         """add_to, and where one kernel can make it too the norm ``following`` of the new x -- else None."""
-        scale = following.fusable() if isinstance(following, RMSNorm) else None
+        scale = following.fusable() if type(following) is RMSNorm else None      # (a norm derived from it may do more)
         if scale is None:
             self.add_to(x, y)
             return None
