@@ -249,8 +249,10 @@ int bc4g_gemm_skinny_emit(const void* x, const void* w, float* out, const float*
                           float* emit_ssq, int emit_stride, int m, int n, int k, int halves, void* stream);
 int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, int ssq_halves, float eps,
                                const void* w, void* out, int epilogue, int m, int n, int k, void* stream);
-// out (bfloat16) = xielu(x w^T) with its two numbers pq, of the product rounded to bfloat16: at most 64 rows.
-int bc4g_gemm_skinny_xielu(const void* x, const void* w, void* out, const float* pq, int m, int n, int k, void* stream);
+// out (bfloat16) = xielu(x w^T) with its two numbers pq, of the product rounded to bfloat16: at most 64 rows.  ssq_parts (null: x as
+// it is), ssq_blocks, ssq_stride and eps as in bc4g_gemm_skinny_prenormed.
+int bc4g_gemm_skinny_xielu(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, float eps, const void* w, void* out,
+                           const float* pq, int m, int n, int k, void* stream);
 }
 
 extern "C" {
@@ -266,9 +268,11 @@ int bc4g_probe_mfma(const void* operands, int iters, float* sink, int workgroups
 extern "C" {
 // x[r, :] += y[r, :] * rsqrt(mean(y[r]^2) + eps) * w: the norm after a sublayer, added to the float residual stream
 // (w float32, as it multiplies; y float32 or bfloat16).  With next_w and out (null: neither), also the RMSNorm of the new x with that
-// scale: hidden a multiple of 8 up to 8192, everything on 16-byte boundaries.
+// scale: hidden a multiple of 8 up to 8192, everything on 16-byte boundaries.  With ssq [n_rows] too (null: not), out is not that norm but
+// bfloat16(new x * next_w), and ssq the rows' sums of squares: what a product that absorbs the norm takes (one part of all of
+// them, bc4g_gemm_skinny_prenormed).
 int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const float* w, const void* next_w, int next_w_dtype, float next_eps,
-                     void* out, int out_dtype, int n_rows, int hidden, float eps, void* stream);
+                     void* out, int out_dtype, float* ssq, int n_rows, int hidden, float eps, void* stream);
 // out[r] = h + bias + (the causal convolution of h) with h = the RMSNorm of x[r], for a step in which request r brings row r alone:
 // bc4g_rmsnorm and bc4g_causal_conv (add_input) in one launch, the same bits.  w float32 [taps][hidden], state [slots, taps - 1, hidden]
 // in the output's type; 2 to 4 taps, hidden a multiple of 8 up to 4096, everything on 16-byte boundaries.

@@ -124,6 +124,16 @@ __device__ inline float xielu_f(float z, float ap, float aq) {
   return z > 0.f ? ap * z * z + 0.5f * z : aq * (expm1f(z) - z) + 0.5f * z;
 }
 
+// sum + v[0]^2 + ... + v[7]^2, or the beginning of such a sum: a lane's share of a row's sum of squares in the product that absorbs
+// a norm and in the kernel that prepares the same for it, so spelt out that both round alike (of an unrolled sum the compiler
+// joins either of the first two products with the other).
+__device__ inline float add_squares(const float (&v)[8], bool begun, float sum) {
+  sum = begun ? fmaf(v[1], v[1], fmaf(v[0], v[0], sum)) : fmaf(v[0], v[0], v[1] * v[1]);
+#pragma unroll
+  for (int e = 2; e < 8; ++e) sum = fmaf(v[e], v[e], sum);
+  return sum;
+}
+
 inline int ceil_div(long a, long b) { return static_cast<int>((a + b - 1) / b); }
 
 }  // namespace bc4g

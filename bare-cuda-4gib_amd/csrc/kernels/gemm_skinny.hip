@@ -431,8 +431,7 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
 #pragma unroll
             for (int i = 0; i < 8; ++i) gv[i] = __uint_as_float(gr[i]);
           }
-#pragma unroll
-          for (int i = 0; i < 8; ++i) ss += xv[i] * xv[i];
+          ss = add_squares(xv, kb + it > 0, ss);
           *reinterpret_cast<uint4*>(stage + static_cast<long>(row) * stage_stride + kk) =
               make_uint4(pack2(xv[0] * gv[0], xv[1] * gv[1]), pack2(xv[2] * gv[2], xv[3] * gv[3]),
                          pack2(xv[4] * gv[4], xv[5] * gv[5]), pack2(xv[6] * gv[6], xv[7] * gv[7]));
@@ -727,13 +726,20 @@ extern "C" int bc4g_gemm_skinny(const void* x, const void* w, void* out, const f
   return launch_epilogue<kPlain>(a, epilogue, static_cast<hipStream_t>(stream));
 }
 
-// out (bfloat16) = xielu(x w^T), pq its two numbers.
-extern "C" int bc4g_gemm_skinny_xielu(const void* x, const void* w, void* out, const float* pq, int m, int n, int k, void* stream) {
+// out (bfloat16) = xielu(x w^T), pq its two numbers.  With ssq_parts x is bfloat16(residual * g), as in bc4g_gemm_skinny_prenormed.
+extern "C" int bc4g_gemm_skinny_xielu(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, float eps, const void* w,
+                                      void* out, const float* pq, int m, int n, int k, void* stream) {
   if (int e = check_common("gemm_skinny_xielu", m, 64, n, k, kXieluBf16)) return e;
   BC4G_REQUIRE(x && w && out && pq, "gemm_skinny_xielu: a tensor is missing");
+  if (ssq_parts)
+    if (int e = check_parts("gemm_skinny_xielu", ssq_parts, ssq_blocks, ssq_stride, m, eps)) return e;
   if (m == 0) return 0;
   SkinnyArgs a = plain_args(x, w, out, m, n, k);
   a.bias = pq;
+  a.ssq_parts = ssq_parts;
+  a.ssq_blocks = ssq_blocks;
+  a.ssq_stride = ssq_stride;
+  a.eps = eps;
   return launch<kXieluBf16, kPlain>(a, static_cast<hipStream_t>(stream));
 }
 

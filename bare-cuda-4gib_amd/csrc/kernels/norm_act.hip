@@ -49,16 +49,24 @@ __device__ inline void store_eight(bf16_t* p, const float (&v)[8]) {
   *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// The same for widths that are a multiple of 8 and at most 2,048 * CHUNKS, on 16-byte boundaries, and with NEXT the RMSNorm that reads
-// the stream next: out[r, :] = x[r, :] * rsqrt(mean(x[r]^2) + next_eps) * next_w of the new x.  A decode step's few rows leave a
-// workgroup a row that does nothing but wait, so everything a row needs is asked for at once and held in registers: 8 rows of
-// 2,048 in a step 4.4 us where two passes over the row took 7.6, and the norm after it, a launch of 4.2 us, costs 0.3.
-// (The norm's sum in the order of the norm kernel's own: the same bits.)
-template <typename TY, typename TN, typename TO, int CHUNKS, bool NEXT>
+enum Following : int { kNothing = 0, kNorm = 1, kPrepared = 2 };
+
+// The same for widths that are a multiple of 8 and at most 2,048 * CHUNKS, on 16-byte boundaries, the same bits -- and what reads
+// the stream next, of the new x.  kNorm: its RMSNorm, out[r, :] = x[r, :] * rsqrt(mean(x[r]^2) + next_eps) * next_w.  kPrepared: what the
+// streaming product that absorbs that norm takes instead, out[r, :] = x[r, :] * next_w in bfloat16 and ssq[r] = the sum of x[r]^2.
+// A decode step's few rows leave a workgroup a row that does nothing but wait, so everything a row needs is asked for at once
+// and held in registers: 8 rows of 2,048 in a step 4.4 us where two passes over the row took 7.6, and the norm after it, a launch
+// of 4.2 us, costs 0.3.
+// Every sum is taken in the order of the kernel whose place this takes, so that the choice of kernel moves no bit: y's
+// by the threads of the kernel above (neighbouring elements in neighbouring threads: the row is turned through LDS), a
+// norm's in the order of the norm kernel's own, a prepared one's in the order of the product that absorbs a norm (gemm_skinny.hip:
+// one wave, a lane eight elements of each 512).
+template <typename TY, typename TN, typename TO, int CHUNKS, int NEXT>
 __global__ __launch_bounds__(kBlock) void rmsnorm_add_rows_kernel(float* __restrict__ x, const TY* __restrict__ y, const float* __restrict__ w,
                                                                   int hidden, float eps, const TN* __restrict__ next_w, TO* __restrict__ out,
-                                                                  float next_eps) {
+                                                                  float* __restrict__ ssq, float next_eps) {
   __shared__ float scratch[2][16];
+  __shared__ __align__(16) float turned[CHUNKS * kBlock * 8];
   const size_t at = static_cast<size_t>(blockIdx.x) * hidden;
   float yv[CHUNKS][8], xv[CHUNKS][8], wv[CHUNKS][8], nv[NEXT ? CHUNKS : 1][8];
 #pragma unroll
@@ -73,11 +81,16 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_add_rows_kernel(float* __restr
       if constexpr (NEXT) load_eight(next_w + i, nv[c]);
     }
   }
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) store_eight(turned + (c * kBlock + threadIdx.x) * 8, yv[c]);
+  __syncthreads();
+  // (fmaf: of an unrolled sum the compiler may join the second product with the first instead of the other way round)
   float ss = 0.f;
 #pragma unroll
-  for (int c = 0; c < CHUNKS; ++c)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss += yv[c][e] * yv[c][e];
+  for (int j = 0; j < CHUNKS * 8; ++j) {
+    const float v = turned[j * kBlock + threadIdx.x];          // (zeros beyond the row)
+    ss = fmaf(v, v, ss);
+  }
   const float scale = 1.0f / sqrtf(block_sum(ss, scratch[0]) / static_cast<float>(hidden) + eps);
   ss = 0.f;
 #pragma unroll
@@ -87,11 +100,18 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_add_rows_kernel(float* __restr
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       xv[c][e] += yv[c][e] * scale * wv[c][e];
-      if constexpr (NEXT) ss += xv[c][e] * xv[c][e];
+      if constexpr (NEXT == kNorm) ss += xv[c][e] * xv[c][e];
     }
     store_eight(x + at + i, xv[c]);
+    if constexpr (NEXT == kPrepared) {
+      float o[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = xv[c][e] * nv[c][e];
+      store_eight(out + at + i, o);
+      store_eight(turned + i, xv[c]);                          // (y has been summed)
+    }
   }
-  if constexpr (NEXT) {
+  if constexpr (NEXT == kNorm) {
     const float next_scale = 1.0f / sqrtf(block_sum(ss, scratch[1]) / static_cast<float>(hidden) + next_eps);
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
@@ -102,6 +122,20 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_add_rows_kernel(float* __restr
       for (int e = 0; e < 8; ++e) o[e] = xv[c][e] * next_scale * nv[c][e];
       store_eight(out + at + i, o);
     }
+  }
+  if constexpr (NEXT == kPrepared) {
+    __syncthreads();
+    if (threadIdx.x >= kWave) return;
+#pragma unroll
+    for (int j = 0; j < CHUNKS * 4; ++j) {
+      const int i = (j * kWave + threadIdx.x) * 8;
+      if (i >= hidden) continue;
+      float v[8];
+      load_eight(turned + i, v);
+      ss = add_squares(v, j > 0, ss);
+    }
+    ss = wave_sum(ss);
+    if (threadIdx.x == 0) ssq[blockIdx.x] = ss;
   }
 }
 
@@ -368,10 +402,11 @@ bool on_16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 }  // namespace bc4g
 
 extern "C" int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const float* w, const void* next_w, int next_w_dtype, float next_eps,
-                                void* out, int out_dtype, int n_rows, int hidden, float eps, void* stream) {
+                                void* out, int out_dtype, float* ssq, int n_rows, int hidden, float eps, void* stream) {
   BC4G_REQUIRE(n_rows >= 0 && hidden > 0 && x && y && w && !next_w == !out, "rmsnorm_add: bad arguments rows=%d H=%d", n_rows, hidden);
   BC4G_REQUIRE((y_dtype == kF32 || y_dtype == kBF16) && (!out || ((next_w_dtype == kF32 || next_w_dtype == kBF16) && (out_dtype == kF32 || out_dtype == kBF16))),
                "rmsnorm_add: unknown dtypes y=%d next=%d out=%d", y_dtype, next_w_dtype, out_dtype);
+  BC4G_REQUIRE(!ssq || (out && out_dtype == kBF16), "rmsnorm_add: a prepared norm is bfloat16 rows and their sums of squares");
   const bool rows = hidden % 8 == 0 && hidden <= 8192 && on_16(x) && on_16(y) && on_16(w) && on_16(next_w) && on_16(out);
   BC4G_REQUIRE(!out || rows, "rmsnorm_add: the norm after it takes widths of a multiple of 8 up to 8192 on 16-byte boundaries (H=%d)", hidden);
   if (n_rows == 0) return 0;
@@ -384,7 +419,7 @@ extern "C" int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const floa
   const int chunks = (hidden + 2047) / 2048;
 #define BC4G_ADD_ROWS(TY, TN, TO, C, NEXT)                                                                                              \
   rmsnorm_add_rows_kernel<TY, TN, TO, C, NEXT><<<n_rows, kBlock, 0, s>>>(x, static_cast<const TY*>(y), w, hidden, eps,                 \
-                                                                         static_cast<const TN*>(next_w), static_cast<TO*>(out), next_eps)
+                                                                         static_cast<const TN*>(next_w), static_cast<TO*>(out), ssq, next_eps)
 #define BC4G_ADD(TY, TN, TO, NEXT)                                   \
   do {                                                               \
     if (chunks == 1) BC4G_ADD_ROWS(TY, TN, TO, 1, NEXT);             \
@@ -393,11 +428,13 @@ extern "C" int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const floa
   } while (0)
 #define BC4G_ADD_NEXT(TY)                                                                   \
   do {                                                                                      \
-    if (!out) BC4G_ADD(TY, float, float, false);                                            \
-    else if (next_w_dtype == kF32 && out_dtype == kF32) BC4G_ADD(TY, float, float, true);   \
-    else if (next_w_dtype == kF32) BC4G_ADD(TY, float, bf16_t, true);                       \
-    else if (out_dtype == kF32) BC4G_ADD(TY, bf16_t, float, true);                          \
-    else BC4G_ADD(TY, bf16_t, bf16_t, true);                                                \
+    if (!out) BC4G_ADD(TY, float, float, kNothing);                                         \
+    else if (ssq && next_w_dtype == kF32) BC4G_ADD(TY, float, bf16_t, kPrepared);           \
+    else if (ssq) BC4G_ADD(TY, bf16_t, bf16_t, kPrepared);                                  \
+    else if (next_w_dtype == kF32 && out_dtype == kF32) BC4G_ADD(TY, float, float, kNorm);  \
+    else if (next_w_dtype == kF32) BC4G_ADD(TY, float, bf16_t, kNorm);                      \
+    else if (out_dtype == kF32) BC4G_ADD(TY, bf16_t, float, kNorm);                         \
+    else BC4G_ADD(TY, bf16_t, bf16_t, kNorm);                                               \
   } while (0)
   if (y_dtype == kF32) BC4G_ADD_NEXT(float);
   else BC4G_ADD_NEXT(bf16_t);

@@ -802,18 +802,23 @@ def gemm_fast(a: torch.Tensor, w, out_dtype=None,
     return out
 
 
-def gemm_xielu(a: torch.Tensor, w, pq: torch.Tensor) -> Optional[torch.Tensor]:
+def gemm_xielu(a: torch.Tensor, w, pq: torch.Tensor, pre: Optional["Prenormed"] = None) -> Optional[torch.Tensor]:
     """xielu(a w^T) in bfloat16 with the activation in the streaming kernel's epilogue (to the product rounded to bfloat16, as
-    the kernel behind a product would find it), where that kernel takes the product; else None."""
+    the kernel behind a product would find it), where that kernel takes the product; else None.  With ``pre`` (a = pre.xb) the norm
+    before the product was prepared by the kernel that last added into the stream."""
     w, packed = _weight(w)
     if not _fast_operands(a, w) or packed is None or a.shape[0] > SKINNY_MAX_ROWS or not streams_weights(a.shape[0], *w.shape):
         return None
-    _dev("gemm_xielu", a, w, pq)
+    parts = pre.parts if pre is not None else None
+    if pre is not None and (a is not pre.xb or parts.dim() != 2):
+        return None
+    _dev("gemm_xielu", a, w, pq, parts)
     _f32("gemm_xielu", "pq", pq, (2,))
     m, k = a.shape
     n = w.shape[0]
     out = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
-    library.call("bc4g_gemm_skinny_xielu", _ptr(a), _ptr(packed), _ptr(out), _ptr(pq), m, n, k, _stream(), cost=_skinny_cost(m, n, k, 2, 2))
+    library.call("bc4g_gemm_skinny_xielu", _ptr(a), _ptr(parts), parts.shape[0] if pre is not None else 0, parts.shape[1] if pre is not None else 0,
+                 pre.eps if pre is not None else 0.0, _ptr(packed), _ptr(out), _ptr(pq), m, n, k, _stream(), cost=_skinny_cost(m, n, k, 2, 2))
     return out
 
 
@@ -825,9 +830,13 @@ def _normed_rows_fit(n_rows: int, k: int, n: int = 0) -> bool:
 
 def gemm_normed_supported(x: torch.Tensor, n_rows: int, g: torch.Tensor, w) -> bool:
     """Whether RMSNorm can be fused into the product: few rows, bfloat16 weights, k a multiple of 8."""
+    return x.is_cuda and x.dtype == torch.float32 and x.shape[1] == w.shape[1] and absorbs_norm(n_rows, g, w)
+
+
+def absorbs_norm(n_rows: int, g: torch.Tensor, w) -> bool:
+    """gemm_normed_supported for a stream of the weight's width that is not at hand yet."""
     w, _ = _weight(w)
-    return (x.is_cuda and x.dtype == torch.float32 and w.dtype == torch.bfloat16 and x.shape[1] == w.shape[1]
-            and _normed_rows_fit(n_rows, x.shape[1], w.shape[0]) and x.shape[1] % 8 == 0 and g.dtype in _CODE)
+    return w.dtype == torch.bfloat16 and _normed_rows_fit(n_rows, w.shape[1], w.shape[0]) and w.shape[1] % 8 == 0 and g.dtype in _CODE
 
 
 def gemm_normed(x: torch.Tensor, rows: Optional[torch.Tensor], n_rows: int, g: torch.Tensor, eps: float,
@@ -1390,17 +1399,20 @@ def _norms_whole_rows(hidden: int, *tensors: Optional[torch.Tensor]) -> bool:
     return hidden % 8 == 0 and hidden <= 8192 and not any(t.data_ptr() % 16 for t in tensors if t is not None)
 
 
-def rmsnorm_add(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float, next_norm=None) -> Optional[torch.Tensor]:
+def rmsnorm_add(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float, next_norm=None, prepare: bool = False):
     """x += y * rsqrt(mean(y^2) + eps) * weight, row by row, in place on the float residual stream x [T, H];
     y [T, H] float32 or bfloat16, weight float32 [H] (as it multiplies).  Returns x.  With ``next_norm`` (scale, eps, dtype) the
-    RMSNorm of the new x is made in the same kernel and returned instead, where the kernel takes the width (else None is)."""
+    RMSNorm of the new x is made in the same kernel and returned instead, where the kernel takes the width (else None is) -- with
+    ``prepare`` (bfloat16) not that norm but what a product that absorbs it takes (Prenormed, in one part)."""
     _dev("rmsnorm_add", x, y, weight)
     if x.dtype != torch.float32 or x.dim() != 2 or tuple(y.shape) != tuple(x.shape):
         raise KernelError(f"rmsnorm_add: x must be float32 [T, H] and y of its shape, got {x.dtype} {tuple(x.shape)} and {tuple(y.shape)}")
     n, hidden = x.shape
     _f32("rmsnorm_add", "weight", weight, (hidden,))
-    scale = out = None
+    scale = out = ssq = None
     next_eps, dtypes = 0.0, (0, 0)
+    if prepare and (next_norm is None or next_norm[2] != torch.bfloat16):
+        raise KernelError("rmsnorm_add: what is prepared is a norm in bfloat16")
     if next_norm is not None and _norms_whole_rows(hidden, x, y, weight, next_norm[0]):
         scale, next_eps = next_norm[0], float(next_norm[1])
         _dev("rmsnorm_add", scale)
@@ -1408,9 +1420,12 @@ def rmsnorm_add(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: flo
             raise KernelError(f"rmsnorm_add: the next norm's scale must be [{hidden}], got {tuple(scale.shape)}")
         out = torch.empty((n, hidden), dtype=next_norm[2], device=x.device)
         dtypes = _code(scale, "rmsnorm_add"), _code(out, "rmsnorm_add")
+        ssq = torch.empty((1, n), dtype=torch.float32, device=x.device) if prepare else None
     library.call("bc4g_rmsnorm_add", _ptr(x), _ptr(y), _code(y, "rmsnorm_add"), _ptr(weight), _ptr(scale), dtypes[0], next_eps, _ptr(out), dtypes[1],
-                 n, hidden, float(eps), _stream(), cost=lambda: (5.0 * n * hidden, n * hidden * (8 + y.element_size())))
-    return x if next_norm is None else out
+                 _ptr(ssq), n, hidden, float(eps), _stream(), cost=lambda: (5.0 * n * hidden, n * hidden * (8 + y.element_size())))
+    if next_norm is None:
+        return x
+    return Prenormed(out, ssq, next_eps) if ssq is not None else out
 
 
 def rmsnorm_conv(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, out_dtype: torch.dtype, weight: torch.Tensor, state: torch.Tensor,

@@ -169,15 +169,18 @@ class SandwichBlock(Part):
         y = self._sum_for(self.mixer, x)
         self.mixer.forward(h, ctx, mixer_cache, y, writes)
         h = None
-        if self.ffn is not None and hasattr(self.mixer_post_norm, "add_and_norm"):     # (one kernel where there is one)
-            h = self.mixer_post_norm.add_and_norm(x, self._sum_of(y), self.ffn_norm)
+        # A feed-forward that says so gets the norm not yet computed: its first product absorbs it for few rows.  The add leaves
+        # what that product takes then, and else the norm (for a feed-forward that does not say which, neither).
+        lazy = self.ffn is not None and getattr(self.ffn, "accepts_lazy_norm", False)
+        absorbs = self.ffn.absorbs_norm(x.shape[0], self.ffn_norm) if hasattr(self.ffn, "absorbs_norm") else None if lazy else False
+        if self.ffn is not None and absorbs is not None and hasattr(self.mixer_post_norm, "add_and_norm"):     # (one kernel where there is one)
+            h = self.mixer_post_norm.add_and_norm(x, self._sum_of(y), self.ffn_norm, prepare=absorbs)
         else:
             self.mixer_post_norm.add_to(x, self._sum_of(y))
         if self.ffn is not None:
             y = self._sum_for(self.ffn, x)
-            # (a feed-forward that says so gets the norm not yet computed: its first product absorbs it for few rows)
-            if getattr(self.ffn, "accepts_lazy_norm", False):
-                h = Normed(x, self.ffn_norm, ctx, done=h)
+            if lazy:
+                h = Normed(x, self.ffn_norm, ctx, pre=h) if absorbs else Normed(x, self.ffn_norm, ctx, done=h)
             elif h is None:
                 h = self.ffn_norm.forward(x, ctx)
             self.ffn.forward(h, ctx, y)

@@ -9,7 +9,7 @@ from ..csrc import ops
 from ..errors import ConfigError
 from ..weights.loader import WeightSpec
 from .base import Part, register_part
-from .linear import linear, linear_squared_relu, linear_swiglu, linear_xielu
+from .linear import absorbs_norm, linear, linear_squared_relu, linear_swiglu, linear_xielu
 
 
 class SwiGLU(Part):
@@ -80,6 +80,10 @@ class DenseXIELU(Part):
         self.w_down = ops.StreamedWeight(tensors["down"])
         self.pq = tensors["act"].to(torch.float32).contiguous()
         self.act_dtype = rt.act_dtype
+
+    def absorbs_norm(self, n_rows: int, norm) -> bool:
+        """Whether the first product absorbs the norm before it at this many rows."""
+        return self.act_dtype == torch.bfloat16 and absorbs_norm(norm, self.w_up, n_rows)
 
     def forward(self, h, ctx, residual) -> None:
         linear(linear_xielu(h, self.w_up, self.pq, self.act_dtype), self.w_down, accumulate_into=residual, ctx=ctx)

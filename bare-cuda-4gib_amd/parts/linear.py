@@ -24,6 +24,12 @@ def _fused_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
     return ops.gemm_normed(x.x, x.rows, x.n_rows, scale[0], scale[1], w, epilogue)
 
 
+def absorbs_norm(norm, w, n_rows: int) -> bool:
+    """Whether a product of n_rows rows of the stream with this weight absorbs the norm before it (_fused_norm)."""
+    scale = norm.fusable() if hasattr(norm, "fusable") else None
+    return scale is not None and ops.absorbs_norm(n_rows, scale[0], w)
+
+
 def _prepared_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
     """The product from what the product before left for this norm, where there is such a thing."""
     if x.pre is None or x._tensor is not None or not ops.gemm_prenormed_supported(x.pre, w, epilogue):
@@ -94,10 +100,17 @@ def linear_squared_relu(x: Union[torch.Tensor, Normed], w, out_dtype: torch.dtyp
 
 
 def linear_xielu(x: Union[torch.Tensor, Normed], w, pq: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
-    """xielu(x W^T) with its two numbers pq: inside the product's kernel where few rows stream the weights, else by a kernel
-    behind it."""
-    if out_dtype == torch.bfloat16 and not (isinstance(x, Normed) and x.pre is not None):
+    """xielu(x W^T) with its two numbers pq: inside the product's kernel where few rows stream the weights (with the norm prepared, if
+    it was), else by a kernel behind it."""
+    if out_dtype == torch.bfloat16:
         if isinstance(x, Normed):
+            if x.pre is not None and x._tensor is None:
+                fast = ops.gemm_xielu(x.pre.xb, w, pq, pre=x.pre)
+                if fast is not None:
+                    return fast
+            z = _fused_norm(x, w, ops.EPI_STORE_BF16)
+            if z is not None:
+                return ops.xielu(z, pq, out=z)
             x = x.tensor()
         fast = ops.gemm_xielu(x, w, pq)
         if fast is not None:

@@ -4,7 +4,7 @@ counted from it: y = x * rsqrt(...) * (offset + w) -- a weight stored around zer
 is cut into that many equal runs of neighbouring channels, every run is brought to unit mean square by itself, and one weight spans the row."""
 from __future__ import annotations
 
-from typing import Dict, Optional
+from typing import Dict
 
 import torch
 
@@ -38,13 +38,14 @@ class RMSNorm(Part):
         """x += norm(y), in place on the float32 residual stream: the norm after a sublayer."""
         return ops.rmsnorm_add(x, y, self._adds_as(), self.eps)
 
-    def add_and_norm(self, x: torch.Tensor, y: torch.Tensor, following) -> Optional[torch.Tensor]:
-        """add_to, and where one kernel can make it too the norm ``following`` of the new x -- else None."""
+    def add_and_norm(self, x: torch.Tensor, y: torch.Tensor, following, prepare: bool = False):
+        """add_to, and where one kernel can make it too the norm ``following`` of the new x -- else None.  ``prepare``: its reader is
+        a product that absorbs the norm, and what that takes (ops.Prenormed) is left instead."""
         scale = following.fusable() if type(following) is RMSNorm else None      # (a norm derived from it may do more)
         if scale is None:
             self.add_to(x, y)
             return None
-        return ops.rmsnorm_add(x, y, self._adds_as(), self.eps, next_norm=(*scale, following.out_dtype))
+        return ops.rmsnorm_add(x, y, self._adds_as(), self.eps, next_norm=(*scale, following.out_dtype), prepare=prepare)
 
     def _adds_as(self) -> torch.Tensor:
         if self.groups != 1:

@@ -41,6 +41,77 @@ def test_add_and_the_norm_after_it(ops, hidden, y_dtype, w_dtype, out_dtype):
         assert torch.equal(made, ops.rmsnorm(alone, g, 1e-5, out_dtype))
 
 
+def beside(t):
+    """The same values one element beside a 16-byte boundary: what only the scalar kernels take."""
+    room = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    room[1:] = t.reshape(-1)
+    return room[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("y_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hidden", [8, 1000, 2048, 2056, 5120, 8192])
+def test_rows_held_in_registers_add_what_the_scalar_kernel_adds(ops, hidden, y_dtype):
+    torch.manual_seed(hidden)
+    x, y, w = torch.randn(5, hidden, device=DEV), (torch.randn(5, hidden, device=DEV) * 3).to(y_dtype), torch.randn(hidden, device=DEV)
+    scalar = beside(x)
+    ops.rmsnorm_add(scalar, y, w, 1e-3)
+    ops.rmsnorm_add(x, y, w, 1e-3)
+    assert torch.equal(x, scalar)
+
+
+@pytest.mark.parametrize("g_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hidden", [8, 512, 520, 2048, 5120, 6136])
+def test_norm_prepared_by_the_add_is_the_norm_a_product_absorbs(ops, hidden, g_dtype):
+    """Float products of 8 rows: a sum of squares that differs in its last bit would show in them."""
+    torch.manual_seed(hidden)
+    w, g = (torch.randn(64, hidden, device=DEV) * hidden ** -0.5).to(torch.bfloat16), torch.randn(hidden, device=DEV).to(g_dtype)
+    for _ in range(20):
+        x, y = torch.randn(8, hidden, device=DEV), torch.randn(8, hidden, device=DEV)
+        pre = ops.rmsnorm_add(x, y, g.float(), 1e-5, next_norm=(g, 1e-6, torch.bfloat16), prepare=True)
+        got = ops.gemm_prenormed(pre, w, ops.EPI_STORE_F32)
+        assert torch.equal(got, ops.gemm_normed(x, None, 8, g, 1e-6, w, ops.EPI_STORE_F32))
+
+
+@pytest.mark.parametrize("g_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [1, 5, 8, 9, 20])
+@pytest.mark.parametrize("hidden, inter", [(64, 200), (1000, 520), (2048, 8192), (4096, 1024)])
+def test_feedforward_behind_the_add_gives_what_its_launches_one_by_one_give(ops, hidden, inter, rows, g_dtype):
+    """A sandwich layer's second half: the sum added to the stream under its norm, and the product with the activation
+    that reads the stream's next norm, which absorbs that norm for few rows."""
+    from bare_cuda_4gib_amd.parts.feedforward import DenseXIELU
+    from bare_cuda_4gib_amd.parts.lazy import Normed
+    from bare_cuda_4gib_amd.parts.linear import linear
+    from bare_cuda_4gib_amd.parts.norm import RMSNorm
+    from bare_cuda_4gib_amd.parts.block import SandwichBlock
+    torch.manual_seed(rows)
+    rt = SimpleNamespace(act_dtype=torch.bfloat16, device=torch.device(DEV))
+    bf16 = lambda *shape: (torch.randn(*shape, device=DEV) * shape[-1] ** -0.5).to(torch.bfloat16)      # noqa: E731
+    norms = [RMSNorm(hidden, 1e-5) for _ in range(4)]
+    for norm in norms:
+        norm.bind({"weight": (1 + torch.randn(hidden, device=DEV) * 0.2).to(g_dtype)}, rt)
+    first, behind, second, last = norms
+    ffn = DenseXIELU(hidden, inter)
+    ffn.bind({"up": bf16(inter, hidden) * 2, "down": bf16(hidden, inter), "act": torch.tensor([0.4, -0.8], device=DEV)}, rt)
+    start, sums = torch.randn(rows, hidden, device=DEV), torch.randn(rows, hidden, device=DEV) * 3
+
+    class Mixer:
+        adds_one_product = True
+
+        def forward(self, h, ctx, cache, y, writes):
+            y.tensor = sums.clone()
+
+    ctx = SimpleNamespace(n_tokens=rows, handoff=SimpleNamespace(reading_next=None))
+    x = start.clone()
+    SandwichBlock(Mixer(), first, behind, ffn, second, last).forward(x, ctx, None)
+    want = start.clone()
+    want_sums = beside(sums)
+    behind.add_to(want, want_sums)
+    z = linear(Normed(want, second), ffn.w_up, out_dtype=torch.bfloat16)
+    y = linear(ops.xielu(z, ffn.pq, out=z), ffn.w_down, out_dtype=torch.float32)
+    last.add_to(want, beside(y))
+    assert torch.equal(x, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("hidden", [8, 1032, 2048, 2056, 4096])
 @pytest.mark.parametrize("taps, bias", [(2, True), (3, False), (4, True), (4, False)])
