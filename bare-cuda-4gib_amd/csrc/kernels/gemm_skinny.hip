@@ -620,15 +620,22 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
       // need half the registers, and all of them are on the CUs at once -- the gate-up product of 8
       // rows after a prepared norm: a decode step 1.020 -> 0.990 ms)
       const int blocks = static_cast<int>(grid.x);
+      // A last batch of eight that four would hold -- every k up to 1,024, where it is the only one, and 2,049 to 3,072 -- adds
+      // nothing but work for zeros: four there (8 rows: 1,024 x 1,024 3.84 us with eight, 3.34 with four, 2,560 x 3,072 6.57 and 6.34,
+      // 256 x 64 2.47 and 2.35).  Without such a batch eight are 0.99 to 1.14 times as fast for one row and 0.94 to 1.08 for 8, over
+      // 512 to 3,072 outputs by 1,152 to 8,192.
+      const int last = (a.k + kWaves * 64 - 1) / (kWaves * 64) * 2 % 8;
+      const bool eights = last == 0 || last > 4;
       if constexpr (EPI == kAccumF32 || EPI == kStoreF32 || EPI == kStoreBf16) {
         if (b.halves) {
           grid.x *= 2;
-          gemm_skinny_kernel<1, EPI, XMODE, 8, 8, true><<<grid, block, 0, s>>>(b);
+          if (eights) gemm_skinny_kernel<1, EPI, XMODE, 8, 8, true><<<grid, block, 0, s>>>(b);
+          else gemm_skinny_kernel<1, EPI, XMODE, 4, 8, true><<<grid, block, 0, s>>>(b);
           return check_launch("gemm_skinny");
         }
       }
       if (blocks > 2 * compute_units()) gemm_skinny_kernel<1, EPI, XMODE, 2, 8><<<grid, block, 0, s>>>(b);
-      else if (4 * blocks <= 3 * compute_units()) gemm_skinny_kernel<1, EPI, XMODE, 8, 8><<<grid, block, 0, s>>>(b);
+      else if (eights && 4 * blocks <= 3 * compute_units()) gemm_skinny_kernel<1, EPI, XMODE, 8, 8><<<grid, block, 0, s>>>(b);
       else gemm_skinny_kernel<1, EPI, XMODE, 4, 8><<<grid, block, 0, s>>>(b);
       return check_launch("gemm_skinny");
     }

@@ -13,7 +13,7 @@ def ops():
 
 
 @pytest.mark.parametrize("m", [1, 2, 7, 8])
-@pytest.mark.parametrize("n, k", [(8, 1024), (24, 1032), (2048, 2048), (2040, 5632), (2048, 1016), (2056, 1024), (3072, 264), (3088, 4096)])
+@pytest.mark.parametrize("n, k", [(8, 1024), (24, 1032), (2048, 2048), (2040, 5632), (2048, 1016), (2056, 1024), (3072, 264), (3088, 4096), (1024, 64), (3000, 1024), (2048, 3072), (2040, 3080), (3072, 2056)])
 def test_eight_rows_are_the_first_of_more(ops, monkeypatch, m, n, k):
     """Every row's sums are the same bits as in a step of 16 rows (other batches, whole blocks) and as with a block a workgroup."""
     torch.manual_seed(n + m)
