@@ -42,7 +42,7 @@ class RMSNorm(Part):
         """add_to, and where one kernel can make it too the norm ``following`` of the new x -- else None.  ``prepare``: its reader is
         a product that absorbs the norm, and what that takes (ops.Prenormed) is left instead."""
         scale = following.fusable() if type(following) is RMSNorm else None      # (a norm derived from it may do more)
-        if scale is None:
+        if scale is None or type(self).add_to is not RMSNorm.add_to:
             self.add_to(x, y)
             return None
         return ops.rmsnorm_add(x, y, self._adds_as(), self.eps, next_norm=(*scale, following.out_dtype), prepare=prepare)

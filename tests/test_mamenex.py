@@ -153,3 +153,18 @@ def test_plain_model_runs_every_configuration():
         # causal: a later token changes nothing before it
         again = plain.forward(config, w, [1, 2, 3, 4, 9, 6, 7])
         assert torch.equal(again[:4], logits[:4]) and not torch.allclose(again[4:], logits[4:])
+
+
+def test_a_norm_that_adds_in_its_own_way_is_left_to_add():
+    """The launch that makes the next norm beside the addition stands for RMSNorm's own addition, not for a derived one's."""
+    from bare_cuda_4gib_amd.parts.norm import RMSNorm
+
+    class Halved(RMSNorm):
+        def add_to(self, x, y):
+            x += 0.5 * y
+            return x
+
+    following = RMSNorm(4, 1e-5)
+    following.weight, following.out_dtype = torch.ones(4), torch.float32
+    x, y = torch.zeros(2, 4), torch.ones(2, 4)
+    assert Halved(4, 1e-5).add_and_norm(x, y, following) is None and torch.equal(x, 0.5 * y)
