@@ -127,11 +127,14 @@ int bc4g_sample(const float* logits, const float* temperature, const double* u, 
 // (engine/src/sampler.cpp:63-104).  Not for a row with neither limit: bc4g_sample walks those in the order of the ids.
 int bc4g_sample_filtered(const float* logits, const int32_t* rows, const float* temperature, const double* u,
                          const int32_t* top_k, const double* top_p, int32_t* out, int n, int vocab, void* stream);
-// A step's tokens at once, the rows' options on the HOST (they travel in the launch's arguments, 64 rows a launch): row i
+// A step's tokens at once, the rows' options on the HOST (they travel in the launch's arguments: at most 64 rows): row i
 // greedy where temperature[i] is not above 0, by bc4g_sample_filtered's law where top_k[i] (of 1 .. vocab - 1) or top_p[i]
 // (below 1) limits it, else by bc4g_sample's.
 int bc4g_choose(const float* logits, const float* temperature, const double* u, const int32_t* top_k, const double* top_p,
                 int32_t* out, int n_rows, int vocab, void* stream);
+// The same for any number of rows, their options on the device; top_k and top_p null: no row has a limit.
+int bc4g_choose_listed(const float* logits, const float* temperature, const double* u, const int32_t* top_k, const double* top_p,
+                       int32_t* out, int n_rows, int vocab, void* stream);
 }
 
 extern "C" {

@@ -816,6 +816,29 @@ struct ChooseArgs {
   float temperature[kChooseRows];
   int top_k[kChooseRows];
 };
+// The same on the device, for any number of rows: entry i is logits row rows[i] (null: row i).
+struct ChooseLists {
+  const int32_t* rows;
+  const float* temperature;
+  const double* u;
+  const int32_t* top_k;
+  const double* top_p;
+};
+
+// One row's token to `to`.  HELD: as draw_filtered has it.
+template <bool HELD>
+__device__ inline void choose_row(Shared& sh, const float* from, int vocab, float temperature, double u, int top_k, double top_p, bool filtered,
+                                  unsigned int* room, int32_t* to) {
+  if (filtered) {
+    const int token = draw_filtered<HELD>(sh, from, vocab, temperature, u, top_k, top_p, room);
+    if (threadIdx.x == 0) *to = token;
+  } else {
+    draw_unfiltered(sh, from, vocab, temperature, u, reinterpret_cast<double*>(room), to);
+  }
+}
+__host__ __device__ inline bool limited(float temperature, int top_k, double top_p, int vocab) {
+  return temperature > 0.f && ((top_k > 0 && top_k < vocab) || top_p < 1.0);
+}
 
 template <bool HELD>
 __global__ __launch_bounds__(kThreads) void choose_kernel(const float* __restrict__ logits, int32_t* __restrict__ out, int vocab,
@@ -823,50 +846,52 @@ __global__ __launch_bounds__(kThreads) void choose_kernel(const float* __restric
   __shared__ Shared sh;
   extern __shared__ __align__(16) unsigned int room[];
   const int row = blockIdx.x;
+  choose_row<HELD>(sh, logits + static_cast<size_t>(row) * vocab, vocab, a.temperature[row], a.u[row], a.top_k[row], a.top_p[row],
+                   limited(a.temperature[row], a.top_k[row], a.top_p[row], vocab), room, out + row);
+}
+
+// kNone: no row has a limit (a kernel of half the registers, so that two workgroups share a CU: a choice of 512
+// rows of 32,000 198 us, 242 with the law with filters beside it); kSome: those that have; kEvery: every row by the law with filters, whatever its limits.
+enum Limits : int { kNone = 0, kSome = 1, kEvery = 2 };
+
+template <bool HELD, bool LIMITS>
+__global__ __launch_bounds__(kThreads) void choose_listed_kernel(const float* __restrict__ logits, int32_t* __restrict__ out, int vocab,
+                                                                 const ChooseLists a, int limits) {
+  __shared__ Shared sh;
+  extern __shared__ __align__(16) unsigned int room[];
+  const int i = blockIdx.x, row = a.rows ? a.rows[i] : i;
   const float* from = logits + static_cast<size_t>(row) * vocab;
-  if (a.temperature[row] > 0.f && ((a.top_k[row] > 0 && a.top_k[row] < vocab) || a.top_p[row] < 1.0)) {
-    const int token = draw_filtered<HELD>(sh, from, vocab, a.temperature[row], a.u[row], a.top_k[row], a.top_p[row], room);
-    if (threadIdx.x == 0) out[row] = token;
+  if constexpr (LIMITS) {
+    choose_row<HELD>(sh, from, vocab, a.temperature[i], a.u[i], a.top_k[i], a.top_p[i],
+                     limits == kEvery || limited(a.temperature[i], a.top_k[i], a.top_p[i], vocab), room, out + row);
   } else {
-    draw_unfiltered(sh, from, vocab, a.temperature[row], a.u[row], reinterpret_cast<double*>(room), out + row);
+    draw_unfiltered(sh, from, vocab, a.temperature[i], a.u[i], reinterpret_cast<double*>(room), out + row);
   }
 }
 
-__global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
-                                                          const double* __restrict__ u, int32_t* __restrict__ out, int vocab) {
-  __shared__ Shared sh;
-  __shared__ double group_sum[kSampleMaxGroups];
-  const int row = blockIdx.x;
-  draw_unfiltered(sh, logits + static_cast<size_t>(row) * vocab, vocab, temperature[row], u[row], group_sum, out + row);
-}
-
-template <bool HELD>
-__global__ __launch_bounds__(kThreads) void sample_filtered_kernel(
-    const float* __restrict__ logits, const int32_t* __restrict__ rows, const float* __restrict__ temperature,
-    const double* __restrict__ u, const int32_t* __restrict__ top_k, const double* __restrict__ top_p,
-    int32_t* __restrict__ out, int vocab) {
-  __shared__ Shared sh;
-  extern __shared__ __align__(16) unsigned int room[];
-  const int i = blockIdx.x, row = rows[i];
-  const int token = draw_filtered<HELD>(sh, logits + static_cast<size_t>(row) * vocab, vocab, temperature[i], u[i], top_k[i], top_p[i], room);
-  if (threadIdx.x == 0) out[row] = token;
-}
-
-constexpr int kRoomBytes = kRoom * 4;
-static_assert((kRoom - kMaxHeld) * 4 >= 3 * kFew * 8 && (kRoom - kMaxHeld) * 4 >= kFine * 8 && kRoomBytes >= kSampleMaxGroups * 8,
+// LDS of a workgroup: with the vocabulary's patterns, a CU to itself; without, room for two on a CU.
+constexpr int kHeldBytes = kRoom * 4, kPlainBytes = kSampleMaxGroups * 8;
+static_assert((kRoom - kMaxHeld) * 4 >= 3 * kFew * 8 && (kRoom - kMaxHeld) * 4 >= kFine * 8 && kPlainBytes >= (kRoom - kMaxHeld) * 4,
               "the sorted tokens, the buckets, and in a mixed launch a plain row's sums over groups");
 
 int raise_room() {
   static std::once_flag once;
   static hipError_t raised = hipSuccess;
   std::call_once(once, [] {
-    const void* kernels[] = {reinterpret_cast<const void*>(sample_filtered_kernel<true>), reinterpret_cast<const void*>(sample_filtered_kernel<false>),
-                             reinterpret_cast<const void*>(choose_kernel<true>), reinterpret_cast<const void*>(choose_kernel<false>)};
+    const void* kernels[] = {reinterpret_cast<const void*>(choose_listed_kernel<true, true>), reinterpret_cast<const void*>(choose_kernel<true>)};
     for (const void* kernel : kernels)
-      if (raised == hipSuccess) raised = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kRoomBytes);
+      if (raised == hipSuccess) raised = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kHeldBytes);
   });
-  if (raised != hipSuccess) return fail("sampling: cannot raise the dynamic LDS limit to %d bytes", kRoomBytes);
+  if (raised != hipSuccess) return fail("sampling: cannot raise the dynamic LDS limit to %d bytes", kHeldBytes);
   return 0;
+}
+
+int choose_listed(const char* what, const float* logits, const ChooseLists& lists, int32_t* out, int n, int vocab, Limits limits, hipStream_t s) {
+  if (int e = raise_room()) return e;
+  if (limits == kNone) choose_listed_kernel<false, false><<<n, kThreads, kPlainBytes, s>>>(logits, out, vocab, lists, limits);
+  else if (vocab <= kMaxHeld) choose_listed_kernel<true, true><<<n, kThreads, kHeldBytes, s>>>(logits, out, vocab, lists, limits);
+  else choose_listed_kernel<false, true><<<n, kThreads, kPlainBytes, s>>>(logits, out, vocab, lists, limits);
+  return check_launch(what);
 }
 
 }  // namespace
@@ -878,8 +903,8 @@ extern "C" int bc4g_sample(const float* logits, const float* temperature, const 
                            int n_rows, int vocab, void* stream) {
   BC4G_REQUIRE(n_rows >= 0 && vocab > 0, "sample: bad sizes rows=%d V=%d", n_rows, vocab);
   if (n_rows == 0) return 0;
-  sample_kernel<<<n_rows, kThreads, 0, static_cast<hipStream_t>(stream)>>>(logits, temperature, u, out, vocab);
-  return check_launch("sample");
+  return choose_listed("sample", logits, ChooseLists{nullptr, temperature, u, nullptr, nullptr}, out, n_rows, vocab, kNone,
+                       static_cast<hipStream_t>(stream));
 }
 
 // For each of n rows: draws the token of logits row rows[i] by the law above with temperature[i] (> 0), the
@@ -890,31 +915,34 @@ extern "C" int bc4g_sample_filtered(const float* logits, const int32_t* rows, co
                                     void* stream) {
   BC4G_REQUIRE(n >= 0 && vocab > 0, "sample_filtered: bad sizes rows=%d V=%d", n, vocab);
   if (n == 0) return 0;
-  if (int e = raise_room()) return e;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (vocab <= kMaxHeld)
-    sample_filtered_kernel<true><<<n, kThreads, kRoomBytes, s>>>(logits, rows, temperature, u, top_k, top_p, out, vocab);
-  else
-    sample_filtered_kernel<false><<<n, kThreads, kRoomBytes, s>>>(logits, rows, temperature, u, top_k, top_p, out, vocab);
-  return check_launch("sample_filtered");
+  return choose_listed("sample_filtered", logits, ChooseLists{rows, temperature, u, top_k, top_p}, out, n, vocab, kEvery,
+                       static_cast<hipStream_t>(stream));
+}
+
+extern "C" int bc4g_choose_listed(const float* logits, const float* temperature, const double* u, const int32_t* top_k, const double* top_p,
+                                  int32_t* out, int n_rows, int vocab, void* stream) {
+  BC4G_REQUIRE(n_rows >= 0 && vocab > 0 && logits && temperature && u && !top_k == !top_p && out,
+               "choose: bad sizes rows=%d V=%d, or a tensor is missing", n_rows, vocab);
+  if (n_rows == 0) return 0;
+  return choose_listed("choose", logits, ChooseLists{nullptr, temperature, u, top_k, top_p}, out, n_rows, vocab, top_k ? kSome : kNone,
+                       static_cast<hipStream_t>(stream));
 }
 
 // temperature, u, top_k and top_p lie on the host.
 extern "C" int bc4g_choose(const float* logits, const float* temperature, const double* u, const int32_t* top_k, const double* top_p,
                            int32_t* out, int n_rows, int vocab, void* stream) {
-  BC4G_REQUIRE(n_rows >= 0 && vocab > 0 && logits && temperature && u && top_k && top_p && out, "choose: bad sizes rows=%d V=%d, or a tensor is missing",
-               n_rows, vocab);
+  BC4G_REQUIRE(n_rows >= 0 && n_rows <= kChooseRows && vocab > 0 && logits && temperature && u && top_k && top_p && out,
+               "choose: bad sizes rows=%d (at most %d) V=%d, or a tensor is missing", n_rows, kChooseRows, vocab);
+  if (n_rows == 0) return 0;
   if (int e = raise_room()) return e;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  for (int first = 0; first < n_rows; first += kChooseRows) {
-    const int rows = n_rows - first < kChooseRows ? n_rows - first : kChooseRows;
-    ChooseArgs a{};
-    for (int i = 0; i < rows; ++i)
-      a.temperature[i] = temperature[first + i], a.u[i] = u[first + i], a.top_k[i] = top_k[first + i], a.top_p[i] = top_p[first + i];
-    const float* from = logits + static_cast<size_t>(first) * vocab;
-    if (vocab <= kMaxHeld) choose_kernel<true><<<rows, kThreads, kRoomBytes, s>>>(from, out + first, vocab, a);
-    else choose_kernel<false><<<rows, kThreads, kRoomBytes, s>>>(from, out + first, vocab, a);
-    if (int e = check_launch("choose")) return e;
+  ChooseArgs a{};
+  bool filtered = false;
+  for (int i = 0; i < n_rows; ++i) {
+    a.temperature[i] = temperature[i], a.u[i] = u[i], a.top_k[i] = top_k[i], a.top_p[i] = top_p[i];
+    filtered = filtered || limited(temperature[i], top_k[i], top_p[i], vocab);
   }
-  return 0;
+  if (filtered && vocab <= kMaxHeld) choose_kernel<true><<<n_rows, kThreads, kHeldBytes, s>>>(logits, out, vocab, a);
+  else choose_kernel<false><<<n_rows, kThreads, kPlainBytes, s>>>(logits, out, vocab, a);
+  return check_launch("choose");
 }

@@ -37,6 +37,7 @@ _SIGNATURES = {
     "bc4g_argmax": [_P, _P, _P, _P, _I, _I, _P],
     "bc4g_sample": [_P, _P, _P, _P, _I, _I, _P],
     "bc4g_choose": [_P, _P, _P, _P, _P, _P, _I, _I, _P],
+    "bc4g_choose_listed": [_P, _P, _P, _P, _P, _P, _I, _I, _P],
     "bc4g_sample_filtered": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _P],
     "bc4g_argmax_static": [_P, _P, _I, _I, _P],
     "bc4g_probe_read": [_P, c_long, _P, _I, _P],

@@ -508,11 +508,15 @@ def sample_filtered(logits: torch.Tensor, out: torch.Tensor, rows: torch.Tensor,
     return out
 
 
+CHOOSE_ROWS = 64            # rows whose options go along as arguments of the launch
+
+
 def choose(logits: torch.Tensor, temperature: Sequence[float], u: Sequence[float], top_k: Sequence[int],
            top_p: Sequence[float]) -> torch.Tensor:
     """Every row's token, int32 [rows], in one launch: row i is greedy where temperature[i] is not above 0, drawn by the law of
     sample_filtered where top_k[i] (of 1 .. vocab - 1) or top_p[i] (below 1) limits it, else by that of sample, with the
-    uniform number u[i].  The options are host numbers: they go along as arguments of the launch."""
+    uniform number u[i].  The options are host numbers: up to CHOOSE_ROWS rows' go along as arguments of the launch, more are
+    uploaded in one piece (several launches of 64 rows would wait for one another: 256 rows of 32,000 without limits 149 us)."""
     _dev("choose", logits)
     if logits.dtype != torch.float32 or logits.dim() != 2:
         raise KernelError("choose: logits must be float32 [rows, vocab]")
@@ -520,9 +524,18 @@ def choose(logits: torch.Tensor, temperature: Sequence[float], u: Sequence[float
     if not len(temperature) == len(u) == len(top_k) == len(top_p) == rows:
         raise KernelError(f"choose: options for {len(temperature)}, {len(u)}, {len(top_k)} and {len(top_p)} rows of {rows}")
     out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
-    options = array.array("f", temperature), array.array("d", u), array.array("i", top_k), array.array("d", top_p)
-    library.call("bc4g_choose", _ptr(logits), *(o.buffer_info()[0] for o in options), _ptr(out), rows, vocab, _stream(),
-                 cost=lambda: (20.0 * rows * vocab, rows * vocab * 4))
+    us, temps = array.array("d", u), array.array("f", temperature)
+    ps, ks = array.array("d", top_p), array.array("i", top_k)
+    cost = lambda: (20.0 * rows * vocab, rows * vocab * 4)      # noqa: E731
+    if rows <= CHOOSE_ROWS:
+        library.call("bc4g_choose", _ptr(logits), *(o.buffer_info()[0] for o in (temps, us, ks, ps)), _ptr(out), rows, vocab, _stream(), cost=cost)
+    else:
+        filtered = max(ks) > 0 or min(ps) < 1.0           # (or no row is)
+        dev = torch.frombuffer(bytearray(b"".join((us, ps, temps, ks) if filtered else (us, temps))), dtype=torch.uint8)
+        dev = dev.to(logits.device, non_blocking=True)
+        at, limits = dev.data_ptr(), 8 * rows if filtered else 0
+        library.call("bc4g_choose_listed", _ptr(logits), at + 8 * rows + limits, at, at + 12 * rows + limits if filtered else None,
+                     at + limits if filtered else None, _ptr(out), rows, vocab, _stream(), cost=cost)
     return out
 
 

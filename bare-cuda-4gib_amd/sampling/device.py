@@ -35,8 +35,8 @@ class DevicePicker:
     temperature are drawn from the request's own uniform number -- by inverse CDF in the order of the ids where
     nothing filters them, and, with top-k or top-p, by the reference's law for those (the tokens by falling weight,
     the k likeliest, the fewest of them that reach top_p, the first at which u of the kept mass is passed:
-    engine/src/sampler.cpp:63-104).  One launch for a step's rows, whose options go along as its arguments; one small
-    download, and none before the next step may start (pick_later)."""
+    engine/src/sampler.cpp:63-104).  One launch for a step's rows, whose options go along as its arguments (beyond 64
+    rows in one upload before it); one small download, and none before the next step may start (pick_later)."""
 
     @staticmethod
     def _filters(p: SamplingParams, vocab: int) -> bool:

@@ -55,6 +55,22 @@ def test_ties_and_ends(ops):
     check(ops, logits, [0.9] * 140, us, ks, ps)
 
 
+@pytest.mark.parametrize("rows", [64, 65, 257])
+@pytest.mark.parametrize("kind", ["greedy and plain", "plain", "limited"])
+def test_any_number_of_rows_is_one_launch(ops, monkeypatch, rows, kind):
+    """Options in the launch's arguments, and beyond them uploaded: every row what it is by itself, and one launch for all."""
+    rng = np.random.default_rng(rows)
+    logits = (rng.standard_normal((rows, 2001)) * 3).astype(np.float32)
+    temps = [0.0 if kind == "greedy and plain" and i % 3 == 0 else 0.7 + 0.01 * (i % 40) for i in range(rows)]
+    ks, ps = ([(0, 1, 40, 5000)[i % 4] for i in range(rows)], [(1.0, 0.9)[i // 4 % 2] for i in range(rows)]) if kind == "limited" else ([0] * rows, [1.0] * rows)
+    us = rng.random(rows).tolist()
+    launched = []
+    call = ops.library.call
+    monkeypatch.setattr(ops.library, "call", lambda name, *a, **k: (launched.append(name), call(name, *a, **k))[1])
+    check(ops, logits, temps, us, ks, ps)
+    assert launched == ["bc4g_choose" if rows <= 64 else "bc4g_choose_listed"]
+
+
 def test_what_it_refuses(ops):
     logits = torch.zeros(2, 8, device=DEV)
     for bad in (dict(temperature=[1.0]), dict(top_k=[1, 2, 3])):
