@@ -9,20 +9,23 @@
 // the count reach k, where does the running sum reach top_p of the total, where does it pass u of the kept
 // mass -- is a search in a histogram over the patterns' leading bits, 64 buckets an octave: the bucket in which the answer
 // lies, and then the bucket's tokens put in order (each counts the keys before its own) with a running sum over them.
-// Where the first question's bucket and those above it hold up to 512 tokens -- a model's peaked rows, every small top-k --
-// these are put in order at once and answer all three.  A bucket's mass is kept as the integer sum of its tokens' mantissas
-// (they share the exponent), added with integer atomics: exact, and the same in every run whatever order the adds arrive in.
-// Rows whose answers lie in a bucket of more tokens than that, or below 2^-32 of the likeliest, go by walks down the patterns'
-// digits: a histogram over the top 8 bits (the exponent) of the tokens in question, the bucket in which the answer lies, then the
-// next 8 bits of that bucket's tokens, and so on over four levels to one exact pattern; tokens that share it are told apart by id.
+// A bucket of more than 512 tokens -- flat rows of a large vocabulary -- is first looked at by its next 11 bits in the same way.
+// Where the first question's bucket and those above it hold up to 512 tokens -- a model's peaked rows, a small top-k of a row that
+// is not flat there -- these are put in order at once and answer all three.  A bucket's mass is kept as the integer sum of its
+// tokens' mantissas (they share the exponent), added with integer atomics: exact, and the same in every run whatever order the
+// adds arrive in.
+// Rows whose answers lie among more tokens of all but one weight than that, or below 2^-32 of the likeliest, go by walks down the
+// patterns' digits: a histogram over the top 8 bits (the exponent) of the tokens in question, the bucket in which the answer lies,
+// then the next 8 bits of that bucket's tokens, and so on over four levels to one exact pattern; tokens that share it are told apart by id.
 // The sums over buckets are doubles.  (Sums in another order than the host's one-by-one walk over a sorted list: a boundary may
 // move by one token when u falls within rounding of it.)
 //
 // A CU takes 64 lanes' instructions a clock, so what a row costs is the number of passes over its tokens times the instructions a
 // token takes in each, and the barriers between them: a vocabulary of up to 32,768 is read once and its patterns stay in LDS.
 // 64 rows of 32,000 tokens, a mixture of limits, two in five of them flat: 26 us, 32 with the rows that have none beside them in one launch (before,
-// with walks for every question and every row's candidates listed in the order of their ids: 73, and 16 for the others' launch);
-// of 128,256: 73, flat rows 100 (130 and 450).
+// with walks for every question and every row's candidates listed in the order of their ids: 73, and 16 for the others' launch).
+// A whole choice, 8 rows of 128,256 at temperature 5 with a top-p of 0.95: 526 us so, 609 with walks for buckets of more than 512 tokens,
+// 157 with their next bits; 262,144 at temperature 1 and 0.9: 938, 1,184 and 227.
 #include <float.h>
 #include <math.h>
 
@@ -342,42 +345,60 @@ __device__ void walk(Shared& sh, const R& row, int vocab, const Prefix& universe
   }
 }
 
-// The row's tokens in 2,048 buckets in the law's order: 64 an octave from 1 down to 2^-32, and all below that in the last one.
-// A bucket's tokens share the exponent, so its mass is the sum of their mantissas, exactly -- but for the last one's, which is
-// summed as it comes.  Thread t owns buckets 2 t and 2 t + 1 from then on, with what lies above them.
+// Tokens in 2,048 buckets in the law's order, all tokens of a bucket with one exponent, so that its mass is the sum of their mantissas,
+// exactly.  Thread t owns buckets 2 t and 2 t + 1 from then on, with what lies above them.
 constexpr int kFine = 2 * kThreads;
-__device__ inline int fine_bucket(unsigned int b) {
-  const int i = 0x1fc0 - static_cast<int>(b >> 17);
-  return i < 0 ? 0 : i < kFine ? i : kFine - 1;
-}
 struct Fine {
   unsigned int count[2], above[2];
   double mass[2], above_mass[2];
   double total;
 };
-template <typename R>
-__device__ Fine look(Shared& sh, const R& row, unsigned long long* sums) {
+// The whole row's: 64 buckets an octave from 1 down to 2^-32, and all below that in the last one, whose mass is summed as it comes.
+struct Octaves {
+  static constexpr bool kLow = true;
+  __device__ int bucket(unsigned int b) const {
+    const int i = 0x1fc0 - static_cast<int>(b >> 17);
+    return i < 0 ? 0 : i < kFine ? i : kFine - 1;
+  }
+  __device__ unsigned int exponent(int i) const { return (0x1fc0u - i) >> 6; }
+};
+// One of those buckets', whose patterns begin with the bits of `first`: by the next 11 bits.
+struct Within {
+  static constexpr bool kLow = false;
+  unsigned int first;
+  __device__ int bucket(unsigned int b) const { return (b ^ first) >> 17 ? -1 : 0x7ff - static_cast<int>((b >> 6) & 0x7ff); }
+  __device__ unsigned int exponent(int) const { return first >> 23; }
+};
+// above, above_mass: what lies above the tokens in question.
+template <typename R, typename B>
+__device__ Fine look(Shared& sh, const R& row, const B& by, unsigned int above, double above_mass, unsigned long long* sums) {
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   sums[2 * tid] = sums[2 * tid + 1] = 0;
   __syncthreads();
   double low = 0.0;
   row.each([&](unsigned int b, int) {
-    const int bucket = fine_bucket(b);
+    const int bucket = by.bucket(b);
+    if (!B::kLow && bucket < 0) return;
     atomicAdd(&sums[bucket], (1ull << kCountShift) + mantissa(b));
-    if (bucket == kFine - 1) low += static_cast<double>(__uint_as_float(b));
+    if (B::kLow && bucket == kFine - 1) low += static_cast<double>(__uint_as_float(b));
   });
+  if constexpr (B::kLow) {
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) low += __shfl_xor(low, off, kWave);
-  if (lane == 0) sh.red_d[wave] = low;
+    for (int off = kWave / 2; off > 0; off >>= 1) low += __shfl_xor(low, off, kWave);
+    if (lane == 0) sh.red_d[wave] = low;
+  }
   __syncthreads();
   Fine f;
-  low = 0.0;
-  for (int w = 0; w < kWaves; ++w) low += sh.red_d[w];
+  if constexpr (B::kLow) {
+    low = 0.0;
+    for (int w = 0; w < kWaves; ++w) low += sh.red_d[w];
+  }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const unsigned long long sum = sums[2 * tid + j];
     f.count[j] = static_cast<unsigned int>(sum >> kCountShift);
-    f.mass[j] = 2 * tid + j == kFine - 1 ? low : f.count[j] ? scaled(sum & ((1ull << kCountShift) - 1ull), (0x1fc0u - (2 * tid + j)) >> 6) : 0.0;
+    f.mass[j] = B::kLow && 2 * tid + j == kFine - 1 ? low
+                : f.count[j] ? scaled(sum & ((1ull << kCountShift) - 1ull), by.exponent(2 * tid + j)) : 0.0;
   }
   const unsigned int with_count = wave_scan_u32(f.count[0] + f.count[1], lane);
   const double with_mass = wave_scan_f64(f.mass[0] + f.mass[1], lane);
@@ -386,8 +407,6 @@ __device__ Fine look(Shared& sh, const R& row, unsigned long long* sums) {
   const unsigned int lanes_count = __shfl_up(with_count, 1, kWave);
   const double lanes_mass = __shfl_up(with_mass, 1, kWave);
   __syncthreads();
-  unsigned int above = 0;
-  double above_mass = 0.0;
   f.total = 0.0;
   for (int w = 0; w < kWaves; ++w) {
     if (w < wave) above += sh.red_u[w], above_mass += sh.red_d[w];
@@ -400,8 +419,13 @@ __device__ Fine look(Shared& sh, const R& row, unsigned long long* sums) {
   return f;
 }
 
-// The bucket in which a goal is reached (as walk's modes have it), into sh.bucket (kFine: in none), and what lies above it.
-__device__ void find_bucket(Shared& sh, const Fine& f, int mode, unsigned int k, double target) {
+// The bucket in which a goal is reached (as walk's modes have it; kFine: in none), what lies above it and how many tokens it holds.
+struct Found {
+  int bucket, count;
+  unsigned int above;
+  double mass;
+};
+__device__ Found find_bucket(Shared& sh, const Fine& f, int mode, unsigned int k, double target) {
   if (threadIdx.x == 0) sh.bucket = kFine;
   __syncthreads();
 #pragma unroll
@@ -416,6 +440,38 @@ __device__ void find_bucket(Shared& sh, const Fine& f, int mode, unsigned int k,
     if (sh.bucket == 2 * static_cast<int>(threadIdx.x) + j)
       sh.bucket_above = f.above[j], sh.bucket_mass = f.above_mass[j], sh.bucket_count = static_cast<int>(f.count[j]);
   __syncthreads();
+  const Found found = {sh.bucket, sh.bucket_count, sh.bucket_above, sh.bucket_mass};
+  __syncthreads();
+  return found;
+}
+
+// Few enough tokens to be put in order among which a goal is reached: those with patterns lo .. hi, and what lies above them.
+constexpr int kFew = 512;
+struct Spot {
+  unsigned int lo, hi, above;
+  int count;
+  double mass;
+};
+enum { kNowhere = 0, kThere = 1, kTooMany = 2 };     // (kNowhere: also below the patterns from `floor` on, or in the last bucket of all)
+// looked: whether the row was looked at again, which takes the place of what was sorted.
+template <typename R>
+__device__ int find_spot(Shared& sh, const R& row, const Fine& fine, int mode, unsigned int k, double target, unsigned int floor,
+                         unsigned long long* room, Spot& spot, bool& looked) {
+  looked = false;
+  Found at = find_bucket(sh, fine, mode, k, target);
+  if (at.bucket >= kFine - 1) return kNowhere;
+  const unsigned int first = (0x1fc0u - at.bucket) << 17;
+  spot.lo = first, spot.hi = at.bucket == 0 ? 0xffffffffu : first | 0x1ffffu;
+  if (spot.hi < floor) return kNowhere;
+  if (at.count > kFew) {
+    looked = true;
+    const Fine part = look(sh, row, Within{first}, at.above, at.mass, room);
+    at = find_bucket(sh, part, mode, k, target);
+    if (at.bucket == kFine || at.count > kFew) return kTooMany;
+    spot.lo = first | (0x7ffu - at.bucket) << 6, spot.hi = spot.lo | 0x3fu;
+  }
+  spot.above = at.above, spot.count = at.count, spot.mass = at.mass;
+  return kThere;
 }
 
 // Where this thread's `mine` items go among those of all the workgroup's threads, in the order of the threads, and
@@ -453,11 +509,10 @@ __device__ void locate(Shared& sh, const R& whole, unsigned int bits, int r) {
   }
 }
 
-// The tokens of fine buckets first .. last, up to kFew of them, in the law's order: their keys (a weight's pattern above, the id's
+// The tokens with patterns lo .. hi, up to kFew of them, in the law's order: their keys (a weight's pattern above, the id's
 // complement below) in `room` + kFew, and returns this thread's running sum, up to and with the token of its number, from `above` on.
-constexpr int kFew = 512;
 template <typename R>
-__device__ double sort_few(Shared& sh, const R& row, int first, int last, double above, unsigned long long* room, int& n) {
+__device__ double sort_few(Shared& sh, const R& row, unsigned int lo, unsigned int hi, double above, unsigned long long* room, int& n) {
   unsigned long long* keys = room;
   unsigned long long* sorted = room + kFew;
   int* rank = reinterpret_cast<int*>(room + 2 * kFew);
@@ -466,8 +521,7 @@ __device__ double sort_few(Shared& sh, const R& row, int first, int last, double
   if (tid < kFew) rank[tid] = 0;
   __syncthreads();
   row.each([&](unsigned int b, int i) {
-    const int bucket = fine_bucket(b);
-    if (bucket < first || bucket > last) return;
+    if (b < lo || b > hi) return;
     const int at = atomicAdd(&sh.listed, 1);
     if (at < kFew) keys[at] = static_cast<unsigned long long>(b) << 32 | static_cast<unsigned int>(~i);
   });
@@ -551,52 +605,41 @@ __device__ int draw_from(Shared& sh, const R& row, int top_k, double p, double u
   const bool count_first = top_k > 0 && top_k < vocab;
   const unsigned int k = count_first ? static_cast<unsigned int>(top_k) : static_cast<unsigned int>(vocab);
   if (vocab > kMaxPacked) return draw_by_walks(sh, row, k, p, u);
-  const Fine fine = look(sh, row, room);
-  // The first question's bucket.  (Questions whose answer lies in the last bucket, which holds many exponents, or in one
-  // with more tokens than can be put in order go the general way.)
-  find_bucket(sh, fine, count_first ? kByCount : kByMassGe, k, p * fine.total);
-  int bucket = sh.bucket;
-  if (bucket >= kFine - 1 || sh.bucket_count > kFew) return draw_by_walks(sh, row, k, p, u);
+  const Fine fine = look(sh, row, Octaves{}, 0u, 0.0, room);
+  // Where the first question's answer lies.  (In the last bucket, which holds many exponents, or among more tokens than can be put
+  // in order: the general way.)
+  Spot at;
+  bool looked;
+  if (find_spot(sh, row, fine, count_first ? kByCount : kByMassGe, k, p * fine.total, 0u, room, at, looked) != kThere)
+    return draw_by_walks(sh, row, k, p, u);
   const unsigned long long* sorted = room + kFew;
   const double* upto = reinterpret_cast<const double*>(room);
-  const bool all = sh.bucket_above + static_cast<unsigned int>(sh.bucket_count) <= static_cast<unsigned int>(kFew);
-  double above = all ? 0.0 : sh.bucket_mass;
-  int before = all ? 0 : static_cast<int>(sh.bucket_above);         // tokens above the sorted ones
+  const bool all = at.above + static_cast<unsigned int>(at.count) <= static_cast<unsigned int>(kFew);
+  if (all) at.hi = 0xffffffffu, at.above = 0, at.mass = 0.0;        // (with every token above it)
   int n;
-  __syncthreads();
-  double mass = sort_few(sh, row, all ? 0 : bucket, bucket, above, room, n);
-  int kept = count_first ? min(static_cast<int>(k) - before, n) : n;      // of the sorted tokens
+  double mass = sort_few(sh, row, at.lo, at.hi, at.mass, room, n);
+  int kept = count_first ? min(static_cast<int>(k - at.above), n) : n;     // of the sorted tokens
   double kept_mass = upto[kept - 1];
+  // A later question's answer lies above the sorted tokens or, rounding included, among them.  False: by walks.
+  auto go_on = [&](int mode, double target) {
+    if (all) return true;
+    Spot there;
+    const int found = find_spot(sh, row, fine, mode, 0u, target, at.lo, room, there, looked);
+    if (found == kTooMany) return false;
+    const bool earlier = found == kThere && there.lo > at.lo;
+    if (earlier) at = there;
+    if (earlier || looked) mass = sort_few(sh, row, at.lo, at.hi, at.mass, room, n);
+    if (earlier) kept = n;
+    return true;
+  };
   if (p < 1.0) {
     const double target = p * (count_first ? kept_mass : fine.total);
-    if (count_first && !all) {
-      // the nucleus may end in an earlier bucket than the k likeliest do
-      find_bucket(sh, fine, kByMassGe, 0, target);
-      const int earlier = sh.bucket, count = sh.bucket_count;
-      above = sh.bucket_mass;
-      __syncthreads();
-      if (earlier < bucket) {
-        if (count > kFew) return draw_by_walks(sh, row, k, p, u);
-        bucket = earlier;
-        mass = sort_few(sh, row, bucket, bucket, above, room, n);
-        kept = n;
-      }
-    }
+    if (count_first && !go_on(kByMassGe, target)) return draw_by_walks(sh, row, k, p, u);
     kept = first_at(sh.first_ge, mass, true, target, kept) + 1;
     kept_mass = upto[kept - 1];
   }
   const double target = u * kept_mass;
-  if (!all) {
-    find_bucket(sh, fine, kByMassGt, 0, target);
-    const int earlier = sh.bucket, count = sh.bucket_count;
-    above = sh.bucket_mass;
-    __syncthreads();
-    if (earlier < bucket) {
-      if (count > kFew) return draw_by_walks(sh, row, k, p, u);
-      mass = sort_few(sh, row, earlier, earlier, above, room, n);
-      kept = n;
-    }
-  }
+  if (!go_on(kByMassGt, target)) return draw_by_walks(sh, row, k, p, u);
   return static_cast<int>(~static_cast<unsigned int>(sorted[first_at(sh.first_gt, mass, false, target, kept)]));
 }
 
@@ -855,7 +898,7 @@ __global__ __launch_bounds__(kThreads) void choose_kernel(const float* __restric
 enum Limits : int { kNone = 0, kSome = 1, kEvery = 2 };
 
 template <bool HELD, bool LIMITS>
-__global__ __launch_bounds__(kThreads) void choose_listed_kernel(const float* __restrict__ logits, int32_t* __restrict__ out, int vocab,
+__global__ __launch_bounds__(kThreads, LIMITS ? 4 : 8) void choose_listed_kernel(const float* __restrict__ logits, int32_t* __restrict__ out, int vocab,
                                                                  const ChooseLists a, int limits) {
   __shared__ Shared sh;
   extern __shared__ __align__(16) unsigned int room[];

@@ -30,9 +30,9 @@ def check(ops, logits, temps, us, ks, ps):
 
 
 # vocabularies at the edges of what is held in LDS, none a multiple of four among them, smaller than a workgroup, and beyond one reading
-@pytest.mark.parametrize("vocab", [1, 37, 1024, 32000, 32767, 32768, 32769, 50257])
-# how far the logits spread: a few candidates, buckets of hundreds, and rows flatter than the buckets resolve
-@pytest.mark.parametrize("spread", [8.0, 2.0, 0.01])
+@pytest.mark.parametrize("vocab", [1, 37, 1024, 32000, 32767, 32768, 32769, 50257, 128256])
+# how far the logits spread: a few candidates, buckets of hundreds, of more than are put in order, and rows flatter than the buckets resolve
+@pytest.mark.parametrize("spread", [8.0, 2.0, 0.4, 0.01])
 def test_every_kind_of_row(ops, vocab, spread):
     rng = np.random.default_rng(vocab)
     options = [(0.0, 0, 1.0), (0.8, 0, 1.0), (0.7, 1, 1.0), (0.7, 40, 1.0), (1.0, 0, 0.9), (1.2, 100, 0.95), (1.0, 3000, 1.0), (1.5, 9000, 0.7),
