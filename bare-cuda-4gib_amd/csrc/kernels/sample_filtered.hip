@@ -43,7 +43,7 @@ constexpr int kBuckets = 256;
 constexpr int kMaxHeld = 32768;              // tokens whose patterns go into LDS when they are first read (128 KB)
 constexpr int kRoom = kMaxHeld + 4096;       // 32-bit words of LDS a row has: the patterns, and beside them the buckets' sums or the sorted tokens
 // A bucket's count rides in the top bits of its mantissa sum, one atomic add for both, where the vocabulary
-// leaves room: 2^19 tokens of 24-bit mantissas sum to less than 2^43.
+// leaves room: 2^19 tokens of 24-bit mantissas sum to less than 2^43.  (Beyond, an add each.)
 constexpr int kCountShift = 44;
 constexpr int kMaxPacked = 1 << 19;
 
@@ -122,6 +122,7 @@ __device__ int ties_needed(int mode, unsigned int k, double target, unsigned int
 struct Cached {
   const unsigned int* bits;
   int n;
+  __device__ bool packed() const { return true; }
   __device__ unsigned int at(int i) const { return bits[i]; }
   template <typename F>
   __device__ inline void each(F f) const {
@@ -138,6 +139,7 @@ struct Logits {
   const float* logits;
   int n;
   float row_max, inv_t;
+  __device__ bool packed() const { return n <= kMaxPacked; }
   __device__ unsigned int bits_of(float l) const { return __float_as_uint(expf((l - row_max) * inv_t)); }
   __device__ unsigned int at(int i) const { return bits_of(logits[i]); }
   template <typename F>
@@ -191,7 +193,7 @@ __device__ void walk(Shared& sh, const R& row, int vocab, const Prefix& universe
   constexpr unsigned int kMask[4] = {0xffu, 0xffu, 0xffu, 0x7fu};
   constexpr int kPerLane = kBuckets / kWave;
   const int tid = threadIdx.x, lane = tid % kWave;
-  const bool packed = vocab <= kMaxPacked;
+  const bool packed = row.packed();
   if (tid == 0) {
     sh.prefix = 0;
     sh.above_count = 0;
@@ -373,13 +375,17 @@ struct Within {
 template <typename R, typename B>
 __device__ Fine look(Shared& sh, const R& row, const B& by, unsigned int above, double above_mass, unsigned long long* sums) {
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const bool packed = row.packed();                   // (else the counts stand behind the sums)
+  unsigned int* counts = reinterpret_cast<unsigned int*>(sums + kFine);
   sums[2 * tid] = sums[2 * tid + 1] = 0;
+  if (!packed) counts[2 * tid] = counts[2 * tid + 1] = 0;
   __syncthreads();
   double low = 0.0;
   row.each([&](unsigned int b, int) {
     const int bucket = by.bucket(b);
     if (!B::kLow && bucket < 0) return;
-    atomicAdd(&sums[bucket], (1ull << kCountShift) + mantissa(b));
+    atomicAdd(&sums[bucket], (packed ? 1ull << kCountShift : 0ull) + mantissa(b));
+    if (!packed) atomicAdd(&counts[bucket], 1u);
     if (B::kLow && bucket == kFine - 1) low += static_cast<double>(__uint_as_float(b));
   });
   if constexpr (B::kLow) {
@@ -396,9 +402,9 @@ __device__ Fine look(Shared& sh, const R& row, const B& by, unsigned int above, 
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const unsigned long long sum = sums[2 * tid + j];
-    f.count[j] = static_cast<unsigned int>(sum >> kCountShift);
+    f.count[j] = packed ? static_cast<unsigned int>(sum >> kCountShift) : counts[2 * tid + j];
     f.mass[j] = B::kLow && 2 * tid + j == kFine - 1 ? low
-                : f.count[j] ? scaled(sum & ((1ull << kCountShift) - 1ull), by.exponent(2 * tid + j)) : 0.0;
+                : f.count[j] ? scaled(packed ? sum & ((1ull << kCountShift) - 1ull) : sum, by.exponent(2 * tid + j)) : 0.0;
   }
   const unsigned int with_count = wave_scan_u32(f.count[0] + f.count[1], lane);
   const double with_mass = wave_scan_f64(f.mass[0] + f.mass[1], lane);
@@ -604,7 +610,6 @@ __device__ int draw_from(Shared& sh, const R& row, int top_k, double p, double u
   const int vocab = row.n;
   const bool count_first = top_k > 0 && top_k < vocab;
   const unsigned int k = count_first ? static_cast<unsigned int>(top_k) : static_cast<unsigned int>(vocab);
-  if (vocab > kMaxPacked) return draw_by_walks(sh, row, k, p, u);
   const Fine fine = look(sh, row, Octaves{}, 0u, 0.0, room);
   // Where the first question's answer lies.  (In the last bucket, which holds many exponents, or among more tokens than can be put
   // in order: the general way.)
@@ -916,6 +921,7 @@ __global__ __launch_bounds__(kThreads, LIMITS ? 4 : 8) void choose_listed_kernel
 constexpr int kHeldBytes = kRoom * 4, kPlainBytes = kSampleMaxGroups * 8;
 static_assert((kRoom - kMaxHeld) * 4 >= 3 * kFew * 8 && (kRoom - kMaxHeld) * 4 >= kFine * 8 && kPlainBytes >= (kRoom - kMaxHeld) * 4,
               "the sorted tokens, the buckets, and in a mixed launch a plain row's sums over groups");
+static_assert(kPlainBytes >= kFine * 12, "the buckets with counts of their own");
 
 int raise_room() {
   static std::once_flag once;

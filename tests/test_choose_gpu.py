@@ -41,6 +41,15 @@ def test_every_kind_of_row(ops, vocab, spread):
     check(ops, logits, [o[0] for o in options], rng.random(len(options)).tolist(), [o[1] for o in options], [o[2] for o in options])
 
 
+@pytest.mark.parametrize("vocab", [524288, 524289, 1100003])
+@pytest.mark.parametrize("spread", [2.0, 0.4])
+def test_vocabularies_whose_counts_have_words_of_their_own(ops, vocab, spread):
+    rng = np.random.default_rng(vocab)
+    options = [(0.0, 0, 1.0), (0.8, 0, 1.0), (0.7, 40, 1.0), (1.0, 0, 0.9), (1.2, 100, 0.95), (1.5, 9000, 0.7)]
+    logits = (rng.standard_normal((len(options), vocab)) * spread).astype(np.float32)
+    check(ops, logits, [o[0] for o in options], rng.random(len(options)).tolist(), [o[1] for o in options], [o[2] for o in options])
+
+
 def test_ties_and_ends(ops):
     """Rows of few distinct weights (tokens told apart by id, buckets of more tokens than are put in order), u at its ends, weights that
     vanish, and more rows than go in one launch."""
