@@ -711,9 +711,11 @@ SkinnyArgs plain_args(const void* x, const void* w, void* out, int m, int n, int
   return a;
 }
 
-int check_parts(const char* what, const float* ssq_parts, int ssq_blocks, int ssq_stride, int m, float eps) {
+int check_parts(const char* what, const float* ssq_parts, int ssq_blocks, int ssq_stride, int ssq_halves, int m, float eps) {
   BC4G_REQUIRE(ssq_parts != nullptr && ssq_blocks > 0 && ssq_stride >= m, "%s: the sums of squares need %d parts of at least %d rows",
                what, ssq_blocks, m);
+  // (where more rows are shared out over workgroups, a row's parts are counted in single numbers)
+  BC4G_REQUIRE(!ssq_halves || m <= kSplitMinRows, "%s: half blocks leave parts of at most %d rows, not of %d", what, kSplitMinRows, m);
   BC4G_REQUIRE(eps >= 0.f, "%s: eps must not be negative", what);
   return 0;
 }
@@ -739,7 +741,7 @@ extern "C" int bc4g_gemm_skinny_xielu(const void* x, const float* ssq_parts, int
   if (int e = check_common("gemm_skinny_xielu", m, 64, n, k, kXieluBf16)) return e;
   BC4G_REQUIRE(x && w && out && pq, "gemm_skinny_xielu: a tensor is missing");
   if (ssq_parts)
-    if (int e = check_parts("gemm_skinny_xielu", ssq_parts, ssq_blocks, ssq_stride, m, eps)) return e;
+    if (int e = check_parts("gemm_skinny_xielu", ssq_parts, ssq_blocks, ssq_stride, 0, m, eps)) return e;
   if (m == 0) return 0;
   SkinnyArgs a = plain_args(x, w, out, m, n, k);
   a.bias = pq;
@@ -777,7 +779,7 @@ extern "C" int bc4g_gemm_skinny_emit(const void* x, const void* w, float* out, c
 extern "C" int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts, int ssq_blocks, int ssq_stride, int ssq_halves, float eps,
                                           const void* w, void* out, int epilogue, int m, int n, int k, void* stream) {
   if (int e = check_common("gemm_skinny_prenormed", m, 64, n, k, epilogue)) return e;
-  if (int e = check_parts("gemm_skinny_prenormed", ssq_parts, ssq_blocks, ssq_stride, m, eps)) return e;
+  if (int e = check_parts("gemm_skinny_prenormed", ssq_parts, ssq_blocks, ssq_stride, ssq_halves, m, eps)) return e;
   BC4G_REQUIRE(epilogue != kAccumF32 && epilogue != kRopeKvBf16, "gemm_skinny_prenormed: epilogue %d is not supported here",
                epilogue);
   if (m == 0) return 0;
@@ -826,7 +828,7 @@ extern "C" int bc4g_gemm_skinny_qkv(const void* x, const void* g, int g_dtype, f
   if (int e = check_rope("gemm_skinny_qkv", r, n)) return e;
   BC4G_REQUIRE(!(g && ssq_parts), "gemm_skinny_qkv: the norm is either fused or prepared, not both");
   if (ssq_parts) {
-    if (int e = check_parts("gemm_skinny_qkv", ssq_parts, ssq_blocks, ssq_stride, m, eps)) return e;
+    if (int e = check_parts("gemm_skinny_qkv", ssq_parts, ssq_blocks, ssq_stride, ssq_halves, m, eps)) return e;
   }
   if (m == 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -1,0 +1,19 @@
+"""What the entries of the streaming product refuse before anything is launched: runs without a GPU."""
+import ctypes
+
+import pytest
+
+from bare_cuda_4gib_amd.csrc import library
+from bare_cuda_4gib_amd.errors import KernelError
+
+ROOM = ctypes.create_string_buffer(64)
+AT = ctypes.addressof(ROOM)            # (an address that is not looked at)
+
+
+@pytest.mark.parametrize("rows", [9, 16, 17, 64])
+def test_parts_of_half_blocks_are_of_eight_rows(rows):
+    """More rows are shared out over workgroups that count a row's parts in single numbers: pairs would be read from other rows."""
+    with pytest.raises(KernelError, match="half blocks leave parts of at most 8 rows"):
+        library.call("bc4g_gemm_skinny_prenormed", AT, AT, 1, rows, 1, 1e-5, AT, AT, 0, rows, 64, 64, None)
+    with pytest.raises(KernelError, match="half blocks leave parts of at most 8 rows"):
+        library.call("bc4g_gemm_skinny_qkv", AT, None, 0, 1e-5, AT, 1, rows, 1, AT, AT, AT, AT, AT, AT, rows, 64, 2, 1, 16, 16, 1e4, 64, 0, None)
