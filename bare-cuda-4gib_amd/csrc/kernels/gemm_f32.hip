@@ -185,7 +185,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
     if (s < n_steps) ask(s);
 
   for (int s = 0; s < n_steps; ++s) {
+    // The ring is one wave's and ordered by waits alone: a step's reads stay below the wait for its loads, and above the one
+    // after which its place is filled anew.  (To the compiler a bare wait is no access to memory: it is told.)
     wait_for_step<PER, STAGES - 1>(min(n_steps - 1, s + STAGES - 1) - s);
+    asm volatile("" ::: "memory");
     const unsigned char* at = ring + (s % STAGES) * kRing;
     const int k0 = (first + s) * kStepK;
     floatx4 wf[2], xf[MT][2];
@@ -206,7 +209,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
       }
     }
     if (s + STAGES < n_steps) {
-      __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));        // the reads are done: their place is filled anew
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the reads are done: their place is filled anew
       ask(s + STAGES);
     }
 #pragma unroll
