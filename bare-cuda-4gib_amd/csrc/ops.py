@@ -10,6 +10,7 @@ from __future__ import annotations
 import array
 import ctypes
 import dataclasses
+import functools
 import math
 from typing import Dict, Optional, Tuple
 
@@ -750,14 +751,24 @@ def streams_weights(m: int, n: int, k: int) -> bool:
     return plan_for(n, k).streams(m)
 
 
-HALF_BLOCKS = 128           # blocks of 16 outputs up to which two workgroups share one: a block for every other CU
+@functools.lru_cache(maxsize=None)
+def _units_of(device: int) -> int:
+    return torch.cuda.get_device_properties(device).multi_processor_count
+
+
+def compute_units() -> int:
+    """Of the current device (256 before there is one), as the kernels' own rules ask for them."""
+    return _units_of(torch.cuda.current_device()) if torch.cuda.is_initialized() else 256
+
+
+HALF_BLOCKS = 128           # blocks of 16 outputs up to which two workgroups share one: with 256 CUs a block for every other one
 HALF_MIN_K = 1024           # (a block of less is pulled in a fraction of what its product takes anyway)
 
 
 def half_blocks(m: int, n: int, k: int) -> bool:
     """Whether the weight-streaming kernel gives every block of 16 outputs to two workgroups: up to 8 rows, a weight of few
     and long blocks (gemm_skinny.hip says why).  The results are the same bits."""
-    return m <= 8 and k >= HALF_MIN_K and -(-n // 16) <= HALF_BLOCKS
+    return m <= 8 and k >= HALF_MIN_K and -(-n // 16) <= HALF_BLOCKS and 2 * -(-n // 16) <= compute_units()
 
 
 EPI_STORE_BF16, EPI_STORE_F32, EPI_ACCUM_F32, EPI_SWIGLU = 0, 1, 2, 3

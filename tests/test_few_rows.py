@@ -3,7 +3,7 @@ import ctypes
 
 import pytest
 
-from bare_cuda_4gib_amd.csrc import library
+from bare_cuda_4gib_amd.csrc import library, ops
 from bare_cuda_4gib_amd.errors import KernelError
 
 ROOM = ctypes.create_string_buffer(64)
@@ -17,3 +17,12 @@ def test_parts_of_half_blocks_are_of_eight_rows(rows):
         library.call("bc4g_gemm_skinny_prenormed", AT, AT, 1, rows, 1, 1e-5, AT, AT, 0, rows, 64, 64, None)
     with pytest.raises(KernelError, match="half blocks leave parts of at most 8 rows"):
         library.call("bc4g_gemm_skinny_qkv", AT, None, 0, 1e-5, AT, 1, rows, 1, AT, AT, AT, AT, AT, AT, rows, 64, 2, 1, 16, 16, 1e4, 64, 0, None)
+
+
+@pytest.mark.parametrize("units, most", [(256, 128), (304, 128), (64, 32), (32, 16)])
+def test_half_blocks_leave_a_block_for_every_other_cu(monkeypatch, units, most):
+    """As the float32 products' rule has it: two workgroups share a block where the blocks are at most half the CUs."""
+    monkeypatch.setattr(ops, "compute_units", lambda: units, raising=False)
+    for blocks in (1, 16, 17, 32, 33, 128, 129):
+        assert ops.half_blocks(8, 16 * blocks, 2048) == (blocks <= most)
+    assert not ops.half_blocks(9, 16, 2048) and not ops.half_blocks(8, 16, 1016)
