@@ -56,6 +56,8 @@ int bc4g_gemm_generic(const void* a, int a_dtype, const void* w, int w_dtype, vo
 // epilogue 0: stored; 1: added to out, with bias [n] (null: none); 2, 3: w holds n / 2 gate rows, then as many up rows, and
 // out [m, n / 2] is silu (3: the gelu written with tanh) of the gate times up.
 int bc4g_gemm_f32(const float* x, const float* w, const float* bias, float* out, int epilogue, int m, int n, int k, void* stream);
+// A question, no launch: rows of x and of w a workgroup of that product takes at once, 0 and 0 where it streams the weights.
+int bc4g_gemm_f32_tile(int m, int n, int k, int* rows, int* cols);
 
 // out[t, i] = silu(gate_i) * up_i                                        (swiglu.cu:17-25)
 // interleaved 0: gu[t] = all gates, then all ups.  1: blocks of 16 = eight gates, then the eight

@@ -452,12 +452,18 @@ int launch_tiled(const Args& a, int form, hipStream_t s) {
   }
 }
 
+// The tiled kernel's form for a product, or -1: the few rows' kernel.
+int tile_for(int m, int n, int k) {
+  if (m <= 64 || k % kStepK != 0) return -1;
+  double tiled;
+  const int form = tile_form(m, n, k, tiled);
+  return stream_time(m, n, k) < tiled ? -1 : form;
+}
+
 template <int EPI>
 int launch(const Args& a, hipStream_t s) {
-  if (a.m <= 64 || a.k % kStepK != 0) return launch_stream<EPI>(a, s);
-  double tiled;
-  const int form = tile_form(a.m, a.n, a.k, tiled);
-  return stream_time(a.m, a.n, a.k) < tiled ? launch_stream<EPI>(a, s) : launch_tiled<EPI>(a, form, s);
+  const int form = tile_for(a.m, a.n, a.k);
+  return form < 0 ? launch_stream<EPI>(a, s) : launch_tiled<EPI>(a, form, s);
 }
 
 }  // namespace
@@ -484,4 +490,11 @@ extern "C" int bc4g_gemm_f32(const float* x, const float* w, const float* bias, 
   }
   if (e) return e;
   return check_launch("gemm_f32");
+}
+
+extern "C" int bc4g_gemm_f32_tile(int m, int n, int k, int* rows, int* cols) {
+  BC4G_REQUIRE(rows != nullptr && cols != nullptr && m > 0 && n > 0 && k > 0, "gemm_f32_tile: sizes and two places for the answer");
+  const int form = tile_for(m, n, k);
+  *rows = form < 0 ? 0 : kTileForm[form][0], *cols = form < 0 ? 0 : kTileForm[form][1];
+  return 0;
 }

@@ -274,6 +274,13 @@ def gemm_f32(x: torch.Tensor, w, accumulate_into: Optional[torch.Tensor] = None,
     return out
 
 
+def gemm_f32_tile(m: int, n: int, k: int) -> Tuple[int, int]:
+    """(rows of x, rows of w) a workgroup of gemm_f32 takes, (0, 0) where it streams the weights."""
+    rows, cols = ctypes.c_int(0), ctypes.c_int(0)
+    library.call("bc4g_gemm_f32_tile", m, n, k, ctypes.byref(rows), ctypes.byref(cols), launches=False)
+    return rows.value, cols.value
+
+
 def _check_bias(what: str, bias: Optional[torch.Tensor], n: int, accumulate_into: Optional[torch.Tensor]) -> None:
     if bias is not None and (accumulate_into is None or bias.dtype != torch.float32 or tuple(bias.shape) != (n,)):
         raise KernelError(f"{what}: a bias is float32 [{n}] and joins a product that is added to something, got {bias.dtype} {tuple(bias.shape)}")
