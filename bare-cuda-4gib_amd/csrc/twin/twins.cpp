@@ -156,6 +156,24 @@ bool gemm_generic() {
       for (size_t i = 0; i < sum.size(); ++i) sum[i] += before[i] + bias[i % n];
       ok &= close("float product added", widen(acc.get()), sum, 1e-5, 1e-5);
     }
+    {   // float x float on the matrix cores: k in whole pieces of four
+      const int k4 = k - k % 4, even = n - n % 2;
+      std::vector<float> a4, w4;
+      for (int r = 0; r < m; ++r) a4.insert(a4.end(), a.begin() + static_cast<size_t>(r) * k, a.begin() + static_cast<size_t>(r) * k + k4);
+      for (int r = 0; r < n; ++r) w4.insert(w4.end(), w.begin() + static_cast<size_t>(r) * k, w.begin() + static_cast<size_t>(r) * k + k4);
+      Dev<float> da(a4), dw(w4), db(bias), out(static_cast<size_t>(m) * n), acc(before), act(static_cast<size_t>(m) * even / 2);
+      RUN(bc4g_gemm_f32(da.p, dw.p, nullptr, out.p, 0, m, n, k4, kStream));
+      RUN(bc4g_gemm_f32(da.p, dw.p, db.p, acc.p, 1, m, n, k4, kStream));
+      RUN(bc4g_gemm_f32(da.p, dw.p, nullptr, act.p, 2, m, even, k4, kStream));
+      const std::vector<double> want = plain::gemm(widen(a4), widen(w4), m, n, k4);
+      ok &= close("float product on the matrix cores", widen(out.get()), want, 1e-5, 1e-5);
+      std::vector<double> sum = want, gated;
+      for (size_t i = 0; i < sum.size(); ++i) sum[i] += before[i] + bias[i % n];
+      ok &= close("float product on the matrix cores, added", widen(acc.get()), sum, 1e-5, 1e-5);
+      for (int r = 0; r < m; ++r)
+        for (int i = 0; i < even / 2; ++i) gated.push_back(plain::swiglu(want[static_cast<size_t>(r) * n + i], want[static_cast<size_t>(r) * n + even / 2 + i]));
+      ok &= close("float product on the matrix cores, gated", widen(act.get()), gated, 1e-4, 1e-4);
+    }
     {   // bfloat16 x bfloat16 -> float
       Dev<bf16> da(as_bf16(a)), dw(as_bf16(w));
       Dev<float> out(static_cast<size_t>(m) * n);
@@ -240,6 +258,14 @@ bool gemm_skinny_norms() {
   std::vector<double> after = plain::gemm(widen(x), widen(w1), m, hidden, k1);
   for (size_t i = 0; i < after.size(); ++i) after[i] += residual[i];
   ok &= close("stream after the adding product", widen(dres.get()), after, 1e-4, 1e-4);
+  {   // the same by two workgroups a block, whose parts are pairs: the same bits
+    Dev<float> dres2(residual), ssq2(static_cast<size_t>((hidden + 15) / 16) * m * 2), y2(static_cast<size_t>(m) * n2);
+    Dev<bf16> emit_x2(static_cast<size_t>(m) * hidden);
+    RUN(bc4g_gemm_skinny_emit(dx.p, p1.p, dres2.p, nullptr, dg.p, 0, emit_x2.p, ssq2.p, m, m, hidden, k1, 1, kStream));
+    RUN(bc4g_gemm_skinny_prenormed(emit_x2.p, ssq2.p, (hidden + 15) / 16, m, 1, eps, p2.p, y2.p, 1, m, n2, hidden, kStream));
+    ok &= close("stream after half blocks", widen(dres2.get()), widen(dres.get()), 0.0, 0.0);
+    ok &= close("norm prepared by half blocks", widen(y2.get()), widen(y.get()), 0.0, 0.0);
+  }
   std::vector<double> normed2;
   for (int r = 0; r < m; ++r) {
     const std::vector<double> row = plain::rmsnorm(take(after, static_cast<size_t>(r) * hidden, hidden), widen(g), eps);
@@ -371,10 +397,11 @@ std::vector<double> twin_attention(const std::vector<std::pair<int, int>>& rows,
   return out;
 }
 
-bool attention_generic() {
-  // float32, the plain cache layout, a head size that is no multiple of 16: two requests' whole prompts in one step
+// float32, the plain cache layout, two requests' whole prompts in one step.
+bool attention_float(int d) {
   Rng rng(8);
-  const int nh = 4, nkv = 2, d = 24, page = 8, width = (nh + 2 * nkv) * d;
+  bool ok = true;
+  const int nh = 4, nkv = 2, page = 8, width = (nh + 2 * nkv) * d;
   const float theta = 10000.0f;
   const std::vector<int> lengths = {19, 11};
   Paged paged(2, page, 19, rng);
@@ -398,17 +425,28 @@ bool attention_generic() {
     values[rows[r].first].push_back(std::vector<double>(row + (nh + nkv) * d, row + width));
   }
   const size_t cache = static_cast<size_t>(paged.num_pages) * nkv * page * d;
-  bool ok = true;
   for (int window : {0, 5}) {
     Dev<float> dq(qkv), kc(cache), vc(cache), out(static_cast<size_t>(t) * nh * d);
     Dev<int32_t> dpos(positions), dslots(slots), dseq(row_seq), dtable(paged.table);
     RUN(bc4g_rope_kv_write(dq.p, 0, dpos.p, dslots.p, kc.p, vc.p, t, nh, nkv, d, d, theta, page, paged.num_pages, 1, 0, kStream));
+    const float scale = 1.0f / std::sqrt(static_cast<float>(d));
+    const std::vector<double> want = twin_attention(rows, q, keys, values, nh, nkv, d, theta, window, false);
     RUN(bc4g_attention_generic(dq.p, width, out.p, 0, kc.p, vc.p, dtable.p, paged.pages_per_seq, dseq.p, dpos.p, t, nh, nkv, d,
-                               page, paged.num_pages, window, 1.0f / std::sqrt(static_cast<float>(d)), kStream));
-    ok &= close(window ? "a window of five keys" : "all keys", widen(out.get()),
-                twin_attention(rows, q, keys, values, nh, nkv, d, theta, window, false), 1e-4, 1e-5);
+                               page, paged.num_pages, window, scale, kStream));
+    ok &= close(window ? "a window of five keys" : "all keys", widen(out.get()), want, 1e-4, 1e-5);
+    if (d % 16) continue;
+    Dev<int32_t> dstart(std::vector<int32_t>{0, lengths[0], t}), dctx(std::vector<int32_t>{0, 0});
+    Dev<float> out2(static_cast<size_t>(t) * nh * d);
+    RUN(bc4g_attention_f32(dq.p, width, out2.p, kc.p, vc.p, dtable.p, paged.pages_per_seq, dstart.p, dctx.p, 2, lengths[0], 0, nh, nkv, d,
+                           page, window, scale, kStream));
+    ok &= close(window ? "a window of five keys on the matrix cores" : "all keys on the matrix cores", widen(out2.get()), want, 1e-4, 1e-5);
   }
   return ok;
+}
+
+bool attention_generic() {      // a head size that is no multiple of 16, and one that the float32 matrix-core kernel takes too
+  const bool odd = attention_float(24);
+  return attention_float(32) && odd;
 }
 
 bool attention_mfma() {
@@ -591,6 +629,20 @@ bool sampling() {
     const int want = temps[r] > 0.0f ? plain::sample(row, temps[r], 0, 1.0, us[r]) : plain::argmax(row);
     if (got[r] != want) {
       std::printf("  without limits, row %d: %d, the twin says %d\n", r, got[r], want);
+      ok = false;
+    }
+  }
+  // a step's rows at once, their options on the host and on the device
+  Dev<int32_t> chosen(n), listed(n);
+  RUN(bc4g_choose(dl.p, temps.data(), us.data(), ks.data(), ps.data(), chosen.p, n, vocab, kStream));
+  RUN(bc4g_choose_listed(dl.p, dt.p, du.p, dk.p, dp.p, listed.p, n, vocab, kStream));
+  got = chosen.get();
+  const std::vector<int32_t> got_listed = listed.get();
+  for (int r = 0; r < n; ++r) {
+    const std::vector<float> row(logits.begin() + static_cast<size_t>(r) * vocab, logits.begin() + static_cast<size_t>(r + 1) * vocab);
+    const int want = temps[r] > 0.0f ? plain::sample(row, temps[r], ks[r], ps[r], us[r]) : plain::argmax(row);
+    if (got[r] != want || got_listed[r] != want) {
+      std::printf("  a step's rows, row %d: %d and %d, the twin says %d\n", r, got[r], got_listed[r], want);
       ok = false;
     }
   }

@@ -23,10 +23,12 @@ def ops():
 
 def check(ops, logits, temps, us, ks, ps):
     from bare_cuda_4gib_amd.sampling import SamplingParams, sample_token
-    got = ops.choose(torch.from_numpy(logits).to(DEV), temps, us, ks, ps).cpu().tolist()
+    on_device = torch.from_numpy(logits).to(DEV)
+    got = ops.choose(on_device, temps, us, ks, ps).cpu().tolist()
     want = [sample_token(row, SamplingParams(temperature=t, top_k=k, top_p=p), Fixed(u)) for row, t, u, k, p in zip(logits, temps, us, ks, ps)]
     # (a boundary may move by one token where u falls within a rounding of it: none of these draws does)
     assert got == want, [(i, g, w) for i, (g, w) in enumerate(zip(got, want)) if g != w]
+    assert ops.choose(on_device, temps, us, ks, ps).cpu().tolist() == got
 
 
 # vocabularies at the edges of what is held in LDS, none a multiple of four among them, smaller than a workgroup, and beyond one reading
@@ -77,7 +79,7 @@ def test_any_number_of_rows_is_one_launch(ops, monkeypatch, rows, kind):
     call = ops.library.call
     monkeypatch.setattr(ops.library, "call", lambda name, *a, **k: (launched.append(name), call(name, *a, **k))[1])
     check(ops, logits, temps, us, ks, ps)
-    assert launched == ["bc4g_choose" if rows <= 64 else "bc4g_choose_listed"]
+    assert launched == ["bc4g_choose" if rows <= 64 else "bc4g_choose_listed"] * 2         # (check asks twice)
 
 
 def test_what_it_refuses(ops):

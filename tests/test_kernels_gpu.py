@@ -622,12 +622,12 @@ FILTERED_ROWS = {
 
 
 @pytest.mark.parametrize("kind", sorted(FILTERED_ROWS))
-@pytest.mark.parametrize("vocab", [7, 1000, 18433, 36864, 36865, 128256])
+@pytest.mark.parametrize("vocab", [7, 1000, 18433, 32768, 32769, 36864, 36865, 128256])
 def test_filtered_sampling_follows_the_law(ops, vocab, kind):
     """Top-k, top-p and both on the device against the host's sorted walk (sampling/host.py, the reference's law)
-    for the same uniform numbers, into chosen places of the output: rows whose candidates fit the kernel's list
-    (peaked) and rows whose do not (flat: their patterns in LDS up to 36,864 tokens, worked out again beyond), rows
-    where many or all tokens share a weight (the order of the ids decides), k beyond what one bucket holds, a
+    for the same uniform numbers, into chosen places of the output: rows whose likeliest tokens are few enough to be put
+    in order at once (peaked) and rows whose are not (flat), their patterns in LDS up to 32,768 tokens and worked out again
+    beyond, rows where many or all tokens share a weight (the order of the ids decides), k beyond what one bucket holds, a
     nucleus of one token, u at both ends.  The same call twice gives the same ids (the sums are integer adds)."""
     from bare_cuda_4gib_amd.sampling import SamplingParams, sample_token
     gen = np.random.default_rng(vocab * 7 + len(kind))
@@ -669,7 +669,7 @@ def test_filtered_sampling_follows_the_law(ops, vocab, kind):
 
 def test_filtered_sampling_beyond_half_a_million_tokens(ops):
     """Beyond 2^19 tokens a bucket's count no longer fits beside its mantissa sum in one word: the kernel keeps the
-    two apart there.  Rows whose candidates fit the list and rows whose do not."""
+    two apart there.  Rows whose likeliest tokens are put in order at once and rows of ties."""
     from bare_cuda_4gib_amd.sampling import SamplingParams, sample_token
     vocab, n = 600001, 6
     gen = np.random.default_rng(5)
