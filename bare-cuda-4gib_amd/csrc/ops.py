@@ -253,7 +253,7 @@ def gemm_f32(x: torch.Tensor, w, accumulate_into: Optional[torch.Tensor] = None,
     ``accumulate_into`` and ``bias`` as in gemm_generic.  ``act`` ("silu" or "gelu_tanh"): w is gate rows followed by as many
     up rows, and the result is act(gate) * up, [M, N / 2]."""
     if (x.dtype != torch.float32 or w.dtype != torch.float32 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]
-            or x.shape[1] % 4 or not 0 < x.shape[0] <= 32 * 65535 or (act is not None and w.shape[0] % 2)):
+            or x.shape[1] % 4 or x.shape[1] > 1 << 24 or not 0 < x.shape[0] <= 32 * 65535 or (act is not None and w.shape[0] % 2)):
         return None
     w = _rows(w)
     if x.data_ptr() % 16 or w.data_ptr() % 16:

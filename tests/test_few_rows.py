@@ -1,7 +1,8 @@
-"""What the entries of the streaming product refuse before anything is launched: runs without a GPU."""
+"""What the entries of products refuse or leave to others before anything is launched: runs without a GPU."""
 import ctypes
 
 import pytest
+import torch
 
 from bare_cuda_4gib_amd.csrc import library, ops
 from bare_cuda_4gib_amd.errors import KernelError
@@ -26,3 +27,9 @@ def test_half_blocks_leave_a_block_for_every_other_cu(monkeypatch, units, most):
     for blocks in (1, 16, 17, 32, 33, 128, 129):
         assert ops.half_blocks(8, 16 * blocks, 2048) == (blocks <= most)
     assert not ops.half_blocks(9, 16, 2048) and not ops.half_blocks(8, 16, 1016)
+
+
+@pytest.mark.parametrize("k", [6, (1 << 24) + 4])
+def test_float32_products_leave_what_their_kernels_refuse_to_the_plain_one(k):
+    row = torch.empty(1, k)
+    assert ops.gemm_f32(row, row) is None
