@@ -888,17 +888,24 @@ __host__ __device__ inline bool limited(float temperature, int top_k, double top
   return temperature > 0.f && ((top_k > 0 && top_k < vocab) || top_p < 1.0);
 }
 
-template <bool HELD>
+// LIMITS false: no row has a limit -- a kernel without the other law's registers and scratch memory (64 rows of 32,000 15.5 us; with that law
+// compiled in beside it, 21.8 in a serving step).
+template <bool HELD, bool LIMITS>
 __global__ __launch_bounds__(kThreads) void choose_kernel(const float* __restrict__ logits, int32_t* __restrict__ out, int vocab,
-                                                          const ChooseArgs a) {
+                                                                          const ChooseArgs a) {
   __shared__ Shared sh;
   extern __shared__ __align__(16) unsigned int room[];
   const int row = blockIdx.x;
-  choose_row<HELD>(sh, logits + static_cast<size_t>(row) * vocab, vocab, a.temperature[row], a.u[row], a.top_k[row], a.top_p[row],
-                   limited(a.temperature[row], a.top_k[row], a.top_p[row], vocab), room, out + row);
+  const float* from = logits + static_cast<size_t>(row) * vocab;
+  if constexpr (LIMITS) {
+    choose_row<HELD>(sh, from, vocab, a.temperature[row], a.u[row], a.top_k[row], a.top_p[row],
+                     limited(a.temperature[row], a.top_k[row], a.top_p[row], vocab), room, out + row);
+  } else {
+    draw_unfiltered(sh, from, vocab, a.temperature[row], a.u[row], reinterpret_cast<double*>(room), out + row);
+  }
 }
 
-// kNone: no row has a limit (a kernel of half the registers, so that two workgroups share a CU: a choice of 512
+// kNone: no row has a limit (a kernel of its own, of half the registers, so that two workgroups share a CU: a choice of 512
 // rows of 32,000 198 us, 242 with the law with filters beside it); kSome: those that have; kEvery: every row by the law with filters, whatever its limits.
 enum Limits : int { kNone = 0, kSome = 1, kEvery = 2 };
 
@@ -927,7 +934,7 @@ int raise_room() {
   static std::once_flag once;
   static hipError_t raised = hipSuccess;
   std::call_once(once, [] {
-    const void* kernels[] = {reinterpret_cast<const void*>(choose_listed_kernel<true, true>), reinterpret_cast<const void*>(choose_kernel<true>)};
+    const void* kernels[] = {reinterpret_cast<const void*>(choose_listed_kernel<true, true>), reinterpret_cast<const void*>(choose_kernel<true, true>)};
     for (const void* kernel : kernels)
       if (raised == hipSuccess) raised = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kHeldBytes);
   });
@@ -991,7 +998,8 @@ extern "C" int bc4g_choose(const float* logits, const float* temperature, const 
     a.temperature[i] = temperature[i], a.u[i] = u[i], a.top_k[i] = top_k[i], a.top_p[i] = top_p[i];
     filtered = filtered || limited(temperature[i], top_k[i], top_p[i], vocab);
   }
-  if (filtered && vocab <= kMaxHeld) choose_kernel<true><<<n_rows, kThreads, kHeldBytes, s>>>(logits, out, vocab, a);
-  else choose_kernel<false><<<n_rows, kThreads, kPlainBytes, s>>>(logits, out, vocab, a);
+  if (!filtered) choose_kernel<false, false><<<n_rows, kThreads, kPlainBytes, s>>>(logits, out, vocab, a);
+  else if (vocab <= kMaxHeld) choose_kernel<true, true><<<n_rows, kThreads, kHeldBytes, s>>>(logits, out, vocab, a);
+  else choose_kernel<false, true><<<n_rows, kThreads, kPlainBytes, s>>>(logits, out, vocab, a);
   return check_launch("choose");
 }
