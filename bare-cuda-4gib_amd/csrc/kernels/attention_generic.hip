@@ -1,7 +1,7 @@
 // Causal softmax attention over the paged cache for any head size up to 256,
 // any head counts, float or bfloat16 storage, in plain float arithmetic.  One
-// wave per (query row, head): the attention of the 32-bit path and the fallback
-// where the MFMA kernels refuse a size.  Prompt portions and single decoded
+// wave per (query row, head): what the matrix-core kernels (bfloat16
+// and float32) refuse.  Prompt portions and single decoded
 // tokens are the same to it: every row carries its request and its position.
 //
 // Keys are walked in ascending order in tiles of 64 with a running maximum and

@@ -8,13 +8,14 @@
 // from memory into a ring of its own in LDS without passing registers -- whole cache lines of 128 bytes a row (lanes that read 16
 // rows' 16 bytes straight into operand order keep the texture path busy four times as long), several steps of 32 k ahead and
 // with no barrier; it reads its fragments there and feeds 16x16x4 MFMAs with w as the A operand.  The shares meet in LDS.
-// Eight rows, weights not in a cache, plain float FMA (gemm_generic) -> this: 32,000 x 2,048 142 -> 49 us (5.4 TB/s), 11,264 x
-// 2,048 61 -> 21, 2,048 x 5,632 86 -> 15; 32 decode steps of 8 requests after their prompts at TinyLlama's sizes 211 -> 87 ms.
+// Eight rows, weights from memory, plain float FMA (gemm_generic) -> this: 32,000 x 2,048 149 -> 51 us (5.1 TB/s), 11,264 x 2,048 59 -> 20,
+// 2,048 x 5,632 82 -> 16, 2,048 x 2,048 32 -> 7.5; 64 rows 223 -> 159, 188 -> 57, 530 -> 23 and 196 -> 11.  With the attention of
+// attention_f32.hip 32 decode steps of 8 requests after their prompts at TinyLlama's sizes take 213 -> 63 ms.
 //
 // gemm_f32_tiled_kernel, many rows, bound by the matrix cores (157 TFLOP/s of float32 at the full clock).  A step's 32 k of the
 // tile's rows of x and of w go straight into a ring of stages in LDS; the waves feed 32x32x2 MFMAs from there and keep
-// two sets of sums, the share's and the total.  2,048 x 11,264 x 2,048: 124 TFLOP/s, 2,048 x 2,048 x 5,632: 125 (plain FMA: 45 to 50); a
-// 1,000-token prompt at TinyLlama's sizes 74 -> 48 ms (30 of which is attention).
+// two sets of sums, the share's and the total.  2,048 rows: 11,264 x 2,048 128 TFLOP/s, 2,048 x 5,632 129 (plain FMA: 54 and 50); 512 rows
+// 104 and 84 (44 and 23).  With attention_f32.hip a 1,000-token prompt at TinyLlama's sizes takes 75 -> 20.5 ms.
 #include <math.h>
 
 #include "api.h"
@@ -269,7 +270,7 @@ int launch_stream(const Args& a, hipStream_t s) {
   const int cols = gated(EPI) ? 8 : 16, n_out = gated(EPI) ? a.n / 2 : a.n;
   // Outputs that would leave every other CU idle: eight a workgroup, half the weights for each CU to bring and the
   // same sums.  A decode step's two such products, 2,048 x 2,048 and
-  // 2,048 x 5,632, from memory, 8 rows: 13.05 -> 11.7 us on average; 32 steps of 8 requests after their prompts 67.6 -> 63.5 ms.
+  // 2,048 x 5,632, from memory, 8 rows, inside a step: 13.05 -> 11.7 us on average; 32 steps of 8 requests after their prompts 67.6 -> 63.5 ms.
   if constexpr (!gated(EPI)) {
     if (a.m <= 8 && 2 * ((n_out + 15) / 16) <= compute_units()) return launch_stream_form<8, 8, EPI, true>(a, s);
   }
