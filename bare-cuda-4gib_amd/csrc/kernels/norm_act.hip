@@ -55,7 +55,7 @@ enum Following : int { kNothing = 0, kNorm = 1, kPrepared = 2 };
 // the stream next, of the new x.  kNorm: its RMSNorm, out[r, :] = x[r, :] * rsqrt(mean(x[r]^2) + next_eps) * next_w.  kPrepared: what the
 // streaming product that absorbs that norm takes instead, out[r, :] = x[r, :] * next_w in bfloat16 and ssq[r] = the sum of x[r]^2.
 // A decode step's few rows leave a workgroup a row that does nothing but wait, so everything a row needs is asked for at once
-// and held in registers: 8 rows of 2,048 in a step 5.0 us where two passes over the row took 7.6, and 4.7 with what the product after it
+// and held in registers: 8 rows of 2,048 in a step 4.4 to 5.0 us where two passes over the row took 7.6, and 4.7 with what the product after it
 // takes, whose norm was a launch of 4.2 us (from a launch to the next in a graph 2.75 us, two passes 3.83).
 // Every sum is taken in the order of the kernel whose place this takes, so that the choice of kernel moves no bit: y's
 // by the threads of the kernel above (neighbouring elements in neighbouring threads: the row is turned through LDS), a
