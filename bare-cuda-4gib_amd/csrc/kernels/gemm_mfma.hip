@@ -4,21 +4,20 @@
 // Both operands are contiguous in k.  A workgroup computes a tile of the output in k-steps of 64:
 // the rows of a and of w that the tile needs are staged in LDS, every wave reads its fragments there
 // and feeds 32x32x16 MFMAs.  Two forms:
-//  - gemm_mfma_direct_kernel: the operand tiles go from memory into LDS without passing registers
-//    (k a multiple of 64, operands on 16-byte boundaries).  Tiles of 256 x 256, 256 x 192,
-//    256 x 128, 128 x 128 or 64 x 64 (and 128 x 64 for q|k|v), whichever lets the busiest CU finish first.
+//  - the operand tiles go from memory into LDS without passing registers (k a multiple of 64, operands on 16-byte
+//    boundaries): gemm_mfma_halves_kernel for tiles of 256 x 256, gemm_mfma_turns_kernel for 256 x 192 and 128 x 128,
+//    gemm_mfma_direct_kernel for 256 x 128 and 64 x 64 (and 128 x 64 for q|k|v); whichever lets the busiest CU finish
+//    first, or two of them side by side (parts_of).
 //  - gemm_mfma_staged_kernel: through registers, 128 x 128 tiles; any k that is a multiple of 8.
 // Every output element is accumulated over k in ascending order in both, whatever the number of
 // rows and the tile: the same bits whichever form and tile a shape selects.
 // Rows and columns beyond the matrix are not stored.
 //
-// What bounds these kernels (clock reads per workgroup, hardware counters): the loop over k is 85-90 %
-// of a tile's time, with the matrix cores busy 40-50 % of it -- a step's loads, fragment reads and
-// MFMAs overlap only so far between two barriers, although LDS (no bank conflicts, a third of its
-// cycles in use) and memory (a ring of three stages is no faster than one of two) both have room;
-// a tile of 128 x 64 was bound by what all CUs pull from L2 together (19 TB/s); the rest
-// is the stores after the loop, which all CUs issue at the same time.  More waves a CU (this form
-// spends no registers on staging) and larger tiles (less traffic per FLOP) are what helped.
+// What bounds these kernels: the loop over k is 85-90 % of a tile's time.  With all waves of a workgroup reading, waiting and
+// multiplying together (gemm_mfma_direct_kernel) the matrix cores are busy 40-50 % of it; where two groups of waves take turns, one
+// multiplying while the other reads, 60-70 %, and then it is LDS that is full (a 256 x 256 tile's step of 64 is 192 KB read and 64 KB
+// written, 2,000 clocks of the 2,048 its MFMAs take) and, over the whole chip, power: MFMAs on random operands alone run at 1,670 of
+// 2,500 TFLOP/s.  The rest is the stores after the loop, which all CUs issue at the same time.
 //
 // Workgroups are numbered so that those sharing rows of a and of w run on the same XCD at the same
 // time (tile_of).
@@ -452,6 +451,29 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_staged_kernel(
   store_patch<EPI, kThreads, kBM, kBN>(tile_out, out, m, n, m0, n0, tid, RowScale{}, bias);
 }
 
+// A tile goes out through LDS so that a thread stores several neighbouring columns of a row at once: every wave for itself,
+// 32 rows of its part at a time through a patch of its own (no barrier).  acc[i][j][r] is row i 32 + 8 (r / 4) + 4 (lane / 32) + r % 4 and
+// column j 32 + lane % 32 of the part, which begins at (m0, n0); part_sum: see row_scaled (the part's first row's sums, rows of a tile apart).
+template <int EPI, int TM, int TN>
+__device__ inline void store_part(const floatx16 (&acc)[TM][TN], float* patch, void* __restrict__ out, int m, int n, int k, long m0, long n0, int lane,
+                                  const RopeKvArgs& ra, const RowScaleArgs& rows, const float* part_sum = nullptr, int tile_rows = 0) {
+  constexpr int kStride = 32 * TN + 4;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) patch[(8 * (r / 4) + 4 * (lane / 32) + r % 4) * kStride + j * 32 + lane % 32] = acc[i][j][r];
+    if constexpr (EPI == kRopeKvBf16)
+      store_patch_rope<kWave, 32, 32 * TN>(patch, static_cast<bf16_t*>(out), m, n, m0 + i * 32, n0, lane, ra);
+    else if constexpr (row_scaled(EPI))
+      store_patch<EPI, kWave, 32, 32 * TN>(patch, out, m, n, m0 + i * 32, n0, lane,
+                                           RowScale{part_sum + i * 32, tile_rows, 1.0f / static_cast<float>(k), rows.eps});
+    else
+      store_patch<EPI, kWave, 32, 32 * TN>(patch, out, m, n, m0 + i * 32, n0, lane, RowScale{}, rows.bias);
+  }
+}
+
 // ---- operands straight into LDS ---------------------------------------------------------------
 // The same product with the operand tiles going from memory into LDS without passing registers
 // (global_load_lds_dwordx4: a wave's 64 lanes bring 16 bytes each to 1 KB of consecutive LDS), in a
@@ -461,7 +483,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_staged_kernel(
 // (2048 x 11264 x 2048: 104 against 131 us; 2048 x 2048 x 5632: 52 against 74; 4096^3: 1,139 against
 // 1,015 TFLOP/s).  What did not help: a deeper ring where the tiles fill the chip (three stages are
 // slower than two; with fewer tiles than CUs a step is as long as a load takes, and four stages of a
-// 64 x 64 tile halve that: 512 x 2048 x 5632 48 -> 28 us), raising the waves' priority around the MFMAs, 128 x 64 parts for a wave with half the waves.
+// 64 x 64 tile halve that: 512 x 2048 x 5632 48 -> 28 us), raising the waves' priority around the MFMAs.
 //
 // The weight comes packed (the weight-streaming kernel's order) and its blocks are copied as they are: see the
 // kernel.  The rows of x lie in LDS without padding, BK * 2 bytes each; the 16-byte segment s of row r lies in
@@ -505,7 +527,7 @@ struct DirectShape {
 template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES, int MINWG>
 __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
     const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, void* __restrict__ out, int m, int n, int k, int m_blocks,
-    int n_blocks, const RopeKvArgs ra, const RowScaleArgs rows) {
+    int n_blocks, int n_first, const RopeKvArgs ra, const RowScaleArgs rows) {
   typedef DirectShape<WM, WN, TM, TN, BK, STAGES> S;
   constexpr int RA = S::kRowsA, RW = S::kRowsW, RB = S::kRowBytes, NW = S::kWaves;
   constexpr int kGroupRows = 1024 / RB;                    // rows a wave-wide load covers
@@ -518,7 +540,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
   const int wm = wave / WN, wn = wave % WN;
   int bm, bn;
   tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
-  const long m0 = static_cast<long>(bm) * RA, n0 = static_cast<long>(bn) * RW;
+  const long m0 = static_cast<long>(bm) * RA, n0 = n_first + static_cast<long>(bn) * RW;
   // gridDim.y > 1: k is cut into that many equal parts (each whole steps), and part y's sums go to an output of
   // its own, out + y * m * n (the plain store epilogues only: whoever reads them adds the parts up in order)
   const int nk = k / BK / static_cast<int>(gridDim.y);
@@ -687,95 +709,440 @@ __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
   }
   lds_barrier();            // the last step has been read: LDS is free for the output
 
-  // The tile goes out through LDS so that a thread stores four neighbouring columns of a row at once:
-  // every wave for itself, 32 rows of its part at a time through a patch of its own (no barrier).
-  // acc[i][j][r] is row i 32 + 8 (r / 4) + 4 (lane / 32) + r % 4 and column j 32 + lane % 32 of the part.
-  constexpr int kStride = 32 * TN + 4;
-  float* patch = reinterpret_cast<float*>(direct_lds) + wave * (S::kPatchBytes / 4);
+  store_part<EPI, TM, TN>(acc, reinterpret_cast<float*>(direct_lds) + wave * (S::kPatchBytes / 4), out, m, n, k, m0 + wm * TM * 32,
+                          n0 + wn * TN * 32, lane, ra, rows, row_scaled(EPI) ? part_sum + wm * TM * 32 : nullptr, RA);
+}
+
+// ---- the same, two groups of waves in turns ------------------------------------------------------
+// Eight waves, two on every SIMD: while four of them multiply, the other four read their next fragments and ask for operands; a
+// barrier ends both and they change places.  (One barrier more at the start sets the second four half a turn behind.)  Fragments are
+// waited for before the barrier, so whatever a group has read by the end of its turn may be written over from the turn after
+// the other group's, and what has been asked for is waited for (by hand: wait_loads) in the turn before it is read, by the waves that
+// asked, in time for both groups.  The parts of the output and their order over k are those of the kernel above.
+#define BC4G_TURN(waits)                                   \
+  do {                                                     \
+    __builtin_amdgcn_sched_barrier(0);                     \
+    asm volatile(waits "s_barrier" ::: "memory");          \
+    __builtin_amdgcn_sched_barrier(0);                     \
+  } while (0)
+#define BC4G_READ "s_waitcnt lgkmcnt(0)\n\t"
+
+// N loads of a wave to N KB of LDS side by side, load i from bases[i] (the same in every lane) plus each lane's offset.  The LDS address
+// is set once and each load adds i * 1,024 bytes to it, and to its memory address, so its base is that much short of its place.
+template <int N>
+__device__ inline void load_side_by_side(const void* const (&bases)[4], const unsigned (&off)[4], unsigned lds_address) {
+  static_assert(N == 2 || N == 4, "loads a statement");
+#define BC4G_LOAD(v, s, o) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #o "\n\t"
+  if constexpr (N == 2)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_LOAD(1, 3, 0) BC4G_LOAD(2, 4, 1024)
+                 ::"s"(lds_address), "v"(off[0]), "v"(off[1]), "s"(bases[0]), "s"(bases[1]) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_LOAD(1, 5, 0) BC4G_LOAD(2, 6, 1024) BC4G_LOAD(3, 7, 2048) BC4G_LOAD(4, 8, 3072)
+                 ::"s"(lds_address), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(bases[0]), "s"(bases[1]), "s"(bases[2]), "s"(bases[3])
+                 : "memory", "m0");
+#undef BC4G_LOAD
+}
+
+// 256 x 256: a wave's part is 128 x 64, and a step of 64 two turns: its first 64 rows by its columns, then the other 64.  So
+// a turn is 16 MFMAs, its reads 24 of 1 KB (or 8: the weight's fragments stay), and the two stages of 64 KB are written over in pieces as
+// they are read: the weight and the first rows of a step are asked for a step and a half before they are read, the other
+// rows as well.  LDS: a stage is the first rows of both row parts, the other rows, then the weight likewise by columns.
+// Against 16 waves that read and multiply together (weights from memory): 2,048 x 28,672 x 4,096 437 -> 384 us, 15,400 x 12,288 x 4,096
+// 1,440 -> 1,210 (1,040 -> 1,280 TFLOP/s), 8,192^3 960 -> 800.  Four turns of eight MFMAs a step: 3-5 % slower; four waves of 128 x 128 on
+// a SIMD each: 15-20 % slower; the waves' priority raised around the MFMAs: the same.
+struct HalvesShape {
+  static constexpr int kThreads = 512, kHalf = 16 * 1024, kStage = 4 * kHalf;
+  static constexpr int kPatchBytes = 32 * (64 + 4) * 4, kLdsBytes = 2 * kStage;
+  static_assert(8 * kPatchBytes <= kLdsBytes, "the output's patches take the stages' place");
+};
+
+template <int EPI>
+__global__ __launch_bounds__(512, 2) void gemm_mfma_halves_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
+                                                                  void* __restrict__ out, int m, int n, int k, int m_blocks, int n_blocks,
+                                                                  int n_first, const RopeKvArgs ra, const RowScaleArgs rows) {
+  typedef HalvesShape S;
+  extern __shared__ __align__(1024) unsigned char direct_lds[];
+  const unsigned lds_base = static_cast<unsigned>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)direct_lds));
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave / 4, wn = wave % 4;
+  int bm, bn;
+  tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
+  const long m0 = static_cast<long>(bm) * 256, n0 = n_first + static_cast<long>(bn) * 256;
+  const int nk = k / 64;
+
+  // What this wave brings of a half of x: 16 of its 128 rows, in two loads (rows past m: the last).  Of a half of the weight: the step's
+  // two blocks of one block row (past n: of the last), 2 KB of memory side by side.
+  const unsigned char* abase = reinterpret_cast<const unsigned char*>(a + m0 * k);
+  unsigned aoff[2][2];
+  const unsigned char* wbase[2];
+  const long w_row_blocks = (static_cast<long>(n) + 15) / 16;
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int hr = (2 * wave + i) * 8 + lane / 8;                 // row of the half,
+      const int trow = (hr / 64) * 128 + h * 64 + hr % 64;          // of the tile
+      const long row = min(static_cast<long>(m) - 1 - m0, static_cast<long>(trow));
+      aoff[h][i] = static_cast<unsigned>(row * k * 2 + ((lane % 8) ^ slot_key<128>(hr)) * 16);
+    }
+    const long block = min(w_row_blocks - 1, n0 / 16 + (wave / 2) * 4 + h * 2 + wave % 2);
+    wbase[h] = reinterpret_cast<const unsigned char*>(w) + block * (k / 32) * 1024;
+  }
+  auto ask = [&](const unsigned char* first, const unsigned char* second_less_1k, unsigned off0, unsigned off1, unsigned to) {
+    const void* bases[4] = {first, second_less_1k};
+    const unsigned off[4] = {off0, off1};
+    load_side_by_side<2>(bases, off, to);
+  };
+  auto ask_a = [&](int step, int h) {
+    const unsigned char* p = abase + static_cast<size_t>(step) * 128;
+    ask(p, p - 1024, aoff[h][0], aoff[h][1], lds_base + (step & 1) * S::kStage + h * S::kHalf + wave * 2048);
+  };
+  auto ask_w = [&](int step, int h) {
+    const unsigned char* p = wbase[h] + static_cast<size_t>(step) * 2048;
+    ask(p, p, lane * 16, lane * 16, lds_base + (step & 1) * S::kStage + (2 + h) * S::kHalf + wave * 2048);
+  };
+
+  floatx16 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  const int frow = lane % 32, fhalf = lane / 32;
+  const unsigned char* aread = direct_lds + (wm * 64 + frow) * 128;
+  const int akey = slot_key<128>(wm * 64 + frow);       // (the same 32 rows further)
+  const unsigned char* wread = direct_lds + 2 * S::kHalf + (wn * 2 + frow / 16) * 2048 + (frow % 16) * 16 + fhalf * 256;
+  uint4 fa[2][4], fw[2][4];
+  auto read_a = [&](int buf, int h) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        fa[i][s] = *reinterpret_cast<const uint4*>(aread + buf * S::kStage + h * S::kHalf + i * 4096 + (((s * 2 + fhalf) ^ akey) * 16));
+  };
+  auto read_w = [&](int buf) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        fw[h][s] = *reinterpret_cast<const uint4*>(wread + buf * S::kStage + h * S::kHalf + (s / 2) * 1024 + (s % 2) * 512);
+  };
+  auto multiply = [&](int i0) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i0 + i][j] = mfma_32x32x16(fa[i][s], fw[j][s], acc[i0 + i][j]);
+  };
+  // A wave's loads in the order asked: ... W(t), first rows (t), other rows (t) ... in 4 + 2 + 2.  In the first turn of step t the
+  // other rows of t are waited for (behind them: 6 of t + 1 and the 2 just asked for), in the second W and the first rows of t + 1
+  // (behind them: 2 of t + 1 and the 6 of t + 2).
+  auto step = [&](int t, int buf) {
+    read_w(buf);
+    read_a(buf, 0);
+    if (t + 1 < nk) ask_a(t + 1, 1);
+    if (t + 2 < nk) wait_loads<8>(); else wait_loads<0>();
+    BC4G_TURN(BC4G_READ);
+    multiply(0);
+    BC4G_TURN("");
+    read_a(buf, 1);
+    if (t + 2 < nk) {
+      ask_w(t + 2, 0), ask_w(t + 2, 1), ask_a(t + 2, 0);
+      wait_loads<8>();
+    } else {
+      wait_loads<0>();
+    }
+    BC4G_TURN(BC4G_READ);
+    multiply(2);
+    BC4G_TURN("");
+  };
+
+  ask_w(0, 0), ask_w(0, 1), ask_a(0, 0), ask_a(0, 1);
+  if (nk > 1) {
+    ask_w(1, 0), ask_w(1, 1), ask_a(1, 0);
+    wait_loads<8>();
+  } else {
+    wait_loads<0>();
+  }
+  BC4G_TURN("");
+  if (wm == 1) BC4G_TURN("");
+  for (int t = 0; t < nk; t += 2) {
+    step(t, 0);
+    if (t + 1 < nk) step(t + 1, 1);
+  }
+  if (wm == 0) BC4G_TURN("");
+  lds_barrier();            // the last step has been read: LDS is free for the output
+  store_part<EPI, 4, 2>(acc, reinterpret_cast<float*>(direct_lds) + wave * (S::kPatchBytes / 4), out, m, n, k, m0 + wm * 128, n0 + wn * 64, lane, ra,
+                        rows);
+}
+
+// Any tile: a turn is a step of BK, in a ring of STAGES.  256 x 192 (steps of 32: what LDS holds five of) and 128 x 128 (steps of 64).
+// Against the kernel above: 2,048 x 11,264 x 2,048 in 256 x 192 102 -> 96 us, 2,048 x 2,048 x 5,632 in 128 x 128 60 -> 56.5, 1,024 x 4,096 x 14,336 134 ->
+// 128.  (256 x 128, whose waves read 64 x 64 parts, is LDS-bound either way: 112.6 and 113.1 us for the first; 256 x 256 so: 5 % slower than in halves.)
+template <int WM, int WN, int TM, int TN, int BK, int STAGES>
+struct TurnsShape {
+  static constexpr int kRowsA = 32 * TM * WM, kRowsW = 32 * TN * WN, kRowBytes = BK * 2;
+  static constexpr int kThreads = 512, kStageBytes = (kRowsA + kRowsW) * kRowBytes;
+  static constexpr int kPatchBytes = 32 * (32 * TN + 4) * 4;                   // a wave's 32 rows of output, as floats
+  static constexpr int kLdsBytes = STAGES * kStageBytes > 8 * kPatchBytes ? STAGES * kStageBytes : 8 * kPatchBytes;
+  static constexpr int kGroupsA = kRowsA * kRowBytes / 1024, kGroupsW = kRowsW * kRowBytes / 1024;
+  static constexpr int kLoads = (kGroupsA + kGroupsW + 7) / 8;                 // a wave's a step
+  static_assert(WM * WN == 8 && kLdsBytes <= 160 * 1024 && (BK == 32 || BK == 64) && STAGES >= 3, "eight waves, LDS, rows of 64 or 128 bytes");
+};
+// which 16-byte slot of its row a segment of x lies in (rows of 64 bytes: four of them share the banks' span)
+template <int ROW_BYTES>
+__device__ inline int turns_key(int row) {
+  return ROW_BYTES == 64 ? (row >> 2) & 3 : slot_key<128>(row);
+}
+
+template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES>
+__global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
+                                                                 void* __restrict__ out, int m, int n, int k, int m_blocks, int n_blocks,
+                                                                 int n_first, const RopeKvArgs ra, const RowScaleArgs rows) {
+  typedef TurnsShape<WM, WN, TM, TN, BK, STAGES> S;
+  constexpr int RA = S::kRowsA, RW = S::kRowsW, RB = S::kRowBytes, N = S::kLoads, kBlocksK = BK / 32, kSlices = BK / 16;
+  constexpr int kGroupRows = 1024 / RB;                    // rows of x a wave-wide load covers
+  extern __shared__ __align__(1024) unsigned char direct_lds[];
+  const unsigned lds_base = static_cast<unsigned>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)direct_lds));
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave / WN, wn = wave % WN;
+  int bm, bn;
+  tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
+  const long m0 = static_cast<long>(bm) * RA, n0 = n_first + static_cast<long>(bn) * RW;
+  const int nk = k / BK;
+
+  // the N groups of rows (of x) or blocks (of w) this wave brings every step, side by side in LDS (waves past the last group bring
+  // the last ones again: the same bytes to the same place); rows past m and blocks past n: the last
+  const int g0 = min(wave * N, S::kGroupsA + S::kGroupsW - N);
+  const unsigned char* base[4];
+  unsigned off[4];
+  int advance[4];
+  const long w_row_blocks = (static_cast<long>(n) + 15) / 16;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int g = g0 + i;
+    if (g < S::kGroupsA) {
+      const int trow = g * kGroupRows + lane * 16 / RB;
+      const long row = min(static_cast<long>(m) - 1 - m0, static_cast<long>(trow));
+      base[i] = reinterpret_cast<const unsigned char*>(a + m0 * k) - i * 1024;
+      off[i] = static_cast<unsigned>(row * k * 2 + ((lane * 16 % RB / 16) ^ turns_key<RB>(trow)) * 16);
+      advance[i] = RB;
+    } else {
+      const int gw = g - S::kGroupsA;
+      const long block = min(w_row_blocks - 1, n0 / 16 + gw / kBlocksK);
+      base[i] = reinterpret_cast<const unsigned char*>(w) + (block * (k / 32) + gw % kBlocksK) * 1024 - i * 1024;
+      off[i] = lane * 16;
+      advance[i] = kBlocksK * 1024;
+    }
+  }
+  auto ask = [&](int slot) {                               // the next step's
+    const void* from[4];
+#pragma unroll
+    for (int i = 0; i < N; ++i) from[i] = base[i], base[i] += advance[i];
+    load_side_by_side<N>(from, off, lds_base + slot * S::kStageBytes + g0 * 1024);
+  };
+
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) patch[(8 * (r / 4) + 4 * (lane / 32) + r % 4) * kStride + j * 32 + lane % 32] = acc[i][j][r];
-    if constexpr (EPI == kRopeKvBf16)
-      store_patch_rope<kWave, 32, 32 * TN>(patch, static_cast<bf16_t*>(out), m, n, m0 + (wm * TM + i) * 32, n0 + wn * TN * 32, lane, ra);
-    else if constexpr (row_scaled(EPI))
-      store_patch<EPI, kWave, 32, 32 * TN>(patch, out, m, n, m0 + (wm * TM + i) * 32, n0 + wn * TN * 32, lane,
-                                           RowScale{part_sum + (wm * TM + i) * 32, RA, 1.0f / static_cast<float>(k), rows.eps});
-    else
-      store_patch<EPI, kWave, 32, 32 * TN>(patch, out, m, n, m0 + (wm * TM + i) * 32, n0 + wn * TN * 32, lane, RowScale{}, rows.bias);
-  }
-}
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES, int MINWG>
-int launch_direct(const bf16_t* ap, const bf16_t* wp, void* out, int m, int n, int k, hipStream_t s, const RopeKvArgs& ra,
-                  int k_parts = 1, const RowScaleArgs& rows = RowScaleArgs{}) {
-  typedef DirectShape<WM, WN, TM, TN, BK, STAGES> S;
-  auto kernel = gemm_mfma_direct_kernel<EPI, WM, WN, TM, TN, BK, STAGES, MINWG>;
-  static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
+  const int frow = lane % 32, fhalf = lane / 32;
+  const unsigned char* aread = direct_lds + (wm * TM * 32 + frow) * RB;
+  const int akey = turns_key<RB>(frow);                    // (the same 32 rows further)
+  const unsigned char* wread = direct_lds + RA * RB + (wn * TN * 2 + frow / 16) * (kBlocksK * 1024) + (frow % 16) * 16 + fhalf * 256;
+  uint4 fa[TM][kSlices], fw[TN][kSlices];
+
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < nk) ask(s);
+  if (nk >= STAGES - 1) wait_loads<N * (STAGES - 2)>(); else wait_loads<0>();
+  BC4G_TURN("");
+  if (wave >= 4) BC4G_TURN("");
+  int slot = 0, free_slot = STAGES - 1;                    // (both groups have read step t - 1 when one of them comes to step t)
+  for (int t = 0; t < nk; ++t) {
+#pragma unroll
+    for (int s = 0; s < kSlices; ++s) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        fw[j][s] = *reinterpret_cast<const uint4*>(wread + slot * S::kStageBytes + j * 2 * kBlocksK * 1024 + (s / 2) * 1024 + (s % 2) * 512);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        fa[i][s] = *reinterpret_cast<const uint4*>(aread + slot * S::kStageBytes + i * 32 * RB + (((s * 2 + fhalf) ^ akey) * 16));
+    }
+    if (t + STAGES - 1 < nk) {
+      ask(free_slot);
+      wait_loads<N * (STAGES - 2)>();                      // step t + 1 is there
+    } else {
+      wait_loads<0>();
+    }
+    BC4G_TURN(BC4G_READ);
+#pragma unroll
+    for (int s = 0; s < kSlices; ++s)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma_32x32x16(fa[i][s], fw[j][s], acc[i][j]);
+    BC4G_TURN("");
+    free_slot = slot;
+    if (++slot == STAGES) slot = 0;
+  }
+  if (wave < 4) BC4G_TURN("");
+  lds_barrier();            // the last step has been read: LDS is free for the output
+  store_part<EPI, TM, TN>(acc, reinterpret_cast<float*>(direct_lds) + wave * (S::kPatchBytes / 4), out, m, n, k, m0 + wm * TM * 32,
+                          n0 + wn * TN * 32, lane, ra, rows);
+}
+#undef BC4G_TURN
+#undef BC4G_READ
+
+// What a product's kernels get: n columns, of which this launch computes n_cols from n_first on (all of them: 0, n).
+struct Operands {
+  const bf16_t* a;
+  const bf16_t* w;
+  void* out;
+  int m, n, k, n_first, n_cols;
+  hipStream_t stream;
+};
+
+// Launches kernel on tiles of rows x cols, with more than the default dynamic LDS allowed (asked for once: `raised` is the caller's).
+template <typename Kernel>
+int launch_tiles(Kernel kernel, bool& raised, int rows, int cols, int threads, int lds, const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale,
+                 int k_parts = 1) {
   if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            S::kLdsBytes) != hipSuccess)
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       return fail("gemm_mfma: cannot raise the dynamic LDS limit");
     raised = true;
   }
-  const long m_blocks = (m + S::kRowsA - 1) / S::kRowsA, n_blocks = (n + S::kRowsW - 1) / S::kRowsW;
-  kernel<<<dim3(static_cast<unsigned>(m_blocks * n_blocks), static_cast<unsigned>(k_parts)), dim3(S::kThreads), S::kLdsBytes, s>>>(
-      ap, wp, out, m, n, k, static_cast<int>(m_blocks), static_cast<int>(n_blocks), ra, rows);
+  const long m_blocks = (o.m + rows - 1) / rows, n_blocks = (o.n_cols + cols - 1) / cols;
+  kernel<<<dim3(static_cast<unsigned>(m_blocks * n_blocks), static_cast<unsigned>(k_parts)), dim3(threads), lds, o.stream>>>(
+      o.a, o.w, o.out, o.m, o.n, o.k, static_cast<int>(m_blocks), static_cast<int>(n_blocks), o.n_first, ra, scale);
   return 0;
 }
 
-// Which tile: the one with which the busiest CU finishes first.  A CU's tiles take their FLOPs over what
-// a CU sustains with that tile (TFLOP/s per CU, measured on shapes that fill the chip), and no tile is
-// faster than its k-steps follow each other when nothing else hides their latency (microseconds a step,
-// measured on shapes with fewer tiles than CUs: the small tile with four stages is for those).  A
-// function of (m, n, k) alone; every tile adds over k in the same order.
-// The rates are measured with the weights coming from memory, as they do inside a model (the caches filled
-// with other data before each run, then the activations and the output touched): a loop over one product
-// finds its weights in the 256 MB cache before memory and flatters the small tiles and the short rings --
-// 128 x 64 with two stages sustains 3.2 TFLOP/s a CU in such a loop and 2.2-2.4 behind a layer's other
-// kernels.  So the tiles that leave room in LDS keep more steps in flight: 128 x 128 (eight waves of 64 x 32,
-// four stages) took the place of 128 x 64 with two stages and four workgroups a CU, which no shape selects any
-// more but the q|k|v product (a product takes 20-29 % less time where it was selected: 2,048 x 2,048 x 5,632 85 -> 65 us), and 256 x 128
-// has three stages (5-18 % less than with two).  Five stages for 128 x 128, three for 128 x 64 (then two
-// workgroups a CU) and 128 x 128 with four waves of 64 x 64 were no better or worse.
+template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES, int MINWG>
+int launch_direct(const Operands& o, const RopeKvArgs& ra = RopeKvArgs{}, const RowScaleArgs& scale = RowScaleArgs{}, int k_parts = 1) {
+  typedef DirectShape<WM, WN, TM, TN, BK, STAGES> S;
+  static bool raised = false;
+  return launch_tiles(gemm_mfma_direct_kernel<EPI, WM, WN, TM, TN, BK, STAGES, MINWG>, raised, S::kRowsA, S::kRowsW, S::kThreads, S::kLdsBytes, o, ra,
+                      scale, k_parts);
+}
+
+template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES>
+int launch_turns(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
+  typedef TurnsShape<WM, WN, TM, TN, BK, STAGES> S;
+  static bool raised = false;
+  return launch_tiles(gemm_mfma_turns_kernel<EPI, WM, WN, TM, TN, BK, STAGES>, raised, S::kRowsA, S::kRowsW, S::kThreads, S::kLdsBytes, o, ra, scale);
+}
+
+template <int EPI>
+int launch_halves(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
+  static bool raised = false;
+  return launch_tiles(gemm_mfma_halves_kernel<EPI>, raised, 256, 256, HalvesShape::kThreads, HalvesShape::kLdsBytes, o, ra, scale);
+}
+
+// Which tile: the one with which the busiest CU finishes first.  A CU's tiles come one after the other, a turn of the chip each;
+// a tile takes its steps of 64, each as long as the fuller the chip is (L2, memory and power are shared: us a step with few tiles on
+// the chip and with one on every CU), a few us around them, and its stores.  All measured with the weights coming from memory, as they do
+// inside a model (forty weights one after the other): a loop over one product finds its weights in the 256 MB cache before
+// memory and flatters the small tiles and the short rings.  The model's times are within 5 % of those measured for 72 to 4,096 rows at
+// outputs of 2,048 to 28,672 and k of 2,048 to 14,336.  A function of (m, n, k) alone; every tile adds over k in the same order.
 struct DirectForm {
   int rows, cols;
-  double tflops_a_cu, us_a_step;
+  double us_a_step_few, us_a_step_full, us_around, us_stores;
 };
 // The last, 128 x 64 with two stages and four workgroups a CU, is for the q|k|v epilogue alone: what comes after the
 // loop is long there (rotation, three destinations), and several workgroups a CU run it beside each other's loops
 // (a 2,048-token TinyLlama prompt 1 % faster with it than with 160 tiles of 256 x 128, both libraries in one process).
 constexpr int kDirectForms = 6;
-constexpr DirectForm kDirectForm[kDirectForms] = {
-    {256, 256, 4.45, 0.5}, {256, 192, 3.9, 0.5}, {256, 128, 3.8, 0.5}, {128, 128, 3.1, 0.5}, {64, 64, 2.2, 0.28}, {128, 64, 2.9, 0.5}};
+constexpr DirectForm kDirectForm[kDirectForms] = {{256, 256, 1.12, 1.48, 4.0, 2.0}, {256, 192, 1.15, 1.40, 4.0, 1.5}, {256, 128, 0.87, 1.06, 4.0, 1.5},
+                                                  {128, 128, 0.50, 0.59, 3.5, 1.0}, {64, 64, 0.25, 0.27, 3.0, 0.25},  {128, 64, 0.67, 0.36, 6.0, 0.0}};
+
+double form_time(const DirectForm& form, int m, int n, int k) {
+  const long tiles = static_cast<long>((m + form.rows - 1) / form.rows) * ((n + form.cols - 1) / form.cols), cus = compute_units();
+  const long full = tiles / cus;
+  const double last = static_cast<double>(tiles % cus) / static_cast<double>(cus), steps = k / 64;
+  const double few = form.us_a_step_few, more = form.us_a_step_full - few;
+  if (more < 0.0) {           // (several workgroups a CU)
+    const double chip = form.us_around + static_cast<double>(tiles) / static_cast<double>(cus) * steps * form.us_a_step_full, chain = 3.0 + steps * few;
+    return chip > chain ? chip : chain;
+  }
+  return form.us_around + full * (steps * (few + more) + form.us_stores) + (last > 0.0 ? steps * (few + more * last) + form.us_stores : 0.0);
+}
 
 int direct_form(int m, int n, int k, bool long_epilogue) {
   int best = 0;
   double best_time = 0.0;
   for (int f = 0; f < (long_epilogue ? kDirectForms : kDirectForms - 1); ++f) {
-    const DirectForm& form = kDirectForm[f];
-    const long tiles = static_cast<long>((m + form.rows - 1) / form.rows) * ((n + form.cols - 1) / form.cols);
-    const long turns = (tiles + compute_units() - 1) / compute_units();
-    const double work = turns * (2.0e-6 * form.rows * form.cols * k) / form.tflops_a_cu;
-    const double chain = 3.0 + (k / 64) * form.us_a_step;
-    const double time = work > chain ? work : chain;
+    const double time = form_time(kDirectForm[f], m, n, k);
     if (f == 0 || time < best_time) best = f, best_time = time;
   }
   return best;
 }
 
+// How an output's columns are cut: the first n1 in tiles of `first`, the rest (if any) in tiles of `second`, one launch each.  Tiles that do not
+// fill the last turn of the chip leave CUs idle for a whole tile (3,000 x 11,264 are 528 tiles of 256 x 256: 256, 256 and 16); columns that fill
+// whole turns with large tiles, and smaller tiles for the others, leave less.  Every element is added up as before, by whichever tile.
+// From k = 512 on (below, a launch is as long as a tile), and where it is 4 % and more by the model, a second launch counted with the 8 us
+// by which cut products were measured to be longer than their parts: 3,000 x 11,264 x 2,048 141 -> 129 us (10,752 columns in 256 x 256, 512 in
+// 64 x 64), 1,400 x 11,264 x 2,048 84 -> 78.5, 1,100 x 28,672 x 4,096 287 -> 254.  Without the 8 us 300 x 11,264 x 2,048 was cut: 35 -> 39.
+constexpr double kCutGap = 8.0;
+struct Parts {
+  int first, n1, second;
+};
+Parts parts_of(int m, int n, int k, bool long_epilogue) {
+  Parts best{direct_form(m, n, k, long_epilogue), n, 0};
+  if (k < 512) return best;
+  double best_time = 0.96 * form_time(kDirectForm[best.first], m, n, k);
+  for (int f = 0; f < 4; ++f) {
+    const DirectForm& form = kDirectForm[f];
+    const long rows = (m + form.rows - 1) / form.rows, cus = compute_units();
+    for (long turns = rows * ((n + form.cols - 1) / form.cols) / cus; turns >= 1 && rows <= turns * cus; --turns) {
+      const long n1 = turns * cus / rows * form.cols;
+      if (n1 <= 0 || n1 >= n) continue;
+      const int rest = n - static_cast<int>(n1), second = direct_form(m, rest, k, long_epilogue);
+      const double time = form_time(form, m, static_cast<int>(n1), k) + form_time(kDirectForm[second], m, rest, k) + kCutGap;
+      if (time < best_time) best = Parts{f, static_cast<int>(n1), second}, best_time = time;
+      break;      // (fewer turns of large tiles leave more for the small ones)
+    }
+  }
+  return best;
+}
+
 template <int EPI>
-int launch_direct_form(const bf16_t* ap, const bf16_t* wp, void* out, int m, int n, int k, hipStream_t s,
-                       const RopeKvArgs& ra = RopeKvArgs{}, const RowScaleArgs& rows = RowScaleArgs{}) {
-  switch (direct_form(m, n, k, EPI == kRopeKvBf16)) {
-    case 0: return launch_direct<EPI, 4, 4, 2, 2, 64, 2, 1>(ap, wp, out, m, n, k, s, ra, 1, rows);
-    case 1: return launch_direct<EPI, 4, 2, 2, 3, 64, 2, 1>(ap, wp, out, m, n, k, s, ra, 1, rows);
-    case 2: return launch_direct<EPI, 4, 2, 2, 2, 64, 3, 1>(ap, wp, out, m, n, k, s, ra, 1, rows);
-    case 3: return launch_direct<EPI, 2, 4, 2, 1, 64, 4, 1>(ap, wp, out, m, n, k, s, ra, 1, rows);
-    case 5: return launch_direct<EPI, 2, 2, 2, 1, 64, 2, 4>(ap, wp, out, m, n, k, s, ra, 1, rows);
-    default: return launch_direct<EPI, 2, 2, 1, 1, 64, 4, 2>(ap, wp, out, m, n, k, s, ra, 1, rows);
+int launch_form(int form, const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
+  switch (form) {
+    case 0: return launch_halves<EPI>(o, ra, scale);
+    case 1: return launch_turns<EPI, 4, 2, 2, 3, 32, 5>(o, ra, scale);
+    case 2: return launch_direct<EPI, 4, 2, 2, 2, 64, 3, 1>(o, ra, scale);
+    case 3: return launch_turns<EPI, 2, 4, 2, 1, 64, 4>(o, ra, scale);
+    case 5: return launch_direct<EPI, 2, 2, 2, 1, 64, 2, 4>(o, ra, scale);
+    default: return launch_direct<EPI, 2, 2, 1, 1, 64, 4, 2>(o, ra, scale);
+  }
+}
+
+template <int EPI>
+int launch_direct_form(const bf16_t* ap, const bf16_t* wp, void* out, int m, int n, int k, hipStream_t s, const RopeKvArgs& ra = RopeKvArgs{},
+                       const RowScaleArgs& scale = RowScaleArgs{}) {
+  Operands o{ap, wp, out, m, n, k, 0, n, s};
+  if constexpr (row_scaled(EPI)) {
+    return launch_direct<EPI, 2, 2, 1, 1, 64, 4, 2>(o, ra, scale);      // (for a decode step's rows, where this is the tile anyway)
+  } else {
+    const Parts parts = parts_of(m, n, k, EPI == kRopeKvBf16);
+    o.n_cols = parts.n1;
+    if (int e = launch_form<EPI>(parts.first, o, ra, scale)) return e;
+    if (parts.n1 == n) return 0;
+    o.n_first = parts.n1, o.n_cols = n - parts.n1;
+    return launch_form<EPI>(parts.second, o, ra, scale);
   }
 }
 
@@ -858,9 +1225,8 @@ extern "C" int bc4g_gemm_mfma_parts(const void* a, const void* w, int w_packed, 
                "gemm_mfma_parts: K=%d must be %d times a multiple of 64, the weight packed and the operands on 16-byte boundaries "
                "(M=%d N=%d)", k, k_parts, m, n);
   BC4G_REQUIRE(((m + 63L) / 64) * ((n + 63L) / 64) <= 2147483647L, "gemm_mfma_parts: too many tiles");
-  if (int e = launch_direct<kStoreF32, 2, 2, 1, 1, 64, 4, 2>(static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), parts, m, n,
-                                                               k, static_cast<hipStream_t>(stream), RopeKvArgs{}, k_parts))
-    return e;
+  const Operands o{static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), parts, m, n, k, 0, n, static_cast<hipStream_t>(stream)};
+  if (int e = launch_direct<kStoreF32, 2, 2, 1, 1, 64, 4, 2>(o, RopeKvArgs{}, RowScaleArgs{}, k_parts)) return e;
   return check_launch("gemm_mfma_parts");
 }
 
@@ -894,7 +1260,7 @@ extern "C" int bc4g_gemm_mfma_qkv(const void* a, const void* w, int w_packed, vo
 extern "C" int bc4g_gemm_mfma_tile(const void* a, const void* w, int m, int n, int k, int qkv, int* rows, int* cols) {
   BC4G_REQUIRE(rows != nullptr && cols != nullptr && m > 0 && n > 0 && k > 0, "gemm_mfma_tile: sizes and two places for the answer");
   if (direct_operands(a, w, k)) {
-    const DirectForm& form = kDirectForm[direct_form(m, n, k, qkv != 0)];
+    const DirectForm& form = kDirectForm[parts_of(m, n, k, qkv != 0).first];
     *rows = form.rows, *cols = form.cols;
   } else {
     *rows = kBM, *cols = kBN;

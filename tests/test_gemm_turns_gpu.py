@@ -1,0 +1,53 @@
+"""The tiled products whose waves take turns, and outputs whose columns are cut between two tiles: against the product in
+float64 and, bit for bit, against the smallest tile (65 rows take it), at the shortest walks over k, an odd and an even number of
+steps, and at edges in both directions."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from bare_cuda_4gib_amd.csrc import ops as _ops
+    return _ops
+
+
+def rnd(*shape, seed):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).bfloat16()
+
+
+@pytest.mark.parametrize("m,n,k,tile", [
+    (3860, 3852, 64, (256, 256)), (3860, 3852, 128, (256, 256)), (3841, 3841, 320, (256, 256)),       # one row, one column in the last tile
+    (2036, 6132, 64, (256, 192)), (2036, 6132, 320, (256, 192)),
+    (2036, 2040, 128, (128, 128)), (1921, 2036, 320, (128, 128)),
+    # columns cut: 10,752 in 256 x 256 and 524 in 64 x 64, 5,376 in 256 x 256 and 780 in 128 x 128
+    (1290, 11276, 1536, (256, 256)), (2900, 6156, 2048, (256, 256))])
+def test_turns_and_cut_columns(ops, m, n, k, tile):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the shapes are chosen for 256 CUs")
+    assert ops.tiled_tile(m, n, k) == tile and ops.tiled_tile(65, n, k) == (64, 64)
+    x, w = rnd(m, k, seed=1).to(DEV), rnd(n, k, seed=2).to(DEV)
+    want = x.double() @ w.double().T
+    bound = 2.0 * k * 2.0 ** -24 * math.sqrt(k)            # k float additions of terms around 1
+    got = ops.gemm_fast(x, w, torch.float32)
+    assert (got.double() - want).abs().max() < bound
+    few = x[:65].contiguous()
+    assert torch.equal(ops.gemm_fast(few, w, torch.float32), got[:65])
+    last = x[m - 65:].contiguous()
+    assert torch.equal(ops.gemm_fast(last, w, torch.float32), got[m - 65:])
+    assert torch.equal(ops.gemm_fast(x, w, torch.bfloat16), got.bfloat16())
+    base, bias = torch.randn(m, n, device=DEV), torch.randn(n, device=DEV)
+    assert torch.equal(ops.gemm_fast(x, w, accumulate_into=base.clone(), bias=bias), base + (got + bias))
+    half = n // 32 * 16                                     # gate and up rows in blocks of eight
+    rows = torch.stack([w[:half].view(-1, 8, k), w[half:2 * half].view(-1, 8, k)], dim=1).reshape(2 * half, k).contiguous()
+    act = ops.gemm_swiglu(x, rows, interleaved=True)
+    assert torch.equal(ops.gemm_swiglu(few, rows, interleaved=True), act[:65])
+    gate, up = want[:, :half], want[:, half:2 * half]
+    exact = gate / (1 + torch.exp(-gate)) * up
+    assert ((act.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + 3 * bound * (1 + gate.abs() + up.abs())).all()
