@@ -56,6 +56,20 @@ int bc4g_gemm_generic(const void* a, int a_dtype, const void* w, int w_dtype, vo
 // epilogue 0: stored; 1: added to out, with bias [n] (null: none); 2, 3: w holds n / 2 gate rows, then as many up rows, and
 // out [m, n / 2] is silu (3: the gelu written with tanh) of the gate times up.
 int bc4g_gemm_f32(const float* x, const float* w, const float* bias, float* out, int epilogue, int m, int n, int k, void* stream);
+// Up to 64 rows of it around an RMSNorm that no kernel of its own computes.  _emit: residual += x w^T (+ bias) and, for the norm with scale g
+// of the new residual, emit_x = residual * g and the rows' sums of squares over blocks of 16 columns, emit_ssq [ceil(n / 16)][m] -- or
+// [ceil(n / 16)][m][2] (halves), which is what m <= 8 rows leave whose blocks of 16 columns are no more than half the compute units.
+// _prenormed: the product of such an x; row by row the sums are multiplied by 1 / sqrt(sum of the parts / k + eps).
+int bc4g_gemm_f32_emit(const float* x, const float* w, const float* bias, float* residual, const float* g, float* emit_x, float* emit_ssq,
+                       int halves, int m, int n, int k, void* stream);
+int bc4g_gemm_f32_prenormed(const float* x, const float* ssq, int ssq_blocks, int ssq_halves, float eps, const float* w, float* out, int epilogue,
+                            int m, int n, int k, void* stream);
+// Up to 64 rows of the q|k|v product (w: query heads, key heads, value heads; head_dim a multiple of 16; x prepared as above, or ssq null), the
+// heads of q [m, n_heads * head_dim] and k rotated over all of head_dim by a table from bc4g_rope_table_double (null: not), keys and values
+// written to the caches as bc4g_rope_kv_write does (write_kv 0: not).
+int bc4g_gemm_f32_qkv(const float* x, const float* ssq, int ssq_blocks, int ssq_halves, float eps, const float* w, float* q, const float* table,
+                      const int32_t* slot_map, float* k_cache, float* v_cache, int m, int k, int n_heads, int n_kv_heads, int head_dim,
+                      int page_tokens, int write_kv, void* stream);
 // A question, no launch: rows of x and of w a workgroup of that product takes at once, 0 and 0 where it streams the weights.
 int bc4g_gemm_f32_tile(int m, int n, int k, int* rows, int* cols);
 
@@ -88,6 +102,8 @@ int bc4g_rope_kv_write(void* qkv, int dtype, const int32_t* positions, const int
 // The angles of a step, for every layer to share: table [n_tokens, rotary_dim / 2, 2] = (cos, sin)
 // of position * theta^(-2i / rotary_dim).
 int bc4g_rope_table(const int32_t* positions, float* table, int n_tokens, int rotary_dim, float theta, void* stream);
+// The same with the angles worked out in double, as the 32-bit path has them.
+int bc4g_rope_table_double(const int32_t* positions, float* table, int n_tokens, int rotary_dim, float theta, void* stream);
 
 // bc4g_rope_kv_write for the block layout (block_pairs), rotating by a table from bc4g_rope_table
 // (rotate != 0: the whole head, rotary_dim == head_dim), in 16-byte pieces.

@@ -294,17 +294,25 @@ __global__ void rope_kv_write_kernel(T* __restrict__ qkv, const int32_t* __restr
 }
 
 // The angles of a step, once for all layers: table[token][i] = (cos, sin) of position * theta^(-2i/dim),
-// i < dim/2, with the precise powf / sincosf of the kernel above.
+// i < dim/2, worked out as the kernel above does: with powf / sincosf, or (DOUBLE, the 32-bit path) in double.
+template <bool DOUBLE>
 __global__ void rope_table_kernel(const int32_t* __restrict__ positions, float2* __restrict__ table, long total,
                                   int rhalf, float theta) {
   const long stride = static_cast<long>(blockDim.x) * gridDim.x;
   for (long idx = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; idx < total; idx += stride) {
     const int i = static_cast<int>(idx % rhalf);
     const long token = idx / rhalf;
-    const float inv_freq = 1.0f / powf(theta, (2.0f * static_cast<float>(i)) / static_cast<float>(2 * rhalf));
-    float s, c;
-    sincosf(static_cast<float>(positions[token]) * inv_freq, &s, &c);
-    table[idx] = make_float2(c, s);
+    if constexpr (DOUBLE) {
+      const double inv_freq = 1.0 / pow(static_cast<double>(theta), (2.0 * i) / static_cast<double>(2 * rhalf));
+      double s, c;
+      sincos(static_cast<double>(positions[token]) * inv_freq, &s, &c);
+      table[idx] = make_float2(static_cast<float>(c), static_cast<float>(s));
+    } else {
+      const float inv_freq = 1.0f / powf(theta, (2.0f * static_cast<float>(i)) / static_cast<float>(2 * rhalf));
+      float s, c;
+      sincosf(static_cast<float>(positions[token]) * inv_freq, &s, &c);
+      table[idx] = make_float2(c, s);
+    }
   }
 }
 
@@ -632,9 +640,20 @@ extern "C" int bc4g_rope_table(const int32_t* positions, float* table, int n_tok
                "rope_table: bad arguments (T=%d, rotary_dim=%d)", n_tokens, rotary_dim);
   if (n_tokens == 0) return 0;
   const long total = static_cast<long>(n_tokens) * (rotary_dim / 2);
-  rope_table_kernel<<<grid_for(total), kBlock, 0, static_cast<hipStream_t>(stream)>>>(
+  rope_table_kernel<false><<<grid_for(total), kBlock, 0, static_cast<hipStream_t>(stream)>>>(
       positions, reinterpret_cast<float2*>(table), total, rotary_dim / 2, theta);
   return check_launch("rope_table");
+}
+
+extern "C" int bc4g_rope_table_double(const int32_t* positions, float* table, int n_tokens, int rotary_dim, float theta,
+                                      void* stream) {
+  BC4G_REQUIRE(n_tokens >= 0 && rotary_dim > 0 && rotary_dim % 2 == 0 && theta > 0.f && positions && table,
+               "rope_table_double: bad arguments (T=%d, rotary_dim=%d)", n_tokens, rotary_dim);
+  if (n_tokens == 0) return 0;
+  const long total = static_cast<long>(n_tokens) * (rotary_dim / 2);
+  rope_table_kernel<true><<<grid_for(total), kBlock, 0, static_cast<hipStream_t>(stream)>>>(
+      positions, reinterpret_cast<float2*>(table), total, rotary_dim / 2, theta);
+  return check_launch("rope_table_double");
 }
 
 extern "C" int bc4g_rope_kv_write_blocks(void* qkv, int dtype, const float* table, const int32_t* slot_map,

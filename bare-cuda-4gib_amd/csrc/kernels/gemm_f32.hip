@@ -11,6 +11,11 @@
 // Eight rows, weights from memory, plain float FMA (gemm_generic) -> this: 32,000 x 2,048 149 -> 51 us (5.1 TB/s), 11,264 x 2,048 59 -> 20,
 // 2,048 x 5,632 82 -> 16, 2,048 x 2,048 32 -> 7.5; 64 rows 223 -> 159, 188 -> 57, 530 -> 23 and 196 -> 11.  With the attention of
 // attention_f32.hip 32 decode steps of 8 requests after their prompts at TinyLlama's sizes take 213 -> 63 ms.
+// What a decode step does between these products -- two norms a layer, the rotation and the cache write, each a launch of 3 to 5 us
+// with next to nothing to do -- they do themselves: one that adds into the residual stream leaves, for the RMSNorm behind it, new
+// residual * g and every row's sum of squares in parts, a workgroup's outputs each (emit); a product whose x was so prepared applies the
+// rows' factor to its sums (ssq); and the q|k|v product holds a rotation's pairs in one workgroup (kRopeKv): a layer's eight
+// launches are five, 72 -> 63 us of kernels (8 rows, TinyLlama's sizes); eight prompts of 24 to 100 tokens and 31 such steps 64.1 -> 60.5 ms.
 //
 // gemm_f32_tiled_kernel, many rows, bound by the matrix cores (157 TFLOP/s of float32 at the full clock).  A step's 32 k of the
 // tile's rows of x and of w go straight into a ring of stages in LDS; the waves feed 32x32x2 MFMAs from there and keep
@@ -31,8 +36,11 @@ constexpr int kStepBytes = kStepK * 4;
 constexpr int kRedPad = 17;
 constexpr int kXcds = 8;
 
-enum Epilogue : int { kStore = 0, kAccum = 1, kSwiglu = 2, kGeglu = 3 };
+// kRopeKv (few rows only): w holds query, key and value heads; queries are stored rotated, keys go rotated into their pages, values into
+// theirs.
+enum Epilogue : int { kStore = 0, kAccum = 1, kSwiglu = 2, kGeglu = 3, kRopeKv = 4 };
 constexpr bool gated(int epi) { return epi == kSwiglu || epi == kGeglu; }
+constexpr bool paired(int epi) { return gated(epi) || epi == kRopeKv; }      // a workgroup's second eight rows of w belong to its first eight
 
 // The activations as the elementwise kernel has them.
 template <int EPI>
@@ -41,12 +49,29 @@ __device__ inline float gate_act(float g) {
   return g / (1.0f + expf(-g));
 }
 
+struct RopeKv {
+  const float2* table;      // [m, head_dim / 2] (cos, sin) (null: no rotation)
+  const int32_t* slot_map;  // [m] page * page_tokens + offset
+  float* k_cache;           // [pages, n_kv, page_tokens, d]
+  float* v_cache;           // [pages, n_kv, d, page_tokens]
+  int n_heads, n_kv_heads, head_dim, page_tokens, write_kv;
+};
 struct Args {
   const float* x;           // [m, k]
   const float* w;           // [n, k]; gated: n / 2 gate rows, then the up rows
   const float* bias;        // kAccum: [n] (null: none)
-  float* out;               // [m, n], gated: [m, n / 2]
+  float* out;               // [m, n], gated: [m, n / 2], kRopeKv: [m, n_heads * head_dim]
   int m, n, k;
+  // the few rows' kernel: x is residual * g of an RMSNorm whose rows' sums of squares come in parts of 16 columns, [ssq_blocks][m], or
+  // their halves, [ssq_blocks][m][2] (null: x as it is)
+  const float* ssq = nullptr;
+  int ssq_blocks = 0, ssq_halves = 0;
+  float eps = 0.f;
+  // kAccum there: what the RMSNorm behind needs (emit_g null: nothing)
+  const float* emit_g = nullptr;      // [n]
+  float* emit_x = nullptr;            // [m, n]
+  float* emit_ssq = nullptr;          // [ceil(n / 16)][m], with eight outputs a workgroup [ceil(n / 16)][m][2]
+  RopeKv rope = {};
 };
 
 // k is added up in eight shares of whole steps, each from zero, and the shares' sums in order: by both kernels, so that a row's
@@ -119,14 +144,18 @@ __device__ inline void wait_for_step(int later) {
 template <int XR, int STAGES, int EPI, bool HALF = false>
 __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a) {
   constexpr int MT = (XR + 15) / 16, WP = HALF ? 1 : 2, PER = WP + XR / 8, kRing = PER * 1024;      // (WP: pieces of w a step)
-  static_assert(!HALF || !gated(EPI), "half a block of a gated product would part gates and ups");
+  static_assert(!HALF || !paired(EPI), "half a block of a gated product would part gates and ups, of a rotated one a pair");
   extern __shared__ __align__(1024) unsigned char stream_lds[];
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int col = lane % 16, grp = lane / 16;
   const int k = a.k, row0 = blockIdx.y * XR, m = min(XR, a.m - row0);
-  constexpr int kCols = gated(EPI) || HALF ? 8 : 16;         // outputs of a workgroup
-  const int n_out = gated(EPI) ? a.n / 2 : a.n, n0 = blockIdx.x * kCols;
+  constexpr int kCols = paired(EPI) || HALF ? 8 : 16;        // outputs (pairs of them) of a workgroup
+  const int n_out = paired(EPI) ? a.n / 2 : a.n;
+  // kRopeKv: pairs 8 b .. of a head, b = blockIdx.x % (d / 16): dimensions 8 b .. and d / 2 further; n0 is the first's row of w
+  const int head_dim = EPI == kRopeKv ? a.rope.head_dim : 16, head = EPI == kRopeKv ? blockIdx.x / (head_dim / 16) : 0;
+  const int pair0 = EPI == kRopeKv ? blockIdx.x % (head_dim / 16) * 8 : 0;
+  const int n0 = EPI == kRopeKv ? head * head_dim + pair0 : blockIdx.x * kCols;
 
   // this wave's steps of k
   const int per_wave = steps_a_share(k), first = wave * per_wave;
@@ -136,7 +165,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
 
   // What is added to is asked for now: item j of a thread is output (threadIdx.x + j * kThreads) of the workgroup's.
   constexpr int kItems = (XR * kCols + kThreads - 1) / kThreads;
-  float prev[kItems], bias[kItems];
+  float prev[kItems], bias[kItems], gain[kItems];
   if constexpr (EPI == kAccum) {
 #pragma unroll
     for (int j = 0; j < kItems; ++j) {
@@ -144,6 +173,31 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
       const bool live = row < m && gn < n_out;
       prev[j] = live ? a.out[static_cast<long>(row0 + row) * n_out + gn] : 0.f;
       bias[j] = live && a.bias != nullptr ? a.bias[gn] : 0.f;
+      gain[j] = live && a.emit_g != nullptr ? a.emit_g[gn] : 0.f;
+    }
+  }
+  // So are a prepared x's parts of the rows' sums of squares -- sixteen chains a row, chain c adding blocks c, c + 16, ... in that order, the
+  // first kAhead of them (4,096 columns) asked for together --, and a rotation's angles and the places in the cache.
+  constexpr int kChains = 16, kAhead = 16;
+  const int part_row = min(static_cast<int>(threadIdx.x) % XR, m - 1), chain = threadIdx.x / XR;
+  const bool sums_parts = a.ssq != nullptr && chain < kChains;
+  auto part_of = [&](int block) {
+    const long at = static_cast<long>(min(block, a.ssq_blocks - 1)) * a.m + row0 + part_row;
+    return a.ssq_halves ? reinterpret_cast<const float2*>(a.ssq)[at] : make_float2(a.ssq[at], 0.f);
+  };
+  float2 part[kAhead];
+  if (sums_parts) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) part[i] = part_of(chain + i * kChains);
+  }
+  float2 angle[kItems];
+  int slot[kItems];
+  if constexpr (EPI == kRopeKv) {
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const int idx = threadIdx.x + j * kThreads, row = min(idx / kCols, m - 1);
+      angle[j] = a.rope.table != nullptr ? a.rope.table[static_cast<long>(row0 + row) * (head_dim / 2) + pair0 + idx % kCols] : make_float2(1.f, 0.f);
+      slot[j] = a.rope.write_kv && head >= a.rope.n_heads ? a.rope.slot_map[row0 + row] : 0;
     }
   }
 
@@ -156,9 +210,11 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
     const int r = (i < WP ? i : i - WP) * 8 + lane / 8, seg = (lane % 8) ^ slot_key(r);
     back[i] = seg * 16;
     if (i < WP) {                                            // (a load's eight rows of w lie together, from a scalar base)
-      const int from = gated(EPI) ? n0 : min(n0 + i * 8, n_out - 1);
-      const int at = min(gated(EPI) ? n0 + lane / 8 : n0 + r, n_out - 1);
-      bases[i] = a.w + static_cast<long>(from + (gated(EPI) ? i * (a.n / 2) : 0)) * k + first * kStepK;
+      // (paired: the second eight rows as far from the first as the ups from the gates, or a pair's halves)
+      const int last = EPI == kRopeKv ? a.n - 1 : n_out - 1;
+      const int from = paired(EPI) ? n0 : min(n0 + i * 8, last);
+      const int at = min(paired(EPI) ? n0 + lane / 8 : n0 + r, last);
+      bases[i] = a.w + static_cast<long>(from + (gated(EPI) ? i * (a.n / 2) : EPI == kRopeKv ? i * (head_dim / 2) : 0)) * k + first * kStepK;
       offsets[i] = static_cast<unsigned>(at - from) * k * 4 + seg * 16;
     } else {
       bases[i] = a.x + static_cast<long>(row0) * k + first * kStepK;
@@ -221,6 +277,17 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
         for (int t = 0; t < MT; ++t) acc[t] = mfma_16x16x4(wf[h][e], xf[t][h][e], acc[t]);
   }
 
+  __shared__ float part_sum[kChains][XR];
+  if (sums_parts) {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) ss += chain + i * kChains < a.ssq_blocks ? part[i].x + part[i].y : 0.f;
+    for (int block = chain + kAhead * kChains; block < a.ssq_blocks; block += kChains) {
+      const float2 later = part_of(block);
+      ss += later.x + later.y;
+    }
+    part_sum[chain][threadIdx.x % XR] = ss;
+  }
   __syncthreads();                                           // the rings' place takes the waves' sums
   typedef float Red[MT][16][kRedPad];
   Red* red = reinterpret_cast<Red*>(stream_lds);
@@ -234,18 +301,67 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
     const int idx = threadIdx.x + j * kThreads, nl = idx % kCols, row = idx / kCols, gn = n0 + nl;
-    if (row >= m || gn >= n_out) continue;
+    const bool live = row < m && (EPI == kRopeKv || gn < n_out);
+    if (EPI != kAccum && !live) continue;                    // (an adding product's lanes exchange sums of squares)
     float sum = 0.f, up = 0.f;
+    if (live) {
 #pragma unroll
-    for (int v = 0; v < kShares; ++v) sum += red[v][row / 16][nl][row % 16];
-    if constexpr (gated(EPI)) {
+      for (int v = 0; v < kShares; ++v) sum += red[v][row / 16][nl][row % 16];
+      if constexpr (paired(EPI)) {
 #pragma unroll
-      for (int v = 0; v < kShares; ++v) up += red[v][row / 16][nl + 8][row % 16];
+        for (int v = 0; v < kShares; ++v) up += red[v][row / 16][nl + 8][row % 16];
+      }
+      if (a.ssq != nullptr) {
+        float ss = 0.f;
+#pragma unroll
+        for (int v = 0; v < kChains; ++v) ss += part_sum[v][row];
+        const float scale = 1.0f / sqrtf(ss / static_cast<float>(k) + a.eps);
+        sum *= scale;
+        up *= scale;
+      }
     }
-    float* to = a.out + static_cast<long>(row0 + row) * n_out + gn;
-    if constexpr (EPI == kAccum) *to = prev[j] + bias[j] + sum;
-    else if constexpr (gated(EPI)) *to = gate_act<EPI>(sum) * up;
-    else *to = sum;
+    if constexpr (EPI == kRopeKv) {
+      const RopeKv& r = a.rope;
+      const bool is_v = head >= r.n_heads + r.n_kv_heads;
+      const int i0 = pair0 + nl, i1 = i0 + head_dim / 2;
+      const float lo = is_v ? sum : sum * angle[j].x - up * angle[j].y, hi = is_v ? up : up * angle[j].x + sum * angle[j].y;
+      if (head < r.n_heads) {
+        float* to = a.out + (static_cast<long>(row0 + row) * r.n_heads + head) * head_dim;
+        to[i0] = lo, to[i1] = hi;
+      } else if (r.write_kv) {
+        const int kvh = is_v ? head - r.n_heads - r.n_kv_heads : head - r.n_heads, off = slot[j] % r.page_tokens;
+        float* to = (is_v ? r.v_cache : r.k_cache) +
+                    (static_cast<long>(slot[j] / r.page_tokens) * r.n_kv_heads + kvh) * head_dim * r.page_tokens;
+        if (is_v) to += off, to[static_cast<long>(i0) * r.page_tokens] = lo, to[static_cast<long>(i1) * r.page_tokens] = hi;
+        else to += static_cast<long>(off) * head_dim, to[i0] = lo, to[i1] = hi;
+      }
+      continue;
+    }
+    const long at = static_cast<long>(row0 + row) * n_out + gn;
+    if constexpr (EPI == kAccum) {
+      const float nv = prev[j] + bias[j] + sum;
+      if (live) a.out[at] = nv;
+      if (a.emit_g != nullptr) {
+        // the row's outputs of this workgroup lie in kCols neighbouring lanes
+        float sq = live ? nv * nv : 0.f;
+#pragma unroll
+        for (int off = 1; off < kCols; off <<= 1) sq += __shfl_xor(sq, off, kWave);
+        if (live) a.emit_x[at] = nv * gain[j];
+        if (nl == 0 && row < m) {
+          if constexpr (HALF) {
+            float* to = a.emit_ssq + (static_cast<long>(blockIdx.x / 2) * a.m + row0 + row) * 2;
+            to[blockIdx.x % 2] = sq;
+            if (blockIdx.x % 2 == 0 && blockIdx.x + 1 == gridDim.x) to[1] = 0.f;      // (a last block that has no second half)
+          } else {
+            a.emit_ssq[static_cast<long>(blockIdx.x) * a.m + row0 + row] = sq;
+          }
+        }
+      }
+    } else if constexpr (gated(EPI)) {
+      a.out[at] = gate_act<EPI>(sum) * up;
+    } else {
+      a.out[at] = sum;
+    }
   }
 }
 
@@ -260,19 +376,22 @@ int launch_stream_form(const Args& a, hipStream_t s) {
       return fail("gemm_f32: cannot raise the dynamic LDS limit");
     raised = true;
   }
-  const int cols = gated(EPI) || HALF ? 8 : 16, n_out = gated(EPI) ? a.n / 2 : a.n;
+  const int cols = paired(EPI) || HALF ? 8 : 16, n_out = paired(EPI) ? a.n / 2 : a.n;
   kernel<<<dim3((n_out + cols - 1) / cols, (a.m + XR - 1) / XR), kThreads, kLds, s>>>(a);
   return 0;
 }
 
+// Outputs a workgroup of few rows' kernel takes of a product that stores or adds.
+int stream_cols(int m, int n) { return m <= 8 && 2 * ((n + 15) / 16) <= compute_units() ? 8 : 16; }
+
 template <int EPI>
 int launch_stream(const Args& a, hipStream_t s) {
-  const int cols = gated(EPI) ? 8 : 16, n_out = gated(EPI) ? a.n / 2 : a.n;
+  const int cols = paired(EPI) ? 8 : 16, n_out = paired(EPI) ? a.n / 2 : a.n;
   // Outputs that would leave every other CU idle: eight a workgroup, half the weights for each CU to bring and the
   // same sums.  A decode step's two such products, 2,048 x 2,048 and
   // 2,048 x 5,632, from memory, 8 rows, inside a step: 13.05 -> 11.7 us on average; 32 steps of 8 requests after their prompts 67.6 -> 63.5 ms.
-  if constexpr (!gated(EPI)) {
-    if (a.m <= 8 && 2 * ((n_out + 15) / 16) <= compute_units()) return launch_stream_form<8, 8, EPI, true>(a, s);
+  if constexpr (!paired(EPI)) {
+    if (stream_cols(a.m, n_out) == 8) return launch_stream_form<8, 8, EPI, true>(a, s);
   }
   // One workgroup a CU where there are no more: a ring as deep as LDS allows.  Else two that overlap.
   const bool few = (n_out + cols - 1) / cols <= compute_units();
@@ -491,6 +610,62 @@ extern "C" int bc4g_gemm_f32(const float* x, const float* w, const float* bias, 
   }
   if (e) return e;
   return check_launch("gemm_f32");
+}
+
+namespace {
+int few_rows(const char* what, const float* x, const float* w, int m, int n, int k) {
+  BC4G_REQUIRE(m > 0 && m <= 64 && n > 0 && k > 0 && k % 4 == 0 && k <= (1 << 24), "%s: bad sizes M=%d N=%d K=%d (1 to 64 rows, K a multiple of 4)", what,
+               m, n, k);
+  BC4G_REQUIRE(x && w && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0,
+               "%s: operands must lie on 16-byte boundaries", what);
+  return 0;
+}
+}  // namespace
+
+extern "C" int bc4g_gemm_f32_emit(const float* x, const float* w, const float* bias, float* residual, const float* g, float* emit_x, float* emit_ssq,
+                                  int halves, int m, int n, int k, void* stream) {
+  if (int e = few_rows("gemm_f32_emit", x, w, m, n, k)) return e;
+  BC4G_REQUIRE((halves != 0) == (stream_cols(m, n) == 8), "gemm_f32_emit: the parts' shape does not fit M=%d N=%d", m, n);
+  BC4G_REQUIRE(residual && g && emit_x && emit_ssq, "gemm_f32_emit: an operand is missing");
+  Args a{x, w, bias, residual, m, n, k};
+  a.emit_g = g, a.emit_x = emit_x, a.emit_ssq = emit_ssq;
+  if (int e = launch_stream<kAccum>(a, static_cast<hipStream_t>(stream))) return e;
+  return check_launch("gemm_f32_emit");
+}
+
+extern "C" int bc4g_gemm_f32_prenormed(const float* x, const float* ssq, int ssq_blocks, int ssq_halves, float eps, const float* w, float* out, int epilogue, int m, int n,
+                                       int k, void* stream) {
+  if (int e = few_rows("gemm_f32_prenormed", x, w, m, n, k)) return e;
+  BC4G_REQUIRE(ssq && ssq_blocks > 0 && eps >= 0.f && out, "gemm_f32_prenormed: the rows' sums of squares come in %d parts", ssq_blocks);
+  BC4G_REQUIRE(!gated(epilogue) || n % 2 == 0, "gemm_f32_prenormed: a gated product has as many gate rows as up rows (N=%d)", n);
+  Args a{x, w, nullptr, out, m, n, k};
+  a.ssq = ssq, a.ssq_blocks = ssq_blocks, a.ssq_halves = ssq_halves, a.eps = eps;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  int e = 0;
+  switch (epilogue) {
+    case kStore: e = launch_stream<kStore>(a, s); break;
+    case kSwiglu: e = launch_stream<kSwiglu>(a, s); break;
+    case kGeglu: e = launch_stream<kGeglu>(a, s); break;
+    default: return fail("gemm_f32_prenormed: unknown epilogue %d", epilogue);
+  }
+  if (e) return e;
+  return check_launch("gemm_f32_prenormed");
+}
+
+extern "C" int bc4g_gemm_f32_qkv(const float* x, const float* ssq, int ssq_blocks, int ssq_halves, float eps, const float* w, float* q, const float* table,
+                                 const int32_t* slot_map, float* k_cache, float* v_cache, int m, int k, int n_heads, int n_kv_heads, int head_dim,
+                                 int page_tokens, int write_kv, void* stream) {
+  BC4G_REQUIRE(n_heads > 0 && n_kv_heads > 0 && head_dim > 0 && head_dim % 16 == 0 && (n_heads + 2L * n_kv_heads) * head_dim <= 2147483647L,
+               "gemm_f32_qkv: %d + 2 x %d heads of %d (a multiple of 16)", n_heads, n_kv_heads, head_dim);
+  const int n = (n_heads + 2 * n_kv_heads) * head_dim;
+  if (int e = few_rows("gemm_f32_qkv", x, w, m, n, k)) return e;
+  BC4G_REQUIRE(q && (ssq == nullptr || (ssq_blocks > 0 && eps >= 0.f)), "gemm_f32_qkv: an operand is missing");
+  BC4G_REQUIRE(!write_kv || (page_tokens > 0 && k_cache && v_cache && slot_map), "gemm_f32_qkv: cache write asked for without a cache");
+  Args a{x, w, nullptr, q, m, n, k};
+  a.ssq = ssq, a.ssq_blocks = ssq_blocks, a.ssq_halves = ssq_halves, a.eps = eps;
+  a.rope = RopeKv{reinterpret_cast<const float2*>(table), slot_map, k_cache, v_cache, n_heads, n_kv_heads, head_dim, page_tokens, write_kv ? 1 : 0};
+  if (int e = launch_stream<kRopeKv>(a, static_cast<hipStream_t>(stream))) return e;
+  return check_launch("gemm_f32_qkv");
 }
 
 extern "C" int bc4g_gemm_f32_tile(int m, int n, int k, int* rows, int* cols) {

@@ -28,9 +28,13 @@ _SIGNATURES = {
     "bc4g_gemm_mfma_swiglu_scaled": [_P, _P, _I, _I, _F, _P, _I, _P, _I, _I, _I, _I, _P],
     "bc4g_gemm_generic": [_P, _I, _P, _I, _P, _I, _I, _P, _I, _I, _I, _P],
     "bc4g_gemm_f32": [_P, _P, _P, _P, _I, _I, _I, _I, _P],
+    "bc4g_gemm_f32_emit": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
+    "bc4g_gemm_f32_prenormed": [_P, _P, _I, _I, _F, _P, _P, _I, _I, _I, _I, _P],
+    "bc4g_gemm_f32_qkv": [_P, _P, _I, _I, _F, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "bc4g_gemm_f32_tile": [_I, _I, _I, _P, _P],
     "bc4g_swiglu": [_P, _P, _I, _I, _I, _I, _I, _P],
     "bc4g_rope_table": [_P, _P, _I, _I, _F, _P],
+    "bc4g_rope_table_double": [_P, _P, _I, _I, _F, _P],
     "bc4g_rope_kv_write_blocks": [_P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "bc4g_rope_kv_write": [_P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _I, _I, _P],
     "bc4g_attention_generic": [_P, _I, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P],

@@ -274,6 +274,93 @@ def gemm_f32(x: torch.Tensor, w, accumulate_into: Optional[torch.Tensor] = None,
     return out
 
 
+GEMM_F32_FEW_ROWS = 64               # rows up to which a float32 product prepares or finishes an RMSNorm
+
+
+def gemm_f32_finishes_norm(n_rows: int, w) -> bool:
+    """Whether the float32 product of this weight takes a prepared norm (Prenormed) at so many rows: always, up to 64 rows of whole
+    16-byte pieces.  (Reading the parts costs the product nothing that shows: they come while its weights do.)"""
+    return w.dtype == torch.float32 and w.is_cuda and 0 < n_rows <= GEMM_F32_FEW_ROWS and w.shape[1] % 4 == 0 and w.shape[1] <= 1 << 24
+
+
+def gemm_f32_emit(x: torch.Tensor, w, residual: torch.Tensor, g: torch.Tensor, eps: float, bias: Optional[torch.Tensor] = None) -> Optional["Prenormed"]:
+    """residual += x w^T (+ ``bias``) in float32, and the next RMSNorm (scale g, eps) prepared, ``xb`` in float32 too; None where
+    the kernel does not take the operands."""
+    if (x.dtype != torch.float32 or w.dtype != torch.float32 or g.dtype != torch.float32 or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]
+            or x.shape[1] % 4 or x.shape[1] > 1 << 24 or not 0 < x.shape[0] <= GEMM_F32_FEW_ROWS or tuple(g.shape) != (w.shape[0],)
+            or not g.is_contiguous()):
+        return None
+    w = _rows(w)
+    if x.data_ptr() % 16 or w.data_ptr() % 16:
+        return None
+    m, k = x.shape
+    n = w.shape[0]
+    _dev("gemm_f32_emit", x, w, residual, g, bias)
+    _check_bias("gemm_f32_emit", bias, n, residual)
+    if residual.dtype != torch.float32 or tuple(residual.shape) != (m, n):
+        raise KernelError(f"gemm_f32_emit: the residual must be float32 [{m}, {n}], got {residual.dtype} {tuple(residual.shape)}")
+    blocks = -(-n // 16)
+    halves = m <= 8 and 2 * blocks <= compute_units()
+    xb = torch.empty((m, n), dtype=torch.float32, device=x.device)
+    parts = torch.empty((blocks, m, 2) if halves else (blocks, m), dtype=torch.float32, device=x.device)
+    library.call("bc4g_gemm_f32_emit", _ptr(x), _ptr(w), _ptr(bias), _ptr(residual), _ptr(g), _ptr(xb), _ptr(parts), 1 if halves else 0, m, n, k,
+                 _stream(), cost=_gemm_cost(m, n, k, 4, 4, 12))
+    return Prenormed(xb, parts, eps)
+
+
+def _prepared_f32(x: torch.Tensor, pre: Optional["Prenormed"]):
+    return (_ptr(x), _ptr(pre.parts), pre.parts.shape[0], pre.parts.dim() - 2, pre.eps) if pre is not None else (_ptr(x), None, 0, 0, 0.0)
+
+
+def gemm_f32_prenormed(pre: "Prenormed", w, act: Optional[str] = None) -> Optional[torch.Tensor]:
+    """rmsnorm(residual) w^T in float32 from what gemm_f32_emit left (``act``: as in gemm_f32); None where the kernel does not take
+    the operands."""
+    x = pre.xb
+    if (x.dtype != torch.float32 or w.dim() != 2 or w.shape[1] != x.shape[1] or not gemm_f32_finishes_norm(x.shape[0], w)
+            or (act is not None and w.shape[0] % 2)):
+        return None
+    w = _rows(w)
+    if w.data_ptr() % 16:
+        return None
+    _dev("gemm_f32_prenormed", x, pre.parts, w)
+    m, k = x.shape
+    n = w.shape[0]
+    out = torch.empty((m, n // 2 if act is not None else n), dtype=torch.float32, device=x.device)
+    library.call("bc4g_gemm_f32_prenormed", *_prepared_f32(x, pre), _ptr(w), _ptr(out), F32_GATED[act] if act is not None else F32_STORE, m, n, k,
+                 _stream(), cost=_gemm_cost(m, n, k, 4, 4, 4.0 * out.shape[1] / n))
+    return out
+
+
+def gemm_f32_qkv_supported(x: torch.Tensor, w, head_dim: int, rotary_dim: int) -> bool:
+    """Whether gemm_f32_qkv takes these operands: few float32 rows, heads rotated whole or not at all."""
+    return (x.dtype == torch.float32 and x.dim() == 2 and x.data_ptr() % 16 == 0 and gemm_f32_finishes_norm(x.shape[0], w)
+            and x.shape[1] == w.shape[1] and w.data_ptr() % 16 == 0 and head_dim % 16 == 0 and rotary_dim in (0, head_dim))
+
+
+def gemm_f32_qkv(x: torch.Tensor, w, table: Optional[torch.Tensor], slot_map: Optional[torch.Tensor], k_cache: Optional[torch.Tensor],
+                 v_cache: Optional[torch.Tensor], n_heads: int, n_kv_heads: int, head_dim: int, write_kv: bool = True,
+                 pre: Optional["Prenormed"] = None) -> torch.Tensor:
+    """The q|k|v product of up to 64 float32 rows with rotary positions (``table``: rope_table(double=True) of the rows' positions; None: no
+    rotation) and the cache write: the rotated queries [m, n_heads * head_dim].  ``pre``: x is its ``xb``, a prepared norm."""
+    w = _rows(w)
+    m, k = x.shape
+    n = (n_heads + 2 * n_kv_heads) * head_dim
+    _dev("gemm_f32_qkv", x, w, table, slot_map, k_cache, v_cache, pre.parts if pre is not None else None)
+    if tuple(w.shape) != (n, k):
+        raise KernelError(f"gemm_f32_qkv: weight must be [{n}, {k}], got {tuple(w.shape)}")
+    if table is not None and (table.dtype != torch.float32 or tuple(table.shape) != (m, head_dim // 2, 2)):
+        raise KernelError(f"gemm_f32_qkv: the table must be float32 [{m}, {head_dim // 2}, 2], got {table.dtype} {tuple(table.shape)}")
+    page_tokens = 0
+    if write_kv:
+        _check_cache("gemm_f32_qkv", k_cache, v_cache, n_kv_heads, head_dim, torch.float32)
+        _i32("gemm_f32_qkv", "slot_map", slot_map, m)
+        page_tokens = k_cache.shape[2]
+    q = torch.empty((m, n_heads * head_dim), dtype=torch.float32, device=x.device)
+    library.call("bc4g_gemm_f32_qkv", *_prepared_f32(x, pre), _ptr(w), _ptr(q), _ptr(table), _ptr(slot_map), _ptr(k_cache), _ptr(v_cache), m, k,
+                 n_heads, n_kv_heads, head_dim, page_tokens, 1 if write_kv else 0, _stream(), cost=_gemm_cost(m, n, k, 4, 4, 4))
+    return q
+
+
 def gemm_f32_tile(m: int, n: int, k: int) -> Tuple[int, int]:
     """(rows of x, rows of w) a workgroup of gemm_f32 takes, (0, 0) where it streams the weights."""
     rows, cols = ctypes.c_int(0), ctypes.c_int(0)
@@ -365,14 +452,14 @@ def rope_kv_write(qkv: torch.Tensor, positions: Optional[torch.Tensor], slot_map
                  cost=lambda: (3.0 * t * (n_heads + n_kv_heads) * head_dim, 2 * t * width * qkv.element_size()))
 
 
-def rope_table(positions: torch.Tensor, rotary_dim: int, theta: float) -> torch.Tensor:
+def rope_table(positions: torch.Tensor, rotary_dim: int, theta: float, double: bool = False) -> torch.Tensor:
     """(cos, sin) of every row's angles, float32 [T, rotary_dim / 2, 2]: computed once a step, read
-    by every layer's rope_kv_write_blocks."""
+    by every layer's rope_kv_write_blocks.  ``double``: worked out in double, for gemm_f32_qkv."""
     _dev("rope_table", positions)
     t = positions.shape[0]
     _i32("rope_table", "positions", positions, t)
     table = torch.empty((t, rotary_dim // 2, 2), dtype=torch.float32, device=positions.device)
-    library.call("bc4g_rope_table", _ptr(positions), _ptr(table), t, int(rotary_dim), float(theta), _stream(),
+    library.call("bc4g_rope_table_double" if double else "bc4g_rope_table", _ptr(positions), _ptr(table), t, int(rotary_dim), float(theta), _stream(),
                  cost=lambda: (0.0, t * rotary_dim * 4))
     return table
 

@@ -118,7 +118,10 @@ class CausalAttention(Part):
 
     def wants_prepared_norm(self, n_rows: int) -> bool:
         """Whether the q|k|v product is better served by a norm that the product before prepared than by fusing
-        the norm or running it: the weight's own plan says (ops.LinearPlan.wants_prepared)."""
+        the norm or running it: the weight's own plan says (ops.LinearPlan.wants_prepared), and few float32 rows
+        always are."""
+        if self.act_dtype == torch.float32:
+            return ops.gemm_f32_finishes_norm(n_rows, self.w_qkv)
         return self.act_dtype == torch.bfloat16 and self.w_qkv.plan.wants_prepared(n_rows)
 
     def forward(self, h, ctx, cache, residual, writes: bool = True) -> None:
@@ -131,6 +134,8 @@ class CausalAttention(Part):
             q = self._fused_qkv(h, ctx, slot_map, k_cache, v_cache, rotary_dim, theta, writes)
         if q is None and self.block_pairs and fused is not None:
             q = self._tiled_qkv(h, ctx, slot_map, k_cache, v_cache, rotary_dim, theta, writes)
+        if not self.block_pairs and fused is not None:
+            q = self._float_qkv(h, ctx, slot_map, k_cache, v_cache, rotary_dim, theta, writes)
         if q is None:
             q = linear(h, self.w_qkv, out_dtype=self.act_dtype)
             if fused is None:
@@ -150,6 +155,22 @@ class CausalAttention(Part):
         o = ops.attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx, (arrays, notes) if notes else None,
                           self.num_heads, self.num_kv_heads, self.head_dim, self.window, self.scale)
         linear(o, self.w_o, accumulate_into=residual, ctx=ctx)
+
+    def _float_qkv(self, h, ctx, slot_map, k_cache, v_cache, rotary_dim, theta, writes):
+        """The q|k|v product of few float32 rows with rotation and cache write in its epilogue, the angles from the step's
+        table; None where that kernel does not take the operands."""
+        pre = h.pre if isinstance(h, Normed) and h._tensor is None else None
+        if pre is None and (h.n_rows if isinstance(h, Normed) else h.shape[0]) > ops.GEMM_F32_FEW_ROWS:
+            return None
+        x = pre.xb if pre is not None else h.tensor() if isinstance(h, Normed) else h
+        if not ops.gemm_f32_qkv_supported(x, self.w_qkv, self.head_dim, rotary_dim):
+            return None
+        table = None
+        if rotary_dim > 0:
+            table = ctx.shared(("rope_table", rotary_dim, theta, "double"),
+                               lambda: ops.rope_table(ctx.positions, rotary_dim, theta, double=True))
+        return ops.gemm_f32_qkv(x, self.w_qkv, table, slot_map, k_cache, v_cache, self.num_heads, self.num_kv_heads,
+                                self.head_dim, write_kv=writes, pre=pre)
 
     def _tiled_qkv(self, h, ctx, slot_map, k_cache, v_cache, rotary_dim, theta, writes):
         """The q|k|v product of many rows (a prompt portion) with rotation and cache write in the tiled kernel's

@@ -4,7 +4,8 @@ choice of kernel for it (reference: matmul dispatch, engine/src/model.cpp:153-19
 up to 64 rows the weight-streaming kernel (with RMSNorm fused in up to 16 rows),
 beyond that the tiled matrix-core kernel, and the plain float kernel for
 what those refuse (k no multiple of 8).  Float32 operands go to the
-float32 matrix-core kernel where it takes them, else to the plain one."""
+float32 matrix-core kernel where it takes them (which up to 64 rows prepares and
+finishes norms too), else to the plain one."""
 from __future__ import annotations
 
 from typing import Optional, Union
@@ -32,7 +33,12 @@ def absorbs_norm(norm, w, n_rows: int) -> bool:
 
 def _prepared_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
     """The product from what the product before left for this norm, where there is such a thing."""
-    if x.pre is None or x._tensor is not None or not ops.gemm_prenormed_supported(x.pre, w, epilogue):
+    if x.pre is None or x._tensor is not None:
+        return None
+    if x.pre.xb.dtype == torch.float32:
+        act = {ops.EPI_STORE_F32: None, ops.EPI_SWIGLU: "silu", ops.EPI_GEGLU: "gelu_tanh"}.get(epilogue, "")
+        return ops.gemm_f32_prenormed(x.pre, w, act) if act != "" else None
+    if not ops.gemm_prenormed_supported(x.pre, w, epilogue):
         return None
     return ops.gemm_prenormed(x.pre, w, epilogue)
 
@@ -72,6 +78,10 @@ def linear(x: Union[torch.Tensor, Normed], w, out_dtype: Optional[torch.dtype] =
             return accumulate_into
         if scale is not None and takes_parts and ops.gemm_emit_supported(x, w, accumulate_into, scale[0]):
             ctx.handoff.leave(norm, ops.gemm_accumulate_emit(x, w, accumulate_into, scale[0], scale[1], bias=bias))
+            return accumulate_into
+        left = ops.gemm_f32_emit(x, w, accumulate_into, scale[0], scale[1], bias=bias) if scale is not None and takes_parts else None
+        if left is not None:
+            ctx.handoff.leave(norm, left)
             return accumulate_into
     fast = ops.gemm_fast(x, w, out_dtype, accumulate_into, bias=bias)
     if fast is None and out_dtype in (None, torch.float32):
@@ -128,6 +138,8 @@ def linear_swiglu(x: Union[torch.Tensor, Normed], w_gate_up, interleaved: bool =
             fused = _prepared_norm(x, w_gate_up, ops.gated_epilogue(act))
             if fused is None:
                 fused = _fused_norm(x, w_gate_up, ops.gated_epilogue(act))
+        elif not interleaved and x.pre is not None and x.pre.xb.dtype == torch.float32:
+            fused = _prepared_norm(x, w_gate_up, ops.gated_epilogue(act))
         if fused is not None:
             return fused
         x = x.tensor()
