@@ -25,7 +25,7 @@ class SwiGLU(Part):
         if act not in ("silu", "gelu_tanh"):
             raise ConfigError(f"gated feed-forward: activation {act!r} ('silu' or 'gelu_tanh')")
         self.act = act
-        self.w_gu = self.w_down = None
+        self.w_gu = self.w_down = self.act_dtype = None
 
     def weight_specs(self) -> Dict[str, WeightSpec]:
         h, i = self.hidden_size, self.intermediate_size
