@@ -280,7 +280,7 @@ GEMM_F32_FEW_ROWS = 64               # rows up to which a float32 product prepar
 def gemm_f32_finishes_norm(n_rows: int, w) -> bool:
     """Whether the float32 product of this weight takes a prepared norm (Prenormed) at so many rows: always, up to 64 rows of whole
     16-byte pieces.  (Reading the parts costs the product nothing that shows: they come while its weights do.)"""
-    return w.dtype == torch.float32 and w.is_cuda and 0 < n_rows <= GEMM_F32_FEW_ROWS and w.shape[1] % 4 == 0 and w.shape[1] <= 1 << 24
+    return getattr(w, "dtype", None) == torch.float32 and w.is_cuda and 0 < n_rows <= GEMM_F32_FEW_ROWS and w.shape[1] % 4 == 0 and w.shape[1] <= 1 << 24
 
 
 def gemm_f32_emit(x: torch.Tensor, w, residual: torch.Tensor, g: torch.Tensor, eps: float, bias: Optional[torch.Tensor] = None) -> Optional["Prenormed"]:
