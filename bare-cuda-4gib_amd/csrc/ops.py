@@ -19,6 +19,7 @@ import torch
 from ..errors import KernelError
 from . import library
 
+_profiler = library._profiler
 F32, BF16 = 0, 1
 _GLU_ACT = {"silu": 0, "gelu_tanh": 1}      # the activations of a gated unit's gate
 _CODE = {torch.float32: F32, torch.bfloat16: BF16}
@@ -33,12 +34,11 @@ def _code(t: torch.Tensor, what: str) -> int:
 
 def _dev(what: str, *tensors: Optional[torch.Tensor]) -> None:
     for t in tensors:
-        if t is None:
+        if t is None or (t.is_cuda and t.is_contiguous()):
             continue
         if not t.is_cuda:
             raise KernelError(f"{what}: tensors must be on the GPU (got {t.device}); there is no CPU path")
-        if not t.is_contiguous():
-            raise KernelError(f"{what}: tensors must be contiguous (got strides {t.stride()} for shape {tuple(t.shape)})")
+        raise KernelError(f"{what}: tensors must be contiguous (got strides {t.stride()} for shape {tuple(t.shape)})")
 
 
 def _i32(what: str, name: str, t: torch.Tensor, n: int) -> None:
@@ -56,12 +56,19 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+def _row(t: torch.Tensor, r: int) -> int:
+    """The address of row r of a contiguous [rows, n] tensor (without the slice, which costs a microsecond)."""
+    return t.data_ptr() + r * t.shape[1] * t.element_size() if r else t.data_ptr()
+
+
 def _gemm_cost(m: int, n: int, k: int, in_bytes: int, w_bytes: int, out_bytes: float, x_readers: int = 1,
                w_readers: int = 1):
     """(operations, bytes moved at least, bytes asked for in all) of an [m, k] x [n, k]^T product; out_bytes per
     output element.  x_readers / w_readers: how many workgroups read every element of x / of w (the
     weight-streaming kernel: every block of 16 columns reads all the rows; the tiled kernel: every row of
-    tiles reads all the weights, every column of tiles all the rows)."""
+    tiles reads all the weights, every column of tiles all the rows).  Only the profiler asks: None while it is off."""
+    if not _profiler.enabled:
+        return None
     ideal = m * k * in_bytes + n * k * w_bytes + m * n * out_bytes
     moved = x_readers * m * k * in_bytes + w_readers * n * k * w_bytes + m * n * out_bytes
     return lambda: (2.0 * m * n * k, ideal, moved)
@@ -81,6 +88,9 @@ def tiled_tile(m: int, n: int, k: int, a_ptr: int = 0, w_ptr: int = 0, qkv: bool
 
 
 def _tiled_cost(m: int, n: int, k: int, out_bytes: float, qkv: bool = False):
+    if not _profiler.enabled:
+        return None
+
     def cost():                                    # asked for by the profiler only: the tile is looked up then
         rows, cols = tiled_tile(m, n, k, qkv=qkv)
         return _gemm_cost(m, n, k, 2, 2, out_bytes, x_readers=-(-n // cols), w_readers=-(-m // rows))()
@@ -419,9 +429,9 @@ def cache_to_plain(k: torch.Tensor, v: torch.Tensor):
 def _check_cache(what: str, k: torch.Tensor, v: torch.Tensor, n_kv_heads: int, head_dim: int, dtype: torch.dtype):
     """k: [pages, kv_heads, page_tokens, head_dim]; v transposed: [pages, kv_heads, head_dim, page_tokens]
     (the order inside a page and head: see cache_fragment_order)."""
-    ok = (k.dim() == 4 and v.dim() == 4 and k.shape[1] == n_kv_heads and k.shape[3] == head_dim
-          and k.dtype == dtype and v.dtype == dtype
-          and tuple(v.shape) == (k.shape[0], n_kv_heads, head_dim, k.shape[2]))
+    ks = k.shape
+    ok = (len(ks) == 4 and ks[1] == n_kv_heads and ks[3] == head_dim and k.dtype == dtype and v.dtype == dtype
+          and v.shape == (ks[0], n_kv_heads, head_dim, ks[2]))
     if not ok:
         raise KernelError(f"{what}: caches must be {dtype}, keys [pages, {n_kv_heads}, page_tokens, {head_dim}] and "
                           f"values [pages, {n_kv_heads}, {head_dim}, page_tokens]; got {k.dtype} {tuple(k.shape)} "
@@ -491,8 +501,8 @@ def rope_kv_write_blocks(qkv: torch.Tensor, table: Optional[torch.Tensor], slot_
 
 def _check_queries(what: str, q: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int) -> None:
     """Queries come as the rows of the fused q|k|v product or as a buffer of queries alone."""
-    widths = ((n_heads + 2 * n_kv_heads) * head_dim, n_heads * head_dim)
-    if q.dim() != 2 or q.shape[1] not in widths:
+    widths, shape = ((n_heads + 2 * n_kv_heads) * head_dim, n_heads * head_dim), q.shape
+    if len(shape) != 2 or shape[1] not in widths:
         raise KernelError(f"{what}: queries must be [T, {widths[0]}] or [T, {widths[1]}], got {tuple(q.shape)}")
 
 
@@ -664,6 +674,7 @@ class StreamedWeight:
 
     def __init__(self, rows: torch.Tensor, keep_rows: Optional[bool] = None):
         self.shape, self.dtype, self.device = rows.shape, rows.dtype, rows.device
+        self.is_cuda = rows.is_cuda          # (asked at every launch)
         ok = rows.is_cuda and rows.dtype == torch.bfloat16 and rows.dim() == 2 and rows.shape[1] % 8 == 0
         self.packed = pack_weight(rows) if ok else None
         if keep_rows is None:
@@ -683,10 +694,6 @@ class StreamedWeight:
         return self._rows is not None
 
     # what the wrappers ask of an operand before they launch (answered without making the rows)
-    @property
-    def is_cuda(self) -> bool:
-        return self.device.type == "cuda"
-
     def dim(self) -> int:
         return len(self.shape)
 
@@ -877,8 +884,9 @@ def gated_epilogue(act: str) -> int:
 
 
 def _fast_operands(a: torch.Tensor, w: torch.Tensor) -> bool:
-    return (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and w.dim() == 2
-            and a.shape[1] == w.shape[1] and a.shape[1] % 8 == 0 and a.shape[0] > 0)
+    x, y = a.shape, w.shape
+    return (a.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and len(x) == 2 and len(y) == 2
+            and x[1] == y[1] and x[1] % 8 == 0 and x[0] > 0)
 
 
 def gemm_fast(a: torch.Tensor, w, out_dtype=None,
@@ -911,7 +919,7 @@ def gemm_fast(a: torch.Tensor, w, out_dtype=None,
         packed = packed if packed is not None else pack_weight(_rows(w))      # (packing per call: tests only)
         for r0 in range(0, m, SKINNY_MAX_ROWS):                        # the weights once for every 64 rows
             rows = min(SKINNY_MAX_ROWS, m - r0)
-            library.call("bc4g_gemm_skinny", _ptr(a[r0:]), _ptr(packed), _ptr(out[r0:]), _ptr(bias), epi, rows, n, k,
+            library.call("bc4g_gemm_skinny", _row(a, r0), _ptr(packed), _row(out, r0), _ptr(bias), epi, rows, n, k,
                          1 if epi <= EPI_ACCUM_F32 and half_blocks(m, n, k) else 0, _stream(),
                          cost=_skinny_cost(rows, n, k, 2, out_bytes))
     else:
@@ -1000,7 +1008,7 @@ def gemm_swiglu(a: torch.Tensor, w_gate_up, interleaved: bool = False, act: str 
             packed = packed if packed is not None else pack_weight(_rows(rows))
             for r0 in range(0, m, SKINNY_MAX_ROWS):
                 part = min(SKINNY_MAX_ROWS, m - r0)
-                library.call("bc4g_gemm_skinny", _ptr(a[r0:]), _ptr(packed), _ptr(out[r0:]), None, gated_epilogue(act), part, n, k, 0,
+                library.call("bc4g_gemm_skinny", _row(a, r0), _ptr(packed), _row(out, r0), None, gated_epilogue(act), part, n, k, 0,
                              _stream(), cost=_skinny_cost(part, n, k, 2, 1))
         else:
             library.call("bc4g_gemm_mfma", _ptr(a), *_tiled_weight(rows, packed, a), _ptr(out), None, gated_epilogue(act), m, n, k, _stream(),
@@ -1051,11 +1059,14 @@ def parts_of_k(m: int, n: int, k: int) -> int:
 def gemm_parts_supported(a: torch.Tensor, w, residual: torch.Tensor, g: torch.Tensor) -> bool:
     """Whether gemm_parts_accumulate_norm takes these operands: bfloat16, 10 to 256 rows, a k that several
     workgroups can share, a plain RMSNorm after it."""
+    # (asked by every adding product of a step: the rows first, which settle most)
     w, _ = _weight(w)
-    return (_fast_operands(a, w) and residual.dtype == torch.float32 and residual.is_contiguous()
-            and tuple(residual.shape) == (a.shape[0], w.shape[0]) and g.dtype in _CODE and tuple(g.shape) == (w.shape[0],)
+    x, y = a.shape, w.shape
+    return (len(x) == 2 and len(y) == 2 and parts_of_k(x[0], y[0], y[1]) > 1
+            and _fast_operands(a, w) and residual.dtype == torch.float32 and residual.is_contiguous()
+            and residual.shape == (x[0], y[0]) and g.dtype in _CODE and g.shape == (y[0],)
             and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and residual.data_ptr() % 16 == 0 and a.is_contiguous()
-            and w.is_contiguous() and parts_of_k(a.shape[0], w.shape[0], w.shape[1]) > 1)
+            and w.is_contiguous())
 
 
 def gemm_parts_accumulate_norm(a: torch.Tensor, w, residual: torch.Tensor, g: torch.Tensor, eps: float,
@@ -1086,8 +1097,9 @@ def gemm_emit_supported(a: torch.Tensor, w, residual: torch.Tensor, g: torch.Ten
     """Whether the adding product of these operands can prepare the next RMSNorm: the
     weight-streaming kernel serves it (bfloat16, few rows: streams_weights)."""
     w, _ = _weight(w)
-    return (_fast_operands(a, w) and 0 < a.shape[0] and streams_weights(a.shape[0], w.shape[0], w.shape[1]) and residual.dtype == torch.float32
-            and g.dtype in _CODE and tuple(g.shape) == (w.shape[0],))
+    y = w.shape
+    return (len(y) == 2 and streams_weights(a.shape[0], y[0], y[1]) and _fast_operands(a, w) and residual.dtype == torch.float32
+            and g.dtype in _CODE and g.shape == (y[0],))
 
 
 def gemm_accumulate_emit(a: torch.Tensor, w, residual: torch.Tensor, g: torch.Tensor, eps: float,
@@ -1108,8 +1120,8 @@ def gemm_accumulate_emit(a: torch.Tensor, w, residual: torch.Tensor, g: torch.Te
     parts = torch.empty((-(-n // 16), m, 2) if halves else (-(-n // 16), m), dtype=torch.float32, device=a.device)
     for r0 in range(0, m, SKINNY_MAX_ROWS):
         rows = min(SKINNY_MAX_ROWS, m - r0)
-        library.call("bc4g_gemm_skinny_emit", _ptr(a[r0:]), _ptr(packed), _ptr(residual[r0:]), _ptr(bias), _ptr(g),
-                     _code(g, "gemm_accumulate_emit"), _ptr(xb[r0:]), _ptr(parts[:, r0:]), m, rows, n, k, 1 if halves else 0, _stream(),
+        library.call("bc4g_gemm_skinny_emit", _row(a, r0), _ptr(packed), _row(residual, r0), _ptr(bias), _ptr(g),
+                     _code(g, "gemm_accumulate_emit"), _row(xb, r0), parts.data_ptr() + r0 * (8 if halves else 4), m, rows, n, k, 1 if halves else 0, _stream(),
                      cost=_skinny_cost(rows, n, k, 2, 10))
     return Prenormed(xb, parts, eps)
 
@@ -1154,8 +1166,8 @@ def gemm_prenormed(pre: Prenormed, w, epilogue: int) -> torch.Tensor:
         return out
     for r0 in range(0, m, SKINNY_MAX_ROWS):
         rows = min(SKINNY_MAX_ROWS, m - r0)
-        library.call("bc4g_gemm_skinny_prenormed", _ptr(pre.xb[r0:]), _ptr(pre.parts[:, r0:]), pre.parts.shape[0], m,
-                     pre.parts.dim() - 2, pre.eps, _ptr(packed), _ptr(out[r0:]), epilogue, rows, n, k, _stream(),
+        library.call("bc4g_gemm_skinny_prenormed", _row(pre.xb, r0), pre.parts.data_ptr() + r0 * pre.parts.stride(1) * 4, pre.parts.shape[0], m,
+                     pre.parts.dim() - 2, pre.eps, _ptr(packed), _row(out, r0), epilogue, rows, n, k, _stream(),
                      cost=_skinny_cost(rows, n, k, 2, out.element_size() * out.shape[1] / n))
     return out
 
@@ -1349,17 +1361,26 @@ def attention_mfma(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         _dev("attention_mfma", items, row_parts)
         _i32("attention_mfma", "items", items, n_items)
         _i32("attention_mfma", "row_parts", row_parts, t)
-    part_o = part_ml = None
-    if n_splits > 1:
-        part_o = torch.empty((n_splits, t, n_heads, head_dim), dtype=torch.float32, device=qkv.device)
-        part_ml = torch.empty((n_splits, t, n_heads, 2), dtype=torch.float32, device=qkv.device)
-    library.call("bc4g_attention_mfma", _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(part_o), _ptr(part_ml), _ptr(k_cache),
+    _launch_attention_mfma(qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start, n_tiles, n_heads, n_kv_heads, head_dim, window,
+                           scale, n_splits, q_tiles, form, work, out, row_seq, single_rows, items, n_items, row_parts)
+    return out
+
+
+def _launch_attention_mfma(qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start, n_tiles, n_heads, n_kv_heads, head_dim, window, scale,
+                           n_splits, q_tiles, form, work, out, row_seq=None, single_rows=False, items=None, n_items=0, row_parts=None) -> None:
+    """attention_mfma for operands that have been looked at."""
+    t, n_seqs = qkv.shape[0], block_table.shape[0]
+    parts = part_ml = None
+    if n_splits > 1:                    # [n_splits, t, n_heads, head_dim] partial outputs, then [n_splits, t, n_heads, 2] statistics
+        walks = n_splits * t * n_heads
+        parts = torch.empty(walks * (head_dim + 2), dtype=torch.float32, device=qkv.device)
+        part_ml = parts.data_ptr() + 4 * walks * head_dim
+    library.call("bc4g_attention_mfma", _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(parts), part_ml, _ptr(k_cache),
                  _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(seq_start), _ptr(seq_ctx),
                  _ptr(tile_start), n_seqs, n_tiles, t, n_heads, n_kv_heads, head_dim, k_cache.shape[2],
                  int(window), float(scale), attention_tile_tokens(n_heads, n_kv_heads), int(q_tiles),
                  int(form), int(n_splits), _ptr(items), int(n_items), _ptr(row_parts), 1 if single_rows else 0,
                  _ptr(row_seq), _stream(), cost=work)
-    return out
 
 
 _DECODE_TILE_STARTS: dict = {}
@@ -1437,7 +1458,9 @@ def attention_plan(batch, n_heads: int, n_kv_heads: int, head_dim: int, window: 
             notes.update(n_items=len(items), most_parts=most)
     if apart:
         arrays["short_tiles"] = short_starts
-        notes.update(n_short=short_starts[-1], longest_short=max(batch.seq_ctx[s] for s in short) + tpt)
+        longest = max(batch.seq_ctx[s] for s in short) + tpt
+        notes.update(n_short=short_starts[-1],
+                     short_splits=attention_splits(short_starts[-1], n_heads, n_kv_heads, longest, attention_shared_waves(head_dim)))
     return arrays, notes
 
 
@@ -1471,10 +1494,10 @@ def attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
             out = attention_mfma(*args, arrays["tiles"], notes["n_tiles"], *sizes, n_splits, q_tiles, 2, work=work,
                                  row_seq=ctx.row_seq if apart else None)
         if apart:
-            n_splits = attention_splits(notes["n_short"], n_heads, n_kv_heads, notes["longest_short"],
-                                        attention_shared_waves(head_dim))
-            attention_mfma(*args, arrays["short_tiles"], notes["n_short"], *sizes, n_splits, 1, 1, out=out,
-                           row_seq=ctx.row_seq)
+            # (the tensors of the launch before, the piece starts aside)
+            _dev("attention", arrays["short_tiles"])
+            _i32("attention", "short_tiles", arrays["short_tiles"], ctx.n_seqs + 1)
+            _launch_attention_mfma(*args, arrays["short_tiles"], notes["n_short"], *sizes, notes["short_splits"], 1, 1, None, out, ctx.row_seq)
         return out
     if ctx.n_seqs <= 65535 and attention_f32_takes(qkv, k_cache, v_cache, head_dim):
         return attention_f32(qkv, k_cache, v_cache, block_table, ctx, n_heads, n_kv_heads, head_dim, window, scale, work=work)

@@ -187,6 +187,8 @@ class CausalAttention(Part):
     def _fused_qkv(self, h, ctx, slot_map, k_cache, v_cache, rotary_dim, theta, writes):
         """The q|k|v product with rotation and cache write in its epilogue, where a kernel takes
         the rows (a decode step); None otherwise."""
+        if (h.n_rows if isinstance(h, Normed) else h.shape[0]) > ops.SKINNY_MAX_ROWS:
+            return None       # beyond this kernel's rows: the plain product takes the norm as it comes, prepared or not
         args = (ctx.positions, slot_map, k_cache, v_cache, self.num_heads, self.num_kv_heads, self.head_dim,
                 rotary_dim, theta, writes)
         if isinstance(h, Normed):
@@ -196,8 +198,6 @@ class CausalAttention(Part):
             scale = h.fusable_scale() if h._tensor is None and h.rows is None else None
             if scale is not None and ops.gemm_qkv_rope_supported(h.x, h.n_rows, True, self.w_qkv, self.head_dim, rotary_dim):
                 return ops.gemm_qkv_rope(h.x, scale[0], scale[1], self.w_qkv, *args)
-            if h.n_rows > ops.SKINNY_MAX_ROWS:
-                return None       # beyond this kernel's rows: the plain product takes the norm as it comes, prepared or not
             h = h.tensor()
         if ops.gemm_qkv_rope_supported(h, h.shape[0], False, self.w_qkv, self.head_dim, rotary_dim):
             return ops.gemm_qkv_rope(h, None, 0.0, self.w_qkv, *args)

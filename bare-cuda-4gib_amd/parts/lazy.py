@@ -8,7 +8,6 @@ once and keeps the result.
 """
 from __future__ import annotations
 
-import contextlib
 from typing import Any, Dict, Optional, Tuple
 
 import torch
@@ -32,6 +31,19 @@ class Normed:
         """(scale vector, eps) if the norm is a plain RMSNorm that a product may absorb, else None."""
         f = getattr(self.norm, "fusable", None)
         return f() if f is not None else None
+
+
+class _Reading:
+    """While it is entered, the handoff's reading_next is what it was given (NormHandoff.reader)."""
+
+    def __init__(self, handoff: "NormHandoff", reading: Optional[Tuple[Any, bool]]):
+        self.handoff, self.reading, self.before = handoff, reading, None
+
+    def __enter__(self) -> None:
+        self.before, self.handoff.reading_next = self.handoff.reading_next, self.reading
+
+    def __exit__(self, *exc) -> None:
+        self.handoff.reading_next = self.before
 
 
 class NormHandoff:
@@ -74,14 +86,8 @@ class NormHandoff:
         self._left.clear()
         self.next_entry = self.reading_next = None
 
-    @contextlib.contextmanager
-    def reader(self, norm, takes_parts: bool = False):
-        before = self.reading_next
-        self.reading_next = (norm, bool(takes_parts)) if norm is not None else None
-        try:
-            yield
-        finally:
-            self.reading_next = before
+    def reader(self, norm, takes_parts: bool = False) -> "_Reading":
+        return _Reading(self, (norm, bool(takes_parts)) if norm is not None else None)
 
     def leave(self, norm, what) -> None:
         self._left[id(norm)] = what
