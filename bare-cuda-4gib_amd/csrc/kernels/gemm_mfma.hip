@@ -6,8 +6,8 @@
 // and feeds 32x32x16 MFMAs.  Two forms:
 //  - the operand tiles go from memory into LDS without passing registers (k a multiple of 64, operands on 16-byte
 //    boundaries): gemm_mfma_halves_kernel for tiles of 256 x 256, gemm_mfma_turns_kernel for 256 x 192 and 128 x 128,
-//    gemm_mfma_direct_kernel for 256 x 128 and 64 x 64 (and 128 x 64 for q|k|v); whichever lets the busiest CU finish
-//    first, or two of them side by side (parts_of).
+//    gemm_mfma_direct_kernel for 256 x 128 (and 128 x 64 for q|k|v), gemm_mfma_ahead_kernel for 64 x 64; whichever lets the
+//    busiest CU finish first, or two of them side by side (parts_of).
 //  - gemm_mfma_staged_kernel: through registers, 128 x 128 tiles; any k that is a multiple of 8.
 // Every output element is accumulated over k in ascending order in both, whatever the number of
 // rows and the tile: the same bits whichever form and tile a shape selects.
@@ -524,6 +524,57 @@ struct DirectShape {
   static_assert(kRowBytes == 128 || kRowBytes == 256, "rows of 128 or 256 bytes (the slot rule)");
 };
 
+// kSwigluScaledBf16: a tile's RA rows' sums of squares from their parts, a chain a thread (its loads all in flight
+// together), beside the first operands' way into LDS.  (The compiler's wait for these loads knows nothing of the
+// operands asked for before them and so waits for those too: loads return in the order asked.  By the loop's own
+// waits, which count the operands' loads alone, these are done.)
+template <int RA, int THREADS>
+__device__ inline void sum_row_parts(float* part_sum, const RowScaleArgs& rows, int m, long m0, int tid) {
+  static_assert(kPartSums * RA % THREADS == 0 && kPartSums * RA / 4 <= THREADS, "whole chains a thread");
+  constexpr int kAhead = 16;              // parts of a chain asked for together: one way to memory and back for 128 parts
+  // Four rows a thread where the parts' rows allow loads of 16 bytes (a tile begins at a multiple of 64 rows): a CU
+  // takes a wave's load every 19 clocks or so, whatever its width, and a row a thread was 128 of them a tile of 64
+  // rows and 128 parts -- a microsecond, with the operands' loads waiting among them.
+  if (rows.stride % 4 == 0 && reinterpret_cast<uintptr_t>(rows.parts) % 16 == 0) {
+    if (tid < kPartSums * RA / 4) {
+      const int row = (tid % (RA / 4)) * 4, chain = tid / (RA / 4);
+      const bool live = m0 + row < m;     // (then all four are within the stride, which is no less than m)
+      const float* p = rows.parts + (live ? m0 + row : 0);
+      floatx4 ss = {0.f, 0.f, 0.f, 0.f};
+      for (int b0 = chain; b0 < rows.blocks; b0 += kAhead * kPartSums) {
+        floatx4 part[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          const int b = b0 + i * kPartSums;
+          part[i] = live && b < rows.blocks ? *reinterpret_cast<const floatx4*>(p + static_cast<long>(b) * rows.stride)
+                                            : floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) ss += part[i];        // (in ascending order; a part that is not there adds 0)
+      }
+      *reinterpret_cast<floatx4*>(part_sum + chain * RA + row) = ss;
+    }
+  } else
+#pragma unroll
+  for (int turn = 0; turn < kPartSums * RA / THREADS; ++turn) {
+    const int slot = turn * THREADS + tid, row = slot % RA, chain = slot / RA;
+    const bool live = m0 + row < m;
+    const float* p = rows.parts + (live ? m0 + row : 0);
+    float ss = 0.f;
+    for (int b0 = chain; b0 < rows.blocks; b0 += kAhead * kPartSums) {
+      float part[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const int b = b0 + i * kPartSums;
+        part[i] = live && b < rows.blocks ? p[static_cast<long>(b) * rows.stride] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) ss += part[i];          // (in ascending order; a part that is not there adds 0)
+    }
+    part_sum[slot] = ss;
+  }
+}
+
 template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES, int MINWG>
 __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
     const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, void* __restrict__ out, int m, int n, int k, int m_blocks,
@@ -541,11 +592,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
   int bm, bn;
   tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
   const long m0 = static_cast<long>(bm) * RA, n0 = n_first + static_cast<long>(bn) * RW;
-  // gridDim.y > 1: k is cut into that many equal parts (each whole steps), and part y's sums go to an output of
-  // its own, out + y * m * n (the plain store epilogues only: whoever reads them adds the parts up in order)
-  const int nk = k / BK / static_cast<int>(gridDim.y);
-  const size_t k_first = static_cast<size_t>(blockIdx.y) * nk * RB;       // in bytes of a row
-  if constexpr (EPI == kStoreF32) out = static_cast<float*>(out) + static_cast<size_t>(blockIdx.y) * m * n;
+  const int nk = k / BK;
   // The weight comes in the order the weight-streaming kernel reads, so that a model keeps every weight once:
   // [n / 16][k / 32][64 lanes][8] -- blocks of 16 rows x 32 k, 1 KB each, the 16 bytes of row r and k 8 c .. 8 c + 7 at
   // ((r / 16) * (k / 32) + c / 4) * 1024 + ((c % 4) * 16 + r % 16) * 16 (rows beyond n are zeros).  A wave-wide load
@@ -575,14 +622,14 @@ __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
       const int seg = ls ^ slot_key<RB>(trow);
       long row = m0 + trow;
       if (row > m - 1) row = m - 1;
-      src[i] = reinterpret_cast<const unsigned char*>(a + row * k) + k_first + seg * 16;
+      src[i] = reinterpret_cast<const unsigned char*>(a + row * k) + seg * 16;
       dst[i] = g * 1024;
     } else {
       const int gw = g - GA;
       long block = n0 / 16 + gw / kBlocksK;
       if (block > w_row_blocks - 1) block = w_row_blocks - 1;
       src[i] = reinterpret_cast<const unsigned char*>(w) +
-               (block * (k / 32) + static_cast<long>(blockIdx.y) * nk * kBlocksK + gw % kBlocksK) * 1024 + lane * 16;
+               (block * (k / 32) + gw % kBlocksK) * 1024 + lane * 16;
       dst[i] = RA * RB + gw * 1024;
     }
     piece_of_w[i] = !of_a;                  // (the same in all lanes of the wave)
@@ -606,57 +653,6 @@ __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < nk) ask(s);
-
-  // kSwigluScaledBf16: the tile's rows' sums of squares from their parts, a chain a thread (its loads all in flight
-  // together), beside the first operands' way into LDS.  (The compiler's wait for these loads knows nothing of the
-  // operands asked for before them and so waits for those too: loads return in the order asked.  By the loop's own
-  // waits, which count the operands' loads alone, these are done.)
-  __shared__ __align__(16) float part_sum[row_scaled(EPI) ? kPartSums * RA : 4];
-  if constexpr (row_scaled(EPI)) {
-    static_assert(kPartSums * RA % S::kThreads == 0 && kPartSums * RA / 4 <= S::kThreads, "whole chains a thread");
-    constexpr int kAhead = 16;              // parts of a chain asked for together: one way to memory and back for 128 parts
-    // Four rows a thread where the parts' rows allow loads of 16 bytes (a tile begins at a multiple of 64 rows): a CU
-    // takes a wave's load every 19 clocks or so, whatever its width, and a row a thread was 128 of them a tile of 64
-    // rows and 128 parts -- a microsecond, with the operands' loads waiting among them.
-    if (rows.stride % 4 == 0 && reinterpret_cast<uintptr_t>(rows.parts) % 16 == 0) {
-      if (tid < kPartSums * RA / 4) {
-        const int row = (tid % (RA / 4)) * 4, chain = tid / (RA / 4);
-        const bool live = m0 + row < m;     // (then all four are within the stride, which is no less than m)
-        const float* p = rows.parts + (live ? m0 + row : 0);
-        floatx4 ss = {0.f, 0.f, 0.f, 0.f};
-        for (int b0 = chain; b0 < rows.blocks; b0 += kAhead * kPartSums) {
-          floatx4 part[kAhead];
-#pragma unroll
-          for (int i = 0; i < kAhead; ++i) {
-            const int b = b0 + i * kPartSums;
-            part[i] = live && b < rows.blocks ? *reinterpret_cast<const floatx4*>(p + static_cast<long>(b) * rows.stride)
-                                              : floatx4{0.f, 0.f, 0.f, 0.f};
-          }
-#pragma unroll
-          for (int i = 0; i < kAhead; ++i) ss += part[i];        // (in ascending order; a part that is not there adds 0)
-        }
-        *reinterpret_cast<floatx4*>(part_sum + chain * RA + row) = ss;
-      }
-    } else
-#pragma unroll
-    for (int turn = 0; turn < kPartSums * RA / S::kThreads; ++turn) {
-      const int slot = turn * S::kThreads + tid, row = slot % RA, chain = slot / RA;
-      const bool live = m0 + row < m;
-      const float* p = rows.parts + (live ? m0 + row : 0);
-      float ss = 0.f;
-      for (int b0 = chain; b0 < rows.blocks; b0 += kAhead * kPartSums) {
-        float part[kAhead];
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-          const int b = b0 + i * kPartSums;
-          part[i] = live && b < rows.blocks ? p[static_cast<long>(b) * rows.stride] : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) ss += part[i];          // (in ascending order; a part that is not there adds 0)
-      }
-      part_sum[slot] = ss;
-    }
-  }
 
   const int frow = lane % 32, fhalf = lane / 32;
   int aoff[TM], woff[TN], aswz[TM];
@@ -710,7 +706,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
   lds_barrier();            // the last step has been read: LDS is free for the output
 
   store_part<EPI, TM, TN>(acc, reinterpret_cast<float*>(direct_lds) + wave * (S::kPatchBytes / 4), out, m, n, k, m0 + wm * TM * 32,
-                          n0 + wn * TN * 32, lane, ra, rows, row_scaled(EPI) ? part_sum + wm * TM * 32 : nullptr, RA);
+                          n0 + wn * TN * 32, lane, ra, rows);
 }
 
 // ---- the same, two groups of waves in turns ------------------------------------------------------
@@ -1005,6 +1001,132 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
 #undef BC4G_TURN
 #undef BC4G_READ
 
+// ---- 64 x 64, fragments a step ahead --------------------------------------------------------------
+// Few rows or few columns: fewer tiles than CUs, or one or two a CU, where a step is as long as its chain (barrier, ask, read, multiply): 580
+// clocks of it with the kernel above, 128 of them MFMAs, whatever the ring's depth (four to nine stages, steps of 64 or 128: the same).  So all
+// fragments of step t + 1 are read while step t multiplies, a wave's four loads of a step lie side by side in LDS (one LDS address a
+// step: setting it anew waits for the load that uses it), and a stage may be asked for again as soon as its fragments are read: four stages
+// are four steps ahead.  What bounds it now is what a CU can pull: 16 KB a step at 65 to 74 bytes a ns.  Weights from memory: 200 rows, 2,560 x
+// 2,048 11.7 -> 10.6 us, 2,048 x 5,632 26.3 -> 24.0, 256 rows 2,048 x 4,096 21.0 -> 19.7; 64 rows and 11,264 x 2,048, which memory bounds: level.
+//
+// gridDim.y > 1: k is cut into that many equal parts (each whole steps), and part y's sums go to an output of its own,
+// out + y * m * n (kStoreF32 only: whoever reads them adds the parts up in order).
+struct AheadShape {
+  static constexpr int kStages = 4, kStageBytes = 16 * 1024, kThreads = 256, kLdsBytes = kStages * kStageBytes;
+  static constexpr int kPatchBytes = 32 * (32 + 4) * 4;
+  static_assert(4 * kPatchBytes <= kLdsBytes, "the output's patches take the stages' place");
+};
+
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_mfma_ahead_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, void* __restrict__ out,
+                                                                 int m, int n, int k, int m_blocks, int n_blocks, int n_first, const RopeKvArgs ra,
+                                                                 const RowScaleArgs rows) {
+  constexpr int kStages = AheadShape::kStages, kStageBytes = AheadShape::kStageBytes;
+  extern __shared__ __align__(1024) unsigned char direct_lds[];
+  const unsigned lds_base = static_cast<unsigned>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)direct_lds));
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave / 2, wn = wave % 2;
+  int bm, bn;
+  tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
+  const long m0 = static_cast<long>(bm) * 64, n0 = n_first + static_cast<long>(bn) * 64;
+  const int nk = k / 64 / static_cast<int>(gridDim.y);
+  const size_t first_step = static_cast<size_t>(blockIdx.y) * nk;
+  if constexpr (EPI == kStoreF32) out = static_cast<float*>(out) + static_cast<size_t>(blockIdx.y) * m * n;
+
+  // What a wave brings every step, 4 KB: waves 0 and 1 half of the rows of x (past m: the last), 2 and 3 the two blocks of two of the
+  // tile's four block rows of the weight (past n: of the last).
+  const unsigned char* base[4];
+  unsigned off[4];
+  const unsigned step_bytes = wave < 2 ? 128 : 2048;
+  const long w_row_blocks = (static_cast<long>(n) + 15) / 16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (wave < 2) {
+      const int trow = wave * 32 + i * 8 + lane / 8;
+      const long row = min(static_cast<long>(m) - 1 - m0, static_cast<long>(trow));
+      base[i] = reinterpret_cast<const unsigned char*>(a + m0 * k) + first_step * 128 - i * 1024;
+      off[i] = static_cast<unsigned>(row * k * 2 + ((lane % 8) ^ slot_key<128>(trow)) * 16);
+    } else {
+      const long block = min(w_row_blocks - 1, n0 / 16 + (wave - 2) * 2 + i / 2);
+      base[i] = reinterpret_cast<const unsigned char*>(w) + (block * (k / 32) + static_cast<long>(first_step) * 2 + i % 2) * 1024 - i * 1024;
+      off[i] = lane * 16;
+    }
+  }
+  auto ask = [&](int step) {                  // (in order: the bases go on by a step each time)
+    const void* from[4] = {base[0], base[1], base[2], base[3]};
+    load_side_by_side<4>(from, off, lds_base + (step % kStages) * kStageBytes + wave * 4096);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) base[i] += step_bytes;
+  };
+#pragma unroll
+  for (int s = 0; s < kStages; ++s)
+    if (s < nk) ask(s);
+
+  __shared__ __align__(16) float part_sum[row_scaled(EPI) ? kPartSums * 64 : 4];
+  if constexpr (row_scaled(EPI)) sum_row_parts<64, 256>(part_sum, rows, m, m0, tid);
+
+  floatx16 acc[1][1];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[0][0][r] = 0.f;
+
+  const int frow = lane % 32, fhalf = lane / 32;
+  const unsigned char* aread = direct_lds + (wm * 32 + frow) * 128;
+  const int akey = slot_key<128>(wm * 32 + frow);
+  const unsigned char* wread = direct_lds + 8192 + (wn * 2 + frow / 16) * 2048 + (frow % 16) * 16 + fhalf * 256;
+  struct Fragments {
+    uint4 a[4], w[4];
+  };
+  auto read = [&](Fragments& f, int step) {
+    const int at = (step % kStages) * kStageBytes;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      f.a[s] = *reinterpret_cast<const uint4*>(aread + at + (((s * 2 + fhalf) ^ akey) * 16));
+      f.w[s] = *reinterpret_cast<const uint4*>(wread + at + (s / 2) * 1024 + (s % 2) * 512);
+    }
+  };
+  // Step t from `now`, the fragments of t + 1 into `next`.  The barrier comes when this wave's loads of t + 1 have landed and its reads of
+  // step t are back (lds_barrier waits for those): behind it everybody's part of t + 1 is there, and t's stage is free.
+  // (No branch between the reads and the MFMAs, and the wait for the reads of t said in the compiler's own terms too: else it waits for all
+  // reads before the first MFMA.)
+  auto wait_lds_reads = []() { __builtin_amdgcn_s_waitcnt(63 >> 4 << 14 | 0 << 8 | 7 << 4 | 15); };      // lgkmcnt(0)
+  auto multiply = [&](const Fragments& now) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc[0][0] = mfma_32x32x16(now.a[s], now.w[s], acc[0][0]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto turn = [&](int t, const Fragments& now, Fragments& next) {             // (t + kStages < nk)
+    wait_loads<4 * (kStages - 2)>();
+    wait_lds_reads();
+    lds_barrier();
+    ask(t + kStages);
+    read(next, t + 1);
+    multiply(now);
+  };
+  auto late_turn = [&](int t, const Fragments& now, Fragments& next) {        // (t + 1 < nk, nothing left to ask for)
+    wait_for_stage<4, kStages - 2>(nk - 2 - t);
+    wait_lds_reads();
+    lds_barrier();
+    read(next, t + 1);
+    multiply(now);
+  };
+  Fragments even, odd;
+  wait_for_stage<4, kStages - 1>(min(nk - 1, kStages - 1));
+  lds_barrier();
+  read(even, 0);
+  int t = 0;
+  for (; t + kStages + 1 < nk; t += 2) turn(t, even, odd), turn(t + 1, odd, even);
+  if (t + kStages < nk) turn(t, even, odd), even = odd, ++t;
+  for (; t + 2 < nk; t += 2) late_turn(t, even, odd), late_turn(t + 1, odd, even);
+  if (t + 1 < nk) late_turn(t, even, odd), even = odd;
+  multiply(even);
+  lds_barrier();            // the last step has been read: LDS is free for the output
+  store_part<EPI, 1, 1>(acc, reinterpret_cast<float*>(direct_lds) + wave * (AheadShape::kPatchBytes / 4), out, m, n, k, m0 + wm * 32, n0 + wn * 32, lane,
+                        ra, rows, row_scaled(EPI) ? part_sum + wm * 32 : nullptr, 64);
+}
+
 // What a product's kernels get: n columns, of which this launch computes n_cols from n_first on (all of them: 0, n).
 struct Operands {
   const bf16_t* a;
@@ -1029,12 +1151,18 @@ int launch_tiles(Kernel kernel, bool& raised, int rows, int cols, int threads, i
   return 0;
 }
 
+template <int EPI>
+int launch_ahead(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale, int k_parts = 1) {
+  static bool raised = false;
+  return launch_tiles(gemm_mfma_ahead_kernel<EPI>, raised, 64, 64, AheadShape::kThreads, AheadShape::kLdsBytes, o, ra, scale, k_parts);
+}
+
 template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES, int MINWG>
-int launch_direct(const Operands& o, const RopeKvArgs& ra = RopeKvArgs{}, const RowScaleArgs& scale = RowScaleArgs{}, int k_parts = 1) {
+int launch_direct(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
   typedef DirectShape<WM, WN, TM, TN, BK, STAGES> S;
   static bool raised = false;
   return launch_tiles(gemm_mfma_direct_kernel<EPI, WM, WN, TM, TN, BK, STAGES, MINWG>, raised, S::kRowsA, S::kRowsW, S::kThreads, S::kLdsBytes, o, ra,
-                      scale, k_parts);
+                      scale);
 }
 
 template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES>
@@ -1126,7 +1254,7 @@ int launch_form(int form, const Operands& o, const RopeKvArgs& ra, const RowScal
     case 2: return launch_direct<EPI, 4, 2, 2, 2, 64, 3, 1>(o, ra, scale);
     case 3: return launch_turns<EPI, 2, 4, 2, 1, 64, 4>(o, ra, scale);
     case 5: return launch_direct<EPI, 2, 2, 2, 1, 64, 2, 4>(o, ra, scale);
-    default: return launch_direct<EPI, 2, 2, 1, 1, 64, 4, 2>(o, ra, scale);
+    default: return launch_ahead<EPI>(o, ra, scale);
   }
 }
 
@@ -1135,7 +1263,7 @@ int launch_direct_form(const bf16_t* ap, const bf16_t* wp, void* out, int m, int
                        const RowScaleArgs& scale = RowScaleArgs{}) {
   Operands o{ap, wp, out, m, n, k, 0, n, s};
   if constexpr (row_scaled(EPI)) {
-    return launch_direct<EPI, 2, 2, 1, 1, 64, 4, 2>(o, ra, scale);      // (for a decode step's rows, where this is the tile anyway)
+    return launch_ahead<EPI>(o, ra, scale);      // (for a decode step's rows, where this is the tile anyway)
   } else {
     const Parts parts = parts_of(m, n, k, EPI == kRopeKvBf16);
     o.n_cols = parts.n1;
@@ -1226,7 +1354,7 @@ extern "C" int bc4g_gemm_mfma_parts(const void* a, const void* w, int w_packed, 
                "(M=%d N=%d)", k, k_parts, m, n);
   BC4G_REQUIRE(((m + 63L) / 64) * ((n + 63L) / 64) <= 2147483647L, "gemm_mfma_parts: too many tiles");
   const Operands o{static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), parts, m, n, k, 0, n, static_cast<hipStream_t>(stream)};
-  if (int e = launch_direct<kStoreF32, 2, 2, 1, 1, 64, 4, 2>(o, RopeKvArgs{}, RowScaleArgs{}, k_parts)) return e;
+  if (int e = launch_ahead<kStoreF32>(o, RopeKvArgs{}, RowScaleArgs{}, k_parts)) return e;
   return check_launch("gemm_mfma_parts");
 }
 
