@@ -724,18 +724,29 @@ __global__ __launch_bounds__(64 * WM * WN, MINWG) void gemm_mfma_direct_kernel(
 #define BC4G_READ "s_waitcnt lgkmcnt(0)\n\t"
 
 // N loads of a wave to N KB of LDS side by side, load i from bases[i] (the same in every lane) plus each lane's offset.  The LDS address
-// is set once and each load adds i * 1,024 bytes to it, and to its memory address, so its base is that much short of its place.
+// is set once and each load adds i * 1,024 bytes to it, and to its memory address, so its base is that much short of its place.  (The offset
+// field reaches from -4,096 to 4,095: five loads count from the middle one's address.)
+constexpr int kMaxLoads = 5;
 template <int N>
-__device__ inline void load_side_by_side(const void* const (&bases)[4], const unsigned (&off)[4], unsigned lds_address) {
-  static_assert(N == 2 || N == 4, "loads a statement");
+__device__ inline void load_side_by_side(const void* const (&bases)[kMaxLoads], const unsigned (&off)[kMaxLoads], unsigned lds_address) {
+  static_assert(N == 2 || N == 4 || N == 5, "loads a statement");
 #define BC4G_LOAD(v, s, o) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #o "\n\t"
-  if constexpr (N == 2)
+  if constexpr (N == 2) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_LOAD(1, 3, 0) BC4G_LOAD(2, 4, 1024)
                  ::"s"(lds_address), "v"(off[0]), "v"(off[1]), "s"(bases[0]), "s"(bases[1]) : "memory", "m0");
-  else
+  } else if constexpr (N == 4) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_LOAD(1, 5, 0) BC4G_LOAD(2, 6, 1024) BC4G_LOAD(3, 7, 2048) BC4G_LOAD(4, 8, 3072)
                  ::"s"(lds_address), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(bases[0]), "s"(bases[1]), "s"(bases[2]), "s"(bases[3])
                  : "memory", "m0");
+  } else {
+    const void* b[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) b[i] = static_cast<const unsigned char*>(bases[i]) + 2048;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_LOAD(1, 6, -2048) BC4G_LOAD(2, 7, -1024) BC4G_LOAD(3, 8, 0) BC4G_LOAD(4, 9, 1024)
+                 BC4G_LOAD(5, 10, 2048)
+                 ::"s"(lds_address + 2048), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]), "s"(b[0]), "s"(b[1]), "s"(b[2]),
+                 "s"(b[3]), "s"(b[4]) : "memory", "m0");
+  }
 #undef BC4G_LOAD
 }
 
@@ -753,9 +764,8 @@ struct HalvesShape {
 };
 
 template <int EPI>
-__global__ __launch_bounds__(512, 2) void gemm_mfma_halves_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
-                                                                  void* __restrict__ out, int m, int n, int k, int m_blocks, int n_blocks,
-                                                                  int n_first, const RopeKvArgs ra, const RowScaleArgs rows) {
+__device__ __forceinline__ void halves_tile(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, void* __restrict__ out, int m, int n, int k,
+                                            long m0, long n0, const RopeKvArgs& ra, const RowScaleArgs& rows) {
   typedef HalvesShape S;
   extern __shared__ __align__(1024) unsigned char direct_lds[];
   const unsigned lds_base = static_cast<unsigned>(
@@ -763,9 +773,6 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_halves_kernel(const bf16_t* 
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave / 4, wn = wave % 4;
-  int bm, bn;
-  tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
-  const long m0 = static_cast<long>(bm) * 256, n0 = n_first + static_cast<long>(bn) * 256;
   const int nk = k / 64;
 
   // What this wave brings of a half of x: 16 of its 128 rows, in two loads (rows past m: the last).  Of a half of the weight: the step's
@@ -787,8 +794,8 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_halves_kernel(const bf16_t* 
     wbase[h] = reinterpret_cast<const unsigned char*>(w) + block * (k / 32) * 1024;
   }
   auto ask = [&](const unsigned char* first, const unsigned char* second_less_1k, unsigned off0, unsigned off1, unsigned to) {
-    const void* bases[4] = {first, second_less_1k};
-    const unsigned off[4] = {off0, off1};
+    const void* bases[kMaxLoads] = {first, second_less_1k};
+    const unsigned off[kMaxLoads] = {off0, off1};
     load_side_by_side<2>(bases, off, to);
   };
   auto ask_a = [&](int step, int h) {
@@ -877,6 +884,15 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_halves_kernel(const bf16_t* 
                         rows);
 }
 
+template <int EPI>
+__global__ __launch_bounds__(512, 2) void gemm_mfma_halves_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
+                                                                  void* __restrict__ out, int m, int n, int k, int m_blocks, int n_blocks,
+                                                                  int n_first, const RopeKvArgs ra, const RowScaleArgs rows) {
+  int bm, bn;
+  tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
+  halves_tile<EPI>(a, w, out, m, n, k, bm * 256L, n_first + bn * 256L, ra, rows);
+}
+
 // Any tile: a turn is a step of BK, in a ring of STAGES.  256 x 192 (steps of 32: what LDS holds five of) and 128 x 128 (steps of 64).
 // Against the kernel above: 2,048 x 11,264 x 2,048 in 256 x 192 102 -> 96 us, 2,048 x 2,048 x 5,632 in 128 x 128 60 -> 56.5, 1,024 x 4,096 x 14,336 134 ->
 // 128.  (256 x 128, whose waves read 64 x 64 parts, is LDS-bound either way: 112.6 and 113.1 us for the first; 256 x 256 so: 5 % slower than in halves.)
@@ -897,9 +913,8 @@ __device__ inline int turns_key(int row) {
 }
 
 template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES>
-__global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
-                                                                 void* __restrict__ out, int m, int n, int k, int m_blocks, int n_blocks,
-                                                                 int n_first, const RopeKvArgs ra, const RowScaleArgs rows) {
+__device__ __forceinline__ void turns_tile(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, void* __restrict__ out, int m, int n, int k,
+                                           long m0, long n0, const RopeKvArgs& ra, const RowScaleArgs& rows) {
   typedef TurnsShape<WM, WN, TM, TN, BK, STAGES> S;
   constexpr int RA = S::kRowsA, RW = S::kRowsW, RB = S::kRowBytes, N = S::kLoads, kBlocksK = BK / 32, kSlices = BK / 16;
   constexpr int kGroupRows = 1024 / RB;                    // rows of x a wave-wide load covers
@@ -909,17 +924,14 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave / WN, wn = wave % WN;
-  int bm, bn;
-  tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
-  const long m0 = static_cast<long>(bm) * RA, n0 = n_first + static_cast<long>(bn) * RW;
   const int nk = k / BK;
 
   // the N groups of rows (of x) or blocks (of w) this wave brings every step, side by side in LDS (waves past the last group bring
   // the last ones again: the same bytes to the same place); rows past m and blocks past n: the last
   const int g0 = min(wave * N, S::kGroupsA + S::kGroupsW - N);
-  const unsigned char* base[4];
-  unsigned off[4];
-  int advance[4];
+  const unsigned char* base[kMaxLoads];
+  unsigned off[kMaxLoads];
+  int advance[kMaxLoads];
   const long w_row_blocks = (static_cast<long>(n) + 15) / 16;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
@@ -939,7 +951,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
     }
   }
   auto ask = [&](int slot) {                               // the next step's
-    const void* from[4];
+    const void* from[kMaxLoads];
 #pragma unroll
     for (int i = 0; i < N; ++i) from[i] = base[i], base[i] += advance[i];
     load_side_by_side<N>(from, off, lds_base + slot * S::kStageBytes + g0 * 1024);
@@ -1001,6 +1013,41 @@ __global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* _
 #undef BC4G_TURN
 #undef BC4G_READ
 
+template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES>
+__global__ __launch_bounds__(512, 2) void gemm_mfma_turns_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
+                                                                 void* __restrict__ out, int m, int n, int k, int m_blocks, int n_blocks,
+                                                                 int n_first, const RopeKvArgs ra, const RowScaleArgs rows) {
+  typedef TurnsShape<WM, WN, TM, TN, BK, STAGES> S;
+  int bm, bn;
+  tile_of(blockIdx.x, m_blocks, n_blocks, bm, bn);
+  turns_tile<EPI, WM, WN, TM, TN, BK, STAGES>(a, w, out, m, n, k, static_cast<long>(bm) * S::kRowsA, n_first + static_cast<long>(bn) * S::kRowsW, ra, rows);
+}
+
+// ---- rows beyond whole tiles, beside them ---------------------------------------------------------
+// A portion of a prompt with decoded tokens beside it has a few rows more than whole tiles (270, 519): another row of large tiles is
+// nearly all padding, and a whole turn of the chip where the tiles just fitted.  So the whole row tiles (256 x 256, or 128 x 128 with LARGE false) and, on the
+// CUs they leave, 64 x 256 tiles of the rows that remain, in one launch; those come last and fill in.  Every element is added up as before.
+// Weights from memory, gate-up products: 270 x 11,264 x 2,048 34.5 -> 23.2 us (176 tiles of 256 x 128 before, 176 of 128 x 128 and 44 of 64 x 256 now),
+// 519 x 28,672 x 4,096 170 -> 139, 1,030 x 28,672 x 4,096 256 -> 210, 519 x 22,016 x 4,096 127 -> 106; a plain store, 270 x 12,288 x 4,096 66 -> 42.
+typedef TurnsShape<2, 4, 1, 2, 64, 3> RestShape;
+template <int EPI, bool LARGE>
+__global__ __launch_bounds__(512, 2) void gemm_mfma_rest_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, void* __restrict__ out,
+                                                                int m, int n, int k, int m_blocks, int n_blocks, const RopeKvArgs ra,
+                                                                const RowScaleArgs rows) {
+  constexpr int kRows = LARGE ? 256 : 128;
+  const int whole = m_blocks * n_blocks, block = blockIdx.x;
+  int bm, bn;
+  if (block < whole) {
+    tile_of(block, m_blocks, n_blocks, bm, bn);
+    if constexpr (LARGE) halves_tile<EPI>(a, w, out, m, n, k, bm * 256L, bn * 256L, ra, rows);
+    else turns_tile<EPI, 2, 4, 2, 1, 64, 4>(a, w, out, m, n, k, bm * 128L, bn * 128L, ra, rows);
+  } else {
+    const int first = m_blocks * kRows, rest_cols = (n + RestShape::kRowsW - 1) / RestShape::kRowsW;
+    tile_of(block - whole, (m - first + RestShape::kRowsA - 1) / RestShape::kRowsA, rest_cols, bm, bn);
+    turns_tile<EPI, 2, 4, 1, 2, 64, 3>(a, w, out, m, n, k, first + static_cast<long>(bm) * RestShape::kRowsA, static_cast<long>(bn) * RestShape::kRowsW, ra, rows);
+  }
+}
+
 // ---- 64 x 64, fragments a step ahead --------------------------------------------------------------
 // Few rows or few columns: fewer tiles than CUs, or one or two a CU, where a step is as long as its chain (barrier, ask, read, multiply): 580
 // clocks of it with the kernel above, 128 of them MFMAs, whatever the ring's depth (four to nine stages, steps of 64 or 128: the same).  So all
@@ -1038,7 +1085,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_ahead_kernel(const bf16_t* _
   // What a wave brings every step, 4 KB: waves 0 and 1 half of the rows of x (past m: the last), 2 and 3 the two blocks of two of the
   // tile's four block rows of the weight (past n: of the last).
   const unsigned char* base[4];
-  unsigned off[4];
+  unsigned off[kMaxLoads];
   const unsigned step_bytes = wave < 2 ? 128 : 2048;
   const long w_row_blocks = (static_cast<long>(n) + 15) / 16;
 #pragma unroll
@@ -1055,7 +1102,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_ahead_kernel(const bf16_t* _
     }
   }
   auto ask = [&](int step) {                  // (in order: the bases go on by a step each time)
-    const void* from[4] = {base[0], base[1], base[2], base[3]};
+    const void* from[kMaxLoads] = {base[0], base[1], base[2], base[3]};
     load_side_by_side<4>(from, off, lds_base + (step % kStages) * kStageBytes + wave * 4096);
 #pragma unroll
     for (int i = 0; i < 4; ++i) base[i] += step_bytes;
@@ -1217,6 +1264,29 @@ int direct_form(int m, int n, int k, bool long_epilogue) {
   return best;
 }
 
+// Rows beyond whole tiles beside them (gemm_mfma_rest_kernel): the 64 x 256 tiles' times, measured as the others' were, and the time of a launch that
+// begins with `whole` tiles of a form and goes on with `rest` such: those first go to the CUs that the last turn of large tiles leaves.
+constexpr DirectForm kRestForm = {64, 256, 0.50, 0.62, 0.0, 1.0};
+double rest_time(const DirectForm& form, int whole, int rest, int k) {
+  const int cus = compute_units(), steps = k / 64;
+  const double fill = whole + rest < cus ? static_cast<double>(whole + rest) / cus : 1.0;
+  const double large = steps * (form.us_a_step_few + (form.us_a_step_full - form.us_a_step_few) * fill) + form.us_stores;
+  const double small = steps * (kRestForm.us_a_step_few + (kRestForm.us_a_step_full - kRestForm.us_a_step_few) * fill) + kRestForm.us_stores;
+  const int full = whole / cus, busy = whole % cus;
+  const double early = full * large, late = busy ? (full + 1) * large : early;
+  // a turn of small tiles after the other, on the CUs free early and on those free late, whichever ends first
+  int left = rest;
+  double a = early + small, b = late + small, end = late;
+  while (left > 0) {
+    const bool first = busy == 0 || a <= b;
+    left -= first ? cus - busy : busy;
+    end = first ? a : b;
+    (first ? a : b) += small;
+  }
+  // (with tiles waiting for CUs measured 3 to 8 % longer than this)
+  return form.us_around + (end > late ? end : late) * (whole + rest > cus ? 1.05 : 1.0);
+}
+
 // How an output's columns are cut: the first n1 in tiles of `first`, the rest (if any) in tiles of `second`, one launch each.  Tiles that do not
 // fill the last turn of the chip leave CUs idle for a whole tile (3,000 x 11,264 are 528 tiles of 256 x 256: 256, 256 and 16); columns that fill
 // whole turns with large tiles, and smaller tiles for the others, leave less.  Every element is added up as before, by whichever tile.
@@ -1224,13 +1294,25 @@ int direct_form(int m, int n, int k, bool long_epilogue) {
 // by which cut products were measured to be longer than their parts: 3,000 x 11,264 x 2,048 141 -> 129 us (10,752 columns in 256 x 256, 512 in
 // 64 x 64), 1,400 x 11,264 x 2,048 84 -> 78.5, 1,100 x 28,672 x 4,096 287 -> 254.  Without the 8 us 300 x 11,264 x 2,048 was cut: 35 -> 39.
 constexpr double kCutGap = 8.0;
+// Or its rows: whole tiles of `first`, and the rows that remain in the same launch (rest_time; up to four turns of the chip, beyond them a turn more matters
+// little).
 struct Parts {
   int first, n1, second;
+  bool rest;
 };
 Parts parts_of(int m, int n, int k, bool long_epilogue) {
-  Parts best{direct_form(m, n, k, long_epilogue), n, 0};
+  Parts best{direct_form(m, n, k, long_epilogue), n, 0, false};
   if (k < 512) return best;
   double best_time = 0.96 * form_time(kDirectForm[best.first], m, n, k);
+  for (int f = 0; f < 4; f += 3) {
+    const DirectForm& form = kDirectForm[f];
+    const int row_tiles = m / form.rows, beyond = m % form.rows;
+    const long whole = static_cast<long>(row_tiles) * ((n + form.cols - 1) / form.cols);
+    if (whole == 0 || beyond == 0 || whole > 4L * compute_units()) continue;
+    const int rest = (beyond + kRestForm.rows - 1) / kRestForm.rows * ((n + kRestForm.cols - 1) / kRestForm.cols);
+    const double time = rest_time(form, static_cast<int>(whole), rest, k);
+    if (time < best_time) best = Parts{f, n, 0, true}, best_time = time;
+  }
   for (int f = 0; f < 4; ++f) {
     const DirectForm& form = kDirectForm[f];
     const long rows = (m + form.rows - 1) / form.rows, cus = compute_units();
@@ -1239,11 +1321,28 @@ Parts parts_of(int m, int n, int k, bool long_epilogue) {
       if (n1 <= 0 || n1 >= n) continue;
       const int rest = n - static_cast<int>(n1), second = direct_form(m, rest, k, long_epilogue);
       const double time = form_time(form, m, static_cast<int>(n1), k) + form_time(kDirectForm[second], m, rest, k) + kCutGap;
-      if (time < best_time) best = Parts{f, static_cast<int>(n1), second}, best_time = time;
+      if (time < best_time) best = Parts{f, static_cast<int>(n1), second, false}, best_time = time;
       break;      // (fewer turns of large tiles leave more for the small ones)
     }
   }
   return best;
+}
+
+template <int EPI, bool LARGE>
+int launch_rest(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
+  constexpr int kRows = LARGE ? 256 : 128, kLds = LARGE ? HalvesShape::kLdsBytes : TurnsShape<2, 4, 2, 1, 64, 4>::kLdsBytes;
+  static_assert(RestShape::kLdsBytes <= kLds, "both tiles in one workgroup's LDS");
+  static bool raised = false;
+  auto kernel = gemm_mfma_rest_kernel<EPI, LARGE>;
+  if (!raised) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+      return fail("gemm_mfma: cannot raise the dynamic LDS limit");
+    raised = true;
+  }
+  const int m_blocks = o.m / kRows, n_blocks = (o.n + kRows - 1) / kRows;
+  const int rest = (o.m % kRows + RestShape::kRowsA - 1) / RestShape::kRowsA * ((o.n + RestShape::kRowsW - 1) / RestShape::kRowsW);
+  kernel<<<dim3(m_blocks * n_blocks + rest), dim3(512), kLds, o.stream>>>(o.a, o.w, o.out, o.m, o.n, o.k, m_blocks, n_blocks, ra, scale);
+  return 0;
 }
 
 template <int EPI>
@@ -1266,6 +1365,7 @@ int launch_direct_form(const bf16_t* ap, const bf16_t* wp, void* out, int m, int
     return launch_ahead<EPI>(o, ra, scale);      // (for a decode step's rows, where this is the tile anyway)
   } else {
     const Parts parts = parts_of(m, n, k, EPI == kRopeKvBf16);
+    if (parts.rest) return parts.first == 0 ? launch_rest<EPI, true>(o, ra, scale) : launch_rest<EPI, false>(o, ra, scale);
     o.n_cols = parts.n1;
     if (int e = launch_form<EPI>(parts.first, o, ra, scale)) return e;
     if (parts.n1 == n) return 0;
