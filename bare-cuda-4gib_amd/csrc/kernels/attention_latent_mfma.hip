@@ -10,10 +10,9 @@
 //            holds, for its query, eight of the 32 keys, so maximum and sum of a query are in-lane plus two lane swaps
 //   output   O^T[latent x queries] += V^T[latent x keys] P^T[keys x queries] with V = the first `rank` numbers of the
 //            same LDS rows: the weights go from the score registers straight into the B operand (which key a k-slot
-//            stands for is free, as long as A agrees); the A operand wants eight keys of one latent number side by
-//            side, so the latent part of a tile is kept a second time in LDS, transposed ([number][key]), written
-//            two bytes at a time while the tile is staged and read eight bytes at a time (gathering the keys from the
-//            rows themselves, two bytes a read, made the walk wait for LDS 256 times a tile)
+//            stands for is free, as long as A agrees); the A operand, eight keys of one latent number a lane, comes from the
+//            rows as they lie by LDS's transposing read (a second, transposed copy of the latent part, written two bytes at a
+//            time, was a sixth of a prompt's time: 3,557 tokens of eight requests, 16 heads, 262 -> 222 us a layer)
 //
 // The keys may be cut into n_splits parts over workgroups (few rows over a long context: a decode step), whose
 // unnormalised float partials a second kernel merges; the sink joins the sum where the sum is finished.
@@ -28,11 +27,25 @@ namespace bc4g {
 namespace {
 
 constexpr int kKeys = 32;                   // cache rows a key tile holds
-constexpr int kVtPitch = 36;                // 16-bit elements of a row of the transposed latent part (32 keys and a pad)
 constexpr float kLog2e = 1.4426950408889634f;
 
 __device__ inline unsigned pack_bf16(float lo, float hi) {
   return static_cast<unsigned>(bf16_bits_from_float(lo)) | (static_cast<unsigned>(bf16_bits_from_float(hi)) << 16);
+}
+
+// Eight keys of one latent number for every lane, from a tile's rows of `pitch` pieces of 16 bytes: number 16 db + c, keys 4 g .. 4 g + 3 and
+// 16 + those (c = lane % 16, g = lane / 16).  The read transposes: a group of 16 lanes points at four rows of 16 numbers, four numbers a
+// lane, and gets, lane by lane, a column of four.
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+__device__ inline const uint16_t* column_of(const uint4* tile, int pitch, int c, int g) {
+  return reinterpret_cast<const uint16_t*>(tile + (4 * g + c / 4) * pitch) + 4 * (c % 4);
+}
+__device__ inline uint4 read_column(const uint16_t* column, int pitch, int db) {
+  const uint16_t* from = column + db * 16;
+  const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4*)from);
+  const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4*)(from + 16 * 8 * pitch));
+  const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
+  return make_uint4(a.x, a.y, b.x, b.y);
 }
 
 // KS: k-steps of 32 over a cache row (dk <= 32 KS); DB: blocks of 16 over the latent (rank <= 16 DB).
@@ -42,7 +55,7 @@ __global__ __launch_bounds__(256, 2) void latent_mfma_kernel(
     const bf16_t* __restrict__ cache, const float* __restrict__ sink, const int32_t* __restrict__ block_table,
     int table_stride, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_ctx, int n_tokens, int heads,
     int rank, int dk, int page_tokens, int window, float scale, int hb, int tpt, int n_hg, int n_splits) {
-  extern __shared__ uint4 tile[];                             // [kKeys][dk / 8 + 1] pieces of 16 bytes, then the transposed part
+  extern __shared__ uint4 tile[];                             // [kKeys][dk / 8 + 1] pieces of 16 bytes
   const int s = blockIdx.y, z = blockIdx.z;
   const int tok0 = seq_start[s], n_tok = seq_start[s + 1] - tok0, cached = seq_ctx[s];
   const int n_tb = (n_tok + tpt - 1) / tpt, n_tiles = n_tb * n_hg;
@@ -87,7 +100,6 @@ __global__ __launch_bounds__(256, 2) void latent_mfma_kernel(
   for (int db = 0; db < DB; ++db) acc[db] = floatx4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   const float scale2 = scale * kLog2e;                        // exponents to the base 2
-  uint16_t* vt = reinterpret_cast<uint16_t*>(tile + kKeys * pitch);     // [rank][kVtPitch]: the latent part, transposed
 
   // Staging: eight threads a key, each with every eighth 16-byte piece of its row -- one look at the block table a
   // thread and tile, all of a thread's loads asked for together, and the next tile's asked for before this tile is
@@ -113,15 +125,6 @@ __global__ __launch_bounds__(256, 2) void latent_mfma_kernel(
     for (int p = 0; p < kPieces; ++p) {
       const int part = st_sub + 8 * p;
       if (part < cpr) tile[st_key * pitch + part] = stage[p];
-      if (part * 8 < rank) {
-        uint16_t* to = vt + part * 8 * kVtPitch + st_key;
-        const unsigned w[4] = {stage[p].x, stage[p].y, stage[p].z, stage[p].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          to[(2 * e) * kVtPitch] = static_cast<uint16_t>(w[e] & 0xffffu);
-          to[(2 * e + 1) * kVtPitch] = static_cast<uint16_t>(w[e] >> 16);
-        }
-      }
     }
     lds_barrier();
     if (wave_live) {
@@ -160,15 +163,10 @@ __global__ __launch_bounds__(256, 2) void latent_mfma_kernel(
       for (int db = 0; db < DB; ++db) acc[db] *= alpha;
     }
     const uint4 pf = make_uint4(pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7]));
-    const uint16_t* col = vt + c * kVtPitch + 4 * g;          // latent number c of a block, keys 4g .. 4g + 3
+    const uint16_t* column = column_of(tile, pitch, c, g);
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
-      if (db * 16 < rank) {
-        const uint2 lo = *reinterpret_cast<const uint2*>(col + db * 16 * kVtPitch);
-        const uint2 hi = *reinterpret_cast<const uint2*>(col + db * 16 * kVtPitch + 16);
-        const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
-        acc[db] = mfma_16x16x32(a, pf, acc[db]);
-      }
+      if (db * 16 < rank) acc[db] = mfma_16x16x32(read_column(column, pitch, db), pf, acc[db]);
     }
     }
     lds_barrier();                                            // the tile has been read by everyone
@@ -205,16 +203,19 @@ __global__ __launch_bounds__(256, 2) void latent_mfma_kernel(
 // the queries and of the sums in registers, and a tile's chain of LDS reads and matrix instructions is that much
 // shorter.  A workgroup has WAVES waves and WAVES / G tiles that follow each other.  Four waves on one tile serve a
 // decode step (a request's one row of up to sixteen heads is one tile).  (Eight waves on four tiles, two a tile, spill
-// nothing and were tried for prompts: no faster at 16 heads and slower at 32 than the form above -- its 90 KB of LDS
+// nothing and were tried for prompts: no faster at 16 heads and slower at 32 than the form above -- its 90 KB of LDS (with a transposed copy)
 // leave one workgroup a CU, whose eight waves then all wait at the same barriers, where two workgroups of the form
 // above stage and compute beside each other.)
+// A decode step's walk of a tile or two is a chain of waits -- the request's place, its table, its keys, then the scores' exchange -- so the first
+// keys are asked for before the queries, and parts beyond the last key neither write sums nor have them merged: 8 requests of 100 to 700 tokens,
+// 16 heads, walk and merge 17.0 -> 15.5 us.
 template <int KS, int DB, int G, int WAVES>
 __global__ __launch_bounds__(kWave * WAVES) void latent_mfma_shared_kernel(
     const float* __restrict__ q_lat, float* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     const bf16_t* __restrict__ cache, const float* __restrict__ sink, const int32_t* __restrict__ block_table,
     int table_stride, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_ctx, int n_tokens, int heads,
     int rank, int dk, int page_tokens, int window, float scale, int hb, int tpt, int n_hg, int n_splits) {
-  extern __shared__ uint4 tile[];                             // the tile, its latent part transposed, the partial scores
+  extern __shared__ uint4 tile[];                             // the tile, the partial scores
   constexpr int KW = (KS + G - 1) / G, DW = (DB + G - 1) / G;   // k-steps and latent blocks of a wave
   constexpr int TILES = WAVES / G, SUBS = 2 * WAVES;            // tiles of a workgroup; threads that stage one key
   const int s = blockIdx.y, z = blockIdx.z;
@@ -240,61 +241,63 @@ __global__ __launch_bounds__(kWave * WAVES) void latent_mfma_shared_kernel(
   const int per = (kt_end - kt_begin + n_splits - 1) / n_splits;
   const int kt_lo = kt_begin + z * per, kt_hi = min(kt_end, kt_lo + per);
 
+  // Staging: SUBS threads a key, each with every SUBS-th 16-byte piece of its row -- one look at the block table a
+  // thread and tile, all of a thread's loads asked for together: the first tile's before the queries', the next one's before a tile
+  // is worked on.
+  constexpr int kPieces = (KS * 4 + SUBS - 1) / SUBS;
+  const int st_key = threadIdx.x / SUBS, st_sub = threadIdx.x % SUBS;
+  uint4 stage[kPieces];
+  auto fetch = [&](int kt) {
+    const int j = kt * kKeys + st_key;
+    const bool there = j >= first_pos && j <= last_pos;
+    const bf16_t* src = cache;
+    if (there) src = cache + (static_cast<long>(table[j / page_tokens]) * page_tokens + j % page_tokens) * dk;
+#pragma unroll
+    for (int p = 0; p < kPieces; ++p) {
+      const int part = st_sub + SUBS * p;
+      stage[p] = there && part < cpr ? load16(src + part * 8) : zero16();
+    }
+  };
+  const long row = static_cast<long>(tok0 + tq) * heads + head;
+  if (kt_lo >= kt_hi) {                                       // (a part without a key: its sums are not written, the merge does not ask for them)
+    if (q_live && part_of_tile == 0 && g == 0) *reinterpret_cast<float2*>(part_ml + (static_cast<long>(z) * n_tokens * heads + row) * 2) = make_float2(-INFINITY, 0.f);
+    return;
+  }
+  fetch(kt_lo);
+
   uint4 qf[KW];
   {
-    const float* qrow = q_lat + (static_cast<long>(tok0 + tq) * heads + head) * dk;
+    const float* qrow = q_lat + row * dk;
+    float4 a[KW], b[KW];
 #pragma unroll
     for (int i = 0; i < KW; ++i) {
       const int ks = part_of_tile + G * i;
-      qf[i] = zero16();
+      a[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (q_live && ks * 32 < dk) {
-        const float4 a = *reinterpret_cast<const float4*>(qrow + ks * 32 + 8 * g);
-        const float4 b = *reinterpret_cast<const float4*>(qrow + ks * 32 + 8 * g + 4);
-        qf[i] = make_uint4(pack_bf16(a.x, a.y), pack_bf16(a.z, a.w), pack_bf16(b.x, b.y), pack_bf16(b.z, b.w));
+        a[i] = *reinterpret_cast<const float4*>(qrow + ks * 32 + 8 * g);
+        b[i] = *reinterpret_cast<const float4*>(qrow + ks * 32 + 8 * g + 4);
       }
     }
+#pragma unroll
+    for (int i = 0; i < KW; ++i)
+      qf[i] = make_uint4(pack_bf16(a[i].x, a[i].y), pack_bf16(a[i].z, a[i].w), pack_bf16(b[i].x, b[i].y), pack_bf16(b[i].z, b[i].w));
   }
   floatx4 acc[DW];
 #pragma unroll
   for (int i = 0; i < DW; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   const float scale2 = scale * kLog2e;
-  uint16_t* vt = reinterpret_cast<uint16_t*>(tile + kKeys * pitch);
-  float4* partial = reinterpret_cast<float4*>(reinterpret_cast<char*>(tile) + kKeys * pitch * 16 + ((rank * kVtPitch * 2 + 15) / 16) * 16);
+  float4* partial = reinterpret_cast<float4*>(tile + kKeys * pitch);
 
-  // Staging: SUBS threads a key, each with every SUBS-th 16-byte piece of its row -- one look at the block table a
-  // thread and tile, all of a thread's loads asked for together.
-  constexpr int kPieces = (KS * 4 + SUBS - 1) / SUBS;
-  const int st_key = threadIdx.x / SUBS, st_sub = threadIdx.x % SUBS;
-  uint4 stage[kPieces];
   for (int kt = kt_lo; kt < kt_hi; ++kt) {
     const int j0 = kt * kKeys;
-    {
-      const int j = j0 + st_key;
-      const bool there = j >= first_pos && j <= last_pos;
-      const bf16_t* src = cache;
-      if (there) src = cache + (static_cast<long>(table[j / page_tokens]) * page_tokens + j % page_tokens) * dk;
-#pragma unroll
-      for (int p = 0; p < kPieces; ++p) {
-        const int part = st_sub + SUBS * p;
-        stage[p] = there && part < cpr ? load16(src + part * 8) : zero16();
-      }
-    }
 #pragma unroll
     for (int p = 0; p < kPieces; ++p) {
       const int part = st_sub + SUBS * p;
       if (part < cpr) tile[st_key * pitch + part] = stage[p];
-      if (part * 8 < rank) {
-        uint16_t* to = vt + part * 8 * kVtPitch + st_key;
-        const unsigned w[4] = {stage[p].x, stage[p].y, stage[p].z, stage[p].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          to[(2 * e) * kVtPitch] = static_cast<uint16_t>(w[e] & 0xffffu);
-          to[(2 * e + 1) * kVtPitch] = static_cast<uint16_t>(w[e] >> 16);
-        }
-      }
     }
     lds_barrier();
+    if (kt + 1 < kt_hi) fetch(kt + 1);
     floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
     if (wave_live) {
 #pragma unroll
@@ -344,15 +347,11 @@ __global__ __launch_bounds__(kWave * WAVES) void latent_mfma_shared_kernel(
         for (int i = 0; i < DW; ++i) acc[i] *= alpha;
       }
       const uint4 pf = make_uint4(pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7]));
-      const uint16_t* col = vt + c * kVtPitch + 4 * g;
+      const uint16_t* column = column_of(tile, pitch, c, g);
 #pragma unroll
       for (int i = 0; i < DW; ++i) {
         const int db = part_of_tile + G * i;
-        if (db * 16 < rank) {
-          const uint2 lo = *reinterpret_cast<const uint2*>(col + db * 16 * kVtPitch);
-          const uint2 hi = *reinterpret_cast<const uint2*>(col + db * 16 * kVtPitch + 16);
-          acc[i] = mfma_16x16x32(make_uint4(lo.x, lo.y, hi.x, hi.y), pf, acc[i]);
-        }
+        if (db * 16 < rank) acc[i] = mfma_16x16x32(read_column(column, pitch, db), pf, acc[i]);
       }
     }
     lds_barrier();                                            // the tile has been read by everyone
@@ -360,7 +359,6 @@ __global__ __launch_bounds__(kWave * WAVES) void latent_mfma_shared_kernel(
   if (!q_live) return;
   l += __shfl_xor(l, 16, kWave);
   l += __shfl_xor(l, 32, kWave);
-  const long row = static_cast<long>(tok0 + tq) * heads + head;
   float inv = 1.f;
   float* o = part_o + (static_cast<long>(z) * n_tokens * heads + row) * rank;
   if (n_splits == 1) {
@@ -388,6 +386,7 @@ __global__ __launch_bounds__(kMergeBlock) void latent_merge_kernel(const float* 
                                                                    const float* __restrict__ sink, float* __restrict__ out,
                                                                    long rows, int heads, int rank, int n_splits) {
   __shared__ float weight[kWave + 1];
+  __shared__ int last_part;
   const long row = blockIdx.x;
   if (threadIdx.x < kWave) {
     const int lane = threadIdx.x;
@@ -400,10 +399,13 @@ __global__ __launch_bounds__(kMergeBlock) void latent_merge_kernel(const float* 
     const float wz = __builtin_amdgcn_exp2f(mz - big);
     const float total = wave_sum(lz * wz) + (sink ? __builtin_amdgcn_exp2f(sink[row % heads] * kLog2e - big) : 0.f);
     weight[lane] = wz;
-    if (lane == 0) weight[kWave] = 1.0f / total;
+    // (parts without a key, the last ones, left no sums)
+    const unsigned long long some = __ballot(mz != -INFINITY);
+    if (lane == 0) weight[kWave] = 1.0f / total, last_part = kWave - __builtin_clzll(some | 1);
   }
   __syncthreads();
   const float inv = weight[kWave];
+  n_splits = __builtin_amdgcn_readfirstlane(last_part);
   for (int d = 4 * threadIdx.x; d < rank; d += 4 * kMergeBlock) {
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 8
@@ -455,17 +457,16 @@ extern "C" int bc4g_attention_latent_mfma(const float* q_lat, float* out, float*
   // wave on each
   const bool one_tile = most_tiles < 4;
   dim3 grid(one_tile ? most_tiles : ceil_div(most_tiles, 4), n_seqs, n_splits);
-  const size_t lds = static_cast<size_t>(kKeys) * (dk / 8 + 1) * 16 + (static_cast<size_t>(rank) * kVtPitch * 2 + 15) / 16 * 16 +
-                     (one_tile ? 4 * kWave * 32 : 0);
+  const size_t lds = static_cast<size_t>(kKeys) * (dk / 8 + 1) * 16 + (one_tile ? 4 * kWave * 32 : 0);
   const bf16_t* kc = static_cast<const bf16_t*>(cache);
   // (more than 64 KB of LDS a workgroup has to be asked for, once for a kernel: the most this kernel ever takes)
 #define BC4G_LATENT(KS, DB)                                                                                                 \
   static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_mfma_kernel<KS, DB>),         \
                                                         hipFuncAttributeMaxDynamicSharedMemorySize,                          \
-                                                        kKeys * (KS * 4 + 1) * 16 + DB * 16 * kVtPitch * 2);                 \
+                                                        kKeys * (KS * 4 + 1) * 16);                 \
   static const hipError_t allowed4 = hipFuncSetAttribute(                                                                    \
       reinterpret_cast<const void*>(&latent_mfma_shared_kernel<KS, DB, 4, 4>), hipFuncAttributeMaxDynamicSharedMemorySize,   \
-      kKeys * (KS * 4 + 1) * 16 + DB * 16 * kVtPitch * 2 + 4 * kWave * 32);                                                  \
+      kKeys * (KS * 4 + 1) * 16 + 4 * kWave * 32);                                                  \
   BC4G_REQUIRE(allowed == hipSuccess && allowed4 == hipSuccess,                                                              \
                "attention_latent_mfma: %zu bytes of LDS a workgroup are refused", lds);                                       \
   if (one_tile)                                                                                                               \

@@ -1,0 +1,80 @@
+"""Latent attention of single decoded rows whose keys are cut into parts, beside requests too short to have a key in every part; and the
+cache row of sizes beside what a thread holds at once: against the same in float64."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+PAGE = 64
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from bare_cuda_4gib_amd.csrc import ops as _ops
+    return _ops
+
+
+def _i32(x):
+    return torch.tensor(x, dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.parametrize("rank,rot,heads", [(512, 64, 16), (256, 64, 5), (64, 32, 20), (96, 32, 16)])
+@pytest.mark.parametrize("lengths", [[1, 700, 33, 32], [2050, 31], [1], [65, 64, 63]])
+@pytest.mark.parametrize("window", [0, 70])
+def test_parts_without_a_key(ops, rank, rot, heads, lengths, window):
+    gen = torch.Generator().manual_seed(rank + sum(lengths))
+    row, n = rank + rot, len(lengths)
+    pages = [-(-x // PAGE) for x in lengths]
+    cache = torch.randn(sum(pages), PAGE, row, generator=gen).bfloat16()
+    q, sink = torch.randn(n, heads, row, generator=gen), torch.randn(heads, generator=gen)
+    order = torch.randperm(sum(pages), generator=gen).tolist()
+    table = torch.zeros(n, max(pages), dtype=torch.int32)
+    for s in range(n):
+        table[s, :pages[s]] = torch.tensor(order[sum(pages[:s]):sum(pages[:s + 1])], dtype=torch.int32)
+    ctx = SimpleNamespace(seq_start=list(range(n + 1)), n_seqs=n, max_kv_len=max(lengths), captured=False, row_seq=_i32(list(range(n))),
+                          positions=_i32([x - 1 for x in lengths]), seq_start_dev=_i32(list(range(n + 1))), seq_ctx_dev=_i32([x - 1 for x in lengths]))
+    scale = row ** -0.5
+    got = ops.attention_latent(q.to(DEV), cache.to(DEV), sink.to(DEV), table.to(DEV), ctx, heads, rank, rot, PAGE, window, scale).cpu()
+    for s, length in enumerate(lengths):
+        first = max(0, length - window) if window else 0
+        keys = torch.cat([cache[p] for p in table[s, :pages[s]].tolist()])[first:length].double()
+        scores = (q[s].bfloat16().double() @ keys.T) * scale
+        p = torch.softmax(torch.cat([scores, sink.double()[:, None]], 1), 1)[:, :-1]
+        want = p @ keys[:, :rank]
+        # weights rounded to bfloat16 (2^-9 of each), and scores in float: a sum of weights of at most one times the largest value
+        assert (got[s].double() - want).abs().max() < 2.0 ** -8 * keys[:, :rank].abs().max()
+
+
+@pytest.mark.parametrize("rank,rot,dims,heads", [(512, 64, 64, 16), (1000, 8, 4, 3), (1, 2, 2, 1), (130, 200, 130, 7), (24, 0, 0, 2)])
+@pytest.mark.parametrize("halves", [False, True])
+def test_cache_rows_of_any_size(ops, rank, rot, dims, heads, halves):
+    gen = torch.Generator().manual_seed(rank)
+    t, plain, eps = 5, 8, 1e-5
+    q, dkv = torch.randn(t, heads * (plain + rot), generator=gen), torch.randn(t, rank + rot, generator=gen)
+    g, angle = torch.randn(rank, generator=gen), torch.randn(t, max(dims // 2, 1), generator=gen)
+    angles = torch.stack([angle.cos(), angle.sin()], -1).contiguous()
+    cache, slots = torch.zeros(2, 4, rank + rot), [6, 0, 3, 5, 1]
+    q_lat = torch.zeros(t, heads, rank + rot)
+    on = [x.to(DEV) for x in (q, dkv, g, angles, cache, q_lat)]
+    ops.latent_prepare(on[0], on[1], on[2], eps, on[3] if dims else None, _i32(slots), on[4], on[5], heads, plain, rot, rank, dims, halves=halves)
+
+    def turned(u):                                   # [t, ..., rot]
+        a = u.double().clone()
+        i = torch.arange(dims // 2)
+        x, y = (i, i + dims // 2) if halves else (2 * i, 2 * i + 1)
+        shape = (t,) + (1,) * (u.dim() - 2) + (dims // 2,)
+        c, s = (angles[:, :dims // 2, k].double().view(shape) for k in (0, 1))
+        a[..., x], a[..., y] = u[..., x].double() * c - u[..., y].double() * s, u[..., y].double() * c + u[..., x].double() * s
+        return a
+
+    lat = dkv[:, :rank].double()
+    rows = torch.cat([lat / torch.sqrt((lat * lat).mean(1, keepdim=True) + eps) * g.double(), turned(dkv[:, rank:])], 1)
+    bound = 2.0 ** -20 * 8                           # a few float roundings of numbers up to 8
+    assert (on[4].cpu().view(8, -1)[slots].double() - rows).abs().max() < bound
+    if rot:
+        want = turned(q.view(t, heads, plain + rot)[..., plain:])
+        assert (on[5].cpu()[..., rank:].double() - want).abs().max() < bound
