@@ -296,9 +296,11 @@ int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const float* w, const
                      void* out, int out_dtype, float* ssq, int n_rows, int hidden, float eps, void* stream);
 // out[r] = h + bias + (the causal convolution of h) with h = the RMSNorm of x[r], for a step in which request r brings row r alone:
 // bc4g_rmsnorm and bc4g_causal_conv (add_input) in one launch, the same bits.  w float32 [taps][hidden], state [slots, taps - 1, hidden]
-// in the output's type; 2 to 4 taps, hidden a multiple of 8 up to 4096, everything on 16-byte boundaries.
-int bc4g_rmsnorm_conv(const float* x, const void* norm_w, int norm_w_dtype, float eps, const float* w, const float* bias, void* out,
-                      void* state, int dtype, const int32_t* slots, int n_rows, int hidden, int taps, void* stream);
+// in the output's type; 2 to 4 taps, hidden a multiple of 8 up to 4096, everything on 16-byte boundaries.  add_y (null: nothing): first
+// x[r] += the RMSNorm of add_y[r] (float32, scale add_w, add_eps), as bc4g_rmsnorm_add does it.
+int bc4g_rmsnorm_conv(float* x, const float* add_y, const float* add_w, float add_eps, const void* norm_w, int norm_w_dtype, float eps,
+                      const float* w, const float* bias, void* out, void* state, int dtype, const int32_t* slots, int n_rows, int hidden,
+                      int taps, void* stream);
 // out = act(in) elementwise with act(z) = softplus(p) z^2 + z / 2 for z > 0 and (1/2 + softplus(q)) (e^z - 1 - z) + z / 2
 // otherwise; pq = (p, q) float32 on the device.
 int bc4g_xielu(const void* in, void* out, int dtype, const float* pq, long total, void* stream);

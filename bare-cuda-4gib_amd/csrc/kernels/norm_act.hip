@@ -143,11 +143,18 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_add_rows_kernel(float* __restr
 // h = the norm of x[r] as the norm kernel leaves it, out[r] = h + (bias + sum_j w[j] tail[j] + w[TAPS - 1] h), and the request's tail
 // moves on by h.  What the two kernels would compute, bit for bit; widths as above.  8 rows of 2,048: 4.5 us where the
 // two took 11.5, the second of them four trips to memory one after the other.
-template <typename TN, typename T, int CHUNKS, int TAPS>
-__global__ __launch_bounds__(kBlock) void rmsnorm_conv_rows_kernel(const float* __restrict__ x, const TN* __restrict__ norm_w, float eps,
+// ADD: what the sublayer before left to be added comes first, x[r] += y[r] * rsqrt(mean(y[r]^2) + add_eps) * add_w (a launch of 4 us between
+// two layers of a step that has next to nothing to do), in the order of rmsnorm_add_rows_kernel, the same bits.
+struct AddFirst {
+  const float* y;
+  const float* w;
+  float eps;
+};
+template <typename TN, typename T, int CHUNKS, int TAPS, bool ADD>
+__global__ __launch_bounds__(kBlock) void rmsnorm_conv_rows_kernel(float* __restrict__ x, const TN* __restrict__ norm_w, float eps,
                                                                    const float* __restrict__ w, const float* __restrict__ bias,
                                                                    T* __restrict__ out, T* __restrict__ state,
-                                                                   const int32_t* __restrict__ slots, int hidden) {
+                                                                   const int32_t* __restrict__ slots, int hidden, const AddFirst add) {
   __shared__ float scratch[16];
   const size_t at = static_cast<size_t>(blockIdx.x) * hidden;
   T* tail = state + static_cast<size_t>(slots[blockIdx.x]) * (TAPS - 1) * hidden;
@@ -165,6 +172,39 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_conv_rows_kernel(const float* 
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) load_eight(tail + static_cast<size_t>(j) * hidden + i, tv[c][j]);
       if (bias != nullptr) load_eight(bias + i, bv[c]);
+    }
+  }
+  if constexpr (ADD) {
+    __shared__ float add_scratch[16];
+    __shared__ __align__(16) float turned[CHUNKS * kBlock * 8];
+    float yv[CHUNKS][8], av[CHUNKS][8];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int i = (c * kBlock + threadIdx.x) * 8;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) yv[c][e] = av[c][e] = 0.f;
+      if (i < hidden) {
+        load_eight(add.y + at + i, yv[c]);
+        load_eight(add.w + i, av[c]);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) store_eight(turned + (c * kBlock + threadIdx.x) * 8, yv[c]);
+    __syncthreads();
+    float sq = 0.f;
+#pragma unroll
+    for (int j = 0; j < CHUNKS * 8; ++j) {
+      const float v = turned[j * kBlock + threadIdx.x];        // (zeros beyond the row)
+      sq = fmaf(v, v, sq);
+    }
+    const float by = 1.0f / sqrtf(block_sum(sq, add_scratch) / static_cast<float>(hidden) + add.eps);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int i = (c * kBlock + threadIdx.x) * 8;
+      if (i >= hidden) continue;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xv[c][e] += yv[c][e] * by * av[c][e];
+      store_eight(x + at + i, xv[c]);
     }
   }
   float ss = 0.f;
@@ -446,18 +486,26 @@ extern "C" int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const floa
   return check_launch("rmsnorm_add");
 }
 
-extern "C" int bc4g_rmsnorm_conv(const float* x, const void* norm_w, int norm_w_dtype, float eps, const float* w, const float* bias, void* out,
-                                 void* state, int dtype, const int32_t* slots, int n_rows, int hidden, int taps, void* stream) {
+extern "C" int bc4g_rmsnorm_conv(float* x, const float* add_y, const float* add_w, float add_eps, const void* norm_w, int norm_w_dtype, float eps,
+                                 const float* w, const float* bias, void* out, void* state, int dtype, const int32_t* slots, int n_rows, int hidden,
+                                 int taps, void* stream) {
   BC4G_REQUIRE(n_rows >= 0 && hidden > 0 && hidden % 8 == 0 && hidden <= 4096 && taps >= 2 && taps <= 4,
                "rmsnorm_conv: rows=%d of H=%d (a multiple of 8, at most 4096) with %d taps (2 to 4)", n_rows, hidden, taps);
   BC4G_REQUIRE(x && norm_w && w && out && state && slots && on_16(x) && on_16(norm_w) && on_16(w) && on_16(bias) && on_16(out) && on_16(state),
                "rmsnorm_conv: a tensor is missing, or not on a 16-byte boundary");
+  BC4G_REQUIRE(!add_y == !add_w && on_16(add_y) && on_16(add_w), "rmsnorm_conv: what is added first is rows and their norm's scale, on 16-byte boundaries");
   BC4G_REQUIRE((norm_w_dtype == kF32 || norm_w_dtype == kBF16) && (dtype == kF32 || dtype == kBF16), "rmsnorm_conv: unknown dtypes w=%d out=%d", norm_w_dtype, dtype);
   if (n_rows == 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define BC4G_NORM_CONV(TN, T, C, TAPS)                                                                                             \
-  rmsnorm_conv_rows_kernel<TN, T, C, TAPS><<<n_rows, kBlock, 0, s>>>(x, static_cast<const TN*>(norm_w), eps, w, bias, static_cast<T*>(out), \
-                                                                     static_cast<T*>(state), slots, hidden)
+  const AddFirst add{add_y, add_w, add_eps};
+#define BC4G_NORM_CONV_ADD(TN, T, C, TAPS, ADD)                                                                                            \
+  rmsnorm_conv_rows_kernel<TN, T, C, TAPS, ADD><<<n_rows, kBlock, 0, s>>>(x, static_cast<const TN*>(norm_w), eps, w, bias, static_cast<T*>(out), \
+                                                                          static_cast<T*>(state), slots, hidden, add)
+#define BC4G_NORM_CONV(TN, T, C, TAPS)                         \
+  do {                                                         \
+    if (add_y) BC4G_NORM_CONV_ADD(TN, T, C, TAPS, true);       \
+    else BC4G_NORM_CONV_ADD(TN, T, C, TAPS, false);            \
+  } while (0)
 #define BC4G_NORM_TAPS(TN, T, C)                       \
   do {                                                 \
     if (taps == 2) BC4G_NORM_CONV(TN, T, C, 2);        \
@@ -476,6 +524,7 @@ extern "C" int bc4g_rmsnorm_conv(const float* x, const void* norm_w, int norm_w_
 #undef BC4G_NORM_WIDTH
 #undef BC4G_NORM_TAPS
 #undef BC4G_NORM_CONV
+#undef BC4G_NORM_CONV_ADD
   return check_launch("rmsnorm_conv");
 }
 

@@ -1570,15 +1570,24 @@ def rmsnorm_add(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: flo
 
 
 def rmsnorm_conv(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, out_dtype: torch.dtype, weight: torch.Tensor, state: torch.Tensor,
-                 ctx, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                 ctx, bias: Optional[torch.Tensor] = None, adds: Optional[Tuple[torch.Tensor, torch.Tensor, float]] = None) -> Optional[torch.Tensor]:
     """h + causal_conv(h) with h = rmsnorm(x) in one kernel, for a step in which every request brings one row (the state moves
     on as causal_conv moves it, bit for bit); None where the kernel does not take the step, the width (a multiple of 8 up to 4,096)
-    or the taps (2 to 4)."""
+    or the taps (2 to 4).  ``adds`` (y, weight, eps): rmsnorm_add(x, y, weight, eps) first, in place, y in float32 (None: nothing has been
+    added either)."""
     taps, hidden = weight.shape
     if (ctx.n_tokens != ctx.n_seqs or ctx.n_tokens == 0 or x.dim() != 2 or x.dtype != torch.float32 or not 2 <= taps <= 4 or hidden > 4096 or state.dtype != out_dtype
             or not _norms_whole_rows(hidden, x, norm_weight, weight, state, bias)):
         return None
-    _dev("rmsnorm_conv", x, norm_weight, weight, state, bias)
+    y = add_weight = None
+    add_eps = 0.0
+    if adds is not None:
+        y, add_weight, add_eps = adds
+        if y.dtype != torch.float32 or not _norms_whole_rows(hidden, y, add_weight):
+            return None
+        _f32("rmsnorm_conv", "y", y, (ctx.n_tokens, hidden))
+        _f32("rmsnorm_conv", "add weight", add_weight, (hidden,))
+    _dev("rmsnorm_conv", x, norm_weight, weight, state, bias, y, add_weight)
     if tuple(x.shape) != (ctx.n_tokens, hidden) or tuple(norm_weight.shape) != (hidden,) or tuple(state.shape[1:]) != (taps - 1, hidden):
         raise KernelError(f"rmsnorm_conv: x {tuple(x.shape)}, norm scale {tuple(norm_weight.shape)} and state {tuple(state.shape)} do not go with {taps} taps of {hidden}")
     _f32("rmsnorm_conv", "weight", weight, (taps, hidden))
@@ -1588,7 +1597,7 @@ def rmsnorm_conv(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, out_dty
     n = ctx.n_tokens
     _check_grouping("rmsnorm_conv", ctx, n)
     out = torch.empty((n, hidden), dtype=out_dtype, device=x.device)
-    library.call("bc4g_rmsnorm_conv", _ptr(x), _ptr(norm_weight), _code(norm_weight, "rmsnorm_conv"), float(eps), _ptr(weight), _ptr(bias), _ptr(out),
+    library.call("bc4g_rmsnorm_conv", _ptr(x), _ptr(y), _ptr(add_weight), float(add_eps), _ptr(norm_weight), _code(norm_weight, "rmsnorm_conv"), float(eps), _ptr(weight), _ptr(bias), _ptr(out),
                  _ptr(state), _code(out, "rmsnorm_conv"), _ptr(ctx.seq_slots_dev), n, hidden, taps, _stream(),
                  cost=lambda: ((3.0 + 2 * taps) * n * hidden, n * hidden * (4 + (2 * taps - 1) * out.element_size())))
     return out

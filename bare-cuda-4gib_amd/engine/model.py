@@ -215,7 +215,8 @@ class Model:
                 self.embedding.part.add_to(x, ctx)
             if getattr(e, "reenter", None) is not None:
                 # the stream is replaced; the kernel that writes it norms it for this layer where the layer's norm can
-                first = layer.first_reader(ctx.n_tokens)[0] if hasattr(layer, "first_reader") else None
+                reading = layer.first_reader(ctx.n_tokens) if hasattr(layer, "first_reader") else None
+                first = reading[0] if reading is not None else None
                 made = self.reentry.part.forward(x, ctx, self.embedding.part, e.reenter, first)
                 if made is not None:
                     from ..csrc import ops

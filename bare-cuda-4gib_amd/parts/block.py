@@ -134,6 +134,15 @@ class PreNormBlock(Part):
         return norm.forward(x, ctx)
 
 
+class AddingReader:
+    """Who reads the stream next, where that is a norm with a convolution behind it that can add a sublayer's normed output first (what
+    a SandwichBlock names as its first reader): in a step of single rows the block before leaves its last output to it, (norm, y), and
+    the stream lacks that output until the reader has come."""
+
+    def takes(self, norm, y, ctx) -> bool:
+        return ctx.n_tokens == ctx.n_seqs and getattr(norm, "added_by_the_reader", None) is not None and norm.added_by_the_reader(y) is not None
+
+
 class SandwichBlock(Part):
     """Every sublayer normed on both sides: x += post(mixer(pre(x))); x += post(ffn(pre(x))).  The mixer may read
     h + conv(h) instead of h = pre(x) (``mixer_conv``: a causal convolution over time whose tail is part of the
@@ -145,6 +154,11 @@ class SandwichBlock(Part):
     def __init__(self, mixer, mixer_norm, mixer_post_norm, ffn=None, ffn_norm=None, ffn_post_norm=None, mixer_conv=None):
         self.mixer, self.mixer_norm, self.mixer_post_norm = mixer, mixer_norm, mixer_post_norm
         self.ffn, self.ffn_norm, self.ffn_post_norm, self.mixer_conv = ffn, ffn_norm, ffn_post_norm, mixer_conv
+        self.reader = AddingReader() if hasattr(mixer_conv, "behind") else None
+
+    def first_reader(self, n_rows: int):
+        """What the entry before may leave its last output to (None: this block begins with a norm that nobody prepares)."""
+        return (self.reader, False) if self.reader is not None else None
 
     def children(self):
         parts = [self.mixer_norm, self.mixer_conv, self.mixer, self.mixer_post_norm, self.ffn_norm, self.ffn, self.ffn_post_norm]
@@ -158,9 +172,14 @@ class SandwichBlock(Part):
 
     def forward(self, x, ctx, cache, writes: bool = True) -> None:
         mixer_cache, h = cache, None
+        left = ctx.handoff.take(self.reader) if self.reader is not None else None       # (norm, y) that the stream still lacks
         if self.mixer_conv is not None:
             mixer_cache = cache.mixer
-            if hasattr(self.mixer_conv, "behind"):             # (norm and convolution in one kernel where there is one)
+            if left is not None:                               # (in the same kernel where there is one)
+                h = self.mixer_conv.behind(self.mixer_norm, x, ctx, cache.conv, adds=left[0].added_by_the_reader(left[1]))
+                if h is None:
+                    left[0].add_to(x, left[1])
+            if h is None and hasattr(self.mixer_conv, "behind"):             # (norm and convolution in one kernel where there is one)
                 h = self.mixer_conv.behind(self.mixer_norm, x, ctx, cache.conv)
         if h is None:
             h = self.mixer_norm.forward(x, ctx)
@@ -175,6 +194,8 @@ class SandwichBlock(Part):
         absorbs = self.ffn.absorbs_norm(x.shape[0], self.ffn_norm) if hasattr(self.ffn, "absorbs_norm") else None if lazy else False
         if self.ffn is not None and absorbs is not None and hasattr(self.mixer_post_norm, "add_and_norm"):     # (one kernel where there is one)
             h = self.mixer_post_norm.add_and_norm(x, self._sum_of(y), self.ffn_norm, prepare=absorbs)
+        elif self.ffn is None:
+            self._add_last(self.mixer_post_norm, x, self._sum_of(y), ctx)
         else:
             self.mixer_post_norm.add_to(x, self._sum_of(y))
         if self.ffn is not None:
@@ -184,7 +205,16 @@ class SandwichBlock(Part):
             elif h is None:
                 h = self.ffn_norm.forward(x, ctx)
             self.ffn.forward(h, ctx, y)
-            self.ffn_post_norm.add_to(x, self._sum_of(y))
+            self._add_last(self.ffn_post_norm, x, self._sum_of(y), ctx)
+
+    @staticmethod
+    def _add_last(norm, x, y, ctx) -> None:
+        """x += norm(y), by whoever reads the stream next where that can."""
+        following = getattr(getattr(ctx, "handoff", None), "next_entry", None)
+        if following is not None and isinstance(following[0], AddingReader) and following[0].takes(norm, y, ctx):
+            ctx.handoff.leave(following[0], (norm, y))
+        else:
+            norm.add_to(x, y)
 
     @staticmethod
     def _sum_for(part, x):

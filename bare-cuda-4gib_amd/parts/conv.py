@@ -44,12 +44,13 @@ class CausalConv(Part):
         return ops.causal_conv(v, self.w, view.tail if self.taps > 1 else None, ctx, in_bias=in_bias, out_bias=self.b,
                                add_input=add_input)
 
-    def behind(self, norm, x: torch.Tensor, ctx, view) -> Optional[torch.Tensor]:
-        """h + the convolution of h with h = norm(x), in one kernel where there is one for the step; else None."""
+    def behind(self, norm, x: torch.Tensor, ctx, view, adds=None) -> Optional[torch.Tensor]:
+        """h + the convolution of h with h = norm(x), in one kernel where there is one for the step; else None.  ``adds`` (y, weight,
+        eps): x += y / rms(y) * weight first, in that kernel (None: x is as it was)."""
         scale = norm.fusable() if type(norm) is RMSNorm else None      # (a norm derived from it may do more)
         if scale is None or self.taps == 1:
             return None
-        return ops.rmsnorm_conv(x, scale[0], scale[1], norm.out_dtype, self.w, view.tail, ctx, bias=self.b)
+        return ops.rmsnorm_conv(x, scale[0], scale[1], norm.out_dtype, self.w, view.tail, ctx, bias=self.b, adds=adds)
 
 
 class TokenShift(Part):

@@ -47,6 +47,12 @@ class RMSNorm(Part):
             return None
         return ops.rmsnorm_add(x, y, self._adds_as(), self.eps, next_norm=(*scale, following.out_dtype), prepare=prepare)
 
+    def added_by_the_reader(self, y: torch.Tensor):
+        """(y, weight, eps) of add_to for a kernel that adds before it reads the stream; None for a norm that adds in its own way."""
+        if type(self).add_to is not RMSNorm.add_to or self.groups != 1 or y.dtype != torch.float32:
+            return None
+        return y, self._adds_as(), self.eps
+
     def _adds_as(self) -> torch.Tensor:
         if self.groups != 1:
             raise ConfigError("rmsnorm: a norm in groups is not added to the stream by a kernel of its own")
