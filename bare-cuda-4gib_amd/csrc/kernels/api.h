@@ -345,12 +345,14 @@ int bc4g_rglru_scan(const float* pre, const void* u, const void* y, int dtype, c
 // that reads another one's latents) only the queries are rotated and dkv, g and slot_map may be null; with rot 0 only
 // the cache row is written and q and q_lat may be null (as they may where the queries do not exist yet).  halves 1: element
 // i of the first dims turns with element i + dims / 2 instead.  low [T, low_rank] (null: none; rows low_row apart): a latent
-// of the queries' own, written to low_out [T, low_rank] as rmsnorm(low) * low_g with the same eps.
+// of the queries' own, written to low_out [T, low_rank] as rmsnorm(low) * low_g with the same eps.  absorb (null: none): bfloat16
+// [heads, rank, plain], and every q_lat[t, h, :rank] = absorb[h] q[t, h, :plain] in the same launch, as bc4g_heads_gemm makes it (up to 32
+// bfloat16 rows, heads on 16-byte boundaries).
 int bc4g_latent_angles(const int32_t* positions, float* table, int n_rows, int dims, float base, void* stream);
 int bc4g_latent_prepare(const void* q, const void* dkv, int dtype, const float* g, float eps, const float* angles,
                         const int32_t* slot_map, void* cache, float* q_lat, int n_rows, int heads, int plain, int rot,
                         int rank, int dims, long q_row, long dkv_row, int halves, const void* low, const float* low_g, void* low_out,
-                        int low_rank, long low_row, void* stream);
+                        int low_rank, long low_row, const void* absorb, void* stream);
 // out[t, h, :n] = w[h] a[t, h, :k] for every head: a at a + t * a_row + h * a_head, out likewise, w [heads, n, k].  gate
 // [T, heads] (null: none; rows gate_row apart): head h's outputs are multiplied by sigmoid(gate[t, h]).
 int bc4g_heads_gemm(const void* a, int a_dtype, long a_row, long a_head, const void* w, int w_dtype, void* out, int out_dtype,

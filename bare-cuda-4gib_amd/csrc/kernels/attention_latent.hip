@@ -70,30 +70,44 @@ struct LowQuery {
 };
 
 template <typename T>
-__global__ __launch_bounds__(kPrepBlock) void latent_prepare_kernel(
-    const T* __restrict__ q, const T* __restrict__ dkv, const float* __restrict__ g, float eps,
-    const float* __restrict__ angles, const int32_t* __restrict__ slot_map, T* __restrict__ cache,
-    float* __restrict__ q_lat, int heads, int plain, int rot, int rank, int dims, long q_row, long dkv_row, int parts, int halves,
-    const LowQuery lq) {
+struct PrepareArgs {
+  const T* q;
+  const T* dkv;
+  const float* g;
+  const float* angles;
+  const int32_t* slot_map;
+  T* cache;
+  float* q_lat;
+  int heads, plain, rot, rank, dims, parts, halves;
+  long q_row, dkv_row;
+  float eps;
+  LowQuery lq;
+};
+
+// A row's `part`th part there is work for (a workgroup each): part 0 norms and stores the cache row, part 1 rotates the queries,
+// part 2 norms the queries' latent.  The work is the workgroup's first kPrepBlock threads', all of which it needs at its barriers.
+template <typename T>
+__device__ inline void latent_prepare_row(const PrepareArgs<T>& a, long row, int part, float* cs) {
   __shared__ float scratch[16];
-  extern __shared__ float cs[];                     // [dims / 2][2]: the row's cosines and sines
-  const long row = blockIdx.x;
-  for (int i = threadIdx.x; i < dims; i += kPrepBlock) cs[i] = angles[row * dims + i];
-  // (a workgroup a row for each part there is work for: part 0 norms and stores the cache row, part 1 rotates the queries,
-  // part 2 norms the queries' latent; blockIdx.y counts the parts that are there)
+  const int heads = a.heads, plain = a.plain, rot = a.rot, rank = a.rank, dims = a.dims, halves = a.halves;
+  const int tid = threadIdx.x;
+  const bool works = tid < kPrepBlock;
+  for (int i = works ? tid : dims; i < dims; i += kPrepBlock) cs[i] = a.angles[row * dims + i];
   int part_no = 0;
-  for (int left = blockIdx.y;; ++part_no)
-    if ((parts >> part_no & 1) && left-- == 0) break;
+  for (int left = part;; ++part_no)
+    if ((a.parts >> part_no & 1) && left-- == 0) break;
   if (part_no == 2) {
+    const LowQuery& lq = a.lq;
     const T* lo = static_cast<const T*>(lq.low) + row * lq.row;
     T* to = static_cast<T*>(lq.out) + row * lq.rank;
+    const int first = works ? tid : lq.rank;
     float sum = 0.f;
-    for (int i = threadIdx.x; i < lq.rank; i += kPrepBlock) {
+    for (int i = first; i < lq.rank; i += kPrepBlock) {
       const float v = to_float(lo[i]);
       sum += v * v;
     }
-    const float by = 1.0f / sqrtf(block_sum(sum, scratch) / static_cast<float>(lq.rank) + eps);
-    for (int i = threadIdx.x; i < lq.rank; i += kPrepBlock) to[i] = from_float<T>(to_float(lo[i]) * by * lq.g[i]);
+    const float by = 1.0f / sqrtf(block_sum(sum, scratch) / static_cast<float>(lq.rank) + a.eps);
+    for (int i = first; i < lq.rank; i += kPrepBlock) to[i] = from_float<T>(to_float(lo[i]) * by * lq.g[i]);
     return;
   }
   auto turned = [&](int i, float v, float other) {
@@ -107,9 +121,10 @@ __global__ __launch_bounds__(kPrepBlock) void latent_prepare_kernel(
   // 16 heads of 64, rank 512, 6.0 -> 4.8 us.
   constexpr int kAhead = 8;
   if (part_no == 1) {
-    const T* qr = q + row * q_row;
-    float* ql = q_lat + row * heads * (rank + rot);
-    for (int e0 = threadIdx.x; e0 < heads * rot || e0 == threadIdx.x; e0 += kAhead * kPrepBlock) {
+    const T* qr = a.q + row * a.q_row;
+    float* ql = a.q_lat + row * heads * (rank + rot);
+    const int first = works ? tid : heads * rot;
+    for (int e0 = first; e0 < heads * rot || e0 == first; e0 += kAhead * kPrepBlock) {
       float own[kAhead], other[kAhead];
 #pragma unroll
       for (int j = 0; j < kAhead; ++j) {
@@ -118,7 +133,7 @@ __global__ __launch_bounds__(kPrepBlock) void latent_prepare_kernel(
         own[j] = to_float(part[i]);
         other[j] = to_float(part[i < dims ? pair_of(i, dims, halves).other : i]);
       }
-      if (e0 == threadIdx.x) __syncthreads();                  // (every thread's first turn)
+      if (e0 == first) __syncthreads();                        // (every thread's first turn)
 #pragma unroll
       for (int j = 0; j < kAhead; ++j) {
         const int e = e0 + j * kPrepBlock;
@@ -127,36 +142,44 @@ __global__ __launch_bounds__(kPrepBlock) void latent_prepare_kernel(
     }
     return;
   }
-  const T* lat = dkv + row * dkv_row;
-  T* to = cache + static_cast<long>(slot_map[row]) * (rank + rot);
+  const T* lat = a.dkv + row * a.dkv_row;
+  const float* g = a.g;
+  T* to = a.cache + static_cast<long>(a.slot_map[row]) * (rank + rot);
   float held[kAhead], gain[kAhead];                            // (a latent's first 1,024 numbers)
 #pragma unroll
   for (int j = 0; j < kAhead; ++j) {
-    const int i = threadIdx.x + j * kPrepBlock < rank ? threadIdx.x + j * kPrepBlock : 0;
+    const int i = tid + j * kPrepBlock < rank ? tid + j * kPrepBlock : 0;
     held[j] = to_float(lat[i]);
     gain[j] = g[i];
   }
-  const int ri = static_cast<int>(threadIdx.x) < rot ? threadIdx.x : 0;      // the rotated part's first 128
+  const int ri = tid < rot ? tid : 0;                          // the rotated part's first 128
   float own = 0.f, other = 0.f;
   if (rot > 0) own = to_float(lat[rank + ri]), other = to_float(lat[rank + (ri < dims ? pair_of(ri, dims, halves).other : ri)]);
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < kAhead; ++j)
-    if (static_cast<int>(threadIdx.x) + j * kPrepBlock < rank) ss = fmaf(held[j], held[j], ss);
-  for (int i = threadIdx.x + kAhead * kPrepBlock; i < rank; i += kPrepBlock) {
+    if (works && tid + j * kPrepBlock < rank) ss = fmaf(held[j], held[j], ss);
+  for (int i = works ? tid + kAhead * kPrepBlock : rank; i < rank; i += kPrepBlock) {
     const float v = to_float(lat[i]);
     ss = fmaf(v, v, ss);
   }
-  const float scale = 1.0f / sqrtf(block_sum(ss, scratch) / static_cast<float>(rank) + eps);   // (a barrier: cs is written)
+  const float scale = 1.0f / sqrtf(block_sum(ss, scratch) / static_cast<float>(rank) + a.eps);   // (a barrier: cs is written)
+  if (!works) return;
 #pragma unroll
   for (int j = 0; j < kAhead; ++j) {
-    const int i = threadIdx.x + j * kPrepBlock;
+    const int i = tid + j * kPrepBlock;
     if (i < rank) to[i] = from_float<T>(held[j] * scale * gain[j]);
   }
-  for (int i = threadIdx.x + kAhead * kPrepBlock; i < rank; i += kPrepBlock) to[i] = from_float<T>(to_float(lat[i]) * scale * g[i]);
-  if (static_cast<int>(threadIdx.x) < rot) to[rank + threadIdx.x] = from_float<T>(turned(threadIdx.x, own, other));
-  for (int i = threadIdx.x + kPrepBlock; i < rot; i += kPrepBlock)
+  for (int i = tid + kAhead * kPrepBlock; i < rank; i += kPrepBlock) to[i] = from_float<T>(to_float(lat[i]) * scale * g[i]);
+  if (tid < rot) to[rank + tid] = from_float<T>(turned(tid, own, other));
+  for (int i = tid + kPrepBlock; i < rot; i += kPrepBlock)
     to[rank + i] = from_float<T>(turned(i, to_float(lat[rank + i]), to_float(lat[rank + (i < dims ? pair_of(i, dims, halves).other : i)])));
+}
+
+template <typename T>
+__global__ __launch_bounds__(kPrepBlock) void latent_prepare_kernel(const PrepareArgs<T> a) {
+  extern __shared__ float cs[];                     // [dims / 2][2]: the row's cosines and sines
+  latent_prepare_row(a, blockIdx.x, blockIdx.y, cs);
 }
 
 // A product's head gate: a number a row and head, of which the sigmoid multiplies the head's outputs (none: 1).
@@ -230,11 +253,9 @@ __device__ inline uint4 load_slots(const float* p) {
 // KW waves of a workgroup take every KW-th k-step and add their sums up through LDS (few rows: more waves on the
 // weights' way in).
 template <typename TA, typename TO, int NB, int KW>
-__global__ __launch_bounds__(kWave * KW) void heads_mfma_kernel(const TA* __restrict__ a, long a_row, long a_head,
-                                                                const bf16_t* __restrict__ w, TO* __restrict__ out, long o_row,
-                                                                long o_head, int m, int n, int k, const HeadGate gate) {
+__device__ inline void heads_mfma_tile(const TA* __restrict__ a, long a_row, long a_head, const bf16_t* __restrict__ w, TO* __restrict__ out, long o_row,
+                                       long o_head, int m, int n, int k, const HeadGate& gate, int h, int m0, int n0) {
   __shared__ floatx4 sums[KW > 1 ? KW : 1][NB][kWave];
-  const int h = blockIdx.z, m0 = blockIdx.x * 16, n0 = blockIdx.y * 16 * NB;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int c = lane % 16, g = lane / 16;
   // (rows and columns beyond the product: the last, their sums are not stored; k beyond it: zeros)
@@ -292,6 +313,30 @@ __global__ __launch_bounds__(kWave * KW) void heads_mfma_kernel(const TA* __rest
       const int r = m0 + 4 * g + i;
       if (r < m) out[r * o_row + h * o_head + n0 + nb * 16 + c] = from_float<TO>(acc[nb][i] * by[i]);
     }
+  }
+}
+
+template <typename TA, typename TO, int NB, int KW>
+__global__ __launch_bounds__(kWave * KW) void heads_mfma_kernel(const TA* __restrict__ a, long a_row, long a_head,
+                                                                const bf16_t* __restrict__ w, TO* __restrict__ out, long o_row,
+                                                                long o_head, int m, int n, int k, const HeadGate gate) {
+  heads_mfma_tile<TA, TO, NB, KW>(a, a_row, a_head, w, out, o_row, o_head, m, n, k, gate, blockIdx.z, blockIdx.x * 16, blockIdx.y * 16 * NB);
+}
+
+// Few rows: the cache rows and the rotated queries in the launch of the absorbed queries' other part, w[h] q[t, h, :plain], which needs neither
+// (a decode step is a chain of launches that wait: 8 rows, 16 heads of 128 + 64, rank 512, 4.8 and 4.7 us one after the other).  The first
+// n_tiles * heads workgroups are the product's, the others a row's parts each.
+constexpr int kFewRows = 32;         // (up to which bc4g_heads_gemm takes this form of the product: the same bits)
+__global__ __launch_bounds__(4 * kWave) void latent_prepare_heads_kernel(const PrepareArgs<bf16_t> a, const bf16_t* __restrict__ w, int m, int m_tiles,
+                                                                         int n_tiles) {
+  extern __shared__ float cs[];
+  const int products = m_tiles * n_tiles * a.heads, block = blockIdx.x;
+  if (block < products) {
+    const int h = block / (m_tiles * n_tiles), tile = block % (m_tiles * n_tiles), row = a.rank + a.rot;
+    heads_mfma_tile<bf16_t, float, 1, 4>(a.q, a.q_row, a.plain + a.rot, w, a.q_lat, static_cast<long>(a.heads) * row, row, m, a.rank, a.plain, HeadGate{}, h,
+                                         tile % m_tiles * 16, tile / m_tiles * 16);
+  } else {
+    latent_prepare_row(a, (block - products) % m, (block - products) / m, cs);
   }
 }
 
@@ -411,7 +456,7 @@ extern "C" int bc4g_latent_prepare(const void* q, const void* dkv, int dtype, co
                                    const float* angles, const int32_t* slot_map, void* cache, float* q_lat,
                                    int n_rows, int heads, int plain, int rot, int rank, int dims, long q_row, long dkv_row,
                                    int halves, const void* low, const float* low_g, void* low_out, int low_rank, long low_row,
-                                   void* stream) {
+                                   const void* absorb, void* stream) {
   BC4G_REQUIRE(n_rows >= 0 && heads > 0 && plain >= 0 && rot >= 0 && rank > 0, "latent_prepare: bad sizes T=%d heads=%d "
                "plain=%d rot=%d rank=%d", n_rows, heads, plain, rot, rank);
   BC4G_REQUIRE(dims >= 0 && dims % 2 == 0 && dims <= rot && dims <= 8192,
@@ -428,15 +473,28 @@ extern "C" int bc4g_latent_prepare(const void* q, const void* dkv, int dtype, co
   const LowQuery lq{low, low_g, low_out, low_row, low_rank};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const size_t lds = static_cast<size_t>(dims > 0 ? dims : 2) * sizeof(float);
-  if (dtype == kF32)
-    latent_prepare_kernel<float><<<dim3(n_rows, n_parts), kPrepBlock, lds, s>>>(static_cast<const float*>(q), static_cast<const float*>(dkv), g,
-                                                                 eps, angles, slot_map, static_cast<float*>(cache), q_lat,
-                                                                 heads, plain, rot, rank, dims, q_row, dkv_row, parts, halves, lq);
-  else if (dtype == kBF16)
-    latent_prepare_kernel<bf16_t><<<dim3(n_rows, n_parts), kPrepBlock, lds, s>>>(static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(dkv),
-                                                                  g, eps, angles, slot_map, static_cast<bf16_t*>(cache),
-                                                                  q_lat, heads, plain, rot, rank, dims, q_row, dkv_row, parts, halves, lq);
-  else return fail("latent_prepare: unknown dtype %d", dtype);
+  if (absorb)
+    BC4G_REQUIRE(q && dtype == kBF16 && n_rows <= kFewRows && plain > 0 && plain % 8 == 0 && (plain + rot) % 8 == 0 && q_row % 8 == 0 &&
+                     reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(absorb) % 16 == 0,
+                 "latent_prepare: the absorbed queries' product takes up to %d bfloat16 rows whose heads lie on 16-byte boundaries", kFewRows);
+  if (dtype == kF32) {
+    latent_prepare_kernel<float><<<dim3(n_rows, n_parts), kPrepBlock, lds, s>>>(
+        PrepareArgs<float>{static_cast<const float*>(q), static_cast<const float*>(dkv), g, angles, slot_map, static_cast<float*>(cache), q_lat,
+                           heads, plain, rot, rank, dims, parts, halves, q_row, dkv_row, eps, lq});
+  } else if (dtype == kBF16) {
+    const PrepareArgs<bf16_t> a{static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(dkv), g, angles, slot_map, static_cast<bf16_t*>(cache), q_lat,
+                                heads, plain, rot, rank, dims, parts, halves, q_row, dkv_row, eps, lq};
+    if (absorb) {
+      const int m_tiles = ceil_div(n_rows, 16), n_tiles = ceil_div(rank, 16);
+      const long blocks = static_cast<long>(m_tiles) * n_tiles * heads + static_cast<long>(n_rows) * n_parts;
+      BC4G_REQUIRE(blocks <= 2147483647L, "latent_prepare: %d heads of rank %d are beyond the grid limit", heads, rank);
+      latent_prepare_heads_kernel<<<static_cast<unsigned>(blocks), 4 * kWave, lds, s>>>(a, static_cast<const bf16_t*>(absorb), n_rows, m_tiles, n_tiles);
+    } else {
+      latent_prepare_kernel<bf16_t><<<dim3(n_rows, n_parts), kPrepBlock, lds, s>>>(a);
+    }
+  } else {
+    return fail("latent_prepare: unknown dtype %d", dtype);
+  }
   return check_launch("latent_prepare");
 }
 
@@ -455,7 +513,7 @@ extern "C" int bc4g_heads_gemm(const void* a, int a_dtype, long a_row, long a_he
   if (w_dtype == kBF16 && k % 8 == 0 && a_row % 8 == 0 && a_head % 8 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(w) % 16 == 0 && (a_bytes == 2 || a_dtype == kF32) && (out_dtype == kF32 || out_dtype == kBF16)) {
     // few rows (a decode step): a wave takes one block of 16 columns, so that more waves share the weights' way in
-    const int nb = m <= 32 ? 1 : 4;
+    const int nb = m <= kFewRows ? 1 : 4;
     dim3 mgrid(ceil_div(m, 16), ceil_div(n, 16 * nb), heads);
     BC4G_REQUIRE(mgrid.y <= 65535, "heads_gemm: n=%d is beyond the grid limit", n);
     const bf16_t* wp = static_cast<const bf16_t*>(w);

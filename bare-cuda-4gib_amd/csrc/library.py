@@ -64,7 +64,7 @@ _SIGNATURES = {
     "bc4g_causal_conv": [_P, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, c_long, _P],
     "bc4g_rglru_scan": [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, c_long, _P],
     "bc4g_latent_angles": [_P, _P, _I, _I, _F, _P],
-    "bc4g_latent_prepare": [_P, _P, _I, _P, _F, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, c_long, c_long, _I, _P, _P, _P, _I, c_long, _P],
+    "bc4g_latent_prepare": [_P, _P, _I, _P, _F, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, c_long, c_long, _I, _P, _P, _P, _I, c_long, _P, _P],
     "bc4g_heads_gemm": [_P, _I, c_long, c_long, _P, _I, _P, _I, c_long, c_long, _I, _I, _I, _I, _P, _I, c_long, _P],
     "bc4g_attention_latent": [_P, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P],
     "bc4g_clamped_glu": [_P, _P, _I, _F, _F, _I, _I, _P],

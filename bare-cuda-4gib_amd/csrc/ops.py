@@ -1769,18 +1769,27 @@ def latent_angles(positions: torch.Tensor, dims: int, base: float) -> torch.Tens
     return table
 
 
+LATENT_FEW_ROWS = 32                # rows up to which the cache rows are made in the launch of the absorbed queries
+
+
 def latent_prepare(q: Optional[torch.Tensor], dkv: Optional[torch.Tensor], g: Optional[torch.Tensor], eps: float, angles: Optional[torch.Tensor],
                    slot_map: Optional[torch.Tensor], cache: Optional[torch.Tensor], q_lat: Optional[torch.Tensor], heads: int, plain: int,
                    rot: int, rank: int, dims: int, *, halves: bool = False, low: Optional[torch.Tensor] = None,
-                   low_g: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                   low_g: Optional[torch.Tensor] = None, absorb: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """Writes [rmsnorm(dkv[:, :rank]) * g | rotate(dkv[:, rank:])] into every row's cache slot (``cache`` None: nowhere)
     and every head's rotated query part into q_lat[:, h, rank:].  ``angles``: latent_angles of the rows (None where
     nothing is rotated, dims 0).  Without a cache dkv and g may be None: only the queries are rotated.  ``halves``: element
     i of the first dims turns with element i + dims / 2 (else neighbours turn together).  ``low`` [T, low_rank]: the queries'
-    own latent; returns rmsnorm(low) * low_g (the same eps), from which they are made -- q and q_lat are None then."""
-    _dev("latent_prepare", g, angles, slot_map, cache, q_lat, low_g)
+    own latent; returns rmsnorm(low) * low_g (the same eps), from which they are made -- q and q_lat are None then.  ``absorb``
+    [heads, rank, plain]: the queries' other part too, q_lat[:, h, :rank] = absorb[h] q[:, h, :plain] (heads_gemm), in the same launch
+    for few rows."""
+    _dev("latent_prepare", g, angles, slot_map, cache, q_lat, low_g, absorb)
+    if absorb is not None and (q is None or tuple(absorb.shape) != (heads, rank, plain)):
+        raise KernelError(f"latent_prepare: absorb {tuple(absorb.shape)} is not [{heads}, {rank}, {plain}], or there are no queries")
     if cache is None and (rot == 0 or q is None) and low is None:
-        return None             # nothing to write
+        if absorb is not None:
+            heads_gemm(q.unflatten(1, (heads, plain + rot)), absorb, q_lat, k=plain, n=rank)
+        return None             # nothing else to write
     some = next(x for x in (q, dkv, low) if x is not None)
     t = some.shape[0]
     # (q, dkv and low may be parts of one product's rows)
@@ -1805,10 +1814,16 @@ def latent_prepare(q: Optional[torch.Tensor], dkv: Optional[torch.Tensor], g: Op
         _i32("latent_prepare", "slot_map", slot_map, t)
     turned = (heads if q is not None else 0) + (1 if cache is not None else 0)
     normed = (rank if cache is not None else 0) + low_rank
+    together = (absorb is not None and t <= LATENT_FEW_ROWS and q.dtype == torch.bfloat16 and absorb.dtype == torch.bfloat16 and plain % 8 == 0
+                and (plain + rot) % 8 == 0 and q_row % 8 == 0 and q.data_ptr() % 16 == 0 and absorb.data_ptr() % 16 == 0)
     library.call("bc4g_latent_prepare", _ptr(q), _ptr(dkv), _code(some, "latent_prepare"), _ptr(g), float(eps),
                  _ptr(angles) if dims else None, _ptr(slot_map) if cache is not None else None, _ptr(cache), _ptr(q_lat), t, heads,
                  plain, rot, rank, int(dims), q_row, dkv_row, 1 if halves else 0, _ptr(low), _ptr(low_g), _ptr(low_out), low_rank, low_row,
-                 _stream(), cost=lambda: (4.0 * t * (normed + turned * rot), t * some.element_size() * ((turned + 1) * rot + 2 * normed)))
+                 _ptr(absorb) if together else None, _stream(),
+                 cost=lambda: (4.0 * t * (normed + turned * rot) + (2.0 * t * heads * rank * plain if together else 0.0),
+                               t * some.element_size() * ((turned + 1) * rot + 2 * normed) + (heads * rank * (2 * plain + 4 * t) if together else 0)))
+    if absorb is not None and not together:
+        heads_gemm(q.unflatten(1, (heads, plain + rot)), absorb, q_lat, k=plain, n=rank)
     return low_out
 
 

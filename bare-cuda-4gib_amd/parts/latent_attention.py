@@ -121,8 +121,7 @@ class LatentAttention(Part):
         if self.q_rank:           # both latents are normed by one kernel, then the queries are made and turned
             low = ops.latent_prepare(None, dkv, self.g, self.eps, angles, where, to, None, *sizes, halves=self.halves, low=q, low_g=self.gq)
             q, dkv, to = linear(low, self.w_uq, out_dtype=self.act_dtype), None, None
-        ops.latent_prepare(q, dkv, self.g, self.eps, angles, where, to, q_lat, *sizes, halves=self.halves)
-        ops.heads_gemm(q.unflatten(1, (H, self.dim + rot)), self.uk_t, q_lat, k=self.dim, n=rank)
+        ops.latent_prepare(q, dkv, self.g, self.eps, angles, where, to, q_lat, *sizes, halves=self.halves, absorb=self.uk_t)
         mixed = ops.attention_latent(q_lat, cache.latent, self.sinks, ctx.block_tables[cache.group], ctx, H, rank, rot,
                                      cache.page_tokens, self.window, self.scale)
         o = torch.empty((t, H, self.vdim), dtype=self.act_dtype, device=q.device)

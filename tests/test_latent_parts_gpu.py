@@ -78,3 +78,26 @@ def test_cache_rows_of_any_size(ops, rank, rot, dims, heads, halves):
     if rot:
         want = turned(q.view(t, heads, plain + rot)[..., plain:])
         assert (on[5].cpu()[..., rank:].double() - want).abs().max() < bound
+
+
+@pytest.mark.parametrize("t", [1, 8, 17, 32, 33])
+@pytest.mark.parametrize("rank,rot,plain,heads", [(512, 64, 128, 16), (80, 24, 40, 3), (64, 0, 32, 2), (100, 8, 8, 1), (64, 6, 16, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_absorbed_queries_beside_the_cache_rows(ops, t, rank, rot, plain, heads, dtype):
+    """The two launches' bits, whether one takes their place or not (33 rows, float32, heads off 16 bytes: not), with queries and latent as
+    parts of one product's rows."""
+    gen = torch.Generator().manual_seed(t)
+    n_q = heads * (plain + rot)
+    qd = torch.randn(t, n_q + rank + rot, generator=gen).to(dtype).to(DEV)
+    g, w = torch.randn(rank, generator=gen).to(DEV), torch.randn(heads, rank, plain, generator=gen).to(dtype).to(DEV)
+    angles = torch.randn(t, max(rot // 2, 1), 2, generator=gen).to(DEV)
+    slots = _i32(list(range(t))[::-1])
+    q, dkv = qd[:, :n_q], qd[:, n_q:]
+    out = []
+    for together in (False, True):
+        cache, q_lat = torch.zeros(1, t, rank + rot, dtype=dtype, device=DEV), torch.zeros(t, heads, rank + rot, device=DEV)
+        ops.latent_prepare(q, dkv, g, 1e-5, angles if rot else None, slots, cache, q_lat, heads, plain, rot, rank, rot, absorb=w if together else None)
+        if not together:
+            ops.heads_gemm(q.unflatten(1, (heads, plain + rot)), w, q_lat, k=plain, n=rank)
+        out.append((cache, q_lat))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
