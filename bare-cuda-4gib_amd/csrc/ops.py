@@ -775,6 +775,13 @@ class LinearPlan:
     def fuses_norm(self, m: int) -> bool:
         return 0 < m <= self.fused_norm_rows
 
+    def norms_apart(self, m: int) -> bool:
+        """Whether the norm before a product that could absorb it is better a kernel of its own.  Every workgroup of 16 outputs stages all
+        the rows again: from five rows on an output of 16,384 and more pays more for that than for a launch (with the norm inside and apart, 8
+        rows: 32,000 x 2,048 31.9 and 25.9 + 2.4 us, 128,256 x 4,096 217 and 182 + 3; five rows 29.3 and 25.7 + 2.4, 202 and 178 + 3; four rows 27.7
+        and 25.8 + 2.4, 180 and 176 + 3; 8 rows 11,264 x 2,048 14.2 and 11.5 + 2.4)."""
+        return m >= 5 and self.n >= 16384
+
     def parts(self, m: int) -> int:
         """Into how many parts an adding product of m rows cuts k over workgroups (1: it does not)."""
         lo, hi = self.parts_rows
@@ -963,6 +970,11 @@ def absorbs_norm(n_rows: int, g: torch.Tensor, w) -> bool:
     """gemm_normed_supported for a stream of the weight's width that is not at hand yet."""
     w, _ = _weight(w)
     return w.dtype == torch.bfloat16 and _normed_rows_fit(n_rows, w.shape[1], w.shape[0]) and w.shape[1] % 8 == 0 and g.dtype in _CODE
+
+
+def norm_apart(n_rows: int, w) -> bool:
+    """Whether a norm that the product could absorb is better run before it (LinearPlan.norms_apart)."""
+    return plan_for(w.shape[0], w.shape[1]).norms_apart(n_rows)
 
 
 def gemm_normed(x: torch.Tensor, rows: Optional[torch.Tensor], n_rows: int, g: torch.Tensor, eps: float,

@@ -20,7 +20,7 @@ def _fused_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
     if x._tensor is not None:
         return None
     scale = x.fusable_scale()
-    if scale is None or not ops.gemm_normed_supported(x.x, x.n_rows, scale[0], w):
+    if scale is None or not ops.gemm_normed_supported(x.x, x.n_rows, scale[0], w) or ops.norm_apart(x.n_rows, w):
         return None
     return ops.gemm_normed(x.x, x.rows, x.n_rows, scale[0], scale[1], w, epilogue)
 
@@ -28,7 +28,7 @@ def _fused_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
 def absorbs_norm(norm, w, n_rows: int) -> bool:
     """Whether a product of n_rows rows of the stream with this weight absorbs the norm before it (_fused_norm)."""
     scale = norm.fusable() if hasattr(norm, "fusable") else None
-    return scale is not None and ops.absorbs_norm(n_rows, scale[0], w)
+    return scale is not None and ops.absorbs_norm(n_rows, scale[0], w) and not ops.norm_apart(n_rows, w)
 
 
 def _prepared_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
