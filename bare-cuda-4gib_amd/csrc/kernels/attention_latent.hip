@@ -250,16 +250,19 @@ __device__ inline uint4 load_slots(const float* p) {
   return make_uint4(two(a.x, a.y), two(a.z, a.w), two(b.x, b.y), two(b.z, b.w));
 }
 
-// KW waves of a workgroup take every KW-th k-step and add their sums up through LDS (few rows: more waves on the
-// weights' way in).
-template <typename TA, typename TO, int NB, int KW>
+// MB blocks of 16 rows a wave.  KW waves of a workgroup take every KW-th k-step and add their sums up through LDS (few rows: more waves on the
+// weights' way in); with KW 1 a workgroup is one wave.
+template <typename TA, typename TO, int NB, int KW, int MB>
 __device__ inline void heads_mfma_tile(const TA* __restrict__ a, long a_row, long a_head, const bf16_t* __restrict__ w, TO* __restrict__ out, long o_row,
                                        long o_head, int m, int n, int k, const HeadGate& gate, int h, int m0, int n0) {
+  static_assert(KW == 1 || MB == 1, "the waves' sums meet a block of rows at a time");
   __shared__ floatx4 sums[KW > 1 ? KW : 1][NB][kWave];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int c = lane % 16, g = lane / 16;
   // (rows and columns beyond the product: the last, their sums are not stored; k beyond it: zeros)
-  const TA* arow = a + min(m0 + c, m - 1) * a_row + h * a_head;
+  const TA* arow[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) arow[mb] = a + min(m0 + mb * 16 + c, m - 1) * a_row + h * a_head;
   const bf16_t* wcol[NB];
   bool col_there[NB];
 #pragma unroll
@@ -267,18 +270,21 @@ __device__ inline void heads_mfma_tile(const TA* __restrict__ a, long a_row, lon
     col_there[nb] = n0 + nb * 16 + c < n;
     wcol[nb] = w + (static_cast<long>(h) * n + min(n0 + nb * 16 + c, n - 1)) * k;
   }
-  floatx4 acc[NB];
+  floatx4 acc[MB][NB];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // Four of the wave's k-steps asked for together, without a condition: with one in each load's way a wave waited for every step's loads
-  // before it asked for the next one's (8 rows of 16 heads, k 512: 7.0 -> 5.8 us).
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // Four of the wave's k-steps asked for together (two with many rows), without a condition: with one in each load's way a wave waited for every
+  // step's loads before it asked for the next one's (8 rows of 16 heads, k 512: 7.0 -> 5.8 us).
   constexpr int kAhead = KW > 1 ? 4 : 2;
   for (int k0 = 32 * wave; k0 < k; k0 += 32 * KW * kAhead) {
-    uint4 av[kAhead], wv[kAhead][NB];
+    uint4 av[kAhead][MB], wv[kAhead][NB];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int at = k0 + 32 * KW * i + 8 * g, from = at < k ? at : 0;
-      av[i] = load_slots(arow + from);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) av[i][mb] = load_slots(arow[mb] + from);
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) wv[i][nb] = load16(wcol[nb] + from);
     }
@@ -286,41 +292,46 @@ __device__ inline void heads_mfma_tile(const TA* __restrict__ a, long a_row, lon
     for (int i = 0; i < kAhead; ++i) {
       if (k0 + 32 * KW * i >= k) break;
       const bool k_there = k0 + 32 * KW * i + 8 * g < k;
-      const uint4 ai = k_there ? av[i] : zero16();
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_16x16x32(ai, k_there ? wv[i][nb] : zero16(), acc[nb]);
+      for (int nb = 0; nb < NB; ++nb) {
+        const uint4 wi = k_there ? wv[i][nb] : zero16();
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[mb][nb] = mfma_16x16x32(k_there ? av[i][mb] : zero16(), wi, acc[mb][nb]);
+      }
     }
   }
   if (KW > 1) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) sums[wave][nb][lane] = acc[nb];
+    for (int nb = 0; nb < NB; ++nb) sums[wave][nb][lane] = acc[0][nb];
     __syncthreads();
     if (wave > 0) return;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int other = 1; other < KW; ++other) acc[nb] += sums[other][nb][lane];
+      for (int other = 1; other < KW; ++other) acc[0][nb] += sums[other][nb][lane];
   }
   // a lane holds column c of every block and rows 4g .. 4g + 3
-  float by[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) by[i] = m0 + 4 * g + i < m ? gate.of(m0 + 4 * g + i, h) : 1.0f;
+  for (int mb = 0; mb < MB; ++mb) {
+    const int r0 = m0 + mb * 16 + 4 * g;
+    float by[4];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    if (!col_there[nb]) continue;
+    for (int i = 0; i < 4; ++i) by[i] = r0 + i < m ? gate.of(r0 + i, h) : 1.0f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = m0 + 4 * g + i;
-      if (r < m) out[r * o_row + h * o_head + n0 + nb * 16 + c] = from_float<TO>(acc[nb][i] * by[i]);
+    for (int nb = 0; nb < NB; ++nb) {
+      if (!col_there[nb]) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (r0 + i < m) out[(r0 + i) * o_row + h * o_head + n0 + nb * 16 + c] = from_float<TO>(acc[mb][nb][i] * by[i]);
     }
   }
 }
 
-template <typename TA, typename TO, int NB, int KW>
+template <typename TA, typename TO, int NB, int KW, int MB>
 __global__ __launch_bounds__(kWave * KW) void heads_mfma_kernel(const TA* __restrict__ a, long a_row, long a_head,
                                                                 const bf16_t* __restrict__ w, TO* __restrict__ out, long o_row,
                                                                 long o_head, int m, int n, int k, const HeadGate gate) {
-  heads_mfma_tile<TA, TO, NB, KW>(a, a_row, a_head, w, out, o_row, o_head, m, n, k, gate, blockIdx.z, blockIdx.x * 16, blockIdx.y * 16 * NB);
+  heads_mfma_tile<TA, TO, NB, KW, MB>(a, a_row, a_head, w, out, o_row, o_head, m, n, k, gate, blockIdx.z, blockIdx.x * 16 * MB, blockIdx.y * 16 * NB);
 }
 
 // Few rows: the cache rows and the rotated queries in the launch of the absorbed queries' other part, w[h] q[t, h, :plain], which needs neither
@@ -333,7 +344,7 @@ __global__ __launch_bounds__(4 * kWave) void latent_prepare_heads_kernel(const P
   const int products = m_tiles * n_tiles * a.heads, block = blockIdx.x;
   if (block < products) {
     const int h = block / (m_tiles * n_tiles), tile = block % (m_tiles * n_tiles), row = a.rank + a.rot;
-    heads_mfma_tile<bf16_t, float, 1, 4>(a.q, a.q_row, a.plain + a.rot, w, a.q_lat, static_cast<long>(a.heads) * row, row, m, a.rank, a.plain, HeadGate{}, h,
+    heads_mfma_tile<bf16_t, float, 1, 4, 1>(a.q, a.q_row, a.plain + a.rot, w, a.q_lat, static_cast<long>(a.heads) * row, row, m, a.rank, a.plain, HeadGate{}, h,
                                          tile % m_tiles * 16, tile / m_tiles * 16);
   } else {
     latent_prepare_row(a, (block - products) % m, (block - products) / m, cs);
@@ -514,17 +525,24 @@ extern "C" int bc4g_heads_gemm(const void* a, int a_dtype, long a_row, long a_he
       reinterpret_cast<uintptr_t>(w) % 16 == 0 && (a_bytes == 2 || a_dtype == kF32) && (out_dtype == kF32 || out_dtype == kBF16)) {
     // few rows (a decode step): a wave takes one block of 16 columns, so that more waves share the weights' way in
     const int nb = m <= kFewRows ? 1 : 4;
-    dim3 mgrid(ceil_div(m, 16), ceil_div(n, 16 * nb), heads);
+    // Many: every wave reads its columns' weights, so from 4,096 waves on (sixteen a CU) it takes two blocks of rows.  16 heads of k 128 and n 512,
+    // 3,557 rows 70 -> 48 us, 700 rows 19.7 -> 15.8; k 512 and n 128 79 -> 70, but 700 rows (1,400 waves) 20.9 -> 28.0; ten of 256 and 256, 3,557 rows
+    // 45 -> 34.  Four blocks: 44, 97 and 32 for the three of 3,557 rows.
+    const int mb = nb > 1 && static_cast<long>(ceil_div(m, 16)) * ceil_div(n, 64) * heads >= 4096 ? 2 : 1;
+    dim3 mgrid(ceil_div(m, 16 * mb), ceil_div(n, 16 * nb), heads);
     BC4G_REQUIRE(mgrid.y <= 65535, "heads_gemm: n=%d is beyond the grid limit", n);
     const bf16_t* wp = static_cast<const bf16_t*>(w);
 #define BC4G_HM(TA, TO)                                                                                                        \
   do {                                                                                                                         \
     if (nb == 1)                                                                                                               \
-      heads_mfma_kernel<TA, TO, 1, 4><<<mgrid, 4 * kWave, 0, s>>>(static_cast<const TA*>(a), a_row, a_head, wp,                \
-                                                                  static_cast<TO*>(out), o_row, o_head, m, n, k, hg);          \
+      heads_mfma_kernel<TA, TO, 1, 4, 1><<<mgrid, 4 * kWave, 0, s>>>(static_cast<const TA*>(a), a_row, a_head, wp,             \
+                                                                     static_cast<TO*>(out), o_row, o_head, m, n, k, hg);       \
+    else if (mb == 1)                                                                                                          \
+      heads_mfma_kernel<TA, TO, 4, 1, 1><<<mgrid, kWave, 0, s>>>(static_cast<const TA*>(a), a_row, a_head, wp,                 \
+                                                                 static_cast<TO*>(out), o_row, o_head, m, n, k, hg);           \
     else                                                                                                                       \
-      heads_mfma_kernel<TA, TO, 4, 1><<<mgrid, kWave, 0, s>>>(static_cast<const TA*>(a), a_row, a_head, wp,                    \
-                                                              static_cast<TO*>(out), o_row, o_head, m, n, k, hg);              \
+      heads_mfma_kernel<TA, TO, 4, 1, 2><<<mgrid, kWave, 0, s>>>(static_cast<const TA*>(a), a_row, a_head, wp,                 \
+                                                                 static_cast<TO*>(out), o_row, o_head, m, n, k, hg);           \
   } while (0)
     if (a_dtype == kBF16 && out_dtype == kF32) BC4G_HM(bf16_t, float);
     else if (a_dtype == kBF16) BC4G_HM(bf16_t, bf16_t);

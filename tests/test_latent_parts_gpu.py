@@ -101,3 +101,16 @@ def test_absorbed_queries_beside_the_cache_rows(ops, t, rank, rot, plain, heads,
             ops.heads_gemm(q.unflatten(1, (heads, plain + rot)), w, q_lat, k=plain, n=rank)
         out.append((cache, q_lat))
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("m,n,k,heads", [(1000, 500, 136, 9), (8193, 64, 8, 8), (515, 512, 128, 16)])      # two blocks of rows a wave, the last in part
+def test_products_per_head_of_many_rows_give_the_bits_of_few(ops, m, n, k, heads):
+    assert -(-m // 16) * -(-n // 64) * heads >= 4096
+    gen = torch.Generator().manual_seed(m)
+    a = torch.randn(m, heads, k, generator=gen).bfloat16().to(DEV)
+    w, gate = torch.randn(heads, n, k, generator=gen).bfloat16().to(DEV), torch.randn(m, heads, generator=gen).to(DEV)
+    out, few = torch.empty(m, heads, n, device=DEV), torch.empty(100, heads, n, device=DEV)
+    ops.heads_gemm(a, w, out, k=k, n=n, gate=gate)
+    for first in (0, m // 2, m - 100):
+        ops.heads_gemm(a[first:first + 100].contiguous(), w, few, k=k, n=n, gate=gate[first:first + 100].contiguous())
+        assert torch.equal(out[first:first + 100], few)
