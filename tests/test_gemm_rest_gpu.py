@@ -53,3 +53,23 @@ def test_gated_rows_beyond(ops, m, half, k, rows):
         few_cols = w[2 * c:2 * c + 2048].contiguous()
         for a in (0, m // 2, m - 65):
             assert torch.equal(ops.gemm_swiglu(x[a:a + 65].contiguous(), few_cols, interleaved=True), got[a:a + 65, c:c + 1024])
+
+
+@pytest.mark.parametrize("nh,nkv,d,m,k,rows", [(32, 32, 128, 270, 512, 128), (172, 86, 64, 519, 512, 256)])
+@pytest.mark.parametrize("page", [64, 16])
+def test_qkv_rows_beyond(ops, nh, nkv, d, m, k, rows, page):
+    """Queries, and the pages that keys and values are written to: the bits of the same rows a few at a time."""
+    n = (nh + 2 * nkv) * d
+    assert ops.tiled_tile(m, n, k, qkv=True) == (rows, rows) and ops.tiled_tile(65, n, k, qkv=True) != (rows, rows)
+    x, w = rnd(m, k, seed=7).to(DEV), (rnd(n, k, seed=8) * 0.2).to(DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)      # noqa: E731
+    pages = -(-m // page) + 1
+    slots = [5 + i for i in range(m)]
+    table = ops.rope_table(i32([3 * i for i in range(m)]), d, 10000.0)
+    caches = [[torch.zeros(pages, nkv, *shape, dtype=torch.bfloat16, device=DEV) for shape in ((page, d), (d, page))] for _ in range(2)]
+    q = ops.gemm_qkv_rope_tiled(x, w, table, i32(slots), *caches[0], nh, nkv, d)
+    for a in range(0, m, 65):
+        b = min(a + 65, m)
+        few = ops.gemm_qkv_rope_tiled(x[a:b].contiguous(), w, table[a:b].contiguous(), i32(slots[a:b]), *caches[1], nh, nkv, d)
+        assert torch.equal(few, q[a:b])
+    assert all(torch.equal(one, two) for one, two in zip(*caches))
