@@ -257,22 +257,35 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
   struct Tile {
     floatx4 k[KB][DB], v[KB][DB];
   };
-  auto fetch_keys = [&](Tile& t, int j0) {
+  // Where a tile's keys and values lie is looked up for both before either is asked for: loads come back in the order asked, and a look at the
+  // block table behind the keys' loads waited for those (a decode step of 8 requests at 24 to 130 tokens: 0.4 us of 8 a layer).
+  struct Places {
+    long k[KB], v[KB];                       // (negative: not there)
+  };
+  auto places_of = [&](int j0) {
+    Places at;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      const int j = j0 + 16 * kb + c;
-      const bool ok = j >= lo && j <= last;
-      const float* p = a.k_cache + (ok ? cache.key(j, 4 * g) : 0);
+      const int j = j0 + 16 * kb + c, jv = j0 + 16 * kb + 4 * g;
+      at.k[kb] = j >= lo && j <= last ? cache.key(j, 4 * g) : -1;
+      at.v[kb] = jv + 3 >= lo && jv <= last ? cache.value(jv, c) : -1;
+    }
+    return at;
+  };
+  auto fetch_keys = [&](Tile& t, const Places& at) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const bool ok = at.k[kb] >= 0;
+      const float* p = a.k_cache + (ok ? at.k[kb] : 0);
 #pragma unroll
       for (int b = 0; b < DB; ++b) t.k[kb][b] = ok && 16 * b + 4 * g < a.dim ? load_floats(p + 16 * b) : no_floats();
     }
   };
-  auto fetch_values = [&](Tile& t, int j0) {
+  auto fetch_values = [&](Tile& t, const Places& at) {
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      const int j = j0 + 16 * kb + 4 * g;
-      const bool ok = j + 3 >= lo && j <= last;
-      const float* p = a.v_cache + (ok ? cache.value(j, c) : 0);
+      const bool ok = at.v[kb] >= 0;
+      const float* p = a.v_cache + (ok ? at.v[kb] : 0);
 #pragma unroll
       for (int b = 0; b < DB; ++b)
         t.v[kb][b] = ok && 16 * b + c < a.dim ? load_floats(p + static_cast<long>(16 * b) * a.page_tokens) : no_floats();
@@ -281,11 +294,7 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
   int j0 = (lo / KT - lo / KT % kFewWaves + wave) * KT;                      // this wave's first tile at or after lo's
   if (j0 < lo - lo % KT) j0 += kFewWaves * KT;
   Tile cur, nxt;
-  if (j0 <= last) {
-    fetch_keys(cur, j0);
-    if constexpr (AHEAD) fetch_values(cur, j0);
-  }
-
+  Places at = places_of(j0);
   floatx4 qf[DB], o[DB];
 #pragma unroll
   for (int b = 0; b < DB; ++b) {
@@ -293,12 +302,18 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
     qf[b] = d < a.dim ? load_floats(a.q + token * a.q_row + static_cast<long>(head) * a.dim + d) : no_floats();
     o[b] = no_floats();
   }
+  if (j0 <= last) {
+    fetch_keys(cur, at);
+    if constexpr (AHEAD) fetch_values(cur, at);
+  }
+
   float m = -FLT_MAX, l = 0.f;
   for (; j0 <= last; j0 += kFewWaves * KT) {
     const int next = j0 + kFewWaves * KT;
     if (AHEAD && next <= last) {
-      fetch_keys(nxt, next);
-      fetch_values(nxt, next);
+      at = places_of(next);
+      fetch_keys(nxt, at);
+      fetch_values(nxt, at);
     }
     floatx4 sc[KB];
 #pragma unroll
@@ -309,7 +324,7 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) sc[kb] = mfma_16x16x4(cur.k[kb][b][e], qf[b][e], sc[kb]);
-    if constexpr (!AHEAD) fetch_values(cur, j0);
+    if constexpr (!AHEAD) fetch_values(cur, at);
     const bool whole = j0 + KT - 1 <= ctx && (a.window <= 0 || j0 > last - a.window);
     const float alpha = softmax_tile<KB>(sc, m, l, a.scale, whole, j0, g, pos, a.window);
 #pragma unroll
@@ -356,7 +371,7 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
     }
     if (next <= last) {
       if constexpr (AHEAD) cur = nxt;
-      else fetch_keys(cur, next);
+      else at = places_of(next), fetch_keys(cur, at);
     }
   }
   l = four_lanes_sum(l);
