@@ -294,6 +294,9 @@ extern "C" {
 // them, bc4g_gemm_skinny_prenormed).
 int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const float* w, const void* next_w, int next_w_dtype, float next_eps,
                      void* out, int out_dtype, float* ssq, int n_rows, int hidden, float eps, void* stream);
+// What bc4g_rmsnorm_add leaves with ssq, of rows of the stream as they lie (rows [n_rows] null: the first n_rows): out[r] = bfloat16(x[rows[r]] * w),
+// ssq[r] the row's sum of squares.  hidden a multiple of 8, everything on 16-byte boundaries.
+int bc4g_rmsnorm_prepare(const float* x, const int32_t* rows, const void* w, int w_dtype, void* out, float* ssq, int n_rows, int hidden, void* stream);
 // out[r] = h + bias + (the causal convolution of h) with h = the RMSNorm of x[r], for a step in which request r brings row r alone:
 // bc4g_rmsnorm and bc4g_causal_conv (add_input) in one launch, the same bits.  w float32 [taps][hidden], state [slots, taps - 1, hidden]
 // in the output's type; 2 to 4 taps, hidden a multiple of 8 up to 4096, everything on 16-byte boundaries.  add_y (null: nothing): first

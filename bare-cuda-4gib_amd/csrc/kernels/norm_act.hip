@@ -139,6 +139,40 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_add_rows_kernel(float* __restr
   }
 }
 
+// What a streaming product that absorbs an RMSNorm takes (kPrepared above) of rows of the stream as they lie: out[r, :] = x[rows[r], :] * w in
+// bfloat16 and ssq[r] = the row's sum of squares, in that product's order.  Every workgroup of the product that absorbs the norm itself stages all
+// the rows again; wide outputs pay more for that than for this launch (ops.LinearPlan.norms_apart has both sides).  A wave a row: a row does
+// nothing but wait, so eight pieces of 512 elements are asked for together, without a condition (those past the row are its first again).
+template <typename TN>
+__global__ __launch_bounds__(kWave) void rmsnorm_prepare_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows,
+                                                                const TN* __restrict__ w, bf16_t* __restrict__ out, float* __restrict__ ssq, int hidden) {
+  constexpr int kAhead = 8, kPiece = kWave * 8;
+  const float* xr = x + static_cast<size_t>(rows ? rows[blockIdx.x] : blockIdx.x) * hidden;
+  bf16_t* to = out + static_cast<size_t>(blockIdx.x) * hidden;
+  float ss = 0.f;
+  for (int i0 = threadIdx.x * 8; i0 < hidden; i0 += kAhead * kPiece) {
+    float xv[kAhead][8], wv[kAhead][8];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int i = i0 + j * kPiece < hidden ? i0 + j * kPiece : 0;
+      load_eight(xr + i, xv[j]);
+      load_eight(w + i, wv[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int i = i0 + j * kPiece;
+      if (i >= hidden) continue;
+      ss = add_squares(xv[j], i >= kPiece, ss);
+      float o[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = xv[j][e] * wv[j][e];
+      store_eight(to + i, o);
+    }
+  }
+  ss = wave_sum(ss);
+  if (threadIdx.x == 0) ssq[blockIdx.x] = ss;
+}
+
 // An RMSNorm and the causal convolution that is added to it, for rows that are one request's only one of the step (a decode step):
 // h = the norm of x[r] as the norm kernel leaves it, out[r] = h + (bias + sum_j w[j] tail[j] + w[TAPS - 1] h), and the request's tail
 // moves on by h.  What the two kernels would compute, bit for bit; widths as above.  8 rows of 2,048: 4.5 us where the
@@ -484,6 +518,18 @@ extern "C" int bc4g_rmsnorm_add(float* x, const void* y, int y_dtype, const floa
 #undef BC4G_ADD
 #undef BC4G_ADD_ROWS
   return check_launch("rmsnorm_add");
+}
+
+extern "C" int bc4g_rmsnorm_prepare(const float* x, const int32_t* rows, const void* w, int w_dtype, void* out, float* ssq, int n_rows, int hidden,
+                                    void* stream) {
+  BC4G_REQUIRE(n_rows >= 0 && hidden > 0 && hidden % 8 == 0 && x && w && out && ssq && on_16(x) && on_16(w) && on_16(out),
+               "rmsnorm_prepare: bad arguments rows=%d H=%d (a multiple of 8, everything on 16-byte boundaries)", n_rows, hidden);
+  BC4G_REQUIRE(w_dtype == kF32 || w_dtype == kBF16, "rmsnorm_prepare: unknown dtype %d of the scale", w_dtype);
+  if (n_rows == 0) return 0;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (w_dtype == kF32) rmsnorm_prepare_kernel<float><<<n_rows, kWave, 0, s>>>(x, rows, static_cast<const float*>(w), static_cast<bf16_t*>(out), ssq, hidden);
+  else rmsnorm_prepare_kernel<bf16_t><<<n_rows, kWave, 0, s>>>(x, rows, static_cast<const bf16_t*>(w), static_cast<bf16_t*>(out), ssq, hidden);
+  return check_launch("rmsnorm_prepare");
 }
 
 extern "C" int bc4g_rmsnorm_conv(float* x, const float* add_y, const float* add_w, float add_eps, const void* norm_w, int norm_w_dtype, float eps,

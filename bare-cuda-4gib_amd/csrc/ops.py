@@ -776,11 +776,13 @@ class LinearPlan:
         return 0 < m <= self.fused_norm_rows
 
     def norms_apart(self, m: int) -> bool:
-        """Whether the norm before a product that could absorb it is better a kernel of its own.  Every workgroup of 16 outputs stages all
-        the rows again: from five rows on an output of 16,384 and more pays more for that than for a launch (with the norm inside and apart, 8
-        rows: 32,000 x 2,048 31.9 and 25.9 + 2.4 us, 128,256 x 4,096 217 and 182 + 3; five rows 29.3 and 25.7 + 2.4, 202 and 178 + 3; four rows 27.7
-        and 25.8 + 2.4, 180 and 176 + 3; 8 rows 11,264 x 2,048 14.2 and 11.5 + 2.4)."""
-        return m >= 5 and self.n >= 16384
+        """Whether the norm before a product that could absorb it is better prepared by a kernel of its own (rmsnorm_prepare: the same bits).
+        Every workgroup of 16 outputs stages all the rows again: from five rows on a wide output pays more for that than for a launch.
+        Weights from memory, 8 rows, microseconds inside and prepared: 32,000 x 2,048 32.8 and 31.0, 32,000 x 4,096 63.7 and 56.3, 128,256 x
+        4,096 219 and 189, 16,384 x 4,096 35.3 and 32.9; five rows of the first two 30.8 and 30.3, 60.4 and 55.2, four rows 29.6 and 30.1, 54.8 and
+        54.6; 11,264 x 2,048 14.1 and 14.9.  A narrow row is little to stage, so there the line lies further out: 16,384 x 512 7.7 and
+        7.9, x 256 6.9 and 6.8, but 32,000 x 512 12.1 and 11.2, x 64 9.0 and 7.8, 128,256 x 64 30.0 and 18.8."""
+        return m >= 5 and self.n >= (16384 if self.k >= 1024 else 24576) and self.streams(m)
 
     def parts(self, m: int) -> int:
         """Into how many parts an adding product of m rows cuts k over workgroups (1: it does not)."""
@@ -973,7 +975,7 @@ def absorbs_norm(n_rows: int, g: torch.Tensor, w) -> bool:
 
 
 def norm_apart(n_rows: int, w) -> bool:
-    """Whether a norm that the product could absorb is better run before it (LinearPlan.norms_apart)."""
+    """Whether a norm that the product could absorb is better prepared before it (LinearPlan.norms_apart)."""
     return plan_for(w.shape[0], w.shape[1]).norms_apart(n_rows)
 
 
@@ -1046,7 +1048,7 @@ class Fresh:
 
 class Prenormed:
     """What a product that added into the residual stream left for the RMSNorm after it
-    (gemm_accumulate_emit): ``xb`` = bfloat16(residual * g) [m, width] and ``parts`` [blocks, m], block
+    (gemm_accumulate_emit), or a kernel made of the stream (rmsnorm_prepare): ``xb`` = bfloat16(residual * g) [m, width] and ``parts`` [blocks, m], block
     b's share (16 columns) of every row's sum of squares -- or [blocks, m, 2], the shares of its halves, where two
     workgroups shared a block (half_blocks).  A product that takes it
     (gemm_prenormed, gemm_qkv_rope) applies the row's rsqrt(sum of parts / width + eps) to its sums."""
@@ -1579,6 +1581,26 @@ def rmsnorm_add(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: flo
     if next_norm is None:
         return x
     return Prenormed(out, ssq, next_eps) if ssq is not None else out
+
+
+def rmsnorm_prepare(x: torch.Tensor, rows: Optional[torch.Tensor], n_rows: int, g: torch.Tensor, eps: float) -> Optional[Prenormed]:
+    """What a product that absorbs the RMSNorm (scale g) of rows of the float stream x [T, H] takes (Prenormed, in one part; ``rows`` as in
+    rmsnorm); None where the kernel does not take the width."""
+    _dev("rmsnorm_prepare", x, rows, g)
+    hidden = x.shape[1]
+    if hidden % 8 or x.data_ptr() % 16 or g.data_ptr() % 16:
+        return None
+    if x.dtype != torch.float32 or x.dim() != 2 or tuple(g.shape) != (hidden,):
+        raise KernelError(f"rmsnorm_prepare: x must be float32 [T, H] and the scale [H], got {x.dtype} {tuple(x.shape)} and {tuple(g.shape)}")
+    if rows is not None:
+        _i32("rmsnorm_prepare", "rows", rows, n_rows)
+    elif n_rows != x.shape[0]:
+        raise KernelError("rmsnorm_prepare: without row indices every row of x is used")
+    xb = torch.empty((n_rows, hidden), dtype=torch.bfloat16, device=x.device)
+    ssq = torch.empty((1, n_rows), dtype=torch.float32, device=x.device)
+    library.call("bc4g_rmsnorm_prepare", _ptr(x), _ptr(rows), _ptr(g), _code(g, "rmsnorm_prepare"), _ptr(xb), _ptr(ssq), n_rows, hidden, _stream(),
+                 cost=lambda: (3.0 * n_rows * hidden, n_rows * hidden * 6 + hidden * g.element_size()))
+    return Prenormed(xb, ssq, eps)
 
 
 def rmsnorm_conv(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, out_dtype: torch.dtype, weight: torch.Tensor, state: torch.Tensor,

@@ -20,7 +20,7 @@ def _fused_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
     if x._tensor is not None:
         return None
     scale = x.fusable_scale()
-    if scale is None or not ops.gemm_normed_supported(x.x, x.n_rows, scale[0], w) or ops.norm_apart(x.n_rows, w):
+    if scale is None or not ops.gemm_normed_supported(x.x, x.n_rows, scale[0], w):
         return None
     return ops.gemm_normed(x.x, x.rows, x.n_rows, scale[0], scale[1], w, epilogue)
 
@@ -28,11 +28,21 @@ def _fused_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
 def absorbs_norm(norm, w, n_rows: int) -> bool:
     """Whether a product of n_rows rows of the stream with this weight absorbs the norm before it (_fused_norm)."""
     scale = norm.fusable() if hasattr(norm, "fusable") else None
-    return scale is not None and ops.absorbs_norm(n_rows, scale[0], w) and not ops.norm_apart(n_rows, w)
+    return scale is not None and ops.absorbs_norm(n_rows, scale[0], w)
+
+
+def _prepare(x: Normed, w) -> None:
+    """What the product would make of the norm in each of its workgroups, by a kernel before it where that is the faster way (the same bits)."""
+    if x.pre is not None or x._tensor is not None or not ops.norm_apart(x.n_rows, w):
+        return
+    scale = x.fusable_scale()
+    if scale is not None and ops.gemm_normed_supported(x.x, x.n_rows, scale[0], w):
+        x.pre = ops.rmsnorm_prepare(x.x, x.rows, x.n_rows, *scale)
 
 
 def _prepared_norm(x: Normed, w, epilogue: int) -> Optional[torch.Tensor]:
-    """The product from what the product before left for this norm, where there is such a thing."""
+    """The product from what the product before left for this norm, or a kernel before it makes, where there is such a thing."""
+    _prepare(x, w)
     if x.pre is None or x._tensor is not None:
         return None
     if x.pre.xb.dtype == torch.float32:
@@ -114,6 +124,7 @@ def linear_xielu(x: Union[torch.Tensor, Normed], w, pq: torch.Tensor, out_dtype:
     it was), else by a kernel behind it."""
     if out_dtype == torch.bfloat16:
         if isinstance(x, Normed):
+            _prepare(x, w)
             if x.pre is not None and x._tensor is None:
                 fast = ops.gemm_xielu(x.pre.xb, w, pq, pre=x.pre)
                 if fast is not None:
