@@ -159,6 +159,8 @@ class CausalAttention(Part):
     def _float_qkv(self, h, ctx, slot_map, k_cache, v_cache, rotary_dim, theta, writes):
         """The q|k|v product of few float32 rows with rotation and cache write in its epilogue, the angles from the step's
         table; None where that kernel does not take the operands."""
+        if self.act_dtype != torch.float32 or self.head_dim % 16 or rotary_dim not in (0, self.head_dim):
+            return None       # (before a norm that the plain product may absorb is run)
         pre = h.pre if isinstance(h, Normed) and h._tensor is None else None
         if pre is None and (h.n_rows if isinstance(h, Normed) else h.shape[0]) > ops.GEMM_F32_FEW_ROWS:
             return None

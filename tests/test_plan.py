@@ -68,3 +68,19 @@ def test_parts_ask_their_weight_s_plan():
     assert attn.wants_prepared_norm(1) and attn.wants_prepared_norm(64)
     attn.act_dtype = torch.float32
     assert not attn.wants_prepared_norm(8)
+
+
+def test_a_layer_in_bfloat16_runs_no_norm_for_the_32_bit_product():
+    """Heads that the matrix-core layouts do not take (a size that is no multiple of 16, rotation of part of a head) go to the plain product,
+    which absorbs the norm of few rows: nothing may have run it before."""
+    import types
+    import torch
+    from bare_cuda_4gib_amd.parts.attention import CausalAttention
+    from bare_cuda_4gib_amd.parts.lazy import Normed
+
+    ran = []
+    norm = types.SimpleNamespace(forward=lambda *a, **k: ran.append(1) or torch.zeros(4, 96))
+    for head_dim, rotary_dim, dtype in ((24, 24, torch.bfloat16), (32, 16, torch.bfloat16), (24, 24, torch.float32), (32, 16, torch.float32)):
+        attn = CausalAttention(96, 4, 2, head_dim)
+        attn.act_dtype, attn.w_qkv = dtype, torch.zeros(8 * head_dim, 96, dtype=dtype)
+        assert attn._float_qkv(Normed(torch.zeros(4, 96), norm), None, None, None, None, rotary_dim, 1e4, True) is None and not ran
