@@ -203,7 +203,7 @@ class Model:
         if self.streams > 1:            # the stream in copies, [T, streams, H]: every copy starts as the embedding
             from ..csrc import ops
             x = ops.streams_fill(x, self.streams)
-        ctx.handoff.end_step()
+        ctx.handoff.begin_step()
         for i, e in enumerate(self.schedule):
             layer = self.layers[e.layer]
             # (nobody prepares the first norm of an entry before which the stream changes once more)

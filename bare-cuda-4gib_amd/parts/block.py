@@ -1,8 +1,7 @@
 """How a layer's parts are arranged around the residual stream."""
 from __future__ import annotations
 
-import torch
-
+import inspect
 from typing import Dict
 
 import torch
@@ -137,7 +136,7 @@ class PreNormBlock(Part):
 class AddingReader:
     """Who reads the stream next, where that is a norm with a convolution behind it that can add a sublayer's normed output first (what
     a SandwichBlock names as its first reader): in a step of single rows the block before leaves its last output to it, (norm, y), and
-    the stream lacks that output until the reader has come."""
+    the stream lacks that output until the reader has come (NormHandoff.owe)."""
 
     def takes(self, norm, y, ctx) -> bool:
         return ctx.n_tokens == ctx.n_seqs and getattr(norm, "added_by_the_reader", None) is not None and norm.added_by_the_reader(y) is not None
@@ -150,11 +149,14 @@ class SandwichBlock(Part):
     norm is added to the float32 stream in one kernel."""
     category = "block"
     graph_safe = True     # launches kernels only: may run inside a captured graph
+    reader = None
 
     def __init__(self, mixer, mixer_norm, mixer_post_norm, ffn=None, ffn_norm=None, ffn_post_norm=None, mixer_conv=None):
         self.mixer, self.mixer_norm, self.mixer_post_norm = mixer, mixer_norm, mixer_post_norm
         self.ffn, self.ffn_norm, self.ffn_post_norm, self.mixer_conv = ffn, ffn_norm, ffn_post_norm, mixer_conv
-        self.reader = AddingReader() if hasattr(mixer_conv, "behind") else None
+        # (a block with a forward of its own may not take what is left, a convolution with a `behind` of its own may not add it)
+        if type(self).forward is SandwichBlock.forward and hasattr(mixer_conv, "behind") and "adds" in inspect.signature(mixer_conv.behind).parameters:
+            self.reader = AddingReader()
 
     def first_reader(self, n_rows: int):
         """What the entry before may leave its last output to (None: this block begins with a norm that nobody prepares)."""
@@ -212,7 +214,7 @@ class SandwichBlock(Part):
         """x += norm(y), by whoever reads the stream next where that can."""
         following = getattr(getattr(ctx, "handoff", None), "next_entry", None)
         if following is not None and isinstance(following[0], AddingReader) and following[0].takes(norm, y, ctx):
-            ctx.handoff.leave(following[0], (norm, y))
+            ctx.handoff.owe(following[0], (norm, y))
         else:
             norm.add_to(x, y)
 

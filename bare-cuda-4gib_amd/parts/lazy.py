@@ -12,6 +12,8 @@ from typing import Any, Dict, Optional, Tuple
 
 import torch
 
+from ..errors import EngineError
+
 
 class Normed:
     def __init__(self, x: torch.Tensor, norm, ctx=None, rows: Optional[torch.Tensor] = None,
@@ -53,7 +55,7 @@ class NormHandoff:
     the model    ``begin_entry(layer, following, n_rows)`` before every schedule entry: what the entry before left
                  for this entry's first norm stays, everything else goes, and the first reader of the entry after
                  this one is noted (``first_reader(n_rows) -> (norm, takes_parts)`` of a block that has one);
-                 ``end_step()`` after the last.
+                 ``begin_step()`` before the first and ``end_step()`` after the last.
     a block      ``with handoff.reader(norm, takes_parts):`` around each part that adds into the stream, naming the
                  norm that reads the stream after that part (``handoff.next_entry`` for its last part), and
                  ``take(norm)`` for what was left for a norm of its own.
@@ -61,20 +63,33 @@ class NormHandoff:
 
     What is left is the finished norm (ops.Finished), which serves every reader, or -- only for a reader that says
     it takes them -- the parts of one that a product can finish (ops.Prenormed).  Nothing left outlives the entry
-    after the one that made it.  A block that does not use any of this stays correct: its norms simply run."""
+    after the one that made it.  A block that does not use any of this stays correct: its norms simply run.
+
+    ``owe(reader, what)`` leaves something of another kind, which the stream lacks until the reader has added it (a
+    sublayer's output for parts.block.AddingReader).  Only a block that takes it in its own forward names such a reader; the
+    entry after this one has to, and where it does not the step ends in an error instead of without that output."""
 
     def __init__(self):
         self.reading_next: Optional[Tuple[Any, bool]] = None
         self.next_entry: Optional[Tuple[Any, bool]] = None
         self._left: Dict[int, Any] = {}
+        self._owed: Optional[Tuple[Any, Any]] = None       # (reader, what) of the entry that runs
+        self._due = False                                  # ... and it was owed to that entry when it began
 
     @staticmethod
     def _first_reader(layer, n_rows: int) -> Optional[Tuple[Any, bool]]:
         first = getattr(layer, "first_reader", None)
         return first(n_rows) if first is not None else None
 
+    def begin_step(self) -> None:
+        self._left.clear()
+        self.next_entry = self.reading_next = self._owed = None
+
     def begin_entry(self, layer, following, n_rows: int) -> None:
         mine = self._first_reader(layer, n_rows)
+        if self._owed is not None and (self._due or mine is None or mine[0] is not self._owed[0]):
+            self._fail()
+        self._due = self._owed is not None
         kept = self._left.pop(id(mine[0]), None) if mine is not None else None
         self._left.clear()
         if kept is not None:
@@ -83,8 +98,14 @@ class NormHandoff:
         self.reading_next = None
 
     def end_step(self) -> None:
-        self._left.clear()
-        self.next_entry = self.reading_next = None
+        if self._owed is not None:
+            self._fail()
+        self.begin_step()
+
+    def _fail(self) -> None:
+        reader = self._owed[0]
+        self.begin_step()
+        raise EngineError(f"a layer's output was left to {type(reader).__name__}, which did not add it to the stream")
 
     def reader(self, norm, takes_parts: bool = False) -> "_Reading":
         return _Reading(self, (norm, bool(takes_parts)) if norm is not None else None)
@@ -92,5 +113,13 @@ class NormHandoff:
     def leave(self, norm, what) -> None:
         self._left[id(norm)] = what
 
+    def owe(self, reader, what) -> None:
+        if self._owed is not None:
+            self._fail()
+        self._owed, self._due = (reader, what), False
+
     def take(self, norm):
+        if self._owed is not None and self._owed[0] is norm:
+            owed, self._owed = self._owed[1], None
+            return owed
         return self._left.pop(id(norm), None)
