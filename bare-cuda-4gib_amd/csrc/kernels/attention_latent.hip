@@ -478,16 +478,17 @@ extern "C" int bc4g_latent_prepare(const void* q, const void* dkv, int dtype, co
                "latent_prepare: a tensor is missing");
   BC4G_REQUIRE((rot == 0 || !q || q_row >= static_cast<long>(heads) * (plain + rot)) && (!cache || dkv_row >= rank + rot),
                "latent_prepare: rows shorter than their parts");
+  BC4G_REQUIRE(!absorb || (q && q_lat && dtype == kBF16 && n_rows <= kFewRows && plain > 0 && plain % 8 == 0 && (plain + rot) % 8 == 0 && q_row % 8 == 0 &&
+                           q_row >= static_cast<long>(heads) * (plain + rot) && reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
+                           reinterpret_cast<uintptr_t>(absorb) % 16 == 0),
+               "latent_prepare: the absorbed queries' product takes up to %d bfloat16 rows whose heads lie on 16-byte boundaries, and a place for them",
+               kFewRows);
   const int parts = (cache ? 1 : 0) | (rot > 0 && q ? 2 : 0) | (low ? 4 : 0);
   const int n_parts = (parts & 1) + (parts >> 1 & 1) + (parts >> 2 & 1);
-  if (n_rows == 0 || parts == 0) return 0;
+  if (n_rows == 0 || (parts == 0 && !absorb)) return 0;
   const LowQuery lq{low, low_g, low_out, low_row, low_rank};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const size_t lds = static_cast<size_t>(dims > 0 ? dims : 2) * sizeof(float);
-  if (absorb)
-    BC4G_REQUIRE(q && dtype == kBF16 && n_rows <= kFewRows && plain > 0 && plain % 8 == 0 && (plain + rot) % 8 == 0 && q_row % 8 == 0 &&
-                     reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(absorb) % 16 == 0,
-                 "latent_prepare: the absorbed queries' product takes up to %d bfloat16 rows whose heads lie on 16-byte boundaries", kFewRows);
   if (dtype == kF32) {
     latent_prepare_kernel<float><<<dim3(n_rows, n_parts), kPrepBlock, lds, s>>>(
         PrepareArgs<float>{static_cast<const float*>(q), static_cast<const float*>(dkv), g, angles, slot_map, static_cast<float*>(cache), q_lat,

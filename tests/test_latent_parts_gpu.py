@@ -114,3 +114,17 @@ def test_products_per_head_of_many_rows_give_the_bits_of_few(ops, m, n, k, heads
     for first in (0, m // 2, m - 100):
         ops.heads_gemm(a[first:first + 100].contiguous(), w, few, k=k, n=n, gate=gate[first:first + 100].contiguous())
         assert torch.equal(out[first:first + 100], few)
+
+
+@pytest.mark.parametrize("t", [1, 17, 32])
+def test_absorbed_queries_with_nothing_else_to_write(ops, t):
+    """rot 0 and neither cache nor queries' latent: the product alone, by the entry point itself."""
+    from bare_cuda_4gib_amd.csrc import library
+    gen = torch.Generator().manual_seed(t)
+    heads, plain, rank = 3, 40, 80
+    q, w = torch.randn(t, heads * plain, generator=gen).bfloat16().to(DEV), torch.randn(heads, rank, plain, generator=gen).bfloat16().to(DEV)
+    got, want = torch.zeros(t, heads, rank, device=DEV), torch.zeros(t, heads, rank, device=DEV)
+    ops.heads_gemm(q.unflatten(1, (heads, plain)), w, want, k=plain, n=rank)
+    library.call("bc4g_latent_prepare", q.data_ptr(), None, 1, None, 1e-5, None, None, None, got.data_ptr(), t, heads, plain, 0, rank, 0, heads * plain, 0, 0,
+                 None, None, None, 0, 0, w.data_ptr(), ops._stream())
+    assert torch.equal(got, want)

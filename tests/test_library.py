@@ -58,3 +58,20 @@ def test_where_the_library_lives(monkeypatch, tmp_path):
     os.chmod(home, 0o777)
     with pytest.raises(KernelError, match="nowhere to build"):
         build._settle()
+
+
+def test_latent_prepare_refuses_absorbed_queries_without_a_place_or_whole_rows():
+    """Whatever else is asked for, and also where nothing is rotated: refused before anything is launched."""
+    if not build.is_built():
+        pytest.skip("the kernel library is not built here")
+    at, heads, plain, rank = 1 << 20, 4, 16, 32                # (no call gets as far as reading from this address)
+
+    def prepare(q=at, q_lat=at, rot=0, q_row=heads * 16, rows=8, dtype=1, cache=None, absorb=at):
+        library.call("bc4g_latent_prepare", q, at, dtype, at, 1e-5, at, at, cache, q_lat, rows, heads, plain, rot, rank, 0, q_row, rank + rot, 0,
+                     None, None, None, 0, 0, absorb, None)
+
+    for wrong in (dict(q_lat=None), dict(q_lat=None, cache=at), dict(q=None), dict(q=None, cache=at), dict(q_row=heads * 16 - 8), dict(q_row=heads * 16 - 8, cache=at),
+                  dict(rows=33), dict(dtype=0), dict(q=at + 8), dict(absorb=at + 8), dict(q_row=heads * 16 + 4)):
+        with pytest.raises(KernelError, match="absorbed queries"):
+            prepare(**wrong)
+    prepare(rows=0)
