@@ -1230,7 +1230,8 @@ int launch_halves(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& s
 // the chip and with one on every CU), a few us around them, and its stores.  All measured with the weights coming from memory, as they do
 // inside a model (forty weights one after the other): a loop over one product finds its weights in the 256 MB cache before
 // memory and flatters the small tiles and the short rings.  The model's times are within 5 % of those measured for 72 to 4,096 rows at
-// outputs of 2,048 to 28,672 and k of 2,048 to 14,336.  A function of (m, n, k) alone; every tile adds over k in the same order.
+// outputs of 2,048 to 28,672 and k of 2,048 to 14,336 (one product after the other without a pause 1 % short to 7 % long at the median, 64 x 64
+// 18 % long).  A function of (m, n, k) alone; every tile adds over k in the same order.
 struct DirectForm {
   int rows, cols;
   double us_a_step_few, us_a_step_full, us_around, us_stores;
@@ -1265,11 +1266,13 @@ int direct_form(int m, int n, int k, bool long_epilogue) {
 }
 
 // Rows beyond whole tiles beside them (gemm_mfma_rest_kernel): the 64 x 256 tiles' times, measured as the others' were, and the time of a launch that
-// begins with `whole` tiles of a form and goes on with `rest` such: those first go to the CUs that the last turn of large tiles leaves.
+// begins with `whole` tiles of a form and goes on with `rest` such: those first go to the CUs that the last turn of large tiles leaves.  (On
+// what the chip shares a tile is a load by its size: four small ones are a 256 x 256.)
 constexpr DirectForm kRestForm = {64, 256, 0.50, 0.62, 0.0, 1.0};
 double rest_time(const DirectForm& form, int whole, int rest, int k) {
   const int cus = compute_units(), steps = k / 64;
-  const double fill = whole + rest < cus ? static_cast<double>(whole + rest) / cus : 1.0;
+  const double load = whole + rest * static_cast<double>(kRestForm.rows * kRestForm.cols) / (form.rows * form.cols);
+  const double fill = load < cus ? load / cus : 1.0;
   const double large = steps * (form.us_a_step_few + (form.us_a_step_full - form.us_a_step_few) * fill) + form.us_stores;
   const double small = steps * (kRestForm.us_a_step_few + (kRestForm.us_a_step_full - kRestForm.us_a_step_few) * fill) + kRestForm.us_stores;
   const int full = whole / cus, busy = whole % cus;
@@ -1290,12 +1293,16 @@ double rest_time(const DirectForm& form, int whole, int rest, int k) {
 // How an output's columns are cut: the first n1 in tiles of `first`, the rest (if any) in tiles of `second`, one launch each.  Tiles that do not
 // fill the last turn of the chip leave CUs idle for a whole tile (3,000 x 11,264 are 528 tiles of 256 x 256: 256, 256 and 16); columns that fill
 // whole turns with large tiles, and smaller tiles for the others, leave less.  Every element is added up as before, by whichever tile.
-// From k = 512 on (below, a launch is as long as a tile), and where it is 4 % and more by the model, a second launch counted with the 8 us
-// by which cut products were measured to be longer than their parts: 3,000 x 11,264 x 2,048 141 -> 129 us (10,752 columns in 256 x 256, 512 in
-// 64 x 64), 1,400 x 11,264 x 2,048 84 -> 78.5, 1,100 x 28,672 x 4,096 287 -> 254.  Without the 8 us 300 x 11,264 x 2,048 was cut: 35 -> 39.
-constexpr double kCutGap = 8.0;
+// From k = 512 on (below, a launch is as long as a tile), and where it is 4 % and more by the model, a second launch counted with 6 us:
+// weights from memory, 3,000 x 11,264 x 2,048 138 -> 125 us (10,752 columns in 256 x 256, 512 in 64 x 64), 1,500 x 11,264 x 2,048 76 -> 69 (the
+// same), 2,300 x 2,048 x 5,632 80 -> 74 (128 x 128 and 64 x 64).
+constexpr double kCutGap = 6.0;
 // Or its rows: whole tiles of `first`, and the rows that remain in the same launch (rest_time; up to four turns of the chip, beyond them a turn more matters
 // little).
+// Over 11,000 products of 257 to 4,200 rows, 2,048 to 30,720 outputs and k 1,024 to 8,192 the times of cut columns and rows beyond are 3 % too long at
+// the median and 20 % too long to 17 % too short at the ends, so forms within 5 % of each other are taken as it falls: what is chosen is 1.3 % slower on average
+// than the fastest of the forms measured, and 0.05 % slower than whole tiles where it displaces them.  (With small tiles counted as large ones in
+// the load and 8 us a cut more than 261 of them took another form: 236 gained 8 % by the change, 25 lost 5.)
 struct Parts {
   int first, n1, second;
   bool rest;
@@ -1483,6 +1490,14 @@ extern "C" int bc4g_gemm_mfma_qkv(const void* a, const void* w, int w_packed, vo
                                               static_cast<hipStream_t>(stream), ra))
     return e;
   return check_launch("gemm_mfma_qkv");
+}
+
+extern "C" int bc4g_gemm_mfma_cut(const void* a, const void* w, int m, int n, int k, int qkv, int* first_cols, int* rows, int* cols, int* beyond) {
+  BC4G_REQUIRE(first_cols && rows && cols && beyond && m > 0 && n > 0 && k > 0, "gemm_mfma_cut: sizes and four places for the answer");
+  const Parts parts = direct_operands(a, w, k) ? parts_of(m, n, k, qkv != 0) : Parts{0, n, 0, false};
+  const bool cut = parts.n1 < n;
+  *first_cols = parts.n1, *rows = cut ? kDirectForm[parts.second].rows : 0, *cols = cut ? kDirectForm[parts.second].cols : 0, *beyond = parts.rest;
+  return 0;
 }
 
 extern "C" int bc4g_gemm_mfma_tile(const void* a, const void* w, int m, int n, int k, int qkv, int* rows, int* cols) {

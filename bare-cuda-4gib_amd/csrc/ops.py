@@ -87,6 +87,15 @@ def tiled_tile(m: int, n: int, k: int, a_ptr: int = 0, w_ptr: int = 0, qkv: bool
     return rows.value, cols.value
 
 
+def tiled_cut(m: int, n: int, k: int, qkv: bool = False) -> Tuple[int, Optional[Tuple[int, int]], bool]:
+    """How that product's output is cut: (columns in tiled_tile's tiles, the tile of the other columns (None: there are none), whether rows beyond
+    whole tiles go beside them in the same launch)."""
+    first, rows, cols, beyond = (ctypes.c_int(0) for _ in range(4))
+    library.call("bc4g_gemm_mfma_cut", None, None, m, n, k, int(qkv), ctypes.byref(first), ctypes.byref(rows), ctypes.byref(cols), ctypes.byref(beyond),
+                 launches=False)
+    return first.value, (rows.value, cols.value) if first.value < n else None, bool(beyond.value)
+
+
 def _tiled_cost(m: int, n: int, k: int, out_bytes: float, qkv: bool = False):
     if not _profiler.enabled:
         return None

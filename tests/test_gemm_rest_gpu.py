@@ -29,7 +29,7 @@ SHAPES = [(257, 11264, 512, 128), (270, 11268, 576, 128), (320, 11012, 2048, 128
 
 @pytest.mark.parametrize("m,n,k,rows", SHAPES)
 def test_rows_beyond(ops, m, n, k, rows):
-    assert ops.tiled_tile(m, n, k) == (rows, rows) and ops.tiled_tile(65, 1028, k) == (64, 64)
+    assert ops.tiled_tile(m, n, k) == (rows, rows) and ops.tiled_tile(65, 1028, k) == (64, 64) and ops.tiled_cut(m, n, k) == (n, None, True)
     x, w = rnd(m, k, seed=1).to(DEV), rnd(n, k, seed=2).to(DEV)
     got = ops.gemm_fast(x, w, torch.float32)
     assert (got.double() - x.double() @ w.double().T).abs().max() < 2.0 * k * 2.0 ** -24 * math.sqrt(k)    # k float additions of terms around 1
@@ -44,7 +44,7 @@ def test_rows_beyond(ops, m, n, k, rows):
 
 @pytest.mark.parametrize("m,half,k,rows", [(270, 5632, 2048, 128), (519, 14336, 576, 256)])
 def test_gated_rows_beyond(ops, m, half, k, rows):
-    assert ops.tiled_tile(m, 2 * half, k) == (rows, rows) and ops.tiled_tile(65, 2048, k) == (64, 64)
+    assert ops.tiled_tile(m, 2 * half, k) == (rows, rows) and ops.tiled_tile(65, 2048, k) == (64, 64) and ops.tiled_cut(m, 2 * half, k) == (2 * half, None, True)
     x = (rnd(m, k, seed=4) * 0.2).to(DEV)
     gate, up = ((rnd(half, k, seed=s) * 0.2).to(DEV).view(half // 8, 8, k) for s in (5, 6))
     w = torch.stack([gate, up], 1).view(2 * half, k)           # every 16 rows: eight gate rows, then the eight up rows of the same outputs
@@ -61,6 +61,7 @@ def test_qkv_rows_beyond(ops, nh, nkv, d, m, k, rows, page):
     """Queries, and the pages that keys and values are written to: the bits of the same rows a few at a time."""
     n = (nh + 2 * nkv) * d
     assert ops.tiled_tile(m, n, k, qkv=True) == (rows, rows) and ops.tiled_tile(65, n, k, qkv=True) != (rows, rows)
+    assert ops.tiled_cut(m, n, k, qkv=True) == (n, None, True)
     x, w = rnd(m, k, seed=7).to(DEV), (rnd(n, k, seed=8) * 0.2).to(DEV)
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)      # noqa: E731
     pages = -(-m // page) + 1

@@ -22,16 +22,23 @@ def rnd(*shape, seed):
     return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).bfloat16()
 
 
+# columns cut between two tiles: the first tile and its columns, the tile of the others
+CUT = [(1430, 11276, 1536, (256, 256), 10752, (64, 64)), (1025, 4100, 14336, (128, 128), 3584, (64, 64)), (2900, 6156, 2048, (256, 256), 5376, (128, 128))]
+CUT_QKV = [(64, 8, 64, 3333, 1024, 4608, (64, 64)), (48, 16, 80, 2821, 2048, 5376, (128, 128)), (24, 24, 128, 2055, 2048, 7168, (128, 64))]
+
+
 @pytest.mark.parametrize("m,n,k,tile", [
     (3860, 3852, 64, (256, 256)), (3860, 3852, 128, (256, 256)), (3841, 3841, 320, (256, 256)),       # one row, one column in the last tile
     (2036, 6132, 64, (256, 192)), (2036, 6132, 320, (256, 192)),
     (2036, 2040, 128, (128, 128)), (1921, 2036, 320, (128, 128)),
-    # columns cut: 10,752 in 256 x 256 and 524 in 64 x 64, 5,376 in 256 x 256 and 780 in 128 x 128
-    (1290, 11276, 1536, (256, 256)), (2900, 6156, 2048, (256, 256))])
+    (1290, 11276, 1536, (256, 256)),                                       # (ten rows beyond whole tiles, beside them)
+    *((m, n, k, tile) for m, n, k, tile, _, _ in CUT)])
 def test_turns_and_cut_columns(ops, m, n, k, tile):
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the shapes are chosen for 256 CUs")
     assert ops.tiled_tile(m, n, k) == tile and ops.tiled_tile(65, n, k) == (64, 64)
+    cut = next((c[4:] for c in CUT if c[:3] == (m, n, k)), (n, None))
+    assert ops.tiled_cut(m, n, k) == (*cut, (m, n, k) == (1290, 11276, 1536))
     x, w = rnd(m, k, seed=1).to(DEV), rnd(n, k, seed=2).to(DEV)
     want = x.double() @ w.double().T
     bound = 2.0 * k * 2.0 ** -24 * math.sqrt(k)            # k float additions of terms around 1
@@ -51,3 +58,24 @@ def test_turns_and_cut_columns(ops, m, n, k, tile):
     gate, up = want[:, :half], want[:, half:2 * half]
     exact = gate / (1 + torch.exp(-gate)) * up
     assert ((act.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + 3 * bound * (1 + gate.abs() + up.abs())).all()
+
+
+@pytest.mark.parametrize("nh,nkv,d,m,k,first,second", CUT_QKV)
+def test_cut_qkv(ops, nh, nkv, d, m, k, first, second):
+    """Queries, and the pages that keys and values are written to: the bits of the same rows a few at a time."""
+    n, page = (nh + 2 * nkv) * d, 64
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the shapes are chosen for 256 CUs")
+    assert ops.tiled_cut(m, n, k, qkv=True) == (first, second, False) and ops.tiled_cut(129, n, k, qkv=True) == (n, None, False)
+    x, w = rnd(m, k, seed=7).to(DEV), (rnd(n, k, seed=8) * 0.2).to(DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)      # noqa: E731
+    slots = [5 + i for i in range(m)]
+    table = ops.rope_table(i32([3 * i for i in range(m)]), d, 10000.0)
+    caches = [[torch.zeros(-(-m // page) + 1, nkv, *shape, dtype=torch.bfloat16, device=DEV) for shape in ((page, d), (d, page))] for _ in range(2)]
+    w = ops.StreamedWeight(w)
+    q = ops.gemm_qkv_rope_tiled(x, w, table, i32(slots), *caches[0], nh, nkv, d)
+    for a in range(0, m, 129):
+        b = min(a + 129, m)
+        few = ops.gemm_qkv_rope_tiled(x[a:b].contiguous(), w, table[a:b].contiguous(), i32(slots[a:b]), *caches[1], nh, nkv, d)
+        assert torch.equal(few, q[a:b])
+    assert all(torch.equal(one, two) for one, two in zip(*caches))
