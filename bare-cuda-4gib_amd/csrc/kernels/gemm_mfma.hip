@@ -6,8 +6,9 @@
 // and feeds 32x32x16 MFMAs.  Two forms:
 //  - the operand tiles go from memory into LDS without passing registers (k a multiple of 64, operands on 16-byte
 //    boundaries): gemm_mfma_halves_kernel for tiles of 256 x 256, gemm_mfma_turns_kernel for 256 x 192 and 128 x 128,
-//    gemm_mfma_direct_kernel for 256 x 128 (and 128 x 64 for q|k|v), gemm_mfma_ahead_kernel for 64 x 64; whichever lets the
-//    busiest CU finish first, or two of them side by side (parts_of).
+//    gemm_mfma_direct_kernel for 256 x 128 (and 128 x 64 for q|k|v), gemm_mfma_ahead_kernel for 64 x 64 -- and for all of
+//    them gemm_mfma_direct_kernel where k is short (short_walk); whichever lets the busiest CU finish first, or two of them
+//    side by side (parts_of).
 //  - gemm_mfma_staged_kernel: through registers, 128 x 128 tiles; any k that is a multiple of 8.
 // Every output element is accumulated over k in ascending order in both, whatever the number of
 // rows and the tile: the same bits whichever form and tile a shape selects.
@@ -1352,15 +1353,24 @@ int launch_rest(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& sca
   return 0;
 }
 
+// Up to which k a form is walked by gemm_mfma_direct_kernel: a short walk is mostly its beginning and its stores, which the kernels whose waves
+// take turns (and the one that reads a step ahead) do with fewer waves or more barriers.  Kernel of before over this one, 40 to 1,800 tiles, k
+// 128, 512 and 1,024: 256 x 256 0.82, 0.98 and 1.09 (adding 0.77, 0.90 and 0.98, at 1,536 1.06; gated 0.88, 1.06 and 1.18), 256 x 192 0.97, 1.05 and 1.10,
+// 128 x 128 0.93, 0.99 and 1.02, 64 x 64 0.94, 1.00 and 1.06.
+constexpr int short_walk(int form, int epi) {
+  return form == 0 && epi == kAccumF32 ? 1024 : form == 0 && gated(epi) ? 384 : form == 1 ? 256 : 576;
+}
+
 template <int EPI>
 int launch_form(int form, const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
+  const bool brief = o.k <= short_walk(form, EPI);
   switch (form) {
-    case 0: return launch_halves<EPI>(o, ra, scale);
-    case 1: return launch_turns<EPI, 4, 2, 2, 3, 32, 5>(o, ra, scale);
+    case 0: return brief ? launch_direct<EPI, 4, 4, 2, 2, 64, 2, 1>(o, ra, scale) : launch_halves<EPI>(o, ra, scale);
+    case 1: return brief ? launch_direct<EPI, 4, 2, 2, 3, 64, 2, 1>(o, ra, scale) : launch_turns<EPI, 4, 2, 2, 3, 32, 5>(o, ra, scale);
     case 2: return launch_direct<EPI, 4, 2, 2, 2, 64, 3, 1>(o, ra, scale);
-    case 3: return launch_turns<EPI, 2, 4, 2, 1, 64, 4>(o, ra, scale);
+    case 3: return brief ? launch_direct<EPI, 2, 4, 2, 1, 64, 4, 1>(o, ra, scale) : launch_turns<EPI, 2, 4, 2, 1, 64, 4>(o, ra, scale);
     case 5: return launch_direct<EPI, 2, 2, 2, 1, 64, 2, 4>(o, ra, scale);
-    default: return launch_ahead<EPI>(o, ra, scale);
+    default: return brief ? launch_direct<EPI, 2, 2, 1, 1, 64, 4, 2>(o, ra, scale) : launch_ahead<EPI>(o, ra, scale);
   }
 }
 

@@ -21,7 +21,7 @@ def rnd(*shape, seed):
     return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).bfloat16()
 
 
-@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 11])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13])      # (up to nine by the kernel without a step ahead)
 @pytest.mark.parametrize("m,n", [(65, 52), (129, 130)])
 def test_short_walks(ops, steps, m, n):
     k = 64 * steps

@@ -35,6 +35,24 @@ def prepared(ops, m, n, seed, k=36):
     return residual, g, pre, few
 
 
+@pytest.mark.parametrize("n", [96, 2048])
+def test_rows_on_both_sides_of_few(ops, n):
+    """64 rows finish the norm behind the product's sums, 65 run it before the product: a row's bits are others, its bound is the same."""
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    f = lambda *shape: torch.randn(*shape, generator=gen, device=DEV)      # noqa: E731
+    x, w, start, g, after = f(65, 36), f(n, 36), f(65, n), 1.0 + 0.2 * f(n), 0.1 * f(42, n)
+    residual = start[:64].clone()
+    pre = ops.gemm_f32_emit(x[:64].contiguous(), w, residual, g, EPS)
+    many = ops.gemm_f32(x, w, accumulate_into=start.clone())
+    assert ops.gemm_f32_emit(x, w, start, g, EPS) is None and not ops.gemm_f32_finishes_norm(65, after) and torch.equal(many[:64], residual)
+    r = residual.double()
+    normed = r * torch.rsqrt((r * r).mean(-1, keepdim=True) + EPS) * g.double()
+    z, size = normed @ after.double().T, normed.abs() @ after.double().abs().T
+    rel = (n + 2 + 40 + n / 256) * U
+    held(ops.gemm_f32_prenormed(pre, after), z, rel * size, "64 rows")
+    held(ops.gemm_f32(ops.rmsnorm(many, g, EPS, torch.float32), after)[:64], z, rel * size, "65 rows")
+
+
 # Rows at the edges of the forms (8, 16 and 32 a workgroup); columns that end inside a block of 16 and inside its half, few enough for
 # eight outputs a workgroup and too many, and more than the 4,096 whose parts a product asks for together.
 @pytest.mark.parametrize("m", [1, 7, 8, 9, 16, 17, 33, 64])

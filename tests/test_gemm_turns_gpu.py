@@ -31,6 +31,9 @@ CUT_QKV = [(64, 8, 64, 3333, 1024, 4608, (64, 64)), (48, 16, 80, 2821, 2048, 537
     (3860, 3852, 64, (256, 256)), (3860, 3852, 128, (256, 256)), (3841, 3841, 320, (256, 256)),       # one row, one column in the last tile
     (2036, 6132, 64, (256, 192)), (2036, 6132, 320, (256, 192)),
     (2036, 2040, 128, (128, 128)), (1921, 2036, 320, (128, 128)),
+    # the shortest walks that the groups in turns take (above: the kernel whose waves go together), of an even and an odd number of steps
+    (3860, 3852, 640, (256, 256)), (3841, 3841, 704, (256, 256)), (3860, 3852, 1088, (256, 256)), (3841, 3841, 1152, (256, 256)),
+    (2036, 6132, 384, (256, 192)), (2036, 6132, 704, (256, 192)), (2036, 2040, 640, (128, 128)), (1921, 2036, 704, (128, 128)),
     (1290, 11276, 1536, (256, 256)),                                       # (ten rows beyond whole tiles, beside them)
     *((m, n, k, tile) for m, n, k, tile, _, _ in CUT)])
 def test_turns_and_cut_columns(ops, m, n, k, tile):
