@@ -140,8 +140,13 @@ __device__ inline void wait_for_step(int later) {
   }
 }
 
+// What a product of few rows has to do with an RMSNorm: nothing, or it finishes one (ssq), or it prepares one (emit_g).  Each its own
+// kernel: one with both in it cost a product without a norm 0.1 to 0.4 us (8 rows, 192 x 64 2.30 us with them in it and 2.19 without, 2,048 x 5,632
+// 16.0 and 15.7).
+enum Norm : int { kNoNorm = 0, kFinishes = 1, kPrepares = 2 };
+
 // XR: rows of x a workgroup takes (blockIdx.y: which).  HALF: eight rows of w a workgroup instead of 16 (see launch_stream).
-template <int XR, int STAGES, int EPI, bool HALF = false>
+template <int XR, int STAGES, int EPI, int NORM, bool HALF = false>
 __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a) {
   constexpr int MT = (XR + 15) / 16, WP = HALF ? 1 : 2, PER = WP + XR / 8, kRing = PER * 1024;      // (WP: pieces of w a step)
   static_assert(!HALF || !paired(EPI), "half a block of a gated product would part gates and ups, of a rotated one a pair");
@@ -173,14 +178,14 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
       const bool live = row < m && gn < n_out;
       prev[j] = live ? a.out[static_cast<long>(row0 + row) * n_out + gn] : 0.f;
       bias[j] = live && a.bias != nullptr ? a.bias[gn] : 0.f;
-      gain[j] = live && a.emit_g != nullptr ? a.emit_g[gn] : 0.f;
+      if constexpr (NORM == kPrepares) gain[j] = live ? a.emit_g[gn] : 0.f;
     }
   }
   // So are a prepared x's parts of the rows' sums of squares -- sixteen chains a row, chain c adding blocks c, c + 16, ... in that order, the
   // first kAhead of them (4,096 columns) asked for together --, and a rotation's angles and the places in the cache.
   constexpr int kChains = 16, kAhead = 16;
   const int part_row = min(static_cast<int>(threadIdx.x) % XR, m - 1), chain = threadIdx.x / XR;
-  const bool sums_parts = a.ssq != nullptr && chain < kChains;
+  const bool sums_parts = NORM == kFinishes && chain < kChains;
   auto part_of = [&](int block) {
     const long at = static_cast<long>(min(block, a.ssq_blocks - 1)) * a.m + row0 + part_row;
     return a.ssq_halves ? reinterpret_cast<const float2*>(a.ssq)[at] : make_float2(a.ssq[at], 0.f);
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
         for (int t = 0; t < MT; ++t) acc[t] = mfma_16x16x4(wf[h][e], xf[t][h][e], acc[t]);
   }
 
-  __shared__ float part_sum[kChains][XR];
+  __shared__ float part_sum[NORM == kFinishes ? kChains : 1][NORM == kFinishes ? XR : 1];
   if (sums_parts) {
     float ss = 0.f;
 #pragma unroll
@@ -302,7 +307,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
   for (int j = 0; j < kItems; ++j) {
     const int idx = threadIdx.x + j * kThreads, nl = idx % kCols, row = idx / kCols, gn = n0 + nl;
     const bool live = row < m && (EPI == kRopeKv || gn < n_out);
-    if (EPI != kAccum && !live) continue;                    // (an adding product's lanes exchange sums of squares)
+    if (NORM != kPrepares && !live) continue;                // (else the lanes exchange sums of squares)
     float sum = 0.f, up = 0.f;
     if (live) {
 #pragma unroll
@@ -311,7 +316,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
 #pragma unroll
         for (int v = 0; v < kShares; ++v) up += red[v][row / 16][nl + 8][row % 16];
       }
-      if (a.ssq != nullptr) {
+      if constexpr (NORM == kFinishes) {
         float ss = 0.f;
 #pragma unroll
         for (int v = 0; v < kChains; ++v) ss += part_sum[v][row];
@@ -341,7 +346,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
     if constexpr (EPI == kAccum) {
       const float nv = prev[j] + bias[j] + sum;
       if (live) a.out[at] = nv;
-      if (a.emit_g != nullptr) {
+      if constexpr (NORM == kPrepares) {
         // the row's outputs of this workgroup lie in kCols neighbouring lanes
         float sq = live ? nv * nv : 0.f;
 #pragma unroll
@@ -365,9 +370,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
   }
 }
 
-template <int XR, int STAGES, int EPI, bool HALF = false>
+template <int XR, int STAGES, int EPI, int NORM, bool HALF = false>
 int launch_stream_form(const Args& a, hipStream_t s) {
-  auto kernel = gemm_f32_stream_kernel<XR, STAGES, EPI, HALF>;
+  auto kernel = gemm_f32_stream_kernel<XR, STAGES, EPI, NORM, HALF>;
   constexpr int kLds = kWaves * STAGES * ((HALF ? 1 : 2) + XR / 8) * 1024;
   static_assert(kLds <= 160 * 1024, "a workgroup's LDS");
   static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
@@ -384,20 +389,20 @@ int launch_stream_form(const Args& a, hipStream_t s) {
 // Outputs a workgroup of few rows' kernel takes of a product that stores or adds.
 int stream_cols(int m, int n) { return m <= 8 && 2 * ((n + 15) / 16) <= compute_units() ? 8 : 16; }
 
-template <int EPI>
+template <int EPI, int NORM = kNoNorm>
 int launch_stream(const Args& a, hipStream_t s) {
   const int cols = paired(EPI) ? 8 : 16, n_out = paired(EPI) ? a.n / 2 : a.n;
   // Outputs that would leave every other CU idle: eight a workgroup, half the weights for each CU to bring and the
   // same sums.  A decode step's two such products, 2,048 x 2,048 and
   // 2,048 x 5,632, from memory, 8 rows, inside a step: 13.05 -> 11.7 us on average; 32 steps of 8 requests after their prompts 67.6 -> 63.5 ms.
   if constexpr (!paired(EPI)) {
-    if (stream_cols(a.m, n_out) == 8) return launch_stream_form<8, 8, EPI, true>(a, s);
+    if (stream_cols(a.m, n_out) == 8) return launch_stream_form<8, 8, EPI, NORM, true>(a, s);
   }
   // One workgroup a CU where there are no more: a ring as deep as LDS allows.  Else two that overlap.
   const bool few = (n_out + cols - 1) / cols <= compute_units();
-  if (a.m <= 8) return few ? launch_stream_form<8, 6, EPI>(a, s) : launch_stream_form<8, 3, EPI>(a, s);
-  if (a.m <= 16) return few ? launch_stream_form<16, 4, EPI>(a, s) : launch_stream_form<16, 2, EPI>(a, s);
-  return few && a.m <= 32 ? launch_stream_form<32, 3, EPI>(a, s) : launch_stream_form<32, 2, EPI>(a, s);
+  if (a.m <= 8) return few ? launch_stream_form<8, 6, EPI, NORM>(a, s) : launch_stream_form<8, 3, EPI, NORM>(a, s);
+  if (a.m <= 16) return few ? launch_stream_form<16, 4, EPI, NORM>(a, s) : launch_stream_form<16, 2, EPI, NORM>(a, s);
+  return few && a.m <= 32 ? launch_stream_form<32, 3, EPI, NORM>(a, s) : launch_stream_form<32, 2, EPI, NORM>(a, s);
 }
 
 // ---- many rows ----------------------------------------------------------------------------------
@@ -629,7 +634,7 @@ extern "C" int bc4g_gemm_f32_emit(const float* x, const float* w, const float* b
   BC4G_REQUIRE(residual && g && emit_x && emit_ssq, "gemm_f32_emit: an operand is missing");
   Args a{x, w, bias, residual, m, n, k};
   a.emit_g = g, a.emit_x = emit_x, a.emit_ssq = emit_ssq;
-  if (int e = launch_stream<kAccum>(a, static_cast<hipStream_t>(stream))) return e;
+  if (int e = launch_stream<kAccum, kPrepares>(a, static_cast<hipStream_t>(stream))) return e;
   return check_launch("gemm_f32_emit");
 }
 
@@ -643,9 +648,9 @@ extern "C" int bc4g_gemm_f32_prenormed(const float* x, const float* ssq, int ssq
   hipStream_t s = static_cast<hipStream_t>(stream);
   int e = 0;
   switch (epilogue) {
-    case kStore: e = launch_stream<kStore>(a, s); break;
-    case kSwiglu: e = launch_stream<kSwiglu>(a, s); break;
-    case kGeglu: e = launch_stream<kGeglu>(a, s); break;
+    case kStore: e = launch_stream<kStore, kFinishes>(a, s); break;
+    case kSwiglu: e = launch_stream<kSwiglu, kFinishes>(a, s); break;
+    case kGeglu: e = launch_stream<kGeglu, kFinishes>(a, s); break;
     default: return fail("gemm_f32_prenormed: unknown epilogue %d", epilogue);
   }
   if (e) return e;
@@ -664,7 +669,8 @@ extern "C" int bc4g_gemm_f32_qkv(const float* x, const float* ssq, int ssq_block
   Args a{x, w, nullptr, q, m, n, k};
   a.ssq = ssq, a.ssq_blocks = ssq_blocks, a.ssq_halves = ssq_halves, a.eps = eps;
   a.rope = RopeKv{reinterpret_cast<const float2*>(table), slot_map, k_cache, v_cache, n_heads, n_kv_heads, head_dim, page_tokens, write_kv ? 1 : 0};
-  if (int e = launch_stream<kRopeKv>(a, static_cast<hipStream_t>(stream))) return e;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (int e = ssq ? launch_stream<kRopeKv, kFinishes>(a, s) : launch_stream<kRopeKv>(a, s)) return e;
   return check_launch("gemm_f32_qkv");
 }
 
