@@ -297,9 +297,21 @@ GEMM_F32_FEW_ROWS = 64               # rows up to which a float32 product prepar
 
 
 def gemm_f32_finishes_norm(n_rows: int, w) -> bool:
-    """Whether the float32 product of this weight takes a prepared norm (Prenormed) at so many rows: always, up to 64 rows of whole
-    16-byte pieces.  (Reading the parts costs the product nothing that shows: they come while its weights do.)"""
+    """Whether the float32 product of this weight can take a prepared norm (Prenormed) at so many rows: up to 64 rows of whole 16-byte pieces."""
     return getattr(w, "dtype", None) == torch.float32 and w.is_cuda and 0 < n_rows <= GEMM_F32_FEW_ROWS and w.shape[1] % 4 == 0 and w.shape[1] <= 1 << 24
+
+
+def gemm_f32_wants_prepared(n_rows: int, w) -> bool:
+    """Whether it is better served by one than by a norm kernel before it.  Every workgroup (16 rows of w, 32 of x) adds the rows' parts up
+    again: up to a workgroup a CU that costs less than the launch, beyond only for few and narrow rows.  An adding product, the norm
+    by its own kernel or prepared, and a gated product behind it, microseconds: 2,816 x 512, 8 rows 10.4 and 8.4, 32 rows 12.2 and 11.3, 64
+    (352 workgroups) 15.0 and 15.5; 11,264 x 2,048 (704 workgroups), 8 rows 32.6 and 31.9, 16 rows 35.2 and 39.2, 64 rows 72 and 81; 22,016 x
+    4,096, one row 92.7 and 97.4, 32 rows 132 and 149.  The same with a q|k|v product: 2,560 x 2,048, 16 rows 28.4 and 27.2, 64 rows 46.0 and 48.2;
+    12,288 x 4,096, 8 rows 84.7 and 88.0."""
+    if not gemm_f32_finishes_norm(n_rows, w):
+        return False
+    workgroups, cus = -(-w.shape[0] // 16) * -(-n_rows // 32), compute_units()
+    return workgroups <= cus or (n_rows <= 8 and workgroups <= 3 * cus and w.shape[1] <= 2048)
 
 
 def gemm_f32_emit(x: torch.Tensor, w, residual: torch.Tensor, g: torch.Tensor, eps: float, bias: Optional[torch.Tensor] = None) -> Optional["Prenormed"]:

@@ -118,10 +118,10 @@ class CausalAttention(Part):
 
     def wants_prepared_norm(self, n_rows: int) -> bool:
         """Whether the q|k|v product is better served by a norm that the product before prepared than by fusing
-        the norm or running it: the weight's own plan says (ops.LinearPlan.wants_prepared), and few float32 rows
-        always are."""
+        the norm or running it: the weight's own plan says (ops.LinearPlan.wants_prepared), for float32
+        rows ops.gemm_f32_wants_prepared."""
         if self.act_dtype == torch.float32:
-            return ops.gemm_f32_finishes_norm(n_rows, self.w_qkv)
+            return ops.gemm_f32_wants_prepared(n_rows, self.w_qkv)
         return self.act_dtype == torch.bfloat16 and self.w_qkv.plan.wants_prepared(n_rows)
 
     def forward(self, h, ctx, cache, residual, writes: bool = True) -> None:

@@ -52,9 +52,9 @@ class SwiGLU(Part):
     def wants_prepared_norm(self, n_rows: int) -> bool:
         """Whether the gate-up product, at this many rows, is better served by a norm that the product before
         prepared than by fusing the norm or running it: the weight's own plan says (ops.LinearPlan.wants_prepared),
-        and few float32 rows always are."""
+        for float32 rows ops.gemm_f32_wants_prepared."""
         if not self.interleaved:
-            return self.act_dtype == torch.float32 and ops.gemm_f32_finishes_norm(n_rows, self.w_gu)
+            return self.act_dtype == torch.float32 and ops.gemm_f32_wants_prepared(n_rows, self.w_gu)
         return self.w_gu.plan.wants_prepared(n_rows, swiglu=True)
 
     def forward(self, h, ctx, residual) -> None:

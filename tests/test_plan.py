@@ -84,3 +84,16 @@ def test_a_layer_in_bfloat16_runs_no_norm_for_the_32_bit_product():
         attn = CausalAttention(96, 4, 2, head_dim)
         attn.act_dtype, attn.w_qkv = dtype, torch.zeros(8 * head_dim, 96, dtype=dtype)
         assert attn._float_qkv(Normed(torch.zeros(4, 96), norm), None, None, None, None, rotary_dim, 1e4, True) is None and not ran
+
+
+def test_float32_rows_prepared_where_few_workgroups_add_the_parts_up():
+    import types
+    import torch
+    if ops.compute_units() != 256:
+        import pytest
+        pytest.skip("the line lies at the number of CUs")
+    weight = lambda n, k, dtype=torch.float32, cuda=True: types.SimpleNamespace(shape=(n, k), dtype=dtype, is_cuda=cuda)      # noqa: E731
+    wanted = lambda *w, **how: [m for m in (0, 1, 8, 9, 32, 33, 64, 65) if ops.gemm_f32_wants_prepared(m, weight(*w, **how))]      # noqa: E731
+    assert wanted(2048, 8192) == [1, 8, 9, 32, 33, 64] and wanted(2049, 64) == [1, 8, 9, 32] == wanted(4096, 8192)
+    assert wanted(4097, 2048) == [1, 8] == wanted(12288, 2048) and wanted(4097, 2052) == [] == wanted(12289, 64)
+    assert wanted(64, 64, dtype=torch.bfloat16) == [] == wanted(64, 64, cuda=False) == wanted(64, 66)
