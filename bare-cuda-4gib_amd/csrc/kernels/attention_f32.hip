@@ -257,35 +257,44 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
   struct Tile {
     floatx4 k[KB][DB], v[KB][DB];
   };
-  // Where a tile's keys and values lie is looked up for both before either is asked for: loads come back in the order asked, and a look at the
-  // block table behind the keys' loads waited for those (a decode step of 8 requests at 24 to 130 tokens: 0.4 us of 8 a layer).
-  struct Places {
-    long k[KB], v[KB];                       // (negative: not there)
+  struct Places {                            // where a tile's keys or values lie, and whether they are there
+    long at[KB];
+    bool ok[KB];
   };
-  auto places_of = [&](int j0) {
-    Places at;
+  auto key_places = [&](int j0) {
+    Places p;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      const int j = j0 + 16 * kb + c, jv = j0 + 16 * kb + 4 * g;
-      at.k[kb] = j >= lo && j <= last ? cache.key(j, 4 * g) : -1;
-      at.v[kb] = jv + 3 >= lo && jv <= last ? cache.value(jv, c) : -1;
+      const int j = j0 + 16 * kb + c;
+      p.ok[kb] = j >= lo && j <= last;
+      p.at[kb] = p.ok[kb] ? cache.key(j, 4 * g) : 0;
     }
-    return at;
+    return p;
   };
-  auto fetch_keys = [&](Tile& t, const Places& at) {
+  auto value_places = [&](int j0) {
+    Places p;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      const bool ok = at.k[kb] >= 0;
-      const float* p = a.k_cache + (ok ? at.k[kb] : 0);
+      const int j = j0 + 16 * kb + 4 * g;
+      p.ok[kb] = j + 3 >= lo && j <= last;
+      p.at[kb] = p.ok[kb] ? cache.value(j, c) : 0;
+    }
+    return p;
+  };
+  auto fetch_keys = [&](Tile& t, const Places& places) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const bool ok = places.ok[kb];
+      const float* p = a.k_cache + places.at[kb];
 #pragma unroll
       for (int b = 0; b < DB; ++b) t.k[kb][b] = ok && 16 * b + 4 * g < a.dim ? load_floats(p + 16 * b) : no_floats();
     }
   };
-  auto fetch_values = [&](Tile& t, const Places& at) {
+  auto fetch_values = [&](Tile& t, const Places& places) {
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      const bool ok = at.v[kb] >= 0;
-      const float* p = a.v_cache + (ok ? at.v[kb] : 0);
+      const bool ok = places.ok[kb];
+      const float* p = a.v_cache + places.at[kb];
 #pragma unroll
       for (int b = 0; b < DB; ++b)
         t.v[kb][b] = ok && 16 * b + c < a.dim ? load_floats(p + static_cast<long>(16 * b) * a.page_tokens) : no_floats();
@@ -294,7 +303,10 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
   int j0 = (lo / KT - lo / KT % kFewWaves + wave) * KT;                      // this wave's first tile at or after lo's
   if (j0 < lo - lo % KT) j0 += kFewWaves * KT;
   Tile cur, nxt;
-  Places at = places_of(j0);
+  // The first tile's places are looked up for both before either is asked for: loads come back in the order asked, and a look at the block table
+  // behind the keys' loads waited for those (8 requests of 100 tokens, 32 heads of 128: 8.4 -> 8.0 us).  Later tiles' are looked up as they are
+  // asked for: with both first 8 heads of 96 over three times 3,000 tokens took 109 us instead of 98, 32 of 128 over eight times 1,000 49 instead of 44.
+  const Places first_keys = key_places(j0), first_values = value_places(j0);
   floatx4 qf[DB], o[DB];
 #pragma unroll
   for (int b = 0; b < DB; ++b) {
@@ -303,17 +315,17 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
     o[b] = no_floats();
   }
   if (j0 <= last) {
-    fetch_keys(cur, at);
-    if constexpr (AHEAD) fetch_values(cur, at);
+    fetch_keys(cur, first_keys);
+    if constexpr (AHEAD) fetch_values(cur, first_values);
   }
+  bool first = true;
 
   float m = -FLT_MAX, l = 0.f;
   for (; j0 <= last; j0 += kFewWaves * KT) {
     const int next = j0 + kFewWaves * KT;
     if (AHEAD && next <= last) {
-      at = places_of(next);
-      fetch_keys(nxt, at);
-      fetch_values(nxt, at);
+      fetch_keys(nxt, key_places(next));
+      fetch_values(nxt, value_places(next));
     }
     floatx4 sc[KB];
 #pragma unroll
@@ -324,7 +336,7 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) sc[kb] = mfma_16x16x4(cur.k[kb][b][e], qf[b][e], sc[kb]);
-    if constexpr (!AHEAD) fetch_values(cur, at);
+    if constexpr (!AHEAD) fetch_values(cur, first ? first_values : value_places(j0)), first = false;
     const bool whole = j0 + KT - 1 <= ctx && (a.window <= 0 || j0 > last - a.window);
     const float alpha = softmax_tile<KB>(sc, m, l, a.scale, whole, j0, g, pos, a.window);
 #pragma unroll
@@ -371,7 +383,7 @@ __global__ __launch_bounds__(kFewWaves * kWave) void attention_f32_few_kernel(co
     }
     if (next <= last) {
       if constexpr (AHEAD) cur = nxt;
-      else at = places_of(next), fetch_keys(cur, at);
+      else fetch_keys(cur, key_places(next));
     }
   }
   l = four_lanes_sum(l);
