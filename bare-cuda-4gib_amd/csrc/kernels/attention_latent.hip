@@ -14,6 +14,8 @@
 #include <float.h>
 #include <math.h>
 
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 #include "mfma.h"
@@ -85,7 +87,7 @@ struct PrepareArgs {
 };
 
 // A row's `part`th part there is work for (a workgroup each): part 0 norms and stores the cache row, part 1 rotates the queries,
-// part 2 norms the queries' latent.  The work is the workgroup's first kPrepBlock threads', all of which it needs at its barriers.
+// part 2 norms the queries' latent.  A norm is the workgroup's first kPrepBlock threads' work, all of which it needs at its barriers.
 template <typename T>
 __device__ inline void latent_prepare_row(const PrepareArgs<T>& a, long row, int part, float* cs) {
   __shared__ float scratch[16];
@@ -116,64 +118,75 @@ __device__ inline void latent_prepare_row(const PrepareArgs<T>& a, long row, int
     const float c = cs[2 * p.angle], s = cs[2 * p.angle + 1];
     return p.second ? v * c + other * s : v * c - other * s;
   };
-  // A row is a workgroup that does little but wait, so what its threads need is asked for together, eight elements a thread at a time and
-  // the first before the angles are waited for (no condition in a load's way: elements that are not there are the first one again): 8 rows of
-  // 16 heads of 64, rank 512, 6.0 -> 4.8 us.
-  constexpr int kAhead = 8;
-  if (part_no == 1) {
+  // A row is a workgroup that does little but wait, so what its threads need is asked for together, up to eight elements a thread at a time and
+  // the first before the angles are waited for (no condition in a load's way: elements that are not there are the first one again, so there
+  // are no more loads than the row has elements for): 8 rows of 16 heads of 64, rank 512, 6.0 -> 4.8 us.
+  auto by_size = [](int n, int threads, auto&& work) {
+    if (n <= threads) work(std::integral_constant<int, 1>{});
+    else if (n <= 2 * threads) work(std::integral_constant<int, 2>{});
+    else if (n <= 4 * threads) work(std::integral_constant<int, 4>{});
+    else work(std::integral_constant<int, 8>{});
+  };
+  if (part_no == 1) {                                          // (every element by itself: all of the workgroup's threads)
     const T* qr = a.q + row * a.q_row;
     float* ql = a.q_lat + row * heads * (rank + rot);
-    const int first = works ? tid : heads * rot;
-    for (int e0 = first; e0 < heads * rot || e0 == first; e0 += kAhead * kPrepBlock) {
-      float own[kAhead], other[kAhead];
+    const int threads = blockDim.x;
+    by_size(heads * rot, threads, [&](auto ahead) {
+      constexpr int kAhead = decltype(ahead)::value;
+      for (int e0 = tid; e0 < heads * rot || e0 == tid; e0 += kAhead * threads) {
+        float own[kAhead], other[kAhead];
 #pragma unroll
-      for (int j = 0; j < kAhead; ++j) {
-        const int e = e0 + j * kPrepBlock < heads * rot ? e0 + j * kPrepBlock : 0, i = e % rot;
-        const T* part = qr + (e / rot) * (plain + rot) + plain;
-        own[j] = to_float(part[i]);
-        other[j] = to_float(part[i < dims ? pair_of(i, dims, halves).other : i]);
-      }
-      if (e0 == first) __syncthreads();                        // (every thread's first turn)
+        for (int j = 0; j < kAhead; ++j) {
+          const int e = e0 + j * threads < heads * rot ? e0 + j * threads : 0, i = e % rot;
+          const T* part = qr + (e / rot) * (plain + rot) + plain;
+          own[j] = to_float(part[i]);
+          other[j] = to_float(part[i < dims ? pair_of(i, dims, halves).other : i]);
+        }
+        if (e0 == tid) __syncthreads();                        // (every thread's first turn)
 #pragma unroll
-      for (int j = 0; j < kAhead; ++j) {
-        const int e = e0 + j * kPrepBlock;
-        if (e < heads * rot) ql[(e / rot) * (rank + rot) + rank + e % rot] = turned(e % rot, own[j], other[j]);
+        for (int j = 0; j < kAhead; ++j) {
+          const int e = e0 + j * threads;
+          if (e < heads * rot) ql[(e / rot) * (rank + rot) + rank + e % rot] = turned(e % rot, own[j], other[j]);
+        }
       }
-    }
+    });
     return;
   }
   const T* lat = a.dkv + row * a.dkv_row;
   const float* g = a.g;
   T* to = a.cache + static_cast<long>(a.slot_map[row]) * (rank + rot);
-  float held[kAhead], gain[kAhead];                            // (a latent's first 1,024 numbers)
+  by_size(rank, kPrepBlock, [&](auto ahead) {
+    constexpr int kAhead = decltype(ahead)::value;
+    float held[kAhead], gain[kAhead];                          // (a latent's first numbers: 1,024, or all of them)
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    const int i = tid + j * kPrepBlock < rank ? tid + j * kPrepBlock : 0;
-    held[j] = to_float(lat[i]);
-    gain[j] = g[i];
-  }
-  const int ri = tid < rot ? tid : 0;                          // the rotated part's first 128
-  float own = 0.f, other = 0.f;
-  if (rot > 0) own = to_float(lat[rank + ri]), other = to_float(lat[rank + (ri < dims ? pair_of(ri, dims, halves).other : ri)]);
-  float ss = 0.f;
+    for (int j = 0; j < kAhead; ++j) {
+      const int i = tid + j * kPrepBlock < rank ? tid + j * kPrepBlock : 0;
+      held[j] = to_float(lat[i]);
+      gain[j] = g[i];
+    }
+    const int ri = tid < rot ? tid : 0;                        // the rotated part's first 128
+    float own = 0.f, other = 0.f;
+    if (rot > 0) own = to_float(lat[rank + ri]), other = to_float(lat[rank + (ri < dims ? pair_of(ri, dims, halves).other : ri)]);
+    float ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j)
-    if (works && tid + j * kPrepBlock < rank) ss = fmaf(held[j], held[j], ss);
-  for (int i = works ? tid + kAhead * kPrepBlock : rank; i < rank; i += kPrepBlock) {
-    const float v = to_float(lat[i]);
-    ss = fmaf(v, v, ss);
-  }
-  const float scale = 1.0f / sqrtf(block_sum(ss, scratch) / static_cast<float>(rank) + a.eps);   // (a barrier: cs is written)
-  if (!works) return;
+    for (int j = 0; j < kAhead; ++j)
+      if (works && tid + j * kPrepBlock < rank) ss = fmaf(held[j], held[j], ss);
+    for (int i = works ? tid + kAhead * kPrepBlock : rank; i < rank; i += kPrepBlock) {
+      const float v = to_float(lat[i]);
+      ss = fmaf(v, v, ss);
+    }
+    const float scale = 1.0f / sqrtf(block_sum(ss, scratch) / static_cast<float>(rank) + a.eps);   // (a barrier: cs is written)
+    if (!works) return;
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    const int i = tid + j * kPrepBlock;
-    if (i < rank) to[i] = from_float<T>(held[j] * scale * gain[j]);
-  }
-  for (int i = tid + kAhead * kPrepBlock; i < rank; i += kPrepBlock) to[i] = from_float<T>(to_float(lat[i]) * scale * g[i]);
-  if (tid < rot) to[rank + tid] = from_float<T>(turned(tid, own, other));
-  for (int i = tid + kPrepBlock; i < rot; i += kPrepBlock)
-    to[rank + i] = from_float<T>(turned(i, to_float(lat[rank + i]), to_float(lat[rank + (i < dims ? pair_of(i, dims, halves).other : i)])));
+    for (int j = 0; j < kAhead; ++j) {
+      const int i = tid + j * kPrepBlock;
+      if (i < rank) to[i] = from_float<T>(held[j] * scale * gain[j]);
+    }
+    for (int i = tid + kAhead * kPrepBlock; i < rank; i += kPrepBlock) to[i] = from_float<T>(to_float(lat[i]) * scale * g[i]);
+    if (tid < rot) to[rank + tid] = from_float<T>(turned(tid, own, other));
+    for (int i = tid + kPrepBlock; i < rot; i += kPrepBlock)
+      to[rank + i] = from_float<T>(turned(i, to_float(lat[rank + i]), to_float(lat[rank + (i < dims ? pair_of(i, dims, halves).other : i)])));
+  });
 }
 
 template <typename T>
@@ -275,31 +288,36 @@ __device__ inline void heads_mfma_tile(const TA* __restrict__ a, long a_row, lon
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // Four of the wave's k-steps asked for together (two with many rows), without a condition: with one in each load's way a wave waited for every
-  // step's loads before it asked for the next one's (8 rows of 16 heads, k 512: 7.0 -> 5.8 us).
-  constexpr int kAhead = KW > 1 ? 4 : 2;
-  for (int k0 = 32 * wave; k0 < k; k0 += 32 * KW * kAhead) {
-    uint4 av[kAhead][MB], wv[kAhead][NB];
+  // Up to four of the wave's k-steps asked for together (two with many rows; no more than it has), without a condition: with one in each load's
+  // way a wave waited for every step's loads before it asked for the next one's (8 rows of 16 heads, k 512: 7.0 -> 5.8 us).
+  auto walk = [&](auto ahead) {
+    constexpr int kAhead = decltype(ahead)::value;
+    for (int k0 = 32 * wave; k0 < k; k0 += 32 * KW * kAhead) {
+      uint4 av[kAhead][MB], wv[kAhead][NB];
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-      const int at = k0 + 32 * KW * i + 8 * g, from = at < k ? at : 0;
+      for (int i = 0; i < kAhead; ++i) {
+        const int at = k0 + 32 * KW * i + 8 * g, from = at < k ? at : 0;
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) av[i][mb] = load_slots(arow[mb] + from);
+        for (int mb = 0; mb < MB; ++mb) av[i][mb] = load_slots(arow[mb] + from);
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) wv[i][nb] = load16(wcol[nb] + from);
-    }
+        for (int nb = 0; nb < NB; ++nb) wv[i][nb] = load16(wcol[nb] + from);
+      }
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-      if (k0 + 32 * KW * i >= k) break;
-      const bool k_there = k0 + 32 * KW * i + 8 * g < k;
+      for (int i = 0; i < kAhead; ++i) {
+        if (k0 + 32 * KW * i >= k) break;
+        const bool k_there = k0 + 32 * KW * i + 8 * g < k;
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const uint4 wi = k_there ? wv[i][nb] : zero16();
+        for (int nb = 0; nb < NB; ++nb) {
+          const uint4 wi = k_there ? wv[i][nb] : zero16();
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) acc[mb][nb] = mfma_16x16x32(k_there ? av[i][mb] : zero16(), wi, acc[mb][nb]);
+          for (int mb = 0; mb < MB; ++mb) acc[mb][nb] = mfma_16x16x32(k_there ? av[i][mb] : zero16(), wi, acc[mb][nb]);
+        }
       }
     }
-  }
+  };
+  if (k <= 32 * KW) walk(std::integral_constant<int, 1>{});
+  else if (KW == 1 || k <= 64 * KW) walk(std::integral_constant<int, 2>{});
+  else walk(std::integral_constant<int, KW == 1 ? 2 : 4>{});
   if (KW > 1) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) sums[wave][nb][lane] = acc[0][nb];
@@ -336,18 +354,18 @@ __global__ __launch_bounds__(kWave * KW) void heads_mfma_kernel(const TA* __rest
 
 // Few rows: the cache rows and the rotated queries in the launch of the absorbed queries' other part, w[h] q[t, h, :plain], which needs neither
 // (a decode step is a chain of launches that wait: 8 rows, 16 heads of 128 + 64, rank 512, 4.8 and 4.7 us one after the other).  The first
-// n_tiles * heads workgroups are the product's, the others a row's parts each.
+// `first` workgroups are a row's parts each -- a row of many heads takes the longest --, the others the product's, m_tiles * n_tiles a head.
 constexpr int kFewRows = 32;         // (up to which bc4g_heads_gemm takes this form of the product: the same bits)
-__global__ __launch_bounds__(4 * kWave) void latent_prepare_heads_kernel(const PrepareArgs<bf16_t> a, const bf16_t* __restrict__ w, int m, int m_tiles,
-                                                                         int n_tiles) {
+__global__ __launch_bounds__(4 * kWave) void latent_prepare_heads_kernel(const PrepareArgs<bf16_t> a, const bf16_t* __restrict__ w, int m, int first,
+                                                                         int m_tiles, int n_tiles) {
   extern __shared__ float cs[];
-  const int products = m_tiles * n_tiles * a.heads, block = blockIdx.x;
-  if (block < products) {
+  const int block = static_cast<int>(blockIdx.x) - first;
+  if (block >= 0) {
     const int h = block / (m_tiles * n_tiles), tile = block % (m_tiles * n_tiles), row = a.rank + a.rot;
     heads_mfma_tile<bf16_t, float, 1, 4, 1>(a.q, a.q_row, a.plain + a.rot, w, a.q_lat, static_cast<long>(a.heads) * row, row, m, a.rank, a.plain, HeadGate{}, h,
                                          tile % m_tiles * 16, tile / m_tiles * 16);
   } else {
-    latent_prepare_row(a, (block - products) % m, (block - products) / m, cs);
+    latent_prepare_row(a, blockIdx.x % m, blockIdx.x / m, cs);
   }
 }
 
@@ -498,9 +516,11 @@ extern "C" int bc4g_latent_prepare(const void* q, const void* dkv, int dtype, co
                                 heads, plain, rot, rank, dims, parts, halves, q_row, dkv_row, eps, lq};
     if (absorb) {
       const int m_tiles = ceil_div(n_rows, 16), n_tiles = ceil_div(rank, 16);
-      const long blocks = static_cast<long>(m_tiles) * n_tiles * heads + static_cast<long>(n_rows) * n_parts;
+      const int first = n_rows * n_parts;
+      const long blocks = static_cast<long>(m_tiles) * n_tiles * heads + first;
       BC4G_REQUIRE(blocks <= 2147483647L, "latent_prepare: %d heads of rank %d are beyond the grid limit", heads, rank);
-      latent_prepare_heads_kernel<<<static_cast<unsigned>(blocks), 4 * kWave, lds, s>>>(a, static_cast<const bf16_t*>(absorb), n_rows, m_tiles, n_tiles);
+      latent_prepare_heads_kernel<<<static_cast<unsigned>(blocks), 4 * kWave, lds, s>>>(a, static_cast<const bf16_t*>(absorb), n_rows, first, m_tiles,
+                                                                                               n_tiles);
     } else {
       latent_prepare_kernel<bf16_t><<<dim3(n_rows, n_parts), kPrepBlock, lds, s>>>(a);
     }
