@@ -1235,32 +1235,37 @@ int launch_halves(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& s
 // 18 % long).  A function of (m, n, k) alone; every tile adds over k in the same order.
 struct DirectForm {
   int rows, cols;
-  double us_a_step_few, us_a_step_full, us_around, us_stores;
+  double us_a_step_few, us_a_step_full, us_around, us_stores, us_qkv;
 };
 // The last, 128 x 64 with two stages and four workgroups a CU, is for the q|k|v epilogue alone: what comes after the
 // loop is long there (rotation, three destinations), and several workgroups a CU run it beside each other's loops
 // (a 2,048-token TinyLlama prompt 1 % faster with it than with 160 tiles of 256 x 128, both libraries in one process).
+// us_qkv: by how much that epilogue is longer than plain stores, a turn, from 4,500 products of 130 to 4,200 rows, 384 to 20,480 outputs (wider ones
+// are not asked: kQkvMeasured) and k 512 to 4,096, every form of each: what is chosen is 0.65 % slower on average than the fastest, 1.4 % without it.
+// 3,628 x 1,536 x 1,024 went to 180 tiles of 256 x 128, 33.4 us, where 128 x 64 takes 26.8; 2,048 x 3,072 x 1,024 31.6 and 27.4.
+constexpr int kQkvMeasured = 20480;
 constexpr int kDirectForms = 6;
-constexpr DirectForm kDirectForm[kDirectForms] = {{256, 256, 1.12, 1.48, 4.0, 2.0}, {256, 192, 1.15, 1.40, 4.0, 1.5}, {256, 128, 0.87, 1.06, 4.0, 1.5},
-                                                  {128, 128, 0.50, 0.59, 3.5, 1.0}, {64, 64, 0.25, 0.27, 3.0, 0.25},  {128, 64, 0.67, 0.36, 6.0, 0.0}};
+constexpr DirectForm kDirectForm[kDirectForms] = {
+    {256, 256, 1.12, 1.48, 4.0, 2.0, 22.5}, {256, 192, 1.15, 1.40, 4.0, 1.5, 17.5}, {256, 128, 0.87, 1.06, 4.0, 1.5, 11.0},
+    {128, 128, 0.50, 0.59, 3.5, 1.0, 5.3},  {64, 64, 0.25, 0.27, 3.0, 0.25, 3.0},   {128, 64, 0.67, 0.36, 8.5, 0.0, 2.0}};
 
-double form_time(const DirectForm& form, int m, int n, int k) {
+double form_time(const DirectForm& form, int m, int n, int k, bool qkv) {
   const long tiles = static_cast<long>((m + form.rows - 1) / form.rows) * ((n + form.cols - 1) / form.cols), cus = compute_units();
   const long full = tiles / cus;
   const double last = static_cast<double>(tiles % cus) / static_cast<double>(cus), steps = k / 64;
-  const double few = form.us_a_step_few, more = form.us_a_step_full - few;
+  const double few = form.us_a_step_few, more = form.us_a_step_full - few, stores = form.us_stores + (qkv ? form.us_qkv : 0.0);
   if (more < 0.0) {           // (several workgroups a CU)
-    const double chip = form.us_around + static_cast<double>(tiles) / static_cast<double>(cus) * steps * form.us_a_step_full, chain = 3.0 + steps * few;
-    return chip > chain ? chip : chain;
+    const double chip = static_cast<double>(tiles) / static_cast<double>(cus) * (steps * form.us_a_step_full + stores), chain = steps * few + stores;
+    return form.us_around + (chip > chain ? chip : chain);
   }
-  return form.us_around + full * (steps * (few + more) + form.us_stores) + (last > 0.0 ? steps * (few + more * last) + form.us_stores : 0.0);
+  return form.us_around + full * (steps * (few + more) + stores) + (last > 0.0 ? steps * (few + more * last) + stores : 0.0);
 }
 
-int direct_form(int m, int n, int k, bool long_epilogue) {
+int direct_form(int m, int n, int k, bool long_epilogue, bool qkv) {
   int best = 0;
   double best_time = 0.0;
   for (int f = 0; f < (long_epilogue ? kDirectForms : kDirectForms - 1); ++f) {
-    const double time = form_time(kDirectForm[f], m, n, k);
+    const double time = form_time(kDirectForm[f], m, n, k, qkv);
     if (f == 0 || time < best_time) best = f, best_time = time;
   }
   return best;
@@ -1269,13 +1274,14 @@ int direct_form(int m, int n, int k, bool long_epilogue) {
 // Rows beyond whole tiles beside them (gemm_mfma_rest_kernel): the 64 x 256 tiles' times, measured as the others' were, and the time of a launch that
 // begins with `whole` tiles of a form and goes on with `rest` such: those first go to the CUs that the last turn of large tiles leaves.  (On
 // what the chip shares a tile is a load by its size: four small ones are a 256 x 256.)
-constexpr DirectForm kRestForm = {64, 256, 0.50, 0.62, 0.0, 1.0};
-double rest_time(const DirectForm& form, int whole, int rest, int k) {
+constexpr DirectForm kRestForm = {64, 256, 0.50, 0.62, 0.0, 1.0, 2.0};
+double rest_time(const DirectForm& form, int whole, int rest, int k, bool qkv) {
   const int cus = compute_units(), steps = k / 64;
   const double load = whole + rest * static_cast<double>(kRestForm.rows * kRestForm.cols) / (form.rows * form.cols);
   const double fill = load < cus ? load / cus : 1.0;
-  const double large = steps * (form.us_a_step_few + (form.us_a_step_full - form.us_a_step_few) * fill) + form.us_stores;
-  const double small = steps * (kRestForm.us_a_step_few + (kRestForm.us_a_step_full - kRestForm.us_a_step_few) * fill) + kRestForm.us_stores;
+  const double large = steps * (form.us_a_step_few + (form.us_a_step_full - form.us_a_step_few) * fill) + form.us_stores + (qkv ? form.us_qkv : 0.0);
+  const double small = steps * (kRestForm.us_a_step_few + (kRestForm.us_a_step_full - kRestForm.us_a_step_few) * fill) + kRestForm.us_stores +
+                       (qkv ? kRestForm.us_qkv : 0.0);
   const int full = whole / cus, busy = whole % cus;
   const double early = full * large, late = busy ? (full + 1) * large : early;
   // a turn of small tiles after the other, on the CUs free early and on those free late, whichever ends first
@@ -1309,16 +1315,17 @@ struct Parts {
   bool rest;
 };
 Parts parts_of(int m, int n, int k, bool long_epilogue) {
-  Parts best{direct_form(m, n, k, long_epilogue), n, 0, false};
+  const bool qkv = long_epilogue && n <= kQkvMeasured;
+  Parts best{direct_form(m, n, k, long_epilogue, qkv), n, 0, false};
   if (k < 512) return best;
-  double best_time = 0.96 * form_time(kDirectForm[best.first], m, n, k);
+  double best_time = 0.96 * form_time(kDirectForm[best.first], m, n, k, qkv);
   for (int f = 0; f < 4; f += 3) {
     const DirectForm& form = kDirectForm[f];
     const int row_tiles = m / form.rows, beyond = m % form.rows;
     const long whole = static_cast<long>(row_tiles) * ((n + form.cols - 1) / form.cols);
     if (whole == 0 || beyond == 0 || whole > 4L * compute_units()) continue;
     const int rest = (beyond + kRestForm.rows - 1) / kRestForm.rows * ((n + kRestForm.cols - 1) / kRestForm.cols);
-    const double time = rest_time(form, static_cast<int>(whole), rest, k);
+    const double time = rest_time(form, static_cast<int>(whole), rest, k, qkv);
     if (time < best_time) best = Parts{f, n, 0, true}, best_time = time;
   }
   for (int f = 0; f < 4; ++f) {
@@ -1327,8 +1334,8 @@ Parts parts_of(int m, int n, int k, bool long_epilogue) {
     for (long turns = rows * ((n + form.cols - 1) / form.cols) / cus; turns >= 1 && rows <= turns * cus; --turns) {
       const long n1 = turns * cus / rows * form.cols;
       if (n1 <= 0 || n1 >= n) continue;
-      const int rest = n - static_cast<int>(n1), second = direct_form(m, rest, k, long_epilogue);
-      const double time = form_time(form, m, static_cast<int>(n1), k) + form_time(kDirectForm[second], m, rest, k) + kCutGap;
+      const int rest = n - static_cast<int>(n1), second = direct_form(m, rest, k, long_epilogue, qkv);
+      const double time = form_time(form, m, static_cast<int>(n1), k, qkv) + form_time(kDirectForm[second], m, rest, k, qkv) + kCutGap;
       if (time < best_time) best = Parts{f, static_cast<int>(n1), second, false}, best_time = time;
       break;      // (fewer turns of large tiles leave more for the small ones)
     }

@@ -24,7 +24,7 @@ def rnd(*shape, seed):
 
 # columns cut between two tiles: the first tile and its columns, the tile of the others
 CUT = [(1430, 11276, 1536, (256, 256), 10752, (64, 64)), (1025, 4100, 14336, (128, 128), 3584, (64, 64)), (2900, 6156, 2048, (256, 256), 5376, (128, 128))]
-CUT_QKV = [(64, 8, 64, 3333, 1024, 4608, (64, 64)), (48, 16, 80, 2821, 2048, 5376, (128, 128)), (24, 24, 128, 2055, 2048, 7168, (128, 64))]
+CUT_QKV = [(78, 13, 128, 1280, 1024, 13056, (64, 64)), (48, 16, 80, 2821, 2048, 5376, (128, 128)), (24, 24, 128, 2055, 2048, 7168, (128, 64))]
 
 
 @pytest.mark.parametrize("m,n,k,tile", [
