@@ -9,18 +9,42 @@ projection.)
 """
 from __future__ import annotations
 
+import collections
+import contextlib
 import dataclasses
+import gc
+import threading
 from typing import Hashable, List, Optional, Sequence
 
 import numpy as np
 import torch
 
-import collections
-
 from ..cache.manager import CacheManager
 from ..errors import EngineError
 from .batch import HostBatch, StepContext
 from .model import Model
+
+
+_collector = dict(lock=threading.Lock(), captures=0, was_on=False)
+
+
+@contextlib.contextmanager
+def collector_off():
+    """While any thread is inside, the cyclic garbage collector does not run.  A captured graph waits for the device when it is destroyed,
+    which is not allowed while a stream of the process is captured and, in a destructor, ends the process: a collection that happened
+    to start inside a capture and to find an engine of before, whose parts refer to each other, aborted it."""
+    with _collector["lock"]:
+        if _collector["captures"] == 0:
+            _collector["was_on"] = gc.isenabled()
+            gc.disable()
+        _collector["captures"] += 1
+    try:
+        yield
+    finally:
+        with _collector["lock"]:
+            _collector["captures"] -= 1
+            if _collector["captures"] == 0 and _collector["was_on"]:
+                gc.enable()
 
 
 @dataclasses.dataclass
@@ -331,7 +355,7 @@ class Executor:
         graph = torch.cuda.CUDAGraph()
         # (thread_local: what another thread does on the device meanwhile -- the caller of an engine whose worker
         # runs this -- neither fails there nor spoils the capture)
-        with torch.cuda.graph(graph, capture_error_mode="thread_local"):
+        with collector_off(), torch.cuda.graph(graph, capture_error_mode="thread_local"):
             logits = self.model.forward(ctx)
         ring = []
         for _ in range(4):
