@@ -755,6 +755,7 @@ def _tiled_weight(w, packed, a: Optional[torch.Tensor] = None):
 
 
 SKINNY_MAX_ROWS = 64                # rows the weight-streaming kernel takes in one launch
+NORMED_MAX_ROWS = 16                # rows whose norm that kernel can take in
 NORMED_STAGE_BYTES = 96 * 1024      # LDS the fused norm may fill with its rows of bf16(x * g)
 
 

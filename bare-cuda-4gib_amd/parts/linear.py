@@ -33,7 +33,7 @@ def absorbs_norm(norm, w, n_rows: int) -> bool:
 
 def _prepare(x: Normed, w) -> None:
     """What the product would make of the norm in each of its workgroups, by a kernel before it where that is the faster way (the same bits)."""
-    if x.pre is not None or x._tensor is not None or not ops.norm_apart(x.n_rows, w):
+    if x.n_rows > ops.NORMED_MAX_ROWS or x.pre is not None or x._tensor is not None or not ops.norm_apart(x.n_rows, w):
         return
     scale = x.fusable_scale()
     if scale is not None and ops.gemm_normed_supported(x.x, x.n_rows, scale[0], w):
