@@ -14,11 +14,13 @@
 // rows and the tile: the same bits whichever form and tile a shape selects.
 // Rows and columns beyond the matrix are not stored.
 //
-// What bounds these kernels: the loop over k is 85-90 % of a tile's time.  With all waves of a workgroup reading, waiting and
-// multiplying together (gemm_mfma_direct_kernel) the matrix cores are busy 40-50 % of it; where two groups of waves take turns, one
-// multiplying while the other reads, 60-70 %, and then it is LDS that is full (a 256 x 256 tile's step of 64 is 192 KB read and 64 KB
-// written, 2,000 clocks of the 2,048 its MFMAs take) and, over the whole chip, power: MFMAs on random operands alone run at 1,670 of
-// 2,500 TFLOP/s.  The rest is the stores after the loop, which all CUs issue at the same time.
+// What bounds these kernels: the loop over k is 85-90 % of a tile's time where k is long.  With all waves of a workgroup reading, waiting and
+// multiplying together (gemm_mfma_direct_kernel) the matrix cores are busy 37 to 39 % of a launch (hardware counters); where two groups of waves
+// take turns, one multiplying while the other reads, 64 % with many turns of 256 x 256 tiles (2,048 x 28,672 x 4,096), 48 % with
+// 256 x 192 (2,048 x 11,264 x 2,048) and 38 % with one turn of 128 x 128 (2,048 x 2,048 x 5,632).  LDS has room: a quarter of its clocks, with 1 to 3 % of
+// conflicts.  The waves spend 26 to 37 % of their time at the turns' barriers and 36 to 47 % until an instruction is done, and the whole chip's
+// power sets the clock: MFMAs on random operands alone run at 1,670 of 2,500 TFLOP/s.  The rest is the stores after the loop, which all
+// CUs issue at the same time.
 //
 // Workgroups are numbered so that those sharing rows of a and of w run on the same XCD at the same
 // time (tile_of).
@@ -752,10 +754,10 @@ __device__ inline void load_side_by_side(const void* const (&bases)[kMaxLoads], 
 }
 
 // 256 x 256: a wave's part is 128 x 64, and a step of 64 two turns: its first 64 rows by its columns, then the other 64.  So
-// a turn is 16 MFMAs, its reads 24 of 1 KB (or 8: the weight's fragments stay), and the two stages of 64 KB are written over in pieces as
+// a turn is 16 MFMAs, its reads 16 of 1 KB (or 8: the weight's fragments stay), and the two stages of 64 KB are written over in pieces as
 // they are read: the weight and the first rows of a step are asked for a step and a half before they are read, the other
 // rows as well.  LDS: a stage is the first rows of both row parts, the other rows, then the weight likewise by columns.
-// Against 16 waves that read and multiply together (weights from memory): 2,048 x 28,672 x 4,096 437 -> 384 us, 15,400 x 12,288 x 4,096
+// Against 16 waves that read and multiply together (weights from memory): 2,048 x 28,672 x 4,096 437 -> 387 us, 15,400 x 12,288 x 4,096
 // 1,440 -> 1,210 (1,040 -> 1,280 TFLOP/s), 8,192^3 960 -> 800.  Four turns of eight MFMAs a step: 3-5 % slower; four waves of 128 x 128 on
 // a SIMD each: 15-20 % slower; the waves' priority raised around the MFMAs: the same.
 struct HalvesShape {
