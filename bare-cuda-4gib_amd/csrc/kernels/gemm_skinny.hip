@@ -29,6 +29,7 @@
 //            (below), together with parts of every row's sum of squares: the row's scale is worked out
 //            from the parts while the weights are on their way and multiplies the finished sum -- the
 //            norm costs neither a kernel of its own nor the staging of the float rows.
+// Plain and prenormed rows go through rings in LDS where k is a multiple of 64 (gemm_ring_kernel, below): the same bits.
 // What goes out (EPI): bfloat16 or float stored; bfloat16 after max(., 0)^2 or xIELU (8 rows,
 // 2,048 to 8,192: product with its norm inside 13.0 us and the activation behind it 5.5; normed before and activated here 8.8);
 // float added into the residual stream; SwiGLU,
@@ -69,19 +70,24 @@ struct RopeKvArgs {
 enum XMode : int { kPlain = 0, kNormedG16 = 1, kNormedG32 = 2 };   // norm scale g in bfloat16 / float
 
 struct SkinnyArgs {
+  // (first, 64 bytes together, what the ring kernel needs before its first load: one trip for them)
   const void* x;            // bf16 [m, k], or float [*, k] in the normed modes
-  const int32_t* rows;      // normed modes: row m of the product reads x[rows[m]] (null: x[m])
-  const void* g;            // normed modes: RMSNorm scale [k]
   const bf16_t* w;          // packed: [ceil(n / 16)][ceil(k / 32)][64 lanes][8]
   void* out;
-  int m, n, k, n_out;
-  int rows_per_block;       // plain mode: blockIdx.y takes rows y * rows_per_block .. of x and out (0: all rows)
-  int m_stage;              // normed modes: rows of x staged in LDS (m rounded up to 4)
-  float eps;
   // prenormed x (plain mode): parts [ssq_blocks][ssq_stride] of the rows' sums of squares (null: x as it is)
   const float* ssq_parts;
+  int m, n, k;
+  int rows_per_block;       // plain mode: blockIdx.y takes rows y * rows_per_block .. of x and out (0: all rows)
+  int chunk;                // ring kernel: a wave's part of k,
+  int last_block;           // the last block of w,
+  int part_stride;          // numbers from one part to the next, and where the last four of all parts begin
+  int last_four;
   int ssq_blocks, ssq_stride;
   int ssq_halves;           // the parts are pairs, [ssq_blocks][ssq_stride][2]
+  float eps;
+  const int32_t* rows;      // normed modes: row m of the product reads x[rows[m]] (null: x[m])
+  const void* g;            // normed modes: RMSNorm scale [k]
+  int m_stage;              // normed modes: rows of x staged in LDS (m rounded up to 4)
   int halves;               // host: two workgroups a block (see launch)
   // kAccumF32: a number a column that joins every row's sums (null: none); kXieluBf16: the activation's two numbers
   const float* bias;
@@ -97,17 +103,12 @@ __device__ inline uint32_t pack2(float a, float b) {
   return static_cast<uint32_t>(bf16_bits_from_float(a)) | (static_cast<uint32_t>(bf16_bits_from_float(b)) << 16);
 }
 
-// MT tiles of 16 rows of x; U k-steps of 32 a batch; ROWS: 16, or 8 where there are no more rows than that (plain x: half the
-// loads and LDS writes for x); HALF: two workgroups share a weight block, each with eight of its outputs (see launch).
-template <int MT, int EPI, int XMODE, int U, int ROWS = 16, bool HALF = false>
-// (The normed form keeps to 80 registers, so that three workgroups share a CU and all the blocks of
-// a 5,632 x 2 wide gate-up matrix are in flight at once.)
-__global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) ? 6 : U == 8 ? 2 : 4) void gemm_skinny_kernel(const SkinnyArgs args) {
-  constexpr bool kNormed = XMODE != kPlain;
-  // Where the weight blocks are too few to occupy the CUs, the rows are shared out over blockIdx.y:
-  // such a workgroup sees its own rows only, as if they were the whole batch.
+// Where the weight blocks are too few to occupy the CUs, the rows are shared out over blockIdx.y (plain mode): such a workgroup sees
+// its own rows only, as if they were the whole batch.
+template <int EPI>
+__device__ inline SkinnyArgs own_rows(const SkinnyArgs& args) {
   SkinnyArgs a = args;
-  if (!kNormed && args.rows_per_block > 0) {
+  if (args.rows_per_block > 0) {
     const long row0 = static_cast<long>(blockIdx.y) * args.rows_per_block;
     a.m = min(args.rows_per_block, args.m - static_cast<int>(row0));
     a.x = static_cast<const bf16_t*>(args.x) + row0 * args.k;
@@ -124,6 +125,110 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
       a.emit_ssq = args.emit_ssq + row0;
     }
   }
+  return a;
+}
+
+// What an output's thread has at hand before its sum is there.
+struct Kept {
+  float prev, g;              // kAccumF32: what the sum is added to (with the bias), and the next norm's scale
+  float cs, sn;               // kRopeKvBf16: its pair's rotation ...
+  int slot;                   // ... and place in the cache
+  float xielu_p, xielu_q;
+};
+
+__device__ inline float emit_scale(const SkinnyArgs& a, int gn) {
+  return a.emit_g_f32 ? static_cast<const float*>(a.emit_g)[gn] : to_float(static_cast<const bf16_t*>(a.emit_g)[gn]);
+}
+
+// The rotation of a pair (its lower dimension's place in the products' columns) at a position.
+__device__ inline void pair_angle(const RopeKvArgs& r, int n0, int nl, int position, float& cs, float& sn) {
+  const int pair = (n0 % r.head_dim) / 2 + nl;            // 8 * block + nl
+  const float inv_freq = 1.0f / powf(r.theta, (2.0f * static_cast<float>(pair)) / static_cast<float>(r.head_dim));
+  sincosf(static_cast<float>(position) * inv_freq, &sn, &cs);
+}
+
+// The finished sum of output nl of the block (or half block) at n0, row `row`, goes out; `partner` is that of output nl + 8 where those belong
+// together.  in_block: the lane stands for a row and column of the block at all (the adding epilogue goes on with every lane: COLS
+// neighbouring lanes, a row's, exchange sums of squares); live: and for a column and row that there are.
+template <int EPI, int COLS, bool HALF>
+__device__ inline void put_output(const SkinnyArgs& a, int n0, int wblock_index, int half, int row, int nl, bool in_block, bool live, float sum, float partner,
+                                  const Kept& kept) {
+  const int gn = n0 + nl;
+  if constexpr (EPI == kStoreBf16) {
+    static_cast<bf16_t*>(a.out)[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(sum);
+  } else if constexpr (EPI == kSquaredReluBf16) {
+    const float z = fmaxf(sum, 0.f);
+    static_cast<bf16_t*>(a.out)[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(z * z);
+  } else if constexpr (EPI == kXieluBf16) {
+    const float z = to_float(from_float<bf16_t>(sum));       // as a kernel behind the product would find it
+    static_cast<bf16_t*>(a.out)[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(xielu_f(z, kept.xielu_p, kept.xielu_q));
+  } else if constexpr (EPI == kStoreF32) {
+    static_cast<float*>(a.out)[static_cast<long>(row) * a.n + gn] = sum;
+  } else if constexpr (EPI == kAccumF32) {
+    const float nv = kept.prev + sum;
+    if (live) static_cast<float*>(a.out)[static_cast<long>(row) * a.n + gn] = nv;
+    if (a.emit_g != nullptr) {
+      // for the RMSNorm that follows: bf16(new residual * g), and this block's part of the row's sum
+      // of squares (a row's 16 columns, or eight of half a block, lie in as many neighbouring lanes)
+      float sq = 0.f;
+      if (live) {
+        a.emit_x[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(nv * kept.g);
+        sq = nv * nv;
+      }
+#pragma unroll
+      for (int off = 1; off < COLS; off <<= 1) sq += __shfl_xor(sq, off, kWave);
+      if (nl == 0 && in_block && row < a.m && wblock_index * 16 < a.n) a.emit_ssq[(static_cast<long>(wblock_index) * a.emit_stride + row) * (HALF ? 2 : 1) + half] = sq;
+    }
+  } else if constexpr (gated(EPI)) {
+    // block b = n0 / 16 holds gates and ups of outputs 8b .. 8b + 7
+    const long o = static_cast<long>(row) * (a.n / 2) + (n0 / 2 + nl);
+    static_cast<bf16_t*>(a.out)[o] = from_float<bf16_t>((EPI == kGegluBf16 ? gelu_tanh_quick(sum) : silu_quick(sum)) * partner);
+  } else {
+    const RopeKvArgs& r = a.rope;
+    const int d = r.head_dim;
+    const int head = n0 / d, in_head = n0 % d + nl;         // the pair lies at in_head and in_head + 8
+    float lo = sum, hi = partner;
+    const bool is_v = head >= r.n_heads + r.n_kv_heads;
+    if (r.rotary_dim > 0 && !is_v) {                        // (spelt out, so that every form of the kernels rounds alike)
+      const float cs = kept.cs, sn = kept.sn, l0 = lo, h0 = hi;
+      lo = fmaf(l0, cs, -(h0 * sn));
+      hi = fmaf(h0, cs, l0 * sn);
+    }
+    if (head < r.n_heads) {
+      bf16_t* q = static_cast<bf16_t*>(a.out) + (static_cast<long>(row) * r.n_heads + head) * d + in_head;
+      q[0] = from_float<bf16_t>(lo);
+      q[8] = from_float<bf16_t>(hi);
+    } else if (r.write_kv) {
+      const int kvh = is_v ? head - r.n_heads - r.n_kv_heads : head - r.n_heads;
+      const int slot = kept.slot;
+      const long page = slot / r.page_tokens, off = slot % r.page_tokens;
+      const long region = (page * r.n_kv_heads + kvh) * d * r.page_tokens;
+      if (r.fragment_order) {
+        bf16_t* dst = (is_v ? r.v_cache : r.k_cache) + region;
+        const int o = static_cast<int>(off);
+        dst[is_v ? frag_v_offset(o, in_head, d) : frag_k_offset(o, in_head, d)] = from_float<bf16_t>(lo);
+        dst[is_v ? frag_v_offset(o, in_head + 8, d) : frag_k_offset(o, in_head + 8, d)] = from_float<bf16_t>(hi);
+      } else if (is_v) {
+        bf16_t* dst = r.v_cache + region + in_head * r.page_tokens + off;
+        dst[0] = from_float<bf16_t>(lo);
+        dst[8L * r.page_tokens] = from_float<bf16_t>(hi);
+      } else {
+        bf16_t* dst = r.k_cache + region + off * d + in_head;
+        dst[0] = from_float<bf16_t>(lo);
+        dst[8] = from_float<bf16_t>(hi);
+      }
+    }
+  }
+}
+
+// MT tiles of 16 rows of x; U k-steps of 32 a batch; ROWS: 16, or 8 where there are no more rows than that (plain x: half the
+// loads and LDS writes for x); HALF: two workgroups share a weight block, each with eight of its outputs (see launch).
+template <int MT, int EPI, int XMODE, int U, int ROWS = 16, bool HALF = false>
+// (The normed form keeps to 80 registers, so that three workgroups share a CU and all the blocks of
+// a 5,632 x 2 wide gate-up matrix are in flight at once.)
+__global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) ? 6 : U == 8 ? 2 : 4) void gemm_skinny_kernel(const SkinnyArgs args) {
+  constexpr bool kNormed = XMODE != kPlain;
+  const SkinnyArgs a = kNormed ? args : own_rows<EPI>(args);
   constexpr bool kTurned = !kNormed;                      // x reaches operand order through LDS
   constexpr int kPieces = 4 * U;                       // 16-byte pieces of a row in one batch of k-steps
   static_assert(!kNormed || MT == 1, "the fused norm handles one tile of rows");
@@ -216,9 +321,7 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
       rope_cs[j] = 1.f;
       rope_sn[j] = 0.f;
       if (live && r.rotary_dim > 0 && !is_v) {
-        const int pair = (n0 % r.head_dim) / 2 + nl;            // 8 * block + nl
-        const float inv_freq = 1.0f / powf(r.theta, (2.0f * static_cast<float>(pair)) / static_cast<float>(r.head_dim));
-        sincosf(static_cast<float>(r.positions[row]) * inv_freq, &rope_sn[j], &rope_cs[j]);
+        pair_angle(r, n0, nl, r.positions[row], rope_cs[j], rope_sn[j]);
       }
       rope_slot[j] = (live && head >= r.n_heads && r.write_kv) ? r.slot_map[row] : 0;
     }
@@ -505,78 +608,386 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
       sum *= scale;
       partner *= scale;
     }
-    if constexpr (EPI == kStoreBf16) {
-      static_cast<bf16_t*>(a.out)[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(sum);
-    } else if constexpr (EPI == kSquaredReluBf16) {
-      const float z = fmaxf(sum, 0.f);
-      static_cast<bf16_t*>(a.out)[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(z * z);
-    } else if constexpr (EPI == kXieluBf16) {
-      const float z = to_float(from_float<bf16_t>(sum));       // as a kernel behind the product would find it
-      static_cast<bf16_t*>(a.out)[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(xielu_f(z, xielu_p, xielu_q));
-    } else if constexpr (EPI == kStoreF32) {
-      static_cast<float*>(a.out)[static_cast<long>(row) * a.n + gn] = sum;
-    } else if constexpr (EPI == kAccumF32) {
-      const float nv = prev[j] + sum;
-      if (live) static_cast<float*>(a.out)[static_cast<long>(row) * a.n + gn] = nv;
-      if (a.emit_g != nullptr) {
-        // for the RMSNorm that follows: bf16(new residual * g), and this block's part of the row's sum
-        // of squares (a row's 16 columns, or eight of half a block, lie in as many neighbouring lanes)
-        float sq = 0.f;
-        if (live) {
-          const float g = a.emit_g_f32 ? static_cast<const float*>(a.emit_g)[gn]
-                                       : to_float(static_cast<const bf16_t*>(a.emit_g)[gn]);
-          a.emit_x[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(nv * g);
-          sq = nv * nv;
-        }
-#pragma unroll
-        for (int off = 1; off < kCols; off <<= 1) sq += __shfl_xor(sq, off, kWave);
-        if (nl == 0 && idx < MT * 16 * kCols && row < m) a.emit_ssq[(static_cast<long>(wblock_index) * a.emit_stride + row) * (HALF ? 2 : 1) + half] = sq;
-      }
-    } else if constexpr (gated(EPI)) {
-      // block b = n0 / 16 holds gates and ups of outputs 8b .. 8b + 7
-      const long o = static_cast<long>(row) * (a.n / 2) + (n0 / 2 + nl);
-      static_cast<bf16_t*>(a.out)[o] = from_float<bf16_t>((EPI == kGegluBf16 ? gelu_tanh_quick(sum) : silu_quick(sum)) * partner);
-    } else {
-      const RopeKvArgs& r = a.rope;
-      const int d = r.head_dim;
-      const int head = n0 / d, in_head = n0 % d + nl;         // the pair lies at in_head and in_head + 8
-      float lo = sum, hi = partner;
-      const bool is_v = head >= r.n_heads + r.n_kv_heads;
-      if (r.rotary_dim > 0 && !is_v) {
-        const float cs = rope_cs[j], sn = rope_sn[j], l0 = lo, h0 = hi;
-        lo = l0 * cs - h0 * sn;
-        hi = h0 * cs + l0 * sn;
-      }
-      if (head < r.n_heads) {
-        bf16_t* q = static_cast<bf16_t*>(a.out) + (static_cast<long>(row) * r.n_heads + head) * d + in_head;
-        q[0] = from_float<bf16_t>(lo);
-        q[8] = from_float<bf16_t>(hi);
-      } else if (r.write_kv) {
-        const int kvh = is_v ? head - r.n_heads - r.n_kv_heads : head - r.n_heads;
-        const int slot = rope_slot[j];
-        const long page = slot / r.page_tokens, off = slot % r.page_tokens;
-        const long region = (page * r.n_kv_heads + kvh) * d * r.page_tokens;
-        if (r.fragment_order) {
-          bf16_t* dst = (is_v ? r.v_cache : r.k_cache) + region;
-          const int o = static_cast<int>(off);
-          dst[is_v ? frag_v_offset(o, in_head, d) : frag_k_offset(o, in_head, d)] = from_float<bf16_t>(lo);
-          dst[is_v ? frag_v_offset(o, in_head + 8, d) : frag_k_offset(o, in_head + 8, d)] = from_float<bf16_t>(hi);
-        } else if (is_v) {
-          bf16_t* dst = r.v_cache + region + in_head * r.page_tokens + off;
-          dst[0] = from_float<bf16_t>(lo);
-          dst[8L * r.page_tokens] = from_float<bf16_t>(hi);
-        } else {
-          bf16_t* dst = r.k_cache + region + off * d + in_head;
-          dst[0] = from_float<bf16_t>(lo);
-          dst[8] = from_float<bf16_t>(hi);
-        }
-      }
-    }
+    const float g = EPI == kAccumF32 && a.emit_g != nullptr && live ? emit_scale(a, gn) : 0.f;
+    put_output<EPI, kCols, HALF>(a, n0, wblock_index, half, row, nl, idx < MT * 16 * kCols, live, sum, partner,
+                                 Kept{EPI == kAccumF32 ? prev[j] : 0.f, g, EPI == kRopeKvBf16 ? rope_cs[j] : 1.f, EPI == kRopeKvBf16 ? rope_sn[j] : 0.f,
+                                      EPI == kRopeKvBf16 ? rope_slot[j] : 0, xielu_p, xielu_q});
   }
 }
 
-constexpr int kMaxStageBytes = 96 * 1024;
+// ---- plain rows through private rings in LDS -----------------------------------------------------
+// k a multiple of 64, operands on 16-byte boundaries: the forms above with x and the weights going from memory into LDS without passing
+// registers (global_load_lds_dwordx4), in a ring of S stages that belongs to one wave -- so there is no barrier in the walk, only the wave's own
+// waits, counted by hand, and what is in flight is what LDS holds (64 to 144 KB a CU) and not what registers are left for.  A stage is KS
+// values of k: ROWS rows of x, 128 bytes each (64 with KS 32), the 16-byte pieces XOR-placed so that a fragment read meets no bank conflict, and
+// the NB blocks of the weight as they lie in memory.  As soon as a stage's fragments are in registers it is asked for again, before they are multiplied.
+// Waves, their parts of k, the MFMA and the order of the sums are those of the kernel above: the same bits.  Arithmetic in front of the first load
+// counts: 24 waves a CU share four SIMDs, and with integer divisions there an 11,264 x 2,048 product of 8 rows took 0.4 us more.
+//
+// What bounds it: a launch and the first trip to memory, 3 to 3.5 us, then the memory's rate for the weights and, with 16 rows and more, what a
+// CU pulls of x through its cache (105 to 120 bytes a ns from L2; with x turned through registers it was 65 of both together).  Weights
+// from memory, us, kernel above and this: 8 rows 2,048 x 2,048 4.39 and 4.07, 2,048 x 5,632 7.74 and 6.81, 11,264 x 2,048 10.84 and 9.90, 28,672 x 4,096
+// 41.4 and 39.3; 16 rows 2,048 x 5,632 9.18 and 7.66, 4,096 x 4,096 10.6 and 8.4, 4,096 x 11,008 26.1 and 19.0, 22,016 x 4,096 37.5 and 35.5; 32 rows
+// 4,096 x 11,008 30.1 and 23.4; 64 rows 2,048 x 2,048 6.53 and 5.95, 4,096 x 4,096 14.9 and 12.5.
+template <int ROWS, int NB, int KS, int S>
+struct RingShape {
+  static constexpr bool kHalf = NB == 0;                      // half a block: two workgroups share one
+  static constexpr int kTiles = (ROWS + 15) / 16, kBlocks = kHalf ? 1 : NB;
+  static constexpr int kXLoads = ROWS * KS / 512, kWLoads = kHalf ? KS / 64 : NB * KS / 32, kLoads = kXLoads + kWLoads;
+  static constexpr int kStageBytes = kLoads * 1024, kRingBytes = kWaves * S * kStageBytes;
+  static constexpr int kRedBytes = kWaves * kBlocks * kTiles * 16 * kRedPad * 4;
+  static constexpr int kLdsBytes = kRingBytes > kRedBytes ? kRingBytes : kRedBytes;
+  static_assert(kLdsBytes <= 152 * 1024 && S * kLoads < 64, "a workgroup's LDS beside what else it keeps there, and a wait's count");
+  static_assert((KS == 64 && ROWS % 8 == 0) || (KS == 32 && ROWS % 16 == 0), "whole loads of x");
+  static_assert(ROWS == 8 || ROWS % 16 == 0, "eight rows or whole tiles");
+};
+
+// N loads of 1 KB to N KB of LDS side by side, load i from bases[i] (the same in every lane) + off[i].
+template <int N>
+__device__ inline void ring_loads(const unsigned char* const* bases, const unsigned* off, unsigned lds_address) {
+  // (the LDS address is set once, to the middle of the stretch: the offset field reaches 4 KB either way, and moves the memory address too)
+  constexpr int kMid = N / 2;
+  const void* b[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(bases[i]) - (i - kMid) * 1024;
+    const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(bits)), hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(bits >> 32));
+    b[i] = reinterpret_cast<const void*>((static_cast<uintptr_t>(hi) << 32) | lo);
+  }
+  const unsigned mid = __builtin_amdgcn_readfirstlane(lds_address + kMid * 1024);
+#define BC4G_LOAD(v, s, o) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #o "\n\t"
+#define BC4G_RING(loads, ...) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" loads ::"s"(mid), __VA_ARGS__ : "memory", "m0")
+  if constexpr (N == 1) BC4G_RING(BC4G_LOAD(1, 2, 0), "v"(off[0]), "s"(b[0]));
+  else if constexpr (N == 2) BC4G_RING(BC4G_LOAD(1, 3, -1024) BC4G_LOAD(2, 4, 0), "v"(off[0]), "v"(off[1]), "s"(b[0]), "s"(b[1]));
+  else if constexpr (N == 3)
+    BC4G_RING(BC4G_LOAD(1, 4, -1024) BC4G_LOAD(2, 5, 0) BC4G_LOAD(3, 6, 1024), "v"(off[0]), "v"(off[1]), "v"(off[2]), "s"(b[0]), "s"(b[1]), "s"(b[2]));
+  else {
+    static_assert(N == 4, "loads a statement");
+    BC4G_RING(BC4G_LOAD(1, 5, -2048) BC4G_LOAD(2, 6, -1024) BC4G_LOAD(3, 7, 0) BC4G_LOAD(4, 8, 1024), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]),
+              "s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3]));
+  }
+#undef BC4G_RING
+#undef BC4G_LOAD
+}
+
+// Lane i's 4 bytes to lds_address + 4 i.
+__device__ inline void load_to_lds_4(const void* global, unsigned lds_address) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(global), "s"(lds_address) : "memory", "m0");
+}
+
+// Until all but the loads of the last `later` stages of LOADS (MOST such at most) have come; no access to LDS moves over it.
+template <int LOADS, int MOST>
+__device__ inline void ring_wait(int later) {
+  if constexpr (MOST == 0) {
+    asm volatile("" ::: "memory");
+    wait_loads<0>();
+    asm volatile("" ::: "memory");
+  } else if (later >= MOST) {
+    asm volatile("" ::: "memory");
+    wait_loads<LOADS * MOST>();
+    asm volatile("" ::: "memory");
+  } else {
+    ring_wait<LOADS, MOST - 1>(later);
+  }
+}
+
+template <int EPI, int ROWS, int NB, int KS, int S>
+__global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs args) {
+  typedef RingShape<ROWS, NB, KS, S> P;
+  constexpr bool kHalf = P::kHalf, kPaired = gated(EPI) || EPI == kRopeKvBf16;
+  static_assert(!kHalf || (ROWS <= 16 && !kPaired), "half blocks: few rows, unpaired outputs");
+  constexpr int TM = P::kTiles, TB = P::kBlocks, kSteps = KS / 32, kPartSums = 8;
+  extern __shared__ __align__(1024) unsigned char ring_lds[];
+  __shared__ float part_sum[kPartSums][ROWS];
+  __shared__ int places[EPI == kRopeKvBf16 ? kWaves : 1][2][kWave];          // positions and cache slots, every wave's own
+  const SkinnyArgs a = own_rows<EPI>(args);
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int col = lane % 16, grp = lane / 16;
+  const int m = a.m, k = a.k;
+  const int first_block = kHalf ? blockIdx.x / 2 : blockIdx.x * TB, half = kHalf ? blockIdx.x % 2 : 0;
+
+  // Item j of a thread is output nl of block b and row `row` of number threadIdx.x + j * kThreads.  What it needs beside its sum is asked for before the
+  // operands and used after the walk.  (Little arithmetic before the first operands: with 24 waves a CU every instruction of it is 40 clocks.)
+  constexpr int kCols = kPaired || kHalf ? 8 : 16, kAll = TB * TM * 16 * kCols, kItems = (kAll + kThreads - 1) / kThreads;
+  auto item = [&](int j, int& nl, int& b, int& row) {
+    const int idx = threadIdx.x + j * kThreads;
+    nl = idx % kCols, b = idx / kCols % TB, row = idx / (kCols * TB);
+    return idx < kAll;
+  };
+  float prev[kItems], bias[kItems];
+  typedef uint32_t uint32_any __attribute__((aligned(2)));
+  uint32_t g[kItems];
+  float cs[kItems], sn[kItems];
+  int slot[kItems];
+  if constexpr (EPI == kAccumF32) {
+    // (every load is made, from a place that there is, whether it is needed or not: behind a branch the compiler waits for it)
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      int nl, b, row;
+      item(j, nl, b, row);
+      const unsigned gn = min((first_block + b) * 16 + 8 * half + nl, a.n - 1), at = min(row, m - 1) * a.n + gn;
+      prev[j] = static_cast<const float*>(a.out)[at];
+      bias[j] = (a.bias != nullptr ? a.bias : static_cast<const float*>(a.out))[gn];
+      // (of a bfloat16 scale the column's and the one before it; the first column's and the one after)
+      const unsigned char* scale = static_cast<const unsigned char*>(a.emit_g != nullptr ? a.emit_g : a.out);
+      g[j] = *reinterpret_cast<const uint32_any*>(scale + (a.emit_g_f32 ? 4 * gn : 2 * max(gn, 1u) - 2));
+    }
+  }
+  if constexpr (EPI == kRopeKvBf16) {
+    auto lds_address = [](const void* p) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const unsigned char*)p)); };
+    if (a.rope.rotary_dim > 0) load_to_lds_4(a.rope.positions + min(lane, m - 1), lds_address(&places[wave][0][0]));
+    if (a.rope.write_kv) load_to_lds_4(a.rope.slot_map + min(lane, m - 1), lds_address(&places[wave][1][0]));
+  }
+
+  // prenormed x: wave j adds up chain j of every row's parts, parts j, j + 8, ... in ascending order.  A part's numbers of ROWS rows (pairs of
+  // them, where half blocks left it) lie side by side: four of them a lane, 2^shift lanes a part, up to 256 parts (128 pairs) asked for before the walk.
+  // (Past the last part or number: the last four, turned into place after the walk.)
+  constexpr int kHeld = ROWS <= 8 ? 1 : ROWS / 8;
+  typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
+  const bool prenormed = EPI != kAccumF32 && a.ssq_parts != nullptr, pairs = ROWS == 8 && a.ssq_halves;
+  const int shift = ROWS == 8 ? 1 + a.ssq_halves : ROWS == 16 ? 2 : 3, parts_a_load = kWave >> shift;
+  const int part_stride = a.part_stride;
+  const int first_row = a.rows_per_block > 0 ? static_cast<int>(blockIdx.y) * a.rows_per_block : 0, last_four = a.last_four - first_row;
+  auto part_at = [&](int h) {
+    return min(wave + kPartSums * (h * parts_a_load + (lane >> shift)), a.ssq_blocks - 1) * part_stride + (lane & ((1 << shift) - 1)) * 4;
+  };
+  floatx4 held[kHeld];
+  if constexpr (EPI != kAccumF32) {
+    const float* parts = prenormed ? a.ssq_parts : static_cast<const float*>(a.x);
+#pragma unroll
+    for (int h = 0; h < kHeld; ++h) held[h] = *reinterpret_cast<const floatx4_any*>(parts + static_cast<unsigned>(prenormed ? min(part_at(h), last_four) : 0));
+  }
+
+  // this wave's part of k, and where its lanes' bytes of a stage come from
+  const int k_begin = wave * a.chunk, steps = max(0, min(k - k_begin, a.chunk)) / static_cast<unsigned>(KS);
+  const unsigned char* mine = ring_lds + wave * (S * P::kStageBytes);
+  const unsigned ring = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const unsigned char*)mine));
+  constexpr int kRowBytes = KS * 2, kPieces = KS / 8, kLoadRows = kWave / kPieces;
+  auto key = [](int row) { return KS == 64 ? (row >> 1) & 7 : (row >> 2) & 3; };      // piece p of a row lies at p ^ key
+  unsigned x_off[P::kXLoads], w_off[P::kWLoads];
+#pragma unroll
+  for (int i = 0; i < P::kXLoads; ++i) {
+    const int row = i * kLoadRows + lane / kPieces;                                    // (rows past m: the last)
+    x_off[i] = static_cast<unsigned>(min(row, m - 1)) * k * 2 + ((lane % kPieces) ^ key(row)) * 16;
+  }
+  // (half a block: its eight rows' 16 bytes of four k-slots side by side, 128 bytes each, of two k-steps a load)
+#pragma unroll
+  for (int i = 0; i < P::kWLoads; ++i) w_off[i] = kHalf ? lane / 32 * 1024 + lane % 32 / 8 * 256 + (8 * half + lane % 8) * 16 : lane * 16;
+  const unsigned char* w_at[TB];
+#pragma unroll
+  for (int b = 0; b < TB; ++b)
+    w_at[b] = reinterpret_cast<const unsigned char*>(a.w) + (static_cast<size_t>(min(first_block + b, a.last_block)) * (static_cast<unsigned>(k) / 32) + static_cast<unsigned>(k_begin) / 32) * 1024;
+  const unsigned char* x_at = static_cast<const unsigned char*>(a.x) + static_cast<unsigned>(k_begin) * 2;
+  auto ask = [&](int t) {
+    const unsigned to = ring + (t % S) * P::kStageBytes;
+    const unsigned char *xs[P::kXLoads], *ws[P::kWLoads];
+#pragma unroll
+    for (int i = 0; i < P::kWLoads; ++i)
+      ws[i] = (kHalf ? w_at[0] + i * 2048 : w_at[i / kSteps] + i % kSteps * 1024) + static_cast<size_t>(t) * (kSteps * 1024);
+#pragma unroll
+    for (int i = 0; i < P::kXLoads; ++i) xs[i] = x_at + static_cast<size_t>(t) * kRowBytes;
+    ring_loads<P::kWLoads>(ws, w_off, to);
+    ring_loads<P::kXLoads>(xs, x_off, to + P::kWLoads * 1024);
+  };
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < steps) ask(s);
+
+  floatx4 acc[TM][TB];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int b = 0; b < TB; ++b) acc[i][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // (while the operands are on their way)
+  float xielu_p = 0.f, xielu_q = 0.f;
+  if constexpr (EPI == kXieluBf16) xielu_p = softplus_f(a.bias[0]), xielu_q = 0.5f + softplus_f(a.bias[1]);
+  if constexpr (EPI == kRopeKvBf16) {
+    ring_wait<P::kLoads, S>(min(S, steps));
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      int nl, b, row;
+      const bool in_block = item(j, nl, b, row);
+      const int n0 = (first_block + b) * 16, head = n0 / a.rope.head_dim;
+      const bool live = in_block && row < m && n0 < a.n;
+      cs[j] = 1.f, sn[j] = 0.f;
+      if (live && a.rope.rotary_dim > 0 && head < a.rope.n_heads + a.rope.n_kv_heads) pair_angle(a.rope, n0, nl, places[wave][0][row], cs[j], sn[j]);
+      slot[j] = live && head >= a.rope.n_heads && a.rope.write_kv ? places[wave][1][row] : 0;
+    }
+  }
+
+  auto wait_lds_reads = []() { __builtin_amdgcn_s_waitcnt(63 >> 4 << 14 | 0 << 8 | 7 << 4 | 15); };      // lgkmcnt(0)
+  const int read_row = ROWS == 8 ? col % 8 : col;
+  for (int t = 0; t < steps; ++t) {
+    ring_wait<P::kLoads, S - 1>(min(steps - 1 - t, S - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    const unsigned char* stage = mine + (t % S) * P::kStageBytes;
+    uint4 fx[kSteps][TM], fw[kSteps][TB];
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+#pragma unroll
+      for (int b = 0; b < TB; ++b) fw[u][b] = load16(kHalf ? stage + u * 512 + grp * 128 + col % 8 * 16 : stage + (b * kSteps + u) * 1024 + lane * 16);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fx[u][i] = load16(stage + P::kWLoads * 1024 + (i * 16 + read_row) * kRowBytes + ((u * 4 + grp) ^ key(read_row)) * 16);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    wait_lds_reads();                         // in registers: the stage may be written over
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + S < steps) ask(t + S);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int b = 0; b < TB; ++b) acc[i][b] = mfma_16x16x32(fw[u][b], fx[u][i], acc[i][b]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  if (prenormed) {
+    // through the wave's own ring, which is free; a part that is not there adds 0
+    unsigned char* own = ring_lds + wave * (S * P::kStageBytes);
+#pragma unroll
+    for (int h = 0; h < kHeld; ++h) {
+      floatx4 v = held[h];
+      if (part_stride < first_row + (pairs ? 2 * ROWS : ROWS)) {                          // (only then a load of the last parts may end past them)
+        const int turn = max(0, part_at(h) - last_four);
+        if (turn & 1) v = floatx4{v[1], v[2], v[3], v[3]};
+        if (turn & 2) v = floatx4{v[2], v[3], v[3], v[3]};
+      }
+      if (wave + kPartSums * (h * parts_a_load + (lane >> shift)) >= a.ssq_blocks) v = floatx4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<floatx4*>(own + (h * kWave + lane) * 16) = v;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int row = lane % ROWS, in_chain = (a.ssq_blocks - wave + kPartSums - 1) / kPartSums;
+    float ss = 0.f;
+    if (pairs) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float2 one = *reinterpret_cast<const float2*>(own + (i * ROWS + row) * 8);
+        ss += one.x + one.y;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ss += *reinterpret_cast<const float*>(own + (i * ROWS + row) * 4);
+      if (in_chain > 16) {
+#pragma unroll
+        for (int i = 16; i < 32; ++i) ss += *reinterpret_cast<const float*>(own + (i * ROWS + row) * 4);
+      }
+    }
+    for (int i = pairs ? 16 : 32; i < in_chain; ++i) {
+      const float* p = a.ssq_parts + static_cast<long>(wave + kPartSums * i) * part_stride + (pairs ? 2 : 1) * min(row, m - 1);
+      ss += pairs ? p[0] + p[1] : p[0];
+    }
+    if (lane < ROWS) part_sum[wave][row] = ss;
+  }
+  __syncthreads();                            // the partial sums take the rings' place
+  typedef float Red[TB][TM][16][kRedPad];
+  Red* red = reinterpret_cast<Red*>(ring_lds);
+#pragma unroll
+  for (int b = 0; b < TB; ++b)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave][b][i][4 * grp + r][col] = acc[i][b][r];
+  __syncthreads();
+
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    int nl, b, row;
+    const bool in_block = item(j, nl, b, row);
+    const int n0 = (first_block + b) * 16 + 8 * half;
+    const bool live = in_block && row < m && n0 + nl < a.n;
+    if (EPI != kAccumF32 && !live) continue;            // (the adding epilogue goes on with every lane)
+    float sum = 0.f, partner = 0.f;
+    if (live) {
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v) sum += red[v][b][row / 16][nl][row % 16];
+      if constexpr (kPaired) {
+#pragma unroll
+        for (int v = 0; v < kWaves; ++v) partner += red[v][b][row / 16][nl + 8][row % 16];
+      }
+      if (prenormed) {
+        float ssq = 0.f;
+#pragma unroll
+        for (int c = 0; c < kPartSums; ++c) ssq += part_sum[c][row];
+        const float scale = 1.0f / sqrtf(ssq / static_cast<float>(k) + a.eps);
+        sum *= scale;
+        partner *= scale;
+      }
+    }
+    Kept kept{0.f, 0.f, 1.f, 0.f, 0, xielu_p, xielu_q};
+    if constexpr (EPI == kAccumF32) {
+      asm volatile("" : "+v"(prev[j]), "+v"(bias[j]), "+v"(g[j]));            // (nothing done with them before the walk, where it would wait for them)
+      kept.prev = a.bias != nullptr ? prev[j] + bias[j] : prev[j];
+      kept.g = __uint_as_float(a.emit_g_f32 ? g[j] : n0 + nl > 0 ? g[j] & 0xffff0000u : g[j] << 16);
+    }
+    if constexpr (EPI == kRopeKvBf16) kept.cs = cs[j], kept.sn = sn[j], kept.slot = slot[j];
+    put_output<EPI, kCols, kHalf>(a, n0, first_block + b, half, row, nl, in_block, live, sum, partner, kept);
+  }
+}
+
+template <int EPI, int ROWS, int NB, int KS, int S>
+int launch_ring(const SkinnyArgs& a, int row_groups, hipStream_t s) {
+  typedef RingShape<ROWS, NB, KS, S> P;
+  auto kernel = gemm_ring_kernel<EPI, ROWS, NB, KS, S>;
+  static bool raised = false;
+  if (!raised) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, P::kLdsBytes) != hipSuccess)
+      return fail("gemm_skinny: cannot raise the dynamic LDS limit");
+    raised = true;
+  }
+  const int blocks = (a.n + 15) / 16;
+  const dim3 grid(P::kHalf ? 2 * blocks : (blocks + NB - 1) / NB, row_groups);
+  SkinnyArgs b = a;
+  b.rows_per_block = row_groups > 1 ? (a.m + row_groups - 1) / row_groups : 0;
+  b.chunk = (a.k + kWaves * 64 - 1) / (kWaves * 64) * 64;
+  b.last_block = blocks - 1;
+  b.part_stride = a.ssq_stride * (a.ssq_halves ? 2 : 1);
+  b.last_four = a.ssq_blocks * b.part_stride - 4;
+  kernel<<<grid, dim3(kThreads), P::kLdsBytes, s>>>(b);
+  return check_launch("gemm_skinny");
+}
+
 constexpr int kSplitMinRows = 8;
+
+// Which rows a workgroup takes, how many blocks of outputs, and how deep its rings are: by what was measured for 1 to 64 rows, outputs of 2,048 to 28,672
+// and k of 2,048 to 11,008 (us, weights from memory).  With at most a workgroup a CU the rings fill LDS; with more of them, two or three share a CU
+// (11,264 x 2,048, 8 rows: rings of two stages 9.90, of four 11.7; 28,672 x 4,096: of three 39.3, of four 41.9).  More than eight rows go to two
+// workgroups where the blocks are at most half the CUs: each pulls half of x, and the weight comes once more from L2 (16 rows 2,048 x 5,632
+// 7.7 and 9.2; but 2,560 x 2,048 5.3 and 5.0).  Wider outputs of 16 rows and more take two or three blocks a workgroup, which so reads x once for all of them
+// (32 rows 11,264 x 2,048: three blocks 12.6, one 13.9; 64 rows 4,096 x 11,008: two 28.5, one 35.6 and above).
+template <int EPI>
+int launch_rings(const SkinnyArgs& a, hipStream_t s) {
+  const int blocks = (a.n + 15) / 16, cus = compute_units();
+  if (a.m <= kSplitMinRows) {
+    if constexpr (EPI == kAccumF32 || EPI == kStoreF32 || EPI == kStoreBf16)
+      if (a.halves) return launch_ring<EPI, 8, 0, 64, 4>(a, 1, s);
+    if (blocks <= cus) return launch_ring<EPI, 8, 1, 64, 4>(a, 1, s);
+    return a.k < 4096 ? launch_ring<EPI, 8, 1, 64, 2>(a, 1, s) : launch_ring<EPI, 8, 1, 64, 3>(a, 1, s);
+  }
+  if (a.m <= 16) {
+    if (2 * blocks <= cus) return launch_ring<EPI, 8, 1, 64, 4>(a, 2, s);
+    if (blocks <= cus) return launch_ring<EPI, 16, 1, 64, 4>(a, 1, s);
+    return 2 * blocks <= 3 * cus ? launch_ring<EPI, 16, 2, 64, 3>(a, 1, s) : launch_ring<EPI, 16, 1, 64, 2>(a, 1, s);
+  }
+  if (a.m <= 32) {
+    if (2 * blocks <= cus) return launch_ring<EPI, 16, 1, 64, 4>(a, 2, s);
+    if (blocks <= cus) return launch_ring<EPI, 32, 1, 64, 3>(a, 1, s);
+    return blocks <= 2 * cus ? launch_ring<EPI, 32, 2, 64, 2>(a, 1, s) : launch_ring<EPI, 32, 3, 32, 2>(a, 1, s);
+  }
+  if (2 * blocks <= cus) return launch_ring<EPI, 32, 1, 64, 3>(a, 2, s);
+  return blocks <= cus ? launch_ring<EPI, 32, 2, 64, 2>(a, 2, s) : launch_ring<EPI, 32, 3, 32, 2>(a, 2, s);
+}
+
+// What the rings take: the loads bring 16 bytes from 16-byte boundaries, a stage is 64 values of k, parts of a norm are read four numbers at a time and the
+// next norm's scale two.
+bool ring_operands(const SkinnyArgs& a) {
+  return a.k % 64 == 0 && (a.ssq_parts == nullptr || static_cast<long>(a.ssq_blocks) * a.ssq_stride >= 4) && (a.emit_g == nullptr || a.n > 1) && reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0;
+}
+
+constexpr int kMaxStageBytes = 96 * 1024;
 
 template <int EPI, int XMODE>
 int launch(const SkinnyArgs& a, hipStream_t s) {
@@ -596,6 +1007,8 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
     }
     kernel<<<grid, block, stage, s>>>(a);
   } else {
+    if (ring_operands(a)) return launch_rings<EPI>(a, s);
+    // (From here on k that is no multiple of 64, or operands off 16-byte boundaries.)
     // Every workgroup reads all its rows of x, and what a CU can pull through its cache is what bounds
     // the kernel once x is as large as the block's weights (16 rows).  Where the weight blocks are
     // few (up to one a CU: n = 4,096), two workgroups share a block's rows: each pulls half of
@@ -659,7 +1072,6 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
 
 template <int XMODE>
 int launch_epilogue(SkinnyArgs& a, int epilogue, hipStream_t s) {
-  a.n_out = a.n;
   switch (epilogue) {
     case kStoreBf16: return launch<kStoreBf16, XMODE>(a, s);
     case kStoreF32: return launch<kStoreF32, XMODE>(a, s);
@@ -709,7 +1121,6 @@ SkinnyArgs plain_args(const void* x, const void* w, void* out, int m, int n, int
   a.m = m;
   a.n = n;
   a.k = k;
-  a.n_out = n;
   return a;
 }
 
@@ -789,7 +1200,7 @@ extern "C" int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts,
   a.ssq_parts = ssq_parts;
   a.ssq_blocks = ssq_blocks;
   a.ssq_stride = ssq_stride;
-  a.ssq_halves = ssq_halves;
+  a.ssq_halves = ssq_halves ? 1 : 0;
   a.eps = eps;
   return launch_epilogue<kPlain>(a, epilogue, static_cast<hipStream_t>(stream));
 }
@@ -842,7 +1253,7 @@ extern "C" int bc4g_gemm_skinny_qkv(const void* x, const void* g, int g_dtype, f
   a.ssq_parts = ssq_parts;
   a.ssq_blocks = ssq_blocks;
   a.ssq_stride = ssq_stride;
-  a.ssq_halves = ssq_halves;
+  a.ssq_halves = ssq_halves ? 1 : 0;
   if (!g) return launch<kRopeKvBf16, kPlain>(a, s);
   if (g_dtype == kBF16) return launch<kRopeKvBf16, kNormedG16>(a, s);
   if (g_dtype == kF32) return launch<kRopeKvBf16, kNormedG32>(a, s);

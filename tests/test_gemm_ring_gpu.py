@@ -1,0 +1,95 @@
+"""The few-row product through rings in LDS against the streaming kernel, which takes the same operands where x lies off a 16-byte
+boundary: the same bits from either, at the edges of the row counts, blocks of outputs and parts of k that a workgroup and its waves take."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+ROWS = [1, 2, 8, 9, 15, 16, 17, 31, 32, 33, 48, 64]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from bare_cuda_4gib_amd.csrc import ops as _ops
+    return _ops
+
+
+def off_by_eight(x):
+    """x at an address that is 8 bytes past a boundary of 16."""
+    room = torch.empty(x.numel() + 4, dtype=x.dtype, device=x.device)
+    room[4:] = x.reshape(-1)
+    return room[4:].view(x.shape)
+
+
+def operands(ops, m, n, k, seed=0):
+    torch.manual_seed(seed + m)
+    return torch.randn(m, k, device=DEV).bfloat16(), ops.StreamedWeight((torch.randn(n, k, device=DEV) * k ** -0.5).bfloat16())
+
+
+# outputs of a few blocks, of fewer than half the CUs, of fewer than all, of one and a half and two a CU and beyond, ragged; k of one step, of fewer
+# and more steps than waves, of parts shorter than a ring and longer
+@pytest.mark.parametrize("n, k", [(16, 64), (1000, 448), (2048, 1088), (2040, 5632), (3648, 2048), (6144, 576), (8184, 2560), (11264, 192)])
+@pytest.mark.parametrize("m", ROWS)
+def test_stored_and_added(ops, m, n, k):
+    x, w = operands(ops, m, n, k)
+    if not ops.streams_weights(m, n, k):
+        pytest.skip("goes to the tiled kernel")
+    bias, base = torch.randn(n, device=DEV), torch.randn(m, n, device=DEV)
+    other = off_by_eight(x)
+    got = ops.gemm_fast(x, w, torch.float32)
+    want = x.double() @ w.rows.double().T
+    assert (got.double() - want).abs().max() < 4 * k ** 0.5 * 2.0 ** -24 * (x.double().abs() @ w.rows.double().abs().T).max()
+    assert torch.equal(got, ops.gemm_fast(other, w, torch.float32))
+    assert torch.equal(ops.gemm_fast(x, w, torch.bfloat16), ops.gemm_fast(other, w, torch.bfloat16))
+    assert torch.equal(ops.gemm_fast(x, w, torch.bfloat16, squared_relu=True), ops.gemm_fast(other, w, torch.bfloat16, squared_relu=True))
+    for b in (None, bias):
+        assert torch.equal(ops.gemm_fast(x, w, accumulate_into=base.clone(), bias=b), ops.gemm_fast(other, w, accumulate_into=base.clone(), bias=b))
+    if n % 16 == 0:
+        for act in ("silu", "gelu_tanh"):
+            assert torch.equal(ops.gemm_swiglu(x, w, True, act), ops.gemm_swiglu(other, w, True, act))
+
+
+@pytest.mark.parametrize("g_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n, k", [(64, 64), (2048, 1024), (1000, 1024), (4096, 320), (6400, 128)])
+@pytest.mark.parametrize("m", ROWS)
+def test_norms_prepared_and_finished(ops, m, n, k, g_dtype):
+    """Parts of whole blocks and of half blocks, of one block (a norm kernel's), of up to 256 blocks and beyond."""
+    x, w = operands(ops, m, n, k)
+    g, base, bias = (1 + 0.1 * torch.randn(n, device=DEV)).to(g_dtype), torch.randn(m, n, device=DEV), torch.randn(n, device=DEV)
+    made = []
+    for a in (x, off_by_eight(x)):
+        res = base.clone()
+        made.append((res, ops.gemm_accumulate_emit(a, w, res, g, 1e-5, bias=bias)))
+    (res, pre), (res2, pre2) = made
+    assert torch.equal(res, res2) and torch.equal(pre.xb, pre2.xb) and torch.equal(pre.parts, pre2.parts)
+    if n % 64:
+        return
+    after = ops.StreamedWeight((torch.randn(1600, n, device=DEV) * n ** -0.5).bfloat16())
+    pq = torch.tensor([0.3, 0.2], device=DEV)
+    one_part = ops.rmsnorm_prepare(res, None, m, g, 1e-5)
+    for left in (pre, one_part):
+        shifted = ops.Prenormed(off_by_eight(left.xb), left.parts, left.eps)
+        for epilogue in (ops.EPI_STORE_BF16, ops.EPI_STORE_F32, ops.EPI_SWIGLU, ops.EPI_SQUARED_RELU):
+            assert torch.equal(ops.gemm_prenormed(left, after, epilogue), ops.gemm_prenormed(shifted, after, epilogue))
+        if left.parts.dim() == 2:
+            assert torch.equal(ops.gemm_xielu(left.xb, after, pq, pre=left), ops.gemm_xielu(shifted.xb, after, pq, pre=shifted))
+
+
+@pytest.mark.parametrize("heads, kv_heads, head_dim, page", [(4, 2, 16, 16), (32, 4, 64, 64), (32, 8, 128, 64), (48, 48, 64, 24)])
+@pytest.mark.parametrize("m", ROWS)
+def test_rotated_and_cached(ops, m, heads, kv_heads, head_dim, page):
+    n, k = (heads + 2 * kv_heads) * head_dim, 768
+    x, w = operands(ops, m, n, k)
+    pos = torch.randint(0, 4000, (m,), dtype=torch.int32, device=DEV)
+    slots = torch.randperm(8 * page, device=DEV)[:m].to(torch.int32)
+    made = []
+    for a in (x, off_by_eight(x)):
+        kc, vc = torch.zeros(8, kv_heads, page, head_dim, dtype=torch.bfloat16, device=DEV), torch.zeros(8, kv_heads, head_dim, page, dtype=torch.bfloat16, device=DEV)
+        q = ops.gemm_qkv_rope(a, None, 0.0, w, pos, slots, kc, vc, heads, kv_heads, head_dim, head_dim, 1e4)
+        plain = ops.gemm_qkv_rope(a, None, 0.0, w, pos, None, None, None, heads, kv_heads, head_dim, 0, 1e4, write_kv=False)
+        made.append((q, kc, vc, plain))
+    assert all(torch.equal(one, other) for one, other in zip(*made))
+    want = (x.float() @ w.rows[:heads * head_dim].float().T)
+    assert (made[0][3].float() - want).abs().max() < 2.0 ** -8 * want.abs().max()
