@@ -24,8 +24,9 @@
 // Decoded tokens bring few tiles and long key walks: there a workgroup is one tile and its WS
 // waves cut the tile's keys between them, then combine their partial results in LDS (in wave
 // order).  On top of that, with n_splits > 1 the key range is cut into that many parts over
-// workgroups (grid z); each part writes unnormalized float partials, and
-// attention_merge_kernel combines them.
+// workgroups (grid z); each part writes unnormalized float partials, and the part that ends last
+// combines them (a counter a tile says which that is: nobody waits for anybody) -- or, without
+// counters, attention_merge_kernel does.
 //
 // A row reads keys max(0, p - window + 1) .. p only.  Keys beyond the tile's last position may
 // never have been written: their scores are replaced by -inf and their values by zero, so that
@@ -109,9 +110,17 @@ struct AttnArgs {
   const int32_t* items;        // prompt form with a work list: workgroup y takes piece items[y] % 2^20, part (items[y] >> 20) % 16 of
                                // items[y] >> 24 parts of that piece's keys (nullptr: the grid's x is the piece, z the part of n_splits)
   const int32_t* row_parts;    // with items: into how many parts each row's keys were cut ([T]; 1: the row is written as it is)
+  uint32_t* arrived;           // decode form: a counter a (tile, head group), zero: the part that ends last merges (nullptr: a kernel behind this one)
   int single_rows;             // every request brings exactly one row (a decode step): request s is tile s and row s
   float scale_log2;            // softmax scale times log2(e)
 };
+
+// Partial results that another workgroup of the same launch reads, maybe on another XCD: past the L2s on both sides (stores that write
+// through, loads that miss), so that neither side has to write back or throw away a whole cache.  By themselves they order nothing:
+// the writer waits for its stores (wait_stores) before it counts itself, the reader comes after the count.
+__device__ inline void store_through(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline float load_through(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // DJ: k-steps of 32 over head_dim for the scores; DB: blocks of 16 output dimensions; QT: 16-row
 // query tiles per wave (consecutive tokens), which share every key and value fragment the wave
@@ -614,12 +623,58 @@ __global__ __launch_bounds__((WS > 1 ? WS : kWavesPerBlock) * kWave, 2) void att
         a.out[(row * a.n_heads + head) * d + c] = from_float<bf16_t>(acc / l);
       } else {
         const long slot = (static_cast<long>(part) * a.n_tokens + row) * a.n_heads + head;
-        a.part_o[slot * d + c] = acc;
+        store_through(a.part_o + slot * d + c, acc);
         if (c == 0) {
-          a.part_ml[slot * 2] = m;
-          a.part_ml[slot * 2 + 1] = l;
+          store_through(a.part_ml + slot * 2, m);
+          store_through(a.part_ml + slot * 2 + 1, l);
         }
       }
+    }
+    if (a.n_splits == 1 || a.arrived == nullptr) return;
+
+    // The part of this tile that ends last adds the parts up, in order of z and by the merge kernels' own steps: the same bits whichever
+    // it is.  (The counter goes back to zero by itself, for the next layer.)  Against a merge kernel behind this one: see launch.
+    int* is_last = reinterpret_cast<int*>(merge_raw);          // (everybody has read what lay there)
+    wait_stores();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const unsigned last = static_cast<unsigned>(a.n_splits) - 1;
+      *is_last = atomicInc(a.arrived + static_cast<long>(tile) * gridDim.y + head_block, last) == last;
+    }
+    __syncthreads();
+    if (*is_last == 0) return;
+    const long rows_heads = static_cast<long>(a.n_tokens) * a.n_heads;
+    for (int idx = threadIdx.x; idx < 16 * d; idx += WS * kWave) {
+      const int r = idx / d, c = idx % d;
+      const int r_tok = r / a.hg, r_head_in_group = hsub * a.hg + r % a.hg;
+      if (r_tok >= a.tpt || r_tok >= ntok || r_head_in_group >= group) continue;
+      const long rh = (row0 + tok0 + r_tok) * a.n_heads + kvh * group + r_head_in_group;
+      constexpr int kAhead = 8;                 // parts asked for together
+      float mz[kAhead], lz[kAhead], oz[kAhead];
+      auto ask = [&](int z0) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          const long slot = static_cast<long>(min(z0 + i, a.n_splits - 1)) * rows_heads + rh;
+          mz[i] = load_through(a.part_ml + slot * 2);
+          lz[i] = load_through(a.part_ml + slot * 2 + 1);
+          oz[i] = load_through(a.part_o + slot * d + c);
+        }
+      };
+      ask(0);
+      float m = -INFINITY, l = 0.f, acc = 0.f;
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) m = fmaxf(m, mz[i]);
+      for (int z = kAhead; z < a.n_splits; ++z) m = fmaxf(m, load_through(a.part_ml + (z * rows_heads + rh) * 2));
+      for (int z0 = 0; z0 < a.n_splits; z0 += kAhead) {
+        if (z0 > 0) ask(z0);
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          const float wz = z0 + i >= a.n_splits || mz[i] == -INFINITY ? 0.f : exp2f(mz[i] - m);
+          l += wz * lz[i];
+          acc += wz * oz[i];
+        }
+      }
+      a.out[rh * d + c] = from_float<bf16_t>(acc * (1.0f / l));
     }
     return;
   }
@@ -793,13 +848,13 @@ int launch_attention(const AttnArgs& a, dim3 grid, dim3 block, size_t lds, hipSt
 }  // namespace
 }  // namespace bc4g
 
-extern "C" int bc4g_attention_mfma(const void* qkv, int q_stride, void* out, float* part_o, float* part_ml, const void* k_cache,
+extern "C" int bc4g_attention_mfma_counted(const void* qkv, int q_stride, void* out, float* part_o, float* part_ml, const void* k_cache,
                                    const void* v_cache, const int32_t* block_table, int table_stride,
                                    const int32_t* seq_start, const int32_t* seq_ctx, const int32_t* tile_start,
                                    int n_seqs, int n_tiles, int n_tokens, int n_heads, int n_kv_heads, int head_dim,
                                    int page_tokens, int window, float scale, int tokens_per_tile, int q_tiles,
                                    int form, int n_splits, const int32_t* items, int n_items, const int32_t* row_parts,
-                                   int single_rows, const int32_t* row_seq, void* stream) {
+                                   int single_rows, const int32_t* row_seq, int32_t* arrived, int n_arrived, void* stream) {
   BC4G_REQUIRE(n_heads > 0 && n_kv_heads > 0 && n_heads % n_kv_heads == 0, "attention_mfma: bad heads %d/%d",
                n_heads, n_kv_heads);
   BC4G_REQUIRE(head_dim >= 16 && head_dim <= 256 && head_dim % 16 == 0,
@@ -845,6 +900,9 @@ extern "C" int bc4g_attention_mfma(const void* qkv, int q_stride, void* out, flo
   a.items = items;
   a.row_parts = items ? row_parts : nullptr;
   a.single_rows = single_rows ? 1 : 0;
+  a.arrived = form == 1 && n_splits > 1 ? reinterpret_cast<uint32_t*>(arrived) : nullptr;
+  BC4G_REQUIRE(a.arrived == nullptr || static_cast<long>(n_tiles) * n_kv_heads * a.n_sub <= n_arrived,
+               "attention_mfma: %d counters are fewer than %d tiles times %d groups of heads", n_arrived, n_tiles, n_kv_heads * a.n_sub);
   BC4G_REQUIRE(!single_rows || (form == 1 && n_tiles == n_seqs && n_tokens == n_seqs),
                "attention_mfma: single rows means one row and one tile a request in the decode form (%d requests, %d "
                "tiles, %d rows)", n_seqs, n_tiles, n_tokens);
@@ -899,7 +957,7 @@ extern "C" int bc4g_attention_mfma(const void* qkv, int q_stride, void* out, flo
   }
   if (status) return status;
   if (int e = check_launch("attention_mfma")) return e;
-  if (n_splits > 1) {
+  if (n_splits > 1 && a.arrived == nullptr) {
     const long rows_heads = static_cast<long>(n_tokens) * n_heads;
     BC4G_REQUIRE(rows_heads <= 2147483647L, "attention_mfma: too many rows to merge");
     constexpr int kFew = 8;
@@ -915,4 +973,16 @@ extern "C" int bc4g_attention_mfma(const void* qkv, int q_stride, void* out, flo
     return check_launch("attention_merge");
   }
   return 0;
+}
+
+extern "C" int bc4g_attention_mfma(const void* qkv, int q_stride, void* out, float* part_o, float* part_ml, const void* k_cache,
+                                   const void* v_cache, const int32_t* block_table, int table_stride,
+                                   const int32_t* seq_start, const int32_t* seq_ctx, const int32_t* tile_start,
+                                   int n_seqs, int n_tiles, int n_tokens, int n_heads, int n_kv_heads, int head_dim,
+                                   int page_tokens, int window, float scale, int tokens_per_tile, int q_tiles,
+                                   int form, int n_splits, const int32_t* items, int n_items, const int32_t* row_parts,
+                                   int single_rows, const int32_t* row_seq, void* stream) {
+  return bc4g_attention_mfma_counted(qkv, q_stride, out, part_o, part_ml, k_cache, v_cache, block_table, table_stride, seq_start, seq_ctx, tile_start,
+                                     n_seqs, n_tiles, n_tokens, n_heads, n_kv_heads, head_dim, page_tokens, window, scale, tokens_per_tile, q_tiles,
+                                     form, n_splits, items, n_items, row_parts, single_rows, row_seq, nullptr, 0, stream);
 }

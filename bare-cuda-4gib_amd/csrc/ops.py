@@ -1363,7 +1363,7 @@ def attention_mfma(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                    n_splits: int, q_tiles: int = 1, form: int = 0, work=None,
                    out: Optional[torch.Tensor] = None, row_seq: Optional[torch.Tensor] = None,
                    single_rows: bool = False, items: Optional[torch.Tensor] = None, n_items: int = 0,
-                   row_parts: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   row_parts: Optional[torch.Tensor] = None, arrived: Optional[torch.Tensor] = None) -> torch.Tensor:
     """form 0: four independent waves a workgroup, tile_start counts pieces of q_tiles tiles; 1: one
     tile a workgroup, its waves share the keys (q_tiles 1); 2: four waves a workgroup that walk their
     keys together through LDS, tile_start counts pieces of 4 * q_tiles tiles (ATTENTION_STAGED_WAVES).
@@ -1373,7 +1373,9 @@ def attention_mfma(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     step), and the kernel then looks nothing up before it asks for the block table and the query.
     ``items`` (form 2; prompt_work_list): a work list of n_items workgroups in the order in which they
     are to start, each a piece, a part and the number of parts of that piece's keys; ``row_parts`` [T]:
-    into how many parts each row's keys are cut; n_splits is then the most parts of any piece."""
+    into how many parts each row's keys are cut; n_splits is then the most parts of any piece.
+    ``arrived`` (form 1): zeros, one int32 a tile and group of heads (attention_counters): the part of a tile's keys that ends last adds
+    the parts up, and no merge kernel follows (the same bits)."""
     _dev("attention_mfma", qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start)
     t = qkv.shape[0]
     _check_queries("attention_mfma", qkv, n_heads, n_kv_heads, head_dim)
@@ -1398,12 +1400,12 @@ def attention_mfma(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         _i32("attention_mfma", "items", items, n_items)
         _i32("attention_mfma", "row_parts", row_parts, t)
     _launch_attention_mfma(qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start, n_tiles, n_heads, n_kv_heads, head_dim, window,
-                           scale, n_splits, q_tiles, form, work, out, row_seq, single_rows, items, n_items, row_parts)
+                           scale, n_splits, q_tiles, form, work, out, row_seq, single_rows, items, n_items, row_parts, arrived)
     return out
 
 
 def _launch_attention_mfma(qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start, n_tiles, n_heads, n_kv_heads, head_dim, window, scale,
-                           n_splits, q_tiles, form, work, out, row_seq=None, single_rows=False, items=None, n_items=0, row_parts=None) -> None:
+                           n_splits, q_tiles, form, work, out, row_seq=None, single_rows=False, items=None, n_items=0, row_parts=None, arrived=None) -> None:
     """attention_mfma for operands that have been looked at."""
     t, n_seqs = qkv.shape[0], block_table.shape[0]
     parts = part_ml = None
@@ -1411,12 +1413,15 @@ def _launch_attention_mfma(qkv, k_cache, v_cache, block_table, seq_start, seq_ct
         walks = n_splits * t * n_heads
         parts = torch.empty(walks * (head_dim + 2), dtype=torch.float32, device=qkv.device)
         part_ml = parts.data_ptr() + 4 * walks * head_dim
-    library.call("bc4g_attention_mfma", _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(parts), part_ml, _ptr(k_cache),
+    if arrived is not None:
+        _dev("attention_mfma", arrived)
+        _i32("attention_mfma", "arrived", arrived, arrived.numel())
+    library.call("bc4g_attention_mfma_counted", _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(parts), part_ml, _ptr(k_cache),
                  _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(seq_start), _ptr(seq_ctx),
                  _ptr(tile_start), n_seqs, n_tiles, t, n_heads, n_kv_heads, head_dim, k_cache.shape[2],
                  int(window), float(scale), attention_tile_tokens(n_heads, n_kv_heads), int(q_tiles),
                  int(form), int(n_splits), _ptr(items), int(n_items), _ptr(row_parts), 1 if single_rows else 0,
-                 _ptr(row_seq), _stream(), cost=work)
+                 _ptr(row_seq), _ptr(arrived), arrived.numel() if arrived is not None else 0, _stream(), cost=work)
 
 
 _DECODE_TILE_STARTS: dict = {}
@@ -1456,6 +1461,13 @@ def prompt_work_list(batch, piece_starts, piece: int, head_blocks: int, window: 
     return [it[1] for it in items], row_parts, most
 
 
+def attention_counters(n_tiles: int, n_heads: int, n_kv_heads: int) -> Dict[str, List[int]]:
+    """The decode form's counters (see attention_mfma) for so many tiles, where their keys may be cut at all: zeros that go up with every step's
+    batch, so that they are the step's own and zero before it."""
+    n = n_tiles * n_kv_heads * -(-(n_heads // n_kv_heads) // 16)
+    return {"arrived": [0] * n} if 0 < 2 * n <= ATTENTION_ENOUGH_GROUPS else {}
+
+
 def attention_plan(batch, n_heads: int, n_kv_heads: int, head_dim: int, window: int = 0):
     """What the matrix-core attention kernel needs to know about a batch before it is launched, worked
     out on the host when the batch is described (``batch``: the step's HostBatch): how every request's
@@ -1473,8 +1485,9 @@ def attention_plan(batch, n_heads: int, n_kv_heads: int, head_dim: int, window: 
             tiles = _DECODE_TILE_STARTS.get(S)
             if tiles is None:
                 tiles = _DECODE_TILE_STARTS[S] = list(range(S + 1))
-            return {"tiles": tiles}, dict(form="decode", n_tiles=S)
-        return {"tiles": list(range(S + 1))}, dict(form="decode", n_tiles=S)
+        else:
+            tiles = list(range(S + 1))
+        return dict(tiles=tiles, **attention_counters(S, n_heads, n_kv_heads)), dict(form="decode", n_tiles=S)
     piece = tpt * attention_q_tiles(head_dim) * ATTENTION_STAGED_WAVES
     new = [start[s + 1] - start[s] for s in range(S)]
     short = [s for s in range(S) if new[s] <= tpt]
@@ -1493,7 +1506,7 @@ def attention_plan(batch, n_heads: int, n_kv_heads: int, head_dim: int, window: 
             arrays.update(items=items, row_parts=row_parts)
             notes.update(n_items=len(items), most_parts=most)
     if apart:
-        arrays["short_tiles"] = short_starts
+        arrays.update(short_tiles=short_starts, **attention_counters(short_starts[-1], n_heads, n_kv_heads))
         longest = max(batch.seq_ctx[s] for s in short) + tpt
         notes.update(n_short=short_starts[-1],
                      short_splits=attention_splits(short_starts[-1], n_heads, n_kv_heads, longest, attention_shared_waves(head_dim)))
@@ -1518,7 +1531,7 @@ def attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
             n_tiles = notes["n_tiles"]
             n_splits = attention_splits(n_tiles, n_heads, n_kv_heads, ctx.max_kv_len, attention_shared_waves(head_dim))
             return attention_mfma(*args, arrays["tiles"], n_tiles, *sizes, n_splits, 1, 1, work=work,
-                                  single_rows=ctx.max_q_len == 1 and ctx.n_tokens == ctx.n_seqs)
+                                  single_rows=ctx.max_q_len == 1 and ctx.n_tokens == ctx.n_seqs, arrived=arrays.get("arrived"))
         q_tiles = attention_q_tiles(head_dim)
         apart = notes["apart"]
         if "items" in arrays:       # the pieces' parts in the order the host chose, longest walks first
@@ -1533,7 +1546,8 @@ def attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
             # (the tensors of the launch before, the piece starts aside)
             _dev("attention", arrays["short_tiles"])
             _i32("attention", "short_tiles", arrays["short_tiles"], ctx.n_seqs + 1)
-            _launch_attention_mfma(*args, arrays["short_tiles"], notes["n_short"], *sizes, notes["short_splits"], 1, 1, None, out, ctx.row_seq)
+            _launch_attention_mfma(*args, arrays["short_tiles"], notes["n_short"], *sizes, notes["short_splits"], 1, 1, None, out, ctx.row_seq,
+                                   arrived=arrays.get("arrived"))
         return out
     if ctx.n_seqs <= 65535 and attention_f32_takes(qkv, k_cache, v_cache, head_dim):
         return attention_f32(qkv, k_cache, v_cache, block_table, ctx, n_heads, n_kv_heads, head_dim, window, scale, work=work)
