@@ -83,6 +83,7 @@ struct RopeKvArgs {
   bf16_t* v_cache;            // [pages, n_kv, d, page_tokens], or likewise
   int n_heads, n_kv_heads, head_dim, page_tokens, write_kv;
   int fragment_order;         // how the cache's pages are laid out (cache_fragment_order)
+  unsigned per_head, per_page;         // for division by head_dim and page_tokens (reciprocal_of)
 };
 
 // Which tile a workgroup takes.  Workgroups are dealt to the 8 XCDs in turn, each with an L2 of its
@@ -133,12 +134,7 @@ __device__ inline void store_patch(const float* patch, void* __restrict__ out, i
       }
       bf16_t* dst = static_cast<bf16_t*>(out) + gm * n_out + (gn / 16) * 8;
       if (n_out % 8 == 0) {
-        uint4 pk;
-        pk.x = static_cast<uint32_t>(bf16_bits_from_float(v[0])) | (static_cast<uint32_t>(bf16_bits_from_float(v[1])) << 16);
-        pk.y = static_cast<uint32_t>(bf16_bits_from_float(v[2])) | (static_cast<uint32_t>(bf16_bits_from_float(v[3])) << 16);
-        pk.z = static_cast<uint32_t>(bf16_bits_from_float(v[4])) | (static_cast<uint32_t>(bf16_bits_from_float(v[5])) << 16);
-        pk.w = static_cast<uint32_t>(bf16_bits_from_float(v[6])) | (static_cast<uint32_t>(bf16_bits_from_float(v[7])) << 16);
-        *reinterpret_cast<uint4*>(dst) = pk;
+        *reinterpret_cast<uint4*>(dst) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) dst[e] = from_float<bf16_t>(v[e]);
@@ -156,12 +152,8 @@ __device__ inline void store_patch(const float* patch, void* __restrict__ out, i
 #pragma unroll
         for (int e = 0; e < 4; ++e) v0[e] = squared_relu(v0[e]), v1[e] = squared_relu(v1[e]);
       }
-      uint4 pk;
-      pk.x = static_cast<uint32_t>(bf16_bits_from_float(v0[0])) | (static_cast<uint32_t>(bf16_bits_from_float(v0[1])) << 16);
-      pk.y = static_cast<uint32_t>(bf16_bits_from_float(v0[2])) | (static_cast<uint32_t>(bf16_bits_from_float(v0[3])) << 16);
-      pk.z = static_cast<uint32_t>(bf16_bits_from_float(v1[0])) | (static_cast<uint32_t>(bf16_bits_from_float(v1[1])) << 16);
-      pk.w = static_cast<uint32_t>(bf16_bits_from_float(v1[2])) | (static_cast<uint32_t>(bf16_bits_from_float(v1[3])) << 16);
-      *reinterpret_cast<uint4*>(static_cast<bf16_t*>(out) + gm * n + gn) = pk;
+      *reinterpret_cast<uint4*>(static_cast<bf16_t*>(out) + gm * n + gn) =
+          make_uint4(pack_bf16x2(v0[0], v0[1]), pack_bf16x2(v0[2], v0[3]), pack_bf16x2(v1[0], v1[1]), pack_bf16x2(v1[2], v1[3]));
     }
   } else {
     const bool vec = n % 4 == 0;
@@ -207,100 +199,130 @@ __device__ inline void store_patch(const float* patch, void* __restrict__ out, i
   }
 }
 
-// The q|k|v epilogue: THREADS threads take ROWS x COLS floats (stride COLS + 4) from LDS, eight neighbouring columns a
-// thread -- a block's eight dimensions, or their eight partners -- rotate them with what lies eight columns away in
-// the patch, and store queries to out [m, n_heads * head_dim], keys and values into their pages.
-template <int THREADS, int ROWS, int COLS>
-__device__ inline void store_patch_rope(const float* patch, bf16_t* __restrict__ out, int m, int n, long m0, long n0, int tid,
-                                        const RopeKvArgs& ra) {
-  constexpr int kStride = COLS + 4;
-  const int d = ra.head_dim;
-  if (ra.fragment_order && n0 >= static_cast<long>(ra.n_heads + ra.n_kv_heads) * d) {
+// x / by and what remains, x below 2^31, by a number prepared on the host, R = floor((2^32 - 1) / by): a true division by a number known at run
+// time only is 25 instructions, of 64 bits over a hundred.  (R > 2^32 / by - 1 - 1 / by, so x R / 2^32 > x / by - 1: short by one at most.)
+inline unsigned reciprocal_of(unsigned by) { return 0xffffffffu / by; }
+__device__ inline int divide(int x, int by, unsigned reciprocal, int& rest) {
+  unsigned q = __umulhi(static_cast<unsigned>(x), reciprocal), r = static_cast<unsigned>(x) - q * by;
+  if (r >= static_cast<unsigned>(by)) r -= by, ++q;
+  rest = static_cast<int>(r);
+  return static_cast<int>(q);
+}
+
+// Where a patch's 32 rows go in the cache, a row a lane (and again in the upper lanes): the part of a key's or value's place that its row gives
+// -- the rest comes from its column --, and from which rows on four consecutive tokens lie side by side in fragment order, a bit a row.
+struct RowPlaces {
+  long key, value;
+  unsigned long long quads;
+};
+__device__ inline RowPlaces row_places(int slot, const RopeKvArgs& ra) {
+  int off;
+  const long page = divide(slot, ra.page_tokens, ra.per_page, off), first = page * ra.n_kv_heads * ra.page_tokens * ra.head_dim;
+  RowPlaces r;
+  r.key = first + (ra.fragment_order ? frag_k_offset(off, 0, ra.head_dim) : static_cast<long>(off) * ra.head_dim);
+  r.value = first + (ra.fragment_order ? frag_v_offset(off, 0, ra.head_dim) : static_cast<long>(off));
+  const bool follow = __shfl_down(slot, 1, kWave) == slot + 1 && __shfl_down(slot, 2, kWave) == slot + 2 && __shfl_down(slot, 3, kWave) == slot + 3;
+  r.quads = __ballot(ra.fragment_order && slot % 4 == 0 && follow);
+  return r;
+}
+__device__ inline long from_row(long v, int row) {
+  const unsigned lo = __shfl(static_cast<unsigned>(v), row, kWave), hi = __shfl(static_cast<unsigned>(v >> 32), row, kWave);
+  return static_cast<long>((static_cast<unsigned long>(hi) << 32) | lo);
+}
+
+// The q|k|v epilogue: a wave takes 32 x COLS floats (stride COLS + 4) from LDS, eight neighbouring columns a lane -- a block's eight
+// dimensions, or their eight partners --, rotates them with what lies eight columns away in the patch, and stores queries to out
+// [m, n_heads * head_dim], keys and values into their pages.  What bounds it is the chain of a lane's items and the vector ALU: with every
+// item's place looked up and divided out by itself a tile of keys and values was 2 to 10 us longer than one of queries, and the product with it (us, weights
+// from memory, before and now): 268 x 2,560 x 2,048 11.4 and 10.5, 1,000 23.8 and 20.5, 4,096 58 and 51; 2,048 x 6,144 x 4,096 104 and
+// 99.5; 2,048 x 12,288 x 4,096 211 and 196, 4,096 363 and 323 (a plain store 184 and 310).
+template <int COLS>
+__device__ inline void store_patch_rope(const float* patch, bf16_t* __restrict__ out, int m, int n, long m0, long n0, int lane,
+                                        const RopeKvArgs& ra, const RowPlaces& places) {
+  constexpr int kRows = 32, kStride = COLS + 4;
+  const int d = ra.head_dim, first_row = static_cast<int>(m0), first_col = static_cast<int>(n0);
+  const long per_head = static_cast<long>(ra.page_tokens) * d;
+  if (ra.fragment_order && first_col >= (ra.n_heads + ra.n_kv_heads) * d) {
     // A patch of value columns only, for a cache in fragment order, where four consecutive tokens of one dimension
-    // lie side by side: a thread takes one column of four rows, and where those four tokens' places are four in a
+    // lie side by side: a lane takes one column of four rows, and where those four tokens' places are four in a
     // row from a multiple of four on (a prompt portion's usually are) it stores them at once.
-    static_assert(ROWS % 4 == 0, "rows in fours");
-    for (int c = tid; c < (ROWS / 4) * COLS; c += THREADS) {
-      const int col = c % COLS, row = (c / COLS) * 4;
-      const long gm = m0 + row, gn = n0 + col;
-      if (gm >= m || gn >= n) continue;
-      const int head = static_cast<int>(gn / d) - ra.n_heads - ra.n_kv_heads, dim = static_cast<int>(gn % d);
-      const int rows = static_cast<int>(min(4L, m - gm));
-      int slot[4];
-      uint16_t bits[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        slot[e] = e < rows ? ra.slot_map[gm + e] : -1;
-        bits[e] = bf16_bits_from_float(patch[(row + e) * kStride + col]);
-      }
-      if (rows == 4 && slot[0] % 4 == 0 && slot[1] == slot[0] + 1 && slot[2] == slot[0] + 2 && slot[3] == slot[0] + 3) {
-        const long page = slot[0] / ra.page_tokens;
-        const int off = slot[0] % ra.page_tokens;
-        bf16_t* region = ra.v_cache + (page * ra.n_kv_heads + head) * static_cast<long>(d) * ra.page_tokens;
-        uint2 pk;
-        pk.x = static_cast<uint32_t>(bits[0]) | (static_cast<uint32_t>(bits[1]) << 16);
-        pk.y = static_cast<uint32_t>(bits[2]) | (static_cast<uint32_t>(bits[3]) << 16);
-        *reinterpret_cast<uint2*>(region + frag_v_offset(off, dim, d)) = pk;
+    for (int it = 0; it < kRows / 4 * COLS / kWave; ++it) {
+      const int c = lane + it * kWave, col = c % COLS, row = (c / COLS) * 4;
+      const int gm = first_row + row, gn = first_col + col;
+      int dim;
+      const int head = divide(min(gn, n - 1), d, ra.per_head, dim) - ra.n_heads - ra.n_kv_heads;
+      const long column = head * per_head + (dim / 16) * 256 + (dim % 16) * 4;          // (frag_v_offset's share of the dimension)
+      const float* mine = patch + row * kStride + col;
+      const uint2 pk = make_uint2(pack_bf16x2(mine[0], mine[kStride]), pack_bf16x2(mine[2 * kStride], mine[3 * kStride]));
+      const long at = from_row(places.value, row) + column;
+      if (__all(gm + 3 < m && (places.quads >> row & 1))) {        // (the lanes together: what a lane asks of another is asked by all)
+        if (gn < n) *reinterpret_cast<uint2*>(ra.v_cache + at) = pk;
       } else {
-        for (int e = 0; e < rows; ++e) {
-          const long page = slot[e] / ra.page_tokens;
-          const int off = slot[e] % ra.page_tokens;
-          bf16_t* region = ra.v_cache + (page * ra.n_kv_heads + head) * static_cast<long>(d) * ra.page_tokens;
-          region[frag_v_offset(off, dim, d)].bits = bits[e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const long to = e == 0 ? at : from_row(places.value, row + e) + column;
+          if (gm + e < m && gn < n) ra.v_cache[to].bits = static_cast<uint16_t>(e % 2 ? (e < 2 ? pk.x : pk.y) >> 16 : (e < 2 ? pk.x : pk.y));
         }
       }
     }
     return;
   }
-  for (int c = tid; c < ROWS * (COLS / 8); c += THREADS) {
-    const int row = c / (COLS / 8), col = (c % (COLS / 8)) * 8;
-    const long gm = m0 + row, gn = n0 + col;
-    if (gm >= m || gn >= n) continue;
-    const int head = static_cast<int>(gn / d), dim = static_cast<int>(gn % d);
-    const bool is_q = head < ra.n_heads, is_v = head >= ra.n_heads + ra.n_kv_heads;
-    if (!is_q && !ra.write_kv) continue;
-    float v[8];
-    {
-      const floatx4 v0 = *reinterpret_cast<const floatx4*>(patch + row * kStride + col);
-      const floatx4 v1 = *reinterpret_cast<const floatx4*>(patch + row * kStride + col + 4);
+  const bool caches = ra.write_kv && first_col + COLS > ra.n_heads * d;
+  constexpr int kItems = kRows * (COLS / 8) / kWave, kTogether = kItems % 2 ? 1 : 2;       // items of a lane; whose angles are asked for together
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = v0[e], v[4 + e] = v1[e];
-    }
-    if (ra.table != nullptr && !is_v) {
-      const bool first = dim % 16 < 8;                       // a block's eight first halves of pairs; their partners lie 8 further
-      const float* partner = patch + row * kStride + (first ? col + 8 : col - 8);
-      const floatx4 o0 = *reinterpret_cast<const floatx4*>(partner), o1 = *reinterpret_cast<const floatx4*>(partner + 4);
-      const floatx4* cs = reinterpret_cast<const floatx4*>(ra.table + gm * (d / 2) + (dim / 16) * 8);   // (cos, sin) of two pairs each
+  for (int i0 = 0; i0 < kItems; i0 += kTogether) {
+    int row[kTogether], col[kTogether], head[kTogether], dim[kTogether];
+    floatx4 cs[kTogether][4];                                  // (cos, sin) of two pairs each
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const floatx4 a = cs[e];
-        const float p0 = e < 2 ? o0[2 * e] : o1[2 * e - 4], p1 = e < 2 ? o0[2 * e + 1] : o1[2 * e - 3];
-        v[2 * e] = first ? v[2 * e] * a[0] - p0 * a[1] : v[2 * e] * a[0] + p0 * a[1];
-        v[2 * e + 1] = first ? v[2 * e + 1] * a[2] - p1 * a[3] : v[2 * e + 1] * a[2] + p1 * a[3];
+    for (int u = 0; u < kTogether; ++u) {
+      const int c = lane + (i0 + u) * kWave;
+      row[u] = c / (COLS / 8), col[u] = c % (COLS / 8) * 8;
+      head[u] = divide(min(first_col + col[u], n - 8), d, ra.per_head, dim[u]);
+      if (ra.table != nullptr) {
+        const floatx4* from = reinterpret_cast<const floatx4*>(ra.table + static_cast<long>(min(first_row + row[u], m - 1)) * (d / 2) + (dim[u] / 16) * 8);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cs[u][e] = from[e];
       }
     }
-    uint4 pk;
-    pk.x = static_cast<uint32_t>(bf16_bits_from_float(v[0])) | (static_cast<uint32_t>(bf16_bits_from_float(v[1])) << 16);
-    pk.y = static_cast<uint32_t>(bf16_bits_from_float(v[2])) | (static_cast<uint32_t>(bf16_bits_from_float(v[3])) << 16);
-    pk.z = static_cast<uint32_t>(bf16_bits_from_float(v[4])) | (static_cast<uint32_t>(bf16_bits_from_float(v[5])) << 16);
-    pk.w = static_cast<uint32_t>(bf16_bits_from_float(v[6])) | (static_cast<uint32_t>(bf16_bits_from_float(v[7])) << 16);
-    if (is_q) {
-      *reinterpret_cast<uint4*>(out + gm * (static_cast<long>(ra.n_heads) * d) + gn) = pk;
-      continue;
-    }
-    const int slot = ra.slot_map[gm];
-    const long page = slot / ra.page_tokens;
-    const int off = slot % ra.page_tokens;
-    if (!is_v) {      // keys: [page][kv head][token][dim], or in fragment order: eight dimensions of 16 tokens together
-      bf16_t* region = ra.k_cache + (page * ra.n_kv_heads + (head - ra.n_heads)) * ra.page_tokens * d;
-      bf16_t* dst = ra.fragment_order ? region + frag_k_offset(off, dim, d) : region + static_cast<long>(off) * d + dim;
-      *reinterpret_cast<uint4*>(dst) = pk;
-    } else {          // values are kept transposed: [page][kv head][dim][token], or in fragment order
-      bf16_t* region = ra.v_cache + (page * ra.n_kv_heads + (head - ra.n_heads - ra.n_kv_heads)) * static_cast<long>(d) * ra.page_tokens;
-      bf16_t* dst = ra.fragment_order ? region + frag_v_offset(off, dim, d) : region + static_cast<long>(dim) * ra.page_tokens + off;
-      const long step = ra.fragment_order ? 4 : ra.page_tokens;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) dst[e * step] = from_float<bf16_t>(v[e]);
+    for (int u = 0; u < kTogether; ++u) {
+      const int gm = first_row + row[u], gn = first_col + col[u];
+      const bool is_q = head[u] < ra.n_heads, is_v = head[u] >= ra.n_heads + ra.n_kv_heads;
+      long key = 0, value = 0;
+      if (caches) key = from_row(places.key, row[u]), value = from_row(places.value, row[u]);          // (by every lane)
+      if (gm >= m || gn >= n || (!is_q && !ra.write_kv)) continue;
+      float v[8];
+      const float* mine = patch + row[u] * kStride + col[u];
+      {
+        const floatx4 v0 = *reinterpret_cast<const floatx4*>(mine), v1 = *reinterpret_cast<const floatx4*>(mine + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = v0[e], v[4 + e] = v1[e];
+      }
+      if (ra.table != nullptr && !is_v) {
+        const bool first = dim[u] % 16 < 8;                    // a block's eight first halves of pairs; their partners lie 8 further
+        const float* partner = first ? mine + 8 : mine - 8;
+        const floatx4 o0 = *reinterpret_cast<const floatx4*>(partner), o1 = *reinterpret_cast<const floatx4*>(partner + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const floatx4 a = cs[u][e];
+          const float p0 = e < 2 ? o0[2 * e] : o1[2 * e - 4], p1 = e < 2 ? o0[2 * e + 1] : o1[2 * e - 3];
+          v[2 * e] = first ? v[2 * e] * a[0] - p0 * a[1] : v[2 * e] * a[0] + p0 * a[1];
+          v[2 * e + 1] = first ? v[2 * e + 1] * a[2] - p1 * a[3] : v[2 * e + 1] * a[2] + p1 * a[3];
+        }
+      }
+      const uint4 pk = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+      if (is_q) {
+        *reinterpret_cast<uint4*>(out + static_cast<long>(gm) * (ra.n_heads * d) + gn) = pk;
+      } else if (!is_v) {      // keys: [page][kv head][token][dim], or in fragment order: eight dimensions of 16 tokens together
+        *reinterpret_cast<uint4*>(ra.k_cache + key + (head[u] - ra.n_heads) * per_head + (ra.fragment_order ? frag_k_offset(0, dim[u], d) : dim[u])) = pk;
+      } else {                 // values are kept transposed: [page][kv head][dim][token], or in fragment order
+        bf16_t* dst = ra.v_cache + value + (head[u] - ra.n_heads - ra.n_kv_heads) * per_head +
+                      (ra.fragment_order ? frag_v_offset(0, dim[u], d) : static_cast<long>(dim[u]) * ra.page_tokens);
+        const long step = ra.fragment_order ? 4 : ra.page_tokens;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dst[e * step].bits = static_cast<uint16_t>(e % 2 ? (&pk.x)[e / 2] >> 16 : (&pk.x)[e / 2]);
+      }
     }
   }
 }
@@ -461,15 +483,24 @@ template <int EPI, int TM, int TN>
 __device__ inline void store_part(const floatx16 (&acc)[TM][TN], float* patch, void* __restrict__ out, int m, int n, int k, long m0, long n0, int lane,
                                   const RopeKvArgs& ra, const RowScaleArgs& rows, const float* part_sum = nullptr, int tile_rows = 0) {
   constexpr int kStride = 32 * TN + 4;
+  // (q|k|v: the rows' places, where the part has columns of keys or values)
+  RowPlaces places{};
+  int slot[TM];
+  const bool caches = EPI == kRopeKvBf16 && ra.write_kv && n0 + 32 * TN > static_cast<long>(ra.n_heads) * ra.head_dim;
+  if (caches) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) slot[i] = ra.slot_map[min(m0 + i * 32 + lane % 32, m - 1L)];
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) patch[(8 * (r / 4) + 4 * (lane / 32) + r % 4) * kStride + j * 32 + lane % 32] = acc[i][j][r];
-    if constexpr (EPI == kRopeKvBf16)
-      store_patch_rope<kWave, 32, 32 * TN>(patch, static_cast<bf16_t*>(out), m, n, m0 + i * 32, n0, lane, ra);
-    else if constexpr (row_scaled(EPI))
+    if constexpr (EPI == kRopeKvBf16) {
+      if (caches) places = row_places(slot[i], ra);
+      store_patch_rope<32 * TN>(patch, static_cast<bf16_t*>(out), m, n, m0 + i * 32, n0, lane, ra, places);
+    } else if constexpr (row_scaled(EPI))
       store_patch<EPI, kWave, 32, 32 * TN>(patch, out, m, n, m0 + i * 32, n0, lane,
                                            RowScale{part_sum + i * 32, tile_rows, 1.0f / static_cast<float>(k), rows.eps});
     else
@@ -1242,9 +1273,11 @@ struct DirectForm {
 // The last, 128 x 64 with two stages and four workgroups a CU, is for the q|k|v epilogue alone: what comes after the
 // loop is long there (rotation, three destinations), and several workgroups a CU run it beside each other's loops
 // (a 2,048-token TinyLlama prompt 1 % faster with it than with 160 tiles of 256 x 128, both libraries in one process).
-// us_qkv: by how much that epilogue is longer than plain stores, a turn, from 4,500 products of 130 to 4,200 rows, 384 to 20,480 outputs (wider ones
+// us_qkv: by how much that epilogue counts as longer than plain stores, a turn, fitted to 4,500 products of 130 to 4,200 rows, 384 to 20,480 outputs (wider ones
 // are not asked: kQkvMeasured) and k 512 to 4,096, every form of each: what is chosen is 0.65 % slower on average than the fastest, 1.4 % without it.
 // 3,628 x 1,536 x 1,024 went to 180 tiles of 256 x 128, 33.4 us, where 128 x 64 takes 26.8; 2,048 x 3,072 x 1,024 31.6 and 27.4.
+// (The epilogue has become shorter since; with four other sets of these numbers, from a seventh to a third of them, 80 products of 72 to 4,096 rows were 0.1 %
+// to 2 % slower.)
 constexpr int kQkvMeasured = 20480;
 constexpr int kDirectForms = 6;
 constexpr DirectForm kDirectForm[kDirectForms] = {
@@ -1503,6 +1536,8 @@ extern "C" int bc4g_gemm_mfma_qkv(const void* a, const void* w, int w_packed, vo
   ra.n_kv_heads = n_kv_heads;
   ra.head_dim = head_dim;
   ra.page_tokens = page_tokens;
+  ra.per_head = reciprocal_of(static_cast<unsigned>(head_dim));
+  ra.per_page = page_tokens > 0 ? reciprocal_of(static_cast<unsigned>(page_tokens)) : 0u;
   ra.write_kv = write_kv ? 1 : 0;
   ra.fragment_order = write_kv && cache_fragment_order(true, head_dim, page_tokens) ? 1 : 0;
   if (int e = launch_direct_form<kRopeKvBf16>(static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(w), out, m, n, k,

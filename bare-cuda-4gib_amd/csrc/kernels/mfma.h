@@ -61,6 +61,13 @@ __device__ inline float gelu_tanh_quick(float z) {
   return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(u2 * -1.4426950408889634f));
 }
 
+// Two floats to two bfloat16 (round to nearest even) in one instruction of gfx950.
+__device__ inline uint32_t pack_bf16x2(float lo, float hi) {
+  uint32_t r;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
+  return r;
+}
+
 __device__ inline uint4 load16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ inline uint4 zero16() { return make_uint4(0u, 0u, 0u, 0u); }
 
