@@ -82,6 +82,7 @@ struct SkinnyArgs {
   int last_block;           // the last block of w,
   int part_stride;          // numbers from one part to the next, and where the last four of all parts begin
   int last_four;
+  int x_row_bytes, g_f32;   // ring kernel, normed modes: LDS of a wave's part of a row of x; whether g is float
   int ssq_blocks, ssq_stride;
   int ssq_halves;           // the parts are pairs, [ssq_blocks][ssq_stride][2]
   float eps;
@@ -629,17 +630,22 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
 // from memory, us, kernel above and this: 8 rows 2,048 x 2,048 4.39 and 4.07, 2,048 x 5,632 7.74 and 6.81, 11,264 x 2,048 10.84 and 9.90, 28,672 x 4,096
 // 41.4 and 39.3; 16 rows 2,048 x 5,632 9.18 and 7.66, 4,096 x 4,096 10.6 and 8.4, 4,096 x 11,008 26.1 and 19.0, 22,016 x 4,096 37.5 and 35.5; 32 rows
 // 4,096 x 11,008 30.1 and 23.4; 64 rows 2,048 x 2,048 6.53 and 5.95, 4,096 x 4,096 14.9 and 12.5.
-template <int ROWS, int NB, int KS, int S>
+// With the norm fused (NORMED: x the float stream, up to eight rows) x and the norm's scale come into LDS once, ahead of the first weights; one wave
+// takes a row's sum of squares, in the order of rmsnorm_prepare and of the kernel above, then every wave turns its part of k into bfloat16(x * g) in
+// its place, and the rings hold weights only.  One row 2,560 x 2,048 6.23 and 5.36, 4,096 x 4,096 12.7 and 9.8, 11,264 x 2,048 11.6 and 11.2, 22,016 x 4,096
+// 40.1 and 36.5; four rows 4,096 x 4,096 12.9 and 11.6.
+template <int ROWS, int NB, int KS, int S, bool NORMED = false>
 struct RingShape {
   static constexpr bool kHalf = NB == 0;                      // half a block: two workgroups share one
   static constexpr int kTiles = (ROWS + 15) / 16, kBlocks = kHalf ? 1 : NB;
-  static constexpr int kXLoads = ROWS * KS / 512, kWLoads = kHalf ? KS / 64 : NB * KS / 32, kLoads = kXLoads + kWLoads;
+  static constexpr int kXLoads = NORMED ? 0 : ROWS * KS / 512, kWLoads = kHalf ? KS / 64 : NB * KS / 32, kLoads = kXLoads + kWLoads;
   static constexpr int kStageBytes = kLoads * 1024, kRingBytes = kWaves * S * kStageBytes;
   static constexpr int kRedBytes = kWaves * kBlocks * kTiles * 16 * kRedPad * 4;
   static constexpr int kLdsBytes = kRingBytes > kRedBytes ? kRingBytes : kRedBytes;
   static_assert(kLdsBytes <= 152 * 1024 && S * kLoads < 64, "a workgroup's LDS beside what else it keeps there, and a wait's count");
   static_assert((KS == 64 && ROWS % 8 == 0) || (KS == 32 && ROWS % 16 == 0), "whole loads of x");
   static_assert(ROWS == 8 || ROWS % 16 == 0, "eight rows or whole tiles");
+  static_assert(!NORMED || (ROWS == 8 && !kHalf && KS == 64), "the fused norm: eight rows, whole blocks");
 };
 
 // N loads of 1 KB to N KB of LDS side by side, load i from bases[i] (the same in every lane) + off[i].
@@ -691,19 +697,20 @@ __device__ inline void ring_wait(int later) {
   }
 }
 
-template <int EPI, int ROWS, int NB, int KS, int S>
+template <int EPI, int ROWS, int NB, int KS, int S, bool NORMED = false>
 __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs args) {
-  typedef RingShape<ROWS, NB, KS, S> P;
+  typedef RingShape<ROWS, NB, KS, S, NORMED> P;
   constexpr bool kHalf = P::kHalf, kPaired = gated(EPI) || EPI == kRopeKvBf16;
   static_assert(!kHalf || (ROWS <= 16 && !kPaired), "half blocks: few rows, unpaired outputs");
   constexpr int TM = P::kTiles, TB = P::kBlocks, kSteps = KS / 32, kPartSums = 8;
-  extern __shared__ __align__(1024) unsigned char ring_lds[];
-  __shared__ float part_sum[kPartSums][ROWS];
+  extern __shared__ __align__(128) unsigned char ring_lds[];
+  __shared__ float part_sum[kPartSums][ROWS];                                // (normed modes: the rows' sums of squares)
   __shared__ int places[EPI == kRopeKvBf16 ? kWaves : 1][2][kWave];          // positions and cache slots, every wave's own
-  const SkinnyArgs a = own_rows<EPI>(args);
+  const SkinnyArgs a = NORMED ? args : own_rows<EPI>(args);
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int col = lane % 16, grp = lane / 16;
   const int m = a.m, k = a.k;
+  auto lds_address = [](const void* p) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const unsigned char*)p)); };
   const int first_block = kHalf ? blockIdx.x / 2 : blockIdx.x * TB, half = kHalf ? blockIdx.x % 2 : 0;
 
   // Item j of a thread is output nl of block b and row `row` of number threadIdx.x + j * kThreads.  What it needs beside its sum is asked for before the
@@ -733,8 +740,11 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
       g[j] = *reinterpret_cast<const uint32_any*>(scale + (a.emit_g_f32 ? 4 * gn : 2 * max(gn, 1u) - 2));
     }
   }
+  int src = lane;                             // normed modes: lane r's row of x
+  if constexpr (NORMED) {
+    if (a.rows != nullptr) src = a.rows[min(lane, m - 1)];
+  }
   if constexpr (EPI == kRopeKvBf16) {
-    auto lds_address = [](const void* p) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const unsigned char*)p)); };
     if (a.rope.rotary_dim > 0) load_to_lds_4(a.rope.positions + min(lane, m - 1), lds_address(&places[wave][0][0]));
     if (a.rope.write_kv) load_to_lds_4(a.rope.slot_map + min(lane, m - 1), lds_address(&places[wave][1][0]));
   }
@@ -744,7 +754,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
   // (Past the last part or number: the last four, turned into place after the walk.)
   constexpr int kHeld = ROWS <= 8 ? 1 : ROWS / 8;
   typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
-  const bool prenormed = EPI != kAccumF32 && a.ssq_parts != nullptr, pairs = ROWS == 8 && a.ssq_halves;
+  const bool prenormed = EPI != kAccumF32 && !NORMED && a.ssq_parts != nullptr, pairs = ROWS == 8 && a.ssq_halves;
   const int shift = ROWS == 8 ? 1 + a.ssq_halves : ROWS == 16 ? 2 : 3, parts_a_load = kWave >> shift;
   const int part_stride = a.part_stride;
   const int first_row = a.rows_per_block > 0 ? static_cast<int>(blockIdx.y) * a.rows_per_block : 0, last_four = a.last_four - first_row;
@@ -752,7 +762,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
     return min(wave + kPartSums * (h * parts_a_load + (lane >> shift)), a.ssq_blocks - 1) * part_stride + (lane & ((1 << shift) - 1)) * 4;
   };
   floatx4 held[kHeld];
-  if constexpr (EPI != kAccumF32) {
+  if constexpr (EPI != kAccumF32 && !NORMED) {
     const float* parts = prenormed ? a.ssq_parts : static_cast<const float*>(a.x);
 #pragma unroll
     for (int h = 0; h < kHeld; ++h) held[h] = *reinterpret_cast<const floatx4_any*>(parts + static_cast<unsigned>(prenormed ? min(part_at(h), last_four) : 0));
@@ -764,7 +774,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
   const unsigned ring = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const unsigned char*)mine));
   constexpr int kRowBytes = KS * 2, kPieces = KS / 8, kLoadRows = kWave / kPieces;
   auto key = [](int row) { return KS == 64 ? (row >> 1) & 7 : (row >> 2) & 3; };      // piece p of a row lies at p ^ key
-  unsigned x_off[P::kXLoads], w_off[P::kWLoads];
+  unsigned x_off[NORMED ? 1 : P::kXLoads], w_off[P::kWLoads];
 #pragma unroll
   for (int i = 0; i < P::kXLoads; ++i) {
     const int row = i * kLoadRows + lane / kPieces;                                    // (rows past m: the last)
@@ -780,15 +790,31 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
   const unsigned char* x_at = static_cast<const unsigned char*>(a.x) + static_cast<unsigned>(k_begin) * 2;
   auto ask = [&](int t) {
     const unsigned to = ring + (t % S) * P::kStageBytes;
-    const unsigned char *xs[P::kXLoads], *ws[P::kWLoads];
+    const unsigned char *xs[NORMED ? 1 : P::kXLoads], *ws[P::kWLoads];
 #pragma unroll
     for (int i = 0; i < P::kWLoads; ++i)
       ws[i] = (kHalf ? w_at[0] + i * 2048 : w_at[i / kSteps] + i % kSteps * 1024) + static_cast<size_t>(t) * (kSteps * 1024);
 #pragma unroll
     for (int i = 0; i < P::kXLoads; ++i) xs[i] = x_at + static_cast<size_t>(t) * kRowBytes;
     ring_loads<P::kWLoads>(ws, w_off, to);
-    ring_loads<P::kXLoads>(xs, x_off, to + P::kWLoads * 1024);
+    if constexpr (!NORMED) ring_loads<P::kXLoads>(xs, x_off, to + P::kWLoads * 1024);
   };
+
+  // normed modes: x and g in pieces of 1 KB, piece p by wave p % 8 (lanes past the row's end: its last 16 bytes)
+  unsigned char *rows_lds = ring_lds + P::kLdsBytes, *scale_lds = rows_lds + m * a.x_row_bytes;
+  if constexpr (NORMED) {
+    for (int at = wave * 1024; at < k * 4; at += kWaves * 1024) {
+      const unsigned from = min(at + lane * 16, k * 4 - 16);
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        if (r < m)
+          load_to_lds_16(static_cast<const unsigned char*>(a.x) + static_cast<size_t>(__builtin_amdgcn_readlane(src, r)) * (static_cast<unsigned>(k) * 4), from,
+                         lds_address(rows_lds + r * a.x_row_bytes + at));
+    }
+    const int g_bytes = a.g_f32 ? 4 * k : 2 * k;
+    for (int at = wave * 1024; at < g_bytes; at += kWaves * 1024)
+      load_to_lds_16(a.g, static_cast<unsigned>(min(at + lane * 16, g_bytes - 16)), lds_address(scale_lds + at));
+  }
 #pragma unroll
   for (int s = 0; s < S; ++s)
     if (s < steps) ask(s);
@@ -815,8 +841,52 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
     }
   }
 
+  if constexpr (NORMED) {
+    ring_wait<P::kLoads, S>(min(S, steps));
+    lds_barrier();                              // (the weights stay in flight)
+    if (wave < m) {
+      // row `wave`: lane l takes elements 8 l .. 8 l + 7 of every 512
+      float ss = 0.f;
+      for (int kk = lane * 8; kk < k; kk += 512) {
+        const float* p = reinterpret_cast<const float*>(rows_lds + wave * a.x_row_bytes) + kk;
+        const floatx4 v0 = *reinterpret_cast<const floatx4*>(p), v1 = *reinterpret_cast<const floatx4*>(p + 4);
+        const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+        ss = add_squares(v, kk >= 512, ss);
+      }
+      ss = wave_sum(ss);
+      if (lane == 0) part_sum[0][wave] = ss;
+    }
+    lds_barrier();
+    // bfloat16(x * g) to the beginning of this wave's part: four numbers a lane, a piece of four rows read before anything is written over it
+    for (int at = lane * 16; at < steps * KS * 4; at += 1024) {
+      floatx4 scale;
+      if (a.g_f32) {
+        scale = *reinterpret_cast<const floatx4*>(scale_lds + k_begin * 4 + at);
+      } else {
+        const uint2 raw = *reinterpret_cast<const uint2*>(scale_lds + k_begin * 2 + at / 2);
+        scale = floatx4{__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u), __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xffff0000u)};
+      }
+      for (int r0 = 0; r0 < m; r0 += 4) {
+        floatx4 v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = *reinterpret_cast<const floatx4*>(rows_lds + min(r0 + r, m - 1) * a.x_row_bytes + k_begin * 4 + at);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = min(r0 + r, m - 1);
+          *reinterpret_cast<uint2*>(rows_lds + row * a.x_row_bytes + k_begin * 4 + (at / 2 ^ row * 16)) =
+              make_uint2(pack_bf16x2(v[r][0] * scale[0], v[r][1] * scale[1]), pack_bf16x2(v[r][2] * scale[2], v[r][3] * scale[3]));
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+
   auto wait_lds_reads = []() { __builtin_amdgcn_s_waitcnt(63 >> 4 << 14 | 0 << 8 | 7 << 4 | 15); };      // lgkmcnt(0)
   const int read_row = ROWS == 8 ? col % 8 : col;
+  const unsigned char* normed_row = rows_lds + min(read_row, m - 1) * a.x_row_bytes + k_begin * 4;
+  const int normed_key = grp * 16 ^ min(read_row, m - 1) * 16;
   for (int t = 0; t < steps; ++t) {
     ring_wait<P::kLoads, S - 1>(min(steps - 1 - t, S - 1));
     __builtin_amdgcn_sched_barrier(0);
@@ -827,7 +897,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
 #pragma unroll
       for (int b = 0; b < TB; ++b) fw[u][b] = load16(kHalf ? stage + u * 512 + grp * 128 + col % 8 * 16 : stage + (b * kSteps + u) * 1024 + lane * 16);
 #pragma unroll
-      for (int i = 0; i < TM; ++i) fx[u][i] = load16(stage + P::kWLoads * 1024 + (i * 16 + read_row) * kRowBytes + ((u * 4 + grp) ^ key(read_row)) * 16);
+      for (int i = 0; i < TM; ++i)
+        fx[u][i] = NORMED ? load16(normed_row + ((t * 128 + u * 64) ^ normed_key))
+                          : load16(stage + P::kWLoads * 1024 + (i * 16 + read_row) * kRowBytes + ((u * 4 + grp) ^ key(read_row)) * 16);
     }
     __builtin_amdgcn_sched_barrier(0);
     wait_lds_reads();                         // in registers: the stage may be written over
@@ -908,10 +980,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
 #pragma unroll
         for (int v = 0; v < kWaves; ++v) partner += red[v][b][row / 16][nl + 8][row % 16];
       }
-      if (prenormed) {
-        float ssq = 0.f;
+      if (NORMED || prenormed) {
+        float ssq = NORMED ? part_sum[0][row] : 0.f;
+        if constexpr (!NORMED) {
 #pragma unroll
-        for (int c = 0; c < kPartSums; ++c) ssq += part_sum[c][row];
+          for (int c = 0; c < kPartSums; ++c) ssq += part_sum[c][row];
+        }
         const float scale = 1.0f / sqrtf(ssq / static_cast<float>(k) + a.eps);
         sum *= scale;
         partner *= scale;
@@ -928,13 +1002,19 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
   }
 }
 
-template <int EPI, int ROWS, int NB, int KS, int S>
+// LDS of a float row, in whole loads, and of all that the normed modes keep beside the rings
+int ring_row_bytes(int k) { return (k * 4 + 1023) / 1024 * 1024; }
+int ring_norm_bytes(int m, int k, bool g_f32) { return m * ring_row_bytes(k) + (g_f32 ? ring_row_bytes(k) : (k * 2 + 1023) / 1024 * 1024); }
+constexpr int kRingNormBytes = 80 * 1024;     // of those at most
+
+template <int EPI, int ROWS, int NB, int KS, int S, bool NORMED = false>
 int launch_ring(const SkinnyArgs& a, int row_groups, hipStream_t s) {
-  typedef RingShape<ROWS, NB, KS, S> P;
-  auto kernel = gemm_ring_kernel<EPI, ROWS, NB, KS, S>;
+  typedef RingShape<ROWS, NB, KS, S, NORMED> P;
+  auto kernel = gemm_ring_kernel<EPI, ROWS, NB, KS, S, NORMED>;
   static bool raised = false;
   if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, P::kLdsBytes) != hipSuccess)
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, P::kLdsBytes + (NORMED ? kRingNormBytes : 0)) !=
+        hipSuccess)
       return fail("gemm_skinny: cannot raise the dynamic LDS limit");
     raised = true;
   }
@@ -946,7 +1026,8 @@ int launch_ring(const SkinnyArgs& a, int row_groups, hipStream_t s) {
   b.last_block = blocks - 1;
   b.part_stride = a.ssq_stride * (a.ssq_halves ? 2 : 1);
   b.last_four = a.ssq_blocks * b.part_stride - 4;
-  kernel<<<grid, dim3(kThreads), P::kLdsBytes, s>>>(b);
+  b.x_row_bytes = NORMED ? ring_row_bytes(a.k) : 0;
+  kernel<<<grid, dim3(kThreads), P::kLdsBytes + (NORMED ? ring_norm_bytes(a.m, a.k, a.g_f32) : 0), s>>>(b);
   return check_launch("gemm_skinny");
 }
 
@@ -981,6 +1062,22 @@ int launch_rings(const SkinnyArgs& a, hipStream_t s) {
   return blocks <= cus ? launch_ring<EPI, 32, 2, 64, 2>(a, 2, s) : launch_ring<EPI, 32, 3, 32, 2>(a, 2, s);
 }
 
+// The same with the norm fused.
+template <int EPI>
+int launch_normed_rings(const SkinnyArgs& a, hipStream_t s) {
+  if ((a.n + 15) / 16 <= compute_units()) return launch_ring<EPI, 8, 1, 64, 4, true>(a, 1, s);
+  return a.k < 4096 ? launch_ring<EPI, 8, 1, 64, 2, true>(a, 1, s) : launch_ring<EPI, 8, 1, 64, 3, true>(a, 1, s);
+}
+
+// Up to eight rows that fit LDS beside the rings, and for wide outputs beside those of two other workgroups of the CU (one from k = 4,096 on): with
+// fewer of them there the kernel above is faster (four rows 11,264 x 2,048 12.5 and 13.1).  Below k = 2,048 too, where fewer waves than eight fetch all of x
+// (2,048 x 1,024: one row 4.33 and 4.53, eight 4.91 and 5.71; 2,048 x 2,048: 6.17 and 5.26, 6.82 and 6.74).
+bool normed_ring_operands(const SkinnyArgs& a) {
+  const int most = (a.n + 15) / 16 <= compute_units() ? kRingNormBytes : a.k < 4096 ? 20 * 1024 : 28 * 1024;
+  return a.k % 64 == 0 && a.k >= 2048 && a.m <= 8 && ring_norm_bytes(a.m, a.k, a.g_f32) <= most &&
+         reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.g) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0;
+}
+
 // What the rings take: the loads bring 16 bytes from 16-byte boundaries, a stage is 64 values of k, parts of a norm are read four numbers at a time and the
 // next norm's scale two.
 bool ring_operands(const SkinnyArgs& a) {
@@ -995,6 +1092,7 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
   dim3 grid((a.n + 15) / 16), block(kThreads);
   if constexpr (XMODE != kPlain) {
     if (mt != 1) return fail("gemm_skinny: the fused norm takes at most 16 rows, got %d", a.m);
+    if (normed_ring_operands(a)) return launch_normed_rings<EPI>(a, s);
     const size_t stage = static_cast<size_t>(a.m_stage) * (a.k + kStagePad) * 2;
     if (stage > kMaxStageBytes) return fail("gemm_skinny: %d rows of k=%d do not fit the staging buffer", a.m, a.k);
     auto kernel = gemm_skinny_kernel<1, EPI, XMODE, 4>;
@@ -1215,6 +1313,7 @@ extern "C" int bc4g_gemm_skinny_normed(const float* x, const int32_t* rows, cons
   SkinnyArgs a = plain_args(x, w, out, m, n, k);
   a.rows = rows;
   a.g = g;
+  a.g_f32 = g_dtype == kF32 ? 1 : 0;
   a.m_stage = ((m + 3) / 4) * 4;
   a.eps = eps;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1247,6 +1346,7 @@ extern "C" int bc4g_gemm_skinny_qkv(const void* x, const void* g, int g_dtype, f
   hipStream_t s = static_cast<hipStream_t>(stream);
   SkinnyArgs a = plain_args(x, w, q_out, m, n, k);
   a.g = g;
+  a.g_f32 = g_dtype == kF32 ? 1 : 0;
   a.m_stage = g ? ((m + 3) / 4) * 4 : 0;
   a.eps = eps;
   a.rope = r;

@@ -93,3 +93,28 @@ def test_rotated_and_cached(ops, m, heads, kv_heads, head_dim, page):
     assert all(torch.equal(one, other) for one, other in zip(*made))
     want = (x.float() @ w.rows[:heads * head_dim].float().T)
     assert (made[0][3].float() - want).abs().max() < 2.0 ** -8 * want.abs().max()
+
+
+# parts of k that end inside a piece of 1 KB, waves without a part; one workgroup a CU and several, with as many rows as then fit beside the rings and more
+@pytest.mark.parametrize("g_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n, k", [(16, 2048), (1000, 2240), (2048, 2112), (4064, 5632), (4128, 2496), (8192, 3008), (4800, 4096)])
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9])
+def test_norm_fused(ops, m, n, k, g_dtype):
+    _, w = operands(ops, m, n, k)
+    x, g = 3 * torch.randn(m + 2, k, device=DEV), (1 + 0.1 * torch.randn(k, device=DEV)).to(g_dtype)
+    if not ops.gemm_normed_supported(x, m, g, w):
+        pytest.skip("the norm runs apart")
+    rows = torch.tensor([m + 1 - r for r in range(m)], dtype=torch.int32, device=DEV)
+    other, first = off_by_eight(x), x[:m].contiguous()
+    epilogues = [ops.EPI_STORE_F32, ops.EPI_STORE_BF16, ops.EPI_SQUARED_RELU] + ([ops.EPI_SWIGLU] if n % 16 == 0 else [])
+    for e in epilogues:
+        assert torch.equal(ops.gemm_normed(x, rows, m, g, 1e-5, w, e), ops.gemm_normed(other, rows, m, g, 1e-5, w, e))
+        assert torch.equal(ops.gemm_normed(first, None, m, g, 1e-5, w, e), ops.gemm_normed(off_by_eight(first), None, m, g, 1e-5, w, e))
+    if n % 64 == 0 and n >= 192:
+        kv = n // 64 // 3
+        made = []
+        for a in (first, off_by_eight(first)):
+            kc, vc = torch.zeros(2, kv, 16, 64, dtype=torch.bfloat16, device=DEV), torch.zeros(2, kv, 64, 16, dtype=torch.bfloat16, device=DEV)
+            at = torch.arange(m, dtype=torch.int32, device=DEV) * 3
+            made.append((ops.gemm_qkv_rope(a, g, 1e-5, w, at, at, kc, vc, n // 64 - 2 * kv, kv, 64, 64, 1e4), kc, vc))
+        assert all(torch.equal(one, two) for one, two in zip(*made))
