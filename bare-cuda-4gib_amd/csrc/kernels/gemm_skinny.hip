@@ -629,7 +629,8 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
 // CU pulls of x through its cache (105 to 120 bytes a ns from L2; with x turned through registers it was 65 of both together).  Weights
 // from memory, us, kernel above and this: 8 rows 2,048 x 2,048 4.39 and 4.07, 2,048 x 5,632 7.74 and 6.81, 11,264 x 2,048 10.84 and 9.90, 28,672 x 4,096
 // 41.4 and 39.3; 16 rows 2,048 x 5,632 9.18 and 7.66, 4,096 x 4,096 10.6 and 8.4, 4,096 x 11,008 26.1 and 19.0, 22,016 x 4,096 37.5 and 35.5; 32 rows
-// 4,096 x 11,008 30.1 and 23.4; 64 rows 2,048 x 2,048 6.53 and 5.95, 4,096 x 4,096 14.9 and 12.5.
+// 4,096 x 11,008 30.1 and 23.4; 64 rows 2,048 x 2,048 6.53 and 5.95, 4,096 x 4,096 14.9 and 12.5.  With weights past the caches (launch_ring) less again:
+// one row 32,000 x 2,048 23.9 -> 21.7 (6 TB/s), 8 rows 11,264 x 2,048 10.6 -> 10.4, 28,672 x 4,096 39.5 -> 36.8, 16 rows 44.4 -> 40.1.
 // With the norm fused (NORMED: x the float stream, up to eight rows) x and the norm's scale come into LDS once, ahead of the first weights; one wave
 // takes a row's sum of squares, in the order of rmsnorm_prepare and of the kernel above, then every wave turns its part of k into bfloat16(x * g) in
 // its place, and the rings hold weights only.  One row 2,560 x 2,048 6.23 and 5.36, 4,096 x 4,096 12.7 and 9.8, 11,264 x 2,048 11.6 and 11.2, 22,016 x 4,096
@@ -648,8 +649,8 @@ struct RingShape {
   static_assert(!NORMED || (ROWS == 8 && !kHalf && KS == 64), "the fused norm: eight rows, whole blocks");
 };
 
-// N loads of 1 KB to N KB of LDS side by side, load i from bases[i] (the same in every lane) + off[i].
-template <int N>
+// N loads of 1 KB to N KB of LDS side by side, load i from bases[i] (the same in every lane) + off[i]; past the caches or through them.
+template <int N, bool PAST>
 __device__ inline void ring_loads(const unsigned char* const* bases, const unsigned* off, unsigned lds_address) {
   // (the LDS address is set once, to the middle of the stretch: the offset field reaches 4 KB either way, and moves the memory address too)
   constexpr int kMid = N / 2;
@@ -661,17 +662,26 @@ __device__ inline void ring_loads(const unsigned char* const* bases, const unsig
     b[i] = reinterpret_cast<const void*>((static_cast<uintptr_t>(hi) << 32) | lo);
   }
   const unsigned mid = __builtin_amdgcn_readfirstlane(lds_address + kMid * 1024);
-#define BC4G_LOAD(v, s, o) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #o "\n\t"
+#define BC4G_LOAD(v, s, o, how) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #o how "\n\t"
 #define BC4G_RING(loads, ...) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" loads ::"s"(mid), __VA_ARGS__ : "memory", "m0")
-  if constexpr (N == 1) BC4G_RING(BC4G_LOAD(1, 2, 0), "v"(off[0]), "s"(b[0]));
-  else if constexpr (N == 2) BC4G_RING(BC4G_LOAD(1, 3, -1024) BC4G_LOAD(2, 4, 0), "v"(off[0]), "v"(off[1]), "s"(b[0]), "s"(b[1]));
-  else if constexpr (N == 3)
-    BC4G_RING(BC4G_LOAD(1, 4, -1024) BC4G_LOAD(2, 5, 0) BC4G_LOAD(3, 6, 1024), "v"(off[0]), "v"(off[1]), "v"(off[2]), "s"(b[0]), "s"(b[1]), "s"(b[2]));
-  else {
-    static_assert(N == 4, "loads a statement");
-    BC4G_RING(BC4G_LOAD(1, 5, -2048) BC4G_LOAD(2, 6, -1024) BC4G_LOAD(3, 7, 0) BC4G_LOAD(4, 8, 1024), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]),
-              "s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3]));
+#define BC4G_RINGS(how)                                                                                                                          \
+  if constexpr (N == 1) BC4G_RING(BC4G_LOAD(1, 2, 0, how), "v"(off[0]), "s"(b[0]));                                                              \
+  else if constexpr (N == 2)                                                                                                                     \
+    BC4G_RING(BC4G_LOAD(1, 3, -1024, how) BC4G_LOAD(2, 4, 0, how), "v"(off[0]), "v"(off[1]), "s"(b[0]), "s"(b[1]));                              \
+  else if constexpr (N == 3)                                                                                                                     \
+    BC4G_RING(BC4G_LOAD(1, 4, -1024, how) BC4G_LOAD(2, 5, 0, how) BC4G_LOAD(3, 6, 1024, how), "v"(off[0]), "v"(off[1]), "v"(off[2]), "s"(b[0]),  \
+              "s"(b[1]), "s"(b[2]));                                                                                                             \
+  else {                                                                                                                                         \
+    static_assert(N == 4, "loads a statement");                                                                                                  \
+    BC4G_RING(BC4G_LOAD(1, 5, -2048, how) BC4G_LOAD(2, 6, -1024, how) BC4G_LOAD(3, 7, 0, how) BC4G_LOAD(4, 8, 1024, how), "v"(off[0]),           \
+              "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3]));                                                \
   }
+  if constexpr (PAST) {
+    BC4G_RINGS(" nt")
+  } else {
+    BC4G_RINGS("")
+  }
+#undef BC4G_RINGS
 #undef BC4G_RING
 #undef BC4G_LOAD
 }
@@ -697,7 +707,8 @@ __device__ inline void ring_wait(int later) {
   }
 }
 
-template <int EPI, int ROWS, int NB, int KS, int S, bool NORMED = false>
+// (PAST: the weights past the caches.  Chosen while a step is asked for it cost 0.3 us a product.)
+template <int EPI, int ROWS, int NB, int KS, int S, bool NORMED, bool PAST>
 __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs args) {
   typedef RingShape<ROWS, NB, KS, S, NORMED> P;
   constexpr bool kHalf = P::kHalf, kPaired = gated(EPI) || EPI == kRopeKvBf16;
@@ -796,8 +807,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
       ws[i] = (kHalf ? w_at[0] + i * 2048 : w_at[i / kSteps] + i % kSteps * 1024) + static_cast<size_t>(t) * (kSteps * 1024);
 #pragma unroll
     for (int i = 0; i < P::kXLoads; ++i) xs[i] = x_at + static_cast<size_t>(t) * kRowBytes;
-    ring_loads<P::kWLoads>(ws, w_off, to);
-    if constexpr (!NORMED) ring_loads<P::kXLoads>(xs, x_off, to + P::kWLoads * 1024);
+    ring_loads<P::kWLoads, PAST>(ws, w_off, to);
+    if constexpr (!NORMED) ring_loads<P::kXLoads, false>(xs, x_off, to + P::kWLoads * 1024);
   };
 
   // normed modes: x and g in pieces of 1 KB, piece p by wave p % 8 (lanes past the row's end: its last 16 bytes)
@@ -1007,10 +1018,10 @@ int ring_row_bytes(int k) { return (k * 4 + 1023) / 1024 * 1024; }
 int ring_norm_bytes(int m, int k, bool g_f32) { return m * ring_row_bytes(k) + (g_f32 ? ring_row_bytes(k) : (k * 2 + 1023) / 1024 * 1024); }
 constexpr int kRingNormBytes = 80 * 1024;     // of those at most
 
-template <int EPI, int ROWS, int NB, int KS, int S, bool NORMED = false>
-int launch_ring(const SkinnyArgs& a, int row_groups, hipStream_t s) {
+template <int EPI, int ROWS, int NB, int KS, int S, bool NORMED, bool PAST>
+int launch_ring_form(const SkinnyArgs& a, int row_groups, hipStream_t s) {
   typedef RingShape<ROWS, NB, KS, S, NORMED> P;
-  auto kernel = gemm_ring_kernel<EPI, ROWS, NB, KS, S, NORMED>;
+  auto kernel = gemm_ring_kernel<EPI, ROWS, NB, KS, S, NORMED, PAST>;
   static bool raised = false;
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, P::kLdsBytes + (NORMED ? kRingNormBytes : 0)) !=
@@ -1029,6 +1040,13 @@ int launch_ring(const SkinnyArgs& a, int row_groups, hipStream_t s) {
   b.x_row_bytes = NORMED ? ring_row_bytes(a.k) : 0;
   kernel<<<grid, dim3(kThreads), P::kLdsBytes + (NORMED ? ring_norm_bytes(a.m, a.k, a.g_f32) : 0), s>>>(b);
   return check_launch("gemm_skinny");
+}
+
+// Past the caches where one group of rows reads the weight: another would find it gone (64 rows 2,048 x 5,632, two groups: in a step 2 % slower).
+template <int EPI, int ROWS, int NB, int KS, int S, bool NORMED = false>
+int launch_ring(const SkinnyArgs& a, int row_groups, hipStream_t s) {
+  return row_groups == 1 && passes_by(a.n, a.k, 2) ? launch_ring_form<EPI, ROWS, NB, KS, S, NORMED, true>(a, row_groups, s)
+                                                   : launch_ring_form<EPI, ROWS, NB, KS, S, NORMED, false>(a, row_groups, s);
 }
 
 constexpr int kSplitMinRows = 8;
