@@ -6,16 +6,19 @@
 // gemm_f32_stream_kernel, few rows (a decode step), bound by reading w once.  A workgroup owns 16 rows of w (or eight gate
 // rows and the eight up rows of the same outputs) and all of k, a share of it each of its 8 waves.  A wave's part of w and of x goes
 // from memory into a ring of its own in LDS without passing registers -- whole cache lines of 128 bytes a row (lanes that read 16
-// rows' 16 bytes straight into operand order keep the texture path busy four times as long), several steps of 32 k ahead and
+// rows' 16 bytes straight into operand order keep the texture path busy four times as long), two steps of 32 k ahead and
 // with no barrier; it reads its fragments there and feeds 16x16x4 MFMAs with w as the A operand.  The shares meet in LDS.
-// Eight rows, weights from memory, plain float FMA (gemm_generic) -> this: 32,000 x 2,048 149 -> 51 us (5.1 TB/s), 11,264 x 2,048 59 -> 20,
-// 2,048 x 5,632 82 -> 16, 2,048 x 2,048 32 -> 7.5; 64 rows 223 -> 159, 188 -> 57, 530 -> 23 and 196 -> 11.  With the attention of
+// Eight rows, weights from memory, plain float FMA (gemm_generic) -> this: 11,264 x 2,048 59 -> 17.2 us (5.4 TB/s), 2,048 x 5,632 82 -> 13.3,
+// 2,048 x 2,048 32 -> 7.4; 64 rows 188 -> 55, 530 -> 23 and 196 -> 11.  With the attention of
 // attention_f32.hip 32 decode steps of 8 requests after their prompts at TinyLlama's sizes take 213 -> 63 ms.
 // What a decode step does between these products -- two norms a layer, the rotation and the cache write, each a launch of 3 to 5 us
 // with next to nothing to do -- they do themselves: one that adds into the residual stream leaves, for the RMSNorm behind it, new
 // residual * g and every row's sum of squares in parts, a workgroup's outputs each (emit); a product whose x was so prepared applies the
 // rows' factor to its sums (ssq); and the q|k|v product holds a rotation's pairs in one workgroup (kRopeKv): a layer's eight
 // launches are five, 72 -> 63 us of kernels (8 rows, TinyLlama's sizes); eight prompts of 24 to 100 tokens and 31 such steps 64.1 -> 60.5 ms.
+// Parts of those sums that every wave asks for at once instead of two waves one after another, w past the caches and two steps ahead instead of
+// three to eight: 8 rows, the q|k|v product 10.1 -> 8.7 us, gates and ups 20.7 -> 18.9, down 15.9 -> 14.4; 16 rows 10.9 -> 9.5, 27.2 -> 20.6, 18.6 -> 17.6; those
+// prompts and steps 58.4 -> 53.6 ms.
 //
 // gemm_f32_tiled_kernel, many rows, bound by the matrix cores (157 TFLOP/s of float32 at the full clock).  A step's 32 k of the
 // tile's rows of x and of w go straight into a ring of stages in LDS; the waves feed 32x32x2 MFMAs from there and keep
@@ -85,8 +88,8 @@ __device__ inline int slot_key(int row) { return (row >> 1) & 7; }
 
 // N wave-wide loads to N KB of consecutive LDS as one statement, load i from its own scalar base and lane offsets: the LDS
 // address travels in m0, set once, and the loads' offset field (which moves the memory address too: taken off the base here)
-// steps through the stretch.
-template <int N>
+// steps through the stretch.  The weights' pieces (the first; the first two of three and more) past the caches or through them.
+template <int N, bool PAST>
 __device__ inline void load_pieces_to_lds(const float* const (&bases)[N], const unsigned (&offsets)[N], unsigned lds_first) {
   static_assert(N == 2 || N == 3 || N == 4 || N == 6, "one or two pieces of weights and one, two or four of x");
   constexpr int kMid = N / 2;
@@ -100,22 +103,29 @@ __device__ inline void load_pieces_to_lds(const float* const (&bases)[N], const 
   }
   const unsigned mid = __builtin_amdgcn_readfirstlane(lds_first + kMid * 1024);
 #define BC4G_PIECE(i, v, s) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #i "\n\t"
-  if constexpr (N == 2) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-1024, 1, 3) BC4G_PIECE(0, 2, 4)
-                 ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "s"(b[0]), "s"(b[1]) : "memory", "m0");
-  } else if constexpr (N == 3) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-1024, 1, 4) BC4G_PIECE(0, 2, 5) BC4G_PIECE(1024, 3, 6)
-                 ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "v"(offsets[2]), "s"(b[0]), "s"(b[1]), "s"(b[2]) : "memory", "m0");
-  } else if constexpr (N == 4) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-2048, 1, 5) BC4G_PIECE(-1024, 2, 6) BC4G_PIECE(0, 3, 7) BC4G_PIECE(1024, 4, 8)
-                 ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "v"(offsets[2]), "v"(offsets[3]), "s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3])
-                 : "memory", "m0");
+#define BC4G_WEIGHT(i, v, s, how) "global_load_lds_dwordx4 %" #v ", %" #s " offset:" #i how "\n\t"
+#define BC4G_PIECES(pieces, ...) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" pieces ::"s"(mid), __VA_ARGS__ : "memory", "m0")
+#define BC4G_STEP(how)                                                                                                                           \
+  if constexpr (N == 2)                                                                                                                          \
+    BC4G_PIECES(BC4G_WEIGHT(-1024, 1, 3, how) BC4G_PIECE(0, 2, 4), "v"(offsets[0]), "v"(offsets[1]), "s"(b[0]), "s"(b[1]));                      \
+  else if constexpr (N == 3)                                                                                                                     \
+    BC4G_PIECES(BC4G_WEIGHT(-1024, 1, 4, how) BC4G_WEIGHT(0, 2, 5, how) BC4G_PIECE(1024, 3, 6), "v"(offsets[0]), "v"(offsets[1]),                \
+                "v"(offsets[2]), "s"(b[0]), "s"(b[1]), "s"(b[2]));                                                                               \
+  else if constexpr (N == 4)                                                                                                                     \
+    BC4G_PIECES(BC4G_WEIGHT(-2048, 1, 5, how) BC4G_WEIGHT(-1024, 2, 6, how) BC4G_PIECE(0, 3, 7) BC4G_PIECE(1024, 4, 8), "v"(offsets[0]),         \
+                "v"(offsets[1]), "v"(offsets[2]), "v"(offsets[3]), "s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3]));                                  \
+  else                                                                                                                                           \
+    BC4G_PIECES(BC4G_WEIGHT(-3072, 1, 7, how) BC4G_WEIGHT(-2048, 2, 8, how) BC4G_PIECE(-1024, 3, 9) BC4G_PIECE(0, 4, 10) BC4G_PIECE(1024, 5, 11) \
+                    BC4G_PIECE(2048, 6, 12), "v"(offsets[0]), "v"(offsets[1]), "v"(offsets[2]), "v"(offsets[3]), "v"(offsets[4]),                \
+                "v"(offsets[5]), "s"(b[0]), "s"(b[1]), "s"(b[2]), "s"(b[3]), "s"(b[4]), "s"(b[5]));
+  if constexpr (PAST) {
+    BC4G_STEP(" nt")
   } else {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" BC4G_PIECE(-3072, 1, 7) BC4G_PIECE(-2048, 2, 8) BC4G_PIECE(-1024, 3, 9) BC4G_PIECE(0, 4, 10)
-                 BC4G_PIECE(1024, 5, 11) BC4G_PIECE(2048, 6, 12)
-                 ::"s"(mid), "v"(offsets[0]), "v"(offsets[1]), "v"(offsets[2]), "v"(offsets[3]), "v"(offsets[4]), "v"(offsets[5]), "s"(b[0]),
-                 "s"(b[1]), "s"(b[2]), "s"(b[3]), "s"(b[4]), "s"(b[5]) : "memory", "m0");
+    BC4G_STEP("")
   }
+#undef BC4G_STEP
+#undef BC4G_PIECES
+#undef BC4G_WEIGHT
 #undef BC4G_PIECE
 }
 
@@ -145,8 +155,8 @@ __device__ inline void wait_for_step(int later) {
 // 16.0 and 15.7).
 enum Norm : int { kNoNorm = 0, kFinishes = 1, kPrepares = 2 };
 
-// XR: rows of x a workgroup takes (blockIdx.y: which).  HALF: eight rows of w a workgroup instead of 16 (see launch_stream).
-template <int XR, int STAGES, int EPI, int NORM, bool HALF = false>
+// XR: rows of x a workgroup takes (blockIdx.y: which).  HALF: eight rows of w a workgroup instead of 16 (see launch_stream).  PAST: w past the caches.
+template <int XR, int STAGES, int EPI, int NORM, bool HALF, bool PAST>
 __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a) {
   constexpr int MT = (XR + 15) / 16, WP = HALF ? 1 : 2, PER = WP + XR / 8, kRing = PER * 1024;      // (WP: pieces of w a step)
   static_assert(!HALF || !paired(EPI), "half a block of a gated product would part gates and ups, of a rotated one a pair");
@@ -168,44 +178,6 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
   unsigned char* ring = stream_lds + wave * (STAGES * kRing);
   const unsigned ring_at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)ring));
 
-  // What is added to is asked for now: item j of a thread is output (threadIdx.x + j * kThreads) of the workgroup's.
-  constexpr int kItems = (XR * kCols + kThreads - 1) / kThreads;
-  float prev[kItems], bias[kItems], gain[kItems];
-  if constexpr (EPI == kAccum) {
-#pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const int idx = threadIdx.x + j * kThreads, row = idx / kCols, gn = n0 + idx % kCols;
-      const bool live = row < m && gn < n_out;
-      prev[j] = live ? a.out[static_cast<long>(row0 + row) * n_out + gn] : 0.f;
-      bias[j] = live && a.bias != nullptr ? a.bias[gn] : 0.f;
-      if constexpr (NORM == kPrepares) gain[j] = live ? a.emit_g[gn] : 0.f;
-    }
-  }
-  // So are a prepared x's parts of the rows' sums of squares -- sixteen chains a row, chain c adding blocks c, c + 16, ... in that order, the
-  // first kAhead of them (4,096 columns) asked for together --, and a rotation's angles and the places in the cache.
-  constexpr int kChains = 16, kAhead = 16;
-  const int part_row = min(static_cast<int>(threadIdx.x) % XR, m - 1), chain = threadIdx.x / XR;
-  const bool sums_parts = NORM == kFinishes && chain < kChains;
-  auto part_of = [&](int block) {
-    const long at = static_cast<long>(min(block, a.ssq_blocks - 1)) * a.m + row0 + part_row;
-    return a.ssq_halves ? reinterpret_cast<const float2*>(a.ssq)[at] : make_float2(a.ssq[at], 0.f);
-  };
-  float2 part[kAhead];
-  if (sums_parts) {
-#pragma unroll
-    for (int i = 0; i < kAhead; ++i) part[i] = part_of(chain + i * kChains);
-  }
-  float2 angle[kItems];
-  int slot[kItems];
-  if constexpr (EPI == kRopeKv) {
-#pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const int idx = threadIdx.x + j * kThreads, row = min(idx / kCols, m - 1);
-      angle[j] = a.rope.table != nullptr ? a.rope.table[static_cast<long>(row0 + row) * (head_dim / 2) + pair0 + idx % kCols] : make_float2(1.f, 0.f);
-      slot[j] = a.rope.write_kv && head >= a.rope.n_heads ? a.rope.slot_map[row0 + row] : 0;
-    }
-  }
-
   // Lane l of a load brings segment (l % 8) ^ key of the eight rows' row l / 8.  Rows beyond the matrix are read from its
   // last row (their results are not stored).
   const float* bases[PER];
@@ -226,6 +198,55 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
       offsets[i] = static_cast<unsigned>(min(r, m - 1)) * k * 4 + seg * 16;
     }
   }
+  // (the offsets before the loads below: a multiplication with a 64-bit addend takes whatever register is beside its own, and waits for it)
+  if constexpr (EPI == kAccum || EPI == kRopeKv || NORM == kFinishes) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) asm volatile("" : "+v"(offsets[i])::"memory");
+  }
+
+  // What is added to is asked for now: item j of a thread is output (threadIdx.x + j * kThreads) of the workgroup's.  (Every load is made, from a
+  // place that there is, and nothing is done with it before the walk: behind a branch, or for its sum, the compiler waits for it.)
+  constexpr int kItems = (XR * kCols + kThreads - 1) / kThreads;
+  float prev[kItems], bias[kItems], gain[kItems];
+  if constexpr (EPI == kAccum) {
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const int idx = threadIdx.x + j * kThreads, gn = min(n0 + idx % kCols, n_out - 1);
+      prev[j] = a.out[static_cast<long>(row0 + min(idx / kCols, m - 1)) * n_out + gn];
+      bias[j] = (a.bias != nullptr ? a.bias : a.out)[gn];
+      if constexpr (NORM == kPrepares) gain[j] = a.emit_g[gn];
+    }
+  }
+  // So are a prepared x's parts of the rows' sums of squares -- sixteen chains a row, chain c adding blocks c, c + 16, ... in that order, the
+  // first kAhead of them (4,096 columns) asked for together, two chains a wave --, and a rotation's angles and the places in the cache.
+  constexpr int kChains = 16, kAhead = 16, kWaveParts = 2 * kAhead * XR / kWave;
+  static_assert(kChains == 2 * kWaves && 2 * XR <= kWave, "two chains a wave, a lane for each row of both");
+  auto part_at = [&](int chain, int i, int row) {
+    return static_cast<unsigned>(min(chain + i * kChains, a.ssq_blocks - 1) * a.m + row0 + min(row, m - 1)) * (1 + a.ssq_halves);
+  };
+  constexpr bool kPairs = XR == 8;                           // (as many rows as halves come with; of more rows they are read after the walk)
+  float part[kWaveParts], second[kPairs ? kWaveParts : 1];   // (second: of a pair of halves, else the same once more)
+  if constexpr (NORM == kFinishes) {
+#pragma unroll
+    for (int j = 0; j < kWaveParts; ++j) {
+      const int idx = (j * kWave + lane) / XR;
+      const float* from = a.ssq + part_at(2 * wave + idx / kAhead, idx % kAhead, lane % XR);
+      part[j] = from[0];
+      if constexpr (kPairs) second[j] = from[a.ssq_halves];
+    }
+  }
+  float2 angle[kItems];
+  int slot[kItems];
+  const bool rotates = EPI == kRopeKv && a.rope.table != nullptr, writes = EPI == kRopeKv && a.rope.write_kv && head >= a.rope.n_heads;
+  if constexpr (EPI == kRopeKv) {
+#pragma unroll
+    for (int j = 0; j < kItems; ++j) {
+      const int idx = threadIdx.x + j * kThreads, row = min(idx / kCols, m - 1);
+      angle[j] = (rotates ? a.rope.table : reinterpret_cast<const float2*>(a.x))[rotates ? (row0 + row) * (head_dim / 2) + pair0 + idx % kCols : 0];
+      slot[j] = (writes ? a.rope.slot_map : reinterpret_cast<const int32_t*>(a.x))[writes ? row0 + row : 0];
+    }
+  }
+
   auto ask = [&](int s) {                                    // step s of this wave's
     const int k0 = (first + s) * kStepK;
     const float* b[PER];
@@ -236,7 +257,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
       // (a segment beyond the row's end: its row's first, it is not used)
       o[i] = k0 + kStepK <= k || k0 * 4 + static_cast<int>(back[i]) < k * 4 ? offsets[i] : offsets[i] - back[i];
     }
-    load_pieces_to_lds<PER>(b, o, ring_at + (s % STAGES) * kRing);
+    load_pieces_to_lds<PER, PAST>(b, o, ring_at + (s % STAGES) * kRing);
   };
 
   floatx4 acc[MT];
@@ -283,15 +304,32 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
   }
 
   __shared__ float part_sum[NORM == kFinishes ? kChains : 1][NORM == kFinishes ? XR : 1];
-  if (sums_parts) {
-    float ss = 0.f;
+  if constexpr (NORM == kFinishes) {
+    // through the wave's own ring, which is free
+    float* own = reinterpret_cast<float*>(ring);
+    static_assert(kWaveParts * kWave * 4 <= STAGES * kRing, "the parts fit the ring");
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) ss += chain + i * kChains < a.ssq_blocks ? part[i].x + part[i].y : 0.f;
-    for (int block = chain + kAhead * kChains; block < a.ssq_blocks; block += kChains) {
-      const float2 later = part_of(block);
-      ss += later.x + later.y;
+    for (int j = 0; j < kWaveParts; ++j) {
+      const int idx = (j * kWave + lane) / XR;
+      float other = 0.f;
+      if constexpr (kPairs) other = second[j];
+      asm volatile("" : "+v"(part[j]), "+v"(other));
+      if (!kPairs && a.ssq_halves) other = a.ssq[part_at(2 * wave + idx / kAhead, idx % kAhead, lane % XR) + 1];
+      own[j * kWave + lane] = 2 * wave + idx / kAhead + idx % kAhead * kChains < a.ssq_blocks ? part[j] + (a.ssq_halves ? other : 0.f) : 0.f;
     }
-    part_sum[chain][threadIdx.x % XR] = ss;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (lane < 2 * XR) {
+      const int chain = 2 * wave + lane / XR;
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) ss += own[(lane / XR * kAhead + i) * XR + lane % XR];
+      for (int i = kAhead; chain + i * kChains < a.ssq_blocks; ++i) {
+        const float* from = a.ssq + part_at(chain, i, lane % XR);
+        ss += from[0] + (a.ssq_halves ? from[1] : 0.f);
+      }
+      part_sum[chain][lane % XR] = ss;
+    }
   }
   __syncthreads();                                           // the rings' place takes the waves' sums
   typedef float Red[MT][16][kRedPad];
@@ -328,12 +366,14 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
     if constexpr (EPI == kRopeKv) {
       const RopeKv& r = a.rope;
       const bool is_v = head >= r.n_heads + r.n_kv_heads;
+      asm volatile("" : "+v"(angle[j].x), "+v"(angle[j].y), "+v"(slot[j]));
+      if (!rotates) angle[j] = make_float2(1.f, 0.f);
       const int i0 = pair0 + nl, i1 = i0 + head_dim / 2;
-      const float lo = is_v ? sum : sum * angle[j].x - up * angle[j].y, hi = is_v ? up : up * angle[j].x + sum * angle[j].y;
+      const float lo = is_v ? sum : fmaf(sum, angle[j].x, -(up * angle[j].y)), hi = is_v ? up : fmaf(up, angle[j].x, sum * angle[j].y);
       if (head < r.n_heads) {
         float* to = a.out + (static_cast<long>(row0 + row) * r.n_heads + head) * head_dim;
         to[i0] = lo, to[i1] = hi;
-      } else if (r.write_kv) {
+      } else if (writes) {
         const int kvh = is_v ? head - r.n_heads - r.n_kv_heads : head - r.n_heads, off = slot[j] % r.page_tokens;
         float* to = (is_v ? r.v_cache : r.k_cache) +
                     (static_cast<long>(slot[j] / r.page_tokens) * r.n_kv_heads + kvh) * head_dim * r.page_tokens;
@@ -344,7 +384,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
     }
     const long at = static_cast<long>(row0 + row) * n_out + gn;
     if constexpr (EPI == kAccum) {
-      const float nv = prev[j] + bias[j] + sum;
+      asm volatile("" : "+v"(prev[j]), "+v"(bias[j]));
+      const float nv = prev[j] + (a.bias != nullptr ? bias[j] : 0.f) + sum;
       if (live) a.out[at] = nv;
       if constexpr (NORM == kPrepares) {
         // the row's outputs of this workgroup lie in kCols neighbouring lanes
@@ -370,9 +411,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_stream_kernel(const Args a)
   }
 }
 
-template <int XR, int STAGES, int EPI, int NORM, bool HALF = false>
-int launch_stream_form(const Args& a, hipStream_t s) {
-  auto kernel = gemm_f32_stream_kernel<XR, STAGES, EPI, NORM, HALF>;
+template <int XR, int STAGES, int EPI, int NORM, bool HALF, bool PAST>
+int launch_stream_kernel(const Args& a, hipStream_t s) {
+  auto kernel = gemm_f32_stream_kernel<XR, STAGES, EPI, NORM, HALF, PAST>;
   constexpr int kLds = kWaves * STAGES * ((HALF ? 1 : 2) + XR / 8) * 1024;
   static_assert(kLds <= 160 * 1024, "a workgroup's LDS");
   static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
@@ -386,6 +427,13 @@ int launch_stream_form(const Args& a, hipStream_t s) {
   return 0;
 }
 
+// Past the caches where one workgroup alone reads a part of w (64 rows, two workgroups a part: 11,264 x 2,048 54.4 us and 59.4 past them).
+template <int XR, int STAGES, int EPI, int NORM, bool HALF = false>
+int launch_stream_form(const Args& a, hipStream_t s) {
+  return a.m <= XR && passes_by(a.n, a.k, 4) ? launch_stream_kernel<XR, STAGES, EPI, NORM, HALF, true>(a, s)
+                                             : launch_stream_kernel<XR, STAGES, EPI, NORM, HALF, false>(a, s);
+}
+
 // Outputs a workgroup of few rows' kernel takes of a product that stores or adds.
 int stream_cols(int m, int n) { return m <= 8 && 2 * ((n + 15) / 16) <= compute_units() ? 8 : 16; }
 
@@ -396,13 +444,14 @@ int launch_stream(const Args& a, hipStream_t s) {
   // same sums.  A decode step's two such products, 2,048 x 2,048 and
   // 2,048 x 5,632, from memory, 8 rows, inside a step: 13.05 -> 11.7 us on average; 32 steps of 8 requests after their prompts 67.6 -> 63.5 ms.
   if constexpr (!paired(EPI)) {
-    if (stream_cols(a.m, n_out) == 8) return launch_stream_form<8, 8, EPI, NORM, true>(a, s);
+    if (stream_cols(a.m, n_out) == 8) return launch_stream_form<8, 2, EPI, NORM, true>(a, s);
   }
-  // One workgroup a CU where there are no more: a ring as deep as LDS allows.  Else two that overlap.
-  const bool few = (n_out + cols - 1) / cols <= compute_units();
-  if (a.m <= 8) return few ? launch_stream_form<8, 6, EPI, NORM>(a, s) : launch_stream_form<8, 3, EPI, NORM>(a, s);
-  if (a.m <= 16) return few ? launch_stream_form<16, 4, EPI, NORM>(a, s) : launch_stream_form<16, 2, EPI, NORM>(a, s);
-  return few && a.m <= 32 ? launch_stream_form<32, 3, EPI, NORM>(a, s) : launch_stream_form<32, 2, EPI, NORM>(a, s);
+  // Two steps ahead, so that a CU holds up to three workgroups: more of them in flight were slower in every product whose weights come from memory
+  // (8 rows: 2,048 x 5,632 rings of 8 steps 16.5 us, of 4 15.3, of 2 14.5; 2,560 x 2,048 of 6 10.0, of 3 9.2, of 2 8.7; 16 rows 11,264 x 2,048 of 3
+  // 26.6, of 2 20.7).
+  if (a.m <= 8) return launch_stream_form<8, 2, EPI, NORM>(a, s);
+  if (a.m <= 16) return launch_stream_form<16, 2, EPI, NORM>(a, s);
+  return launch_stream_form<32, 2, EPI, NORM>(a, s);
 }
 
 // ---- many rows ----------------------------------------------------------------------------------

@@ -115,3 +115,22 @@ def test_refusals(ops):
         ops.gemm_f32_emit(x[:3].contiguous(), w, torch.zeros(4, 96, device=DEV), g, EPS)
     with pytest.raises(KernelError):
         ops.gemm_f32_qkv(x[:3].contiguous(), w, None, None, None, None, 4, 2, 32, write_kv=False)
+
+
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 32, 33])
+def test_large_weights_as_small_ones(ops, m):
+    """A weight that is read past the caches against its halves, which are not: the same bits in every column."""
+    gen = torch.Generator(device=DEV).manual_seed(m)
+    f = lambda *shape: torch.randn(*shape, generator=gen, device=DEV)      # noqa: E731
+    n, k = 816, 2052
+    assert n * k * 4 >= 6 << 20 > n // 2 * k * 4
+    x, w, add, g = f(m, k), 0.1 * f(n, k), f(m, n), 1.0 + 0.2 * f(k)
+    halves = [w[:n // 2].contiguous(), w[n // 2:].contiguous()]
+    assert torch.equal(ops.gemm_f32(x, w), torch.cat([ops.gemm_f32(x, h) for h in halves], 1))
+    added = [ops.gemm_f32(x, h, accumulate_into=a.contiguous()) for h, a in zip(halves, add.chunk(2, 1))]
+    assert torch.equal(ops.gemm_f32(x, w, accumulate_into=add.clone()), torch.cat(added, 1))
+    pre = ops.gemm_f32_emit(f(m, 36), f(k, 36), f(m, k), g, EPS)
+    assert torch.equal(ops.gemm_f32_prenormed(pre, w), torch.cat([ops.gemm_f32_prenormed(pre, h) for h in halves], 1))
+    order = torch.cat([torch.arange(0, n // 4), torch.arange(n // 2, 3 * n // 4)])
+    gates = torch.cat([ops.gemm_f32_prenormed(pre, w[(order + d).to(w.device)].contiguous(), "silu") for d in (0, n // 4)], 1)
+    assert torch.equal(ops.gemm_f32_prenormed(pre, w, "silu"), gates)
