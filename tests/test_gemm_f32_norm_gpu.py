@@ -127,7 +127,7 @@ def test_large_weights_as_small_ones(ops, m):
     x, w, add, g = f(m, k), 0.1 * f(n, k), f(m, n), 1.0 + 0.2 * f(k)
     halves = [w[:n // 2].contiguous(), w[n // 2:].contiguous()]
     assert torch.equal(ops.gemm_f32(x, w), torch.cat([ops.gemm_f32(x, h) for h in halves], 1))
-    added = [ops.gemm_f32(x, h, accumulate_into=a.contiguous()) for h, a in zip(halves, add.chunk(2, 1))]
+    added = [ops.gemm_f32(x, h, accumulate_into=a.clone(memory_format=torch.contiguous_format)) for h, a in zip(halves, add.chunk(2, 1))]
     assert torch.equal(ops.gemm_f32(x, w, accumulate_into=add.clone()), torch.cat(added, 1))
     pre = ops.gemm_f32_emit(f(m, 36), f(k, 36), f(m, k), g, EPS)
     assert torch.equal(ops.gemm_f32_prenormed(pre, w), torch.cat([ops.gemm_f32_prenormed(pre, h) for h in halves], 1))
