@@ -45,3 +45,17 @@ def test_parts_of_k(ops, m, n, k, parts):
     for p in range(parts):
         want = x[:, p * step:(p + 1) * step].double() @ w[:, p * step:(p + 1) * step].double().T
         assert (out[p].double() - want).abs().max() < 2.0 * step * 2.0 ** -24 * math.sqrt(step)
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 11264, 2048), (64, 11250, 2048), (64, 9600, 4096)])
+def test_weights_past_the_caches(ops, m, n, k):
+    """One tile of rows of a large weight, which is read past the caches, against the same rows among more of them: the same bits."""
+    assert not ops.streams_weights(m, n, k) and ops.tiled_tile(m, n, k) == (64, 64) and n * k * 2 >= 6 << 20
+    x, w = rnd(65, k, seed=6).to(DEV), (rnd(n, k, seed=7) * k ** -0.5).to(DEV)
+    few = x[:m].contiguous()
+    got = ops.gemm_fast(few, w, torch.float32)
+    assert torch.equal(got, ops.gemm_fast(x, w, torch.float32)[:m])
+    assert torch.equal(ops.gemm_fast(few, w, torch.bfloat16), ops.gemm_fast(x, w, torch.bfloat16)[:m])
+    assert (got.double() - few.double() @ w.double().T).abs().max() < 2.0 * k * 2.0 ** -24
+    if n % 16 == 0:
+        assert torch.equal(ops.gemm_swiglu(few, w, True), ops.gemm_swiglu(x, w, True)[:m])
