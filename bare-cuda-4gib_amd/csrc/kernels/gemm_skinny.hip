@@ -29,7 +29,7 @@
 //            (below), together with parts of every row's sum of squares: the row's scale is worked out
 //            from the parts while the weights are on their way and multiplies the finished sum -- the
 //            norm costs neither a kernel of its own nor the staging of the float rows.
-// Plain and prenormed rows go through rings in LDS where k is a multiple of 64 (gemm_ring_kernel, below): the same bits.
+// Plain and prenormed rows, and few normed ones, go through rings in LDS where k is a multiple of 64 (gemm_ring_kernel, below): the same bits.
 // What goes out (EPI): bfloat16 or float stored; bfloat16 after max(., 0)^2 or xIELU (8 rows,
 // 2,048 to 8,192: product with its norm inside 13.0 us and the activation behind it 5.5; normed before and activated here 8.8);
 // float added into the residual stream; SwiGLU,
@@ -82,7 +82,7 @@ struct SkinnyArgs {
   int last_block;           // the last block of w,
   int part_stride;          // numbers from one part to the next, and where the last four of all parts begin
   int last_four;
-  int x_row_bytes, g_f32;   // ring kernel, normed modes: LDS of a wave's part of a row of x; whether g is float
+  int x_row_bytes, g_f32;   // ring kernel, normed modes: LDS of a float row of x; whether g is float
   int ssq_blocks, ssq_stride;
   int ssq_halves;           // the parts are pairs, [ssq_blocks][ssq_stride][2]
   float eps;
@@ -797,7 +797,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
   const unsigned char* w_at[TB];
 #pragma unroll
   for (int b = 0; b < TB; ++b)
-    w_at[b] = reinterpret_cast<const unsigned char*>(a.w) + (static_cast<size_t>(min(first_block + b, a.last_block)) * (static_cast<unsigned>(k) / 32) + static_cast<unsigned>(k_begin) / 32) * 1024;
+    w_at[b] = reinterpret_cast<const unsigned char*>(a.w) +
+              (static_cast<size_t>(min(first_block + b, a.last_block)) * (static_cast<unsigned>(k) / 32) + static_cast<unsigned>(k_begin) / 32) * 1024;
   const unsigned char* x_at = static_cast<const unsigned char*>(a.x) + static_cast<unsigned>(k_begin) * 2;
   auto ask = [&](int t) {
     const unsigned to = ring + (t % S) * P::kStageBytes;
@@ -1099,7 +1100,8 @@ bool normed_ring_operands(const SkinnyArgs& a) {
 // What the rings take: the loads bring 16 bytes from 16-byte boundaries, a stage is 64 values of k, parts of a norm are read four numbers at a time and the
 // next norm's scale two.
 bool ring_operands(const SkinnyArgs& a) {
-  return a.k % 64 == 0 && (a.ssq_parts == nullptr || static_cast<long>(a.ssq_blocks) * a.ssq_stride >= 4) && (a.emit_g == nullptr || a.n > 1) && reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0;
+  return a.k % 64 == 0 && (a.ssq_parts == nullptr || static_cast<long>(a.ssq_blocks) * a.ssq_stride >= 4) && (a.emit_g == nullptr || a.n > 1) &&
+         reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0;
 }
 
 constexpr int kMaxStageBytes = 96 * 1024;
