@@ -122,7 +122,19 @@ __device__ inline void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "me
 constexpr int kMergePad = 4;   // floats between rows of the partial outputs in LDS
 
 // EXACT: the head size is exactly 16 * DB (the usual sizes 64, 128, 256): no test against it is left.
-template <int DJ, int DB, int QT, int WS, bool EXACT>
+// 16 or 8 bytes, past the caches (PAST) or through them.
+template <bool PAST, typename T>
+__device__ inline T load_once(const void* p) {
+  typedef uint32_t Words __attribute__((ext_vector_type(sizeof(T) / 4)));
+  const Words* from = reinterpret_cast<const Words*>(p);
+  Words v;
+  if constexpr (PAST) v = __builtin_nontemporal_load(from);
+  else v = *from;
+  return __builtin_bit_cast(T, v);
+}
+
+// PAST: keys and values past the caches, where one workgroup reads them (see launch_attention).
+template <int DJ, int DB, int QT, int WS, bool EXACT, bool PAST>
 __global__ __launch_bounds__((WS > 1 ? WS : kWavesPerBlock) * kWave, 2) void attention_mfma_kernel(
     const AttnArgs a) {
   static_assert(WS <= 1 || QT == 1, "waves share a tile's keys for single query tiles only");
@@ -337,10 +349,10 @@ __global__ __launch_bounds__((WS > 1 ? WS : kWavesPerBlock) * kWave, 2) void att
         const bf16_t* vbase = a.v_cache + block_at[h];
 #pragma unroll
         for (int j = 0; j < DJ; ++j)
-          t.k[h][j] = (t.ok[h] && (EXACT || 32 * j + 8 * grp < d)) ? load16(kbase + 512 * j + k_lane) : zero16();
+          t.k[h][j] = (t.ok[h] && (EXACT || 32 * j + 8 * grp < d)) ? load_once<PAST, uint4>(kbase + 512 * j + k_lane) : zero16();
 #pragma unroll
         for (int b = 0; b < DB; ++b)
-          t.v[h][b] = (t.ok[h] && (EXACT || 16 * b < d)) ? *reinterpret_cast<const uint2*>(vbase + 256 * b + v_lane)
+          t.v[h][b] = (t.ok[h] && (EXACT || 16 * b < d)) ? load_once<PAST, uint2>(vbase + 256 * b + v_lane)
                                               : make_uint2(0u, 0u);
       }
     }
@@ -820,25 +832,25 @@ using namespace bc4g;
 
 namespace bc4g {
 namespace {
-template <int DJ, int DB, int QT, int WS>
+template <int DJ, int DB, int QT, int WS, bool PAST = false>
 int launch_attention(const AttnArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
   // per instantiation, once: the staged form's ring may need more than the default dynamic LDS
   static std::once_flag once;
   static hipError_t raised = hipSuccess;
   if (lds > 48 * 1024) {
     std::call_once(once, [] {
-      raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_mfma_kernel<DJ, DB, QT, WS, true>),
+      raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_mfma_kernel<DJ, DB, QT, WS, true, PAST>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
       if (raised == hipSuccess)
-        raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_mfma_kernel<DJ, DB, QT, WS, false>),
+        raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_mfma_kernel<DJ, DB, QT, WS, false, PAST>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     });
     if (raised != hipSuccess)
       return fail("attention_mfma: cannot raise the dynamic LDS limit to the %zu bytes of the key tiles' ring (%s)", lds,
                   hipGetErrorString(raised));
   }
-  if (a.head_dim == 16 * DB) attention_mfma_kernel<DJ, DB, QT, WS, true><<<grid, block, lds, s>>>(a);
-  else attention_mfma_kernel<DJ, DB, QT, WS, false><<<grid, block, lds, s>>>(a);
+  if (a.head_dim == 16 * DB) attention_mfma_kernel<DJ, DB, QT, WS, true, PAST><<<grid, block, lds, s>>>(a);
+  else attention_mfma_kernel<DJ, DB, QT, WS, false, PAST><<<grid, block, lds, s>>>(a);
   return 0;
 }
 }  // namespace
@@ -935,9 +947,18 @@ extern "C" int bc4g_attention_mfma_counted(const void* qkv, int q_stride, void* 
     // one workgroup per tile; its waves (8, or 4 for the largest heads) cut the keys between them
     dim3 grid(n_tiles, n_kv_heads * a.n_sub, n_splits);
     auto lds = [&](int ws) { return static_cast<size_t>(ws) * 16 * (head_dim + kMergePad + 2) * sizeof(float); };
-    if (dj <= 2 && db <= 4) status = launch_attention<2, 4, 1, 8>(a, grid, 8 * kWave, lds(8), s);
-    else if (dj <= 4 && db <= 8) status = launch_attention<4, 8, 1, 8>(a, grid, 8 * kWave, lds(8), s);
-    else status = launch_attention<8, 16, 1, 4>(a, grid, 4 * kWave, lds(4), s);
+    // A decode step's requests, one row each and the heads of a KV head in one tile: every key is read once.  Where the block tables have room for 32 MB
+    // and more of keys and values a layer, the layers behind it will have put them out by the next step: past the caches, as large weights go (16
+    // requests of 1,000 tokens, 32 KV heads of 128 52.8 -> 47.8 us a layer, 5.5 TB/s; 8 of 4,000, 8 KV heads 31.4 -> 28.1; but 22 layers of 8 requests of 540
+    // tokens, 4 KV heads of 64, whose 97 MB stay: a step 1.4 % slower).
+    constexpr long kRoom = 32L << 20;
+    const bool past = single_rows && a.n_sub == 1 && static_cast<long>(n_seqs) * table_stride * page_tokens * n_kv_heads * head_dim * 4 >= kRoom;
+    if (dj <= 2 && db <= 4)
+      status = past ? launch_attention<2, 4, 1, 8, true>(a, grid, 8 * kWave, lds(8), s) : launch_attention<2, 4, 1, 8>(a, grid, 8 * kWave, lds(8), s);
+    else if (dj <= 4 && db <= 8)
+      status = past ? launch_attention<4, 8, 1, 8, true>(a, grid, 8 * kWave, lds(8), s) : launch_attention<4, 8, 1, 8>(a, grid, 8 * kWave, lds(8), s);
+    else
+      status = past ? launch_attention<8, 16, 1, 4, true>(a, grid, 4 * kWave, lds(4), s) : launch_attention<8, 16, 1, 4>(a, grid, 4 * kWave, lds(4), s);
   } else {
     dim3 grid((n_tiles + kWavesPerBlock - 1) / kWavesPerBlock, n_kv_heads * a.n_sub, n_splits);
     dim3 block(kWavesPerBlock * kWave);

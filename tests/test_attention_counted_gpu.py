@@ -72,3 +72,21 @@ def test_too_few_counters_are_refused(ops):
 def test_counters_go_up_with_the_batch(ops):
     assert ops.attention_counters(8, 32, 4) == {"arrived": [0] * 32} and ops.attention_counters(33, 32, 4) == {} == ops.attention_counters(0, 32, 4)
     assert ops.attention_counters(1, 64, 2) == {"arrived": [0] * 4}
+
+
+@pytest.mark.parametrize("n_splits", [1, 3])
+@pytest.mark.parametrize("S, heads, kv_heads, d", [(16, 32, 8, 64), (8, 32, 8, 128), (4, 8, 8, 256), (5, 16, 16, 80)])
+def test_room_for_much_as_for_little(ops, S, heads, kv_heads, d, n_splits):
+    """Block tables with room for 32 MB of keys and values and more, which are then read past the caches, against tables as wide as the contexts."""
+    gen = torch.Generator().manual_seed(S + d)
+    page, width = 64, 4
+    draw = lambda *shape: torch.randn(*shape, generator=gen).bfloat16().to(DEV)      # noqa: E731
+    kc, vc, q = draw(S * width, kv_heads, page, d), draw(S * width, kv_heads, d, page), draw(S, heads * d)
+    table = torch.randperm(S * width, generator=gen).view(S, width).int().to(DEV)
+    ctx = torch.randint(1, width * page, (S,), generator=gen).int().to(DEV)
+    rows = torch.arange(S + 1, dtype=torch.int32, device=DEV)
+    room = -(-(32 << 20) // (S * page * kv_heads * d * 4))
+    wide = torch.full((S, room), -1, dtype=torch.int32, device=DEV)
+    wide[:, :width] = table
+    one, two = (ops.attention_mfma(q, kc, vc, t, rows, ctx, rows, S, heads, kv_heads, d, 0, d ** -0.5, n_splits, 1, 1, single_rows=True) for t in (table, wide))
+    assert room > width and torch.equal(one, two)
