@@ -131,7 +131,9 @@ __device__ inline SkinnyArgs own_rows(const SkinnyArgs& args) {
 
 // What an output's thread has at hand before its sum is there.
 struct Kept {
-  float prev, g;              // kAccumF32: what the sum is added to (with the bias), and the next norm's scale
+  float prev;                 // kAccumF32: what the sum is added to (with the bias),
+  bool ask_g;                 // whether the next norm's scale is yet to be asked for (behind the store of the sum), or
+  float g;                    // that scale
   float cs, sn;               // kRopeKvBf16: its pair's rotation ...
   int slot;                   // ... and place in the cache
   float xielu_p, xielu_q;
@@ -173,7 +175,7 @@ __device__ inline void put_output(const SkinnyArgs& a, int n0, int wblock_index,
       // of squares (a row's 16 columns, or eight of half a block, lie in as many neighbouring lanes)
       float sq = 0.f;
       if (live) {
-        a.emit_x[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(nv * kept.g);
+        a.emit_x[static_cast<long>(row) * a.n + gn] = from_float<bf16_t>(nv * (kept.ask_g ? emit_scale(a, gn) : kept.g));
         sq = nv * nv;
       }
 #pragma unroll
@@ -229,6 +231,10 @@ template <int MT, int EPI, int XMODE, int U, int ROWS = 16, bool HALF = false>
 // a 5,632 x 2 wide gate-up matrix are in flight at once.)
 __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) ? 6 : U == 8 ? 2 : 4) void gemm_skinny_kernel(const SkinnyArgs args) {
   constexpr bool kNormed = XMODE != kPlain;
+  // Every line of the arguments in one trip: left to itself the compiler asks for the norm's, in the second line, behind the first loads, and waits
+  // for them there (one row, weights from memory: 768 x 768 after a prepared norm 3.20 and 3.07 us, 32,000 x 512 8.6 and 7.9).
+  if constexpr (!kNormed) asm volatile("" ::"s"(args.m), "s"(args.ssq_blocks), "s"(args.ssq_stride), "s"(args.ssq_halves), "s"(args.eps));
+  if constexpr (EPI == kAccumF32) asm volatile("" ::"s"(args.bias), "s"(args.emit_stride));
   const SkinnyArgs a = kNormed ? args : own_rows<EPI>(args);
   constexpr bool kTurned = !kNormed;                      // x reaches operand order through LDS
   constexpr int kPieces = 4 * U;                       // 16-byte pieces of a row in one batch of k-steps
@@ -609,9 +615,8 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
       sum *= scale;
       partner *= scale;
     }
-    const float g = EPI == kAccumF32 && a.emit_g != nullptr && live ? emit_scale(a, gn) : 0.f;
     put_output<EPI, kCols, HALF>(a, n0, wblock_index, half, row, nl, idx < MT * 16 * kCols, live, sum, partner,
-                                 Kept{EPI == kAccumF32 ? prev[j] : 0.f, g, EPI == kRopeKvBf16 ? rope_cs[j] : 1.f, EPI == kRopeKvBf16 ? rope_sn[j] : 0.f,
+                                 Kept{EPI == kAccumF32 ? prev[j] : 0.f, EPI == kAccumF32, 0.f, EPI == kRopeKvBf16 ? rope_cs[j] : 1.f, EPI == kRopeKvBf16 ? rope_sn[j] : 0.f,
                                       EPI == kRopeKvBf16 ? rope_slot[j] : 0, xielu_p, xielu_q});
   }
 }
@@ -1003,7 +1008,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
         partner *= scale;
       }
     }
-    Kept kept{0.f, 0.f, 1.f, 0.f, 0, xielu_p, xielu_q};
+    Kept kept{0.f, false, 0.f, 1.f, 0.f, 0, xielu_p, xielu_q};
     if constexpr (EPI == kAccumF32) {
       asm volatile("" : "+v"(prev[j]), "+v"(bias[j]), "+v"(g[j]));            // (nothing done with them before the walk, where it would wait for them)
       kept.prev = a.bias != nullptr ? prev[j] + bias[j] : prev[j];
