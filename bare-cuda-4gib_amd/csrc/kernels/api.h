@@ -236,6 +236,9 @@ int bc4g_gemm_mfma_tile(const void* a, const void* w, int m, int n, int k, int q
 // How it cuts the output: *first_cols columns (n: all) in those tiles, the others in tiles of *rows x *cols (0, 0: there are none) by a
 // second launch; *beyond 1: rows beyond whole tiles in 64 x 256 tiles in the same launch.  Launches nothing.
 int bc4g_gemm_mfma_cut(const void* a, const void* w, int m, int n, int k, int qkv, int* first_cols, int* rows, int* cols, int* beyond);
+// Whether a few-row product of aligned operands whose norm is not fused goes through rings in LDS (rings: 1) or to the streaming kernel (0), by its
+// epilogue and whether it finishes a prepared norm.
+int bc4g_gemm_skinny_rings(int m, int n, int k, int epilogue, int finishes_norm, int* rings);
 // The q|k|v product of many rows with rotation and cache write in its epilogue, as bc4g_gemm_skinny_qkv for few (k a
 // multiple of 64, operands on 16-byte boundaries): w [n, k] holds n_heads query, n_kv_heads key and as many value heads of
 // head_dim (a multiple of 16), every head's rows in blocks of eight dimensions followed by their rotation partners.  out

@@ -1119,6 +1119,16 @@ bool ring_operands(const SkinnyArgs& a) {
          reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0;
 }
 
+// Which of those the streaming kernel takes all the same, because it is the faster one for them (the same bits from either).  us, weights from memory,
+// streaming kernel and rings:
+// - more than 32 rows and more than one and a half blocks a CU (beyond two the tiled kernel takes the product): the rings' two groups of rows are then
+//   more workgroups than run at once.  48 rows 8,000 x 1,024 8.0 and 10.7, 7,168 x 4,096 21.9 and 26.7, 64 rows 25.7 and 28.3; but 6,144 x 4,096 25.4 and 17.8.
+bool rings_are_slower([[maybe_unused]] int epilogue, int m, int n, [[maybe_unused]] int k, [[maybe_unused]] bool finishes_norm) {
+  const int blocks = (n + 15) / 16, cus = compute_units();
+  if (m > 32 && 2 * blocks > 3 * cus) return true;
+  return false;
+}
+
 constexpr int kMaxStageBytes = 96 * 1024;
 
 template <int EPI, int XMODE>
@@ -1140,8 +1150,7 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
     }
     kernel<<<grid, block, stage, s>>>(a);
   } else {
-    if (ring_operands(a)) return launch_rings<EPI>(a, s);
-    // (From here on k that is no multiple of 64, or operands off 16-byte boundaries.)
+    if (ring_operands(a) && !rings_are_slower(EPI, a.m, a.n, a.k, a.ssq_parts != nullptr)) return launch_rings<EPI>(a, s);
     // Every workgroup reads all its rows of x, and what a CU can pull through its cache is what bounds
     // the kernel once x is as large as the block's weights (16 rows).  Where the weight blocks are
     // few (up to one a CU: n = 4,096), two workgroups share a block's rows: each pulls half of
@@ -1336,6 +1345,14 @@ extern "C" int bc4g_gemm_skinny_prenormed(const void* x, const float* ssq_parts,
   a.ssq_halves = ssq_halves ? 1 : 0;
   a.eps = eps;
   return launch_epilogue<kPlain>(a, epilogue, static_cast<hipStream_t>(stream));
+}
+
+// Whether a product of aligned operands whose norm is not fused goes through rings in LDS (rings: 1) or to the streaming kernel (0).
+extern "C" int bc4g_gemm_skinny_rings(int m, int n, int k, int epilogue, int finishes_norm, int* rings) {
+  if (int e = check_common("gemm_skinny_rings", m, 64, n, k, epilogue)) return e;
+  BC4G_REQUIRE(rings != nullptr, "gemm_skinny_rings: a place for the answer");
+  *rings = k % 64 == 0 && !rings_are_slower(epilogue, m, n, k, finishes_norm != 0) ? 1 : 0;
+  return 0;
 }
 
 extern "C" int bc4g_gemm_skinny_normed(const float* x, const int32_t* rows, const void* g, int g_dtype,

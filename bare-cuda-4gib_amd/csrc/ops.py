@@ -96,6 +96,14 @@ def tiled_cut(m: int, n: int, k: int, qkv: bool = False) -> Tuple[int, Optional[
     return first.value, (rows.value, cols.value) if first.value < n else None, bool(beyond.value)
 
 
+def skinny_rings(m: int, n: int, k: int, epilogue: int = 0, finishes_norm: bool = False) -> bool:
+    """Whether the few-row product of aligned operands, with this epilogue and a prepared norm to finish or none, goes through rings in LDS (else
+    to the streaming kernel, for the same bits)."""
+    rings = ctypes.c_int(0)
+    library.call("bc4g_gemm_skinny_rings", m, n, k, epilogue, int(finishes_norm), ctypes.byref(rings), launches=False)
+    return bool(rings.value)
+
+
 def _tiled_cost(m: int, n: int, k: int, out_bytes: float, qkv: bool = False):
     if not _profiler.enabled:
         return None

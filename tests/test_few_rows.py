@@ -29,6 +29,15 @@ def test_half_blocks_leave_a_block_for_every_other_cu(monkeypatch, units, most):
     assert not ops.half_blocks(9, 16, 2048) and not ops.half_blocks(8, 16, 1016)
 
 
+@pytest.mark.parametrize("k", [1024, 4096])
+def test_rings_leave_many_rows_of_wide_outputs_to_the_streaming_kernel(k):
+    """Two groups of rows of more than one and a half blocks of outputs a CU are more workgroups than run at once."""
+    edge = 16 * (3 * ops.compute_units() // 2)
+    assert ops.skinny_rings(33, edge, k) and ops.skinny_rings(64, edge, k) and ops.skinny_rings(32, edge + 1, k)
+    assert not ops.skinny_rings(33, edge + 1, k) and not ops.skinny_rings(64, 2 * edge, k)
+    assert not ops.skinny_rings(8, 2048, k + 32)
+
+
 @pytest.mark.parametrize("k", [6, (1 << 24) + 4])
 def test_float32_products_leave_what_their_kernels_refuse_to_the_plain_one(k):
     row = torch.empty(1, k)
