@@ -1123,9 +1123,22 @@ bool ring_operands(const SkinnyArgs& a) {
 // streaming kernel and rings:
 // - more than 32 rows and more than one and a half blocks a CU (beyond two the tiled kernel takes the product): the rings' two groups of rows are then
 //   more workgroups than run at once.  48 rows 8,000 x 1,024 8.0 and 10.7, 7,168 x 4,096 21.9 and 26.7, 64 rows 25.7 and 28.3; but 6,144 x 4,096 25.4 and 17.8.
-bool rings_are_slower([[maybe_unused]] int epilogue, int m, int n, [[maybe_unused]] int k, [[maybe_unused]] bool finishes_norm) {
+// - wide outputs of a short k: a workgroup's walk is one or two stages, and its rings only make a launch of many workgroups longer.  Up to 8 rows, from three
+//   blocks a CU on: k up to 512, but for a gated product behind a prepared norm, and plain stores up to 768 (128,256 x 512 behind a norm, one row 22.9 and 29.7,
+//   gated 30.6 and 30.3; 32,000 x 512 8 rows 8.4 and 10.0; 32,000 x 768 stored, one row 10.1 and 10.3, behind a norm 13.2 and 11.8; 12,288 x 512 4.76 and 4.75).
+//   Four blocks a CU behind a norm also at 1,024: 8 rows 8.2 and 8.8.  9 to 16 rows, from two blocks a CU on: k up to 512 (128,256 x 512 26.1 and 37.8, 12,288 x 512
+//   behind a norm 5.1 and 6.3; but 8,192 x 512 4.7 and 4.4), up to 1,024 what neither adds nor rotates nor finishes a norm before gates (32,000 x 768 stored 11.7 and
+//   13.6, rotated 17.7 and 16.1, gated behind a norm 15.5 and 15.1; 32,000 x 1,152 16.0 and 16.3).
+bool rings_are_slower(int epilogue, int m, int n, int k, bool finishes_norm) {
   const int blocks = (n + 15) / 16, cus = compute_units();
   if (m > 32 && 2 * blocks > 3 * cus) return true;
+  const bool adds = epilogue == kAccumF32, rotates = epilogue == kRopeKvBf16, gates_normed = gated(epilogue) && finishes_norm;
+  if (m > kSplitMinRows && m <= 16 && blocks > 2 * cus) return k <= 512 || (k <= 1024 && !adds && !rotates && !gates_normed);
+  if (m <= kSplitMinRows && blocks > 3 * cus) {
+    if (k <= 512) return !gates_normed;
+    if (adds || rotates || gated(epilogue)) return false;
+    return finishes_norm ? k > 768 && k <= 1024 && blocks <= 4 * cus : k <= 768;
+  }
   return false;
 }
 

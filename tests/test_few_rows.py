@@ -38,6 +38,26 @@ def test_rings_leave_many_rows_of_wide_outputs_to_the_streaming_kernel(k):
     assert not ops.skinny_rings(8, 2048, k + 32)
 
 
+def test_rings_leave_wide_outputs_of_a_short_k_to_the_streaming_kernel():
+    """Workgroups of one or two stages each, many of them: by rows, blocks a CU, k and what follows the sums."""
+    block = 16 * ops.compute_units()
+    for m in (1, 8):
+        for epilogue in (ops.EPI_STORE_BF16, ops.EPI_STORE_F32, ops.EPI_SQUARED_RELU, ops.EPI_ACCUM_F32):
+            assert not ops.skinny_rings(m, 3 * block + 1, 64, epilogue) and not ops.skinny_rings(m, 30 * block, 512, epilogue)
+            assert ops.skinny_rings(m, 3 * block, 512, epilogue) and ops.skinny_rings(m, 30 * block, 832, epilogue)
+            assert ops.skinny_rings(m, 30 * block, 768, epilogue) == (epilogue == ops.EPI_ACCUM_F32)
+        assert not ops.skinny_rings(m, 8 * block, 512, ops.EPI_STORE_F32, True) and ops.skinny_rings(m, 8 * block, 576, ops.EPI_STORE_F32, True)
+        assert not ops.skinny_rings(m, 4 * block, 1024, ops.EPI_STORE_F32, True) and ops.skinny_rings(m, 5 * block, 1024, ops.EPI_STORE_F32, True)
+        assert not ops.skinny_rings(m, 8 * block, 512, ops.EPI_SWIGLU) and ops.skinny_rings(m, 8 * block, 512, ops.EPI_SWIGLU, True)
+    for m in (9, 16):
+        for epilogue in (ops.EPI_STORE_BF16, ops.EPI_SWIGLU):
+            assert not ops.skinny_rings(m, 2 * block + 16, 1024, epilogue) and ops.skinny_rings(m, 2 * block, 512, epilogue)
+            assert ops.skinny_rings(m, 8 * block, 1088, epilogue)
+        assert ops.skinny_rings(m, 8 * block, 576, ops.EPI_ACCUM_F32) and ops.skinny_rings(m, 8 * block, 576, ops.EPI_SWIGLU, True)
+        assert not ops.skinny_rings(m, 8 * block, 512, ops.EPI_ACCUM_F32) and not ops.skinny_rings(m, 8 * block, 512, ops.EPI_SWIGLU, True)
+    assert ops.skinny_rings(17, 2 * block + 16, 512)
+
+
 @pytest.mark.parametrize("k", [6, (1 << 24) + 4])
 def test_float32_products_leave_what_their_kernels_refuse_to_the_plain_one(k):
     row = torch.empty(1, k)
