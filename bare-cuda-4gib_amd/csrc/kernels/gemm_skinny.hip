@@ -1129,10 +1129,18 @@ bool ring_operands(const SkinnyArgs& a) {
 //   Four blocks a CU behind a norm also at 1,024: 8 rows 8.2 and 8.8.  9 to 16 rows, from two blocks a CU on: k up to 512 (128,256 x 512 26.1 and 37.8, 12,288 x 512
 //   behind a norm 5.1 and 6.3; but 8,192 x 512 4.7 and 4.4), up to 1,024 what neither adds nor rotates nor finishes a norm before gates (32,000 x 768 stored 11.7 and
 //   13.6, rotated 17.7 and 16.1, gated behind a norm 15.5 and 15.1; 32,000 x 1,152 16.0 and 16.3).
+// - small weights of a k that gives a wave two stages: one trip and a second through LDS.  k from 576 to 1,024 and up to 640 numbers of k times blocks a CU, up to 32
+//   rows (9 to 16 where the rows are shared out), what neither adds nor rotates (one row 768 x 768 2.44 and 2.67, 2,304 x 768 2.98 and 3.13, behind a norm
+//   3.31 and 3.53, 24 rows 4.17 and 4.62; but rotated 4.78 and 4.34, added 3.65 and 3.56; 3,072 x 1,024 3.50 and 3.30, 4,096 x 768 3.45 and 3.28).
+// - a norm to finish for more than 16 rows of k up to 512: more parts of sums of squares than operands (24 rows 4,096 x 256 3.35 and 3.70, 48 rows 512 x 512 3.45 and
+//   3.65; rotated 4.52 and 4.48).
 bool rings_are_slower(int epilogue, int m, int n, int k, bool finishes_norm) {
   const int blocks = (n + 15) / 16, cus = compute_units();
   if (m > 32 && 2 * blocks > 3 * cus) return true;
   const bool adds = epilogue == kAccumF32, rotates = epilogue == kRopeKvBf16, gates_normed = gated(epilogue) && finishes_norm;
+  const bool plain = !adds && !rotates, shared_out = m <= kSplitMinRows || m > 16 || 2 * blocks <= cus;
+  if (plain && m <= 32 && shared_out && k > 512 && k <= 1024 && static_cast<long>(blocks) * k <= 640L * cus) return true;
+  if (finishes_norm && !rotates && m > 16 && k <= 512) return true;
   if (m > kSplitMinRows && m <= 16 && blocks > 2 * cus) return k <= 512 || (k <= 1024 && !adds && !rotates && !gates_normed);
   if (m <= kSplitMinRows && blocks > 3 * cus) {
     if (k <= 512) return !gates_normed;

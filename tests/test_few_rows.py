@@ -58,6 +58,19 @@ def test_rings_leave_wide_outputs_of_a_short_k_to_the_streaming_kernel():
     assert ops.skinny_rings(17, 2 * block + 16, 512)
 
 
+def test_rings_leave_small_weights_of_two_stages_a_wave_to_the_streaming_kernel():
+    cus = ops.compute_units()
+    for k in (576, 768, 1024):
+        n = 16 * (640 * cus // k)
+        for m in (1, 8, 17, 32):
+            assert not ops.skinny_rings(m, n, k) and ops.skinny_rings(m, n + 1, k) and ops.skinny_rings(m, n, k, ops.EPI_ACCUM_F32)
+        assert ops.skinny_rings(33, n, k) and ops.skinny_rings(9, n, k) and not ops.skinny_rings(9, 8 * cus, k)
+    assert ops.skinny_rings(1, 768, 512) and ops.skinny_rings(1, 768, 1088)
+    for m in (17, 32, 64):
+        assert not ops.skinny_rings(m, 2048, 512, ops.EPI_STORE_F32, True) and ops.skinny_rings(m, 2048, 512, ops.EPI_STORE_F32)
+    assert ops.skinny_rings(16, 2048, 512, ops.EPI_STORE_F32, True)
+
+
 @pytest.mark.parametrize("k", [6, (1 << 24) + 4])
 def test_float32_products_leave_what_their_kernels_refuse_to_the_plain_one(k):
     row = torch.empty(1, k)
