@@ -35,7 +35,15 @@ int compute_units() {
   return cus[dev];
 }
 
+static thread_local bool g_weights_stay = false;
+bool weights_stay() { return g_weights_stay; }
+
 }  // namespace bc4g
+
+extern "C" int bc4g_weights_stay(int stay) {
+  bc4g::g_weights_stay = stay != 0;
+  return 0;
+}
 
 #ifndef BC4G_SOURCES_DIGEST
 #define BC4G_SOURCES_DIGEST "unknown"

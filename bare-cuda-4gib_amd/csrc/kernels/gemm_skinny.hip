@@ -1376,6 +1376,12 @@ extern "C" int bc4g_gemm_skinny_rings(int m, int n, int k, int epilogue, int fin
   return 0;
 }
 
+extern "C" int bc4g_weight_passes(int n, int k, int bytes_a_number, int* passes) {
+  BC4G_REQUIRE(n > 0 && k > 0 && bytes_a_number > 0 && passes != nullptr, "weight_passes: sizes and a place for the answer");
+  *passes = passes_by(n, k, bytes_a_number) ? 1 : 0;
+  return 0;
+}
+
 extern "C" int bc4g_gemm_skinny_normed(const float* x, const int32_t* rows, const void* g, int g_dtype,
                                        float eps, const void* w, void* out, int epilogue, int m, int n, int k,
                                        void* stream) {

@@ -8,6 +8,7 @@ library, or on a CPU tensor, they raise.
 from __future__ import annotations
 
 import array
+import contextlib
 import ctypes
 import dataclasses
 import functools
@@ -94,6 +95,24 @@ def tiled_cut(m: int, n: int, k: int, qkv: bool = False) -> Tuple[int, Optional[
     library.call("bc4g_gemm_mfma_cut", None, None, m, n, k, int(qkv), ctypes.byref(first), ctypes.byref(rows), ctypes.byref(cols), ctypes.byref(beyond),
                  launches=False)
     return first.value, (rows.value, cols.value) if first.value < n else None, bool(beyond.value)
+
+
+@contextlib.contextmanager
+def weights_stay():
+    """Around the launches of a step whose weights, all together, stay in the caches from step to step: none of them is then loaded past the caches,
+    however large it is.  For this thread's launches and no longer than the block; what is computed is the same."""
+    library.call("bc4g_weights_stay", 1, launches=False)
+    try:
+        yield
+    finally:
+        library.call("bc4g_weights_stay", 0, launches=False)
+
+
+def weight_passes(n: int, k: int, bytes_a_number: int = 2) -> bool:
+    """Whether a weight of n x k numbers that few rows are multiplied by is loaded past the caches."""
+    passes = ctypes.c_int(0)
+    library.call("bc4g_weight_passes", n, k, bytes_a_number, ctypes.byref(passes), launches=False)
+    return bool(passes.value)
 
 
 def skinny_rings(m: int, n: int, k: int, epilogue: int = 0, finishes_norm: bool = False) -> bool:

@@ -32,6 +32,14 @@ class _Bound:
                 for local, ws in self.part.weight_specs().items()}
 
 
+# Weights that a step reads, all together, up to which they stay in the card's 256 MB of cache from one decode step to the next, beside keys, values and
+# activations, and are not loaded past the caches.  us a captured step, large weights (6 MB and more) past the caches and through them: two layers of 2,048 and a
+# head of 8,000, 209 MB, 1, 8 and 32 rows 74.2, 85.1, 95.1 and 73.8, 81.4, 88.4; three layers of 1,536 and a head of 16,000, 200 MB, 100.3, 102.5, 121.6 and 98.4, 99.2,
+# 112.1; six 32-bit layers of 768, 195 MB, 8 rows 182.4 and 178.0.  Beyond the line: 12 layers of 768 and a head of 32,000, 219 MB, 1, 8 and 32 rows 252.8, 258.0,
+# 345.6 and 253.1, 254.1, 355.8; three layers of 2,048, 297 MB, 102.9, 117.0, 130.6 and 107.0, 117.4, 139.0.
+WEIGHTS_STAY_BYTES = 208 << 20
+
+
 class Model:
     def __init__(self, spec: ModelSpec):
         self.spec = spec
@@ -70,6 +78,7 @@ class Model:
         self.max_seq_len = spec.max_seq_len
         self.streams = int(getattr(spec, "streams", 1))
         self.rt: Optional[Runtime] = None
+        self.weights_stay = False         # whether the weights of a step stay in the caches from one to the next
 
     def all_parts(self) -> List[Part]:
         """Every part of the model, nested ones included: embedding, each layer's block with its norms,
@@ -100,12 +109,15 @@ class Model:
         """Place the loaded tensors on the device and hand each part its own."""
         self.rt = rt
         placed: Dict[str, torch.Tensor] = {}
+        read = set()                      # the tensors that a step reads whole: all but the table its rows are looked up in
         cuda = rt.device.type == "cuda"
         before = torch.cuda.memory_allocated(rt.device) if cuda else 0
 
         def get(name: str) -> Optional[torch.Tensor]:
             if name not in placed and name in tensors:
                 placed[name] = rt.place_weight(tensors[name])
+            if name in placed and b is not self.embedding:
+                read.add(name)
             return placed.get(name)
 
         for b in self._all_bound():
@@ -122,6 +134,7 @@ class Model:
         # the tensors as loaded, and what they take on the device once the parts have packed them and what
         # nobody holds any more has gone (a linear map's weight is kept once, in the order its kernels read)
         self.weight_bytes = sum(t.numel() * t.element_size() for t in placed.values())
+        self.weights_stay = sum(placed[n].numel() * placed[n].element_size() for n in read) <= WEIGHTS_STAY_BYTES
         placed.clear()
         tensors = mine = None
         self.device_weight_bytes = torch.cuda.memory_allocated(rt.device) - before if cuda else self.weight_bytes
@@ -199,6 +212,13 @@ class Model:
     def forward(self, ctx: StepContext) -> Optional[torch.Tensor]:
         """Run the batch through every schedule entry; float32 logits at the
         wanted rows ([n_logits, vocab]), or None if none are wanted."""
+        if not self.weights_stay or self.rt.device.type != "cuda":
+            return self._forward(ctx)
+        from ..csrc import ops
+        with ops.weights_stay():
+            return self._forward(ctx)
+
+    def _forward(self, ctx: StepContext) -> Optional[torch.Tensor]:
         x = self.embedding.part.forward(ctx)
         if self.streams > 1:            # the stream in copies, [T, streams, H]: every copy starts as the embedding
             from ..csrc import ops
