@@ -221,6 +221,17 @@ class CacheManager:
         self._leaves[sid] = view
         return view
 
+    def bytes_read(self, length: int) -> int:
+        """Device bytes of the pages' tensors that the next token of a request of ``length`` tokens reads, over all streams that keep something per token."""
+        total = 0
+        for view in self._leaves.values():
+            if view.paged:
+                group = self.groups[view.group]
+                passed = min(max(0, int(group.first_kept(length))), length)
+                tokens = length - passed + min(group.always_kept, passed)
+                total += tokens * sum(t[0].numel() * t.element_size() for t in view.tensors.values()) // self.page_tokens
+        return total
+
     # ---- requests ---------------------------------------------------------
     def has(self, request: Hashable) -> bool:
         return request in self._requests

@@ -115,13 +115,8 @@ __device__ inline void store_through(float* p, float v) { __hip_atomic_store(p, 
 __device__ inline float load_through(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ inline void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// DJ: k-steps of 32 over head_dim for the scores; DB: blocks of 16 output dimensions; QT: 16-row
-// query tiles per wave (consecutive tokens), which share every key and value fragment the wave
-// loads -- prompt portions use 4 (or 2 for large heads), decoded tokens 1.
-// WS: 1, or the number of waves that share one tile's keys.
 constexpr int kMergePad = 4;   // floats between rows of the partial outputs in LDS
 
-// EXACT: the head size is exactly 16 * DB (the usual sizes 64, 128, 256): no test against it is left.
 // 16 or 8 bytes, past the caches (PAST) or through them.
 template <bool PAST, typename T>
 __device__ inline T load_once(const void* p) {
@@ -133,7 +128,12 @@ __device__ inline T load_once(const void* p) {
   return __builtin_bit_cast(T, v);
 }
 
-// PAST: keys and values past the caches, where one workgroup reads them (see launch_attention).
+// DJ: k-steps of 32 over head_dim for the scores; DB: blocks of 16 output dimensions; QT: 16-row
+// query tiles per wave (consecutive tokens), which share every key and value fragment the wave
+// loads -- prompt portions use 4 (or 2 for large heads), decoded tokens 1.
+// WS: 1, or the number of waves that share one tile's keys.
+// EXACT: the head size is exactly 16 * DB (the usual sizes 64, 128, 256): no test against it is left.
+// PAST: keys and values past the caches, where one workgroup reads them (past_caches).
 template <int DJ, int DB, int QT, int WS, bool EXACT, bool PAST>
 __global__ __launch_bounds__((WS > 1 ? WS : kWavesPerBlock) * kWave, 2) void attention_mfma_kernel(
     const AttnArgs a) {
@@ -862,7 +862,7 @@ extern "C" int bc4g_attention_mfma_counted(const void* qkv, int q_stride, void* 
                                    int n_seqs, int n_tiles, int n_tokens, int n_heads, int n_kv_heads, int head_dim,
                                    int page_tokens, int window, float scale, int tokens_per_tile, int q_tiles,
                                    int form, int n_splits, const int32_t* items, int n_items, const int32_t* row_parts,
-                                   int single_rows, const int32_t* row_seq, int32_t* arrived, int n_arrived, void* stream) {
+                                   int single_rows, const int32_t* row_seq, int32_t* arrived, int n_arrived, int past_caches, void* stream) {
   BC4G_REQUIRE(n_heads > 0 && n_kv_heads > 0 && n_heads % n_kv_heads == 0, "attention_mfma: bad heads %d/%d",
                n_heads, n_kv_heads);
   BC4G_REQUIRE(head_dim >= 16 && head_dim <= 256 && head_dim % 16 == 0,
@@ -947,12 +947,10 @@ extern "C" int bc4g_attention_mfma_counted(const void* qkv, int q_stride, void* 
     // one workgroup per tile; its waves (8, or 4 for the largest heads) cut the keys between them
     dim3 grid(n_tiles, n_kv_heads * a.n_sub, n_splits);
     auto lds = [&](int ws) { return static_cast<size_t>(ws) * 16 * (head_dim + kMergePad + 2) * sizeof(float); };
-    // A decode step's requests, one row each and the heads of a KV head in one tile: every key is read once.  Where the block tables have room for 32 MB
-    // and more of keys and values a layer, the layers behind it will have put them out by the next step: past the caches, as large weights go (16
-    // requests of 1,000 tokens, 32 KV heads of 128 52.8 -> 47.8 us a layer, 5.5 TB/s; 8 of 4,000, 8 KV heads 31.4 -> 28.1; but 22 layers of 8 requests of 540
-    // tokens, 4 KV heads of 64, whose 97 MB stay: a step 1.4 % slower).
-    constexpr long kRoom = 32L << 20;
-    const bool past = single_rows && a.n_sub == 1 && static_cast<long>(n_seqs) * table_stride * page_tokens * n_kv_heads * head_dim * 4 >= kRoom;
+    // A decode step's requests, one row each and the heads of a KV head in one tile: every key is read once, and where the caller knows that the step's
+    // keys and values do not stay in the caches until the next one (past_caches), past them, as large weights go (16 requests of 1,000 tokens, 32 KV
+    // heads of 128 52.8 -> 47.8 us a layer, 5.5 TB/s; 8 of 4,000, 8 KV heads 31.4 -> 28.1).
+    const bool past = past_caches && single_rows && a.n_sub == 1;
     if (dj <= 2 && db <= 4)
       status = past ? launch_attention<2, 4, 1, 8, true>(a, grid, 8 * kWave, lds(8), s) : launch_attention<2, 4, 1, 8>(a, grid, 8 * kWave, lds(8), s);
     else if (dj <= 4 && db <= 8)
@@ -1001,5 +999,5 @@ extern "C" int bc4g_attention_mfma(const void* qkv, int q_stride, void* out, flo
                                    int single_rows, const int32_t* row_seq, void* stream) {
   return bc4g_attention_mfma_counted(qkv, q_stride, out, part_o, part_ml, k_cache, v_cache, block_table, table_stride, seq_start, seq_ctx, tile_start,
                                      n_seqs, n_tiles, n_tokens, n_heads, n_kv_heads, head_dim, page_tokens, window, scale, tokens_per_tile, q_tiles,
-                                     form, n_splits, items, n_items, row_parts, single_rows, row_seq, nullptr, 0, stream);
+                                     form, n_splits, items, n_items, row_parts, single_rows, row_seq, nullptr, 0, 0, stream);
 }

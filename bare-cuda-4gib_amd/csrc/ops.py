@@ -1391,7 +1391,7 @@ def attention_mfma(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                    n_splits: int, q_tiles: int = 1, form: int = 0, work=None,
                    out: Optional[torch.Tensor] = None, row_seq: Optional[torch.Tensor] = None,
                    single_rows: bool = False, items: Optional[torch.Tensor] = None, n_items: int = 0,
-                   row_parts: Optional[torch.Tensor] = None, arrived: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   row_parts: Optional[torch.Tensor] = None, arrived: Optional[torch.Tensor] = None, past_caches: bool = False) -> torch.Tensor:
     """form 0: four independent waves a workgroup, tile_start counts pieces of q_tiles tiles; 1: one
     tile a workgroup, its waves share the keys (q_tiles 1); 2: four waves a workgroup that walk their
     keys together through LDS, tile_start counts pieces of 4 * q_tiles tiles (ATTENTION_STAGED_WAVES).
@@ -1403,7 +1403,8 @@ def attention_mfma(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     are to start, each a piece, a part and the number of parts of that piece's keys; ``row_parts`` [T]:
     into how many parts each row's keys are cut; n_splits is then the most parts of any piece.
     ``arrived`` (form 1): zeros, one int32 a tile and group of heads (attention_counters): the part of a tile's keys that ends last adds
-    the parts up, and no merge kernel follows (the same bits)."""
+    the parts up, and no merge kernel follows (the same bits).
+    ``past_caches`` (with single_rows): keys and values are loaded past the caches (StepContext.cache_passes; the same bits)."""
     _dev("attention_mfma", qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start)
     t = qkv.shape[0]
     _check_queries("attention_mfma", qkv, n_heads, n_kv_heads, head_dim)
@@ -1428,12 +1429,13 @@ def attention_mfma(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         _i32("attention_mfma", "items", items, n_items)
         _i32("attention_mfma", "row_parts", row_parts, t)
     _launch_attention_mfma(qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start, n_tiles, n_heads, n_kv_heads, head_dim, window,
-                           scale, n_splits, q_tiles, form, work, out, row_seq, single_rows, items, n_items, row_parts, arrived)
+                           scale, n_splits, q_tiles, form, work, out, row_seq, single_rows, items, n_items, row_parts, arrived, past_caches)
     return out
 
 
 def _launch_attention_mfma(qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start, n_tiles, n_heads, n_kv_heads, head_dim, window, scale,
-                           n_splits, q_tiles, form, work, out, row_seq=None, single_rows=False, items=None, n_items=0, row_parts=None, arrived=None) -> None:
+                           n_splits, q_tiles, form, work, out, row_seq=None, single_rows=False, items=None, n_items=0, row_parts=None, arrived=None,
+                           past_caches=False) -> None:
     """attention_mfma for operands that have been looked at."""
     t, n_seqs = qkv.shape[0], block_table.shape[0]
     parts = part_ml = None
@@ -1449,7 +1451,7 @@ def _launch_attention_mfma(qkv, k_cache, v_cache, block_table, seq_start, seq_ct
                  _ptr(tile_start), n_seqs, n_tiles, t, n_heads, n_kv_heads, head_dim, k_cache.shape[2],
                  int(window), float(scale), attention_tile_tokens(n_heads, n_kv_heads), int(q_tiles),
                  int(form), int(n_splits), _ptr(items), int(n_items), _ptr(row_parts), 1 if single_rows else 0,
-                 _ptr(row_seq), _ptr(arrived), arrived.numel() if arrived is not None else 0, _stream(), cost=work)
+                 _ptr(row_seq), _ptr(arrived), arrived.numel() if arrived is not None else 0, int(past_caches), _stream(), cost=work)
 
 
 _DECODE_TILE_STARTS: dict = {}
@@ -1559,7 +1561,8 @@ def attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
             n_tiles = notes["n_tiles"]
             n_splits = attention_splits(n_tiles, n_heads, n_kv_heads, ctx.max_kv_len, attention_shared_waves(head_dim))
             return attention_mfma(*args, arrays["tiles"], n_tiles, *sizes, n_splits, 1, 1, work=work,
-                                  single_rows=ctx.max_q_len == 1 and ctx.n_tokens == ctx.n_seqs, arrived=arrays.get("arrived"))
+                                  single_rows=ctx.max_q_len == 1 and ctx.n_tokens == ctx.n_seqs, arrived=arrays.get("arrived"),
+                                  past_caches=ctx.cache_passes)
         q_tiles = attention_q_tiles(head_dim)
         apart = notes["apart"]
         if "items" in arrays:       # the pieces' parts in the order the host chose, longest walks first

@@ -56,6 +56,15 @@ class StepEntry:
     want: Sequence[int] = ()
 
 
+# Keys and values of a decode step, as far as its requests may reach, beside the weights that go through the caches, from which on they are loaded past the
+# card's 256 MB of cache: two fifths more, as a captured step plans for the end of a context bucket and its contexts are three quarters of that on average.  us a
+# step, through the caches and past them, by bytes at the bound: TinyLlama's 22 layers, 8 requests, at 500 tokens (185 MB) 779.6 and 801.4, at 1,500 (369 MB) 822.9
+# and 829.0, 16 at 2,000 (738 MB) 1,049.7 and 1,045.2; eight layers of Llama-3-8B's, 8 requests at 250 (67 MB) 846.4 and 858.5, 16 at 500 (268 MB) 1,033.9 and 1,041.8,
+# 8 at 2,000 (537 MB) 950.2 and 934.2; 12 layers of 768, 94 MB of weights through the caches, 8 at 250 (75 and 94 MB) 268.6 and 277.7, 16 at 500 (302 and 94) 367.8 and
+# 351.4.
+CACHE_HOLDS_BYTES = 360 << 20
+
+
 class Executor:
     """Owns a model's cache and runs steps on it.
 
@@ -133,6 +142,10 @@ class Executor:
 
     def length(self, request: Hashable) -> int:
         return self.cache.length(request)
+
+    def cache_passes(self, n_requests: int, max_kv: int) -> bool:
+        """Whether a decode step of so many requests of up to max_kv tokens reads its keys and values past the caches."""
+        return n_requests * self.cache.bytes_read(max_kv) + self.model.cached_weight_bytes >= CACHE_HOLDS_BYTES
 
     # ---- the step -----------------------------------------------------------
     def _validate(self, entries: Sequence[StepEntry]) -> int:
@@ -254,7 +267,8 @@ class Executor:
             seq_slots=host["seq_slots"], seq_start_dev=parts["seq_start"], seq_ctx_dev=parts["seq_ctx"],
             seq_slots_dev=parts["seq_slots"], logit_rows=parts["logit_rows"], n_logits=host["n_logits"],
             block_tables=block_tables, slot_maps=slot_maps, max_q_len=host["max_q"], max_kv_len=host["max_kv"],
-            cache_views=self._views, step_data=step_data, captured=host["captured"])
+            cache_views=self._views, step_data=step_data, captured=host["captured"],
+            cache_passes=host["max_q"] == 1 and self.cache_passes(S, host["max_kv"]))
 
     def build_context(self, entries: Sequence[StepEntry]) -> StepContext:
         """Host arrays of the batch, uploaded in one copy."""

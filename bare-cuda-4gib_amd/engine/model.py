@@ -79,6 +79,7 @@ class Model:
         self.streams = int(getattr(spec, "streams", 1))
         self.rt: Optional[Runtime] = None
         self.weights_stay = False         # whether the weights of a step stay in the caches from one to the next
+        self.cached_weight_bytes = 0      # of those weights, what a step of few rows loads through the caches
 
     def all_parts(self) -> List[Part]:
         """Every part of the model, nested ones included: embedding, each layer's block with its norms,
@@ -134,10 +135,18 @@ class Model:
         # the tensors as loaded, and what they take on the device once the parts have packed them and what
         # nobody holds any more has gone (a linear map's weight is kept once, in the order its kernels read)
         self.weight_bytes = sum(t.numel() * t.element_size() for t in placed.values())
-        self.weights_stay = sum(placed[n].numel() * placed[n].element_size() for n in read) <= WEIGHTS_STAY_BYTES
+        read_bytes = sum(placed[n].numel() * placed[n].element_size() for n in read)
+        self.weights_stay = read_bytes <= WEIGHTS_STAY_BYTES
         placed.clear()
         tensors = mine = None
         self.device_weight_bytes = torch.cuda.memory_allocated(rt.device) - before if cuda else self.weight_bytes
+        self.cached_weight_bytes = read_bytes
+        if cuda and not self.weights_stay:
+            from ..csrc import ops
+            maps = {id(w): w for part in self.all_parts() for w in vars(part).values() if isinstance(w, ops.StreamedWeight)}
+            for w in maps.values():
+                if w.dim() == 2 and ops.weight_passes(*w.shape, w.element_size()):
+                    self.cached_weight_bytes -= w.shape[0] * w.shape[1] * w.element_size()
 
     # ---- cache --------------------------------------------------------------
     def _cache_spec(self, layer: int):

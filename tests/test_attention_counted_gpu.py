@@ -75,9 +75,10 @@ def test_counters_go_up_with_the_batch(ops):
 
 
 @pytest.mark.parametrize("n_splits", [1, 3])
+@pytest.mark.parametrize("counted", [False, True])
 @pytest.mark.parametrize("S, heads, kv_heads, d", [(16, 32, 8, 64), (8, 32, 8, 128), (4, 8, 8, 256), (5, 16, 16, 80)])
-def test_room_for_much_as_for_little(ops, S, heads, kv_heads, d, n_splits):
-    """Block tables with room for 32 MB of keys and values and more, which are then read past the caches, against tables as wide as the contexts."""
+def test_past_the_caches_as_through_them(ops, S, heads, kv_heads, d, n_splits, counted):
+    """Keys and values read past the caches, and tables with room for much more than the contexts, with the last part merging and with a kernel behind it."""
     gen = torch.Generator().manual_seed(S + d)
     page, width = 64, 4
     draw = lambda *shape: torch.randn(*shape, generator=gen).bfloat16().to(DEV)      # noqa: E731
@@ -88,5 +89,9 @@ def test_room_for_much_as_for_little(ops, S, heads, kv_heads, d, n_splits):
     room = -(-(32 << 20) // (S * page * kv_heads * d * 4))
     wide = torch.full((S, room), -1, dtype=torch.int32, device=DEV)
     wide[:, :width] = table
-    one, two = (ops.attention_mfma(q, kc, vc, t, rows, ctx, rows, S, heads, kv_heads, d, 0, d ** -0.5, n_splits, 1, 1, single_rows=True) for t in (table, wide))
-    assert room > width and torch.equal(one, two)
+    arrived = torch.zeros(S * kv_heads, dtype=torch.int32, device=DEV) if counted else None
+    run = lambda t, past: ops.attention_mfma(q, kc, vc, t, rows, ctx, rows, S, heads, kv_heads, d, 0, d ** -0.5, n_splits, 1, 1, single_rows=True,      # noqa: E731
+                                             arrived=arrived, past_caches=past)
+    want = run(table, False)
+    assert room > width and all(torch.equal(run(t, past), want) for t in (table, wide) for past in (False, True))
+    assert arrived is None or not arrived.any()
