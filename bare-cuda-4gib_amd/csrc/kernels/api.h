@@ -202,7 +202,7 @@ int bc4g_attention_mfma(const void* qkv, int q_stride, void* out, float* part_o,
                         int page_tokens, int window, float scale, int tokens_per_tile, int q_tiles,
                         int form, int n_splits, const int32_t* items, int n_items, const int32_t* row_parts,
                         int single_rows, const int32_t* row_seq, void* stream);
-// The same; with arrived (form 1; n_arrived int32, all zero, one a tile and group of heads at least: n_tiles * n_kv_heads * ceil(group / 16)) the part of
+// The same; with arrived (form 1, where the parts are few and a tile's outputs no more than its threads: else they are not looked at; n_arrived int32, all zero, one a tile and group of heads at least: n_tiles * n_kv_heads * ceil(group / 16)) the part of
 // a tile's keys that ends last adds the parts up, and no kernel follows.  They are zero again when the launch has ended: launches one after the
 // other may share them, launches beside each other may not.  past_caches: single rows' keys and values are loaded past the caches (the same bits).
 int bc4g_attention_mfma_counted(const void* qkv, int q_stride, void* out, float* part_o, float* part_ml, const void* k_cache,

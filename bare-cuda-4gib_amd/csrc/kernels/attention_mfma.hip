@@ -115,6 +115,7 @@ __device__ inline void store_through(float* p, float v) { __hip_atomic_store(p, 
 __device__ inline float load_through(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ inline void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+constexpr int kMergeParts = 8;  // parts that the one that ends last adds up
 constexpr int kMergePad = 4;   // floats between rows of the partial outputs in LDS
 
 // 16 or 8 bytes, past the caches (PAST) or through them.
@@ -638,10 +639,8 @@ __global__ __launch_bounds__((WS > 1 ? WS : kWavesPerBlock) * kWave, 2) void att
     if (a.n_splits == 1 || a.arrived == nullptr) return;
 
     // The part of this tile that ends last adds the parts up, in order of z and by the merge kernels' own steps: the same bits whichever
-    // it is.  (The counter goes back to zero by itself, for the next layer.)  What it
-    // costs is three trips past the L2s, 2 to 2.5 us; the merge kernel's launch and trip were 3 to 3.5.  us, caches from memory, merge kernel and
-    // this: 8 requests of 540 tokens in three parts 8.6 and 7.8, 16 of them 8.9 and 8.3, one of 1,000 in four 7.3 and 7.1, one of 1,900 in
-    // eight 8.3 and 7.3, 8 of 1,900 in eight 10.4 and 9.6.
+    // it is.  (The counter goes back to zero by itself, for the next layer.)  What it costs is three trips past the L2s, 2 to 2.5 us, where one trip asks for
+    // all that a thread adds up; the merge kernel's launch and trip are 3 to 3.5 (see merges_itself).
     int* is_last = reinterpret_cast<int*>(merge_raw);          // (everybody has read what lay there)
     wait_stores();
     __syncthreads();
@@ -657,30 +656,22 @@ __global__ __launch_bounds__((WS > 1 ? WS : kWavesPerBlock) * kWave, 2) void att
       const int r_tok = r / a.hg, r_head_in_group = hsub * a.hg + r % a.hg;
       if (r_tok >= a.tpt || r_tok >= ntok || r_head_in_group >= group) continue;
       const long rh = (row0 + tok0 + r_tok) * a.n_heads + kvh * group + r_head_in_group;
-      constexpr int kAhead = 8;                 // parts asked for together
-      float mz[kAhead], lz[kAhead], oz[kAhead];
-      auto ask = [&](int z0) {
+      float mz[kMergeParts], lz[kMergeParts], oz[kMergeParts];
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-          const long slot = static_cast<long>(min(z0 + i, a.n_splits - 1)) * rows_heads + rh;
-          mz[i] = load_through(a.part_ml + slot * 2);
-          lz[i] = load_through(a.part_ml + slot * 2 + 1);
-          oz[i] = load_through(a.part_o + slot * d + c);
-        }
-      };
-      ask(0);
+      for (int i = 0; i < kMergeParts; ++i) {
+        const long slot = static_cast<long>(min(i, a.n_splits - 1)) * rows_heads + rh;
+        mz[i] = load_through(a.part_ml + slot * 2);
+        lz[i] = load_through(a.part_ml + slot * 2 + 1);
+        oz[i] = load_through(a.part_o + slot * d + c);
+      }
       float m = -INFINITY, l = 0.f, acc = 0.f;
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) m = fmaxf(m, mz[i]);
-      for (int z = kAhead; z < a.n_splits; ++z) m = fmaxf(m, load_through(a.part_ml + (z * rows_heads + rh) * 2));
-      for (int z0 = 0; z0 < a.n_splits; z0 += kAhead) {
-        if (z0 > 0) ask(z0);
+      for (int i = 0; i < kMergeParts; ++i) m = fmaxf(m, mz[i]);
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-          const float wz = z0 + i >= a.n_splits || mz[i] == -INFINITY ? 0.f : exp2f(mz[i] - m);
-          l += wz * lz[i];
-          acc += wz * oz[i];
-        }
+      for (int i = 0; i < kMergeParts; ++i) {
+        const float wz = i >= a.n_splits || mz[i] == -INFINITY ? 0.f : exp2f(mz[i] - m);
+        l += wz * lz[i];
+        acc += wz * oz[i];
       }
       a.out[rh * d + c] = from_float<bf16_t>(acc * (1.0f / l));
     }
@@ -832,6 +823,12 @@ using namespace bc4g;
 
 namespace bc4g {
 namespace {
+// Whether the part that ends last merges, given counters, and not a kernel behind: up to as many parts as it asks for together, and where a token's outputs
+// in a tile are no more than the workgroup's threads.  us, caches from memory, kernel and last part: 8 requests of 520 tokens, 8 heads of 64 a tile, three parts 8.4 and
+// 8.0, of 2,000 in eight 10.4 and 9.9; one of 520 with every head's own keys, 128, 10.2 and 9.1; but one of 4,000 in sixteen parts, 8 heads of 64, 9.4 and 10.6, of 128
+// 13.2 and 16.1; 8 heads of 128 a tile, one of 520 8.3 and 9.0; 4 of 256 (256 threads) 10.7 and 13.2, of 4,000 in 32 parts 20.4 and 36.7.
+bool merges_itself(int n_splits, int outputs, int threads) { return n_splits <= kMergeParts && outputs <= threads; }
+
 template <int DJ, int DB, int QT, int WS, bool PAST = false>
 int launch_attention(const AttnArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
   // per instantiation, once: the staged form's ring may need more than the default dynamic LDS
@@ -908,7 +905,8 @@ extern "C" int bc4g_attention_mfma_counted(const void* qkv, int q_stride, void* 
   a.items = items;
   a.row_parts = items ? row_parts : nullptr;
   a.single_rows = single_rows ? 1 : 0;
-  a.arrived = form == 1 && n_splits > 1 ? reinterpret_cast<uint32_t*>(arrived) : nullptr;
+  const int shared_waves = head_dim <= 128 ? 8 : 4;         // of the decode form's workgroups
+  a.arrived = form == 1 && n_splits > 1 && merges_itself(n_splits, a.hg * head_dim, shared_waves * kWave) ? reinterpret_cast<uint32_t*>(arrived) : nullptr;
   BC4G_REQUIRE(a.arrived == nullptr || static_cast<long>(n_tiles) * n_kv_heads * a.n_sub <= n_arrived,
                "attention_mfma: %d counters are fewer than %d tiles times %d groups of heads", n_arrived, n_tiles, n_kv_heads * a.n_sub);
   BC4G_REQUIRE(!single_rows || (form == 1 && n_tiles == n_seqs && n_tokens == n_seqs),

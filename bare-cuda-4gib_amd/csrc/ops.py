@@ -1377,8 +1377,9 @@ def attention_splits(n_tiles: int, n_heads: int, n_kv_heads: int, max_kv_len: in
         walk = -(-key_tiles // shared_waves)
         parts = max(1, min(-(-walk // ATTENTION_SHARED_WALK), ATTENTION_ENOUGH_GROUPS // max(waves, 1),
                            ATTENTION_MAX_SPLITS))
-        # a cut that shortens a wave's walk by less than ATTENTION_WORTH_A_CUT tiles does not pay for the merge kernel
-        # (32 requests at 548 tokens of context, two parts: a wave walks 2 tiles instead of 3, a step 1.209 against 1.165 ms)
+        # a cut that shortens a wave's walk by less than ATTENTION_WORTH_A_CUT tiles does not pay for the adding up, whoever does it (TinyLlama's 22
+        # layers, us a step with cuts from two tiles on and from one: 8 requests at 300 tokens 774 and 797, one at 500 722 and 734, 4 at 400 819 and 836)
+        # (with a merge kernel behind it, 32 requests at 548 tokens in two parts: a wave walks 2 tiles instead of 3, a step 1.209 against 1.165 ms)
         return parts if walk - -(-walk // parts) >= ATTENTION_WORTH_A_CUT else 1
     groups = max(1, -(-waves // ATTENTION_STAGED_WAVES))
     return max(1, min(-(-ATTENTION_PROMPT_GROUPS // groups), ATTENTION_MAX_PROMPT_SPLITS,
@@ -1403,7 +1404,7 @@ def attention_mfma(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     are to start, each a piece, a part and the number of parts of that piece's keys; ``row_parts`` [T]:
     into how many parts each row's keys are cut; n_splits is then the most parts of any piece.
     ``arrived`` (form 1): zeros, one int32 a tile and group of heads (attention_counters): the part of a tile's keys that ends last adds
-    the parts up, and no merge kernel follows (the same bits).
+    the parts up, and no merge kernel follows where that is the faster way (attention_mfma.hip, merges_itself; the same bits).
     ``past_caches`` (with single_rows): keys and values are loaded past the caches (StepContext.cache_passes; the same bits)."""
     _dev("attention_mfma", qkv, k_cache, v_cache, block_table, seq_start, seq_ctx, tile_start)
     t = qkv.shape[0]

@@ -59,6 +59,20 @@ def test_the_last_part_merges(ops, S, heads, kv_heads, d, rows, longest, n_split
             assert all(torch.equal(one, want) for one in got) and not arrived.any()
 
 
+# more parts than are asked for together; more outputs a tile than threads: 8 heads of 128, 4 of 256
+@pytest.mark.parametrize("heads, kv_heads, d, n_splits, used", [(8, 8, 64, 8, True), (8, 8, 64, 9, False), (8, 1, 64, 8, True), (4, 1, 128, 8, True), (8, 1, 128, 2, False),
+                                                                (1, 1, 256, 8, True), (2, 1, 256, 2, False)])
+def test_counters_are_left_alone_where_a_kernel_merges(ops, heads, kv_heads, d, n_splits, used):
+    gen = torch.Generator().manual_seed(d + n_splits)
+    draw = lambda *shape: torch.randn(*shape, generator=gen).bfloat16().to(DEV)      # noqa: E731
+    kc, vc, q = draw(8, kv_heads, 64, d), draw(8, kv_heads, d, 64), draw(1, heads * d)
+    table, rows = torch.arange(8, dtype=torch.int32, device=DEV).view(1, 8), torch.arange(2, dtype=torch.int32, device=DEV)
+    arrived = torch.full((kv_heads,), 0 if used else 77, dtype=torch.int32, device=DEV)
+    run = lambda counters: ops.attention_mfma(q, kc, vc, table, rows, rows[1:] * 500, rows, 1, heads, kv_heads, d, 0, d ** -0.5, n_splits, 1, 1,      # noqa: E731
+                                              single_rows=True, arrived=counters)
+    assert torch.equal(run(arrived), run(None)) and (arrived == (0 if used else 77)).all()
+
+
 def test_too_few_counters_are_refused(ops):
     from bare_cuda_4gib_amd.errors import KernelError
     z = lambda *shape: torch.zeros(*shape, dtype=torch.int32, device=DEV)      # noqa: E731
