@@ -1158,9 +1158,9 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
   dim3 grid((a.n + 15) / 16), block(kThreads);
   if constexpr (XMODE != kPlain) {
     if (mt != 1) return fail("gemm_skinny: the fused norm takes at most 16 rows, got %d", a.m);
-    if (normed_ring_operands(a)) return launch_normed_rings<EPI>(a, s);
     const size_t stage = static_cast<size_t>(a.m_stage) * (a.k + kStagePad) * 2;
     if (stage > kMaxStageBytes) return fail("gemm_skinny: %d rows of k=%d do not fit the staging buffer", a.m, a.k);
+    if (normed_ring_operands(a)) return launch_normed_rings<EPI>(a, s);
     auto kernel = gemm_skinny_kernel<1, EPI, XMODE, 4>;
     static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
     if (!raised) {

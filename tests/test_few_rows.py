@@ -71,6 +71,14 @@ def test_rings_leave_small_weights_of_two_stages_a_wave_to_the_streaming_kernel(
     assert ops.skinny_rings(16, 2048, 512, ops.EPI_STORE_F32, True)
 
 
+@pytest.mark.parametrize("rows, k", [(1, 12288), (4, 12352), (5, 6144), (16, 3072)])
+def test_rows_too_long_for_the_fused_norm(rows, k):
+    """Rounded up to four they do not fit the staging buffer: refused whichever kernel would take them (one row of 12,288 fits beside the rings)."""
+    with pytest.raises(KernelError, match="do not fit the staging buffer"):
+        at = -(-AT // 16) * 16
+        library.call("bc4g_gemm_skinny_normed", at, None, at, 1, 1e-5, at, at, 1, rows, 64, k, None)
+
+
 @pytest.mark.parametrize("k", [6, (1 << 24) + 4])
 def test_float32_products_leave_what_their_kernels_refuse_to_the_plain_one(k):
     row = torch.empty(1, k)
