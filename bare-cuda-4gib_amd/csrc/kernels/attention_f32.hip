@@ -414,7 +414,7 @@ int launch_attention(const AttnF32Args& a, int n_seqs, bool many, bool few, hipS
   constexpr int kLds = (KT * (DB * 16 + 4) + DB * 16 * (KT + 4)) * 4, kFewLds = kFewWaves * DB * 16 * 17 * 4;
   auto kernel = attention_f32_kernel<DB, KT>;
   auto few_kernel = attention_f32_few_kernel<DB, FEW_KT, AHEAD>;
-  static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
+  static std::atomic<bool> raised{false};   // per instantiation: allow more than the default dynamic LDS
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess ||
         hipFuncSetAttribute(reinterpret_cast<const void*>(few_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds) != hipSuccess)

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 namespace bc4g {
 
 constexpr int kWave = 64;  // CDNA wavefront width

@@ -24,7 +24,7 @@ int check_launch(const char* what) {
 }
 
 int compute_units() {
-  static int cus[64] = {0};
+  static std::atomic<int> cus[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
   if (cus[dev] == 0) {

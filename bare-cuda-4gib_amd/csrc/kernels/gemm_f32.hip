@@ -416,7 +416,7 @@ int launch_stream_kernel(const Args& a, hipStream_t s) {
   auto kernel = gemm_f32_stream_kernel<XR, STAGES, EPI, NORM, HALF, PAST>;
   constexpr int kLds = kWaves * STAGES * ((HALF ? 1 : 2) + XR / 8) * 1024;
   static_assert(kLds <= 160 * 1024, "a workgroup's LDS");
-  static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
+  static std::atomic<bool> raised{false};   // per instantiation: allow more than the default dynamic LDS
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
       return fail("gemm_f32: cannot raise the dynamic LDS limit");
@@ -581,7 +581,7 @@ int launch_tiled_form(const Args& a, hipStream_t s) {
   auto kernel = gemm_f32_tiled_kernel<WM, WN, TM, TN, STAGES, MINWG, EPI>;
   constexpr int RA = 32 * TM * WM, RW = 32 * TN * WN, kLds = STAGES * (RA + RW) * kStepBytes;
   static_assert(kLds * MINWG <= 160 * 1024, "the workgroups' LDS");
-  static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
+  static std::atomic<bool> raised{false};   // per instantiation: allow more than the default dynamic LDS
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
       return fail("gemm_f32: cannot raise the dynamic LDS limit");

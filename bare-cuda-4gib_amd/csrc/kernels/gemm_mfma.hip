@@ -1229,7 +1229,7 @@ struct Operands {
 
 // Launches kernel on tiles of rows x cols, with more than the default dynamic LDS allowed (asked for once: `raised` is the caller's).
 template <typename Kernel>
-int launch_tiles(Kernel kernel, bool& raised, int rows, int cols, int threads, int lds, const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale,
+int launch_tiles(Kernel kernel, std::atomic<bool>& raised, int rows, int cols, int threads, int lds, const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale,
                  int k_parts = 1) {
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
@@ -1244,7 +1244,7 @@ int launch_tiles(Kernel kernel, bool& raised, int rows, int cols, int threads, i
 
 template <int EPI>
 int launch_ahead(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale, int k_parts = 1) {
-  static bool raised = false, raised_past = false;
+  static std::atomic<bool> raised{false}, raised_past{false};
   if (o.m <= 64 && passes_by(o.n, o.k, 2))
     return launch_tiles(gemm_mfma_ahead_kernel<EPI, true>, raised_past, 64, 64, AheadShape::kThreads, AheadShape::kLdsBytes, o, ra, scale, k_parts);
   return launch_tiles(gemm_mfma_ahead_kernel<EPI, false>, raised, 64, 64, AheadShape::kThreads, AheadShape::kLdsBytes, o, ra, scale, k_parts);
@@ -1253,7 +1253,7 @@ int launch_ahead(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& sc
 template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES, int MINWG>
 int launch_direct(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
   typedef DirectShape<WM, WN, TM, TN, BK, STAGES> S;
-  static bool raised = false;
+  static std::atomic<bool> raised{false};
   return launch_tiles(gemm_mfma_direct_kernel<EPI, WM, WN, TM, TN, BK, STAGES, MINWG>, raised, S::kRowsA, S::kRowsW, S::kThreads, S::kLdsBytes, o, ra,
                       scale);
 }
@@ -1261,13 +1261,13 @@ int launch_direct(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& s
 template <int EPI, int WM, int WN, int TM, int TN, int BK, int STAGES>
 int launch_turns(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
   typedef TurnsShape<WM, WN, TM, TN, BK, STAGES> S;
-  static bool raised = false;
+  static std::atomic<bool> raised{false};
   return launch_tiles(gemm_mfma_turns_kernel<EPI, WM, WN, TM, TN, BK, STAGES>, raised, S::kRowsA, S::kRowsW, S::kThreads, S::kLdsBytes, o, ra, scale);
 }
 
 template <int EPI>
 int launch_halves(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
-  static bool raised = false;
+  static std::atomic<bool> raised{false};
   return launch_tiles(gemm_mfma_halves_kernel<EPI>, raised, 256, 256, HalvesShape::kThreads, HalvesShape::kLdsBytes, o, ra, scale);
 }
 
@@ -1394,7 +1394,7 @@ template <int EPI, bool LARGE>
 int launch_rest(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& scale) {
   constexpr int kRows = LARGE ? 256 : 128, kLds = LARGE ? HalvesShape::kLdsBytes : TurnsShape<2, 4, 2, 1, 64, 4>::kLdsBytes;
   static_assert(RestShape::kLdsBytes <= kLds, "both tiles in one workgroup's LDS");
-  static bool raised = false;
+  static std::atomic<bool> raised{false};
   auto kernel = gemm_mfma_rest_kernel<EPI, LARGE>;
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)

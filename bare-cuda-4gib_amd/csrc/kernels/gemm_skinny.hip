@@ -1038,7 +1038,7 @@ template <int EPI, int ROWS, int NB, int KS, int S, bool NORMED, bool PAST>
 int launch_ring_form(const SkinnyArgs& a, int row_groups, hipStream_t s) {
   typedef RingShape<ROWS, NB, KS, S, NORMED> P;
   auto kernel = gemm_ring_kernel<EPI, ROWS, NB, KS, S, NORMED, PAST>;
-  static bool raised = false;
+  static std::atomic<bool> raised{false};
   if (!raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, P::kLdsBytes + (NORMED ? kRingNormBytes : 0)) !=
         hipSuccess)
@@ -1162,7 +1162,7 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
     if (stage > kMaxStageBytes) return fail("gemm_skinny: %d rows of k=%d do not fit the staging buffer", a.m, a.k);
     if (normed_ring_operands(a)) return launch_normed_rings<EPI>(a, s);
     auto kernel = gemm_skinny_kernel<1, EPI, XMODE, 4>;
-    static bool raised = false;   // per instantiation: allow more than the default dynamic LDS
+    static std::atomic<bool> raised{false};   // per instantiation: allow more than the default dynamic LDS
     if (!raised) {
       if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                               kMaxStageBytes) != hipSuccess)
