@@ -73,6 +73,34 @@ def test_counters_are_left_alone_where_a_kernel_merges(ops, heads, kv_heads, d, 
     assert torch.equal(run(arrived), run(None)) and (arrived == (0 if used else 77)).all()
 
 
+@pytest.mark.parametrize("n_splits", [2, 8])
+@pytest.mark.parametrize("heads, kv_heads, d", [(8, 2, 64), (32, 4, 64), (4, 4, 128)])
+def test_short_requests_beside_others(ops, heads, kv_heads, d, n_splits):
+    """A mixed step: tiles of the short requests alone, rows of the others left as another launch made them."""
+    gen = torch.Generator().manual_seed(heads + n_splits)
+    new, lengths, width = [1, 70, 2, 1, 33, 1], [900, 0, 40, 1500, 64, 3], 26
+    S, rows = len(new), sum(new)
+    draw = lambda *shape: torch.randn(*shape, generator=gen).bfloat16().to(DEV)      # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)      # noqa: E731
+    kc, vc, q = draw(S * width, kv_heads, 64, d), draw(S * width, kv_heads, d, 64), draw(rows, heads * d)
+    table = torch.randperm(S * width, generator=gen).view(S, width).int().to(DEV)
+    starts, tiles, tpt = [0], [0], ops.attention_tile_tokens(heads, kv_heads)
+    for n in new:
+        starts.append(starts[-1] + n)
+        tiles.append(tiles[-1] + (-(-n // tpt) if n <= tpt else 0))
+    row_seq = i32([s for s, n in enumerate(new) for _ in range(n)])
+    others, arrived = draw(rows, heads * d), torch.zeros(tiles[-1] * kv_heads, dtype=torch.int32, device=DEV)
+
+    def run(counters):
+        return ops.attention_mfma(q, kc, vc, table, i32(starts), i32(lengths), i32(tiles), tiles[-1], heads, kv_heads, d, 0, d ** -0.5, n_splits, 1, 1,
+                                  out=others.clone(), row_seq=row_seq, arrived=counters)
+    want = run(None)
+    long_rows = torch.tensor([n > tpt for n in new], device=DEV)[row_seq.long()]
+    assert torch.equal(want[long_rows], others[long_rows]) and not torch.equal(want[~long_rows], others[~long_rows])
+    for _ in range(3):
+        assert torch.equal(run(arrived), want) and not arrived.any()
+
+
 def test_too_few_counters_are_refused(ops):
     from bare_cuda_4gib_amd.errors import KernelError
     z = lambda *shape: torch.zeros(*shape, dtype=torch.int32, device=DEV)      # noqa: E731

@@ -18,9 +18,12 @@ def ops():
 
 def off_by_eight(x):
     """x at an address that is 8 bytes past a boundary of 16."""
-    room = torch.empty(x.numel() + 4, dtype=x.dtype, device=x.device)
-    room[4:] = x.reshape(-1)
-    return room[4:].view(x.shape)
+    past = 8 // x.element_size()
+    room = torch.empty(x.numel() + past, dtype=x.dtype, device=x.device)
+    room[past:] = x.reshape(-1)
+    moved = room[past:].view(x.shape)
+    assert x.data_ptr() % 16 == 0 and moved.data_ptr() % 16 == 8
+    return moved
 
 
 def operands(ops, m, n, k, seed=0):
@@ -105,7 +108,12 @@ def test_norm_fused(ops, m, n, k, g_dtype):
     if not ops.gemm_normed_supported(x, m, g, w):
         pytest.skip("the norm runs apart")
     rows = torch.tensor([m + 1 - r for r in range(m)], dtype=torch.int32, device=DEV)
-    other, first = off_by_eight(x), x[:m].contiguous()
+    other, first = off_by_eight(x), x[:m].clone()
+    # against float64: the operands are bfloat16(x * g), the sums and the rows' scales float32
+    turned, scale = (first * g.float()).bfloat16().double(), torch.rsqrt((first.double() ** 2).mean(1, keepdim=True) + 1e-5)
+    want = turned @ w.rows.double().T * scale
+    bound = 4 * k ** 0.5 * 2.0 ** -24 * (turned.abs() @ w.rows.double().abs().T * scale).max() + 2.0 ** -21 * want.abs().max()
+    assert (ops.gemm_normed(first, None, m, g, 1e-5, w, ops.EPI_STORE_F32).double() - want).abs().max() < bound
     epilogues = [ops.EPI_STORE_F32, ops.EPI_STORE_BF16, ops.EPI_SQUARED_RELU] + ([ops.EPI_SWIGLU] if n % 16 == 0 else [])
     for e in epilogues:
         assert torch.equal(ops.gemm_normed(x, rows, m, g, 1e-5, w, e), ops.gemm_normed(other, rows, m, g, 1e-5, w, e))
