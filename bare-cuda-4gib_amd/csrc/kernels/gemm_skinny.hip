@@ -1,19 +1,23 @@
 // out[m, n] = sum_k x[m, k] * w[n, k] for few rows m (a decode step: m <= 64), bfloat16 weights.
 //
-// The weights are read once, straight from memory into matrix-core registers: a workgroup owns
+// Two kernels, the same bits.  gemm_ring_kernel (below) brings weights and rows through rings in LDS and takes most products of k in whole steps of 64;
+// gemm_skinny_kernel, the streaming kernel, takes them straight into registers, and serves every other k, operands off 16-byte boundaries, the
+// fused norm of many or short rows, and the sizes at which it is the faster one (rings_are_slower).  What both do:
+//
+// The weights are read once: a workgroup owns
 // 16 output columns n (16 rows of w) and all of k; its 8 waves split k between them, each wave
 // feeding 16x16x32 MFMAs with w as the A operand and x as the B operand.  The weights come
 // *packed in fragment order*: for every block of 16 rows and every k-step of 32, the 1 KB that a
 // wave's 64 lanes load (lane l: row l % 16, k 8 * (l / 16) .. + 7) lies contiguous, blocks and
 // k-steps in order -- so every load instruction reads eight whole cache lines and a wave walks
 // straight through memory (rows past n and k past the matrix are stored as zeros).  Loads run
-// one batch of k-steps ahead of the MFMAs that use them.  The waves' partial sums meet in LDS
+// ahead of the MFMAs that use them, by a batch of k-steps in registers or by as many stages as the rings have.  The waves' partial sums meet in LDS
 // and are added in wave order, so a result does not depend on the number of rows or on timing.
 // Where the weight blocks are few and the rows of x more than eight, two workgroups share a block,
 // each with half of the rows of x (what a CU can pull through its cache bounds the kernel, so the
 // pulling is spread).
 //
-// What comes in (XMODE):
+// What comes in (XMODE; as the streaming kernel takes it):
 //   plain    x is bfloat16 [m, k].  The B operand's own pattern (a lane group reads 16 bytes of
 //            each of 16 rows) keeps the texture path busy four times as long as a load of whole
 //            cache lines, and with 64 rows x is four times the weights' traffic: so x comes in row
@@ -29,7 +33,6 @@
 //            (below), together with parts of every row's sum of squares: the row's scale is worked out
 //            from the parts while the weights are on their way and multiplies the finished sum -- the
 //            norm costs neither a kernel of its own nor the staging of the float rows.
-// Plain and prenormed rows, and few normed ones, go through rings in LDS where k is a multiple of 64 (gemm_ring_kernel, below): the same bits.
 // What goes out (EPI): bfloat16 or float stored; bfloat16 after max(., 0)^2 or xIELU (8 rows,
 // 2,048 to 8,192: product with its norm inside 13.0 us and the activation behind it 5.5; normed before and activated here 8.8);
 // float added into the residual stream; SwiGLU,
@@ -338,11 +341,9 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
   // the parts of blocks j, j + 8, ... in ascending order; the eight sums meet in LDS and are added in
   // order of j after the product: the order of the additions, and so the rounding, is the same for
   // every number of rows.  (After the first weights have been asked for.)  How many parts a thread asks
-  // for together, by what was measured inside a model: sixteen -- one way to memory and back for 128
-  // parts instead of four -- up to 8 rows in the kernels that serve those (four k-steps a turn, and the
-  // SwiGLU product: a decode step at TinyLlama's sizes 1.000 -> 0.983 ms at 8 rows, 0.922 -> 0.917 at
-  // one), four otherwise (with sixteen or eight a step of 16 rows was 0.4-0.8 % longer, and the other
-  // kernels of two k-steps a turn spilled).
+  // for together: sixteen -- one way to memory and back for 128 parts instead of four -- where a workgroup has up to 8 rows, in the kernels
+  // of four k-steps a turn and before gates (us, weights from memory, four and sixteen: 8 rows 4,096 x 2,720 8.4 and 8.0, 11,264 x 2,080 gated 12.6 and 11.9,
+  // 12 rows as two workgroups of six 2,048 x 5,480 13.0 and 11.5), four otherwise (the other kernels of two k-steps a turn spill with more).
   constexpr int kPartSums = 8;
   __shared__ float part_sum[kPartSums][MT * 16];
   const bool prenormed = !kNormed && a.ssq_parts != nullptr;
@@ -404,10 +405,9 @@ __global__ __launch_bounds__(kThreads, (XMODE != kPlain || (MT == 1 && U == 2)) 
   // may be skipped it cannot know how many were issued after the ones it waits for and waits for all of them, and a
   // copy from one set of registers to the other waits for the load it copies -- every batch then waits for the batch
   // asked for just before it.  With 32 rows a workgroup, whole batches are loaded so and multiplied from the
-  // registers they were loaded into, two a turn (64 rows as two workgroups of 32: the down projection of 5,632
-  // 10.9 -> 9.0 us, the others 2-4 % less); with 16 rows the plain loop is the faster one (4.2 against 4.7 us for a
-  // 2,048 x 2,048 block of weights), and with 48 and 64 rows a workgroup the second set of registers does not fit the
-  // 128 a wave has (spilled, the q|k|v product of 64 rows and 4,096 columns took 127 instead of 44 us).
+  // registers they were loaded into, two a turn (us, weights from memory, without and so: 64 rows as two workgroups of 32 2,048 x 5,480 15.5 and 14.3, behind
+  // a norm 18.3 and 15.6; 32 rows 11,264 x 2,080 gated 19.7 and 16.4); with 16 rows the plain loop is the faster one, and with 48 and 64 rows a workgroup
+  // the second set of registers does not fit the 128 a wave has (spilled, a product took three times as long).
   constexpr bool kPingPong = MT == 2;
   const int last_row_offset = (m - 1) * k;              // (m <= 64 rows: an int)
   int turn_offset[kXLoads];
@@ -1175,9 +1175,8 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
     // Every workgroup reads all its rows of x, and what a CU can pull through its cache is what bounds
     // the kernel once x is as large as the block's weights (16 rows).  Where the weight blocks are
     // few (up to one a CU: n = 4,096), two workgroups share a block's rows: each pulls half of
-    // x, and the block's weights are read twice, once of it from L2 (measured at TinyLlama's sizes:
-    // 1.80 -> 1.51 ms a step at 64 rows, 1.36 -> 1.26 at 32, 1.15 -> 1.12 at 16; four workgroups a
-    // block, or splitting the wide gate-up product too, are no faster).
+    // x, and the block's weights are read twice, once of it from L2 (us, weights from memory, one and two: 2,048 x 5,480 16 rows 10.8 and 9.6, 32 rows 15.2 and
+    // 10.6, 64 rows 22.5 and 14.3; 32 rows 2,048 x 1,024 4.8 and 3.7; not at 16 rows of wider ones, 2,720 x 1,376 4.9 and 5.5).
     SkinnyArgs b = a;
     int tiles = mt;
     if (a.m > kSplitMinRows && static_cast<int>(grid.x) <= compute_units()) {
@@ -1186,22 +1185,18 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
       grid.y = 2;
     }
     if (a.m <= kSplitMinRows) {
-      // Few rows.  What bounds a weight of few blocks (2,048 x 5,632: 128 of 180 KB) is how many of its bytes are on their way
+      // Few rows.  What bounds a weight of few blocks (2,048 x 5,480: 128 of 175 KB) is how many of its bytes are on their way
       // at once, so with at most three blocks for every four CUs a wave asks for eight k-steps together (two workgroups of
       // four would not share a CU anyway), and with at most a block for every other CU and a long k two workgroups
       // share a block, each with eight of its outputs (b.halves; the lanes of the other eight rows repeat
-      // theirs, the same sums in the same order).  One row, weights from memory: 2,048 x 5,632 8.6 -> 7.3 us, 2,048 x
-      // 2,048 4.6 -> 4.3, 2,560 x 2,048 4.75 -> 4.5; a decode step at TinyLlama's sizes 0.846 -> 0.806 ms for one request, 0.949 ->
-      // 0.894 for 4, 0.99 -> 0.959 for 8 (eight k-steps from 9 rows on: 16 requests 1.054 -> 1.082, so only here).
-      // (Four k-steps for more blocks: 4,096 x 4,096 takes 8.3 us, with eight 8.5.)
-      // (a wide product's many workgroups, more than two a CU: with fewer k-steps in flight each they
-      // need half the registers, and all of them are on the CUs at once -- the gate-up product of 8
-      // rows after a prepared norm: a decode step 1.020 -> 0.990 ms)
+      // theirs, the same sums in the same order).  us, weights from memory, four k-steps and eight: 2,048 x 5,480 one row 8.8 and 7.5, 8 rows 9.0 and 8.3, 2,720 x 1,376
+      // behind a norm, one row 5.1 and 4.7; whole blocks and halves: 2,048 x 5,480 one row 7.8 and 7.5, 8 rows 9.2 and 8.3, 1,024 x 5,480 8.0 and 6.9.
+      // (A wide product's many workgroups, more than two a CU: with fewer k-steps in flight each they
+      // need half the registers, and all of them are on the CUs at once.  Four k-steps and two: 8 rows 11,264 x 2,080 behind a norm, gated, 15.5 and 11.9, one row
+      // 32,000 x 512 9.4 and 7.3.)
       const int blocks = static_cast<int>(grid.x);
       // A last batch of eight that four would hold -- every k up to 1,024, where it is the only one, and 2,049 to 3,072 -- adds
-      // nothing but work for zeros: four there (8 rows: 1,024 x 1,024 3.84 us with eight, 3.34 with four, 2,560 x 3,072 6.57 and 6.34,
-      // 256 x 64 2.47 and 2.35).  Without such a batch eight are 0.99 to 1.14 times as fast for one row and 0.94 to 1.08 for 8, over
-      // 512 to 3,072 outputs by 1,152 to 8,192.
+      // nothing but work for zeros: four there (8 rows: 1,024 x 1,024 3.84 us with eight, 3.34 with four).
       const int last = (a.k + kWaves * 64 - 1) / (kWaves * 64) * 2 % 8;
       const bool eights = last == 0 || last > 4;
       if constexpr (EPI == kAccumF32 || EPI == kStoreF32 || EPI == kStoreBf16) {
@@ -1220,7 +1215,7 @@ int launch(const SkinnyArgs& a, hipStream_t s) {
     switch (tiles) {
       // k-steps per batch chosen so that two batches of operands fit 128 registers (two workgroups a CU)
       case 1:
-        // (a wide product's many workgroups: as above)
+        // (a wide product's many workgroups: as above; 16 rows 32,000 x 512 behind a norm 12.1 and 9.0)
         if (static_cast<int>(grid.x) > 2 * compute_units()) gemm_skinny_kernel<1, EPI, XMODE, 2><<<grid, block, 0, s>>>(b);
         else gemm_skinny_kernel<1, EPI, XMODE, 4><<<grid, block, 0, s>>>(b);
         break;
