@@ -767,7 +767,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
 
   // prenormed x: wave j adds up chain j of every row's parts, parts j, j + 8, ... in ascending order.  A part's numbers of ROWS rows (pairs of
   // them, where half blocks left it) lie side by side: four of them a lane, 2^shift lanes a part, up to 256 parts (128 pairs) asked for before the walk.
-  // (Past the last part or number: the last four, turned into place after the walk.)
+  // (Past the last part, or the last of its rows that the call names -- the parts may be those of more rows, and the call's their last --: the last four,
+  // turned into place after the walk.)
   constexpr int kHeld = ROWS <= 8 ? 1 : ROWS / 8;
   typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
   const bool prenormed = EPI != kAccumF32 && !NORMED && a.ssq_parts != nullptr, pairs = ROWS == 8 && a.ssq_halves;
@@ -938,7 +939,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_ring_kernel(const SkinnyArgs
 #pragma unroll
     for (int h = 0; h < kHeld; ++h) {
       floatx4 v = held[h];
-      if (part_stride < first_row + (pairs ? 2 * ROWS : ROWS)) {                          // (only then a load of the last parts may end past them)
+      if (m < ROWS) {                                                                     // (only then a load of the last parts may end past them)
         const int turn = max(0, part_at(h) - last_four);
         if (turn & 1) v = floatx4{v[1], v[2], v[3], v[3]};
         if (turn & 2) v = floatx4{v[2], v[3], v[3], v[3]};
@@ -1052,7 +1053,7 @@ int launch_ring_form(const SkinnyArgs& a, int row_groups, hipStream_t s) {
   b.chunk = (a.k + kWaves * 64 - 1) / (kWaves * 64) * 64;
   b.last_block = blocks - 1;
   b.part_stride = a.ssq_stride * (a.ssq_halves ? 2 : 1);
-  b.last_four = a.ssq_blocks * b.part_stride - 4;
+  b.last_four = (a.ssq_blocks - 1) * b.part_stride + a.m * (a.ssq_halves ? 2 : 1) - 4;
   b.x_row_bytes = NORMED ? ring_row_bytes(a.k) : 0;
   kernel<<<grid, dim3(kThreads), P::kLdsBytes + (NORMED ? ring_norm_bytes(a.m, a.k, a.g_f32) : 0), s>>>(b);
   return check_launch("gemm_skinny");
@@ -1115,7 +1116,7 @@ bool normed_ring_operands(const SkinnyArgs& a) {
 // What the rings take: the loads bring 16 bytes from 16-byte boundaries, a stage is 64 values of k, parts of a norm are read four numbers at a time and the
 // next norm's scale two.
 bool ring_operands(const SkinnyArgs& a) {
-  return a.k % 64 == 0 && (a.ssq_parts == nullptr || static_cast<long>(a.ssq_blocks) * a.ssq_stride >= 4) && (a.emit_g == nullptr || a.n > 1) &&
+  return a.k % 64 == 0 && (a.ssq_parts == nullptr || (a.ssq_blocks - 1L) * a.ssq_stride + a.m >= 4) && (a.emit_g == nullptr || a.n > 1) &&
          reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && reinterpret_cast<uintptr_t>(a.w) % 16 == 0;
 }
 

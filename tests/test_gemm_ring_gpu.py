@@ -1,5 +1,7 @@
 """The few-row product through rings in LDS against the streaming kernel, which takes the same operands where x lies off a 16-byte
 boundary: the same bits from either, at the edges of the row counts, blocks of outputs and parts of k that a workgroup and its waves take."""
+import dataclasses
+
 import pytest
 import torch
 
@@ -78,6 +80,22 @@ def test_norms_prepared_and_finished(ops, m, n, k, g_dtype):
             assert torch.equal(ops.gemm_prenormed(left, after, epilogue), ops.gemm_prenormed(shifted, after, epilogue))
         if left.parts.dim() == 2:
             assert torch.equal(ops.gemm_xielu(left.xb, after, pq, pre=left), ops.gemm_xielu(shifted.xb, after, pq, pre=shifted))
+
+
+@pytest.mark.parametrize("n", [64, 2048])
+@pytest.mark.parametrize("m", [65, 67, 72, 73, 77, 81, 97])
+def test_norms_of_more_rows_than_one_launch_takes(ops, monkeypatch, m, n):
+    """Rows from the 65th on go into a launch of their own, whose parts end with them and not with a whole part of all rows."""
+    x, w = operands(ops, m, n, 512)
+    after = ops.StreamedWeight((torch.randn(1600, n, device=DEV) * n ** -0.5).bfloat16())
+    for weight in (w, after):
+        monkeypatch.setitem(ops._PLANS, tuple(weight.shape), dataclasses.replace(ops.plan_for(*weight.shape), stream_rows=128))
+    g, base = 1 + 0.1 * torch.randn(n, device=DEV), torch.randn(m, n, device=DEV)
+    pre = ops.gemm_accumulate_emit(x, w, base.clone(), g, 1e-5)
+    both = ops.gemm_prenormed(pre, after, ops.EPI_STORE_F32)
+    for rows in (slice(0, 64), slice(64, m)):
+        own = ops.Prenormed(pre.xb[rows].contiguous(), pre.parts[:, rows].contiguous(), pre.eps)
+        assert torch.equal(both[rows], ops.gemm_prenormed(own, after, ops.EPI_STORE_F32))
 
 
 @pytest.mark.parametrize("heads, kv_heads, head_dim, page", [(4, 2, 16, 16), (32, 4, 64, 64), (32, 8, 128, 64), (48, 48, 64, 24)])
