@@ -11,9 +11,9 @@
 extern "C" {
 
 const char* bc4g_last_error();
-// Of the calling thread's launches from here on: whether the weights of its steps, all together, stay in the caches from step to step (stay: 1), so
-// that none of them is loaded past the caches, or need not (0, as every thread begins).  What is computed is the same.
-int bc4g_weights_stay(int stay);
+// Of the calling thread's launches from here on: whether the weights of its steps, all together, are more than the caches keep from step to step
+// (pass: 1), so that large ones that few rows are multiplied by are loaded past them, or may stay (0, as every thread begins).  What is computed is the same.
+int bc4g_weights_pass(int pass);
 // Whether a weight of n x k numbers that few rows are multiplied by would be loaded past the caches (passes: 1) by this thread.
 int bc4g_weight_passes(int n, int k, int bytes_a_number, int* passes);
 int bc4g_version();

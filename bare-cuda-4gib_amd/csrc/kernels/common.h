@@ -118,10 +118,10 @@ enum DType : int { kF32 = 0, kBF16 = 1 };
 // Records a message for bc4g_last_error() and returns a non-zero status.
 int fail(const char* fmt, ...);
 int check_launch(const char* what);
-int compute_units();
+int compute_units();   // of the current device (256 if it cannot be asked)
 
-// What this thread has last said by bc4g_weights_stay.
-bool weights_stay();   // of the current device (256 if it cannot be asked)
+// What this thread has last said by bc4g_weights_pass.
+bool weights_pass();
 
 __device__ inline float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 // softplus(p) z^2 + z / 2 for z > 0, (1/2 + softplus(q)) (e^z - 1 - z) + z / 2 otherwise: ap = softplus(p), aq = 1/2 + softplus(q).

@@ -35,13 +35,13 @@ int compute_units() {
   return cus[dev];
 }
 
-static thread_local bool g_weights_stay = false;
-bool weights_stay() { return g_weights_stay; }
+static thread_local bool g_weights_pass = false;
+bool weights_pass() { return g_weights_pass; }
 
 }  // namespace bc4g
 
-extern "C" int bc4g_weights_stay(int stay) {
-  bc4g::g_weights_stay = stay != 0;
+extern "C" int bc4g_weights_pass(int pass) {
+  bc4g::g_weights_pass = pass != 0;
   return 0;
 }
 

@@ -94,11 +94,11 @@ __device__ inline void load_to_lds_16(const void* wave_base, unsigned lane_offse
 }
 
 // Whether a weight that every workgroup reads its own part of once is loaded past the caches ("nt"): with a model of some hundred MB behind it
-// nothing of it is left by the next step, and what it would put out is.  From 6 MB a weight on (8 rows, bfloat16, weights from memory, 2,048 x 5,632 7.1 us
-// and 6.8 past the caches, 2,560 x 2,048 5.7 and 5.4), unless the caller has said that all the weights of its steps stay in the 256 MB of cache
-// (bc4g_weights_stay; the model's total decides, see Model.bind): there the same two take 6.3 and 6.9, 5.2 and 5.5.
+// nothing of it is left by the next step, and what it would put out is.  Where the caller has said that its steps read more weights than the 256 MB of cache
+// keep (bc4g_weights_pass; the model's total decides, see Model.bind), from 6 MB a weight on: 8 rows, bfloat16, weights from memory, 2,048 x 5,632 7.1 us
+// and 6.8 past the caches, 2,560 x 2,048 5.7 and 5.4; with the weight still in the cache 6.3 and 6.9, 5.2 and 5.5.
 constexpr long kPassingBytes = 6L << 20;
-inline bool passes_by(int n, int k, int bytes_a_number) { return !weights_stay() && static_cast<long>(n) * k * bytes_a_number >= kPassingBytes; }
+inline bool passes_by(int n, int k, int bytes_a_number) { return weights_pass() && static_cast<long>(n) * k * bytes_a_number >= kPassingBytes; }
 
 // Several such loads to one stretch of LDS as ONE statement: N chunks of 1 KB side by side, chunk r from bases[r]
 // (the same in every lane) plus each lane's offset in bytes.  The LDS address is set once, to the chunk in the

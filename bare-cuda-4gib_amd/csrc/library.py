@@ -50,7 +50,7 @@ _SIGNATURES = {
     "bc4g_gemm_skinny": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "bc4g_gemm_mfma": [_P, _P, _I, _P, _P, _I, _I, _I, _I, _P],
     "bc4g_gemm_mfma_tile": [_P, _P, _I, _I, _I, _I, _P, _P],
-    "bc4g_weights_stay": [_I],
+    "bc4g_weights_pass": [_I],
     "bc4g_weight_passes": [_I, _I, _I, _P],
     "bc4g_gemm_skinny_rings": [_I, _I, _I, _I, _I, _P],
     "bc4g_gemm_mfma_cut": [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P],

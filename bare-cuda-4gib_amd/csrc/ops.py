@@ -98,14 +98,14 @@ def tiled_cut(m: int, n: int, k: int, qkv: bool = False) -> Tuple[int, Optional[
 
 
 @contextlib.contextmanager
-def weights_stay():
-    """Around the launches of a step whose weights, all together, stay in the caches from step to step: none of them is then loaded past the caches,
-    however large it is.  For this thread's launches and no longer than the block; what is computed is the same."""
-    library.call("bc4g_weights_stay", 1, launches=False)
+def weights_pass():
+    """Around the launches of a step whose weights, all together, are more than the caches keep from step to step: large ones that few rows are multiplied
+    by are then loaded past the caches.  For this thread's launches and no longer than the block; what is computed is the same."""
+    library.call("bc4g_weights_pass", 1, launches=False)
     try:
         yield
     finally:
-        library.call("bc4g_weights_stay", 0, launches=False)
+        library.call("bc4g_weights_pass", 0, launches=False)
 
 
 def weight_passes(n: int, k: int, bytes_a_number: int = 2) -> bool:

@@ -78,7 +78,7 @@ class Model:
         self.max_seq_len = spec.max_seq_len
         self.streams = int(getattr(spec, "streams", 1))
         self.rt: Optional[Runtime] = None
-        self.weights_stay = False         # whether the weights of a step stay in the caches from one to the next
+        self.weights_stay = True          # whether the weights of a step stay in the caches from one to the next
         self.cached_weight_bytes = 0      # of those weights, what a step of few rows loads through the caches
 
     def all_parts(self) -> List[Part]:
@@ -144,9 +144,9 @@ class Model:
         if cuda and not self.weights_stay:
             from ..csrc import ops
             maps = {id(w): w for part in self.all_parts() for w in vars(part).values() if isinstance(w, ops.StreamedWeight)}
-            for w in maps.values():
-                if w.dim() == 2 and ops.weight_passes(*w.shape, w.element_size()):
-                    self.cached_weight_bytes -= w.shape[0] * w.shape[1] * w.element_size()
+            with ops.weights_pass():
+                passing = [w for w in maps.values() if w.dim() == 2 and ops.weight_passes(*w.shape, w.element_size())]
+            self.cached_weight_bytes -= sum(w.shape[0] * w.shape[1] * w.element_size() for w in passing)
 
     # ---- cache --------------------------------------------------------------
     def _cache_spec(self, layer: int):
@@ -221,10 +221,10 @@ class Model:
     def forward(self, ctx: StepContext) -> Optional[torch.Tensor]:
         """Run the batch through every schedule entry; float32 logits at the
         wanted rows ([n_logits, vocab]), or None if none are wanted."""
-        if not self.weights_stay or self.rt.device.type != "cuda":
+        if self.weights_stay or self.rt.device.type != "cuda":
             return self._forward(ctx)
         from ..csrc import ops
-        with ops.weights_stay():
+        with ops.weights_pass():
             return self._forward(ctx)
 
     def _forward(self, ctx: StepContext) -> Optional[torch.Tensor]:

@@ -14,7 +14,8 @@ EPS = 1e-5
 @pytest.fixture(scope="module")
 def ops():
     from bare_cuda_4gib_amd.csrc import ops as o
-    return o
+    with o.weights_pass():                # (weights of 6 MB and more past the caches, as in the steps of a large model)
+        yield o
 
 
 def held(got, want, bound, what):

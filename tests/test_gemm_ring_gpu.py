@@ -15,7 +15,8 @@ def ops():
     if not torch.cuda.is_available():
         pytest.skip("needs a GPU")
     from bare_cuda_4gib_amd.csrc import ops as _ops
-    return _ops
+    with _ops.weights_pass():             # (weights of 6 MB and more past the caches, as in the steps of a large model)
+        yield _ops
 
 
 def off_by_eight(x):

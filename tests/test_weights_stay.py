@@ -1,4 +1,4 @@
-"""Weights of models that stay in the caches are not loaded past them: which models those are, for which launches that holds, and the same bits."""
+"""Large weights are loaded past the caches by models whose weights do not stay there: which models those are, for which launches, and the same bits."""
 import threading
 
 import pytest
@@ -31,19 +31,19 @@ def test_the_weights_a_step_reads_decide(monkeypatch, tied):
         assert bound(tied).weights_stay is stays
 
 
-def test_weights_of_a_model_that_stays_are_loaded_through_the_caches():
-    """However large each is: a narrow model's wide head, a 32-bit matrix."""
-    assert ops.weight_passes(32000, 768) and ops.weight_passes(1536, 1024, 4) and not ops.weight_passes(1536, 2044)
+def test_a_thread_s_launches_inside_the_block():
+    """However large a weight is, by itself it is loaded through the caches: a narrow model's wide head, a 32-bit matrix."""
+    assert not ops.weight_passes(32000, 768) and not ops.weight_passes(1536, 1024, 4)
     seen = []
-    with ops.weights_stay():
-        assert not ops.weight_passes(32000, 768) and not ops.weight_passes(1536, 1024, 4)
+    with ops.weights_pass():
+        assert ops.weight_passes(32000, 768) and ops.weight_passes(1536, 1024, 4) and not ops.weight_passes(1536, 2044)
         other = threading.Thread(target=lambda: seen.append(ops.weight_passes(32000, 768)))
         other.start(), other.join()
-    assert seen == [True] and ops.weight_passes(32000, 768)
+    assert seen == [False] and not ops.weight_passes(32000, 768)
     with pytest.raises(ZeroDivisionError):
-        with ops.weights_stay():
+        with ops.weights_pass():
             1 / 0
-    assert ops.weight_passes(32000, 768)
+    assert not ops.weight_passes(32000, 768)
 
 
 @pytest.mark.parametrize("stays", [False, True])
@@ -51,7 +51,7 @@ def test_a_step_says_so_for_its_own_launches(monkeypatch, stays):
     model = bound(False)
     model.weights_stay, model.rt = stays, Runtime(torch.device("cuda:0"), torch.float32)
     monkeypatch.setattr(model, "_forward", lambda ctx: ops.weight_passes(32000, 768))
-    assert model.forward(None) is not stays and ops.weight_passes(32000, 768)
+    assert model.forward(None) is not stays and not ops.weight_passes(32000, 768)
 
 
 @pytest.mark.gpu
@@ -61,7 +61,7 @@ def test_the_same_bits_either_way(m, dtype):
     gen = torch.Generator(device="cuda:0").manual_seed(m)
     x, w = (torch.randn(n, 1088, generator=gen, device="cuda:0").to(dtype) for n in (m, 8208))
     product = (lambda: ops.gemm_f32(x, w)) if dtype == torch.float32 else (lambda: ops.gemm_fast(x, w, torch.float32))
-    past = product()
-    with ops.weights_stay():
-        through = product()
+    through = product()
+    with ops.weights_pass():
+        past = product()
     assert torch.equal(past, through)
