@@ -59,7 +59,7 @@ class StepContext:
     # the part noted for itself on the host).
     step_data: Dict[Hashable, Tuple[Dict[str, torch.Tensor], Any]] = dataclasses.field(default_factory=dict)
     captured: bool = False               # see HostBatch
-    # Whether what the requests may hold up to max_kv_len tokens each, and the weights that go through the caches beside it, is more than those keep
+    # Whether the requests' keys and values, as far as max_kv_len tells, and the weights that go through the caches beside them are more than those keep
     # from one decode step to the next: kernels then read keys and values past them (Executor.cache_passes).
     cache_passes: bool = False
     # Who reads the residual stream next and what the product before left for that reader: see NormHandoff.

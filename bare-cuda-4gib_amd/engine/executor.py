@@ -56,13 +56,14 @@ class StepEntry:
     want: Sequence[int] = ()
 
 
-# Keys and values of a decode step, as far as its requests may reach, beside the weights that go through the caches, from which on they are loaded past the
-# card's 256 MB of cache: two fifths more, as a captured step plans for the end of a context bucket and its contexts are three quarters of that on average.  us a
-# step, through the caches and past them, by bytes at the bound: TinyLlama's 22 layers, 8 requests, at 500 tokens (185 MB) 779.6 and 801.4, at 1,500 (369 MB) 822.9
-# and 829.0, 16 at 2,000 (738 MB) 1,049.7 and 1,045.2; eight layers of Llama-3-8B's, 8 requests at 250 (67 MB) 846.4 and 858.5, 16 at 500 (268 MB) 1,033.9 and 1,041.8,
-# 8 at 2,000 (537 MB) 950.2 and 934.2; 12 layers of 768, 94 MB of weights through the caches, 8 at 250 (75 and 94 MB) 268.6 and 277.7, 16 at 500 (302 and 94) 367.8 and
-# 351.4.
-CACHE_HOLDS_BYTES = 360 << 20
+# A captured decode step serves contexts up to its bucket's bound: 256 tokens, or a power of two beyond, down to half of it.
+FIRST_BUCKET = 256
+# Keys and values of a decode step, at the middle of its contexts' bucket, and the weights that go through the caches beside them, from which on the keys and
+# values are loaded past the card's 256 MB of cache.  us a step, through the caches and past them, by MB of both: TinyLlama's 22 layers, 8 requests, at 500
+# tokens (138) 779.6 and 801.4, at 1,500 (277) 822.9 and 829.0, 16 at 2,000 (554) 1,049.7 and 1,045.2; eight layers of Llama-3-8B's, 8 requests at 250 (34) 846.4 and
+# 858.5, 16 at 500 (201) 1,033.9 and 1,041.8, 8 at 2,000 (403) 950.2 and 934.2; 12 layers of 768 with 94 MB of such weights, 8 at 250 (132) 268.6 and 277.7, 32 at 20 (245)
+# 345.0 and 353.6, 16 at 500 (320) 367.8 and 351.4.
+CACHE_HOLDS_BYTES = 280 << 20
 
 
 class Executor:
@@ -143,8 +144,10 @@ class Executor:
     def length(self, request: Hashable) -> int:
         return self.cache.length(request)
 
-    def cache_passes(self, n_requests: int, max_kv: int) -> bool:
-        """Whether a decode step of so many requests of up to max_kv tokens reads its keys and values past the caches."""
+    def cache_passes(self, n_requests: int, max_kv: int, captured: bool) -> bool:
+        """Whether a decode step of so many requests of up to max_kv tokens (captured: a bucket's bound) reads its keys and values past the caches."""
+        if captured:
+            max_kv = max_kv // 2 if max_kv <= FIRST_BUCKET else max_kv * 3 // 4
         return n_requests * self.cache.bytes_read(max_kv) + self.model.cached_weight_bytes >= CACHE_HOLDS_BYTES
 
     # ---- the step -----------------------------------------------------------
@@ -268,7 +271,7 @@ class Executor:
             seq_slots_dev=parts["seq_slots"], logit_rows=parts["logit_rows"], n_logits=host["n_logits"],
             block_tables=block_tables, slot_maps=slot_maps, max_q_len=host["max_q"], max_kv_len=host["max_kv"],
             cache_views=self._views, step_data=step_data, captured=host["captured"],
-            cache_passes=host["max_q"] == 1 and self.cache_passes(S, host["max_kv"]))
+            cache_passes=host["max_q"] == 1 and self.cache_passes(S, host["max_kv"], host["captured"]))
 
     def build_context(self, entries: Sequence[StepEntry]) -> StepContext:
         """Host arrays of the batch, uploaded in one copy."""
@@ -302,7 +305,7 @@ class Executor:
         if S > n_real:                      # the rows that stand for no request: the scratch slot, nothing cached
             slots = np.concatenate([slots, np.full(S - n_real, cache.scratch_slot, dtype=np.int32)])
         ctx = cache.lengths_by_slot[slots]
-        bucket = 256
+        bucket = FIRST_BUCKET
         while bucket < int(ctx.max()) + 1:
             bucket *= 2
         key = (S, bucket)

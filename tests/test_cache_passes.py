@@ -57,12 +57,13 @@ def test_a_captured_step_plans_for_its_bucket(monkeypatch):
             asked.append(args[-2])
         return call(name, *args, **more)
     monkeypatch.setattr(ops.library, "call", watched)
-    for most, reach, past in ((300, 256, 0), (4096, 256, 0), (300, 255, 1), (4096, 255, 1)):
+    # (the middle of a bucket: 128 tokens of the first, of up to 256, and 384 of the one after it)
+    for most, tokens, reach, past in ((300, 20, 128, 0), (4096, 20, 128, 0), (300, 20, 127, 1), (4096, 20, 127, 1), (600, 300, 384, 0), (4096, 300, 383, 1)):
         run = executor("cuda:0", torch.bfloat16, num_pages=80, max_requests=2, max_tokens=most)
         monkeypatch.setattr(executor_file, "CACHE_HOLDS_BYTES", run.model.cached_weight_bytes + 2 * reach * 256 + 1)
         for r in range(2):
             run.admit(r)
-            run.step([StepEntry(r, [3] * (20 + r), [])])
+            run.step([StepEntry(r, [3] * (tokens + r), [])])
         asked.clear()
         run.step([StepEntry(r, [1], [0]) for r in range(2)])
         assert run.captures == 1 and asked == [past] * 4            # (once outside the capture and once inside, two layers)
