@@ -74,3 +74,45 @@ def test_what_parts_cannot_hold(ops, m):
     x[0, 7], x[1], w[3, 7] = torch.finfo(torch.float32).max, 1.0, 0.5
     got = ops.gemm_f32(x, w)
     assert float(got[0, 3]) == torch.finfo(torch.float32).max / 2 and bool(torch.isfinite(got[1]).all())
+
+
+def small_and_large(seed, m, n, k, x_exp, w_exp):
+    gen = torch.Generator().manual_seed(seed)
+    at = lambda rows, exp: (torch.randn(rows, k, generator=gen, dtype=torch.float64) * 2.0 ** exp).float()      # noqa: E731
+    return at(m, x_exp), at(n, w_exp)
+
+
+# Operands down to the smallest denormals beside large ones, whichever of the two is small: every bit of an operand counts, however small it is.
+@pytest.mark.parametrize("m,n,k", [(3, 96, 256), (8, 96, 256), (8, 8200, 256), (12, 96, 256), (40, 96, 260), (100, 96, 256), (1000, 96, 256), (300, 2050, 1056)])
+@pytest.mark.parametrize("x_exp,w_exp", [(-112, 60), (-122, 60), (-125, 70), (-140, 75), (70, -125), (60, -140), (-70, -60), (-75, -70)])
+def test_small_operands(ops, m, n, k, x_exp, w_exp):
+    x, w = small_and_large(m + k, m, n, k, x_exp, w_exp)
+    got = ops.gemm_f32(x.to(DEV), w.to(DEV)).double().cpu()
+    z, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    # (a sum below the smallest normal float is rounded to multiples of 2^-149, each share's at most)
+    assert float(((got - z).abs() / ((k + 2) * U * size + 20 * 2.0 ** -149)).max()) <= 1.0
+
+
+@pytest.mark.parametrize("m", [3, 8, 12, 40, 100])
+def test_what_is_left_of_small_operands_that_cancel(ops, m):
+    """Products that take each other off but for the last bits of a small operand, and a sum of tiny products: neither is nothing."""
+    n, k = 32, 256
+    x, w = torch.zeros(m, k), torch.zeros(n, k)
+    x[:, 3], x[:, 200], w[:, 3], w[:, 200] = 2.0 ** -120 * (1 + 2.0 ** -23), -(2.0 ** -120), 2.0 ** 100, 2.0 ** 100
+    assert bool((ops.gemm_f32(x.to(DEV), w.to(DEV)) == 2.0 ** -43).all())
+    x, w = torch.full((m, k), 2.0 ** -70), torch.full((n, k), 2.0 ** -70)
+    assert bool((ops.gemm_f32(x.to(DEV), w.to(DEV)) == 2.0 ** -132).all())
+
+
+@pytest.mark.parametrize("m", [3, 8, 12, 40, 100])
+def test_large_operands_and_sums(ops, m):
+    """Beyond what the parts hold: operands up to the largest float, sums that are finite and such as are not."""
+    n, k = 40, 256
+    x, w = small_and_large(m, m, n, k, 100, 15)
+    x[0, 5], w[:, 5] = torch.finfo(torch.float32).max, 0.25
+    x[1] = 2.0 ** 100
+    w[7] = 2.0 ** 30
+    got = ops.gemm_f32(x.to(DEV), w.to(DEV)).double().cpu()
+    z, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    live = size < 2.0 ** 127
+    assert float(((got - z).abs() / ((k + 2) * U * size))[live].max()) <= 1.0 and bool(torch.isposinf(got[1, 7])) and not bool(live[1, 7])
