@@ -2,6 +2,8 @@
 33 to 64 rows, a k that ends inside a pair of shares, and operands that three bfloat16 cannot hold.
 
 Tolerance: a float32 sum of k products, in any order, is off by at most k 2^-24 sum |x w|."""
+import math
+
 import pytest
 import torch
 
@@ -116,3 +118,63 @@ def test_large_operands_and_sums(ops, m):
     z, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
     live = size < 2.0 ** 127
     assert float(((got - z).abs() / ((k + 2) * U * size))[live].max()) <= 1.0 and bool(torch.isposinf(got[1, 7])) and not bool(live[1, 7])
+
+
+INVALID = [(3, 96, 256), (8, 2048, 2080), (8, 11264, 512), (16, 90, 260), (40, 2050, 2048), (100, 2560, 2048), (300, 2046, 1056), (1000, 2562, 1056)]
+
+
+@pytest.mark.parametrize("m,n,k", INVALID)
+@pytest.mark.parametrize("epilogue", ["store", "add with bias", "silu"])
+def test_invalid_and_infinite_sums(ops, m, n, k, epilogue):
+    """What float arithmetic gives of them, in every kernel: a NaN, infinities of both signs and beside zeros, sums beyond the parts' range and
+    beyond float's.  The finite ones have the same bits whatever rows are beside them, and so have the rows without any of these."""
+    x, w = operands(m, n, k, m + n)
+    base, bias = torch.randn(m, n, device=DEV), torch.randn(n, device=DEV)
+
+    def product(rows):
+        if epilogue == "add with bias":
+            return ops.gemm_f32(x[rows].clone(), w, accumulate_into=base[rows].clone(), bias=bias)
+        return ops.gemm_f32(x[rows].clone(), w, act=None if epilogue == "store" else epilogue)
+
+    every = torch.arange(m, device=DEV)
+    before = product(every)
+    x[0, k // 2], x[1, k - 1] = float("nan"), -float("inf")
+    x[m - 1] *= 2.0 ** 90
+    w[n - 1, k - 1] = 0.0
+    got = product(every)
+    w_last = w[:, k - 1]
+    assert bool(torch.isnan(got[0]).all())
+    if epilogue != "silu":
+        assert bool(torch.isnan(got[1, n - 1])) and torch.equal(torch.isposinf(got[1]), w_last < 0) and torch.equal(torch.isneginf(got[1]), w_last > 0)
+        z, size = x[m - 1].double() @ w.double().T, x[m - 1].double().abs() @ w.double().abs().T
+        assert float(((got[m - 1].double() - z).abs() / ((k + 4) * U * size)).max()) <= 1.0
+    others = every[2:m - 1]
+    assert torch.equal(got[others, :-1], before[others, :-1])
+    for rows in ([m - 1], [0, m - 1], [1, 0, m - 1]):
+        assert torch.equal(product(torch.tensor(rows, device=DEV))[-1], got[m - 1])
+    w[:, k // 3] = float("inf")                             # every sum of every row
+    x[2:m - 1, k // 3] = 1.0
+    got = product(every)
+    assert bool((torch.isposinf(got) | torch.isnan(got))[2:m - 1].all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 11264, 2048), (256, 2048, 5632), (64, 11264, 2048), (8, 2048, 5632)])
+@pytest.mark.parametrize("what", ["all NaN", "an infinity a row", "one infinity"])
+def test_invalid_rows_do_not_hold_up_the_others(ops, m, n, k, what):
+    """A product with them takes a few times what it takes without (before they were added up by whole waves: 30 to 160 times)."""
+    x, w = operands(m, n, k, 1)
+    bad = x.clone()
+    if what == "all NaN":
+        bad[:] = float("nan")
+    else:
+        bad[:m if what == "an infinity a row" else 1, k // 2] = float("inf")
+
+    def fastest(y):
+        best = math.inf
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record(), ops.gemm_f32(y, w), b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+    assert fastest(bad) < 12.0 * fastest(x)
