@@ -61,8 +61,10 @@ int bc4g_gemm_generic(const void* a, int a_dtype, const void* w, int w_dtype, vo
 // epilogue 0: stored; 1: added to out, with bias [n] (null: none); 2, 3: w holds n / 2 gate rows, then as many up rows, and
 // out [m, n / 2] is silu (3: the gelu written with tanh) of the gate times up.
 int bc4g_gemm_f32(const float* x, const float* w, const float* bias, float* out, int epilogue, int m, int n, int k, void* stream);
-// With scratch memory of bc4g_gemm_f32_scratch's size on a 16-byte boundary: the same bits, many rows faster (scratch null: bc4g_gemm_f32).
-int bc4g_gemm_f32_many(const float* x, const float* w, const float* bias, float* out, void* scratch, int epilogue, int m, int n, int k, void* stream);
+// With scratch memory of `bytes`, at least what bc4g_gemm_f32_scratch says on the same device, on a 16-byte boundary: the same bits, many rows faster (scratch
+// null: bc4g_gemm_f32).
+int bc4g_gemm_f32_many(const float* x, const float* w, const float* bias, float* out, void* scratch, long bytes, int epilogue, int m, int n, int k,
+                       void* stream);
 // Up to 64 rows of it around an RMSNorm that no kernel of its own computes.  _emit: residual += x w^T (+ bias) and, for the norm with scale g
 // of the new residual, emit_x = residual * g and the rows' sums of squares over blocks of 16 columns, emit_ssq [ceil(n / 16)][m] -- or
 // [ceil(n / 16)][m][2] (halves), which is what m <= 8 rows leave whose blocks of 16 columns are no more than half the compute units.
@@ -79,7 +81,7 @@ int bc4g_gemm_f32_qkv(const float* x, const float* ssq, int ssq_blocks, int ssq_
                       int page_tokens, int write_kv, void* stream);
 // A question, no launch: rows of x and of w a workgroup of that product takes at once, 0 and 0 where it streams the weights.
 int bc4g_gemm_f32_tile(int m, int n, int k, int* rows, int* cols);
-// Another: the bytes of scratch memory bc4g_gemm_f32_many wants for a product (0: none).
+// Another: the bytes of scratch memory bc4g_gemm_f32_many wants for a product on the current device (0: none).
 int bc4g_gemm_f32_scratch(int m, int n, int k, long* bytes);
 
 // out[t, i] = silu(gate_i) * up_i                                        (swiglu.cu:17-25)

@@ -29,7 +29,7 @@ _SIGNATURES = {
     "bc4g_gemm_mfma_swiglu_scaled": [_P, _P, _I, _I, _F, _P, _I, _P, _I, _I, _I, _I, _P],
     "bc4g_gemm_generic": [_P, _I, _P, _I, _P, _I, _I, _P, _I, _I, _I, _P],
     "bc4g_gemm_f32": [_P, _P, _P, _P, _I, _I, _I, _I, _P],
-    "bc4g_gemm_f32_many": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
+    "bc4g_gemm_f32_many": [_P, _P, _P, _P, _P, c_long, _I, _I, _I, _I, _P],
     "bc4g_gemm_f32_scratch": [_I, _I, _I, _P],
     "bc4g_gemm_f32_emit": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "bc4g_gemm_f32_prenormed": [_P, _P, _I, _I, _F, _P, _P, _I, _I, _I, _I, _P],

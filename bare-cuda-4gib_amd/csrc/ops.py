@@ -315,16 +315,16 @@ def gemm_f32(x: torch.Tensor, w, accumulate_into: Optional[torch.Tensor] = None,
     else:
         epi = F32_GATED[act] if act is not None else F32_STORE
         out = torch.empty((m, n // 2 if act is not None else n), dtype=torch.float32, device=x.device)
-    nbytes = _gemm_f32_scratch(m, n, k)
+    nbytes = _gemm_f32_scratch(m, n, k, x.device.index)
     scratch = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
-    library.call("bc4g_gemm_f32_many", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), _ptr(scratch), epi, m, n, k, _stream(),
+    library.call("bc4g_gemm_f32_many", _ptr(x), _ptr(w), _ptr(bias), _ptr(out), _ptr(scratch), nbytes, epi, m, n, k, _stream(),
                  cost=_gemm_cost(m, n, k, 4, 4, 8 if accumulate_into is not None else 4.0 * out.shape[1] / n))
     return out
 
 
 @functools.lru_cache(maxsize=4096)
-def _gemm_f32_scratch(m: int, n: int, k: int) -> int:
-    """Bytes of scratch memory the float32 product of these sizes wants (0: none, few rows)."""
+def _gemm_f32_scratch(m: int, n: int, k: int, device: Optional[int] = None) -> int:
+    """Bytes of scratch memory the float32 product of these sizes wants on this device, the current one (0: none, few rows)."""
     if m <= 32 or k % 32:
         return 0
     nbytes = ctypes.c_long()

@@ -83,3 +83,17 @@ def test_rows_too_long_for_the_fused_norm(rows, k):
 def test_float32_products_leave_what_their_kernels_refuse_to_the_plain_one(k):
     row = torch.empty(1, k)
     assert ops.gemm_f32(row, row) is None
+
+
+def test_a_float32_product_asks_every_device_for_its_scratch_memory(monkeypatch):
+    """How much it is follows from the device's compute units: what one device said does not answer for another."""
+    wants = iter([4096, 65536])
+
+    def call(name, m, n, k, place, launches):
+        assert name == "bc4g_gemm_f32_scratch" and (m, n, k) == (2991, 1237, 1760) and not launches
+        place._obj.value = next(wants)
+    monkeypatch.setattr(ops.library, "call", call)
+    try:
+        assert [ops._gemm_f32_scratch(2991, 1237, 1760, device) for device in (0, 1, 0, 1)] == [4096, 65536, 4096, 65536]
+    finally:
+        ops._gemm_f32_scratch.cache_clear()

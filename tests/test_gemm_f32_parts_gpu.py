@@ -204,3 +204,18 @@ def test_error_of_lopsided_operands(ops, m, n, k, kind):
         plain = part if first == 0 else plain + part
     rms = lambda t: float(t.double().square().mean().sqrt())      # noqa: E731
     assert rms(got - z) <= 2.0 * max(rms(plain.double() - z[:rows]), 2.0 ** -26 * rms(z))
+
+
+def test_too_little_scratch_memory_is_refused(ops):
+    """Before anything is launched, whoever worked the size out."""
+    m, n, k = 300, 2048, 5632
+    x, w = operands(m, n, k, 3)
+    wants, out = ops._gemm_f32_scratch(m, n, k), torch.zeros(m, n, device=DEV)
+    scratch = torch.empty(wants, dtype=torch.uint8, device=DEV)
+    many = lambda nbytes: ops.library.call("bc4g_gemm_f32_many", x.data_ptr(), w.data_ptr(), None, out.data_ptr(), scratch.data_ptr(), nbytes, 0,      # noqa: E731
+                                           m, n, k, torch.cuda.current_stream().cuda_stream)
+    with pytest.raises(ops.KernelError, match="scratch memory"):
+        many(wants - 1)
+    assert not bool(out.any())
+    many(wants)
+    assert torch.equal(out, ops.gemm_f32(x, w))
