@@ -332,6 +332,19 @@ def _gemm_f32_scratch(m: int, n: int, k: int, device: Optional[int] = None) -> i
     return nbytes.value
 
 
+PRODUCT_SCRATCH_BYTES = 1 << 28      # the most that any product takes for itself while it runs: gemm_f32 x in parts and quarters' sums (kMostScratch in
+                                     # gemm_f32.hip), gemm_parts_accumulate_norm its parts (rows up to where 256 x 128 tiles fill the chip, times eight)
+
+
+def product_scratch_bytes(rows: int, layer_row_bytes: float, elem: int) -> float:
+    """An upper bound of what a product of a step with so many rows takes for itself, beside its output, in a layer whose products' outputs take
+    ``layer_row_bytes`` a row in activations of ``elem`` bytes: in float32 6 bytes a number of x and 16 an output; in bfloat16 up to eight parts of four bytes
+    an output of a product that is added to the stream, twice of which at least a layer has.  (Up to 64 rows parts are 4 MB at most.)"""
+    if rows <= (32 if elem == 4 else SKINNY_MAX_ROWS):
+        return 0.0
+    return min(PRODUCT_SCRATCH_BYTES, (4 if elem == 4 else 8) * rows * layer_row_bytes)
+
+
 GEMM_F32_FEW_ROWS = 64               # rows up to which a float32 product prepares or finishes an RMSNorm
 
 

@@ -211,11 +211,12 @@ class Model:
     def working_bytes(self, rows: int, n_logits: int, elem: int) -> int:
         """Device bytes a step of ``rows`` rows with logits at ``n_logits`` of them needs beyond weights and cache, as
         the parts state it: the float residual stream and a normed copy of it, the layer that needs most (one
-        layer's activations are given back before the next runs), and the float logits."""
+        layer's activations are given back before the next runs) with what its products take for themselves, and the float logits."""
+        from ..csrc import ops
         layer = max((part.working_bytes_per_row(elem) for part in self.layers), default=0.0)
         head = self.final_norm.part.working_bytes_per_row(elem) + self.hidden_size * elem
         per_row = self.hidden_size * (4 * self.streams + 4 + elem) + self.embedding.part.working_bytes_per_row(elem) + layer
-        return int(rows * per_row + n_logits * (head + 4 * self.vocab_size))
+        return int(rows * per_row + ops.product_scratch_bytes(rows, layer, elem) + n_logits * (head + 4 * self.vocab_size))
 
     # ---- forward ------------------------------------------------------------
     def forward(self, ctx: StepContext) -> Optional[torch.Tensor]:

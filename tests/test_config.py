@@ -96,3 +96,24 @@ def test_working_memory_is_what_the_parts_state():
     limited = working_memory_estimate(model, max_seqs=4, max_batch_tokens=32, graphs=0)
     unlimited = working_memory_estimate(model, max_seqs=4, max_batch_tokens=0, graphs=0, max_tokens=128)
     assert limited == model.working_bytes(32, 4, 2) and unlimited == model.working_bytes(128, 4, 2) > limited
+
+
+@pytest.mark.parametrize("h,q,kv,inter", [(64, 64, 32, 176), (2048, 2048, 256, 5632), (4096, 4096, 1024, 14336), (8192, 8192, 1024, 28672)])
+def test_working_memory_holds_what_the_products_take_for_themselves(h, q, kv, inter):
+    """Beside the parts' own: the scratch memory of float32 products, and the parts of k of bfloat16 ones that are added to the stream.  Neither is
+    ever more than PRODUCT_SCRATCH_BYTES, which only rows of an unheard-of length pass."""
+    from bare_cuda_4gib_amd.csrc import ops
+    from bare_cuda_4gib_amd.engine.model import Model
+    cfg = dict(helpers.TINY_A, hidden_size=h, num_attention_heads=q // 64 or 1, num_key_value_heads=kv // 64 or 1, head_dim=64, intermediate_size=inter)
+    model = Model(architecture_for(cfg).describe(LlamaConfig.from_dict(cfg)))
+    q, kv = 64 * cfg["num_attention_heads"], 64 * cfg["num_key_value_heads"]
+    products = [(q + 2 * kv, h), (h, q), (2 * inter, h), (h, inter)]
+    for rows in (33, 64, 65, 100, 256, 257, 270, 512, 1000, 1792, 2048, 3840, 4096, 8192, 50000):
+        for elem in (2, 4):
+            layer = max(part.working_bytes_per_row(elem) for part in model.layers)
+            counted = model.working_bytes(rows, 0, elem) - rows * (h * (8 + elem) + layer)
+            if elem == 4:
+                taken = max(ops._gemm_f32_scratch(rows, n, k) for n, k in products)
+            else:
+                taken = max(0 if parts == 1 or rows <= 64 else 4 * parts * rows * n for n, k in products[1::2] for parts in [ops.compute_plan(n, k).parts_tiles(rows)[0]])
+            assert taken <= ops.PRODUCT_SCRATCH_BYTES and taken <= counted <= ops.PRODUCT_SCRATCH_BYTES, (rows, elem)
