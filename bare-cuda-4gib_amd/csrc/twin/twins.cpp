@@ -184,6 +184,39 @@ bool gemm_generic() {
   return ok;
 }
 
+bool gemm_f32_tiles() {
+  Rng rng(44);
+  bool ok = true;
+  // tiles of all three sizes, and the first cut into quarters of k: with scratch memory and without, the same bits
+  const int sizes[][3] = {{300, 2046, 544}, {1000, 2562, 1056}, {70, 8190, 96}, {200, 6144, 2080}};
+  for (const auto& size : sizes) {
+    const int m = size[0], n = size[1], k = size[2];
+    const std::vector<float> x = normals(rng, static_cast<size_t>(m) * k), w = normals(rng, static_cast<size_t>(n) * k, 0.1f);
+    const std::vector<float> before = normals(rng, static_cast<size_t>(m) * n), bias = normals(rng, n);
+    long bytes = 0;
+    RUN(bc4g_gemm_f32_scratch(m, n, k, &bytes));
+    Dev<float> dx(x), dw(w), db(bias), out(static_cast<size_t>(m) * n), with(static_cast<size_t>(m) * n), acc(before);
+    Dev<unsigned char> scratch(static_cast<size_t>(bytes));
+    RUN(bc4g_gemm_f32(dx.p, dw.p, nullptr, out.p, 0, m, n, k, kStream));
+    RUN(bc4g_gemm_f32_many(dx.p, dw.p, nullptr, with.p, bytes ? scratch.p : nullptr, bytes, 0, m, n, k, kStream));
+    RUN(bc4g_gemm_f32_many(dx.p, dw.p, db.p, acc.p, bytes ? scratch.p : nullptr, bytes, 1, m, n, k, kStream));
+    const std::vector<float> got = out.get(), same = with.get(), added = acc.get();
+    std::vector<double> some, want, some_added, want_added;      // (a few rows: the plain twin walks them one by one)
+    for (int r : {0, 1, m / 2, m - 2, m - 1}) {
+      const std::vector<float> row(x.begin() + static_cast<size_t>(r) * k, x.begin() + static_cast<size_t>(r + 1) * k);
+      const std::vector<double> z = plain::gemm(widen(row), widen(w), 1, n, k);
+      for (int i = 0; i < n; ++i) {
+        const size_t at = static_cast<size_t>(r) * n + i;
+        some.push_back(got[at]), want.push_back(z[i]), some_added.push_back(added[at]), want_added.push_back(z[i] + before[at] + bias[i]);
+      }
+    }
+    ok &= close("float product on tiles", some, want, 1e-5, 1e-5);
+    ok &= close("float product on tiles, added", some_added, want_added, 1e-5, 1e-5);
+    ok &= close("float product on tiles with scratch memory and without", widen(same), widen(got), 0.0, 0.0);
+  }
+  return ok;
+}
+
 bool gemm_skinny() {
   Rng rng(5);
   bool ok = true;
@@ -681,6 +714,7 @@ const std::vector<std::pair<std::string, std::function<bool()>>>& tests() {
       {"rmsnorm", rmsnorm},
       {"swiglu", swiglu},
       {"gemm_generic", gemm_generic},
+      {"gemm_f32_tiles", gemm_f32_tiles},
       {"gemm_skinny", gemm_skinny},
       {"gemm_skinny_norms", gemm_skinny_norms},
       {"gemm_mfma", gemm_mfma},

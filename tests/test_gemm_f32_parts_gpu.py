@@ -237,3 +237,39 @@ def test_rows_in_blocks(ops, m, n, k, epilogue):
     got = product(slice(0, m))
     for first in list(range(0, m - 5, 311)) + [m - 5]:
         assert torch.equal(product(slice(first, first + 5)), got[first:first + 5])
+
+
+def without_scratch(ops, x, w, epilogue, out, bias=None):
+    (m, k), n = x.shape, w.shape[0]
+    ops.library.call("bc4g_gemm_f32", x.data_ptr(), w.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                     {"store": 0, "add with bias": 1, "silu": 2, "gelu_tanh": 3}[epilogue], m, n, k, torch.cuda.current_stream().cuda_stream)
+    return out
+
+
+# Callers without scratch memory: tiles of each size whose waves split x themselves, rows and columns that end inside one, k that ends inside a pair.
+@pytest.mark.parametrize("m,n,k", [(1000, 2562, 1056), (1793, 2050, 544), (300, 8190, 96), (129, 11262, 2080), (700, 1030, 4128), (65, 28672, 64), (40, 2048, 2048)])
+@pytest.mark.parametrize("epilogue", ["store", "add with bias", "silu", "gelu_tanh"])
+def test_without_scratch_memory(ops, m, n, k, epilogue):
+    x, w = operands(m, n, k, m + 2 * k)
+    base, bias = torch.randn(m, n, device=DEV), torch.randn(n, device=DEV) if epilogue == "add with bias" else None
+    x[m - 2, k - 3], x[m // 2, 1] = float("nan"), float("inf")
+    out = base.clone() if bias is not None else torch.full((m, n if epilogue == "store" else n // 2), -7.0, device=DEV)
+    got = without_scratch(ops, x, w, epilogue, out, bias)
+    want = ops.gemm_f32(x, w, accumulate_into=base.clone(), bias=bias) if bias is not None else ops.gemm_f32(x, w, act=None if epilogue == "store" else epilogue)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+def test_many_rows_without_scratch_memory_go_to_tiles(ops):
+    """They take up to twice the time of a product with it (the few rows' kernel, where they went in between: 2.5 times)."""
+    x, w = operands(1000, 11264, 2048, 5)
+    out = torch.empty(1000, 11264, device=DEV)
+
+    def fastest(f):
+        best = math.inf
+        for _ in range(8):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record(), f(), b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+    assert fastest(lambda: without_scratch(ops, x, w, "store", out)) < 2.0 * fastest(lambda: ops.gemm_f32(x, w))
