@@ -865,12 +865,11 @@ class LinearPlan:
         return m >= 5 and self.n >= (16384 if self.k >= 1024 else 24576) and self.streams(m)
 
     def parts(self, m: int) -> int:
-        """Into how many parts an adding product of few rows, up to 256, cuts k over workgroups (1: it does not)."""
-        return self.parts_tiles(m)[0] if m <= 256 else 1
+        """Into how many parts an adding product of m rows cuts k over workgroups (1: it does not)."""
+        return self.parts_tiles(m)[0]
 
     def parts_tiles(self, m: int) -> Tuple[int, int]:
-        """The same for any number of rows: the parts, and the rows of the tiles they are computed in (of 64 x 64, 128 x 128 or
-        256 x 128)."""
+        """The parts, and the rows of the tiles they are computed in (of 64 x 64, 128 x 128 or 256 x 128)."""
         lo, hi = self.parts_rows
         if not (lo <= m <= hi):
             return 1, 64
@@ -1183,18 +1182,13 @@ class Finished:
         self.tensor = tensor
 
 
-def parts_of_k(m: int, n: int, k: int) -> int:
-    """Into how many parts gemm_parts_accumulate_norm cuts k of a product of few rows (LinearPlan.parts)."""
-    return plan_for(n, k).parts(m)
-
-
 def gemm_parts_supported(a: torch.Tensor, w, residual: torch.Tensor, g: torch.Tensor) -> bool:
     """Whether gemm_parts_accumulate_norm takes these operands: bfloat16, rows whose product the plan cuts over
     workgroups, a plain RMSNorm after it."""
     # (asked by every adding product of a step: the rows first, which settle most)
     w, _ = _weight(w)
     x, y = a.shape, w.shape
-    return (len(x) == 2 and len(y) == 2 and plan_for(y[0], y[1]).parts_tiles(x[0])[0] > 1
+    return (len(x) == 2 and len(y) == 2 and plan_for(y[0], y[1]).parts(x[0]) > 1
             and _fast_operands(a, w) and residual.dtype == torch.float32 and residual.is_contiguous()
             and residual.shape == (x[0], y[0]) and g.dtype in _CODE and g.shape == (y[0],)
             and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and residual.data_ptr() % 16 == 0 and a.is_contiguous()

@@ -155,7 +155,7 @@ def test_tinyllama_widths_steps_of_65_to_256_rows(tinyllama, dtype):
     from bare_cuda_4gib_amd.engine import Executor, StepEntry, load_model
     folder, _, plain, _ = tinyllama(dtype)
     model, _ = load_model(folder, dtype, "cuda:0")
-    assert ops.parts_of_k(80, 2048, 2048) > 1 and ops.parts_of_k(120, 2048, 5632) > 1 and ops.parts_of_k(200, 2048, 5632) > 1
+    assert ops.plan_for(2048, 2048).parts(80) > 1 and ops.plan_for(2048, 5632).parts(120) > 1 and ops.plan_for(2048, 5632).parts(200) > 1
     n = 40
     prompts = [helpers.random_ids(17 + (3 * i) % 5, 32000, 1500 + i) for i in range(n)]
     want = [plain_rows(plain, ids, range(len(ids) - 12, len(ids))) for ids in prompts]
@@ -221,7 +221,7 @@ def test_decode_batch_of_16_at_llama3_8b_widths_in_a_captured_graph(tmp_path_fac
     folder = os.path.join(str(tmp_path_factory.getbasetemp()), "llama3_8b_widths")
     if not os.path.exists(os.path.join(folder, "model.safetensors")):
         write_random_model(LLAMA3_8B_WIDTHS, 41, folder, "bfloat16", norm_std=0.1, scales={"lm_head.weight": 0.125})
-    assert ops.parts_of_k(16, 4096, 4096) > 1 and ops.parts_of_k(16, 4096, 14336) > 1
+    assert ops.plan_for(4096, 4096).parts(16) > 1 and ops.plan_for(4096, 14336).parts(16) > 1
     n, tail = 16, 4
     prompts = [helpers.random_ids(6 + i % 5 + tail, 128256, 1700 + i) for i in range(n)]
     plain = PlainLlama(folder)

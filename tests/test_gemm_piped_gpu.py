@@ -58,7 +58,7 @@ def test_parts_of_k(ops, m, n, k, parts, tile):
 def test_an_adding_product_and_the_norm_behind_it(ops, m, n, k, parts, tile):
     """As many parts as the weight's plan says, against float64: the sums to k float additions of terms around k ** -0.5, the norm to a rounding."""
     plan = ops.plan_for(n, k)
-    assert plan.parts_tiles(m) == (parts, tile) and plan.parts(m) == (parts if m <= 256 else 1)
+    assert plan.parts_tiles(m) == (parts, tile) and plan.parts(m) == parts
     if parts == 1:
         return
     x, w = rnd(m, k, seed=6).to(DEV), (rnd(n, k, seed=7) * k ** -0.5).to(DEV)

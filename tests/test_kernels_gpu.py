@@ -66,7 +66,8 @@ def test_rmsnorm(ops, wdt, odt):
 def test_adding_product_in_parts_of_k_with_the_norm_after_it(ops, m, n, k):
     """A few dozen rows: the product's k cut over workgroups, the parts added to the residual in order by the kernel
     that norms it -- against the definition, and the residual against the product that adds at once."""
-    assert ops.parts_of_k(m, n, k) > 1 and ops.parts_of_k(9, n, k) == 1 and ops.parts_of_k(257, n, k) == 1
+    plan = ops.plan_for(n, k)
+    assert plan.parts(m) > 1 and plan.parts(9) == 1 and plan.parts(plan.parts_rows[1] + 1) == 1
     a, w = bf(rnd(m, k, seed=80)), bf(rnd(n, k, seed=81, scale=0.3))
     base, g = rnd(m, n, seed=82).float(), (1.0 + 0.1 * rnd(n, seed=83)).bfloat16()
     resid = base.clone().to(DEV)

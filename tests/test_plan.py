@@ -25,6 +25,21 @@ def test_plans_of_the_known_shapes():
     assert ops.compute_plan(2048, 11008).fused_norm_rows == 4 and ops.compute_plan(4096, 14336).fused_norm_rows == 0
 
 
+def test_parts_of_products_that_are_added_to_the_stream():
+    """What production asks (parts_tiles), up to where 256 x 128 tiles fill the chip and beyond 256 rows: the parts and the tiles' rows."""
+    square, down, long = ops.compute_plan(2048, 2048), ops.compute_plan(2048, 5632), ops.compute_plan(4096, 14336)
+    assert square.parts_rows == down.parts_rows == (65, 3840) and long.parts_rows == (10, 1792)
+    assert [square.parts_tiles(m) for m in (64, 65, 256, 257)] == [(1, 64), (4, 64), (2, 64), (1, 64)]
+    assert [down.parts_tiles(m) for m in (256, 257, 300, 512, 1000)] == [(2, 64), (4, 128), (4, 128), (1, 64), (2, 128)]
+    assert [long.parts_tiles(m) for m in (65, 256, 257, 512, 1000)] == [(8, 128), (4, 128), (2, 128), (4, 256), (2, 256)]
+    for plan in (square, down, long):
+        lo, hi = plan.parts_rows
+        assert plan.parts(lo - 1) == 1 == plan.parts(hi + 1) and plan.parts(lo) > 1
+        assert all(plan.parts(m) == plan.parts_tiles(m)[0] and plan.k % (64 * plan.parts(m)) == 0 for m in range(1, hi + 2))
+    two = ops.compute_plan(2048, 5632, cus=128)                # half the chip: its tiles are full at half the rows
+    assert two.parts_rows == (65, 1792)
+
+
 def test_another_width_or_machine_gets_thresholds_of_its_own():
     assert ops.compute_plan(8192, 2048).stream_rows == 23 and ops.compute_plan(8128, 2048).stream_rows == 64
     assert ops.compute_plan(8192, 2048, cus=304).stream_rows == 64             # more CUs: a wider output to fill them
