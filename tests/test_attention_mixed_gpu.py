@@ -56,6 +56,8 @@ def test_portions_and_tokens_together(ops, nh, nkv, d, page, window, monkeypatch
     monkeypatch.setattr(ops, "ATTENTION_TOGETHER_CONTEXT", 4000)
     apart, notes = run()
     assert notes["apart"] and not notes["together"]
-    # weights and outputs are rounded to bfloat16 in both: 2 ** -8 of values around 1, the sums' order aside
+    # weights and outputs are rounded to bfloat16 in both: 2 ** -9 of a value each, of 16 to 256 values a head.  By head and row, as outputs shrink with
+    # the context: of the row at 4,090 tokens, cut into the most parts, any one tile of 32 keys is 2 to 5 times this bound (in 64 bits, 150 rows).
     for got, want, what in ((together, plain, "plain"), (together, apart, "two launches")):
-        assert (got.float() - want.float()).abs().max() < 2e-2, what
+        off, size = ((t.float().view(start[-1], nh, d).abs().amax(2)) for t in (got.float() - want.float(), want))
+        assert float((off / (2.0 ** -6 * size + 1e-6)).max()) <= 1.0, what
