@@ -6,11 +6,14 @@
 // and feeds 32x32x16 MFMAs.  Two forms:
 //  - the operand tiles go from memory into LDS without passing registers (k a multiple of 64, operands on 16-byte
 //    boundaries): gemm_mfma_halves_kernel for tiles of 256 x 256, gemm_mfma_turns_kernel for 256 x 192,
-//    gemm_mfma_piped_kernel for 256 x 128, 128 x 128 and 128 x 64 (q|k|v), gemm_mfma_ahead_kernel for 64 x 64 -- and gemm_mfma_direct_kernel for most of them where k is short (short_walk); whichever lets the busiest CU finish
-//    first, or two of them side by side (parts_of).
+//    gemm_mfma_piped_kernel for 256 x 128, 128 x 128 and 128 x 64 (q|k|v), gemm_mfma_ahead_kernel for 64 x 64 -- and
+//    gemm_mfma_direct_kernel for most of them where k is short (short_walk); whichever lets the busiest CU finish first, or two of them
+//    side by side (parts_of).
 //  - gemm_mfma_staged_kernel: through registers, 128 x 128 tiles; any k that is a multiple of 8.
 // Every output element is accumulated over k in ascending order in both, whatever the number of
-// rows and the tile: the same bits whichever form and tile a shape selects.
+// rows and the tile: the same bits whichever form and tile a shape selects.  (Products that are added to the residual stream may be cut into
+// parts of k by their callers, bc4g_gemm_mfma_parts and _large, whose sums are added up afterwards: other bits, by a rounding of float, and
+// whether and into how many depends on the number of rows, up to 3,840 of them for 2,048 outputs.)
 // Rows and columns beyond the matrix are not stored.
 //
 // What bounds these kernels: the loop over k is 85-90 % of a tile's time where k is long.  With all waves of a workgroup reading, waiting and
@@ -1421,6 +1424,10 @@ int launch_halves(const Operands& o, const RopeKvArgs& ra, const RowScaleArgs& s
 // memory and flatters the small tiles and the short rings.  The model's times are within 5 % of those measured for 72 to 4,096 rows at
 // outputs of 2,048 to 28,672 and k of 2,048 to 14,336 (one product after the other without a pause 1 % short to 7 % long at the median, 64 x 64
 // 18 % long).  A function of (m, n, k) alone; every tile adds over k in the same order.
+// That is what they were fitted to, and of 256 x 128 and 128 x 128 tiles, and of the 64 x 256 ones beside whole tiles (kRestForm), it is no more: these were walked by
+// kernels whose waves go together or take turns, and gemm_mfma_piped_kernel, which walks them now, takes 0.55 / 0.84 and 0.31 / 0.52 us a step (kQkvForm).  kDirectForm still
+// ranks the forms as measured then (256 x 128, 0.87 / 1.06, a little lower since); over 48 products the tiles it chooses take 0.944 of the time with the kernels of
+// now, 1,025 rows of 4,096 x 14,336 189 -> 194 us and 270 rows of 28,672 x 4,096 90 -> 91 the other way.
 struct DirectForm {
   int rows, cols;
   double us_a_step_few, us_a_step_full, us_around, us_stores;
