@@ -81,7 +81,7 @@ int bc4g_gemm_f32_qkv(const float* x, const float* ssq, int ssq_blocks, int ssq_
                       int page_tokens, int write_kv, void* stream);
 // A question, no launch: rows of x and of w a workgroup of that product takes at once, 0 and 0 where it streams the weights.
 int bc4g_gemm_f32_tile(int m, int n, int k, int* rows, int* cols);
-// Another: the bytes of scratch memory bc4g_gemm_f32_many wants for a product on the current device (0: none; k up to 349,525: 2^28 at most).
+// Another: the bytes of scratch memory bc4g_gemm_f32_many wants for a product on the current device (0: none; k up to 1,398,101: 2^30 at most).
 int bc4g_gemm_f32_scratch(int m, int n, int k, long* bytes);
 
 // out[t, i] = silu(gate_i) * up_i                                        (swiglu.cu:17-25)

@@ -332,8 +332,9 @@ def _gemm_f32_scratch(m: int, n: int, k: int, device: Optional[int] = None) -> i
     return nbytes.value
 
 
-PRODUCT_SCRATCH_BYTES = 1 << 28      # the most that any product takes for itself while it runs: gemm_f32 x in parts and quarters' sums (kMostScratch in
-                                     # gemm_f32.hip), gemm_parts_accumulate_norm its parts (rows up to where 256 x 128 tiles fill the chip, times eight)
+# The most that a product takes for itself while it runs, by the bytes of an activation: gemm_f32 x in parts and quarters' sums (kMostScratch in gemm_f32.hip),
+# gemm_parts_accumulate_norm its parts (rows up to where 256 x 128 tiles fill the chip, times eight).
+PRODUCT_SCRATCH_BYTES = {4: 1 << 30, 2: 1 << 28}
 
 
 def product_scratch_bytes(rows: int, layer_row_bytes: float, elem: int) -> float:
@@ -342,7 +343,7 @@ def product_scratch_bytes(rows: int, layer_row_bytes: float, elem: int) -> float
     an output of a product that is added to the stream, twice of which at least a layer has.  (Up to 64 rows parts are 4 MB at most.)"""
     if rows <= (32 if elem == 4 else SKINNY_MAX_ROWS):
         return 0.0
-    return min(PRODUCT_SCRATCH_BYTES, (4 if elem == 4 else 8) * rows * layer_row_bytes)
+    return min(PRODUCT_SCRATCH_BYTES[elem], (4 if elem == 4 else 8) * rows * layer_row_bytes)
 
 
 GEMM_F32_FEW_ROWS = 64               # rows up to which a float32 product prepares or finishes an RMSNorm

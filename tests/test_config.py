@@ -116,4 +116,4 @@ def test_working_memory_holds_what_the_products_take_for_themselves(h, q, kv, in
                 taken = max(ops._gemm_f32_scratch(rows, n, k) for n, k in products)
             else:
                 taken = max(0 if parts == 1 or rows <= 64 else 4 * parts * rows * n for n, k in products[1::2] for parts in [ops.compute_plan(n, k).parts_tiles(rows)[0]])
-            assert taken <= ops.PRODUCT_SCRATCH_BYTES and taken <= counted <= ops.PRODUCT_SCRATCH_BYTES, (rows, elem)
+            assert taken <= ops.PRODUCT_SCRATCH_BYTES[elem] and taken <= counted <= ops.PRODUCT_SCRATCH_BYTES[elem], (rows, elem)
